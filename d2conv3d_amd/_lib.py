@@ -22,6 +22,8 @@ EXPORTS = (
     "d2c_conv3d_prepared_bytes", "d2c_conv3d_forward_prepared", "d2c_conv3d_backward_prepared",
     "d2c_conv3d_columns_bytes", "d2c_conv3d_forward_columns", "d2c_conv3d_backward_columns_workspace_bytes",
     "d2c_conv3d_backward_columns",
+    "d2c_plain_conv3d_input_bytes", "d2c_plain_conv3d_forward_workspace_bytes",
+    "d2c_plain_conv3d_backward_workspace_bytes", "d2c_plain_conv3d_forward", "d2c_plain_conv3d_backward",
     "d2c_conv1d_check", "d2c_conv1d_algo", "d2c_conv1d_forward_workspace_bytes", "d2c_conv1d_backward_workspace_bytes",
     "d2c_conv1d_forward", "d2c_conv1d_backward", "d2c_conv3d_corner_index", "d2c_conv3d_sample",
     "d2c_conv3d_offset_histogram",
@@ -140,6 +142,13 @@ def load():
     lib.d2c_conv3d_forward_columns.restype = ctypes.c_int
     lib.d2c_conv3d_backward_columns.argtypes = [p3, vp] + [vp] * 5 + [vp, sz] + [vp] * 5 + [vp, sz, vp]
     lib.d2c_conv3d_backward_columns.restype = ctypes.c_int
+    for name in ("input_bytes", "forward_workspace_bytes", "backward_workspace_bytes"):
+        f = getattr(lib, f"d2c_plain_conv3d_{name}")
+        f.argtypes, f.restype = [p3], sz
+    lib.d2c_plain_conv3d_forward.argtypes = [p3] + [vp] * 5 + [sz, vp, sz, vp]
+    lib.d2c_plain_conv3d_forward.restype = ctypes.c_int
+    lib.d2c_plain_conv3d_backward.argtypes = [p3, vp, vp, sz] + [vp] * 5 + [sz, vp]
+    lib.d2c_plain_conv3d_backward.restype = ctypes.c_int
     lib.d2c_conv1d_algo.argtypes, lib.d2c_conv1d_algo.restype = [p1], ctypes.c_int
     lib.d2c_conv3d_corner_index.argtypes = [p3, vp, vp, vp, vp]
     lib.d2c_conv3d_corner_index.restype = ctypes.c_int

@@ -578,6 +578,70 @@ def deform_conv3d_packed(input, deformation, weight, bias, lead, mask_activation
         int(offset_groups), float(relu_scale), bool(want_stats), int(offset_axes), int(backward_flags))
 
 
+def _plain_desc(input, weight, stride, padding, dilation):
+    N, Cin, D, H, W = input.shape
+    Cout, _, kd, kh, kw = weight.shape
+    dims = [(n + 2 * p - (d * (k - 1) + 1)) // s + 1
+            for n, k, s, p, d in zip((D, H, W), (kd, kh, kw), stride, padding, dilation)]
+    return _lib.Conv3dDesc(N, Cin, Cout, D, H, W, kd, kh, kw, *stride, *padding, *dilation, 1, 1, *dims,
+                           _DT[input.dtype], _DT[input.dtype], _lib.EPILOGUE_NONE, 1.0)
+
+
+def plain_conv3d_supported(input, weight, stride, padding, dilation):
+    """Whether plain_conv3d takes these tensors (bfloat16, one weight group, input channels a multiple of 64)."""
+    if not input.is_cuda or input.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
+        return False
+    desc = _plain_desc(input, weight, stride, padding, dilation)
+    return _lib.load().d2c_plain_conv3d_input_bytes(ctypes.byref(desc)) > 0
+
+
+class _PlainConv3dFunction(torch.autograd.Function):
+    """conv3d of a deformation branch on the library's matrix-core kernels (d2c_plain_conv3d_*).  The channels-last
+    copy of the input that the forward call makes is what the backward call keeps, not the input."""
+
+    @staticmethod
+    def forward(ctx, input, weight, bias, stride, padding, dilation):
+        lib = _lib.load()
+        input, weight = input.contiguous(), weight.contiguous()
+        bias = bias.contiguous() if bias is not None else None
+        desc = _plain_desc(input, weight, stride, padding, dilation)
+        ref, dev = ctypes.byref(desc), input.device
+        out = torch.empty((desc.N, desc.Cout, desc.Do, desc.Ho, desc.Wo), dtype=input.dtype, device=dev)
+        with torch.cuda.device(dev):
+            copy = torch.empty(lib.d2c_plain_conv3d_input_bytes(ref), dtype=torch.uint8, device=dev)
+            nb = lib.d2c_plain_conv3d_forward_workspace_bytes(ref)
+            ws = _workspace(nb, dev)
+            rc = lib.d2c_plain_conv3d_forward(ref, _ptr(input), _ptr(weight), _ptr(bias), _ptr(out), _ptr(copy),
+                                              copy.numel(), _ptr(ws), nb, _stream(dev))
+        _lib.check(rc, "plain_conv3d forward")
+        ctx.save_for_backward(copy, weight)
+        ctx.desc, ctx.has_bias, ctx.input_shape = desc, bias is not None, input.shape
+        return out
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, grad_out):
+        lib = _lib.load()
+        copy, weight = ctx.saved_tensors
+        ref, dev, need = ctypes.byref(ctx.desc), weight.device, ctx.needs_input_grad
+        grad_out = grad_out.contiguous()
+        gx = torch.empty(ctx.input_shape, dtype=weight.dtype, device=dev) if need[0] else None
+        gw = torch.empty_like(weight) if need[1] else None
+        gb = torch.empty(weight.shape[0], dtype=weight.dtype, device=dev) if (ctx.has_bias and need[2]) else None
+        with torch.cuda.device(dev):
+            nb = lib.d2c_plain_conv3d_backward_workspace_bytes(ref)
+            ws = _workspace(nb, dev)
+            rc = lib.d2c_plain_conv3d_backward(ref, _ptr(grad_out), _ptr(copy), copy.numel(), _ptr(weight), _ptr(gx),
+                                               _ptr(gw), _ptr(gb), _ptr(ws), nb, _stream(dev))
+        _lib.check(rc, "plain_conv3d backward")
+        return gx, gw, gb, None, None, None
+
+
+def plain_conv3d(input, weight, bias, stride, padding, dilation):
+    """The ordinary convolution conv3d(input, weight, bias, stride, padding, dilation) where plain_conv3d_supported."""
+    return _PlainConv3dFunction.apply(input, weight, bias, tuple(stride), tuple(padding), tuple(dilation))
+
+
 class _GroupNormFromStats(torch.autograd.Function):
     """torch.nn.functional.group_norm on the output of a convolution whose forward kernels already added up the
     per-(sample, channel) sums (d2c_conv3d_forward_stats): d2c_group_norm_forward / _backward."""

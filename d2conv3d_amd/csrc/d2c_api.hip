@@ -464,6 +464,47 @@ int d2c_conv3d_backward_prepared(const d2c_conv3d_desc *q, const void *gout, con
                               prep.base ? &prep : nullptr);
 }
 
+size_t d2c_plain_conv3d_input_bytes(const d2c_conv3d_desc *q)
+{
+    return d2c_conv3d_check(q) == D2C_OK && d2c_plain_supported(*q) ? d2c_plain_input_bytes(*q) : 0;
+}
+size_t d2c_plain_conv3d_forward_workspace_bytes(const d2c_conv3d_desc *q)
+{
+    return d2c_plain_conv3d_input_bytes(q) ? d2c_plain_forward_ws(*q) : 0;
+}
+size_t d2c_plain_conv3d_backward_workspace_bytes(const d2c_conv3d_desc *q)
+{
+    return d2c_plain_conv3d_input_bytes(q) ? d2c_plain_backward_ws(*q) : 0;
+}
+
+static int check_plain(const d2c_conv3d_desc *q, const void *copy, size_t copy_bytes)
+{
+    if (int rc = d2c_conv3d_check(q)) return rc;
+    if (!d2c_plain_supported(*q)) {
+        d2c_set_error("d2c_plain_conv3d: bfloat16, one weight group and input channels a multiple of 64 only");
+        return D2C_ERR_UNSUPPORTED;
+    }
+    return check_ws(d2c_plain_input_bytes(*q), const_cast<void *>(copy), copy_bytes);
+}
+
+int d2c_plain_conv3d_forward(const d2c_conv3d_desc *q, const void *x, const void *weight, const void *bias, void *out, void *copy,
+                             size_t copy_bytes, void *ws, size_t ws_bytes, void *stream)
+{
+    if (int rc = check_plain(q, copy, copy_bytes)) return rc;
+    if (!x || !weight || !out) { d2c_set_error("null tensor pointer"); return D2C_ERR_SHAPE; }
+    if (int rc = check_ws(d2c_plain_forward_ws(*q), ws, ws_bytes)) return rc;
+    return d2c_plain_forward(*q, x, weight, bias, out, copy, ws, (hipStream_t)stream);
+}
+
+int d2c_plain_conv3d_backward(const d2c_conv3d_desc *q, const void *gout, const void *copy, size_t copy_bytes, const void *weight,
+                              void *gx, void *gw, void *gb, void *ws, size_t ws_bytes, void *stream)
+{
+    if (int rc = check_plain(q, copy, copy_bytes)) return rc;
+    if (!gout || !weight) { d2c_set_error("null tensor pointer"); return D2C_ERR_SHAPE; }
+    if (int rc = check_ws(d2c_plain_backward_ws(*q), ws, ws_bytes)) return rc;
+    return d2c_plain_backward(*q, gout, copy, weight, gx, gw, gb, ws, (hipStream_t)stream);
+}
+
 size_t d2c_static_workspace_bytes(void) { return (size_t)D2C_STATIC_WORKSPACE_BYTES; }
 
 int d2c_conv3d_forward_static(const d2c_conv3d_desc *q, const void *x, const void *offset, const void *mask,

@@ -1,0 +1,770 @@
+// The ordinary convolution of a layer's deformation branch (`deform_params`, network/layers.py:66-68), bfloat16, on
+// the matrix cores.  It has no sampling points: a tap of an output position is one voxel, so the three products below
+// read 128-byte pieces of channels-last rows straight into LDS, one per (position, tap), where the deformable operator
+// at zero offsets interpolates eight and the backward pass goes through grad-column rows, sample lists and kept columns.
+//
+//   forward       out[o, m]   = bias[o] + sum_{tap, c} W[o, c, tap] * x[vox(m, tap), c]      conv_rows_kernel
+//   grad_input    gx[c, v]    = sum_{tap, o} W[o, c, tap] * gout[pos(v, tap), o]             conv_rows_kernel
+//   grad_weight   gW[o, c, tap] = sum_m gout[o, m] * x[vox(m, tap), c]                       conv_weight_kernel
+//
+// (m: output positions over the whole batch, v: input voxels; a row that a tap puts outside the volume is a row of
+// zeros.)  Everything the kernels need in another order is made by one launch per direction (conv_prepare_kernel).
+// Sums that are shared out between workgroups are written as float partial results and added up in a fixed order by
+// the finishing kernels: nothing is cleared, and equal inputs give equal bits.
+//
+// 1024 -> 30 channels on 8x30x54 (forward): 0.51 ms at zero offsets on the gather kernel; figures of these kernels
+// are at each one.
+#include "d2c_mma.hpp"
+#include <algorithm>
+
+namespace {
+
+constexpr int kThreads = 256;
+constexpr int kMT = 128;              // rows (positions) per workgroup of conv_rows_kernel
+constexpr int kCW = 64;               // positions per step of conv_weight_kernel
+
+D2C_DEV int xcd_swizzle(int bid, int n)
+{
+    const int x = bid & 7, idx = bid >> 3;
+    const int q = n >> 3, r = n & 7;
+    return x * q + (x < r ? x : r) + idx;
+}
+
+// One spatial axis triple of a gather: rows on the grid (d, h, w) read rows on the grid (sd, sh, sw).
+struct RowMap {
+    int N, P;                         // samples, rows per sample (the grid's points)
+    int d, h, w;                      // grid of the result rows
+    int sd, sh, sw;                   // grid of the source rows
+    TapGeom g;
+    int back;                         // 0: source = o * stride - pad + tap * dilation; 1: the transposed map
+    FastDiv dP, dHW, dW;
+};
+inline RowMap row_map(const d2c_conv3d_desc &q, bool back)
+{
+    RowMap r;
+    r.N = q.N;
+    r.back = back ? 1 : 0;
+    r.g = make_geom(q);
+    r.d = back ? q.D : q.Do; r.h = back ? q.H : q.Ho; r.w = back ? q.W : q.Wo;
+    r.sd = back ? q.Do : q.D; r.sh = back ? q.Ho : q.H; r.sw = back ? q.Wo : q.W;
+    r.P = r.d * r.h * r.w;
+    r.dP = make_fastdiv(r.P); r.dHW = make_fastdiv(r.h * r.w); r.dW = make_fastdiv(r.w);
+    return r;
+}
+
+// grid point of row m: sample and the source coordinates of tap (0, 0, 0), unclipped (transposed map: before the
+// division by the stride)
+struct RowPos {
+    int b, z, y, x;
+    bool ok;
+};
+D2C_DEV RowPos row_pos(const RowMap &r, int m)
+{
+    RowPos p;
+    p.ok = m < r.N * r.P;
+    const int mm = p.ok ? m : 0;
+    p.b = fdiv(mm, r.dP);
+    const int q = mm - p.b * r.P, z = fdiv(q, r.dHW), rem = q - z * (r.h * r.w), y = fdiv(rem, r.dW), x = rem - y * r.w;
+    p.z = r.back ? z + r.g.pd : z * r.g.sd - r.g.pd;
+    p.y = r.back ? y + r.g.ph : y * r.g.sh - r.g.ph;
+    p.x = r.back ? x + r.g.pw : x * r.g.sw - r.g.pw;
+    return p;
+}
+// source row of (row, tap (kz, ky, kx)), or -1
+D2C_DEV int source_row(const RowMap &r, const RowPos &p, int kz, int ky, int kx)
+{
+    int z, y, x;
+    bool ok = p.ok;
+    if (r.back) {
+        z = p.z - kz * r.g.dd; y = p.y - ky * r.g.dh; x = p.x - kx * r.g.dw;
+        ok = ok && z >= 0 && y >= 0 && x >= 0;
+        if (r.g.sd != 1 || r.g.sh != 1 || r.g.sw != 1) {
+            const int qz = z / r.g.sd, qy = y / r.g.sh, qx = x / r.g.sw;
+            ok = ok && qz * r.g.sd == z && qy * r.g.sh == y && qx * r.g.sw == x;
+            z = qz; y = qy; x = qx;
+        }
+    } else {
+        z = p.z + kz * r.g.dd; y = p.y + ky * r.g.dh; x = p.x + kx * r.g.dw;
+        ok = ok && z >= 0 && y >= 0 && x >= 0;
+    }
+    ok = ok && z < r.sd && y < r.sh && x < r.sw;
+    return ok ? ((p.b * r.sd + z) * r.sh + y) * r.sw + x : -1;
+}
+
+// ---- LDS reads of data that DMA transfers filled (see lds_row_read in d2c_mma.hpp), and counted waits
+template <int N> D2C_DEV void wait_lds(u32x4_t &a) { asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(a) : "n"(N)); }
+template <int N> D2C_DEV void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+D2C_DEV void group_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+D2C_DEV void dma16(const void *src, unsigned char *lds)
+{
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
+                                     (__attribute__((address_space(3))) void *)lds, 16, 0, 0);
+}
+D2C_DEV u32x4_t lds_read16(unsigned a)
+{
+    u32x4_t v;
+    asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(a));
+    return v;
+}
+
+// 16-byte slot of channel vector v of row r in an LDS tile of KC-channel rows: consecutive rows spread over all 16
+// slots of the 64 banks, so that the reads of 16 lanes, one row each, do not meet.  The copies in device memory that
+// are read as whole tiles (the weights) have it built in.
+template <int KC> __host__ __device__ inline int tile_slot(int r, int v)
+{
+    return KC == 64 ? (v ^ ((r >> 1) & 7)) : (v ^ ((r >> 2) & 3));
+}
+
+// ============================================================ forward and grad_input
+//   D[n, m] = sum_{step} B[step][n][KC] * A[source_row(m, tap of the step)][chunk of the step][KC]
+// One workgroup = 128 rows m x NT columns n, four wavefronts; a step is one tap and KC channels.  Both tiles of a step
+// go to LDS by DMA (1 KiB requests; a lane's 16 bytes come from the row its position and tap name), NST stages deep;
+// the source rows of a tap are worked out once by the lanes of the wavefront that fetches them and handed round by
+// permutes.  Steps are tap-major, so that happens once per tap.
+// What bounds it: with 32 columns the row requests (64 bytes per clock and compute unit: every position's row once
+// per tap), with 128 the matrix instructions and the requests alike (32 KiB and 512 matrix clocks per step).
+struct ConvRowsArgs {
+    RowMap map;
+    const unsigned char *src;         // rows of `rowb` bytes, then a row of zeros at byte `zrow`
+    const unsigned char *wt;          // [step][column tile][NT][KC] bfloat16, slots swizzled
+    const bf16_t *bias;               // or NULL
+    bf16_t *out;                      // [N][C][P], or NULL: partial sums
+    float *part;                      // [split][C][N * P]
+    unsigned rowb, zrow;
+    int C;                            // columns that exist
+    int nchunk, S;                    // KC-channel chunks per row, steps
+    int ntile, nctile, nsplit;
+};
+
+template <int NT, int KC>
+__global__ void __launch_bounds__(kThreads, 2) conv_rows_kernel(ConvRowsArgs a)
+{
+    constexpr int WO = NT == 128 ? 2 : 1, WP = 4 / WO;     // wavefronts along columns / rows
+    constexpr int OB = NT / 32 / WO, PB = kMT / 32 / WP;   // 32-blocks of a wavefront
+    constexpr int ROWB = KC * 2, RPD = 1024 / ROWB, VPR = ROWB / 16;
+    constexpr int ABYTES = kMT * ROWB, BBYTES = NT * ROWB, STAGE = ABYTES + BBYTES;
+    constexpr int NST = STAGE > 24 * 1024 ? 2 : 3;
+    constexpr int AD = ABYTES / 4096;                      // DMA requests per wavefront and step: rows,
+    constexpr int BD = (BBYTES + 4095) / 4096;             // ... weights (2 KiB of them: the first two wavefronts)
+    constexpr int NKG = KC / 16;
+    __shared__ __align__(1024) unsigned char s_t[NST * STAGE];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int id = xcd_swizzle(blockIdx.x, gridDim.x);
+    const int ct = id % a.nctile; id /= a.nctile;
+    const int split = id % a.nsplit, tile = id / a.nsplit;
+    const int st_lo = (int)((long)a.S * split / a.nsplit), st_hi = (int)((long)a.S * (split + 1) / a.nsplit);
+    const int m0 = tile * kMT;
+
+    // --- rows this wavefront fetches: wave * 32 + (0 .. 31), lane l works out row l & 31
+    const RowPos rp = row_pos(a.map, m0 + wave * 32 + (lane & 31));
+    const int lrow = lane / VPR, lslot = lane % VPR;       // this lane's row within a request, its 16-byte slot
+    unsigned aoff[AD], ainc[AD];
+    int chunk = st_lo % a.nchunk, tap = st_lo / a.nchunk;
+    auto tap_rows = [&](int k, int j) {
+        const int kx = k % a.map.g.kw, ky = (k / a.map.g.kw) % a.map.g.kh, kz = k / (a.map.g.kw * a.map.g.kh);
+        const int row = source_row(a.map, rp, kz, ky, kx);
+#pragma unroll
+        for (int i = 0; i < AD; i++) {
+            const int rl = i * RPD + lrow;                  // row of this request and lane, 0 .. 31
+            const int sr = __builtin_amdgcn_ds_bpermute(rl << 2, row);
+            const unsigned vb = (unsigned)tile_slot<KC>(rl, lslot) * 16u;    // (wave * 32 is a multiple of the pattern)
+            aoff[i] = sr >= 0 ? (unsigned)sr * a.rowb + (unsigned)j * ROWB + vb : a.zrow + vb;
+            ainc[i] = sr >= 0 ? ROWB : 0u;
+        }
+    };
+    static_assert(AD * RPD == 32, "a wavefront fetches 32 rows per step");
+    const unsigned char *bsrc = a.wt + ((long)st_lo * a.nctile + ct) * BBYTES + (wave % (BBYTES >= 4096 ? 4 : BBYTES / 1024)) * 1024 + lane * 16;
+    const long bstep = (long)a.nctile * BBYTES;
+    auto issue = [&](int buf) {
+        unsigned char *sa = s_t + buf * STAGE + wave * (32 * ROWB), *sb = s_t + buf * STAGE + ABYTES;
+#pragma unroll
+        for (int i = 0; i < AD; i++) {
+            dma16(a.src + aoff[i], sa + i * 1024);
+            aoff[i] += ainc[i];
+        }
+#pragma unroll
+        for (int i = 0; i < BD; i++) {
+            // (fewer than four pieces: wavefronts fetch the same one twice, which keeps the counts equal)
+            const int piece = BBYTES >= 4096 ? i * 4 + wave : wave % (BBYTES / 1024);
+            dma16(bsrc + (BBYTES >= 4096 ? i * 4096 : 0), sb + piece * 1024);
+        }
+        bsrc += bstep;
+        if (++chunk == a.nchunk) {
+            chunk = 0; tap++;
+            if (tap * a.nchunk < st_hi) tap_rows(tap, 0);
+        }
+    };
+
+    f32x16 acc[OB][PB];
+#pragma unroll
+    for (int ob = 0; ob < OB; ob++)
+#pragma unroll
+        for (int pb = 0; pb < PB; pb++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[ob][pb][r] = 0.f;
+    const int wo = wave % WO, wp = wave / WO;
+    // byte offsets of this lane's operand vectors of k-group 0 .. NKG-1 within a tile (blocks of 32 rows repeat them)
+    unsigned slot[NKG];
+#pragma unroll
+    for (int kg = 0; kg < NKG; kg++)
+        slot[kg] = (unsigned)((lane & 31) * ROWB + tile_slot<KC>(lane & 31, kg * 2 + (lane >> 5)) * 16);
+    const unsigned ra = lds_address(s_t) + wp * PB * 32 * ROWB, rb = lds_address(s_t) + ABYTES + wo * OB * 32 * ROWB;
+
+    tap_rows(tap, chunk);
+    issue(0);
+    if (NST == 3 && st_lo + 1 < st_hi) issue(1);
+    int buf = 0, nbuf = NST - 1;
+    for (int st = st_lo; st < st_hi; st++) {
+        if (NST == 3 && st + 1 < st_hi) wait_vm<AD + BD>(); else wait_vm<0>();
+        group_barrier();
+        if (st + NST - 1 < st_hi) issue(nbuf);
+        const unsigned pa = ra + buf * STAGE, pb_ = rb + buf * STAGE;
+        u32x4_t fa[2][PB], fb[2][OB];
+        auto fetch = [&](int kg, int s) {
+#pragma unroll
+            for (int ob = 0; ob < OB; ob++) fb[s][ob] = lds_read16(pb_ + slot[kg] + ob * 32 * ROWB);
+#pragma unroll
+            for (int pb = 0; pb < PB; pb++) fa[s][pb] = lds_read16(pa + slot[kg] + pb * 32 * ROWB);
+        };
+        fetch(0, 0);
+#pragma unroll
+        for (int kg = 0; kg < NKG; kg++) {
+            const int s = kg & 1;
+            if (kg + 1 < NKG) fetch(kg + 1, s ^ 1);
+#pragma unroll
+            for (int ob = 0; ob < OB; ob++) { if (kg + 1 < NKG) wait_lds<OB + PB>(fb[s][ob]); else wait_lds<0>(fb[s][ob]); }
+#pragma unroll
+            for (int pb = 0; pb < PB; pb++) { if (kg + 1 < NKG) wait_lds<OB + PB>(fa[s][pb]); else wait_lds<0>(fa[s][pb]); }
+#pragma unroll
+            for (int ob = 0; ob < OB; ob++)
+#pragma unroll
+                for (int pb = 0; pb < PB; pb++)
+                    mma_kgroup<bf16_t, false>(acc[ob][pb], __builtin_bit_cast(uint4, fb[s][ob]), __builtin_bit_cast(uint4, fa[s][pb]));
+        }
+        buf = buf + 1 == NST ? 0 : buf + 1;
+        nbuf = nbuf + 1 == NST ? 0 : nbuf + 1;
+    }
+
+    const int M = a.map.N * a.map.P;
+#pragma unroll
+    for (int pb = 0; pb < PB; pb++) {
+        const int m = m0 + (wp * PB + pb) * 32 + (lane & 31);
+        if (m >= M) continue;
+        const int b = fdiv(m, a.map.dP), p = m - b * a.map.P;
+#pragma unroll
+        for (int ob = 0; ob < OB; ob++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int n = ct * NT + (wo * OB + ob) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                if (n >= a.C) continue;
+                if (a.out)
+                    a.out[((long)b * a.C + n) * a.map.P + p] =
+                        f32_to_bf16(acc[ob][pb][r] + (a.bias ? bf16_to_f32(a.bias[n]) : 0.f));
+                else a.part[((long)split * a.C + n) * M + m] = acc[ob][pb][r];
+            }
+    }
+}
+
+// out[b][n][p] = bias[n] + the partial sums of (n, b * P + p)
+__global__ void __launch_bounds__(256) conv_rows_finish_kernel(const float *part, const bf16_t *bias, bf16_t *out, int nsplit,
+                                                               int C, int P, FastDiv dP, int M)
+{
+    const int m = blockIdx.x * 256 + threadIdx.x, n = blockIdx.y;
+    if (m >= M) return;
+    float v = bias ? bf16_to_f32(bias[n]) : 0.f;
+    const float *q = part + (long)n * M + m;
+    for (int s = 0; s < nsplit; s++) v += q[(long)s * C * M];
+    const int b = fdiv(m, dP), p = m - b * P;
+    out[((long)b * C + n) * P + p] = f32_to_bf16(v);
+}
+
+// ============================================================ grad_weight
+// One workgroup = one tap, 128 input channels, 32 * OBT output channels, over its share of the 64-position tiles.  A
+// step brings 64 input rows of 256 bytes and the grad_out fragments of 64 positions to LDS by DMA; the rows are read
+// with the transposing LDS load (the reduction runs over positions).  Wavefronts share the step: WO along the output
+// channels, 4 / WO along the input channels.  Bound by the requests (20 - 32 KiB per step and 128 - 512 matrix clocks).
+struct ConvWeightArgs {
+    RowMap map;                       // forward map
+    const unsigned char *src;         // channels-last input, rows of `rowb` bytes, a row of zeros at `zrow`
+    const uint4 *gp;                  // grad_out fragments [tile of 64][row block of 32][k-group][lane]
+    float *part;                      // [split][tap][128-channel block][C][128]
+    unsigned rowb, zrow;
+    int C, OBP;                       // output channels; row blocks of the fragment copy
+    int ncb, K, notile, nsplit, ntile;
+    int half_last;                    // the last block of 128 channels has 64 only
+};
+
+template <int OBT>
+__global__ void __launch_bounds__(kThreads, 2) conv_weight_kernel(ConvWeightArgs a)
+{
+    constexpr int WO = OBT == 4 ? 2 : 1;
+    constexpr int OB = OBT / WO, CB = WO;                  // 32-blocks of a wavefront: output / input channels
+    constexpr int XB = kCW * 256, GB = OBT * 4096, STAGE = XB + GB;
+    constexpr int NST = STAGE > 24 * 1024 ? 2 : 3;
+    constexpr int XD = 4, GD = OBT;
+    __shared__ __align__(1024) unsigned char s_t[NST * STAGE];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int id = xcd_swizzle(blockIdx.x, gridDim.x);
+    // (neighbouring workgroups: the taps of one channel block and share of positions, whose rows overlap)
+    const int ot = id % a.notile; id /= a.notile;
+    const int k = id % a.K; id /= a.K;
+    const int split = id % a.nsplit, cb = id / a.nsplit;
+    const int t_lo = (int)((long)a.ntile * split / a.nsplit), t_hi = (int)((long)a.ntile * (split + 1) / a.nsplit);
+    const int kx = k % a.map.g.kw, ky = (k / a.map.g.kw) % a.map.g.kh, kz = k / (a.map.g.kw * a.map.g.kh);
+
+    // rows of a request: 4 x 256 bytes; wavefront w fetches rows 16 w .. 16 w + 15
+    const int lrow = lane >> 4, lslot = lane & 15;
+    const bool cut = a.half_last && cb == a.ncb - 1;
+    auto issue = [&](int t, int buf) {
+        const RowPos rp = row_pos(a.map, t * kCW + wave * 16 + (lane & 15));
+        const int row = source_row(a.map, rp, kz, ky, kx);
+        unsigned char *sx = s_t + buf * STAGE + wave * 4096, *sg = s_t + buf * STAGE + XB;
+#pragma unroll
+        for (int i = 0; i < XD; i++) {
+            const int rl = i * 4 + lrow;
+            const int sr = __builtin_amdgcn_ds_bpermute(rl << 2, row);
+            const int v = lslot ^ ((rl & 3) << 2);         // channel vector of this slot, see the reads below
+            const bool ok = sr >= 0 && !(cut && v >= 8);
+            const unsigned o = ok ? (unsigned)sr * a.rowb + (unsigned)(cb * 256 + v * 16) : a.zrow + (unsigned)(v & 7) * 16u;
+            dma16(a.src + o, sx + i * 1024);
+        }
+        const unsigned char *g = reinterpret_cast<const unsigned char *>(a.gp) +
+                                 ((long)t * a.OBP + ot * OBT) * 4096 + wave * 1024 + lane * 16;
+#pragma unroll
+        for (int i = 0; i < GD; i++) dma16(g + i * 4096, sg + i * 4096 + wave * 1024);
+    };
+
+    f32x16 acc[OB][CB];
+#pragma unroll
+    for (int ob = 0; ob < OB; ob++)
+#pragma unroll
+        for (int c = 0; c < CB; c++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[ob][c][r] = 0.f;
+    const int wo = wave % WO, wc = wave / WO;
+    // transposing reads: lane -> position (g16 >> 1) * 8 + (l16 >> 2), channel block + (g16 & 1) * 16 + (l16 & 3) * 4;
+    // the 64-byte segments of four consecutive rows lie in different quarters of the banks
+    const int l16 = lane & 15, g16 = lane >> 4;
+    const int prow = (g16 >> 1) * 8 + (l16 >> 2);
+    unsigned xo[CB];
+#pragma unroll
+    for (int c = 0; c < CB; c++)
+        xo[c] = lds_address(s_t) + prow * 256 + (((wc * CB + c) ^ (prow & 3)) * 64) + (g16 & 1) * 32 + (l16 & 3) * 8;
+    const unsigned go = lds_address(s_t) + XB + wo * OB * 4096 + lane * 16;
+    typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
+
+    if (t_lo < t_hi) {
+        issue(t_lo, 0);
+        if (NST == 3 && t_lo + 1 < t_hi) issue(t_lo + 1, 1);
+    }
+    int buf = 0, nbuf = NST - 1;
+    for (int t = t_lo; t < t_hi; t++) {
+        if (NST == 3 && t + 1 < t_hi) wait_vm<XD + GD>(); else wait_vm<0>();
+        group_barrier();
+        if (t + NST - 1 < t_hi) issue(t + NST - 1, nbuf);
+        const unsigned bo = buf * STAGE;
+#pragma unroll
+        for (int kg = 0; kg < 4; kg++) {
+            u32x4_t fg[OB];
+            u32x2_t lo[CB], hi[CB];
+#pragma unroll
+            for (int ob = 0; ob < OB; ob++) fg[ob] = lds_read16(go + bo + ob * 4096 + kg * 1024);
+#pragma unroll
+            for (int c = 0; c < CB; c++) {
+                asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(lo[c]) : "v"(xo[c] + bo + kg * 4096));
+                asm volatile("ds_read_b64_tr_b16 %0, %1 offset:1024" : "=v"(hi[c]) : "v"(xo[c] + bo + kg * 4096));
+            }
+#pragma unroll
+            for (int ob = 0; ob < OB; ob++) wait_lds<0>(fg[ob]);
+#pragma unroll
+            for (int c = 0; c < CB; c++) asm volatile("" : "+v"(lo[c]), "+v"(hi[c]));
+#pragma unroll
+            for (int ob = 0; ob < OB; ob++)
+#pragma unroll
+                for (int c = 0; c < CB; c++)
+                    mma_kgroup<bf16_t, false>(acc[ob][c], __builtin_bit_cast(uint4, fg[ob]),
+                                              make_uint4(lo[c].x, lo[c].y, hi[c].x, hi[c].y));
+        }
+        buf = buf + 1 == NST ? 0 : buf + 1;
+        nbuf = nbuf + 1 == NST ? 0 : nbuf + 1;
+    }
+    float *part = a.part + (((long)split * a.K + k) * a.ncb + cb) * a.C * 128;
+#pragma unroll
+    for (int ob = 0; ob < OB; ob++)
+#pragma unroll
+        for (int c = 0; c < CB; c++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int o = (ot * OBT + wo * OB + ob) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                if (o < a.C) part[(long)o * 128 + (wc * CB + c) * 32 + (lane & 31)] = acc[ob][c][r];
+            }
+}
+
+// partial sums -> gW[o][c][tap]: a workgroup takes one output channel and one block of 128 input channels, through LDS
+// (the sums of a tap are rows of channels, grad_weight has the taps of a channel side by side)
+constexpr int kFinishTaps = 64;       // taps per round
+__global__ void __launch_bounds__(256) conv_weight_finish_kernel(const float *part, bf16_t *gw, int nsplit, int K, int ncb, int C,
+                                                                 int Cin)
+{
+    __shared__ bf16_t t[128 * (kFinishTaps + 1)];
+    const int cb = blockIdx.x % ncb, o = blockIdx.x / ncb;
+    const int nc = min(128, Cin - cb * 128);
+    const long sstr = (long)K * ncb * C * 128;
+    for (int k0 = 0; k0 < K; k0 += kFinishTaps) {
+        const int nk = min(kFinishTaps, K - k0);
+        for (int i = threadIdx.x; i < nk * 128; i += 256) {
+            const int c = i & 127, k = i >> 7;
+            const float *q = part + (((long)(k0 + k) * ncb + cb) * C + o) * 128 + c;
+            float v = 0.f;
+            for (int s = 0; s < nsplit; s++) v += q[s * sstr];
+            t[c * nk + k] = f32_to_bf16(v);
+        }
+        __syncthreads();
+        bf16_t *d = gw + ((long)o * Cin + cb * 128) * K + k0;
+        if (nk == K) {
+            for (int i = threadIdx.x; i < nc * nk; i += 256) d[i] = t[i];
+        } else {
+            for (int i = threadIdx.x; i < nc * nk; i += 256) d[(long)(i / nk) * K + i % nk] = t[i];
+        }
+        __syncthreads();
+    }
+}
+
+// ============================================================ operand orders, one launch per direction
+struct ConvPrepArgs {
+    // input -> channels-last rows, then a row of zeros
+    const bf16_t *x;
+    bf16_t *xcl;
+    int C, vol, N, nbx, nby, nblk_x, wide;
+    // weights: column tiles [step][tile][NT][KC]; back: the transposed product (columns = input channels)
+    const bf16_t *w;
+    uint4 *wt;
+    int Cout, Cin, K, NT, KC, nchunk, nct, back, nblk_w;
+    long nvec;
+    // grad_out -> channels-last rows of Cp channels (+ a row of zeros) and fragments
+    const bf16_t *gout;
+    bf16_t *gcl;
+    uint4 *gp;
+    int Cp, OBP, P, M, ngt, ngc, nblk_g;
+    FastDiv dP;
+    // bias gradient
+    bf16_t *gb;
+    int nblk_b;
+};
+
+__global__ void __launch_bounds__(256) conv_prepare_kernel(ConvPrepArgs a)
+{
+    constexpr int RS = 66;            // LDS row stride in elements
+    __shared__ __align__(16) bf16_t s_t[64 * 72];
+    int b = blockIdx.x;
+    if (b < a.nblk_x) {
+        // 64 voxels x 64 channels
+        const int bx = b % a.nbx, by = (b / a.nbx) % a.nby, n = b / (a.nbx * a.nby);
+        const int v0 = bx * 64, c0 = by * 64;
+        const bf16_t *xb = a.x + (long)n * a.C * a.vol;
+        bf16_t *ob = a.xcl + (long)n * a.C * a.vol;
+        if (b == 0 && threadIdx.x < 128) reinterpret_cast<unsigned *>(a.xcl + (long)a.N * a.C * a.vol)[threadIdx.x] = 0u;
+        if (a.wide) {
+            for (int i = threadIdx.x; i < 512; i += 256) {
+                const int c = c0 + i / 8, v = v0 + (i % 8) * 8;
+                if (v < a.vol) {
+                    const uint4 q = *reinterpret_cast<const uint4 *>(xb + (long)c * a.vol + v);
+                    const unsigned u[4] = {q.x, q.y, q.z, q.w};
+                    bf16_t *t = s_t + ((i % 8) * 8) * RS + i / 8;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        t[(2 * e) * RS] = (bf16_t)(u[e] & 0xffffu);
+                        t[(2 * e + 1) * RS] = (bf16_t)(u[e] >> 16);
+                    }
+                }
+            }
+        } else {
+            for (int i = threadIdx.x; i < 4096; i += 256) {
+                const int c = i / 64, v = i % 64;
+                if (v0 + v < a.vol) s_t[v * RS + c] = xb[(long)(c0 + c) * a.vol + v0 + v];
+            }
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < 512; i += 256) {
+            const int v = v0 + i / 8, c = c0 + (i % 8) * 8;
+            if (v < a.vol) {
+                const unsigned *t = reinterpret_cast<const unsigned *>(s_t + (i / 8) * RS + (i % 8) * 8);
+                *reinterpret_cast<uint4 *>(ob + (long)v * a.C + c) = make_uint4(t[0], t[1], t[2], t[3]);
+            }
+        }
+        return;
+    }
+    b -= a.nblk_x;
+    if (b < a.nblk_w) {
+        // one 16-byte vector of the result per thread and turn, taps fastest (the runs of W)
+        const int R = a.back ? a.Cin : a.Cout;              // columns that exist
+        const int Rp = a.nct * a.NT, D = a.back ? a.Cout : a.Cin, VPR = a.KC / 8, nv = a.nchunk * VPR;
+        for (long i = (long)b * 256 + threadIdx.x; i < a.nvec; i += (long)a.nblk_w * 256) {
+            const int k = (int)(i % a.K);
+            long r = i / a.K;
+            int col, v;                                      // column, channel vector along the reduction
+            if (a.back) { col = (int)(r % Rp); v = (int)(r / Rp); }
+            else { v = (int)(r % nv); col = (int)(r / nv); }
+            alignas(16) bf16_t e[8];
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                const int d = v * 8 + q;
+                const bool ok = col < R && d < D;
+                const long src = a.back ? ((long)d * a.Cin + col) * a.K + k : ((long)col * a.Cin + d) * a.K + k;
+                e[q] = ok ? a.w[src] : (bf16_t)0;
+            }
+            const int ct = col / a.NT, cr = col % a.NT, j = v / VPR, vv = v % VPR;
+            const int slot = a.KC == 64 ? tile_slot<64>(cr, vv) : tile_slot<32>(cr, vv);
+            a.wt[((((long)k * a.nchunk + j) * a.nct + ct) * a.NT + cr) * VPR + slot] = *reinterpret_cast<const uint4 *>(e);
+        }
+        return;
+    }
+    b -= a.nblk_w;
+    if (b < a.nblk_g) {
+        // 64 positions x 64 channels of grad_out, into both orders
+        const int gt = b % a.ngt, gc = b / a.ngt;
+        constexpr int GS = 72;                               // [channel][position], 16-byte aligned rows
+        for (int i = threadIdx.x; i < 4096; i += 256) {
+            const int c = gc * 64 + i / 64, m = gt * 64 + i % 64;
+            bf16_t v = 0;
+            if (c < a.Cout && m < a.M) {
+                const int n = fdiv(m, a.dP), p = m - n * a.P;
+                v = a.gout[((long)n * a.Cout + c) * a.P + p];
+            }
+            s_t[(i / 64) * GS + i % 64] = v;
+        }
+        __syncthreads();
+        if (a.gp) {
+            for (int i = threadIdx.x; i < 512; i += 256) {
+                const int ln = i & 63, kg = (i >> 6) & 3, ob = i >> 8;
+                if (gc * 2 + ob < a.OBP)
+                    a.gp[(((long)gt * a.OBP + gc * 2 + ob) * 4 + kg) * 64 + ln] =
+                        *reinterpret_cast<const uint4 *>(s_t + (ob * 32 + (ln & 31)) * GS + kg * 16 + (ln >> 5) * 8);
+            }
+        }
+        if (a.gcl) {
+            if (b == 0 && threadIdx.x < 128) reinterpret_cast<unsigned *>(a.gcl + (long)a.M * a.Cp)[threadIdx.x] = 0u;
+            for (int i = threadIdx.x; i < 512; i += 256) {
+                const int m = gt * 64 + i / 8, c = (i % 8) * 8;
+                if (m < a.M && gc * 64 + c < a.Cp) {
+                    alignas(16) bf16_t e[8];
+#pragma unroll
+                    for (int q = 0; q < 8; q++) e[q] = s_t[(c + q) * GS + i / 8];
+                    *reinterpret_cast<uint4 *>(a.gcl + (long)m * a.Cp + gc * 64 + c) = *reinterpret_cast<const uint4 *>(e);
+                }
+            }
+        }
+        return;
+    }
+    b -= a.nblk_g;
+    if (b < a.nblk_b) bias_grad_body<bf16_t, 256>(a.gout, a.gb, a.N, a.Cout, a.P, b);
+}
+
+// ============================================================ host side
+struct RowsPlan {
+    int NT, KC, nchunk, nct, S, ntile, nsplit;
+    size_t wt_bytes, part_bytes;
+};
+// columns C, reduction over `depth` channels per tap, M rows
+RowsPlan rows_plan(int C, int depth, int K, int M, int ncu)
+{
+    RowsPlan p;
+    p.KC = depth <= 32 ? 32 : 64;
+    p.NT = C <= 32 ? 32 : (C <= 64 ? 64 : 128);
+    p.nchunk = (depth + p.KC - 1) / p.KC;
+    p.nct = (C + p.NT - 1) / p.NT;
+    p.S = K * p.nchunk;
+    p.ntile = (M + kMT - 1) / kMT;
+    // Steps shared out between `nsplit` workgroups where the tiles alone leave compute units idle.  Two workgroups run
+    // on a compute unit at a time; a piece costs its steps, about four more for its start and end, and its share of the
+    // partial sums, which are written and read once more each (about a step per 32 columns).
+    const long items = (long)p.ntile * p.nct, slots = 2L * ncu;
+    long best = -1;
+    p.nsplit = 1;
+    for (int s = 1; s <= 16 && s <= p.S; s++) {
+        const long rounds = (items * s + slots - 1) / slots;
+        const long cost = rounds * ((p.S + s - 1) / s + 4) + (s > 1 ? (items * s * (p.NT / 32) + slots - 1) / slots : 0);
+        if (best < 0 || cost * 20 < best * 19) { best = cost; p.nsplit = s; }
+    }
+    p.wt_bytes = d2c_align_up((size_t)p.S * p.nct * p.NT * p.KC * 2);
+    p.part_bytes = p.nsplit > 1 ? d2c_align_up((size_t)p.nsplit * C * M * sizeof(float)) : 0;
+    return p;
+}
+
+template <int NT, int KC> int launch_rows(const ConvRowsArgs &a, hipStream_t st)
+{
+    D2cProfScope prof(D2C_PROF_FWD, st, "conv_rows_kernel");
+    hipLaunchKernelGGL((conv_rows_kernel<NT, KC>), dim3((unsigned)(a.ntile * a.nsplit * a.nctile)), dim3(kThreads), 0, st, a);
+    return d2c_check_launch("conv_rows_kernel");
+}
+
+int run_rows(const RowsPlan &p, const RowMap &map, const void *src, unsigned rowb, unsigned zrow, const void *wt, const void *bias,
+             void *out, float *part, int C, hipStream_t st)
+{
+    ConvRowsArgs a{map, (const unsigned char *)src, (const unsigned char *)wt, p.nsplit > 1 ? nullptr : (const bf16_t *)bias,
+                   p.nsplit > 1 ? nullptr : (bf16_t *)out, part, rowb, zrow, C, p.nchunk, p.S, p.ntile, p.nct, p.nsplit};
+    int rc;
+    if (p.KC == 32) rc = p.NT == 32 ? launch_rows<32, 32>(a, st) : (p.NT == 64 ? launch_rows<64, 32>(a, st) : launch_rows<128, 32>(a, st));
+    else rc = p.NT == 32 ? launch_rows<32, 64>(a, st) : (p.NT == 64 ? launch_rows<64, 64>(a, st) : launch_rows<128, 64>(a, st));
+    if (rc || p.nsplit == 1) return rc;
+    const int M = map.N * map.P;
+    D2cProfScope prof(D2C_PROF_PACK, st);
+    hipLaunchKernelGGL(conv_rows_finish_kernel, dim3((M + 255) / 256, C), dim3(256), 0, st, part, (const bf16_t *)bias, (bf16_t *)out,
+                       p.nsplit, C, map.P, map.dP, M);
+    return d2c_check_launch("conv_rows_finish_kernel");
+}
+
+struct WeightPlan {
+    int obt, OBP, notile, ncb, ntile, nsplit;
+    size_t gp_bytes, part_bytes;
+};
+WeightPlan weight_plan(const d2c_conv3d_desc &q, int K, int ncu)
+{
+    WeightPlan p;
+    const int M = q.N * q.Do * q.Ho * q.Wo;
+    p.obt = q.Cout <= 32 ? 1 : (q.Cout <= 64 ? 2 : 4);
+    p.notile = (q.Cout + 32 * p.obt - 1) / (32 * p.obt);
+    p.OBP = p.notile * p.obt;
+    p.ncb = (q.Cin + 127) / 128;
+    p.ntile = (M + kCW - 1) / kCW;
+    const long items = (long)K * p.ncb * p.notile, slots = 2L * ncu;
+    long best = -1;
+    p.nsplit = 1;
+    for (int s = 1; s <= 16 && s <= p.ntile; s++) {
+        const long rounds = (items * s + slots - 1) / slots;
+        const long cost = rounds * ((p.ntile + s - 1) / s + 6) + (s > 1 ? (items * s * p.obt + slots - 1) / slots : 0);
+        if (best < 0 || cost * 20 < best * 19) { best = cost; p.nsplit = s; }
+    }
+    p.gp_bytes = d2c_align_up((size_t)p.ntile * p.OBP * 4096);
+    p.part_bytes = d2c_align_up((size_t)p.nsplit * K * p.ncb * q.Cout * 128 * sizeof(float));
+    return p;
+}
+
+inline int padded_channels(int c) { return c <= 32 ? 32 : (c + 63) / 64 * 64; }
+inline bool plain_shape_ok(const d2c_conv3d_desc &q)
+{
+    const size_t lim = (size_t)1 << 32, P = (size_t)q.Do * q.Ho * q.Wo;
+    return q.dtype == D2C_BF16 && q.groups == 1 && q.Cin % 64 == 0 &&
+           (size_t)q.N * q.Cin * q.D * q.H * q.W * 2 + 1024 < lim && (size_t)q.N * padded_channels(q.Cout) * P * 2 + 1024 < lim &&
+           (size_t)q.N * P < (1u << 30) && (size_t)q.N * q.D * q.H * q.W < (1u << 30);
+}
+inline int weight_blocks(long nvec) { return (int)std::min<long>((nvec + 255) / 256, 4096); }
+
+}  // namespace
+
+bool d2c_plain_supported(const d2c_conv3d_desc &q) { return plain_shape_ok(q); }
+size_t d2c_plain_input_bytes(const d2c_conv3d_desc &q) { return (size_t)q.N * q.Cin * q.D * q.H * q.W * 2 + 1024; }
+
+size_t d2c_plain_forward_ws(const d2c_conv3d_desc &q)
+{
+    const int K = q.kd * q.kh * q.kw, ncu = d2c_num_cus();
+    if (ncu <= 0) return 0;
+    const RowsPlan p = rows_plan(q.Cout, q.Cin, K, q.N * q.Do * q.Ho * q.Wo, ncu);
+    return p.wt_bytes + p.part_bytes;
+}
+
+int d2c_plain_forward(const d2c_conv3d_desc &q, const void *x, const void *w, const void *bias, void *out, void *xcl, void *ws,
+                      hipStream_t st)
+{
+    const int K = q.kd * q.kh * q.kw, ncu = d2c_num_cus(), vol = q.D * q.H * q.W;
+    if (ncu <= 0) return D2C_ERR_LAUNCH;
+    const RowsPlan p = rows_plan(q.Cout, q.Cin, K, q.N * q.Do * q.Ho * q.Wo, ncu);
+    char *base = (char *)ws;
+    {
+        ConvPrepArgs a{};
+        a.x = (const bf16_t *)x; a.xcl = (bf16_t *)xcl; a.C = q.Cin; a.vol = vol; a.N = q.N;
+        a.nbx = (vol + 63) / 64; a.nby = q.Cin / 64; a.nblk_x = a.nbx * a.nby * q.N;
+        a.wide = vol % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+        a.w = (const bf16_t *)w; a.wt = (uint4 *)base; a.Cout = q.Cout; a.Cin = q.Cin; a.K = K;
+        a.NT = p.NT; a.KC = p.KC; a.nchunk = p.nchunk; a.nct = p.nct; a.back = 0;
+        a.nvec = (long)p.nct * p.NT * p.nchunk * (p.KC / 8) * K;
+        a.nblk_w = weight_blocks(a.nvec);
+        D2cProfScope prof(D2C_PROF_PACK, st);
+        hipLaunchKernelGGL(conv_prepare_kernel, dim3((unsigned)(a.nblk_x + a.nblk_w)), dim3(256), 0, st, a);
+        if (int rc = d2c_check_launch("conv_prepare_kernel")) return rc;
+    }
+    return run_rows(p, row_map(q, false), xcl, (unsigned)q.Cin * 2u, (unsigned)((size_t)q.N * q.Cin * vol * 2), base, bias, out,
+                    (float *)(base + p.wt_bytes), q.Cout, st);
+}
+
+namespace {
+struct PlainBwdWs {
+    size_t gcl, gp, wt, part, total;
+};
+PlainBwdWs plain_bwd_ws(const d2c_conv3d_desc &q, const RowsPlan &r, const WeightPlan &w)
+{
+    PlainBwdWs l;
+    l.gcl = 0;
+    l.gp = d2c_align_up((size_t)q.N * q.Do * q.Ho * q.Wo * padded_channels(q.Cout) * 2 + 1024);
+    l.wt = l.gp + w.gp_bytes;
+    l.part = l.wt + r.wt_bytes;
+    // (grad_input's partial sums are done with before grad_weight's are written)
+    l.total = l.part + std::max(r.part_bytes, w.part_bytes);
+    return l;
+}
+}  // namespace
+
+size_t d2c_plain_backward_ws(const d2c_conv3d_desc &q)
+{
+    const int K = q.kd * q.kh * q.kw, ncu = d2c_num_cus();
+    if (ncu <= 0) return 0;
+    return plain_bwd_ws(q, rows_plan(q.Cin, padded_channels(q.Cout), K, q.N * q.D * q.H * q.W, ncu), weight_plan(q, K, ncu)).total;
+}
+
+int d2c_plain_backward(const d2c_conv3d_desc &q, const void *gout, const void *xcl, const void *w, void *gx, void *gw, void *gb,
+                       void *ws, hipStream_t st)
+{
+    const int K = q.kd * q.kh * q.kw, ncu = d2c_num_cus(), vol = q.D * q.H * q.W, P = q.Do * q.Ho * q.Wo, M = q.N * P;
+    if (ncu <= 0) return D2C_ERR_LAUNCH;
+    if (!gx && !gw && !gb) return D2C_OK;
+    const int Cp = padded_channels(q.Cout);
+    const RowsPlan r = rows_plan(q.Cin, Cp, K, q.N * vol, ncu);
+    const WeightPlan p = weight_plan(q, K, ncu);
+    const PlainBwdWs l = plain_bwd_ws(q, r, p);
+    char *base = (char *)ws;
+    {
+        ConvPrepArgs a{};
+        a.w = (const bf16_t *)w; a.wt = (uint4 *)(base + l.wt); a.Cout = q.Cout; a.Cin = q.Cin; a.K = K;
+        a.NT = r.NT; a.KC = r.KC; a.nchunk = r.nchunk; a.nct = r.nct; a.back = 1; a.N = q.N;
+        a.nvec = (long)r.nct * r.NT * r.nchunk * (r.KC / 8) * K;
+        a.nblk_w = gx ? weight_blocks(a.nvec) : 0;
+        a.gout = (const bf16_t *)gout;
+        a.gcl = gx ? (bf16_t *)(base + l.gcl) : nullptr;
+        a.gp = gw ? (uint4 *)(base + l.gp) : nullptr;
+        a.Cp = Cp; a.OBP = p.OBP; a.P = P; a.M = M; a.dP = make_fastdiv(P);
+        a.ngt = (M + 63) / 64;
+        a.ngc = std::max((Cp + 63) / 64, (p.OBP + 1) / 2);
+        a.nblk_g = (gx || gw) ? a.ngt * a.ngc : 0;
+        a.gb = (bf16_t *)gb;
+        a.nblk_b = gb ? q.Cout : 0;
+        D2cProfScope prof(D2C_PROF_PACK, st);
+        hipLaunchKernelGGL(conv_prepare_kernel, dim3((unsigned)(a.nblk_w + a.nblk_g + a.nblk_b)), dim3(256), 0, st, a);
+        if (int rc = d2c_check_launch("conv_prepare_kernel")) return rc;
+    }
+    if (gx) {
+        if (int rc = run_rows(r, row_map(q, true), base + l.gcl, (unsigned)Cp * 2u, (unsigned)((size_t)M * Cp * 2), base + l.wt, nullptr,
+                              gx, (float *)(base + l.part), q.Cin, st))
+            return rc;
+    }
+    if (gw) {
+        ConvWeightArgs a{row_map(q, false), (const unsigned char *)xcl, (const uint4 *)(base + l.gp), (float *)(base + l.part),
+                         (unsigned)q.Cin * 2u, (unsigned)((size_t)q.N * q.Cin * vol * 2), q.Cout, p.OBP, p.ncb, K, p.notile,
+                         p.nsplit, p.ntile, q.Cin % 128 != 0};
+        const dim3 grid((unsigned)((long)K * p.ncb * p.notile * p.nsplit));
+        {
+            D2cProfScope prof(D2C_PROF_BWD_WEIGHT, st, "conv_weight_kernel");
+            if (p.obt == 1) hipLaunchKernelGGL(conv_weight_kernel<1>, grid, dim3(kThreads), 0, st, a);
+            else if (p.obt == 2) hipLaunchKernelGGL(conv_weight_kernel<2>, grid, dim3(kThreads), 0, st, a);
+            else hipLaunchKernelGGL(conv_weight_kernel<4>, grid, dim3(kThreads), 0, st, a);
+            if (int rc = d2c_check_launch("conv_weight_kernel")) return rc;
+        }
+        D2cProfScope prof(D2C_PROF_PACK, st);
+        hipLaunchKernelGGL(conv_weight_finish_kernel, dim3((unsigned)(q.Cout * p.ncb)), dim3(256), 0, st, (const float *)a.part,
+                           (bf16_t *)gw, p.nsplit, K, p.ncb, q.Cout, q.Cin);
+        return d2c_check_launch("conv_weight_finish_kernel");
+    }
+    return D2C_OK;
+}

@@ -44,3 +44,13 @@ int d2c_tiled1d_forward(const d2c_conv1d_desc &q, const void *x, const void *off
 int d2c_tiled1d_backward(const d2c_conv1d_desc &q, const void *gout, const void *x, const void *off,
                          const void *mask, const void *w, void *gx, void *goff, void *gmask, void *gw, void *gb,
                          void *ws, hipStream_t st);
+
+// The ordinary convolution of a deformation branch (d2c_conv.hip).
+bool d2c_plain_supported(const d2c_conv3d_desc &q);
+size_t d2c_plain_input_bytes(const d2c_conv3d_desc &q);
+size_t d2c_plain_forward_ws(const d2c_conv3d_desc &q);
+size_t d2c_plain_backward_ws(const d2c_conv3d_desc &q);
+int d2c_plain_forward(const d2c_conv3d_desc &q, const void *x, const void *w, const void *bias, void *out, void *xcl, void *ws,
+                      hipStream_t st);
+int d2c_plain_backward(const d2c_conv3d_desc &q, const void *gout, const void *xcl, const void *w, void *gx, void *gw, void *gb,
+                       void *ws, hipStream_t st);

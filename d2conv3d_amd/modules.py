@@ -72,6 +72,9 @@ def _branch_conv(layer, x):
         from .deform_conv import deform_conv3d
         k, s, p, d = conv.kernel_size, conv.stride, conv.padding, conv.dilation
         dims = tuple((x.shape[2 + i] + 2 * p[i] - d[i] * (k[i] - 1) - 1) // s[i] + 1 for i in range(3))
+        if (min(dims) > 0 and x.dtype == torch.bfloat16 and (conv.bias is None or conv.bias.dtype == x.dtype)
+                and _ops.plain_conv3d_supported(x, conv.weight, s, p, d)):
+            return _ops.plain_conv3d(x, conv.weight, conv.bias, s, p, d)
         if min(dims) > 0:
             off0 = _zero_offsets(x.device, x.shape[0], 3 * k[0] * k[1] * k[2], dims)
             if _ops.conv3d_algo(x, off0, None, conv.weight, s, p, d, 1, 1) == "mfma":

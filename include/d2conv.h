@@ -247,6 +247,23 @@ int d2c_conv3d_backward_prepared(const d2c_conv3d_desc *desc, const void *grad_o
                                  void *prepared, size_t prepared_bytes, int32_t reuse, void *workspace,
                                  size_t workspace_bytes, void *stream);
 
+/*
+ * The ordinary convolution (no sampling points) of a layer's deformation branch, `deform_params`
+ * (network/layers.py:66-68): bfloat16, one weight group, input channels a multiple of 64.  The description's offset
+ * fields and epilogue are ignored.  d2c_plain_conv3d_input_bytes() is 0 for descriptions it does not serve; else the
+ * forward call leaves the input's channels-last copy in a caller's buffer of that size (256-byte aligned), which the
+ * backward call takes in place of the input.
+ */
+size_t d2c_plain_conv3d_input_bytes(const d2c_conv3d_desc *desc);
+size_t d2c_plain_conv3d_forward_workspace_bytes(const d2c_conv3d_desc *desc);
+size_t d2c_plain_conv3d_backward_workspace_bytes(const d2c_conv3d_desc *desc);
+int d2c_plain_conv3d_forward(const d2c_conv3d_desc *desc, const void *x, const void *weight, const void *bias, void *out,
+                             void *input_copy, size_t input_copy_bytes, void *workspace, size_t workspace_bytes,
+                             void *stream);
+int d2c_plain_conv3d_backward(const d2c_conv3d_desc *desc, const void *grad_out, const void *input_copy,
+                              size_t input_copy_bytes, const void *weight, void *grad_x, void *grad_weight,
+                              void *grad_bias, void *workspace, size_t workspace_bytes, void *stream);
+
 int d2c_conv1d_check(const d2c_conv1d_desc *desc);
 int d2c_conv1d_algo(const d2c_conv1d_desc *desc);   /* D2C_ALGO_GENERIC or D2C_ALGO_MFMA */
 size_t d2c_conv1d_forward_workspace_bytes(const d2c_conv1d_desc *desc);
