@@ -1,0 +1,666 @@
+// Offset / mask gradient and grad_input of a three-dimensional problem as dense matrix products over bricks of the
+// input volume (dconv3d_gpu.cu:562-643, :708-864 in another formulation).
+//
+// A sampling point reaches the 2 x 2 x 2 voxels above its base voxel floor(z, y, x).  All points whose base voxel
+// lies in a block of 1 x 3 x 3 voxels reach the same brick of 2 x 4 x 4 = 32 voxels.  With the points sorted by block
+//
+//   T[v, s]   = x[v, :] . gcol[s, :]           32 voxels x 32 points x channels: one matrix product; a point's eight
+//                                              corner dots are among its 32, and grad_offset / grad_mask follow
+//   gx[v, :] += W[v, s] * gcol[s, :]           W = the points' corner weights times modulation, zero off the corners
+//
+// Three quarters of the products are with zeros, on matrix cores that have them to spare; in exchange nothing is
+// gathered: a grad-column row is read once, for both results, and a brick's input rows stay in LDS.  (The kernels
+// that gather -- eight corner rows per point through the L1, grad-column rows 3.4 times -- took 1.73 + 1.47 ms for
+// 256 channels on 32x60x108, bound by the L1 path, the vector ALU and row latency.)
+#include <utility>
+
+#include "d2c_mma.hpp"
+#include "d2c_tiled.hpp"
+#include "d2c_brick.hpp"
+
+namespace {
+
+typedef short v4s __attribute__((ext_vector_type(4)));
+
+template <class F, int... I> D2C_DEV void for_each_const(F &&f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+
+// One sampling point as the sort sees it.
+struct BrickPoint {
+    bool in;              // a corner is inside the volume
+    int seg;              // its block
+    float y, x, hz;       // place inside the block along y and x, fraction along z
+};
+D2C_DEV int brick_seg(const BrickDims &d, int bg, int zi, int by, int bx) { return ((bg * d.nz + zi) * d.nby + by) * d.nbx + bx; }
+// (`c`: what tap_offsets_issue() read)
+template <bool AUX16, bool SIZED>
+D2C_DEV BrickPoint brick_point(const TiledShape &s, const BrickDims &d, float *c, int b, int g, int k, int p)
+{
+    tap_offsets_finish<AUX16, SIZED>(s, k, c);
+    const int oz = fdiv(p, s.dHW), rem = p - oz * (s.Wo * s.Ho);
+    const int oy = fdiv(rem, s.dW), ox = rem - oy * s.Wo;
+    int bz, by, bx;
+    tap_base(s.geo, k, oz, oy, ox, bz, by, bx);
+    const Tap3<float> t = tiled_tap3(s, bz, by, bx, c[0], c[1], c[2]);
+    BrickPoint r;
+    r.in = t.inrange != 0;
+    const int yq = (t.y0 + 1) / 3, xq = (t.x0 + 1) / 3;       // (base voxels start at -1)
+    // (exact from position 4 on, where a fraction has at most 21 bits, and within 2^-23 of a voxel below)
+    // (and never rounded up to the next base voxel, where the derivative is another one)
+    const float yb = (float)(t.y0 + 1 - yq * 3), xb = (float)(t.x0 + 1 - xq * 3);
+    r.y = fminf(yb + t.hy, yb + (1.f - 0x1p-22f)); r.x = fminf(xb + t.hx, xb + (1.f - 0x1p-22f));
+    r.hz = t.hz;
+    r.seg = brick_seg(d, b * s.G + g, t.z0 + 1, yq, xq);
+    return r;
+}
+
+// ---- the sort: count the points of every block (a point remembers its place), give every block a range, file ------
+// A workgroup works on 256 positions and up to kTaps taps, and requests what it reads of all of them first.  Points of
+// neighbouring positions fall into few blocks: they are counted in a hash table in LDS, and each block's number goes to
+// the global count in one addition.  (One global atomic per point, taps in workgroups of their own: 0.24 ms for 5.6 M
+// points in 8 offset groups on 8x30x54.)
+// Workgroups of the passes over all points: an XCD takes a contiguous part of the positions, the tap groups of a block
+// of 256 one after the other, so that the lines which several workgroups write or read in parts meet in one L2.
+constexpr int kTaps = 9, kSlots = 4096;             // (more slots than a workgroup has points: a probe always ends)
+struct PointUnit {
+    int b, g, bg, k0, p;
+};
+D2C_DEV PointUnit point_unit(const TiledShape &s, int ngrp)
+{
+    const int nt = (int)gridDim.x, q = nt >> 3, r = nt & 7, xcd = blockIdx.x & 7;
+    const int u = xcd * q + (xcd < r ? xcd : r) + (int)(blockIdx.x >> 3);
+    const int npb = (s.P + 255) / 256, blk = u / ngrp;
+    PointUnit t;
+    t.bg = blk / npb; t.b = t.bg / s.G; t.g = t.bg - t.b * s.G;
+    t.k0 = (u - blk * ngrp) * kTaps; t.p = (blk - t.bg * npb) * 256 + threadIdx.x;
+    return t;
+}
+template <bool AUX16, bool SIZED>
+__global__ void __launch_bounds__(256)
+brick_count_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, int ngrp)
+{
+    __shared__ int s_key[kSlots], s_cnt[kSlots];
+    static_assert(kTaps * 256 < kSlots && kSlots <= 65536, "table size");
+    const PointUnit un = point_unit(s, ngrp);
+    const int k0 = un.k0, bg = un.bg, b = un.b, g = un.g, p = un.p, pl = min(p, s.P - 1);
+    float c[kTaps][3];
+#pragma unroll
+    for (int i = 0; i < kTaps; i++) tap_offsets_issue<AUX16, SIZED>(s, off, b, g, min(k0 + i, s.K - 1), pl, c[i]);
+    for (int i = threadIdx.x; i < kSlots; i += 256) { s_key[i] = -1; s_cnt[i] = 0; }
+    __syncthreads();
+    unsigned pt[kTaps];                              // slot << 16 | place among the workgroup's points there, or all ones
+#pragma unroll
+    for (int i = 0; i < kTaps; i++) {
+        pt[i] = ~0u;
+        if (p >= s.P || k0 + i >= s.K) continue;
+        const BrickPoint q = brick_point<AUX16, SIZED>(s, d, c[i], b, g, k0 + i, p);
+        if (!q.in) continue;
+        unsigned sl = ((unsigned)q.seg * 2654435761u) >> 20;
+        for (;;) {
+            const int old = atomicCAS(&s_key[sl], -1, q.seg);
+            if (old == -1 || old == q.seg) break;
+            sl = (sl + 1) & (kSlots - 1);
+        }
+        pt[i] = (sl << 16) | (unsigned)atomicAdd(&s_cnt[sl], 1);
+    }
+    __syncthreads();
+    // (through a buffer descriptor, an empty slot's addition past its end: no branch, so that all are on their way at once)
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc(L.count, 0, L.cursor - L.count > 0 ? (int)((L.cursor - L.count) * 4) : 0, 0x00020000);
+    int base[kSlots / 256];
+#pragma unroll
+    for (int i = 0; i < kSlots / 256; i++) {
+        const int key = s_key[i * 256 + threadIdx.x];
+        base[i] = __builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(s_cnt[i * 256 + threadIdx.x], rs, key >= 0 ? key * 4 : -16, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < kSlots / 256; i++) s_cnt[i * 256 + threadIdx.x] = base[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kTaps; i++)
+        if (p < s.P && k0 + i < s.K)
+            L.place[((long)bg * s.K + k0 + i) * s.P + p] = pt[i] == ~0u ? -1 : s_cnt[pt[i] >> 16] + (int)(pt[i] & 0xffffu);
+}
+// (the order of the ranges does not matter: a wavefront adds up its 64 counts and takes one range for all)
+__global__ void __launch_bounds__(256) brick_range_kernel(BrickLists L, int nseg)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63;
+    const int n = i < nseg ? L.count[i] : 0;
+    int sum = n;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int v = __shfl_up(sum, d, 64);
+        if (lane >= d) sum += v;
+    }
+    int base = 0;
+    if (lane == 63) base = atomicAdd(L.cursor, sum);
+    base = __shfl(base, 63, 64);
+    if (i < nseg) L.start[i] = base + sum - n;
+}
+// (all taps of a position in one workgroup: the places a workgroup's points were given in a block follow each other)
+template <bool AUX16, bool SIZED>
+__global__ void __launch_bounds__(256)
+brick_file_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, const void *mask, int ngrp)
+{
+    typedef typename std::conditional<AUX16, bf16_t, float>::type AT;
+    const PointUnit un = point_unit(s, ngrp);
+    const int k0 = un.k0, bg = un.bg, b = un.b, g = un.g, p = un.p;
+    if (p >= s.P) return;
+    int *place = L.place + ((long)bg * s.K + k0) * s.P + p;
+    float c[kTaps][3], al[kTaps];
+    int rank[kTaps], start[kTaps];
+    BrickPoint q[kTaps];
+#pragma unroll
+    for (int i = 0; i < kTaps; i++) {
+        const int k = min(k0 + i, s.K - 1);
+        rank[i] = k0 + i < s.K ? place[(long)i * s.P] : -1;
+        tap_offsets_issue<AUX16, SIZED>(s, off, b, g, k, p, c[i]);
+        al[i] = mask ? ld_auxT<AUX16>(mask, mask_index(s, b, g, k, p)) : 1.f;
+    }
+#pragma unroll
+    for (int i = 0; i < kTaps; i++) {
+        q[i] = brick_point<AUX16, SIZED>(s, d, c[i], b, g, min(k0 + i, s.K - 1), p);
+        start[i] = rank[i] >= 0 ? L.start[q[i].seg] : 0;
+    }
+#pragma unroll
+    for (int i = 0; i < kTaps; i++) {
+        if (rank[i] < 0) continue;
+        const int at = start[i] + rank[i];
+        place[(long)i * s.P] = at;
+        L.pt[at] = make_uint4((unsigned)((k0 + i) * s.M + b * s.P + p) * 128u, __float_as_uint(q[i].y), __float_as_uint(q[i].x),
+                              __float_as_uint(q[i].hz));
+        L.alpha[at] = (mask && s.mact) ? mask_act<AT>(s.mact, al[i]) : al[i];
+    }
+}
+
+// ---- the products -------------------------------------------------------------------------------------------------
+// A workgroup takes a column of bricks (one 3 x 3 block of base voxels along y and x, a range of z) and up to four chunks
+// of 64 channels, a wavefront each; all walk the same points, 32 at a time.  Going up in z, the upper plane of a brick is the
+// lower one of the next: a plane's input rows and its grad_input sums stay where they are (plane z in slot z & 1),
+// one plane is loaded and one is added to the accumulator per step.
+//
+// Matrix operands (v_mfma_f32_32x32x16_bf16):
+//   T:  A = x rows (lane = voxel), B = grad-column rows (lane = point), both from LDS
+//   gx: A = the weights, two bfloat16 terms, B = the rows, both through LDS (lane = point there, transposing reads)
+// Voxel m of the brick: plane slot m / 16, y (m / 4) % 4, x m % 4.  A lane of T holds point lane % 32 and, in
+// register r, voxel 8 * (r / 4) + 4 * (lane / 32) + r % 4: x = r % 4, slot = r / 8, y = 2 * ((r / 4) % 2) + lane / 32, so
+// that of a point's two corner rows along y each half of the wavefront holds one.
+struct BrickArgs {
+    BrickDims d;
+    BrickLists L;
+    const bf16_t *xcl;       // [N][vol][Cin]
+    const bf16_t *gcol;      // [chunk][tap][N*P][64]
+    float *gxcl;             // [N][vol][Cin] sums (cleared), or NULL
+    float2 *res;             // [set][point][2]: sum over its channels of (mask, x), (z, y) per unit of modulation; or NULL
+    long nres;               // points per set
+    int zlen, nzr;           // base planes per workgroup, ranges of them
+    int nset;                // sets of up to kMaxWaves chunks
+    int G, cpc, Cin, D, H, W, vol;
+    long chunk_rows;         // K * M
+};
+
+constexpr int kMaxWaves = 4;
+constexpr int kWaveLds = 32 * 128 + 2 * 32 * 64;
+D2C_DEV void lds_only_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+D2C_DEV void wave_fence() { asm volatile("" ::: "memory"); __builtin_amdgcn_wave_barrier(); }
+
+__global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs a, const int *__restrict__ seg_start, const int *__restrict__ seg_count)
+{
+#define INLINE __attribute__((always_inline))
+    const int lane = threadIdx.x & 63, h = lane >> 5, n = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+    // A wavefront's grad-column rows of 32 points x 64 channels, and their weights [term][point][voxel of 32].  16-byte pieces of a row are
+    // permuted so that neither the row-wise accesses (16 lanes on the same piece of 16 rows) nor the transposing reads
+    // (4 rows x 64 bytes) meet a bank twice.
+    extern __shared__ __align__(16) unsigned char smem[];
+    unsigned char *const s_g = smem + wave * kWaveLds, *const s_w = s_g + 32 * 128;
+    float2 *const s_part = reinterpret_cast<float2 *>(smem + nw * kWaveLds);       // [2][wave][lane]: sums over a chunk each
+    auto g_swz = [](int row) INLINE { return (((row >> 1) & 1) << 2) | (((row >> 2) & 1) << 1) | ((row >> 3) & 1); };
+
+    // task: set of chunks, then block column along x, y, then z range, group and sample; an XCD takes a contiguous part of them
+    const int nt = (int)gridDim.x, xq = nt >> 3, xr = nt & 7, xcd = blockIdx.x & 7;
+    int t = xcd * xq + (xcd < xr ? xcd : xr) + (int)(blockIdx.x >> 3);
+    const int set = t % a.nset; t /= a.nset;
+    const int bx = t % a.d.nbx; t /= a.d.nbx;
+    const int by = t % a.d.nby; t /= a.d.nby;
+    const int zr = t % a.nzr; const int bg = t / a.nzr;
+    const int b = bg / a.G, g = bg - b * a.G;
+    const bool here = set * nw + wave < a.cpc;                       // (the last set can be short: a wavefront that only keeps step)
+    const int cc0 = g * a.cpc + (here ? set * nw + wave : 0);        // its chunk
+    const bool want_gx = a.gxcl != nullptr && here;
+    const int res_bytes = a.res ? 16 : 0;
+    const int y0 = by * 3 - 1, x0 = bx * 3 - 1;
+    const int zi_lo = zr * a.zlen, zi_hi = min(zi_lo + a.zlen, a.d.nz);
+    constexpr unsigned kNone = 0xFFFFFFF0u;                          // an offset past every buffer: nothing is stored
+
+    f32x16 gacc[2];
+#pragma unroll
+    for (int r = 0; r < 16; r++) gacc[0][r] = gacc[1][r] = 0.f;
+
+    // input rows as the operand of T: lane = voxel n of the brick, its 8 channels of every k-step.  load_plane changes
+    // the lanes of slot z & 1 (zeros outside the volume).
+    u32x4_t xa[4];
+    auto load_plane = [&](int z) INLINE {
+        int fn = n;
+        opaque_v(fn);
+        if ((fn >> 4) != (z & 1)) return;
+        const int vox_y = y0 + ((fn >> 2) & 3), vox_x = x0 + (fn & 3);
+        const bool in = vox_y >= 0 && vox_y < a.H && vox_x >= 0 && vox_x < a.W && z >= 0 && z < a.D;
+        const bf16_t *xp = a.xcl + ((long)b * a.vol + ((long)(in ? z : 0) * a.H + (in ? vox_y : 0)) * a.W + (in ? vox_x : 0)) * a.Cin
+                           + cc0 * 64 + h * 8;
+        for_each_const([&](auto I) INLINE {
+            constexpr int ks = decltype(I)::value;
+            xa[ks] = u32x4_t{0u, 0u, 0u, 0u};
+            if (in && here) xa[ks] = *reinterpret_cast<const u32x4_t *>(xp + ks * 16);
+        }, std::make_integer_sequence<int, 4>{});
+    };
+    // sums of plane z (slot z & 1) -> accumulator, and cleared.  (Through a buffer descriptor of the plane: an add that
+    // goes nowhere has an offset past its end, and no branch stands between the adds.)
+    const unsigned plane_bytes = (unsigned)a.H * (unsigned)a.W * (unsigned)a.Cin * 4u;
+    auto flush_plane = [&](int z) INLINE {
+        const bool odd = z & 1, zin = z >= 0 && z < a.D;
+        // (worked out anew each time: kept across the points, these offsets would take the registers of the products)
+        int fn = n, fh = h;
+        opaque_v(fn); opaque_v(fh);
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc(a.gxcl + ((long)b * a.vol + (long)(zin ? z : 0) * a.H * a.W) * a.Cin, 0,
+                                                          (int)plane_bytes, 0x00020000);
+        for_each_const([&](auto I) INLINE {
+            constexpr int r = decltype(I)::value;
+            constexpr int dy = 2 * (r >> 2), dx = r & 3;
+            const int y = y0 + fh + dy, x = x0 + dx;
+            const bool in = zin && y >= 0 && y < a.H && x >= 0 && x < a.W;
+            const unsigned o = in ? (unsigned)((y * a.W + x) * a.Cin + cc0 * 64 + fn) * 4u : kNone;
+            for_each_const([&](auto Q) INLINE {
+                constexpr int q = decltype(Q)::value;
+                const float v = odd ? gacc[q][8 + r] : gacc[q][r];
+                gacc[q][r] = odd ? gacc[q][r] : 0.f;
+                gacc[q][8 + r] = odd ? 0.f : gacc[q][8 + r];
+                __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(v, rs, (int)o, q * 128, 0);
+            }, std::make_integer_sequence<int, 2>{});
+        }, std::make_integer_sequence<int, 8>{});
+    };
+
+    // LDS places of this lane: rows as they are loaded (8 lanes to a row: lanes of one load that each take 16 bytes of
+    // another row cost the L1 four times the lookups), as the operand of T, weights as they are made, and transposing
+    // reads of both (within 16 lanes, lane l element j comes from lane 4j + l/4, element l%4)
+    const int pv = lane >> 3, pc = lane & 7;
+    unsigned char *const g_st = s_g + pv * 128 + ((pc ^ g_swz(pv)) << 4), *const g_st1 = s_g + pv * 128 + ((pc ^ g_swz(pv) ^ 1) << 4);
+    const unsigned g_ld = lds_address(s_g) + n * 128 + ((h ^ g_swz(n)) << 4);
+    unsigned char *const w_st = s_w + n * 64 + (((h * 2) ^ ((n >> 2) & 3)) << 4), *const w_st1 = s_w + n * 64 + (((h * 2 + 1) ^ ((n >> 2) & 3)) << 4);
+    const int tr_row = h * 8 + ((lane & 15) >> 2), tr_pc = ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1), tr_in = (lane & 1) * 8;
+    const unsigned g_tr = lds_address(s_g) + tr_row * 128 + ((tr_pc ^ g_swz(tr_row)) << 4) + tr_in;
+    const unsigned w_tr = lds_address(s_w) + tr_row * 64 + ((tr_pc ^ (h * 2)) << 4) + tr_in;
+    auto tr_read = [](unsigned addr) INLINE {
+        return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s *)(size_t)addr));
+    };
+    auto operand = [](uint2 lo, uint2 hi) INLINE { return __builtin_bit_cast(bf16x8_t, make_uint4(lo.x, lo.y, hi.x, hi.y)); };
+
+    // Points are worked on 32 at a time; entries are requested three such steps ahead, grad-column rows two.
+    uint4 e0, e1, e2, e3;
+    float a0, a1, a2, a3;
+    u32x4_t row_a[4], row_b[4];
+    int e_lo = 0, cnt = 0;
+    auto entry = [&](int i, uint4 &q, float &al) INLINE {
+        const int e = max(e_lo + min(i + n, cnt - 1), 0);
+        q = a.L.pt[e]; al = a.L.alpha[e];
+    };
+    const auto rsg = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(a.gcol) + (long)cc0 * a.chunk_rows * 64, 0, (int)(unsigned)(a.chunk_rows * 128), 0x00020000);
+    auto rows = [&](const uint4 &q, u32x4_t (&row)[4]) INLINE {
+        for_each_const([&](auto I) INLINE {
+            constexpr int i = decltype(I)::value;
+            row[i] = __builtin_amdgcn_raw_buffer_load_b128(rsg, __builtin_amdgcn_ds_bpermute((i * 8 + pv) << 2, (int)q.x) + pc * 16, 0, 0);
+        }, std::make_integer_sequence<int, 4>{});
+    };
+    // what base plane zi - 1 needs: its points (the range `range` asked for) and the plane above it
+    int r_lo, r_n;
+    auto range = [&](int zi) INLINE {
+        const int sg = brick_seg(a.d, bg, min(zi, zi_hi - 1), by, bx);
+        r_lo = seg_start[sg]; r_n = seg_count[sg];
+    };
+    auto begin = [&](int zi) INLINE {
+        e_lo = __builtin_amdgcn_readfirstlane(r_lo); cnt = __builtin_amdgcn_readfirstlane(r_n);
+        if (cnt > 0) {
+            entry(0, e0, a0);
+            entry(32, e1, a1);
+            entry(64, e2, a2);
+        }
+        load_plane(zi);
+        if (cnt > 0) {
+            rows(e0, row_a);
+            rows(e1, row_b);
+        }
+    };
+    int par = 0, turn = 0;
+    range(zi_lo);
+    load_plane(zi_lo - 1);
+    begin(zi_lo);
+    for (int zi = zi_lo; zi < zi_hi; zi++) {
+        const int z = zi - 1;
+        const bool low = z & 1;                      // slot of the base plane
+        range(zi + 1);
+        auto step = [&](int i0, u32x4_t (&row)[4]) INLINE {
+            // the rows to LDS, others requested in their place.  (The entry first: loads complete in order, and it is
+            // wanted first.  Past the last point: its row again.)
+            entry(i0 + 96, e3, a3);
+            __builtin_amdgcn_sched_barrier(0);
+            *reinterpret_cast<u32x4_t *>(g_st) = row[0];
+            *reinterpret_cast<u32x4_t *>(g_st1 + 1024) = row[1];
+            *reinterpret_cast<u32x4_t *>(g_st + 2048) = row[2];
+            *reinterpret_cast<u32x4_t *>(g_st1 + 3072) = row[3];
+            rows(e2, row);
+            __builtin_amdgcn_sched_barrier(0);
+            const bool ok = i0 + n < cnt;
+            const float py = __uint_as_float(e0.y), px = __uint_as_float(e0.z), hz = __uint_as_float(e0.w), lz = 1.f - hz;
+            // ---- weights (lane = point, the 16 voxels of slot h)
+            {
+                const float wz = (ok ? a0 : 0.f) * ((h != 0) == low ? lz : hz);
+                float tx[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) tx[i] = __builtin_amdgcn_fmed3f(1.f - fabsf((float)i - px), 0.f, 1.f);
+                for_each_const([&](auto Y) INLINE {
+                    constexpr int y = decltype(Y)::value * 2;
+                    uint32_t wh[4], wl[4];
+#pragma unroll
+                    for (int j = 0; j < 8; j += 2) {
+                        const float ty = __builtin_amdgcn_fmed3f(1.f - fabsf((float)(y + j / 4) - py), 0.f, 1.f) * wz;
+                        const float w0 = ty * tx[j & 3], w1 = ty * tx[(j & 3) + 1];
+                        wh[j / 2] = pack_bf16x2(w0, w1);
+                        wl[j / 2] = pack_bf16x2(w0 - __uint_as_float(wh[j / 2] << 16), w1 - __uint_as_float(wh[j / 2] & 0xffff0000u));
+                    }
+                    *reinterpret_cast<uint4 *>(y ? w_st1 : w_st) = make_uint4(wh[0], wh[1], wh[2], wh[3]);
+                    *reinterpret_cast<uint4 *>((y ? w_st1 : w_st) + 2048) = make_uint4(wl[0], wl[1], wl[2], wl[3]);
+                }, std::make_integer_sequence<int, 2>{});
+            }
+            wave_fence();
+            // ---- the two products
+            f32x16 T;
+#pragma unroll
+            for (int r = 0; r < 16; r++) T[r] = 0.f;
+            for_each_const([&](auto KG) INLINE {
+                constexpr int kg = decltype(KG)::value;            // 16 points, and half of T's channels
+                const bf16x8_t wh = operand(tr_read(w_tr + kg * 1024), tr_read((w_tr ^ 16) + kg * 1024 + 256));
+                const bf16x8_t wl = operand(tr_read(w_tr + kg * 1024 + 2048), tr_read((w_tr ^ 16) + kg * 1024 + 2304));
+                for_each_const([&](auto Q) INLINE {
+                    constexpr int q = decltype(Q)::value, ks = kg * 2 + q;
+                    const u32x4_t gq = *reinterpret_cast<const __attribute__((address_space(3))) u32x4_t *>((size_t)(g_ld ^ (ks * 32)));
+                    T = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, xa[ks]), __builtin_bit_cast(bf16x8_t, gq), T, 0, 0, 0);
+                    const bf16x8_t gb = operand(tr_read((g_tr ^ (q * 64)) + kg * 2048), tr_read((g_tr ^ (q * 64) ^ 32) + kg * 2048 + 512));
+                    gacc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wh, gb, gacc[q], 0, 0, 0);
+                    gacc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wl, gb, gacc[q], 0, 0, 0);
+                }, std::make_integer_sequence<int, 2>{});
+            }, std::make_integer_sequence<int, 2>{});
+            wave_fence();
+            // ---- grad_offset / grad_mask from the point's corner dots
+            {
+                const bool y1 = py >= 1.f, y2 = py >= 2.f, x1 = px >= 1.f, x2 = px >= 2.f;
+                const float hy = py - (y2 ? 2.f : (y1 ? 1.f : 0.f)), hx = px - (x2 ? 2.f : (x1 ? 1.f : 0.f));
+                const bool q = h ? y2 : y1;                       // the corner row along y this half holds ...
+                const bool hi = (y1 != y2) != (h != 0);           // ... and whether it is the upper one
+                // (single registers from here on: a choice between two elements of T is not to become a variable index)
+                float tv[16];
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    tv[r] = T[r];
+                    opaque_v(tv[r]);
+                }
+                float sx[2], ex[2];
+#pragma unroll
+                for (int zz = 0; zz < 2; zz++) {
+                    float ty[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) ty[i] = q ? tv[zz * 8 + 4 + i] : tv[zz * 8 + i];
+                    const float d0 = x2 ? ty[2] : (x1 ? ty[1] : ty[0]);
+                    const float d1 = x2 ? ty[3] : (x1 ? ty[2] : ty[1]);
+                    sx[zz] = fmaf(hx, d1 - d0, d0);
+                    ex[zz] = d1 - d0;
+                }
+                const float w0 = low ? hz : lz, w1 = low ? lz : hz;
+                const float sz = fmaf(w1, sx[1], w0 * sx[0]), ez = fmaf(w1, ex[1], w0 * ex[0]);
+                const float dz = low ? sx[0] - sx[1] : sx[1] - sx[0];
+                const float wy = hi ? hy : 1.f - hy;
+                const float r_m = wy * sz, r_y = hi ? sz : -sz, r_x = wy * ez, r_z = wy * dz;
+                // the two halves of a point: lanes 0 - 31 end with (mask, x), the others with (z, y)
+                const auto u = __builtin_amdgcn_permlane32_swap(__float_as_uint(r_m), __float_as_uint(r_z), false, false);
+                const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(r_x), __float_as_uint(r_y), false, false);
+                float2 r = make_float2(__uint_as_float(u[0]) + __uint_as_float(u[1]), __uint_as_float(v[0]) + __uint_as_float(v[1]));
+                if (nw > 1) {
+                    // the chunks of the other wavefronts, which take turns in adding up and storing
+                    s_part[(par * nw + wave) * 64 + lane] = r;
+                    lds_only_barrier();
+                    if (turn == wave) {
+                        r = make_float2(0.f, 0.f);
+                        for (int w = 0; w < nw; w++) {
+                            const float2 q2 = s_part[(par * nw + w) * 64 + lane];
+                            r.x += q2.x; r.y += q2.y;
+                        }
+                    }
+                }
+                // (a store of every lane through a descriptor of the 32 results: no branch, see flush_plane)
+                typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+                const auto rs = __builtin_amdgcn_make_buffer_rsrc(a.res + (set * a.nres + e_lo + i0) * 2, 0,
+                                                                  turn == wave ? min(cnt - i0, 32) * res_bytes : 0, 0x00020000);
+                __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(r.x), __float_as_uint(r.y)}, rs, n * 16 + h * 8, 0, 0);
+                par ^= 1;
+                if (++turn == nw) turn = 0;
+            }
+            e0 = e1; a0 = a1;
+            e1 = e2; a1 = a2;
+            e2 = e3; a2 = a3;
+        };
+        for (int i0 = 0; i0 < cnt; i0 += 64) {
+            step(i0, row_a);
+            if (i0 + 32 < cnt) step(i0 + 32, row_b);
+        }
+        // (the loads of the next base plane first: a wait for them then is no wait for the adds)
+        if (zi + 1 < zi_hi) begin(zi + 1);
+        if (want_gx) flush_plane(z);
+    }
+    if (want_gx) flush_plane(zi_hi - 1);
+#undef INLINE
+}
+
+// ---- per-point sums -> gradients in their storage type and layout --------------------------------------------------
+D2C_DEV void brick_point_sums(const float2 *res, long nres, int nset, int at, float2 &mx, float2 &zy)
+{
+    mx = zy = make_float2(0.f, 0.f);
+    if (at < 0) return;
+    for (int i = 0; i < nset; i++) {
+        const float4 v = reinterpret_cast<const float4 *>(res)[i * nres + at];
+        mx.x += v.x; mx.y += v.y; zy.x += v.z; zy.y += v.w;
+    }
+}
+template <bool AUX16>
+__global__ void __launch_bounds__(256)
+brick_finish_kernel(TiledShape s, BrickLists L, const float2 *res, long nres, int nset, const void *mask, void *goff, void *gmask,
+                    int ngrp)
+{
+    typedef typename std::conditional<AUX16, bf16_t, float>::type AT;
+    const PointUnit un = point_unit(s, ngrp);
+    const int k0 = un.k0, bg = un.bg, b = un.b, g = un.g, p = un.p;
+    if (p >= s.P) return;
+    int at[kTaps];
+    float al[kTaps];
+    float2 mx[kTaps], zy[kTaps];
+#pragma unroll
+    for (int i = 0; i < kTaps; i++) {
+        const int k = min(k0 + i, s.K - 1);
+        at[i] = L.place[((long)bg * s.K + k) * s.P + p];
+        al[i] = mask ? ld_auxT<AUX16>(mask, mask_index(s, b, g, k, p)) : 1.f;
+    }
+#pragma unroll
+    for (int i = 0; i < kTaps; i++) brick_point_sums(res, nres, nset, at[i], mx[i], zy[i]);
+#pragma unroll
+    for (int i = 0; i < kTaps; i++) {
+        const int k = k0 + i;
+        if (k >= s.K) break;
+        const bool in = at[i] >= 0;
+        if (mask && s.mact) { al[i] = mask_act<AT>(s.mact, al[i]); mx[i].x *= mask_act_grad(s.mact, al[i]); }
+        if (gmask) reinterpret_cast<AT *>(gmask)[mask_index(s, b, g, k, p)] = f32_to_elem<AT>(in ? mx[i].x : 0.f);
+        if (goff) {
+            AT *o = reinterpret_cast<AT *>(goff) + offset_index(s, b, g, k, p);
+            o[0] = f32_to_elem<AT>(in && (s.axes & 1) ? al[i] * zy[i].x : 0.f);
+            o[s.P] = f32_to_elem<AT>(in && (s.axes & 2) ? al[i] * zy[i].y : 0.f);
+            o[2 * (long)s.P] = f32_to_elem<AT>(in && (s.axes & 4) ? al[i] * mx[i].y : 0.f);
+        }
+    }
+}
+// Size-map source: d(offset_a) / d(size_a) = base_a[k_a], so the taps of a position add up; the axes that a channel of
+// the raw map feeds add up, times the derivative of the size activation.  A workgroup is 64 positions x 4 shares of the
+// taps.
+template <bool AUX16>
+__global__ void __launch_bounds__(256)
+brick_finish_size_kernel(TiledShape s, BrickLists L, const float2 *res, long nres, int nset, const void *mask, const void *raw,
+                         void *graw, void *gmask)
+{
+    typedef typename std::conditional<AUX16, bf16_t, float>::type AT;
+    __shared__ float s_sum[4][3][64];
+    const int b = blockIdx.y, lane = threadIdx.x & 63, part = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + lane;
+    float sum[3] = {0.f, 0.f, 0.f};
+    if (p < s.P)
+#pragma unroll 4
+        for (int k = part; k < s.K; k += 4) {
+            const int at = L.place[((long)b * s.K + k) * s.P + p];
+            float2 mx, zy;
+            brick_point_sums(res, nres, nset, at, mx, zy);
+            float al = 1.f;
+            if (mask) {
+                const long mi = mask_index(s, b, 0, k, p);
+                al = ld_auxT<AUX16>(mask, mi);
+                if (s.mact) { al = mask_act<AT>(s.mact, al); mx.x *= mask_act_grad(s.mact, al); }
+                if (gmask) reinterpret_cast<AT *>(gmask)[mi] = f32_to_elem<AT>(at < 0 ? 0.f : mx.x);
+            }
+            if (at < 0) continue;
+            const int kx = k % s.geo.kw, ky = (k / s.geo.kw) % s.geo.kh, kz = k / (s.geo.kw * s.geo.kh);
+            sum[0] += s.ss.base[0][kz] * (al * zy.x);
+            sum[1] += s.ss.base[1][ky] * (al * zy.y);
+            sum[2] += s.ss.base[2][kx] * (al * mx.y);
+        }
+#pragma unroll
+    for (int ax = 0; ax < 3; ax++) s_sum[part][ax][lane] = sum[ax];
+    __syncthreads();
+    const int c = part;                               // channel of the map
+    if (!graw || p >= s.P || c >= mode_channels(s.ss.mode)) return;
+    float v = 0.f;
+#pragma unroll
+    for (int ax = 0; ax < 3; ax++)
+        if (axis_channel(s.ss.mode, ax) == c) v += (s_sum[0][ax][lane] + s_sum[1][ax][lane]) + (s_sum[2][ax][lane] + s_sum[3][ax][lane]);
+    const long ri = (long)b * s.obs + (long)c * s.P + p;
+    v *= size_act_grad(s.ss.act, ld_auxT<AUX16>(raw, ri));
+    reinterpret_cast<AT *>(graw)[ri] = f32_to_elem<AT>(v);
+}
+
+BrickDims brick_dims(const TiledShape &s) { return BrickDims{s.D + 1, (s.H + 3) / 3, (s.W + 3) / 3}; }
+long brick_nseg(const TiledShape &s)
+{
+    const BrickDims d = brick_dims(s);
+    return (long)s.N * s.G * d.nz * d.nby * d.nbx;
+}
+long brick_points(const TiledShape &s) { return (long)s.N * s.G * s.K * s.P; }
+int brick_sets(const TiledShape &s) { return (s.cpg / 64 + kMaxWaves - 1) / kMaxWaves; }
+BrickLists brick_lists(const TiledShape &s, char *base)
+{
+    const BrickWs w = d2c_brick_ws(s);
+    return BrickLists{(int *)(base + w.count), (int *)(base + w.count) + brick_nseg(s), (int *)(base + w.start), (int *)(base + w.place),
+                      (uint4 *)(base + w.pt), (float *)(base + w.alpha)};
+}
+
+}  // namespace
+
+// The bricks serve bfloat16 problems in three dimensions whose blocks hold enough points to fill most of a matrix
+// product of 32: below about half a product on average (few taps, strided outputs) the gathering kernels are as good.
+bool d2c_brick_supported(const TiledShape &s, int dtype)
+{
+    if (s.nd != 3 || dtype != D2C_BF16 || s.cpg % 64) return false;
+    const double mean = 9.0 * s.K * s.P / s.vol;
+    return mean >= 16.0 && s.K <= 65535 && (long)s.N * s.G <= 65535 && brick_nseg(s) < (1L << 31) - 1024 &&
+           brick_points(s) < (1L << 31) - 64 && (size_t)s.K * s.M * 128 < 0xFFFFFF00u &&
+           (size_t)s.H * s.W * s.Cin * 4 < 0xFFFFFFF0u;
+}
+BrickWs d2c_brick_ws(const TiledShape &s)
+{
+    const size_t n = (size_t)brick_points(s), nseg = (size_t)brick_nseg(s);
+    BrickWs w;
+    w.count = 0;                                                   // [nseg] counts, then the cursor: one clear
+    w.start = d2c_align_up((nseg + 1) * 4);
+    w.place = w.start + d2c_align_up(nseg * 4);
+    w.pt = w.place + d2c_align_up(n * 4);
+    w.alpha = w.pt + d2c_align_up(n * 16);
+    w.res = w.alpha + d2c_align_up(n * 4);
+    w.total = w.res + d2c_align_up(n * 16) * brick_sets(s);
+    return w;
+}
+
+// Sorts the points.
+int d2c_brick_sort(const TiledShape &s, const void *off, const void *mask, void *ws, hipStream_t st)
+{
+    D2cProfScope prof(D2C_PROF_PACK, st);
+    const BrickDims d = brick_dims(s);
+    const BrickLists L = brick_lists(s, (char *)ws);
+    const int nseg = (int)brick_nseg(s);
+    d2c_fill_zero(L.count, ((size_t)nseg + 1) * 4, st);
+    const int ngrp = (s.K + kTaps - 1) / kTaps;
+    const dim3 grid((unsigned)((long)((s.P + 255) / 256) * ngrp * s.N * s.G)), blk(256);
+    auto go = [&](auto A, auto Z) {
+        constexpr bool A16 = decltype(A)::value, SZ = decltype(Z)::value;
+        hipLaunchKernelGGL((brick_count_kernel<A16, SZ>), grid, blk, 0, st, s, d, L, off, ngrp);
+        hipLaunchKernelGGL(brick_range_kernel, dim3((nseg + 255) / 256), blk, 0, st, L, nseg);
+        hipLaunchKernelGGL((brick_file_kernel<A16, SZ>), grid, blk, 0, st, s, d, L, off, mask, ngrp);
+    };
+    if (s.adt == D2C_BF16) {
+        if (s.ss.on) go(std::true_type{}, std::true_type{});
+        else go(std::true_type{}, std::false_type{});
+    } else {
+        if (s.ss.on) go(std::false_type{}, std::true_type{});
+        else go(std::false_type{}, std::false_type{});
+    }
+    return d2c_check_launch("brick_file_kernel");
+}
+
+// `gxcl` (cleared here), `goff` (size-map source: the gradient of the raw map `raw`) and `gmask` may be NULL.
+int d2c_brick_grad(const TiledShape &s, const void *xcl, const void *gcol, const void *mask, const void *raw, float *gxcl,
+                   void *goff, void *gmask, void *ws, hipStream_t st)
+{
+    const BrickWs w = d2c_brick_ws(s);
+    const long n = brick_points(s);
+    BrickArgs a{};
+    a.d = brick_dims(s); a.L = brick_lists(s, (char *)ws);
+    a.xcl = (const bf16_t *)xcl; a.gcol = (const bf16_t *)gcol; a.gxcl = gxcl;
+    a.res = (goff || gmask) ? (float2 *)((char *)ws + w.res) : nullptr;
+    a.nres = (long)(d2c_align_up((size_t)n * 16) / 16);
+    a.G = s.G; a.cpc = s.cpg / 64; a.Cin = s.Cin; a.D = s.D; a.H = s.H; a.W = s.W; a.vol = s.vol;
+    a.chunk_rows = (long)s.K * s.M;
+    if (gxcl) {
+        // (what grad_input costs beside the kernel it shares with the offset / mask gradient)
+        D2cProfScope prof(D2C_PROF_GX_OWNER, st, "brick_grad_kernel");
+        d2c_fill_zero(gxcl, (size_t)s.N * s.vol * s.Cin * sizeof(float), st);
+    }
+    a.nset = brick_sets(s);
+    const int nw = (a.cpc + a.nset - 1) / a.nset;
+    // enough workgroups to fill the chip several times over; a range of z costs one more plane than it has bases
+    const int ncu = d2c_num_cus();
+    const long cols = (long)a.d.nbx * a.d.nby * s.N * s.G * a.nset;
+    a.zlen = a.d.nz;
+    while (a.zlen > 1 && cols * ((a.d.nz + a.zlen - 1) / a.zlen)  * nw < 64L * ncu) a.zlen = (a.zlen + 1) / 2;
+    a.nzr = (a.d.nz + a.zlen - 1) / a.zlen;
+    const unsigned grid = (unsigned)(cols * a.nzr);
+    {
+        D2cProfScope prof(D2C_PROF_BWD_AUX, st, "brick_grad_kernel");
+        hipLaunchKernelGGL(brick_grad_kernel, dim3(grid), dim3(64 * nw), nw * kWaveLds + (nw > 1 ? nw * 1024 : 0), st, a, a.L.start, a.L.count);
+        if (int rc = d2c_check_launch("brick_grad_kernel")) return rc;
+    }
+    if (!a.res) return D2C_OK;
+    D2cProfScope prof(D2C_PROF_PACK, st);
+    const bool a16 = s.adt == D2C_BF16;
+    if (s.ss.on) {
+        auto fin = a16 ? &brick_finish_size_kernel<true> : &brick_finish_size_kernel<false>;
+        hipLaunchKernelGGL(fin, dim3((s.P + 63) / 64, s.N), dim3(256), 0, st, s, a.L, a.res, a.nres, a.nset, mask, raw, goff, gmask);
+    } else {
+        auto fin = a16 ? &brick_finish_kernel<true> : &brick_finish_kernel<false>;
+        const int ngrp = (s.K + kTaps - 1) / kTaps;
+        hipLaunchKernelGGL(fin, dim3((unsigned)((long)((s.P + 255) / 256) * ngrp * s.N * s.G)), dim3(256), 0, st, s, a.L, a.res, a.nres, a.nset, mask,
+                           goff, gmask, ngrp);
+    }
+    return d2c_check_launch("brick_finish_kernel");
+}

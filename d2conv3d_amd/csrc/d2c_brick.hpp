@@ -1,0 +1,24 @@
+// The sampling points of a problem sorted by the block of base voxels they lie in, and the kernels that work on them
+// brick by brick (d2c_brick.hip).
+#pragma once
+#include "d2c_mma.hpp"
+
+struct BrickDims {
+    int nz, nby, nbx;        // base planes -1 .. D-1; blocks of three base voxels along y and x
+};
+struct BrickLists {
+    int *count;              // points per block
+    int *cursor;             // entries given out
+    int *start;              // first entry of a block
+    int *place;              // [n * G + g][tap][p]: a point's entry, -1: no corner inside the volume
+    uint4 *pt;               // byte offset of the point's row of 64 channels, y and x inside the block, fraction along z
+    float *alpha;            // modulation
+};
+struct BrickWs {
+    size_t count, start, place, pt, alpha, res, total;
+};
+bool d2c_brick_supported(const TiledShape &s, int dtype);
+BrickWs d2c_brick_ws(const TiledShape &s);
+int d2c_brick_sort(const TiledShape &s, const void *off, const void *mask, void *ws, hipStream_t st);
+int d2c_brick_grad(const TiledShape &s, const void *xcl, const void *gcol, const void *mask, const void *raw, float *gxcl,
+                   void *goff, void *gmask, void *ws, hipStream_t st);

@@ -2,6 +2,7 @@
 // dispatch.  Forward / backward kernels live in d2c_tiled_fwd.hip and
 // d2c_tiled_bwd.hip.
 #include "d2c_tiled.hpp"
+#include "d2c_brick.hpp"
 #include "d2c_mma.hpp"
 
 int d2c_fwd_out_tile(const TiledShape &s);
@@ -548,6 +549,13 @@ bool use_aux_kernel(const d2c_conv3d_desc &q, const TiledShape &s)
     return d2c_tiled_bwd_single_pass(s, q.dtype) || (s.nd == 3 && d2c_gx_mode() >= 1 && d2c_lists_supported(s));
 }
 
+// grad_offset, grad_mask and grad_input from bricks of sorted points (d2c_brick.hip): wherever whole grad-column rows are
+// at hand.  (A bucket capacity asked for by the test hook is a matter of the lists.)
+bool use_brick(const d2c_conv3d_desc &q, const TiledShape &s)
+{
+    return d2c_gx_mode() == 1 && use_lists(q, s) && use_aux_kernel(q, s) && d2c_brick_supported(s, q.dtype);
+}
+
 // grad_weight as a matrix product over sampled columns that the offset / mask gradient kernel writes on its way
 // (needs that kernel to run: the caller wants grad_offset or grad_mask)
 // (0 sample again, 1 columns in a buffer of their own, 2 columns over the grad-column rows: the description's
@@ -594,7 +602,7 @@ BwdSlices bwd_slices(const d2c_conv3d_desc &q, const TiledShape &s)
 }
 
 struct BwdWs {
-    size_t xcl, wt, gxcl, gwacc, goutp, auxacc, gcol, counts, entries, ovf, gsacc, sm1, col, total;
+    size_t xcl, wt, gxcl, gwacc, goutp, auxacc, gcol, counts, entries, ovf, gsacc, sm1, brick, col, total;
 };
 // `saved_columns`: the caller brings the sampled columns of the forward call (no column region, no slices)
 BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns = false)
@@ -636,6 +644,8 @@ BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns =
     if (s.ss.on) w.total += d2c_align_up((size_t)s.N * 3 * s.P * sizeof(float));
     w.sm1 = w.total;       // ... and (size - 1) per axis
     if (s.ss.on) w.total += d2c_align_up((size_t)s.N * 3 * s.P * sizeof(float));
+    w.brick = w.total;
+    if (use_brick(q, s)) w.total += d2c_brick_ws(s).total;
     w.col = w.total;       // sampled columns for the grad-weight product
     if (!saved_columns && use_col_weight(q, s) && !col_in_place(q, s))
         w.total += d2c_align_up(d2c_bwd_col_bytes(s, q.dtype, sl.cgs ? sl.cgs * (s.cpg / 64) : 0));
@@ -774,18 +784,21 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
             // runs, by a pass of their own otherwise
             // size-map source: `goff` is the gradient of the raw size map; the offset / mask gradient kernel adds
             // into fp32 sums per axis, which a finishing kernel folds into it
+            gw_from_col = gw && (columns ? d2c_bwd_weight_from_kept_col(s, q.dtype) : (auxk && use_col_weight(q, s)));
+            const bool brick = use_brick(q, s) && !(gw_from_col && !columns);
             void *goff_k = goff;
-            if (s.ss.on && goff) {
+            if (s.ss.on && goff && !brick) {
                 goff_k = base + l.gsacc;
                 D2cProfScope prof(D2C_PROF_PACK, st);
                 d2c_fill_zero(goff_k, (size_t)s.N * 3 * s.P * sizeof(float), st);
             }
-            gw_from_col = gw && (columns ? d2c_bwd_weight_from_kept_col(s, q.dtype) : (auxk && use_col_weight(q, s)));
             // (the sampled columns over the grad-column rows: grad_input has to be done with the rows before the
             // offset / mask gradient kernel runs, so the samples are filed by a pass of their own)
             gw_in_place = gw_from_col && !columns && col_in_place(q, s);
             SampleLists L{nullptr, nullptr, nullptr, 0, 0, 0};
-            if (lists) {
+            if (brick) {
+                if (int rc = d2c_brick_sort(s, off, mask, base + l.brick, st)) return rc;
+            } else if (lists) {
                 L = d2c_lists_make(s, Elem<T>::DT, base + l.counts, base + l.entries, base + l.ovf);
                 if (int rc = (auxk && !gw_in_place) ? d2c_lists_clear(L, st) : d2c_lists_build(s, off, mask, L, st)) return rc;
             }
@@ -801,13 +814,15 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
                 d2c_fill_zero(base + l.gcol + (size_t)(s.Cin / bkc_of(q.dtype)) * s.K * s.M * bkc_of(q.dtype) * sizeof(T),
                               (size_t)64 * bkc_of(q.dtype) * sizeof(T), st);
             }
-            if (auxk)
+            if (brick) {
+                if (int rc = d2c_brick_grad(s, xcl_p, base + l.gcol, mask, size_raw, gxcl, goff, gmask, base + l.brick, st)) return rc;
+            } else if (auxk)
                 if (int rc = d2c_aux_grad_launch<T>(s, xcl_p, off, mask, base + l.gcol, goff_k, gmask,
                                                     (lists && !gw_in_place) ? &L : nullptr,
                                                     (gw_from_col && !columns) ? (gw_in_place ? base + l.gcol : base + l.col) : nullptr,
                                                     gw_in_place, st))
                     return rc;
-            if (s.ss.on && goff) {
+            if (s.ss.on && goff && !brick) {
                 D2cProfScope prof(D2C_PROF_PACK, st);
                 long gr = ((long)s.N * s.P + 255) / 256;
                 if (gr > 8192) gr = 8192;
@@ -819,7 +834,7 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
                                        (const float *)goff_k, size_raw, goff);
                 if (int rc = d2c_check_launch("size_grad_finish_kernel")) return rc;
             }
-            if (lists && !gw_in_place)
+            if (lists && !gw_in_place && !brick)
                 if (int rc = d2c_gx_owner_launch<T>(s, base + l.gcol, L, gxcl, st)) return rc;
             if (gx)
                 if (int rc = d2c_tiled_unpack_gx<T>(s, gxcl, gx, st)) return rc;
