@@ -4,6 +4,11 @@
 // and read every input value from memory (:25-92 forward, :97-175 grad_input,
 // :178-276 grad_weight with a shared-memory reduction per output channel).
 //
+// The usual filter of the backbone -- 3x3x3, unit stride and dilation, padding 1, one output channel per input channel --
+// runs on kernels that march along z (dwc_march_*): a thread owns kVW x kMR elements of a plane, every plane is read
+// once and serves three output planes from registers; the backward kernel forms grad_input, grad_weight and grad_bias
+// from the same reads.  The other shapes:
+//
 // Here the tensors stay NCDHW (W contiguous) and a thread owns kVW consecutive
 // elements along W: for 3x3x3 filters with unit stride and dilation along W
 // (the backbone's case) an input row segment of kVW + 2 values serves 3 taps of
@@ -389,6 +394,267 @@ __global__ void __launch_bounds__(kThreadsDw) dwc_bias_grad_kernel(DwcShape s, c
     block_add<CT>(acc, gbacc + co, s_red);
 }
 
+// ---------------------------------------------------------------- marching kernels
+// A workgroup = one (sample, channel), kTY * kMR rows, kTX * kVW columns, a range of planes.  What bounds them is memory:
+// 2x256x8x56x56 float moves 103 MB forward, 154 MB backward (20 and 30 us at the rate of a large copy); with a row of
+// nine segments read per output row (the kernels above) forward took 48 us, backward 66 + 102 us and three small launches.
+constexpr int kMR = 2;                          // rows per thread
+constexpr int kMTaps = 28;                      // 27 taps and the bias
+struct MarchTiles {
+    int ty, tx, nz, zlen;                       // tiles along y and x, ranges of planes and their length
+};
+MarchTiles march_tiles(const d2c_dwconv3d_desc &q)
+{
+    MarchTiles t;
+    t.ty = (q.H + kTY * kMR - 1) / (kTY * kMR); t.tx = (q.W + kTX * kVW - 1) / (kTX * kVW);
+    t.zlen = q.D;
+    // (a range reads two planes more than it has: no shorter than 4 for the sake of more workgroups)
+    while (t.zlen > 4 && (long)q.N * q.C * t.ty * t.tx * ((q.D + t.zlen - 1) / t.zlen) < 2048) t.zlen = (t.zlen + 1) / 2;
+    t.nz = (q.D + t.zlen - 1) / t.zlen;
+    return t;
+}
+bool march_ok(const d2c_dwconv3d_desc &q)
+{
+    return q.dtype != D2C_F64 && q.Cout == q.C && q.kd == 3 && q.kh == 3 && q.kw == 3 && q.sd == 1 && q.sh == 1 && q.sw == 1 &&
+           q.pd == 1 && q.ph == 1 && q.pw == 1 && q.dd == 1 && q.dh == 1 && q.dw == 1;
+}
+// kVW elements of a row of `width` from x0 on, zeros outside it.  VEC: rows kVW-aligned in memory, whole groups.
+template <typename ST, bool VEC> D2C_DEV void march_load(const ST *row, int x0, int width, bool ok, float *m)
+{
+    if constexpr (VEC) {
+        m[0] = m[1] = m[2] = m[3] = 0.f;
+        if (ok && x0 < width) {
+            if constexpr (sizeof(ST) == 4) {
+                const float4 t = *reinterpret_cast<const float4 *>(row + x0);
+                m[0] = t.x; m[1] = t.y; m[2] = t.z; m[3] = t.w;
+            } else {
+                const uint2 t = *reinterpret_cast<const uint2 *>(row + x0);
+                m[0] = __uint_as_float(t.x << 16); m[1] = __uint_as_float(t.x & 0xffff0000u);
+                m[2] = __uint_as_float(t.y << 16); m[3] = __uint_as_float(t.y & 0xffff0000u);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < kVW; i++) m[i] = (ok && x0 + i < width) ? ldv<ST>(row, x0 + i) : 0.f;
+    }
+}
+template <typename ST, bool VEC> D2C_DEV void march_store(ST *row, int x0, int width, const float *m)
+{
+    if constexpr (VEC) {
+        if (x0 >= width) return;
+        if constexpr (sizeof(ST) == 4) *reinterpret_cast<float4 *>(row + x0) = make_float4(m[0], m[1], m[2], m[3]);
+        else *reinterpret_cast<uint2 *>(row + x0) = make_uint2(f32_to_bf16(m[0]) | ((uint32_t)f32_to_bf16(m[1]) << 16),
+                                                               f32_to_bf16(m[2]) | ((uint32_t)f32_to_bf16(m[3]) << 16));
+    } else {
+#pragma unroll
+        for (int i = 0; i < kVW; i++)
+            if (x0 + i < width) stv<ST>(row, x0 + i, m[i]);
+    }
+}
+// One plane's rows y0 - 1 .. y0 + kMR of a thread, as they come from memory ...
+struct MarchRows {
+    float m[kMR + 2][kVW];
+    float l[kMR + 2], r[kMR + 2];               // the elements beside the tile (its first and last lane)
+};
+template <typename ST, bool VEC>
+D2C_DEV void march_rows(const ST *plane, bool plane_ok, int y0, int x0, int H, int W, MarchRows &o)
+{
+    const int tx = threadIdx.x % kTX;
+#pragma unroll
+    for (int j = 0; j < kMR + 2; j++) {
+        const int y = y0 - 1 + j;
+        const bool ok = plane_ok && y >= 0 && y < H;
+        const ST *row = plane + (long)(ok ? y : 0) * W;
+        march_load<ST, VEC>(row, x0, W, ok, o.m[j]);
+        o.l[j] = (ok && tx == 0 && x0 > 0) ? ldv<ST>(row, x0 - 1) : 0.f;
+        o.r[j] = (ok && tx == kTX - 1 && x0 + kVW < W) ? ldv<ST>(row, x0 + kVW) : 0.f;
+    }
+}
+// ... and row j with its neighbours along x: v[i] is element x0 - 1 + i.  (The 16 lanes of a row are one DPP row.)
+D2C_DEV void march_segment(const MarchRows &o, int j, float *v)
+{
+    const int tx = threadIdx.x % kTX;
+    const float left = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(o.m[j][3]), 0x111, 0xF, 0xF, true));    // row_shr 1
+    const float right = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(o.m[j][0]), 0x101, 0xF, 0xF, true));   // row_shl 1
+    v[0] = tx == 0 ? o.l[j] : left;
+    v[1] = o.m[j][0]; v[2] = o.m[j][1]; v[3] = o.m[j][2]; v[4] = o.m[j][3];
+    v[5] = tx == kTX - 1 ? o.r[j] : right;
+}
+struct MarchPos {
+    int nc, c, y0, x0, z_lo, z_hi, tile;
+};
+D2C_DEV MarchPos march_pos(const d2c_dwconv3d_desc &q, const MarchTiles &t)
+{
+    MarchPos p;
+    p.nc = blockIdx.x;
+    p.c = p.nc % q.C;
+    int b = blockIdx.y;
+    const int bx = b % t.tx; b /= t.tx;
+    const int by = b % t.ty, bz = b / t.ty;
+    p.y0 = (by * kTY + (int)(threadIdx.x / kTX)) * kMR;
+    p.x0 = (bx * kTX + (int)(threadIdx.x % kTX)) * kVW;
+    p.z_lo = bz * t.zlen; p.z_hi = min(p.z_lo + t.zlen, q.D);
+    p.tile = (p.nc / q.C) * (int)gridDim.y + (int)blockIdx.y;
+    return p;
+}
+
+template <typename ST, bool VEC>
+__global__ void __launch_bounds__(kThreadsDw) dwc_march_fwd_kernel(d2c_dwconv3d_desc q, MarchTiles t, const ST *__restrict__ x,
+                                                                   const ST *__restrict__ w, const ST *__restrict__ bias,
+                                                                   ST *__restrict__ out)
+{
+    const MarchPos p = march_pos(q, t);
+    const long HW = (long)q.H * q.W;
+    const ST *xc = x + (long)p.nc * q.D * HW;
+    ST *oc = out + (long)p.nc * q.D * HW;
+    float wv[27];
+#pragma unroll
+    for (int k = 0; k < 27; k++) wv[k] = ldv<ST>(w, (long)p.c * 27 + k);
+    const float bv = bias ? ldv<ST>(bias, p.c) : 0.f;
+    float acc[3][kMR][kVW];                     // output planes z - 1, z, z + 1 while input plane z is worked on
+#pragma unroll
+    for (int i = 0; i < 3 * kMR * kVW; i++) (&acc[0][0][0])[i] = bv;
+    MarchRows cur, nxt;
+    march_rows<ST, VEC>(xc + max(p.z_lo - 1, 0) * HW, p.z_lo > 0, p.y0, p.x0, q.H, q.W, cur);
+    for (int z = p.z_lo - 1; z <= p.z_hi; z++) {
+        if (z < p.z_hi) march_rows<ST, VEC>(xc + min(z + 1, q.D - 1) * HW, z + 1 < q.D, p.y0, p.x0, q.H, q.W, nxt);
+#pragma unroll
+        for (int j = 0; j < kMR + 2; j++) {
+            float v[kVW + 2];
+            march_segment(cur, j, v);
+#pragma unroll
+            for (int r = 0; r < kMR; r++) {
+                const int ky = j - r;           // row y0 + r reads rows y0 + r - 1 + ky
+                if (ky < 0 || ky > 2) continue;
+#pragma unroll
+                for (int kz = 0; kz < 3; kz++)
+#pragma unroll
+                    for (int kx = 0; kx < 3; kx++)
+#pragma unroll
+                        for (int i = 0; i < kVW; i++)
+                            acc[2 - kz][r][i] = fmaf(wv[(kz * 3 + ky) * 3 + kx], v[i + kx], acc[2 - kz][r][i]);
+            }
+        }
+        if (z - 1 >= p.z_lo) {
+#pragma unroll
+            for (int r = 0; r < kMR; r++)
+                if (p.y0 + r < q.H) march_store<ST, VEC>(oc + (z - 1) * HW + (long)(p.y0 + r) * q.W, p.x0, q.W, acc[0][r]);
+        }
+#pragma unroll
+        for (int r = 0; r < kMR; r++)
+#pragma unroll
+            for (int i = 0; i < kVW; i++) { acc[0][r][i] = acc[1][r][i]; acc[1][r][i] = acc[2][r][i]; acc[2][r][i] = bv; }
+        cur = nxt;
+    }
+}
+
+// part[tile][channel][kMTaps]: the workgroup's sums of grad_weight and grad_bias (or NULL); gx or NULL
+template <typename ST, bool VEC>
+__global__ void __launch_bounds__(kThreadsDw) dwc_march_bwd_kernel(d2c_dwconv3d_desc q, MarchTiles t, const ST *__restrict__ gout,
+                                                                   const ST *__restrict__ x, const ST *__restrict__ w,
+                                                                   ST *__restrict__ gx, float *__restrict__ part)
+{
+    const MarchPos p = march_pos(q, t);
+    const long HW = (long)q.H * q.W;
+    const ST *gc = gout + (long)p.nc * q.D * HW, *xc = x + (long)p.nc * q.D * HW;
+    float wv[27];
+#pragma unroll
+    for (int k = 0; k < 27; k++) wv[k] = ldv<ST>(w, (long)p.c * 27 + k);
+    float acc[3][kMR][kVW], xv[3][kMR][kVW];    // grad_input and input of planes z - 1, z, z + 1 while grad_out plane z is worked on
+    float gw[kMTaps];
+#pragma unroll
+    for (int i = 0; i < 3 * kMR * kVW; i++) (&acc[0][0][0])[i] = (&xv[0][0][0])[i] = 0.f;
+#pragma unroll
+    for (int k = 0; k < kMTaps; k++) gw[k] = 0.f;
+    // (input outside the range is another workgroup's: zero here)
+    auto load_x = [&](int z, float (*o)[kVW]) {
+#pragma unroll
+        for (int r = 0; r < kMR; r++)
+            march_load<ST, VEC>(xc + min(z, q.D - 1) * HW + (long)min(p.y0 + r, q.H - 1) * q.W, p.x0, q.W,
+                                part && z < p.z_hi && p.y0 + r < q.H, o[r]);
+    };
+    MarchRows cur, nxt;
+    float xn[kMR][kVW];
+    march_rows<ST, VEC>(gc + max(p.z_lo - 1, 0) * HW, p.z_lo > 0, p.y0, p.x0, q.H, q.W, cur);
+    load_x(p.z_lo, xv[2]);
+    for (int z = p.z_lo - 1; z <= p.z_hi; z++) {
+        if (z < p.z_hi) {
+            march_rows<ST, VEC>(gc + min(z + 1, q.D - 1) * HW, z + 1 < q.D, p.y0, p.x0, q.H, q.W, nxt);
+            load_x(z + 2, xn);
+        }
+        // grad_input plane z' takes tap kz of grad_out plane z = z' + 1 - kz: z' = z - 1 + kz; and grad_weight the same pair
+#pragma unroll
+        for (int j = 0; j < kMR + 2; j++) {
+            float v[kVW + 2];
+            march_segment(cur, j, v);
+            if (j >= 1 && j <= kMR && z >= p.z_lo && z < p.z_hi) gw[27] += (v[1] + v[2]) + (v[3] + v[4]);
+#pragma unroll
+            for (int r = 0; r < kMR; r++) {
+                const int ky = r + 2 - j;       // row y0 + r takes tap ky from row y0 + r + 1 - ky
+                if (ky < 0 || ky > 2) continue;
+#pragma unroll
+                for (int kz = 0; kz < 3; kz++)
+#pragma unroll
+                    for (int kx = 0; kx < 3; kx++) {
+                        const int k = (kz * 3 + ky) * 3 + kx;
+#pragma unroll
+                        for (int i = 0; i < kVW; i++) {
+                            acc[kz][r][i] = fmaf(wv[k], v[i + 2 - kx], acc[kz][r][i]);
+                            gw[k] = fmaf(xv[kz][r][i], v[i + 2 - kx], gw[k]);
+                        }
+                    }
+            }
+        }
+        if (gx && z - 1 >= p.z_lo) {
+#pragma unroll
+            for (int r = 0; r < kMR; r++)
+                if (p.y0 + r < q.H)
+                    march_store<ST, VEC>(gx + (long)p.nc * q.D * HW + (z - 1) * HW + (long)(p.y0 + r) * q.W, p.x0, q.W, acc[0][r]);
+        }
+#pragma unroll
+        for (int r = 0; r < kMR; r++)
+#pragma unroll
+            for (int i = 0; i < kVW; i++) {
+                acc[0][r][i] = acc[1][r][i]; acc[1][r][i] = acc[2][r][i]; acc[2][r][i] = 0.f;
+                xv[0][r][i] = xv[1][r][i]; xv[1][r][i] = xv[2][r][i]; xv[2][r][i] = xn[r][i];
+            }
+        cur = nxt;
+    }
+    if (!part) return;
+    __shared__ float s_red[kThreadsDw / 64][kMTaps];
+#pragma unroll
+    for (int k = 0; k < kMTaps; k++) {
+        const float v = wave_sum<float>(gw[k]);
+        if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6][k] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < kMTaps) {
+        float v = 0.f;
+#pragma unroll
+        for (int i = 0; i < kThreadsDw / 64; i++) v += s_red[i][threadIdx.x];
+        part[((long)p.tile * q.C + p.c) * kMTaps + threadIdx.x] = v;
+    }
+}
+// One workgroup per channel: the tiles' sums -> grad_weight, grad_bias (either may be NULL)
+template <typename ST>
+__global__ void __launch_bounds__(256) dwc_march_finish_kernel(const float *part, int C, int ntile, ST *gw, ST *gb)
+{
+    __shared__ float s_sum[8][32];
+    const int k = threadIdx.x & 31, sl = threadIdx.x >> 5, c = blockIdx.x;
+    float v = 0.f;
+    if (k < kMTaps)
+        for (int i = sl; i < ntile; i += 8) v += part[((long)i * C + c) * kMTaps + k];
+    s_sum[sl][k] = v;
+    __syncthreads();
+    if (threadIdx.x >= kMTaps) return;
+    v = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) v += s_sum[i][k];
+    if (k < 27) {
+        if (gw) stv<ST>(gw, (long)c * 27 + k, v);
+    } else if (gb) stv<ST>(gb, c, v);
+}
+
 DwcShape make_shape(const d2c_dwconv3d_desc &q)
 {
     DwcShape s;
@@ -420,6 +686,19 @@ template <typename ST> bool vec_ok(const d2c_dwconv3d_desc &q, const void *a, co
 template <typename ST>
 int forward_t(const d2c_dwconv3d_desc &q, const void *x, const void *w, const void *bias, void *out, hipStream_t st)
 {
+    if constexpr (sizeof(ST) <= 4) {
+        if (march_ok(q)) {
+            const MarchTiles t = march_tiles(q);
+            const dim3 grid((unsigned)(q.N * q.C), (unsigned)(t.ty * t.tx * t.nz));
+            if (vec_ok<ST>(q, x, out))
+                hipLaunchKernelGGL((dwc_march_fwd_kernel<ST, true>), grid, dim3(kThreadsDw), 0, st, q, t, (const ST *)x, (const ST *)w,
+                                   (const ST *)bias, (ST *)out);
+            else
+                hipLaunchKernelGGL((dwc_march_fwd_kernel<ST, false>), grid, dim3(kThreadsDw), 0, st, q, t, (const ST *)x, (const ST *)w,
+                                   (const ST *)bias, (ST *)out);
+            return d2c_check_launch("dwc_march_fwd_kernel");
+        }
+    }
     const DwcShape s = make_shape(q);
     const unsigned nc = (unsigned)(q.N * q.Cout);
     const dim3 tiles(nc, tiles_of(q.Do, q.Ho, (q.Wo + kVW - 1) / kVW));
@@ -447,6 +726,22 @@ int backward_t(const d2c_dwconv3d_desc &q, const void *gout, const void *x, cons
                void *ws, hipStream_t st)
 {
     typedef typename Acc<ST>::type CT;
+    if constexpr (sizeof(ST) <= 4) {
+        if (march_ok(q)) {
+            if (!gx && !gw && !gb) return D2C_OK;
+            const MarchTiles t = march_tiles(q);
+            const dim3 grid((unsigned)(q.N * q.C), (unsigned)(t.ty * t.tx * t.nz));
+            float *part = gw || gb ? (float *)ws : nullptr;
+            auto kern = vec_ok<ST>(q, gout, x) && reinterpret_cast<uintptr_t>(gx) % (kVW * sizeof(ST)) == 0
+                            ? &dwc_march_bwd_kernel<ST, true> : &dwc_march_bwd_kernel<ST, false>;
+            hipLaunchKernelGGL(kern, grid, dim3(kThreadsDw), 0, st, q, t, (const ST *)gout, (const ST *)x, (const ST *)w, (ST *)gx, part);
+            if (int rc = d2c_check_launch("dwc_march_bwd_kernel")) return rc;
+            if (!part) return D2C_OK;
+            hipLaunchKernelGGL(dwc_march_finish_kernel<ST>, dim3((unsigned)q.C), dim3(256), 0, st, part, q.C, q.N * (int)grid.y, (ST *)gw,
+                               (ST *)gb);
+            return d2c_check_launch("dwc_march_finish_kernel");
+        }
+    }
     const DwcShape s = make_shape(q);
     const bool blocked = host_blocked(q);
     if (gx) {
@@ -567,6 +862,10 @@ int d2c_dwconv3d_check(const d2c_dwconv3d_desc *q)
 size_t d2c_dwconv3d_backward_workspace_bytes(const d2c_dwconv3d_desc *q)
 {
     if (d2c_dwconv3d_check(q) != D2C_OK) return 0;
+    if (march_ok(*q)) {
+        const MarchTiles t = march_tiles(*q);
+        return d2c_align_up((size_t)q->N * t.ty * t.tx * t.nz * q->C * kMTaps * sizeof(float));
+    }
     return d2c_align_up((size_t)q->Cout * (q->kd * q->kh * q->kw + 1) * (q->dtype == D2C_F64 ? 8 : 4));
 }
 
