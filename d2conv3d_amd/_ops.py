@@ -63,6 +63,29 @@ def _workspace_bytes_cached():
     return {k: v.numel() for k, v in _WS_CACHE.items()}
 
 
+# The calls that need nothing special, in native code (csrc/torch/native.cpp): operator call and autograd node.  A native
+# function returns None for a call that it leaves to the Python code below.
+try:
+    from . import _native
+except ImportError:
+    _native = None
+else:
+    _native.init(_WS_CACHE, _WS_CACHE_ON, _workspace)
+
+
+def _try_native(name, *args):
+    if _native is None:
+        return None
+    try:
+        return getattr(_native, name)(*args)
+    except TypeError:      # (an argument of another type: the Python code converts it or says what is wrong)
+        return None
+
+
+def _keep_max():
+    return _KEEP_COLUMNS["max_bytes"] if _KEEP_COLUMNS["on"] else 0
+
+
 def _check_common(nd, input, offset, alpha, weight, bias, groups, offset_groups):
     """SANITY_CHECK_DCONV_INPUTS / _GROUPS of dconv_gpu_common.h:17-43."""
     def req(cond, msg):
@@ -291,6 +314,11 @@ def deform_conv3d(input, offset, alpha, weight, bias, stride_d, stride_h, stride
     channels come back zero (matrix-core kernels only, see conv3d_algo).  `backward_flags`: the description's field
     of that name (_lib.BWD_GW_* | _lib.bwd_slices(n)): how the backward pass trades workspace for time.  `prepared`: a
     PreparedRegion kept by the calling layer (see DeformConv3d.reuse_prepared)."""
+    if not relu_scale > 0 and not want_stats and prepared is None:
+        out = _try_native("conv3d", input, offset, alpha, weight, bias, (stride_d, stride_h, stride_w), (pad_d, pad_h, pad_w),
+                          (dilation_d, dilation_h, dilation_w), groups, offset_groups, offset_axes, backward_flags, _keep_max())
+        if out is not None:
+            return out
     _check_common(3, input, offset, alpha, weight, bias, groups, offset_groups)
     input, offset, alpha, weight, bias = _unify(input, offset, alpha, weight, bias)
     return _DeformConv3dFunction.apply(
@@ -387,6 +415,19 @@ class _DeformConv3dSizedFunction(torch.autograd.Function):
         return (gx, gsize, galpha, gw, gb) + (None,) * 8
 
 
+_SIZE_CHANNELS = {"xyz": 3, "xxz": 2, "xy": 2, "x": 1}
+_SIZE_TEMPLATES = {}
+
+
+def _size_template(mode, kernel_shape, dilation, activation):
+    """The bytes of a size-map description, all but what the call's tensor decides (batch size, positions, element type)."""
+    key = (mode, kernel_shape, dilation, activation)
+    if key not in _SIZE_TEMPLATES:
+        from .grid import size_map_desc
+        _SIZE_TEMPLATES[key] = bytes(size_map_desc(torch.empty(1, 1, 1, device="meta"), mode, kernel_shape, dilation, activation))
+    return _SIZE_TEMPLATES[key]
+
+
 def deform_conv3d_sized(input, size_raw, alpha, weight, bias, mode, activation, stride, padding, dilation, groups=1,
                         relu_scale=0.0, want_stats=False):
     """Deformable convolution whose tap offsets follow from a predicted size map:
@@ -395,6 +436,12 @@ def deform_conv3d_sized(input, size_raw, alpha, weight, bias, mode, activation, 
     from torch.nn.modules.utils import _triple
     stride, padding, dilation = (tuple(int(v) for v in _triple(t)) for t in (stride, padding, dilation))
     mode = mode.lower()
+    if not relu_scale > 0 and not want_stats and mode in _SIZE_CHANNELS and weight.dim() == 5:
+        out = _try_native("conv3d_sized", input, size_raw, alpha, weight, bias,
+                          _size_template(mode, tuple(weight.shape[2:]), dilation, activation), _SIZE_CHANNELS[mode], stride, padding,
+                          dilation, groups, _keep_max())
+        if out is not None:
+            return out
     want_c = {"xyz": 3, "xxz": 2, "xy": 2, "x": 1}[mode]
     K = weight.shape[2] * weight.shape[3] * weight.shape[4]
     if size_raw.dim() != 5 or size_raw.shape[1] != want_c:
@@ -552,12 +599,28 @@ def deform_conv3d_packed_supported(input, deformation, weight, lead, mask_activa
         return bool(lib.d2c_conv3d_packed_supported(ctypes.byref(desc), ctypes.byref(sdesc) if sdesc is not None else None))
 
 
+def native_packed(input, deformation, weight, bias, lead, mask_activation, stride, padding, dilation, groups, offset_groups,
+                  mode=None, size_activation="linear", offset_axes=7, backward_flags=0):
+    """deform_conv3d_packed in native code, or None where the call is not one for it or the kernels do not take the
+    deformation tensor as it is (see deform_conv3d_packed_supported)."""
+    if mask_activation not in _lib.MASK_ACTIVATIONS or weight.dim() != 5:
+        return None
+    size = b"" if mode is None else _size_template(mode, tuple(weight.shape[2:]), tuple(dilation), size_activation)
+    return _try_native("conv3d_packed", input, deformation, weight, bias, lead, _lib.MASK_ACTIVATIONS[mask_activation], size,
+                       stride, padding, dilation, groups, offset_groups, offset_axes, backward_flags, _keep_max())
+
+
 def deform_conv3d_packed(input, deformation, weight, bias, lead, mask_activation, stride, padding, dilation, groups,
                          offset_groups, mode=None, size_activation="linear", relu_scale=0.0, want_stats=False,
                          offset_axes=7, backward_flags=0):
     """deform_conv3d / deform_conv3d_sized on the un-split output of the deformation branch: see
     _DeformConv3dPackedFunction.  `lead`: channels in front of the modulation values (3*G*K offsets, or the size
     map's 1 | 2 | 3 with `mode`); `mask_activation`: "sigmoid" | "relu" | "tanh" | "linear"."""
+    if not relu_scale > 0 and not want_stats:
+        out = native_packed(input, deformation, weight, bias, lead, mask_activation, stride, padding, dilation, groups,
+                            offset_groups, mode, size_activation, offset_axes, backward_flags)
+        if out is not None:
+            return out
     K = weight.shape[2] * weight.shape[3] * weight.shape[4]
     GK = offset_groups * K
     if deformation.dim() != 5 or deformation.shape[1] != lead + GK:
@@ -639,6 +702,9 @@ class _PlainConv3dFunction(torch.autograd.Function):
 
 def plain_conv3d(input, weight, bias, stride, padding, dilation):
     """The ordinary convolution conv3d(input, weight, bias, stride, padding, dilation) where plain_conv3d_supported."""
+    out = _try_native("plain_conv3d", input, weight, bias, stride, padding, dilation)
+    if out is not None:
+        return out
     return _PlainConv3dFunction.apply(input, weight, bias, tuple(stride), tuple(padding), tuple(dilation))
 
 
@@ -771,6 +837,10 @@ def deform_conv1d(input, offset, alpha, weight, bias, stride, pad, dilation, gro
     takes plain ints and defined tensors only, 1-tuples for stride / pad /
     dilation and None for `alpha` / `bias` are accepted (DeformConv1d.forward,
     deform_conv.py:168-172, passes exactly those)."""
+    out = _try_native("conv1d", input, offset, alpha, weight, bias, _one(stride), _one(pad), _one(dilation), groups, offset_groups,
+                      bool(reference_quirks))
+    if out is not None:
+        return out
     _check_common(1, input, offset, alpha, weight, bias, groups, offset_groups)
     input, offset, alpha, weight, bias = _unify(input, offset, alpha, weight, bias)
     return _DeformConv1dFunction.apply(

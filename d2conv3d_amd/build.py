@@ -1,9 +1,9 @@
-"""Builds libd2conv.so (the C-ABI HIP library) for gfx950 with hipcc.
+"""Builds libd2conv.so (the C-ABI HIP library) for gfx950 with hipcc, and _native.so (its torch binding) with g++.
 
     python -m d2conv3d_amd.build [--force]
 
 Each csrc/*.hip is compiled to an object under csrc/build/ and the objects are
-linked into d2conv3d_amd/libd2conv.so.  No torch headers are involved.
+linked into d2conv3d_amd/libd2conv.so; no torch headers are involved there.
 """
 import concurrent.futures
 import glob
@@ -61,5 +61,31 @@ def build_library(force=False, jobs=8):
     return LIB
 
 
+NATIVE_SRC = os.path.join(CSRC, "torch", "native.cpp")
+NATIVE = os.path.join(HERE, "_native.so")
+
+
+def build_native(force=False):
+    """The torch binding (host code only), linked to the library beside it."""
+    if not (force or _newer(NATIVE_SRC, NATIVE, [os.path.join(HERE, "..", "include", "d2conv.h")])):
+        return NATIVE
+    import sysconfig
+    import torch
+    root = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(HIPCC)))
+    if not os.path.exists(os.path.join(rocm, "include", "hip")):
+        rocm = "/opt/rocm"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include", f"-I{rocm}/include", f"-I{sysconfig.get_paths()['include']}",
+           NATIVE_SRC, "-o", NATIVE, f"-L{root}/lib", "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip", f"-L{HERE}",
+           "-ld2conv", f"-L{rocm}/lib", "-lamdhip64", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed for {NATIVE_SRC}:\n{r.stderr}")
+    return NATIVE
+
+
 if __name__ == "__main__":
     print(build_library(force="--force" in sys.argv))
+    print(build_native(force="--force" in sys.argv))

@@ -72,7 +72,8 @@ def deform_conv1d(input, offset, alpha, weight, bias=None, stride=1, padding=0, 
                   n_weight_groups=1, n_offset_groups=1):
     """deform_conv.py:19-40.  `alpha=None` means no modulation and `bias=None`
     no bias (the reference materialises ones / zeros for them, :30-35)."""
-    input, offset, alpha, weight, bias = _upcast_half(input, offset, alpha, weight, bias)
+    if _any_half_inputs(input, offset, alpha, weight, bias):
+        input, offset, alpha, weight, bias = _upcast_half(input, offset, alpha, weight, bias)
     return _ops.deform_conv1d(input, offset, alpha, weight, bias, stride, padding, dilation,
                               n_weight_groups, n_offset_groups)
 
@@ -103,6 +104,12 @@ def deform_conv3d(input, offset, alpha, weight, bias=None, stride=(1, 1, 1), pad
              "resample": _lib.BWD_GW_RESAMPLE}[backward_memory] | _lib.bwd_slices(backward_slices)
     if backward_f32_split:
         flags |= _lib.BWD_F32_SPLIT
+    if not output_relu and not output_stats and prepared is None:
+        # (what the rest of this function prepares is for other calls than those that the native code takes)
+        out = _ops._try_native("conv3d", input, offset, alpha, weight, bias, _triple(stride), _triple(padding), _triple(dilation),
+                               n_weight_groups, n_offset_groups, offset_axes, flags, _ops._keep_max())
+        if out is not None:
+            return out
     input, offset, alpha, weight, bias = _upcast_half(input, offset, alpha, weight, bias)
     stride_d, stride_h, stride_w = _triple(stride)
     pad_d, pad_h, pad_w = _triple(padding)
@@ -132,6 +139,13 @@ def deform_conv3d_sized(input, size_map, alpha, weight, bias=None, mode="xyz", s
     with one offset group, but the tap offsets are formed inside the sampler from the raw size prediction
     `size_map` [N, 3|2|2|1, Do, Ho, Wo] (mode "xyz" | "xxz" | "xy" | "x"); its gradient comes back in that shape.
     Half inputs are up-cast like in deform_conv3d."""
+    if input.is_cuda and input.dtype != torch.half and not output_relu and not output_stats and mode.lower() in _ops._SIZE_CHANNELS:
+        triples = tuple(_triple(t) for t in (stride, padding, dilation))
+        out = _ops._try_native("conv3d_sized", input, size_map, alpha, weight, bias,
+                               _ops._size_template(mode.lower(), tuple(weight.shape[2:]), triples[2], size_activation),
+                               _ops._SIZE_CHANNELS[mode.lower()], *triples, n_weight_groups, _ops._keep_max())
+        if out is not None:
+            return out
     input, size_map, alpha, weight, bias = _upcast_half(input, size_map, alpha, weight, bias)
     # (the size map has the spatial shape of the offsets it stands for, which is all the question needs of it)
     input, size_map, alpha, weight, bias, rounded = _float32_for_unchunked_bfloat16(

@@ -16,7 +16,7 @@ import torch.nn.functional as F
 from torch.nn.modules.utils import _triple
 
 from . import _lib
-from ._ops import _DT, _ptr, _stream
+from ._ops import _DT, _ptr, _stream, _try_native
 
 
 def _check(cond, msg):
@@ -110,6 +110,9 @@ def depthwise_separable_conv3d(input, weight, bias, stride, padding, dilation):
     they are (sums in float32 / float64); float16, which the reference computes in half with float sums
     (csrc/grouped_conv3d.cu:419), is computed in float32 and returned as float16."""
     stride, padding, dilation = _triple(stride), _triple(padding), _triple(dilation)
+    out = _try_native("dwconv3d", input, weight, bias, stride, padding, dilation)
+    if out is not None:
+        return out
     if input.dtype == torch.float16:
         out = _DepthwiseConv3dFunction.apply(input.float(), weight.float(), None if bias is None else bias.float(),
                                              stride, padding, dilation)

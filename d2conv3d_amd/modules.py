@@ -71,6 +71,10 @@ def _branch_conv(layer, x):
         from . import _ops
         from .deform_conv import deform_conv3d
         k, s, p, d = conv.kernel_size, conv.stride, conv.padding, conv.dilation
+        if x.dtype == torch.bfloat16:
+            out = _ops._try_native("plain_conv3d", x, conv.weight, conv.bias, s, p, d)
+            if out is not None:
+                return out
         dims = tuple((x.shape[2 + i] + 2 * p[i] - d[i] * (k[i] - 1) - 1) // s[i] + 1 for i in range(3))
         if (min(dims) > 0 and x.dtype == torch.bfloat16 and (conv.bias is None or conv.bias.dtype == x.dtype)
                 and _ops.plain_conv3d_supported(x, conv.weight, s, p, d)):
@@ -166,6 +170,12 @@ def _deformation_tensor(layer, input):
     return _branch_conv(layer, deform_input)
 
 
+def _backward_flags(dc):
+    from . import _lib
+    return {"default": _lib.BWD_GW_DEFAULT, "columns": _lib.BWD_GW_COLUMNS, "in_place": _lib.BWD_GW_IN_PLACE,
+            "resample": _lib.BWD_GW_RESAMPLE}[dc.backward_memory] | _lib.bwd_slices(dc.backward_slices)
+
+
 def _packed_forward(layer, input, deformation, lead, mode=None, offset_axes=7):
     """The operator on the un-split output of the deformation branch (`lead` channels of offsets or of the raw size
     map, then the raw modulation values): the kernels read both parts where they lie and apply the modulation
@@ -174,17 +184,19 @@ def _packed_forward(layer, input, deformation, lead, mode=None, offset_axes=7):
     from . import _ops
     dc = layer.deform_conv
     name = layer._activation_name
+    if name is not None and not dc.output_relu_scale and not dc.keep_output_stats:
+        out = _ops.native_packed(input, deformation, dc.weight, dc.bias, lead, name, dc.stride, dc.padding, dc.dilation, dc.groups,
+                                 dc.offset_groups, mode, layer.size_activation, offset_axes, _backward_flags(dc))
+        if out is not None:
+            return out
     if name is None or not _ops.deform_conv3d_packed_supported(input, deformation, dc.weight, lead, name, mode,
                                                              layer.size_activation, dc.stride, dc.padding, dc.dilation,
                                                              dc.groups, dc.offset_groups, offset_axes):
         return None
-    from . import _lib
-    flags = {"default": _lib.BWD_GW_DEFAULT, "columns": _lib.BWD_GW_COLUMNS, "in_place": _lib.BWD_GW_IN_PLACE,
-             "resample": _lib.BWD_GW_RESAMPLE}[dc.backward_memory] | _lib.bwd_slices(dc.backward_slices)
     out = _ops.deform_conv3d_packed(input, deformation, dc.weight, dc.bias, lead, name, dc.stride, dc.padding,
                                     dc.dilation, dc.groups, dc.offset_groups, mode, layer.size_activation,
                                     float(dc.output_relu_scale) if dc.output_relu_scale else 0.0, dc.keep_output_stats,
-                                    offset_axes, flags)
+                                    offset_axes, _backward_flags(dc))
     if dc.keep_output_stats:
         out, dc.last_output_stats = out
     return out
