@@ -20,7 +20,7 @@ EXPORTS = (
     "d2c_conv3d_forward_workspace_bytes", "d2c_conv3d_backward_workspace_bytes",
     "d2c_conv3d_forward", "d2c_conv3d_backward", "d2c_conv3d_forward_static", "d2c_static_workspace_bytes",
     "d2c_conv3d_prepared_bytes", "d2c_conv3d_forward_prepared", "d2c_conv3d_backward_prepared",
-    "d2c_conv3d_columns_bytes", "d2c_conv3d_forward_columns", "d2c_conv3d_backward_columns_workspace_bytes",
+    "d2c_conv3d_columns_bytes", "d2c_conv3d_keep_bytes", "d2c_conv3d_forward_columns", "d2c_conv3d_backward_columns_workspace_bytes",
     "d2c_conv3d_backward_columns",
     "d2c_plain_conv3d_input_bytes", "d2c_plain_conv3d_forward_workspace_bytes",
     "d2c_plain_conv3d_backward_workspace_bytes", "d2c_plain_conv3d_forward", "d2c_plain_conv3d_backward",
@@ -136,6 +136,7 @@ def load():
     lib.d2c_conv3d_backward_prepared.restype = ctypes.c_int
     # (the second argument: a pointer to a size-map description, or None)
     lib.d2c_conv3d_columns_bytes.argtypes, lib.d2c_conv3d_columns_bytes.restype = [p3, vp], sz
+    lib.d2c_conv3d_keep_bytes.argtypes, lib.d2c_conv3d_keep_bytes.restype = [p3, vp], sz
     lib.d2c_conv3d_backward_columns_workspace_bytes.argtypes = [p3, vp]
     lib.d2c_conv3d_backward_columns_workspace_bytes.restype = sz
     lib.d2c_conv3d_forward_columns.argtypes = [p3, vp] + [vp] * 6 + [vp, sz, vp, sz, vp]

@@ -183,7 +183,7 @@ def _set_keep_columns(on=True, max_bytes=None):
 def _columns_for(lib, desc, sdesc, weight_grad_wanted, dev):
     if not (_KEEP_COLUMNS["on"] and weight_grad_wanted):
         return None
-    n = lib.d2c_conv3d_columns_bytes(ctypes.byref(desc), ctypes.byref(sdesc) if sdesc is not None else None)
+    n = lib.d2c_conv3d_keep_bytes(ctypes.byref(desc), ctypes.byref(sdesc) if sdesc is not None else None)
     if n == 0 or n > _KEEP_COLUMNS["max_bytes"]:
         return None
     try:

@@ -681,6 +681,12 @@ size_t d2c_conv3d_columns_bytes(const d2c_conv3d_desc *q, const d2c_size_map_des
     return columns_served(*q, z) ? d2c_tiled_columns_bytes(*q, z) : 0;
 }
 
+size_t d2c_conv3d_keep_bytes(const d2c_conv3d_desc *q, const d2c_size_map_desc *z)
+{
+    if ((z ? sized_check(q, z) : d2c_conv3d_check(q)) != D2C_OK) return 0;
+    return columns_served(*q, z) ? d2c_tiled_keep_bytes(*q, z) : 0;
+}
+
 static int check_columns(const d2c_conv3d_desc &q, const d2c_size_map_desc *z, const void *columns, size_t columns_bytes)
 {
     const size_t need = columns_served(q, z) ? d2c_tiled_columns_bytes(q, z) : 0;
@@ -703,7 +709,8 @@ int d2c_conv3d_forward_columns(const d2c_conv3d_desc *q, const d2c_size_map_desc
     if (!x || !offset || !weight || !out) { d2c_set_error("null tensor pointer"); return D2C_ERR_SHAPE; }
     if (int rc = check_columns(*q, z, columns, columns_bytes)) return rc;
     if (int rc = check_ws(d2c_tiled_forward_ws(*q), ws, ws_bytes)) return rc;
-    return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, (hipStream_t)stream, z, nullptr, nullptr, columns);
+    return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, (hipStream_t)stream, z, nullptr, nullptr, columns,
+                             columns_bytes);
 }
 
 size_t d2c_conv3d_backward_columns_workspace_bytes(const d2c_conv3d_desc *q, const d2c_size_map_desc *z)
@@ -722,7 +729,7 @@ int d2c_conv3d_backward_columns(const d2c_conv3d_desc *q, const d2c_size_map_des
     if (int rc = check_columns(*q, z, columns, columns_bytes)) return rc;
     if (int rc = check_ws(d2c_tiled_backward_ws(*q, z, true), ws, ws_bytes)) return rc;
     return d2c_tiled_backward(*q, gout, x, offset, mask, weight, gx, goff, gmask, gw, gb, ws, (hipStream_t)stream, z,
-                              nullptr, columns);
+                              nullptr, columns, columns_bytes);
 }
 
 int d2c_conv3d_corner_index(const d2c_conv3d_desc *q, const void *offset, int32_t *base, uint8_t *flags,

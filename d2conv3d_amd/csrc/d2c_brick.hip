@@ -12,7 +12,6 @@
 // gathered: a grad-column row is read once, for both results, and a brick's input rows stay in LDS.  (The kernels
 // that gather -- eight corner rows per point through the L1, grad-column rows 3.4 times -- took 1.73 + 1.47 ms for
 // 256 channels on 32x60x108, bound by the L1 path, the vector ALU and row latency.)
-#include <utility>
 
 #include "d2c_mma.hpp"
 #include "d2c_tiled.hpp"
@@ -21,11 +20,6 @@
 namespace {
 
 typedef short v4s __attribute__((ext_vector_type(4)));
-
-template <class F, int... I> D2C_DEV void for_each_const(F &&f, std::integer_sequence<int, I...>)
-{
-    (f(std::integral_constant<int, I>{}), ...);
-}
 
 // One sampling point as the sort sees it.
 struct BrickPoint {
@@ -122,6 +116,20 @@ brick_count_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, int
         if (p < s.P && k0 + i < s.K)
             L.place[((long)bg * s.K + k0 + i) * s.P + p] = pt[i] == ~0u ? -1 : s_cnt[pt[i] >> 16] + (int)(pt[i] & 0xffffu);
 }
+// Few points: one global addition each.  (62 000 points: 5 us, the table 17 us; 700 000: 27 and 20 us.)
+template <bool AUX16, bool SIZED>
+__global__ void __launch_bounds__(256)
+brick_count_few_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, int ngrp)
+{
+    const int u = blockIdx.x, npb = (s.P + 255) / 256, bgk = u / npb, bg = bgk / s.K, k = bgk - bg * s.K, b = bg / s.G, g = bg - b * s.G;
+    const int p = (u - bgk * npb) * 256 + threadIdx.x;
+    if (p >= s.P) return;
+    float c[3];
+    tap_offsets_issue<AUX16, SIZED>(s, off, b, g, k, p, c);
+    const BrickPoint q = brick_point<AUX16, SIZED>(s, d, c, b, g, k, p);
+    L.place[((long)bg * s.K + k) * s.P + p] = q.in ? atomicAdd(&L.count[q.seg], 1) : -1;
+}
+constexpr long kFewPoints = 400000;
 // (the order of the ranges does not matter: a wavefront adds up its 64 counts and takes one range for all)
 __global__ void __launch_bounds__(256) brick_range_kernel(BrickLists L, int nseg)
 {
@@ -141,7 +149,7 @@ __global__ void __launch_bounds__(256) brick_range_kernel(BrickLists L, int nseg
 // (all taps of a position in one workgroup: the places a workgroup's points were given in a block follow each other)
 template <bool AUX16, bool SIZED>
 __global__ void __launch_bounds__(256)
-brick_file_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, const void *mask, int ngrp)
+brick_file_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, const void *mask, int ngrp, long n)
 {
     typedef typename std::conditional<AUX16, bf16_t, float>::type AT;
     const PointUnit un = point_unit(s, ngrp);
@@ -171,6 +179,27 @@ brick_file_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, cons
         L.pt[at] = make_uint4((unsigned)((k0 + i) * s.M + b * s.P + p) * 128u, __float_as_uint(q[i].y), __float_as_uint(q[i].x),
                               __float_as_uint(q[i].hz));
         L.alpha[at] = (mask && s.mact) ? mask_act<AT>(s.mact, al[i]) : al[i];
+    }
+    // points outside the volume: their rows among all groups' rows, listed downwards from the end of the entries (which the
+    // points inside leave free), one addition to the counter per wavefront
+    unsigned long long m[kTaps];
+    int total = 0;
+#pragma unroll
+    for (int i = 0; i < kTaps; i++) {
+        m[i] = __ballot(rank[i] < 0 && k0 + i < s.K);
+        total += __popcll(m[i]);
+    }
+    if (total == 0) return;
+    const int lane = threadIdx.x & 63;
+    int at = 0;
+    if (lane == 0) at = atomicAdd(L.cursor + 1, total);
+    at = __builtin_amdgcn_readfirstlane(at);
+    unsigned *const end = reinterpret_cast<unsigned *>(L.pt + n) - 1;
+#pragma unroll
+    for (int i = 0; i < kTaps; i++) {
+        if (rank[i] < 0 && k0 + i < s.K)
+            end[-(long)(at + __popcll(m[i] & ((1ull << lane) - 1)))] = (unsigned)((g * s.K + k0 + i) * s.M + b * s.P + p);
+        at += __popcll(m[i]);
     }
 }
 
@@ -207,7 +236,6 @@ D2C_DEV void wave_fence() { asm volatile("" ::: "memory"); __builtin_amdgcn_wave
 
 __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs a, const int *__restrict__ seg_start, const int *__restrict__ seg_count)
 {
-#define INLINE __attribute__((always_inline))
     const int lane = threadIdx.x & 63, h = lane >> 5, n = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
     // A wavefront's grad-column rows of 32 points x 64 channels, and their weights [term][point][voxel of 32].  16-byte pieces of a row are
@@ -457,7 +485,181 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
         if (want_gx) flush_plane(z);
     }
     if (want_gx) flush_plane(zi_hi - 1);
-#undef INLINE
+}
+
+// ---- sampled columns ------------------------------------------------------------------------------------------------
+// col[chunk][tap][rows][64] = modulation * interpolated input of every point (rows: N*P and a few): x^T[64 channels, 32 voxels] * W[32 voxels, 32
+// points], two bfloat16 terms of the weights.  W is made by the lanes that hold the points, in the operand's own order
+// (lane = point, half h of the wavefront: the voxels of rows y = 2h, 2h + 1 of each plane); the brick's input is kept as
+// the other operand, one plane changed per step in z.  Rows leave whole, through LDS.  Bound by the rows it writes:
+// 5.6 M points x 256 channels (32x60x108, 27 taps), 2.9 GB: 700 us (the whole forward pass: 2.3 ms gathering, 1.7 ms sorted).
+// (Workgroups as in brick_grad_kernel: a column of bricks, a wavefront per chunk.)
+struct BrickSampleArgs {
+    BrickDims d;
+    BrickLists L;
+    const bf16_t *xcl;       // [N][vol][Cin]
+    bf16_t *col;
+    int zlen, nzr, nset, G, cpc, Cin, D, H, W, vol;
+    long chunk_rows;         // K * rows of a tap
+    int K, rows, pad;        // taps; rows of a tap, those beyond N*P
+    int M, nzero;            // N*P; workgroups in front that clear rows
+    long npoint;
+    FastDiv dM, dKM;
+};
+__global__ void __launch_bounds__(64 * kMaxWaves, 4) brick_sample_kernel(BrickSampleArgs a, const int *__restrict__ seg_start, const int *__restrict__ seg_count)
+{
+    const int lane = threadIdx.x & 63, h = lane >> 5, n = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+    __shared__ __align__(16) unsigned char s_all[kMaxWaves][32 * 128];
+    unsigned char *const s_r = s_all[wave];                          // a plane's 16 input rows; 32 rows on their way out
+    const int pv = lane >> 3, pc = lane & 7;
+    if ((int)blockIdx.x < a.nzero) {
+        // rows of the points outside the volume, and those behind the last position: zeros (8 lanes to a chunk's row)
+        const int w = (int)blockIdx.x * nw + wave, nwave = a.nzero * nw, nout = a.L.cursor[1];
+        const unsigned *const end = reinterpret_cast<const unsigned *>(a.L.pt + a.npoint) - 1;
+        for (int o0 = w * 64; o0 < nout; o0 += nwave * 64) {
+            const unsigned e = o0 + lane < nout ? end[-(long)(o0 + lane)] : 0u;
+            for (int i = 0; i < 64 && o0 + i < nout; i += 8) {
+                const int o = __builtin_amdgcn_ds_bpermute((i + pv) << 2, (int)e);
+                if (o0 + i + pv >= nout) continue;
+                const int g = fdiv(o, a.dKM), r = o - g * (a.K * a.M), row = r + fdiv(r, a.dM) * a.pad;
+                for (int c = 0; c < a.cpc; c++)
+                    reinterpret_cast<uint4 *>(a.col + ((long)(g * a.cpc + c) * a.chunk_rows + row) * 64)[pc] = make_uint4(0, 0, 0, 0);
+            }
+        }
+        const int tails = a.G * a.cpc * a.K * a.pad;
+        for (int i = w * 8 + pv; i < tails; i += nwave * 8) {
+            const int t = i / a.pad;
+            reinterpret_cast<uint4 *>(a.col + ((long)t * a.rows + a.M + (i - t * a.pad)) * 64)[pc] = make_uint4(0, 0, 0, 0);
+        }
+        return;
+    }
+    const int bid = (int)blockIdx.x - a.nzero, nt = (int)gridDim.x - a.nzero, xq = nt >> 3, xr = nt & 7, xcd = bid & 7;
+    int t = xcd * xq + (xcd < xr ? xcd : xr) + (bid >> 3);
+    const int set = t % a.nset; t /= a.nset;
+    const int bx = t % a.d.nbx; t /= a.d.nbx;
+    const int by = t % a.d.nby; t /= a.d.nby;
+    const int zr = t % a.nzr; const int bg = t / a.nzr;
+    const int b = bg / a.G, g = bg - b * a.G;
+    if (set * nw + wave >= a.cpc) return;
+    const int cc0 = g * a.cpc + set * nw + wave;
+    const int y0 = by * 3 - 1, x0 = bx * 3 - 1;
+    const int zi_lo = zr * a.zlen, zi_hi = min(zi_lo + a.zlen, a.d.nz);
+
+    uint4 pl[2];
+    auto load_plane = [&](int z) INLINE {
+        for_each_const([&](auto I) INLINE {
+            constexpr int i = decltype(I)::value;
+            const int v = i * 8 + pv, y = y0 + (v >> 2), x = x0 + (v & 3);
+            pl[i] = make_uint4(0, 0, 0, 0);
+            if (z >= 0 && z < a.D && y >= 0 && y < a.H && x >= 0 && x < a.W)
+                pl[i] = *reinterpret_cast<const uint4 *>(a.xcl + ((long)b * a.vol + ((long)z * a.H + y) * a.W + x) * a.Cin + cc0 * 64 + pc * 8);
+        }, std::make_integer_sequence<int, 2>{});
+    };
+    // the plane as matrix operand: lane = channel, 8 voxels (half h: y = 2h, 2h + 1).  The channel of a lane is the one that
+    // makes a lane of the result hold 16 consecutive channels of its point: row m of the operand = channel
+    // 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3).
+    const int q4 = ((lane >> 4) & 1) * 4 + (lane & 3), ch = (q4 & 1) * 16 + (q4 >> 1) * 4;
+    const unsigned p_tr = lds_address(s_r) + (h * 8 + ((lane & 15) >> 2)) * 128 + ch * 2;
+    auto tr_read = [](unsigned addr) INLINE {
+        return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s *)(size_t)addr));
+    };
+    bf16x8_t xl[2], xh[2];                                           // [channels 0-31, 32-63] of the lower and the upper plane
+    auto take_plane = [&]() INLINE {
+        for_each_const([&](auto I) INLINE {
+            constexpr int i = decltype(I)::value;
+            *reinterpret_cast<uint4 *>(s_r + (i * 8 + pv) * 128 + pc * 16) = pl[i];
+        }, std::make_integer_sequence<int, 2>{});
+        wave_fence();
+        for_each_const([&](auto C) INLINE {
+            constexpr int c = decltype(C)::value;
+            const uint2 lo = tr_read(p_tr + c * 64), hi = tr_read(p_tr + c * 64 + 512);
+            xh[c] = __builtin_bit_cast(bf16x8_t, make_uint4(lo.x, lo.y, hi.x, hi.y));
+        }, std::make_integer_sequence<int, 2>{});
+        wave_fence();
+    };
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc(a.col + (long)cc0 * a.chunk_rows * 64, 0, (int)(unsigned)(a.chunk_rows * 128), 0x00020000);
+    constexpr unsigned kNone = 0xFFFFFFF0u;
+    // rows on their way out: written 16 bytes a time by the lane of the point, read 8 lanes to a row; pieces permuted against
+    // bank conflicts (16 lanes on one piece of 16 rows)
+    const int swz = (n >> 1) & 7;
+
+    auto range = [&](int zi, int &lo, int &cnt) INLINE {
+        const int sg = brick_seg(a.d, bg, min(zi, zi_hi - 1), by, bx);
+        lo = __builtin_amdgcn_readfirstlane(seg_start[sg]); cnt = __builtin_amdgcn_readfirstlane(seg_count[sg]);
+    };
+    uint4 e0, e1;
+    float a0, a1;
+    auto entry = [&](int lo, int cnt, int i, uint4 &q, float &al) INLINE {
+        const int e = max(lo + min(i + n, cnt - 1), 0);
+        q = a.L.pt[e]; al = a.L.alpha[e];
+    };
+    int lo, cnt;
+    range(zi_lo, lo, cnt);
+    load_plane(zi_lo - 1);
+    entry(lo, cnt, 0, e0, a0);
+    take_plane();
+    load_plane(zi_lo);
+    for (int zi = zi_lo; zi < zi_hi; zi++) {
+        xl[0] = xh[0]; xl[1] = xh[1];
+        take_plane();
+        int nlo, ncnt;
+        range(zi + 1, nlo, ncnt);
+        load_plane(zi + 1);
+        for (int i0 = 0; i0 < cnt; i0 += 32) {
+            // (the next entries: of this block, or the first of the next plane's)
+            if (i0 + 32 < cnt) entry(lo, cnt, i0 + 32, e1, a1);
+            else entry(nlo, ncnt, 0, e1, a1);
+            const float py = __uint_as_float(e0.y), px = __uint_as_float(e0.z), hz = __uint_as_float(e0.w);
+            const float wlo = a0 * (1.f - hz), whi = a0 * hz;
+            float tx[4], ty[2];
+#pragma unroll
+            for (int i = 0; i < 4; i++) tx[i] = __builtin_amdgcn_fmed3f(1.f - fabsf((float)i - px), 0.f, 1.f);
+            const float yb = py - (float)(2 * h);
+#pragma unroll
+            for (int i = 0; i < 2; i++) ty[i] = __builtin_amdgcn_fmed3f(1.f - fabsf((float)i - yb), 0.f, 1.f);
+            f32x16 r0, r1;
+#pragma unroll
+            for (int r = 0; r < 16; r++) r0[r] = r1[r] = 0.f;
+            for_each_const([&](auto S) INLINE {
+                constexpr int slot = decltype(S)::value;
+                uint32_t wh[4], wl[4];
+#pragma unroll
+                for (int j = 0; j < 8; j += 2) {
+                    const float t2 = ty[j / 4] * (slot ? whi : wlo), w0 = t2 * tx[j & 3], w1 = t2 * tx[(j & 3) + 1];
+                    wh[j / 2] = pack_bf16x2(w0, w1);
+                    wl[j / 2] = pack_bf16x2(w0 - __uint_as_float(wh[j / 2] << 16), w1 - __uint_as_float(wh[j / 2] & 0xffff0000u));
+                }
+                const bf16x8_t bh = __builtin_bit_cast(bf16x8_t, make_uint4(wh[0], wh[1], wh[2], wh[3]));
+                const bf16x8_t bl = __builtin_bit_cast(bf16x8_t, make_uint4(wl[0], wl[1], wl[2], wl[3]));
+                r0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(slot ? xh[0] : xl[0], bh, r0, 0, 0, 0);
+                r1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(slot ? xh[1] : xl[1], bh, r1, 0, 0, 0);
+                r0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(slot ? xh[0] : xl[0], bl, r0, 0, 0, 0);
+                r1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(slot ? xh[1] : xl[1], bl, r1, 0, 0, 0);
+            }, std::make_integer_sequence<int, 2>{});
+            for_each_const([&](auto P) INLINE {
+                constexpr int q = decltype(P)::value, c = q >> 1, r = (q & 1) * 8;      // channels 32 c + 16 h + r ..
+                const f32x16 &v = c ? r1 : r0;
+                *reinterpret_cast<uint4 *>(s_r + n * 128 + (((c * 4 + h * 2 + (q & 1)) ^ swz) << 4)) =
+                    make_uint4(pack_bf16x2(v[r], v[r + 1]), pack_bf16x2(v[r + 2], v[r + 3]), pack_bf16x2(v[r + 4], v[r + 5]),
+                               pack_bf16x2(v[r + 6], v[r + 7]));
+            }, std::make_integer_sequence<int, 4>{});
+            wave_fence();
+            const unsigned to = e0.x + (unsigned)(fdiv((int)(e0.x >> 7), a.dM) * a.pad) * 128u;      // (the entry counts N*P rows per tap)
+            for_each_const([&](auto I) INLINE {
+                constexpr int i = decltype(I)::value;
+                const int row = i * 8 + pv;
+                const u32x4_t v = *reinterpret_cast<const u32x4_t *>(s_r + row * 128 + ((pc ^ ((row >> 1) & 7)) << 4));
+                const unsigned o = (unsigned)__builtin_amdgcn_ds_bpermute(row << 2, (int)to) + pc * 16;
+                __builtin_amdgcn_raw_buffer_store_b128(v, rs, i0 + row < cnt ? (int)o : (int)kNone, 0, 2);
+            }, std::make_integer_sequence<int, 4>{});
+            wave_fence();
+            e0 = e1; a0 = a1;
+        }
+        // (a plane without points has asked for nothing: the next one's entries)
+        if (cnt == 0) entry(nlo, ncnt, 0, e0, a0);
+        lo = nlo; cnt = ncnt;
+    }
 }
 
 // ---- per-point sums -> gradients in their storage type and layout --------------------------------------------------
@@ -575,20 +777,20 @@ bool d2c_brick_supported(const TiledShape &s, int dtype)
     if (s.nd != 3 || dtype != D2C_BF16 || s.cpg % 64) return false;
     const double mean = 9.0 * s.K * s.P / s.vol;
     return mean >= 16.0 && s.K <= 65535 && (long)s.N * s.G <= 65535 && brick_nseg(s) < (1L << 31) - 1024 &&
-           brick_points(s) < (1L << 31) - 64 && (size_t)s.K * s.M * 128 < 0xFFFFFF00u &&
+           brick_points(s) < (1L << 31) - 64 && (size_t)s.K * (s.M + 64) * 128 < 0xFFFFFF00u &&
            (size_t)s.H * s.W * s.Cin * 4 < 0xFFFFFFF0u;
 }
 BrickWs d2c_brick_ws(const TiledShape &s)
 {
     const size_t n = (size_t)brick_points(s), nseg = (size_t)brick_nseg(s);
     BrickWs w;
-    w.count = 0;                                                   // [nseg] counts, then the cursor: one clear
-    w.start = d2c_align_up((nseg + 1) * 4);
+    w.count = 0;                                                   // [nseg] counts, then the cursor and the number of points outside: one clear
+    w.start = d2c_align_up((nseg + 2) * 4);
     w.place = w.start + d2c_align_up(nseg * 4);
     w.pt = w.place + d2c_align_up(n * 4);
     w.alpha = w.pt + d2c_align_up(n * 16);
-    w.res = w.alpha + d2c_align_up(n * 4);
-    w.total = w.res + d2c_align_up(n * 16) * brick_sets(s);
+    w.total = w.alpha + d2c_align_up(n * 4);
+    w.res_bytes = d2c_align_up(n * 16) * brick_sets(s);
     return w;
 }
 
@@ -599,14 +801,17 @@ int d2c_brick_sort(const TiledShape &s, const void *off, const void *mask, void 
     const BrickDims d = brick_dims(s);
     const BrickLists L = brick_lists(s, (char *)ws);
     const int nseg = (int)brick_nseg(s);
-    d2c_fill_zero(L.count, ((size_t)nseg + 1) * 4, st);
+    d2c_fill_zero(L.count, ((size_t)nseg + 2) * 4, st);
     const int ngrp = (s.K + kTaps - 1) / kTaps;
     const dim3 grid((unsigned)((long)((s.P + 255) / 256) * ngrp * s.N * s.G)), blk(256);
     auto go = [&](auto A, auto Z) {
         constexpr bool A16 = decltype(A)::value, SZ = decltype(Z)::value;
-        hipLaunchKernelGGL((brick_count_kernel<A16, SZ>), grid, blk, 0, st, s, d, L, off, ngrp);
+        if (brick_points(s) <= kFewPoints)
+            hipLaunchKernelGGL((brick_count_few_kernel<A16, SZ>), dim3((unsigned)((long)((s.P + 255) / 256) * s.K * s.N * s.G)), blk, 0, st, s, d, L,
+                               off, ngrp);
+        else hipLaunchKernelGGL((brick_count_kernel<A16, SZ>), grid, blk, 0, st, s, d, L, off, ngrp);
         hipLaunchKernelGGL(brick_range_kernel, dim3((nseg + 255) / 256), blk, 0, st, L, nseg);
-        hipLaunchKernelGGL((brick_file_kernel<A16, SZ>), grid, blk, 0, st, s, d, L, off, mask, ngrp);
+        hipLaunchKernelGGL((brick_file_kernel<A16, SZ>), grid, blk, 0, st, s, d, L, off, mask, ngrp, brick_points(s));
     };
     if (s.adt == D2C_BF16) {
         if (s.ss.on) go(std::true_type{}, std::true_type{});
@@ -620,14 +825,13 @@ int d2c_brick_sort(const TiledShape &s, const void *off, const void *mask, void 
 
 // `gxcl` (cleared here), `goff` (size-map source: the gradient of the raw map `raw`) and `gmask` may be NULL.
 int d2c_brick_grad(const TiledShape &s, const void *xcl, const void *gcol, const void *mask, const void *raw, float *gxcl,
-                   void *goff, void *gmask, void *ws, hipStream_t st)
+                   void *goff, void *gmask, const void *lists, void *res, hipStream_t st)
 {
-    const BrickWs w = d2c_brick_ws(s);
     const long n = brick_points(s);
     BrickArgs a{};
-    a.d = brick_dims(s); a.L = brick_lists(s, (char *)ws);
+    a.d = brick_dims(s); a.L = brick_lists(s, (char *)const_cast<void *>(lists));
     a.xcl = (const bf16_t *)xcl; a.gcol = (const bf16_t *)gcol; a.gxcl = gxcl;
-    a.res = (goff || gmask) ? (float2 *)((char *)ws + w.res) : nullptr;
+    a.res = (goff || gmask) ? (float2 *)res : nullptr;
     a.nres = (long)(d2c_align_up((size_t)n * 16) / 16);
     a.G = s.G; a.cpc = s.cpg / 64; a.Cin = s.Cin; a.D = s.D; a.H = s.H; a.W = s.W; a.vol = s.vol;
     a.chunk_rows = (long)s.K * s.M;
@@ -663,4 +867,27 @@ int d2c_brick_grad(const TiledShape &s, const void *xcl, const void *gcol, const
                            goff, gmask, ngrp);
     }
     return d2c_check_launch("brick_finish_kernel");
+}
+
+// The sampled columns [chunk][tap][rows][64] of sorted points.
+int d2c_brick_columns(const TiledShape &s, const void *xcl, void *col, int rows, const void *lists, hipStream_t st)
+{
+    BrickSampleArgs a{};
+    a.d = brick_dims(s); a.L = brick_lists(s, (char *)const_cast<void *>(lists));
+    a.xcl = (const bf16_t *)xcl; a.col = (bf16_t *)col;
+    a.G = s.G; a.cpc = s.cpg / 64; a.Cin = s.Cin; a.D = s.D; a.H = s.H; a.W = s.W; a.vol = s.vol;
+    a.K = s.K; a.rows = rows; a.M = s.M; a.chunk_rows = (long)s.K * rows; a.pad = rows - s.M;
+    a.dM = make_fastdiv(s.M); a.dKM = make_fastdiv(s.K * s.M);
+    a.nset = brick_sets(s);
+    const int nw = (a.cpc + a.nset - 1) / a.nset;
+    const int ncu = d2c_num_cus();
+    const long cols = (long)a.d.nbx * a.d.nby * s.N * s.G * a.nset;
+    a.zlen = a.d.nz;
+    while (a.zlen > 1 && cols * ((a.d.nz + a.zlen - 1) / a.zlen) * nw < 64L * ncu) a.zlen = (a.zlen + 1) / 2;
+    a.nzr = (a.d.nz + a.zlen - 1) / a.zlen;
+    a.npoint = brick_points(s);
+    a.nzero = (int)std::min<long>(2048, (a.npoint + 511) / 512) / nw + 1;
+    D2cProfScope prof(D2C_PROF_BWD_AUX, st, "brick_sample_kernel");
+    hipLaunchKernelGGL(brick_sample_kernel, dim3((unsigned)(cols * a.nzr + a.nzero)), dim3(64 * nw), 0, st, a, a.L.start, a.L.count);
+    return d2c_check_launch("brick_sample_kernel");
 }

@@ -8,17 +8,19 @@ struct BrickDims {
 };
 struct BrickLists {
     int *count;              // points per block
-    int *cursor;             // entries given out
+    int *cursor;             // entries given out, then: points outside the volume
     int *start;              // first entry of a block
     int *place;              // [n * G + g][tap][p]: a point's entry, -1: no corner inside the volume
     uint4 *pt;               // byte offset of the point's row of 64 channels, y and x inside the block, fraction along z
     float *alpha;            // modulation
 };
 struct BrickWs {
-    size_t count, start, place, pt, alpha, res, total;
+    size_t count, start, place, pt, alpha, total;     // the sorted points
+    size_t res_bytes;                                 // per-point sums of d2c_brick_grad
 };
 bool d2c_brick_supported(const TiledShape &s, int dtype);
 BrickWs d2c_brick_ws(const TiledShape &s);
 int d2c_brick_sort(const TiledShape &s, const void *off, const void *mask, void *ws, hipStream_t st);
 int d2c_brick_grad(const TiledShape &s, const void *xcl, const void *gcol, const void *mask, const void *raw, float *gxcl,
-                   void *goff, void *gmask, void *ws, hipStream_t st);
+                   void *goff, void *gmask, const void *lists, void *res, hipStream_t st);
+int d2c_brick_columns(const TiledShape &s, const void *xcl, void *col, int rows, const void *lists, hipStream_t st);

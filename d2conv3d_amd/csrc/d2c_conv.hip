@@ -4,7 +4,7 @@
 // at zero offsets interpolates eight and the backward pass goes through grad-column rows, sample lists and kept columns.
 //
 //   forward       out[o, m]   = bias[o] + sum_{tap, c} W[o, c, tap] * x[vox(m, tap), c]      conv_rows_kernel
-//   grad_input    gx[c, v]    = sum_{tap, o} W[o, c, tap] * gout[pos(v, tap), o]             conv_rows_kernel
+//   grad_input    gx[c, v]    = sum_{tap, o} W[o, c, tap] * gout[pos(v, tap), o]             ... and conv_wide_kernel
 //   grad_weight   gW[o, c, tap] = sum_m gout[o, m] * x[vox(m, tap), c]                       conv_weight_kernel
 //
 // (m: output positions over the whole batch, v: input voxels; a row that a tap puts outside the volume is a row of
@@ -21,6 +21,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kMT = 128;              // rows (positions) per workgroup of conv_rows_kernel
+constexpr int kWMT = 256;             // ... of conv_wide_kernel
 constexpr int kCW = 64;               // positions per step of conv_weight_kernel
 
 D2C_DEV int xcd_swizzle(int bid, int n)
@@ -134,9 +135,13 @@ struct ConvRowsArgs {
     int C;                            // columns that exist
     int nchunk, S;                    // KC-channel chunks per row, steps
     int ntile, nctile, nsplit;
+    // COLS: `src` is [chunk][tap][row][KC], a step's rows lie one after the other
+    int K, tap_rows;                  // taps, rows of a tap
+    int act;                          // epilogue (d2c_epilogue)
+    float act_scale;
 };
 
-template <int NT, int KC>
+template <int NT, int KC, bool COLS>
 __global__ void __launch_bounds__(kThreads, 2) conv_rows_kernel(ConvRowsArgs a)
 {
     constexpr int WO = NT == 128 ? 2 : 1, WP = 4 / WO;     // wavefronts along columns / rows
@@ -158,11 +163,23 @@ __global__ void __launch_bounds__(kThreads, 2) conv_rows_kernel(ConvRowsArgs a)
     const int m0 = tile * kMT;
 
     // --- rows this wavefront fetches: wave * 32 + (0 .. 31), lane l works out row l & 31
-    const RowPos rp = row_pos(a.map, m0 + wave * 32 + (lane & 31));
+    const RowPos rp = COLS ? RowPos{} : row_pos(a.map, m0 + wave * 32 + (lane & 31));
+    const unsigned char *asrc = a.src;                     // (COLS: the rows of the step)
+    const long tap_bytes = (long)a.tap_rows * ROWB;
     const int lrow = lane / VPR, lslot = lane % VPR;       // this lane's row within a request, its 16-byte slot
     unsigned aoff[AD], ainc[AD];
     int chunk = st_lo % a.nchunk, tap = st_lo / a.nchunk;
     auto tap_rows = [&](int k, int j) {
+        if constexpr (COLS) {
+            asrc = a.src + ((long)j * a.K + k) * tap_bytes;
+#pragma unroll
+            for (int i = 0; i < AD; i++) {
+                const int rl = i * RPD + lrow;
+                // (a tile's rows past the last one: the last one again, stored nowhere)
+                aoff[i] = (unsigned)min(m0 + wave * 32 + rl, a.map.N * a.map.P - 1) * ROWB + (unsigned)tile_slot<KC>(rl, lslot) * 16u;
+            }
+            return;
+        }
         const int kx = k % a.map.g.kw, ky = (k / a.map.g.kw) % a.map.g.kh, kz = k / (a.map.g.kw * a.map.g.kh);
         const int row = source_row(a.map, rp, kz, ky, kx);
 #pragma unroll
@@ -181,9 +198,10 @@ __global__ void __launch_bounds__(kThreads, 2) conv_rows_kernel(ConvRowsArgs a)
         unsigned char *sa = s_t + buf * STAGE + wave * (32 * ROWB), *sb = s_t + buf * STAGE + ABYTES;
 #pragma unroll
         for (int i = 0; i < AD; i++) {
-            dma16(a.src + aoff[i], sa + i * 1024);
-            aoff[i] += ainc[i];
+            dma16(asrc + aoff[i], sa + i * 1024);
+            if constexpr (!COLS) aoff[i] += ainc[i];
         }
+        if constexpr (COLS) asrc += a.K * tap_bytes;       // (the next chunk of the tap)
 #pragma unroll
         for (int i = 0; i < BD; i++) {
             // (fewer than four pieces: wavefronts fetch the same one twice, which keeps the counts equal)
@@ -261,15 +279,191 @@ __global__ void __launch_bounds__(kThreads, 2) conv_rows_kernel(ConvRowsArgs a)
                 if (n >= a.C) continue;
                 if (a.out)
                     a.out[((long)b * a.C + n) * a.map.P + p] =
-                        f32_to_bf16(acc[ob][pb][r] + (a.bias ? bf16_to_f32(a.bias[n]) : 0.f));
+                        f32_to_bf16(d2c_epilogue(acc[ob][pb][r] + (a.bias ? bf16_to_f32(a.bias[n]) : 0.f), a.act, a.act_scale));
                 else a.part[((long)split * a.C + n) * M + m] = acc[ob][pb][r];
             }
     }
 }
 
+// The same product for larger problems: a workgroup = 256 rows x NT columns (256 or 128), four wavefronts of 128 x NT/2,
+// one workgroup per compute unit.  A step of 64 channels is 2048 matrix clocks (NT = 256) against 1024 clocks of LDS
+// reads and 512 of DMA writes; the 128 x 128 tile above has 768 clocks of LDS traffic for 512 matrix clocks.  Rows are
+// fetched two steps ahead (three buffers; they come from device memory), weights one (two buffers; they come from L2).
+// The operand reads of a k-group and the DMA requests go between the matrix instructions of the k-group before; a step's
+// only barrier stands in front of its last k-group, when every wavefront holds the last operands of the step in
+// registers: from there on the buffers of the step are free and the next step's first operands are read.
+// Over sampled columns, 512 -> 512 channels on 2x8x30x54: 520 us with the tile above (its partial sums included), 348 us
+// (1.05 PFLOP/s); 256 -> 256 on 32x60x108: 1015 and 746 us, of which reading 2.9 GB of columns once takes 520.
+template <int NT, bool COLS>
+__global__ void __launch_bounds__(kThreads, 1) conv_wide_kernel(ConvRowsArgs a)
+{
+    constexpr int OB = NT / 64, PB = 4;                    // 32-blocks of a wavefront: columns, rows
+    constexpr int ROWB = 128, ABYTES = kWMT * ROWB, BBYTES = NT * ROWB;
+    constexpr int AD = 8, BD = BBYTES / 4096, NM = OB * PB;
+    __shared__ __align__(1024) unsigned char s_t[3 * ABYTES + 2 * BBYTES];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int id = xcd_swizzle(blockIdx.x, gridDim.x);
+    const int ct = id % a.nctile; id /= a.nctile;
+    const int split = id % a.nsplit, tile = id / a.nsplit;
+    const int st_lo = (int)((long)a.S * split / a.nsplit), st_hi = (int)((long)a.S * (split + 1) / a.nsplit);
+    const int m0 = tile * kWMT, M = a.map.N * a.map.P;
+
+    // --- rows this wavefront fetches: wave * 64 + (0 .. 63), eight per request; lane l works out row l
+    const RowPos rp = COLS ? RowPos{} : row_pos(a.map, m0 + wave * 64 + lane);
+    const unsigned char *asrc = a.src;                     // (COLS: the rows of the step)
+    const long tap_bytes = (long)a.tap_rows * ROWB;
+    const int lrow = lane >> 3;                            // this lane's row within a request
+    unsigned aoff[AD], ainc[AD];
+    int achunk = st_lo % a.nchunk, atap = st_lo / a.nchunk, ast = st_lo;      // the step that the next rows belong to
+    if (COLS) {
+#pragma unroll
+        for (int i = 0; i < AD; i++) {
+            // (a tile's rows past the last one: the last one again, stored nowhere)
+            const int rl = i * 8 + lrow;
+            aoff[i] = (unsigned)min(m0 + wave * 64 + rl, M - 1) * ROWB + (unsigned)tile_slot<64>(rl, lane & 7) * 16u;
+        }
+    }
+    auto tap_rows = [&]() {
+        if constexpr (COLS) {
+            asrc = a.src + ((long)achunk * a.K + atap) * tap_bytes;
+        } else {
+            const int kx = atap % a.map.g.kw, ky = (atap / a.map.g.kw) % a.map.g.kh, kz = atap / (a.map.g.kw * a.map.g.kh);
+            const int row = source_row(a.map, rp, kz, ky, kx);
+#pragma unroll
+            for (int i = 0; i < AD; i++) {
+                const int rl = i * 8 + lrow;
+                const int sr = __builtin_amdgcn_ds_bpermute(rl << 2, row);
+                const unsigned vb = (unsigned)tile_slot<64>(rl, lane & 7) * 16u;
+                aoff[i] = sr >= 0 ? (unsigned)sr * a.rowb + (unsigned)achunk * ROWB + vb : a.zrow + vb;
+                ainc[i] = sr >= 0 ? ROWB : 0u;
+            }
+        }
+    };
+    // to the next step's rows (after the last step: its rows again, which nothing reads)
+    auto advance = [&]() {
+        if (ast + 1 >= st_hi) return;
+        ast++;
+        if (++achunk == a.nchunk) {
+            achunk = 0; atap++;
+            tap_rows();
+        } else if constexpr (COLS) {
+            asrc += a.K * tap_bytes;
+        } else {
+#pragma unroll
+            for (int i = 0; i < AD; i++) aoff[i] += ainc[i];
+        }
+    };
+    const unsigned char *bsrc = a.wt + ((long)st_lo * a.nctile + ct) * BBYTES + wave * 1024 + lane * 16;
+    const long bstep = (long)a.nctile * BBYTES;
+    unsigned char *const sa = s_t + wave * (64 * ROWB), *const sb = s_t + 3 * ABYTES + wave * 1024;
+    auto row_request = [&](int i, int buf) { dma16(asrc + aoff[i], sa + buf * ABYTES + i * 1024); };
+    auto weight_request = [&](int i, int buf) { dma16(bsrc + i * 4096, sb + buf * BBYTES + i * 4096); };
+
+    f32x16 acc[OB][PB];
+#pragma unroll
+    for (int ob = 0; ob < OB; ob++)
+#pragma unroll
+        for (int pb = 0; pb < PB; pb++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[ob][pb][r] = 0.f;
+    const int wo = wave & 1, wp = wave >> 1;
+    unsigned slot[4];
+#pragma unroll
+    for (int kg = 0; kg < 4; kg++)
+        slot[kg] = (unsigned)((lane & 31) * ROWB + tile_slot<64>(lane & 31, kg * 2 + (lane >> 5)) * 16);
+    const unsigned ra = lds_address(s_t) + wp * PB * 32 * ROWB, rb = lds_address(s_t) + 3 * ABYTES + wo * OB * 32 * ROWB;
+    u32x4_t fa[2][PB], fb[2][OB];
+    // operand vector i of a k-group: weights first
+    auto operand = [&](auto I, auto S, unsigned pa, unsigned pb, unsigned sl) INLINE {
+        constexpr int i = decltype(I)::value, s = decltype(S)::value;
+        if constexpr (i < OB) fb[s][i] = lds_read16(pb + sl + i * 32 * ROWB);
+        else fa[s][i - OB] = lds_read16(pa + sl + (i - OB) * 32 * ROWB);
+    };
+
+    tap_rows();
+    for (int i = 0; i < AD; i++) row_request(i, 0);
+    for (int i = 0; i < BD; i++) weight_request(i, 0);
+    advance();
+    for (int i = 0; i < AD; i++) row_request(i, 1);
+    advance();
+    wait_vm<AD>();
+    group_barrier();
+    for_each_const([&](auto I) INLINE { operand(I, std::integral_constant<int, 0>{}, ra, rb, slot[0]); }, std::make_integer_sequence<int, OB + PB>{});
+    int abuf = 0, bbuf = 0;
+    for (int st = st_lo; st < st_hi; st++) {
+        if (st + 1 < st_hi) bsrc += bstep;
+        const int a1 = abuf == 2 ? 0 : abuf + 1, a2 = a1 == 2 ? 0 : a1 + 1, b1 = bbuf ^ 1;
+        for_each_const([&](auto KG) INLINE {
+            constexpr int kg = decltype(KG)::value, s = kg & 1;
+#pragma unroll
+            for (int ob = 0; ob < OB; ob++) wait_lds<0>(fb[s][ob]);
+#pragma unroll
+            for (int pb = 0; pb < PB; pb++) asm volatile("" : "+v"(fa[s][pb]));
+            unsigned pa = ra + abuf * ABYTES, pb_ = rb + bbuf * BBYTES;
+            if constexpr (kg == 3) {
+                wait_vm<AD>();                             // (the rows of the step after the next one may be under way)
+                asm volatile("s_barrier" ::: "memory");
+                pa = ra + a1 * ABYTES; pb_ = rb + b1 * BBYTES;
+            }
+            for_each_const([&](auto I) INLINE {
+                constexpr int i = decltype(I)::value, ob = i / PB, pb = i % PB;
+                mma_kgroup<bf16_t, false>(acc[ob][pb], __builtin_bit_cast(uint4, fb[s][ob]), __builtin_bit_cast(uint4, fa[s][pb]));
+                if constexpr (i < OB + PB) operand(I, std::integral_constant<int, s ^ 1>{}, pa, pb_, slot[(kg + 1) & 3]);
+                if constexpr (kg == 0 && i < BD) weight_request(i, b1);
+                if constexpr ((kg == 1 || kg == 2) && i < AD / 2) row_request((kg - 1) * (AD / 2) + i, a2);
+                __builtin_amdgcn_sched_barrier(0);
+            }, std::make_integer_sequence<int, NM>{});
+        }, std::make_integer_sequence<int, 4>{});
+        advance();
+        abuf = a1; bbuf = b1;
+    }
+    // (the reads and requests behind the last step)
+#pragma unroll
+    for (int ob = 0; ob < OB; ob++) wait_lds<0>(fb[0][ob]);
+#pragma unroll
+    for (int pb = 0; pb < PB; pb++) asm volatile("" : "+v"(fa[0][pb]));
+    wait_vm<0>();
+
+    // results, by stores that drop what lies outside (offset kNone); how they end is one choice for all of them
+    constexpr unsigned kNone = 0xFFFFFFF0u;
+    const int h4 = (lane >> 5) * 4, nl = ct * NT + wo * OB * 32;
+    auto finish = [&](auto MODE) INLINE {
+        constexpr int mode = decltype(MODE)::value;        // 0: partial sums, 1: results, 2: results through the epilogue
+        const auto rs = mode == 0 ? __builtin_amdgcn_make_buffer_rsrc(a.part + (long)split * a.C * M, 0, (int)((unsigned)a.C * (unsigned)M * 4u), 0x00020000)
+                                  : __builtin_amdgcn_make_buffer_rsrc(a.out, 0, (int)((unsigned)a.C * (unsigned)M * 2u), 0x00020000);
+        unsigned at[PB];
+        const unsigned step = mode == 0 ? (unsigned)M * 4u : (unsigned)a.map.P * 2u;
+#pragma unroll
+        for (int pb = 0; pb < PB; pb++) {
+            const int m = m0 + (wp * PB + pb) * 32 + (lane & 31), b = fdiv(m, a.map.dP), p = m - b * a.map.P;
+            at[pb] = m >= M ? kNone : (mode == 0 ? (unsigned)m * 4u : ((unsigned)b * a.C * a.map.P + p) * 2u) + (unsigned)h4 * step;
+        }
+        for_each_const([&](auto I) INLINE {
+            constexpr int ob = decltype(I)::value / 16, r = decltype(I)::value % 16;
+            const int n0 = nl + ob * 32 + 8 * (r >> 2) + (r & 3);
+            const bool ok = n0 + h4 < a.C;
+            float bias = 0.f;
+            if (mode != 0 && a.bias) bias = bf16_to_f32(a.bias[ok ? n0 + h4 : 0]);
+            for_each_const([&](auto J) INLINE {
+                constexpr int pb = decltype(J)::value;
+                const unsigned o = ok && at[pb] != kNone ? at[pb] + (unsigned)n0 * step : kNone;
+                const float v = acc[ob][pb][r] + bias;
+                if constexpr (mode == 0) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rs, (int)o, 0, 0);
+                else __builtin_amdgcn_raw_buffer_store_b16((short)f32_to_bf16(mode == 2 ? d2c_epilogue(v, a.act, a.act_scale) : v), rs, (int)o, 0, 0);
+            }, std::make_integer_sequence<int, PB>{});
+            __builtin_amdgcn_sched_barrier(0);
+        }, std::make_integer_sequence<int, OB * 16>{});
+    };
+    if (!a.out) finish(std::integral_constant<int, 0>{});
+    else if (a.act == D2C_EPILOGUE_NONE) finish(std::integral_constant<int, 1>{});
+    else finish(std::integral_constant<int, 2>{});
+}
+
 // out[b][n][p] = bias[n] + the partial sums of (n, b * P + p)
 __global__ void __launch_bounds__(256) conv_rows_finish_kernel(const float *part, const bf16_t *bias, bf16_t *out, int nsplit,
-                                                               int C, int P, FastDiv dP, int M)
+                                                               int C, int P, FastDiv dP, int M, int act, float act_scale)
 {
     const int m = blockIdx.x * 256 + threadIdx.x, n = blockIdx.y;
     if (m >= M) return;
@@ -277,7 +471,7 @@ __global__ void __launch_bounds__(256) conv_rows_finish_kernel(const float *part
     const float *q = part + (long)n * M + m;
     for (int s = 0; s < nsplit; s++) v += q[(long)s * C * M];
     const int b = fdiv(m, dP), p = m - b * P;
-    out[((long)b * C + n) * P + p] = f32_to_bf16(v);
+    out[((long)b * C + n) * P + p] = f32_to_bf16(d2c_epilogue(v, act, act_scale));
 }
 
 // ============================================================ grad_weight
@@ -565,55 +759,74 @@ __global__ void __launch_bounds__(256) conv_prepare_kernel(ConvPrepArgs a)
 
 // ============================================================ host side
 struct RowsPlan {
-    int NT, KC, nchunk, nct, S, ntile, nsplit;
+    int MT, NT, KC, nchunk, nct, S, ntile, nsplit;
     size_t wt_bytes, part_bytes;
 };
+constexpr long kPartClocks = 100;     // a block of 32 x 32 partial sums, per compute unit
 // columns C, reduction over `depth` channels per tap, M rows
 RowsPlan rows_plan(int C, int depth, int K, int M, int ncu)
 {
     RowsPlan p;
     p.KC = depth <= 32 ? 32 : 64;
-    p.NT = C <= 32 ? 32 : (C <= 64 ? 64 : 128);
     p.nchunk = (depth + p.KC - 1) / p.KC;
-    p.nct = (C + p.NT - 1) / p.NT;
     p.S = K * p.nchunk;
-    p.ntile = (M + kMT - 1) / kMT;
-    // Steps shared out between `nsplit` workgroups where the tiles alone leave compute units idle.  Two workgroups run
-    // on a compute unit at a time; a piece costs its steps, about four more for its start and end, and its share of the
-    // partial sums, which are written and read once more each (about a step per 32 columns).
-    const long items = (long)p.ntile * p.nct, slots = 2L * ncu;
+    // Tile and number of pieces that the steps of a tile are shared out to, by what they cost in matrix clocks of a
+    // compute unit: rounds over the workgroups that run at a time (two per compute unit with 128 rows, one with 256),
+    // each its steps and about four more for its start and end; a piece's partial sums are written and read once more.
+    // (clocks of a step: from the rates on large problems)
     long best = -1;
-    p.nsplit = 1;
-    for (int s = 1; s <= 16 && s <= p.S; s++) {
-        const long rounds = (items * s + slots - 1) / slots;
-        const long cost = rounds * ((p.S + s - 1) / s + 4) + (s > 1 ? (items * s * (p.NT / 32) + slots - 1) / slots : 0);
-        if (best < 0 || cost * 20 < best * 19) { best = cost; p.nsplit = s; }
-    }
+    auto consider = [&](int MT, int NT, long slots, long step_clocks) {
+        const int nct = (C + NT - 1) / NT, ntile = (M + MT - 1) / MT;
+        const long items = (long)ntile * nct;
+        for (int s = 1; s <= 16 && s <= p.S; s++) {
+            const long rounds = (items * s + slots - 1) / slots;
+            const long cost = rounds * ((p.S + s - 1) / s + 4) * step_clocks +
+                              (s > 1 ? (items * s * (MT / 32) * (NT / 32) + ncu - 1) / ncu * kPartClocks : 0);
+            if (best < 0 || cost * 20 < best * 19) { best = cost; p.MT = MT; p.NT = NT; p.nct = nct; p.ntile = ntile; p.nsplit = s; }
+        }
+    };
+    consider(kMT, C <= 32 ? 32 : (C <= 64 ? 64 : 128), 2L * ncu, C <= 32 ? 1500 : (C <= 64 ? 2000 : 3000));
+    // (its results and partial sums are written through 32-bit offsets)
+    const bool wide = p.KC == 64 && (size_t)C * M * 4 < 0xFFFF0000u;
+    if (wide && C > 64) consider(kWMT, 128, ncu, 1700);
+    if (wide && C > 128) consider(kWMT, 256, ncu, 2800);
     p.wt_bytes = d2c_align_up((size_t)p.S * p.nct * p.NT * p.KC * 2);
     p.part_bytes = p.nsplit > 1 ? d2c_align_up((size_t)p.nsplit * C * M * sizeof(float)) : 0;
     return p;
 }
 
-template <int NT, int KC> int launch_rows(const ConvRowsArgs &a, hipStream_t st)
+template <int NT, int KC, bool COLS = false> int launch_rows(const ConvRowsArgs &a, hipStream_t st)
 {
     D2cProfScope prof(D2C_PROF_FWD, st, "conv_rows_kernel");
-    hipLaunchKernelGGL((conv_rows_kernel<NT, KC>), dim3((unsigned)(a.ntile * a.nsplit * a.nctile)), dim3(kThreads), 0, st, a);
+    hipLaunchKernelGGL((conv_rows_kernel<NT, KC, COLS>), dim3((unsigned)(a.ntile * a.nsplit * a.nctile)), dim3(kThreads), 0, st, a);
     return d2c_check_launch("conv_rows_kernel");
 }
 
+template <int NT, bool COLS> int launch_wide(const ConvRowsArgs &a, hipStream_t st)
+{
+    D2cProfScope prof(D2C_PROF_FWD, st, "conv_wide_kernel");
+    hipLaunchKernelGGL((conv_wide_kernel<NT, COLS>), dim3((unsigned)(a.ntile * a.nsplit * a.nctile)), dim3(kThreads), 0, st, a);
+    return d2c_check_launch("conv_wide_kernel");
+}
+
 int run_rows(const RowsPlan &p, const RowMap &map, const void *src, unsigned rowb, unsigned zrow, const void *wt, const void *bias,
-             void *out, float *part, int C, hipStream_t st)
+             void *out, float *part, int C, hipStream_t st, int cols_K = 0, int cols_rows = 0, int act = 0, float act_scale = 1.f)
 {
     ConvRowsArgs a{map, (const unsigned char *)src, (const unsigned char *)wt, p.nsplit > 1 ? nullptr : (const bf16_t *)bias,
-                   p.nsplit > 1 ? nullptr : (bf16_t *)out, part, rowb, zrow, C, p.nchunk, p.S, p.ntile, p.nct, p.nsplit};
+                   p.nsplit > 1 ? nullptr : (bf16_t *)out, part, rowb, zrow, C, p.nchunk, p.S, p.ntile, p.nct, p.nsplit,
+                   cols_K, cols_rows, act, act_scale};
     int rc;
-    if (p.KC == 32) rc = p.NT == 32 ? launch_rows<32, 32>(a, st) : (p.NT == 64 ? launch_rows<64, 32>(a, st) : launch_rows<128, 32>(a, st));
+    if (p.MT == kWMT)
+        rc = p.NT == 256 ? (cols_K > 0 ? launch_wide<256, true>(a, st) : launch_wide<256, false>(a, st))
+                         : (cols_K > 0 ? launch_wide<128, true>(a, st) : launch_wide<128, false>(a, st));
+    else if (cols_K > 0) rc = p.NT == 32 ? launch_rows<32, 64, true>(a, st) : (p.NT == 64 ? launch_rows<64, 64, true>(a, st) : launch_rows<128, 64, true>(a, st));
+    else if (p.KC == 32) rc = p.NT == 32 ? launch_rows<32, 32>(a, st) : (p.NT == 64 ? launch_rows<64, 32>(a, st) : launch_rows<128, 32>(a, st));
     else rc = p.NT == 32 ? launch_rows<32, 64>(a, st) : (p.NT == 64 ? launch_rows<64, 64>(a, st) : launch_rows<128, 64>(a, st));
     if (rc || p.nsplit == 1) return rc;
     const int M = map.N * map.P;
     D2cProfScope prof(D2C_PROF_PACK, st);
     hipLaunchKernelGGL(conv_rows_finish_kernel, dim3((M + 255) / 256, C), dim3(256), 0, st, part, (const bf16_t *)bias, (bf16_t *)out,
-                       p.nsplit, C, map.P, map.dP, M);
+                       p.nsplit, C, map.P, map.dP, M, act, act_scale);
     return d2c_check_launch("conv_rows_finish_kernel");
 }
 
@@ -654,6 +867,34 @@ inline bool plain_shape_ok(const d2c_conv3d_desc &q)
 inline int weight_blocks(long nvec) { return (int)std::min<long>((nvec + 255) / 256, 4096); }
 
 }  // namespace
+
+// ---- the same product over sampled columns [chunk][tap][rows][64] (d2c_brick.hip): the forward pass of the deformable
+// operator, one weight group
+size_t d2c_col_forward_ws(const d2c_conv3d_desc &q)
+{
+    const int ncu = d2c_num_cus();
+    if (ncu <= 0) return 0;
+    const RowsPlan p = rows_plan(q.Cout, q.Cin, q.kd * q.kh * q.kw, q.N * q.Do * q.Ho * q.Wo, ncu);
+    return p.wt_bytes + p.part_bytes;
+}
+int d2c_col_forward(const d2c_conv3d_desc &q, const void *col, int rows, const void *w, const void *bias, void *out, void *ws, hipStream_t st)
+{
+    const int K = q.kd * q.kh * q.kw, ncu = d2c_num_cus();
+    if (ncu <= 0) return D2C_ERR_LAUNCH;
+    const RowsPlan p = rows_plan(q.Cout, q.Cin, K, q.N * q.Do * q.Ho * q.Wo, ncu);
+    {
+        ConvPrepArgs a{};
+        a.w = (const bf16_t *)w; a.wt = (uint4 *)ws; a.Cout = q.Cout; a.Cin = q.Cin; a.K = K;
+        a.NT = p.NT; a.KC = p.KC; a.nchunk = p.nchunk; a.nct = p.nct; a.back = 0;
+        a.nvec = (long)p.nct * p.NT * p.nchunk * (p.KC / 8) * K;
+        a.nblk_w = weight_blocks(a.nvec);
+        D2cProfScope prof(D2C_PROF_PACK, st);
+        hipLaunchKernelGGL(conv_prepare_kernel, dim3((unsigned)a.nblk_w), dim3(256), 0, st, a);
+        if (int rc = d2c_check_launch("conv_prepare_kernel")) return rc;
+    }
+    return run_rows(p, row_map(q, false), col, 0, 0, ws, bias, out, (float *)((char *)ws + p.wt_bytes), q.Cout, st, K, rows, q.epilogue,
+                    q.epilogue_scale);
+}
 
 bool d2c_plain_supported(const d2c_conv3d_desc &q) { return plain_shape_ok(q); }
 size_t d2c_plain_input_bytes(const d2c_conv3d_desc &q) { return (size_t)q.N * q.Cin * q.D * q.H * q.W * 2 + 1024; }

@@ -13,6 +13,7 @@
 //   D: lane l holds col  n = l % 32, rows m = 8*(r/4) + 4*(l/32) + r%4 for r = 0..15
 #pragma once
 #include <type_traits>
+#include <utility>
 #include "d2c_common.hpp"
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -20,6 +21,14 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+
+// f(integral_constant 0), f(integral_constant 1), ... for indices that have to be constants (f: a lambda marked INLINE)
+template <class F, int... I> D2C_DEV void for_each_const(F &&f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+
+#define INLINE __attribute__((always_inline))
 
 template <typename T> struct Elem;
 template <> struct Elem<bf16_t> {

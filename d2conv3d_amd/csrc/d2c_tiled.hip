@@ -5,6 +5,8 @@
 #include "d2c_brick.hpp"
 #include "d2c_mma.hpp"
 
+size_t d2c_col_forward_ws(const d2c_conv3d_desc &q);
+int d2c_col_forward(const d2c_conv3d_desc &q, const void *col, int rows, const void *w, const void *bias, void *out, void *ws, hipStream_t st);
 int d2c_fwd_out_tile(const TiledShape &s);
 template <typename T>
 int d2c_tiled_fwd_launch(const TiledShape &s, const void *xcl, const void *off, const void *mask, const void *wp,
@@ -375,7 +377,12 @@ __global__ void __launch_bounds__(256) size_minus_one_kernel(TiledShape s, const
 
 struct FwdWs {
     size_t xcl, wp, outacc, total;
+    size_t lists, col, gemm;        // forward over sampled columns: sorted points, columns, operands of the product
 };
+bool use_brick_forward(const d2c_conv3d_desc &q, const TiledShape &s, bool kept);
+// columns; and what a forward call can leave for its backward call: the sorted points behind them
+size_t brick_col_bytes(const TiledShape &s) { return (size_t)(s.Cin / 64) * s.K * d2c_columns_rows(s) * 128; }
+size_t brick_keep_bytes(const TiledShape &s) { return brick_col_bytes(s) + d2c_brick_ws(s).total; }
 // Caller-held prepared region (d2c_conv3d_prepared_bytes): channels-last input + zero row | forward weights in
 // fragment order | backward weights transposed per step (single-pass reductions only)
 struct PreparedLayout {
@@ -384,15 +391,24 @@ struct PreparedLayout {
 FwdWs fwd_ws(const d2c_conv3d_desc &q, const TiledShape &s)
 {
     const size_t es = d2c_elem_size(q.dtype);
-    FwdWs w;
+    FwdWs w{};
     w.xcl = 0;
     w.wp = d2c_align_up((size_t)s.N * s.vol * s.Cin * es + 256);   // input, then a 256-byte row of zeros
+    if (use_brick_forward(q, s, true)) {
+        w.gemm = w.wp;
+        w.lists = w.gemm + d2c_align_up(d2c_col_forward_ws(q));
+        w.col = w.lists + d2c_brick_ws(s).total;
+        w.total = w.col + (use_brick_forward(q, s, false) ? brick_col_bytes(s) : 0);
+        // (a call with a prepared region runs on the gather kernels, whose workspace this covers)
+    }
+    const size_t brick_total = w.total;
     w.outacc = w.wp + d2c_align_up((size_t)s.groups * s.nchunk * s.K * s.ogp * bkc_of(q.dtype) * es);
     // fp32 partial sums of the output, used only when the forward kernel splits its steps (as whole tiles of
     // 64 positions x padded output channels in the DMA-gather kernel)
     w.total = w.outacc;
     if (d2c_fwd_split(s) > 1)
         w.total += d2c_align_up((size_t)((s.M + 63) / 64 * 64) * s.ogp * s.groups * sizeof(float));
+    if (w.total < brick_total) w.total = brick_total;
     return w;
 }
 
@@ -491,7 +507,7 @@ DwWs dw_ws(const d2c_conv3d_desc &q, const TiledShape &s)
 template <typename T>
 int forward_t(const d2c_conv3d_desc &q, const void *x, const void *off, const void *mask, const void *w,
               const void *bias, void *out, void *ws, hipStream_t st, int nd = 3, const d2c_size_map_desc *sz = nullptr,
-              float *stats = nullptr, const D2cPrepared *prep = nullptr, void *columns = nullptr)
+              float *stats = nullptr, const D2cPrepared *prep = nullptr, void *columns = nullptr, size_t columns_bytes = 0)
 {
     const TiledShape s = tiled_shape(q, nd, 0, sz);
     char *base = (char *)ws;
@@ -508,6 +524,15 @@ int forward_t(const d2c_conv3d_desc &q, const void *x, const void *off, const vo
     char *wp_p = prep ? (char *)prep->base + pl.wp : base + l.wp;
     if (!(prep && (prep->reuse & D2C_REUSE_INPUT)))
         if (int rc = pack_input<T>(s, x, xcl_p, st, true)) return rc;   // with the row of zeros behind it
+    if (nd == 3 && !prep && !stats && use_brick_forward(q, s, columns != nullptr)) {
+        // sort the points, sample the columns (the caller's buffer, with the sorted points behind them for its backward
+        // call, or the workspace), multiply
+        char *col = columns ? (char *)columns : base + l.col;
+        char *lists = columns && columns_bytes >= brick_keep_bytes(s) ? col + brick_col_bytes(s) : base + l.lists;
+        if (int rc = d2c_brick_sort(s, off, mask, lists, st)) return rc;
+        if (int rc = d2c_brick_columns(s, xcl_p, col, (int)d2c_columns_rows(s), lists, st)) return rc;
+        return d2c_col_forward(q, col, (int)d2c_columns_rows(s), w, bias, out, base + l.gemm, st);
+    }
     const long total = (long)s.groups * s.nchunk * s.K * (s.ogp / 32) * 4 * 64;
     long g = (total + 255) / 256;
     if (g > 8192) g = 8192;
@@ -554,6 +579,17 @@ bool use_aux_kernel(const d2c_conv3d_desc &q, const TiledShape &s)
 bool use_brick(const d2c_conv3d_desc &q, const TiledShape &s)
 {
     return d2c_gx_mode() == 1 && use_lists(q, s) && use_aux_kernel(q, s) && d2c_brick_supported(s, q.dtype);
+}
+
+// The forward pass over sampled columns: sort, sample, multiply.  `kept`: the caller keeps the columns and the backward
+// call takes the sorted points over.  Picoseconds per point and chunk of 64 channels, C columns: sort 60 / chunks of a
+// group, sampling 33, product 0.13 C; the gathering kernel 55 + 0.15 C (192 - 512 columns).  So with the sort paid for by
+// the backward pass the columns win throughout, without it from four chunks on (256 -> 192 channels on 5x72x100: 360 and
+// 356 us, 2048 -> 512 with its branch: 2.8 and 4.2 ms).  Below some 12 000 positions the fixed times of the six launches
+// take the difference.
+bool use_brick_forward(const d2c_conv3d_desc &q, const TiledShape &s, bool kept)
+{
+    return use_brick(q, s) && s.groups == 1 && s.M >= 12288 && brick_col_bytes(s) < (4ull << 30) && (kept || s.cpg / 64 >= 4);
 }
 
 // grad_weight as a matrix product over sampled columns that the offset / mask gradient kernel writes on its way
@@ -645,7 +681,7 @@ BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns =
     w.sm1 = w.total;       // ... and (size - 1) per axis
     if (s.ss.on) w.total += d2c_align_up((size_t)s.N * 3 * s.P * sizeof(float));
     w.brick = w.total;
-    if (use_brick(q, s)) w.total += d2c_brick_ws(s).total;
+    if (use_brick(q, s)) w.total += d2c_brick_ws(s).total + d2c_brick_ws(s).res_bytes;
     w.col = w.total;       // sampled columns for the grad-weight product
     if (!saved_columns && use_col_weight(q, s) && !col_in_place(q, s))
         w.total += d2c_align_up(d2c_bwd_col_bytes(s, q.dtype, sl.cgs ? sl.cgs * (s.cpg / 64) : 0));
@@ -656,7 +692,7 @@ template <typename T>
 int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const void *off, const void *mask,
                const void *w, void *gx, void *goff, void *gmask, void *gw, void *gb, void *ws, hipStream_t st,
                int nd = 3, int quirks = 0, const d2c_size_map_desc *sz = nullptr, const D2cPrepared *prep = nullptr,
-               const void *columns = nullptr)
+               const void *columns = nullptr, size_t columns_bytes = 0)
 {
     TiledShape s = tiled_shape(q, nd, quirks, sz);
     char *base = (char *)ws;
@@ -785,7 +821,7 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
             // size-map source: `goff` is the gradient of the raw size map; the offset / mask gradient kernel adds
             // into fp32 sums per axis, which a finishing kernel folds into it
             gw_from_col = gw && (columns ? d2c_bwd_weight_from_kept_col(s, q.dtype) : (auxk && use_col_weight(q, s)));
-            const bool brick = use_brick(q, s) && !(gw_from_col && !columns);
+            const bool brick = use_brick(q, s) && !(gw && gw_mode(q) == 2);      // (not: columns in the rows' place)
             void *goff_k = goff;
             if (s.ss.on && goff && !brick) {
                 goff_k = base + l.gsacc;
@@ -796,8 +832,12 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
             // offset / mask gradient kernel runs, so the samples are filed by a pass of their own)
             gw_in_place = gw_from_col && !columns && col_in_place(q, s);
             SampleLists L{nullptr, nullptr, nullptr, 0, 0, 0};
+            // (kept columns of a forward call over sorted points: those follow the columns)
+            const bool sorted = columns && use_brick_forward(q, s, true) && columns_bytes >= brick_keep_bytes(s);
+            char *const lists_p = sorted ? (char *)const_cast<void *>(columns) + brick_col_bytes(s) : base + l.brick;
             if (brick) {
-                if (int rc = d2c_brick_sort(s, off, mask, base + l.brick, st)) return rc;
+                if (!sorted)
+                    if (int rc = d2c_brick_sort(s, off, mask, lists_p, st)) return rc;
             } else if (lists) {
                 L = d2c_lists_make(s, Elem<T>::DT, base + l.counts, base + l.entries, base + l.ovf);
                 if (int rc = (auxk && !gw_in_place) ? d2c_lists_clear(L, st) : d2c_lists_build(s, off, mask, L, st)) return rc;
@@ -815,7 +855,11 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
                               (size_t)64 * bkc_of(q.dtype) * sizeof(T), st);
             }
             if (brick) {
-                if (int rc = d2c_brick_grad(s, xcl_p, base + l.gcol, mask, size_raw, gxcl, goff, gmask, base + l.brick, st)) return rc;
+                if (gw_from_col && !columns) {
+                    if (int rc = d2c_brick_columns(s, xcl_p, base + l.col, (int)d2c_columns_rows(s), lists_p, st)) return rc;
+                }
+                if (int rc = d2c_brick_grad(s, xcl_p, base + l.gcol, mask, size_raw, gxcl, goff, gmask, lists_p,
+                                            base + l.brick + d2c_brick_ws(s).total, st)) return rc;
             } else if (auxk)
                 if (int rc = d2c_aux_grad_launch<T>(s, xcl_p, off, mask, base + l.gcol, goff_k, gmask,
                                                     (lists && !gw_in_place) ? &L : nullptr,
@@ -968,10 +1012,19 @@ size_t d2c_tiled_columns_bytes(const d2c_conv3d_desc &q, const d2c_size_map_desc
     if (is_depthwise(q) || !mfma_channels_ok(q)) return 0;
     if (sz && !d2c_tiled_sized_supported(q, true)) return 0;
     const TiledShape s = tiled_shape(q, 3, 0, sz);
+    if (use_brick_forward(q, s, true)) return d2c_bwd_weight_from_kept_col(s, q.dtype) && use_aux_kernel(q, s) ? brick_col_bytes(s) : 0;
     if (!d2c_fwd_writes_columns(s, q.dtype) || !d2c_bwd_weight_from_kept_col(s, q.dtype) || !use_aux_kernel(q, s)) return 0;
     const long rows = d2c_columns_rows(s), chunks = s.Cin / bkc_of(q.dtype);
     if (chunks * s.K * rows >= (1L << 31)) return 0;      // (the kernel counts rows in 32 bits)
     return (size_t)chunks * s.K * rows * bkc_of(q.dtype) * d2c_elem_size(q.dtype);
+}
+
+// ... and what is worth keeping beside them: the sampling points that the forward pass sorted, behind the columns
+size_t d2c_tiled_keep_bytes(const d2c_conv3d_desc &q, const d2c_size_map_desc *sz)
+{
+    const size_t n = d2c_tiled_columns_bytes(q, sz);
+    const TiledShape s = tiled_shape(q, 3, 0, sz);
+    return n > 0 && use_brick_forward(q, s, true) ? brick_keep_bytes(s) : n;
 }
 
 // The matrix-core kernels can form the offsets from a size map themselves; the backward pass then needs the
@@ -985,10 +1038,10 @@ bool d2c_tiled_sized_supported(const d2c_conv3d_desc &q, bool backward)
 
 int d2c_tiled_forward(const d2c_conv3d_desc &q, const void *x, const void *off, const void *mask, const void *w,
                       const void *bias, void *out, void *ws, hipStream_t st, const d2c_size_map_desc *sz, float *stats,
-                      const D2cPrepared *prep, void *columns)
+                      const D2cPrepared *prep, void *columns, size_t columns_bytes)
 {
-    if (q.dtype == D2C_BF16) return forward_t<bf16_t>(q, x, off, mask, w, bias, out, ws, st, 3, sz, stats, prep, columns);
-    return forward_t<float>(q, x, off, mask, w, bias, out, ws, st, 3, sz, stats, prep, columns);
+    if (q.dtype == D2C_BF16) return forward_t<bf16_t>(q, x, off, mask, w, bias, out, ws, st, 3, sz, stats, prep, columns, columns_bytes);
+    return forward_t<float>(q, x, off, mask, w, bias, out, ws, st, 3, sz, stats, prep, columns, columns_bytes);
 }
 
 // Bytes of the caller-held prepared region of a description (0: the kernel family keeps nothing worth holding)
@@ -1001,15 +1054,15 @@ size_t d2c_tiled_prepared_bytes(const d2c_conv3d_desc &q)
 // The forward kernels of this description add up per-channel statistics of the output on their way.
 bool d2c_tiled_forward_fills_stats(const d2c_conv3d_desc &q)
 {
-    return !is_depthwise(q) && mfma_channels_ok(q) && d2c_fwd_fills_stats(tiled_shape(q));
+    return !is_depthwise(q) && mfma_channels_ok(q) && d2c_fwd_fills_stats(tiled_shape(q)) && !use_brick_forward(q, tiled_shape(q), false);
 }
 
 int d2c_tiled_backward(const d2c_conv3d_desc &q, const void *gout, const void *x, const void *off,
                        const void *mask, const void *w, void *gx, void *goff, void *gmask, void *gw, void *gb,
                        void *ws, hipStream_t st, const d2c_size_map_desc *sz, const D2cPrepared *prep,
-                       const void *columns)
+                       const void *columns, size_t columns_bytes)
 {
     if (q.dtype == D2C_BF16)
-        return backward_t<bf16_t>(q, gout, x, off, mask, w, gx, goff, gmask, gw, gb, ws, st, 3, 0, sz, prep, columns);
-    return backward_t<float>(q, gout, x, off, mask, w, gx, goff, gmask, gw, gb, ws, st, 3, 0, sz, prep, columns);
+        return backward_t<bf16_t>(q, gout, x, off, mask, w, gx, goff, gmask, gw, gb, ws, st, 3, 0, sz, prep, columns, columns_bytes);
+    return backward_t<float>(q, gout, x, off, mask, w, gx, goff, gmask, gw, gb, ws, st, 3, 0, sz, prep, columns, columns_bytes);
 }

@@ -131,7 +131,7 @@ Tensor forward_3d(const Call3d &c, const Tensor &x, const Tensor &off, const Ten
     Tensor out = at::empty({q.N, q.Cout, q.Do, q.Ho, q.Wo}, x.options().requires_grad(false));
     const size_t nb = c.sized ? d2c_conv3d_sized_forward_workspace_bytes(&q, &c.size) : d2c_conv3d_forward_workspace_bytes(&q);
     if (keep) {
-        const size_t n = d2c_conv3d_columns_bytes(&q, c.sz());
+        const size_t n = d2c_conv3d_keep_bytes(&q, c.sz());
         if (n > 0 && n <= keep_max) {
             try {
                 columns = at::empty({(int64_t)n}, x.options().dtype(at::kByte).requires_grad(false));

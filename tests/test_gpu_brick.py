@@ -1,0 +1,65 @@
+"""The kernels over sampling points sorted by 1x3x3 blocks of voxels, bfloat16: forward and all gradients against the CPU
+oracle where a block, a product of 32 points, a set of channel chunks or the volume ends, with points on, across and beyond the
+border; and the matrix product of the forward pass over sampled columns at the edges of its tiles, at zero offsets against
+the plain convolution."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+import d2conv3d_amd as d2c
+from oracle import cpu
+from _util import out_dims, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+# (N, Cin, Cout, dims, kernel, stride, dilation, G, mask)
+CASES = {
+    "one_voxel": (1, 64, 40, (1, 1, 1), (3, 3, 3), 1, 1, 1, True),
+    "five_chunks": (2, 320, 40, (3, 7, 11), (3, 3, 3), 1, 1, 1, True),
+    "two_groups_stride": (1, 128, 136, (5, 9, 10), (3, 3, 3), 2, 1, 2, True),
+    "bar_without_mask": (1, 192, 64, (4, 5, 33), (1, 7, 1), 1, 1, 1, False),
+    "nine_chunks_three_groups_dilated": (1, 576, 33, (2, 6, 8), (3, 3, 3), 1, 2, 3, True),
+    "kept_columns_ragged": (1, 128, 72, (13, 31, 31), (3, 3, 3), 1, 1, 2, True),
+    "columns_forward_ragged": (1, 256, 16, (1, 95, 131), (3, 3, 3), 1, 1, 1, True),
+}
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_sorted_points_against_the_oracle(name, dev):
+    N, Cin, Cout, dims, ks, stride, dil, G, masked = CASES[name]
+    pad = tuple(dil * (k // 2) for k in ks)
+    od = out_dims(dims, ks, (stride,) * 3, pad, (dil,) * 3)
+    K = ks[0] * ks[1] * ks[2]
+    g = torch.Generator().manual_seed(len(name))
+    x = torch.randn(N, Cin, *dims, generator=g).bfloat16()
+    w = (torch.randn(Cout, Cin, *ks, generator=g) / (Cin * K) ** 0.5).bfloat16()
+    b = torch.randn(Cout, generator=g).bfloat16()
+    off = torch.randn(N, G * 3 * K, *od, generator=g) * 1.5
+    flat = off.view(-1)
+    flat[::7] = flat[::7].round()                     # on a voxel, some of them on the border
+    flat[::11] *= 8                                   # far outside
+    m = torch.sigmoid(torch.randn(N, G * K, *od, generator=g)) if masked else None
+    gout = torch.randn(N, Cout, *od, generator=g).bfloat16()
+    f = lambda t: t.float() if t is not None else None
+    exp = cpu.conv3d_forward(f(x), off, m, f(w), f(b), stride, pad, dil, 1, G)
+    eg = cpu.conv3d_backward(f(gout), f(x), off, m, f(w), True, stride, pad, dil, 1, G)
+    ts = [t.to(dev) if t is not None else None for t in (x, off, m, w, b)]
+    assert rel_l2(d2c.deform_conv3d(*ts, stride, pad, dil, 1, G), exp) < 1e-2
+    ts = [t.requires_grad_(True) if t is not None else None for t in ts]
+    out = d2c.deform_conv3d(*ts, stride, pad, dil, 1, G)
+    out.backward(gout.to(dev))
+    assert rel_l2(out, exp) < 1e-2
+    for what, t, e in zip(("grad_input", "grad_offset", "grad_mask", "grad_weight", "grad_bias"), ts, eg):
+        if t is not None:
+            assert rel_l2(t.grad, e) < 2e-2, (what, rel_l2(t.grad, e))
+
+
+@pytest.mark.parametrize("Cin,Cout,dims", [(256, 130, (13, 31, 31)), (256, 300, (1, 111, 115)), (320, 72, (6, 45, 46)),
+                                           (512, 257, (2, 80, 81))])
+def test_columns_forward_at_tile_edges(Cin, Cout, dims, dev):
+    g = torch.Generator().manual_seed(Cin + Cout)
+    x = torch.randn(1, Cin, *dims, generator=g).bfloat16()
+    w = (torch.randn(Cout, Cin, 3, 3, 3, generator=g) / (Cin * 27) ** 0.5).bfloat16()
+    b = torch.randn(Cout, generator=g).bfloat16()
+    out = d2c.deform_conv3d(x.to(dev), torch.zeros(1, 81, *dims, device=dev), None, w.to(dev), b.to(dev), 1, 1, 1, 1, 1)
+    assert rel_l2(out, F.conv3d(x.float(), w.float(), b.float(), padding=1)) < 5e-3
