@@ -135,6 +135,7 @@ struct ConvRowsArgs {
     int C;                            // columns that exist
     int nchunk, S;                    // KC-channel chunks per row, steps
     int ntile, nctile, nsplit;
+    int nfull;                        // conv_wide_kernel: tiles (row tile major) whose steps are not shared out
     // COLS: `src` is [chunk][tap][row][KC], a step's rows lie one after the other
     int K, tap_rows;                  // taps, rows of a tap
     int act;                          // epilogue (d2c_epilogue)
@@ -288,12 +289,13 @@ __global__ void __launch_bounds__(kThreads, 2) conv_rows_kernel(ConvRowsArgs a)
 // The same product for larger problems: a workgroup = 256 rows x NT columns (256 or 128), four wavefronts of 128 x NT/2,
 // one workgroup per compute unit.  A step of 64 channels is 2048 matrix clocks (NT = 256) against 1024 clocks of LDS
 // reads and 512 of DMA writes; the 128 x 128 tile above has 768 clocks of LDS traffic for 512 matrix clocks.  Rows are
-// fetched two steps ahead (three buffers; they come from device memory), weights one (two buffers; they come from L2).
+// fetched two steps ahead (three buffers; they come from device memory), weights one (two buffers; they come from L2),
+// each into the buffer that the step's barrier has just freed.
 // The operand reads of a k-group and the DMA requests go between the matrix instructions of the k-group before; a step's
 // only barrier stands in front of its last k-group, when every wavefront holds the last operands of the step in
 // registers: from there on the buffers of the step are free and the next step's first operands are read.
-// Over sampled columns, 512 -> 512 channels on 2x8x30x54: 520 us with the tile above (its partial sums included), 348 us
-// (1.05 PFLOP/s); 256 -> 256 on 32x60x108: 1015 and 746 us, of which reading 2.9 GB of columns once takes 520.
+// Over sampled columns, 512 -> 512 channels on 2x8x30x54: 520 us with the tile above (its partial sums included), 341 us
+// (1.08 PFLOP/s); 256 -> 256 on 32x60x108: 1015 and 683 us, of which reading 2.9 GB of columns once takes 520.
 template <int NT, bool COLS>
 __global__ void __launch_bounds__(kThreads, 1) conv_wide_kernel(ConvRowsArgs a)
 {
@@ -304,10 +306,13 @@ __global__ void __launch_bounds__(kThreads, 1) conv_wide_kernel(ConvRowsArgs a)
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int id = xcd_swizzle(blockIdx.x, gridDim.x);
-    const int ct = id % a.nctile; id /= a.nctile;
-    const int split = id % a.nsplit, tile = id / a.nsplit;
-    const int st_lo = (int)((long)a.S * split / a.nsplit), st_hi = (int)((long)a.S * (split + 1) / a.nsplit);
+    // the first `nfull` tiles are whole ones, the rest is shared out to nsplit workgroups each
+    const bool whole = (int)blockIdx.x < a.nfull;
+    const int piece = whole ? 0 : xcd_swizzle((int)blockIdx.x - a.nfull, (int)gridDim.x - a.nfull);
+    const int item = whole ? xcd_swizzle(blockIdx.x, a.nfull) : a.nfull + piece / a.nsplit;
+    const int split = whole ? 0 : piece % a.nsplit, nsplit = whole ? 1 : a.nsplit;
+    const int ct = item % a.nctile, tile = item / a.nctile;
+    const int st_lo = (int)((long)a.S * split / nsplit), st_hi = (int)((long)a.S * (split + 1) / nsplit);
     const int m0 = tile * kWMT, M = a.map.N * a.map.P;
 
     // --- rows this wavefront fetches: wave * 64 + (0 .. 63), eight per request; lane l works out row l
@@ -388,12 +393,14 @@ __global__ void __launch_bounds__(kThreads, 1) conv_wide_kernel(ConvRowsArgs a)
     advance();
     for (int i = 0; i < AD; i++) row_request(i, 1);
     advance();
-    wait_vm<AD>();
+    if (st_lo + 1 < st_hi) bsrc += bstep;
+    for (int i = 0; i < BD; i++) weight_request(i, 1);
+    wait_vm<AD + BD>();
     group_barrier();
     for_each_const([&](auto I) INLINE { operand(I, std::integral_constant<int, 0>{}, ra, rb, slot[0]); }, std::make_integer_sequence<int, OB + PB>{});
     int abuf = 0, bbuf = 0;
     for (int st = st_lo; st < st_hi; st++) {
-        if (st + 1 < st_hi) bsrc += bstep;
+        if (st + 2 < st_hi) bsrc += bstep;
         const int a1 = abuf == 2 ? 0 : abuf + 1, a2 = a1 == 2 ? 0 : a1 + 1, b1 = bbuf ^ 1;
         for_each_const([&](auto KG) INLINE {
             constexpr int kg = decltype(KG)::value, s = kg & 1;
@@ -411,8 +418,8 @@ __global__ void __launch_bounds__(kThreads, 1) conv_wide_kernel(ConvRowsArgs a)
                 constexpr int i = decltype(I)::value, ob = i / PB, pb = i % PB;
                 mma_kgroup<bf16_t, false>(acc[ob][pb], __builtin_bit_cast(uint4, fb[s][ob]), __builtin_bit_cast(uint4, fa[s][pb]));
                 if constexpr (i < OB + PB) operand(I, std::integral_constant<int, s ^ 1>{}, pa, pb_, slot[(kg + 1) & 3]);
-                if constexpr (kg == 0 && i < BD) weight_request(i, b1);
-                if constexpr ((kg == 1 || kg == 2) && i < AD / 2) row_request((kg - 1) * (AD / 2) + i, a2);
+                if constexpr ((kg == 0 || kg == 1) && i < AD / 2) row_request(kg * (AD / 2) + i, a2);
+                if constexpr (kg == 3 && i < BD) weight_request(i, bbuf);
                 __builtin_amdgcn_sched_barrier(0);
             }, std::make_integer_sequence<int, NM>{});
         }, std::make_integer_sequence<int, 4>{});
@@ -431,19 +438,21 @@ __global__ void __launch_bounds__(kThreads, 1) conv_wide_kernel(ConvRowsArgs a)
     const int h4 = (lane >> 5) * 4, nl = ct * NT + wo * OB * 32;
     auto finish = [&](auto MODE) INLINE {
         constexpr int mode = decltype(MODE)::value;        // 0: partial sums, 1: results, 2: results through the epilogue
-        const auto rs = mode == 0 ? __builtin_amdgcn_make_buffer_rsrc(a.part + (long)split * a.C * M, 0, (int)((unsigned)a.C * (unsigned)M * 4u), 0x00020000)
+        const auto rs = mode == 0 ? __builtin_amdgcn_make_buffer_rsrc(a.part + (long)piece * NT * kWMT, 0, NT * kWMT * 4, 0x00020000)
                                   : __builtin_amdgcn_make_buffer_rsrc(a.out, 0, (int)((unsigned)a.C * (unsigned)M * 2u), 0x00020000);
         unsigned at[PB];
-        const unsigned step = mode == 0 ? (unsigned)M * 4u : (unsigned)a.map.P * 2u;
+        const unsigned step = mode == 0 ? kWMT * 4u : (unsigned)a.map.P * 2u;
+        const int n_lo = mode == 0 ? wo * OB * 32 : nl;
 #pragma unroll
         for (int pb = 0; pb < PB; pb++) {
-            const int m = m0 + (wp * PB + pb) * 32 + (lane & 31), b = fdiv(m, a.map.dP), p = m - b * a.map.P;
-            at[pb] = m >= M ? kNone : (mode == 0 ? (unsigned)m * 4u : ((unsigned)b * a.C * a.map.P + p) * 2u) + (unsigned)h4 * step;
+            const int mt = (wp * PB + pb) * 32 + (lane & 31), m = m0 + mt, b = fdiv(m, a.map.dP), p = m - b * a.map.P;
+            at[pb] = mode == 0 ? (unsigned)mt * 4u + (unsigned)h4 * step
+                               : (m >= M ? kNone : ((unsigned)b * a.C * a.map.P + p) * 2u + (unsigned)h4 * step);
         }
         for_each_const([&](auto I) INLINE {
             constexpr int ob = decltype(I)::value / 16, r = decltype(I)::value % 16;
-            const int n0 = nl + ob * 32 + 8 * (r >> 2) + (r & 3);
-            const bool ok = n0 + h4 < a.C;
+            const int n0 = n_lo + ob * 32 + 8 * (r >> 2) + (r & 3);
+            const bool ok = mode == 0 || n0 + h4 < a.C;
             float bias = 0.f;
             if (mode != 0 && a.bias) bias = bf16_to_f32(a.bias[ok ? n0 + h4 : 0]);
             for_each_const([&](auto J) INLINE {
@@ -456,9 +465,22 @@ __global__ void __launch_bounds__(kThreads, 1) conv_wide_kernel(ConvRowsArgs a)
             __builtin_amdgcn_sched_barrier(0);
         }, std::make_integer_sequence<int, OB * 16>{});
     };
-    if (!a.out) finish(std::integral_constant<int, 0>{});
+    if (!whole) finish(std::integral_constant<int, 0>{});
     else if (a.act == D2C_EPILOGUE_NONE) finish(std::integral_constant<int, 1>{});
     else finish(std::integral_constant<int, 2>{});
+}
+
+// out = bias + the partial sums of conv_wide_kernel's tiles from `nfull` on: a workgroup = a column of a tile
+__global__ void __launch_bounds__(kWMT) conv_wide_finish_kernel(ConvRowsArgs a, int NT)
+{
+    const int rest = blockIdx.x / NT, nt = blockIdx.x - rest * NT, item = a.nfull + rest, ct = item % a.nctile, tile = item / a.nctile;
+    const int n = ct * NT + nt, m = tile * kWMT + threadIdx.x;
+    if (n >= a.C || m >= a.map.N * a.map.P) return;
+    float v = a.bias ? bf16_to_f32(a.bias[n]) : 0.f;
+    const float *q = a.part + ((long)rest * a.nsplit * NT + nt) * kWMT + threadIdx.x;
+    for (int s = 0; s < a.nsplit; s++) v += q[(long)s * NT * kWMT];
+    const int b = fdiv(m, a.map.dP), p = m - b * a.map.P;
+    a.out[((long)b * a.C + n) * a.map.P + p] = f32_to_bf16(d2c_epilogue(v, a.act, a.act_scale));
 }
 
 // out[b][n][p] = bias[n] + the partial sums of (n, b * P + p)
@@ -759,10 +781,9 @@ __global__ void __launch_bounds__(256) conv_prepare_kernel(ConvPrepArgs a)
 
 // ============================================================ host side
 struct RowsPlan {
-    int MT, NT, KC, nchunk, nct, S, ntile, nsplit;
+    int MT, NT, KC, nchunk, nct, S, ntile, nsplit, nfull;
     size_t wt_bytes, part_bytes;
 };
-constexpr long kPartClocks = 100;     // a block of 32 x 32 partial sums, per compute unit
 // columns C, reduction over `depth` channels per tap, M rows
 RowsPlan rows_plan(int C, int depth, int K, int M, int ncu)
 {
@@ -770,28 +791,35 @@ RowsPlan rows_plan(int C, int depth, int K, int M, int ncu)
     p.KC = depth <= 32 ? 32 : 64;
     p.nchunk = (depth + p.KC - 1) / p.KC;
     p.S = K * p.nchunk;
-    // Tile and number of pieces that the steps of a tile are shared out to, by what they cost in matrix clocks of a
-    // compute unit: rounds over the workgroups that run at a time (two per compute unit with 128 rows, one with 256),
-    // each its steps and about four more for its start and end; a piece's partial sums are written and read once more.
-    // (clocks of a step: from the rates on large problems)
+    // Tile, and number of pieces that the steps of a tile are shared out to, by what they cost in clocks of a compute unit:
+    // rounds over the workgroups that run at a time, each its steps and about four more for its start and end; partial sums
+    // are written and read once more.  (clocks of a step: from the rates on large problems)
     long best = -1;
-    auto consider = [&](int MT, int NT, long slots, long step_clocks) {
-        const int nct = (C + NT - 1) / NT, ntile = (M + MT - 1) / MT;
-        const long items = (long)ntile * nct;
-        for (int s = 1; s <= 16 && s <= p.S; s++) {
-            const long rounds = (items * s + slots - 1) / slots;
-            const long cost = rounds * ((p.S + s - 1) / s + 4) * step_clocks +
-                              (s > 1 ? (items * s * (MT / 32) * (NT / 32) + ncu - 1) / ncu * kPartClocks : 0);
-            if (best < 0 || cost * 20 < best * 19) { best = cost; p.MT = MT; p.NT = NT; p.nct = nct; p.ntile = ntile; p.nsplit = s; }
-        }
+    auto take = [&](long cost, int MT, int NT, int s, long full) {
+        if (best >= 0 && cost * 20 >= best * 19) return;
+        best = cost;
+        p.MT = MT; p.NT = NT; p.nsplit = s; p.nfull = (int)full; p.nct = (C + NT - 1) / NT; p.ntile = (M + MT - 1) / MT;
     };
-    consider(kMT, C <= 32 ? 32 : (C <= 64 ? 64 : 128), 2L * ncu, C <= 32 ? 1500 : (C <= 64 ? 2000 : 3000));
-    // (its results and partial sums are written through 32-bit offsets)
-    const bool wide = p.KC == 64 && (size_t)C * M * 4 < 0xFFFF0000u;
-    if (wide && C > 64) consider(kWMT, 128, ncu, 1700);
-    if (wide && C > 128) consider(kWMT, 256, ncu, 2800);
+    auto parts = [&](long pieces, int MT, int NT) { return (pieces * (MT / 32) * (NT / 32) + ncu - 1) / ncu * 600 + 8000; };
+    {
+        // two workgroups to a compute unit; all tiles are shared out alike
+        const int NT = C <= 32 ? 32 : (C <= 64 ? 64 : 128);
+        const long items = (long)((M + kMT - 1) / kMT) * ((C + NT - 1) / NT), slots = 2L * ncu, clocks = C <= 32 ? 1500 : (C <= 64 ? 2000 : 2700);
+        for (int s = 1; s <= 16 && s <= p.S; s++)
+            take((items * s + slots - 1) / slots * ((p.S + s - 1) / s + 4) * clocks + (s > 1 ? parts(items * s, kMT, NT) : 0), kMT, NT, s, 0);
+    }
+    // one workgroup to a compute unit; the tiles of the last, partly filled round are shared out (results are written through
+    // 32-bit offsets)
+    for (int NT = 128; NT <= 256 && C > NT / 2 && p.KC == 64 && (size_t)C * M * 2 < 0xFFFF0000u; NT *= 2) {
+        const long items = (long)((M + kWMT - 1) / kWMT) * ((C + NT - 1) / NT), full = items / ncu * ncu, rest = items - full,
+                   clocks = NT == 256 ? 3500 : 2100;
+        for (int s = 1; s <= 16 && s <= p.S; s++)
+            take(full / ncu * (p.S + 4) * clocks + (rest * s + ncu - 1) / ncu * ((p.S + s - 1) / s + 4) * clocks + (s > 1 ? parts(rest * s, kWMT, NT) : 0),
+                 kWMT, NT, s, s == 1 ? items : full);
+    }
     p.wt_bytes = d2c_align_up((size_t)p.S * p.nct * p.NT * p.KC * 2);
-    p.part_bytes = p.nsplit > 1 ? d2c_align_up((size_t)p.nsplit * C * M * sizeof(float)) : 0;
+    p.part_bytes = p.nsplit == 1 ? 0
+                 : d2c_align_up((p.MT == kWMT ? ((size_t)p.ntile * p.nct - p.nfull) * p.nsplit * kWMT * p.NT : (size_t)p.nsplit * C * M) * sizeof(float));
     return p;
 }
 
@@ -805,24 +833,27 @@ template <int NT, int KC, bool COLS = false> int launch_rows(const ConvRowsArgs 
 template <int NT, bool COLS> int launch_wide(const ConvRowsArgs &a, hipStream_t st)
 {
     D2cProfScope prof(D2C_PROF_FWD, st, "conv_wide_kernel");
-    hipLaunchKernelGGL((conv_wide_kernel<NT, COLS>), dim3((unsigned)(a.ntile * a.nsplit * a.nctile)), dim3(kThreads), 0, st, a);
+    const int rest = a.ntile * a.nctile - a.nfull;
+    hipLaunchKernelGGL((conv_wide_kernel<NT, COLS>), dim3((unsigned)(a.nfull + rest * a.nsplit)), dim3(kThreads), 0, st, a);
+    if (rest > 0) hipLaunchKernelGGL(conv_wide_finish_kernel, dim3((unsigned)(rest * NT)), dim3(kWMT), 0, st, a, NT);
     return d2c_check_launch("conv_wide_kernel");
 }
 
 int run_rows(const RowsPlan &p, const RowMap &map, const void *src, unsigned rowb, unsigned zrow, const void *wt, const void *bias,
              void *out, float *part, int C, hipStream_t st, int cols_K = 0, int cols_rows = 0, int act = 0, float act_scale = 1.f)
 {
-    ConvRowsArgs a{map, (const unsigned char *)src, (const unsigned char *)wt, p.nsplit > 1 ? nullptr : (const bf16_t *)bias,
-                   p.nsplit > 1 ? nullptr : (bf16_t *)out, part, rowb, zrow, C, p.nchunk, p.S, p.ntile, p.nct, p.nsplit,
+    const bool wide = p.MT == kWMT, sums = p.nsplit > 1 && !wide;
+    ConvRowsArgs a{map, (const unsigned char *)src, (const unsigned char *)wt, sums ? nullptr : (const bf16_t *)bias,
+                   sums ? nullptr : (bf16_t *)out, part, rowb, zrow, C, p.nchunk, p.S, p.ntile, p.nct, p.nsplit, p.nfull,
                    cols_K, cols_rows, act, act_scale};
     int rc;
-    if (p.MT == kWMT)
+    if (wide)
         rc = p.NT == 256 ? (cols_K > 0 ? launch_wide<256, true>(a, st) : launch_wide<256, false>(a, st))
                          : (cols_K > 0 ? launch_wide<128, true>(a, st) : launch_wide<128, false>(a, st));
     else if (cols_K > 0) rc = p.NT == 32 ? launch_rows<32, 64, true>(a, st) : (p.NT == 64 ? launch_rows<64, 64, true>(a, st) : launch_rows<128, 64, true>(a, st));
     else if (p.KC == 32) rc = p.NT == 32 ? launch_rows<32, 32>(a, st) : (p.NT == 64 ? launch_rows<64, 32>(a, st) : launch_rows<128, 32>(a, st));
     else rc = p.NT == 32 ? launch_rows<32, 64>(a, st) : (p.NT == 64 ? launch_rows<64, 64>(a, st) : launch_rows<128, 64>(a, st));
-    if (rc || p.nsplit == 1) return rc;
+    if (rc || !sums) return rc;
     const int M = map.N * map.P;
     D2cProfScope prof(D2C_PROF_PACK, st);
     hipLaunchKernelGGL(conv_rows_finish_kernel, dim3((M + 255) / 256, C), dim3(256), 0, st, part, (const bf16_t *)bias, (bf16_t *)out,
