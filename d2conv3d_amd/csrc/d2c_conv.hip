@@ -286,6 +286,43 @@ __global__ void __launch_bounds__(kThreads, 2) conv_rows_kernel(ConvRowsArgs a)
     }
 }
 
+// One k-group of the wide kernels below: OB x PB matrix instructions on operand set KG & 1, and between them the reads of the
+// next k-group's operands into the other set and whatever `request` has for a slot.  The reads are spread over the group (the
+// four wavefronts share the LDS)
+// and waited for one by one, in the order in which the instructions need them: weights 0, rows 0 .. PB-1, weights 1 ...
+// The last k-group of a step meets `sync` in slot kSync and reads from the next step's buffers after it.
+template <int OB, int PB, int KG, class Read, class Request, class Sync>
+D2C_DEV void wide_group(f32x16 (&acc)[OB][PB], u32x4_t (&fa)[2][PB], u32x4_t (&fb)[2][OB], Read read, Request request, Sync sync)
+{
+    constexpr int NM = OB * PB, NR = OB + PB, s = KG & 1, lo = KG == 3 ? NM * 3 / 8 : 0;
+    for_each_const([&](auto I) INLINE {
+        constexpr int i = decltype(I)::value, ob = i / PB, pb = i % PB;
+        constexpr int issued = i <= lo ? 0 : ((i - lo) * NR + NM - lo - 1) / (NM - lo);        // reads of this group before slot i
+        if constexpr (KG == 3 && i == lo) sync();
+        if constexpr (pb == 0 || ob == 0) {
+            // the operand(s) that this instruction is the first to need
+            constexpr int need = ob == 0 ? 1 + pb : PB + ob, later = NR - 1 - need + issued;
+            if constexpr (KG == 3 && i >= lo) {
+                if constexpr (pb == 0) asm volatile("" : "+v"(fb[s][ob]));
+                if constexpr (ob == 0) asm volatile("" : "+v"(fa[s][pb]));
+            } else {
+                if constexpr (pb == 0) wait_lds<later>(fb[s][ob]);
+                if constexpr (ob == 0) wait_lds<later>(fa[s][pb]);
+            }
+        }
+        mma_kgroup<bf16_t, false>(acc[ob][pb], __builtin_bit_cast(uint4, fb[s][ob]), __builtin_bit_cast(uint4, fa[s][pb]));
+        constexpr int next = i < lo ? 0 : ((i + 1 - lo) * NR + NM - lo - 1) / (NM - lo);
+        for_each_const([&](auto R) INLINE {
+            constexpr int r = issued + decltype(R)::value;
+            if constexpr (r == 0) read(std::integral_constant<int, 0>{}, fb[s ^ 1][0]);
+            else if constexpr (r <= PB) read(std::integral_constant<int, OB + r - 1>{}, fa[s ^ 1][r - 1]);
+            else read(std::integral_constant<int, r - PB>{}, fb[s ^ 1][r - PB]);
+        }, std::make_integer_sequence<int, next - issued>{});
+        request(I);
+        __builtin_amdgcn_sched_barrier(0);
+    }, std::make_integer_sequence<int, NM>{});
+}
+
 // The same product for larger problems: a workgroup = 256 rows x NT columns (256 or 128), four wavefronts of 128 x NT/2,
 // one workgroup per compute unit.  A step of 64 channels is 2048 matrix clocks (NT = 256) against 1024 clocks of LDS
 // reads and 512 of DMA writes; the 128 x 128 tile above has 768 clocks of LDS traffic for 512 matrix clocks.  Rows are
@@ -380,11 +417,10 @@ __global__ void __launch_bounds__(kThreads, 1) conv_wide_kernel(ConvRowsArgs a)
         slot[kg] = (unsigned)((lane & 31) * ROWB + tile_slot<64>(lane & 31, kg * 2 + (lane >> 5)) * 16);
     const unsigned ra = lds_address(s_t) + wp * PB * 32 * ROWB, rb = lds_address(s_t) + 3 * ABYTES + wo * OB * 32 * ROWB;
     u32x4_t fa[2][PB], fb[2][OB];
-    // operand vector i of a k-group: weights first
-    auto operand = [&](auto I, auto S, unsigned pa, unsigned pb, unsigned sl) INLINE {
-        constexpr int i = decltype(I)::value, s = decltype(S)::value;
-        if constexpr (i < OB) fb[s][i] = lds_read16(pb + sl + i * 32 * ROWB);
-        else fa[s][i - OB] = lds_read16(pa + sl + (i - OB) * 32 * ROWB);
+    // operand vector i of a k-group: weights, then rows
+    auto operand = [&](auto I, u32x4_t &v, unsigned pa, unsigned pb, unsigned sl) INLINE {
+        constexpr int i = decltype(I)::value;
+        v = i < OB ? lds_read16(pb + sl + i * 32 * ROWB) : lds_read16(pa + sl + (i - OB) * 32 * ROWB);
     };
 
     tap_rows();
@@ -397,31 +433,27 @@ __global__ void __launch_bounds__(kThreads, 1) conv_wide_kernel(ConvRowsArgs a)
     for (int i = 0; i < BD; i++) weight_request(i, 1);
     wait_vm<AD + BD>();
     group_barrier();
-    for_each_const([&](auto I) INLINE { operand(I, std::integral_constant<int, 0>{}, ra, rb, slot[0]); }, std::make_integer_sequence<int, OB + PB>{});
+    // (in the order of wide_group)
+    operand(std::integral_constant<int, 0>{}, fb[0][0], ra, rb, slot[0]);
+    for_each_const([&](auto I) INLINE { operand(std::integral_constant<int, OB + decltype(I)::value>{}, fa[0][decltype(I)::value], ra, rb, slot[0]); },
+                   std::make_integer_sequence<int, PB>{});
+    for_each_const([&](auto I) INLINE { operand(std::integral_constant<int, 1 + decltype(I)::value>{}, fb[0][1 + decltype(I)::value], ra, rb, slot[0]); },
+                   std::make_integer_sequence<int, OB - 1>{});
     int abuf = 0, bbuf = 0;
     for (int st = st_lo; st < st_hi; st++) {
         if (st + 2 < st_hi) bsrc += bstep;
         const int a1 = abuf == 2 ? 0 : abuf + 1, a2 = a1 == 2 ? 0 : a1 + 1, b1 = bbuf ^ 1;
         for_each_const([&](auto KG) INLINE {
-            constexpr int kg = decltype(KG)::value, s = kg & 1;
-#pragma unroll
-            for (int ob = 0; ob < OB; ob++) wait_lds<0>(fb[s][ob]);
-#pragma unroll
-            for (int pb = 0; pb < PB; pb++) asm volatile("" : "+v"(fa[s][pb]));
-            unsigned pa = ra + abuf * ABYTES, pb_ = rb + bbuf * BBYTES;
-            if constexpr (kg == 3) {
-                wait_vm<AD>();                             // (the rows of the step after the next one may be under way)
-                asm volatile("s_barrier" ::: "memory");
-                pa = ra + a1 * ABYTES; pb_ = rb + b1 * BBYTES;
-            }
-            for_each_const([&](auto I) INLINE {
-                constexpr int i = decltype(I)::value, ob = i / PB, pb = i % PB;
-                mma_kgroup<bf16_t, false>(acc[ob][pb], __builtin_bit_cast(uint4, fb[s][ob]), __builtin_bit_cast(uint4, fa[s][pb]));
-                if constexpr (i < OB + PB) operand(I, std::integral_constant<int, s ^ 1>{}, pa, pb_, slot[(kg + 1) & 3]);
-                if constexpr ((kg == 0 || kg == 1) && i < AD / 2) row_request(kg * (AD / 2) + i, a2);
-                if constexpr (kg == 3 && i < BD) weight_request(i, bbuf);
-                __builtin_amdgcn_sched_barrier(0);
-            }, std::make_integer_sequence<int, NM>{});
+            constexpr int kg = decltype(KG)::value;
+            const unsigned pa = ra + (kg == 3 ? a1 : abuf) * ABYTES, pb_ = rb + (kg == 3 ? b1 : bbuf) * BBYTES;
+            wide_group<OB, PB, kg>(acc, fa, fb, [&](auto I, u32x4_t &v) INLINE { operand(I, v, pa, pb_, slot[(kg + 1) & 3]); },
+                [&](auto I) INLINE {
+                    constexpr int i = decltype(I)::value, n = NM / (AD / 2);
+                    if constexpr ((kg == 1 || kg == 2) && i % n == 0) row_request((kg - 1) * (AD / 2) + i / n, a2);
+                    if constexpr (kg == 3 && i >= NM * 3 / 8 && i - NM * 3 / 8 < BD) weight_request(i - NM * 3 / 8, bbuf);
+                },
+                // (the rows of the step after the next one may be under way)
+                [&]() INLINE { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(AD) : "memory"); });
         }, std::make_integer_sequence<int, 4>{});
         advance();
         abuf = a1; bbuf = b1;
@@ -494,6 +526,192 @@ __global__ void __launch_bounds__(256) conv_rows_finish_kernel(const float *part
     for (int s = 0; s < nsplit; s++) v += q[(long)s * C * M];
     const int b = fdiv(m, dP), p = m - b * P;
     out[((long)b * C + n) * P + p] = f32_to_bf16(d2c_epilogue(v, act, act_scale));
+}
+
+// ============================================================ grad-column rows of the deformable operator
+//   gcol[pair][m][c] = sum_o gout[m][o] * W[o][64 j + c][tap]     (pair = chunk j of 64 input channels and tap)
+// The pipeline of conv_wide_kernel over 256 rows x 256 columns (four pairs), with a reduction of a few steps only: so a
+// workgroup goes through a run of tiles, one per compute unit in all, and the requests for the next tile's first steps are
+// under way while a tile ends.  Runs go along the columns of a row tile.  An XCD's workgroups share a range of column tiles
+// whose weights fit its L2 (cgroups ranges) and, where there are fewer than eight, a range of row tiles.  The rows of the
+// weight operand are permuted so that a lane's 16 results of a 32 x 32 block are 16 consecutive channels.  Results leave by
+// whole rows, through LDS (16 bytes a lane, 64 rows apart: twice the time for the whole kernel).  Both operands come from the
+// caches, so one step of requests ahead is enough.
+// 256 -> 256 channels on 32x60x108: 0.97 ms and 0.06 for the operands, before 1.23; writing 2.9 GB of rows takes 0.6.
+struct GradColArgs {
+    const unsigned char *src;         // channels-last grad_out, rows of `rowb` bytes
+    const unsigned char *wt;          // [column tile][step][256][64] bfloat16, slots swizzled
+    bf16_t *gcol;
+    unsigned rowb;
+    int M, npair, S, ntile, nct, cgroups;
+};
+__global__ void __launch_bounds__(kThreads, 1) grad_col_kernel(GradColArgs a)
+{
+    constexpr int OB = 4, PB = 4, NT = 256;
+    constexpr int ROWB = 128, ABYTES = kWMT * ROWB, BBYTES = NT * ROWB;
+    constexpr int AD = 8, BD = BBYTES / 4096, NM = OB * PB;
+    __shared__ __align__(1024) unsigned char s_t[2 * ABYTES + 2 * BBYTES + 4 * 4096];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int xcd = blockIdx.x & 7, j = (int)blockIdx.x >> 3, per = (int)gridDim.x >> 3, rgroups = 8 / a.cgroups;
+    const int cg = xcd % a.cgroups, rg = xcd / a.cgroups;
+    const int c_lo = a.nct * cg / a.cgroups, c_hi = a.nct * (cg + 1) / a.cgroups, nc = c_hi - c_lo;
+    const int r_lo = a.ntile * rg / rgroups, r_hi = a.ntile * (rg + 1) / rgroups;
+    const long units = (long)(r_hi - r_lo) * nc;
+    const int u_lo = (int)(units * j / per), u_hi = (int)(units * (j + 1) / per);
+    if (u_lo >= u_hi) return;
+
+    // --- what is requested next: a step of the rows, a step of the weights
+    const int lrow = lane >> 3;
+    int arow = r_lo + u_lo / nc, acol = c_lo + u_lo % nc, aj = 0, aleft = (u_hi - u_lo) * a.S - 1;
+    int bj = 0, bcol = acol, bleft = aleft;
+    unsigned aoff[AD];
+    const unsigned char *asrc = a.src;
+    auto row_tile = [&]() {
+#pragma unroll
+        for (int i = 0; i < AD; i++) {
+            const int rl = wave * 64 + i * 8 + lrow;       // (rows past the last one: the last one, stored nowhere)
+            aoff[i] = (unsigned)min(arow * kWMT + rl, a.M - 1) * a.rowb + (unsigned)tile_slot<64>(rl & 31, lane & 7) * 16u;
+        }
+    };
+    // (after the last step: that step again, which nothing reads)
+    auto advance_rows = [&]() {
+        if (aleft == 0) return;
+        aleft--;
+        asrc += ROWB;
+        if (++aj < a.S) return;
+        aj = 0; asrc = a.src;
+        if (++acol < c_hi) return;
+        acol = c_lo; arow++;
+        row_tile();
+    };
+    const unsigned char *bsrc = a.wt + (long)bcol * a.S * BBYTES + wave * 1024 + lane * 16;
+    auto advance_weights = [&]() {
+        if (bleft == 0) return;
+        bleft--;
+        bsrc += BBYTES;
+        if (++bj < a.S) return;
+        bj = 0;
+        if (++bcol < c_hi) return;
+        bcol = c_lo;
+        bsrc -= (long)nc * a.S * BBYTES;
+    };
+    unsigned char *const sa = s_t + wave * (64 * ROWB), *const sb = s_t + 2 * ABYTES + wave * 1024;
+    auto row_request = [&](int i, int buf) { dma16(asrc + aoff[i], sa + buf * ABYTES + i * 1024); };
+    auto weight_request = [&](int i, int buf) { dma16(bsrc + i * 4096, sb + buf * BBYTES + i * 4096); };
+
+    f32x16 acc[OB][PB];
+    const int wo = wave & 1, wp = wave >> 1, h = lane >> 5;
+    unsigned slot[4];
+#pragma unroll
+    for (int kg = 0; kg < 4; kg++)
+        slot[kg] = (unsigned)((lane & 31) * ROWB + tile_slot<64>(lane & 31, kg * 2 + h) * 16);
+    const unsigned ra = lds_address(s_t) + wp * PB * 32 * ROWB, rb = lds_address(s_t) + 2 * ABYTES + wo * OB * 32 * ROWB;
+    u32x4_t fa[2][PB], fb[2][OB];
+    // operand vector i of a k-group: weights, then rows
+    auto operand = [&](auto I, u32x4_t &v, unsigned pa, unsigned pb, unsigned sl) INLINE {
+        constexpr int i = decltype(I)::value;
+        v = i < OB ? lds_read16(pb + sl + i * 32 * ROWB) : lds_read16(pa + sl + (i - OB) * 32 * ROWB);
+    };
+
+    row_tile();
+    for (int i = 0; i < AD; i++) row_request(i, 0);
+    for (int i = 0; i < BD; i++) weight_request(i, 0);
+    advance_rows();
+    advance_weights();
+    for (int i = 0; i < AD; i++) row_request(i, 1);
+    for (int i = 0; i < BD; i++) weight_request(i, 1);
+    wait_vm<AD + BD>();
+    group_barrier();
+    // (in the order of wide_group)
+    operand(std::integral_constant<int, 0>{}, fb[0][0], ra, rb, slot[0]);
+    for_each_const([&](auto I) INLINE { operand(std::integral_constant<int, OB + decltype(I)::value>{}, fa[0][decltype(I)::value], ra, rb, slot[0]); },
+                   std::make_integer_sequence<int, PB>{});
+    for_each_const([&](auto I) INLINE { operand(std::integral_constant<int, 1 + decltype(I)::value>{}, fb[0][1 + decltype(I)::value], ra, rb, slot[0]); },
+                   std::make_integer_sequence<int, OB - 1>{});
+    // a wavefront's results on their way out: 32 rows of a pair, written by (row, half), read 8 lanes to a row
+    const unsigned stage = lds_address(s_t) + 2 * ABYTES + 2 * BBYTES + wave * 4096;
+    const unsigned ov = (lane >> 3) * 128u + (lane & 7) * 16u;
+    int buf = 0;
+    int row = r_lo + u_lo / nc, col = c_lo + u_lo % nc;
+    for (int u = u_lo; u < u_hi; u++) {
+#pragma unroll
+        for (int ob = 0; ob < OB; ob++)
+#pragma unroll
+            for (int pb = 0; pb < PB; pb++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[ob][pb][r] = 0.f;
+        for (int st = 0; st < a.S; st++) {
+            advance_rows();
+            advance_weights();
+            const int nbuf = buf ^ 1;
+            auto group = [&](auto KG) INLINE {
+                constexpr int kg = decltype(KG)::value;
+                const int b = kg == 3 ? nbuf : buf;
+                const unsigned pa = ra + b * ABYTES, pb_ = rb + b * BBYTES;
+                wide_group<OB, PB, kg>(acc, fa, fb, [&](auto I, u32x4_t &v) INLINE { operand(I, v, pa, pb_, slot[(kg + 1) & 3]); },
+                    [&](auto I) INLINE {
+                        constexpr int d = decltype(I)::value - NM * 3 / 8;
+                        if constexpr (kg == 3 && d >= 0 && d < AD) { row_request(d, buf); weight_request(d, buf); }
+                    },
+                    [&]() INLINE {
+                        // (the stores of the tile before, younger than these requests, may be under way)
+                        if (st == 0 && u > u_lo) wait_vm<32>(); else wait_vm<0>();
+                        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                    });
+            };
+            for_each_const(group, std::make_integer_sequence<int, 4>{});
+            buf = nbuf;
+        }
+        // results, 32 rows of a pair at a time, by whole rows; those past the last one fall outside the pair's descriptor
+        u32x4_t v[2][4];
+        for_each_const([&](auto R) INLINE {
+            constexpr int r = decltype(R)::value;
+            if constexpr (r < 8) {
+                constexpr int pb = r & 3;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const f32x16 &x = acc[(r >> 2) * 2 + (q >> 1)][pb];
+                    const int e = (q & 1) * 8;
+                    u32x4_t t = {pack_bf16x2(x[e], x[e + 1]), pack_bf16x2(x[e + 2], x[e + 3]), pack_bf16x2(x[e + 4], x[e + 5]), pack_bf16x2(x[e + 6], x[e + 7])};
+                    asm volatile("ds_write_b128 %0, %1" ::"v"(stage + (lane & 31) * 128u + tile_slot<64>(lane & 31, (q >> 1) * 4 + h * 2 + (q & 1)) * 16u), "v"(t));
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    v[r & 1][i] = lds_read16(stage + i * 1024 + (lane >> 3) * 128u + tile_slot<64>(i * 8 + (lane >> 3), lane & 7) * 16u);
+            }
+            if constexpr (r > 0) {
+                constexpr int o = r - 1, pb = o & 3;
+                const int pair = col * 4 + wo * 2 + (o >> 2);
+                const auto rs = __builtin_amdgcn_make_buffer_rsrc(a.gcol + (long)pair * a.M * 64, 0, pair < a.npair ? (int)((unsigned)a.M * 128u) : 0, 0x00020000);
+#pragma unroll
+                for (int i = 0; i < 4; i++) wait_lds<r < 8 ? 8 : 0>(v[o & 1][i]);
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    __builtin_amdgcn_raw_buffer_store_b128(v[o & 1][i], rs, (int)((unsigned)(row * kWMT + (wp * PB + pb) * 32 + i * 8) * 128u + ov), 0, 2);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }, std::make_integer_sequence<int, 9>{});
+        if (++col == c_hi) { col = c_lo; row++; }
+    }
+#pragma unroll
+    for (int ob = 0; ob < OB; ob++) wait_lds<0>(fb[0][ob]);
+#pragma unroll
+    for (int pb = 0; pb < PB; pb++) asm volatile("" : "+v"(fa[0][pb]));
+    wait_vm<0>();
+}
+// W[o][c][tap] -> the operand order above: a thread makes one vector of eight o of a (channel, tap)
+__global__ void __launch_bounds__(256) grad_col_weights_kernel(const bf16_t *w, uint4 *wt, int Cout, int Cin, int K, FastDiv dK, int S)
+{
+    const int e = blockIdx.x * 256 + threadIdx.x, v = blockIdx.y, CK = Cin * K;
+    if (e >= CK) return;
+    alignas(16) bf16_t t[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) t[q] = v * 8 + q < Cout ? w[(long)(v * 8 + q) * CK + e] : (bf16_t)0;
+    const int c = fdiv(e, dK), k = e - c * K, pair = (c >> 6) * K + k, ch = c & 31;
+    const int r = (pair & 3) * 64 + (c & 32) + 8 * ((ch & 15) >> 2) + 4 * (ch >> 4) + (ch & 3);
+    wt[(((long)(pair >> 2) * S + (v >> 3)) * 256 + r) * 8 + tile_slot<64>(r & 31, v & 7)] = *reinterpret_cast<const uint4 *>(t);
 }
 
 // ============================================================ grad_weight
@@ -664,12 +882,14 @@ struct ConvPrepArgs {
     const bf16_t *gout;
     bf16_t *gcl;
     uint4 *gp;
-    int Cp, OBP, P, M, ngt, ngc, nblk_g;
+    int Cp, OBP, P, M, ngt, ngc, nblk_g, gwide;
     FastDiv dP;
     // bias gradient
     bf16_t *gb;
     int nblk_b;
 };
+// eight positions at a time: whole in a sample, and aligned
+inline int wide_gout(const void *gout, int P) { return P % 8 == 0 && reinterpret_cast<uintptr_t>(gout) % 16 == 0; }
 
 __global__ void __launch_bounds__(256) conv_prepare_kernel(ConvPrepArgs a)
 {
@@ -743,7 +963,17 @@ __global__ void __launch_bounds__(256) conv_prepare_kernel(ConvPrepArgs a)
         // 64 positions x 64 channels of grad_out, into both orders
         const int gt = b % a.ngt, gc = b / a.ngt;
         constexpr int GS = 72;                               // [channel][position], 16-byte aligned rows
-        for (int i = threadIdx.x; i < 4096; i += 256) {
+        if (a.gwide) {
+            for (int i = threadIdx.x; i < 512; i += 256) {
+                const int c = gc * 64 + i / 8, m = gt * 64 + (i % 8) * 8;
+                uint4 v = make_uint4(0, 0, 0, 0);
+                if (c < a.Cout && m < a.M) {
+                    const int n = fdiv(m, a.dP), p = m - n * a.P;
+                    v = *reinterpret_cast<const uint4 *>(a.gout + ((long)n * a.Cout + c) * a.P + p);
+                }
+                *reinterpret_cast<uint4 *>(s_t + (i / 8) * GS + (i % 8) * 8) = v;
+            }
+        } else for (int i = threadIdx.x; i < 4096; i += 256) {
             const int c = gc * 64 + i / 64, m = gt * 64 + i % 64;
             bf16_t v = 0;
             if (c < a.Cout && m < a.M) {
@@ -927,6 +1157,61 @@ int d2c_col_forward(const d2c_conv3d_desc &q, const void *col, int rows, const v
                     q.epilogue_scale);
 }
 
+// ---- grad-column rows [chunk][tap][N*P][64] of the deformable operator's backward pass, one weight group
+namespace {
+struct GradColPlan {
+    int Cp, S, ntile, nct, cgroups;
+    size_t wt_bytes, total;
+};
+GradColPlan grad_col_plan(const d2c_conv3d_desc &q)
+{
+    GradColPlan p;
+    const int M = q.N * q.Do * q.Ho * q.Wo;
+    p.Cp = (q.Cout + 63) / 64 * 64;
+    p.S = p.Cp / 64;
+    p.ntile = (M + kWMT - 1) / kWMT;
+    p.nct = (q.Cin / 64 * q.kd * q.kh * q.kw + 3) / 4;
+    p.wt_bytes = d2c_align_up((size_t)p.nct * p.S * 256 * 128);
+    p.total = p.wt_bytes + d2c_align_up((size_t)M * p.Cp * 2 + 1024);
+    p.cgroups = 1;
+    while (p.cgroups < 8 && p.wt_bytes / p.cgroups > (2u << 20)) p.cgroups *= 2;
+    return p;
+}
+}  // namespace
+// Where there are tiles enough for every compute unit to take several, and up to 256 output channels (with more, the kernel
+// that holds a grad_out tile in LDS and reads grad_out where it lies reaches the same rate: 512 -> 512 on 2x8x30x54 380 us
+// against 400, and 40 to put the operands in order); grad_out within 32-bit offsets.
+bool d2c_grad_col_supported(const d2c_conv3d_desc &q)
+{
+    const GradColPlan p = grad_col_plan(q);
+    return q.dtype == D2C_BF16 && q.groups == 1 && q.Cin % 64 == 0 && q.Cout > 32 && q.Cout <= 256 &&
+           (size_t)q.N * q.Do * q.Ho * q.Wo * p.Cp * 2 + 1024 < 0xFFFF0000u && (long)p.ntile * p.nct >= 4L * d2c_num_cus() &&
+           (long)p.ntile * p.nct * p.S < (1L << 30) && (size_t)q.N * q.Do * q.Ho * q.Wo * 128 < 0xFFFF0000u;
+}
+size_t d2c_grad_col_ws(const d2c_conv3d_desc &q) { return grad_col_plan(q).total; }
+int d2c_grad_col(const d2c_conv3d_desc &q, const void *gout, const void *w, void *gcol, void *ws, hipStream_t st)
+{
+    const GradColPlan p = grad_col_plan(q);
+    const int K = q.kd * q.kh * q.kw, P = q.Do * q.Ho * q.Wo, M = q.N * P, ncu = d2c_num_cus();
+    if (ncu <= 0) return D2C_ERR_LAUNCH;
+    char *const gcl = (char *)ws + p.wt_bytes;
+    {
+        D2cProfScope prof(D2C_PROF_PACK, st);
+        hipLaunchKernelGGL(grad_col_weights_kernel, dim3((unsigned)((q.Cin * K + 255) / 256), (unsigned)(p.S * 8)), dim3(256), 0, st,
+                           (const bf16_t *)w, (uint4 *)ws, q.Cout, q.Cin, K, make_fastdiv(K), p.S);
+        ConvPrepArgs a{};
+        a.gout = (const bf16_t *)gout; a.gcl = (bf16_t *)gcl; a.Cout = q.Cout; a.Cp = p.Cp; a.P = P; a.M = M; a.dP = make_fastdiv(P);
+        a.gwide = wide_gout(gout, P); a.ngt = (M + 63) / 64; a.ngc = p.Cp / 64; a.nblk_g = a.ngt * a.ngc;
+        hipLaunchKernelGGL(conv_prepare_kernel, dim3((unsigned)a.nblk_g), dim3(256), 0, st, a);
+        if (int rc = d2c_check_launch("conv_prepare_kernel")) return rc;
+    }
+    GradColArgs a{(const unsigned char *)gcl, (const unsigned char *)ws, (bf16_t *)gcol, (unsigned)p.Cp * 2u, M, q.Cin / 64 * K, p.S, p.ntile,
+                  p.nct, p.cgroups};
+    D2cProfScope prof(D2C_PROF_BWD_DATA, st, "grad_col_kernel");
+    hipLaunchKernelGGL(grad_col_kernel, dim3((unsigned)std::max(8, ncu / 8 * 8)), dim3(kThreads), 0, st, a);
+    return d2c_check_launch("grad_col_kernel");
+}
+
 bool d2c_plain_supported(const d2c_conv3d_desc &q) { return plain_shape_ok(q); }
 size_t d2c_plain_input_bytes(const d2c_conv3d_desc &q) { return (size_t)q.N * q.Cin * q.D * q.H * q.W * 2 + 1024; }
 
@@ -1007,6 +1292,7 @@ int d2c_plain_backward(const d2c_conv3d_desc &q, const void *gout, const void *x
         a.gcl = gx ? (bf16_t *)(base + l.gcl) : nullptr;
         a.gp = gw ? (uint4 *)(base + l.gp) : nullptr;
         a.Cp = Cp; a.OBP = p.OBP; a.P = P; a.M = M; a.dP = make_fastdiv(P);
+        a.gwide = wide_gout(gout, P);
         a.ngt = (M + 63) / 64;
         a.ngc = std::max((Cp + 63) / 64, (p.OBP + 1) / 2);
         a.nblk_g = (gx || gw) ? a.ngt * a.ngc : 0;

@@ -7,6 +7,9 @@
 
 size_t d2c_col_forward_ws(const d2c_conv3d_desc &q);
 int d2c_col_forward(const d2c_conv3d_desc &q, const void *col, int rows, const void *w, const void *bias, void *out, void *ws, hipStream_t st);
+bool d2c_grad_col_supported(const d2c_conv3d_desc &q);
+size_t d2c_grad_col_ws(const d2c_conv3d_desc &q);
+int d2c_grad_col(const d2c_conv3d_desc &q, const void *gout, const void *w, void *gcol, void *ws, hipStream_t st);
 int d2c_fwd_out_tile(const TiledShape &s);
 template <typename T>
 int d2c_tiled_fwd_launch(const TiledShape &s, const void *xcl, const void *off, const void *mask, const void *wp,
@@ -638,7 +641,7 @@ BwdSlices bwd_slices(const d2c_conv3d_desc &q, const TiledShape &s)
 }
 
 struct BwdWs {
-    size_t xcl, wt, gxcl, gwacc, goutp, auxacc, gcol, counts, entries, ovf, gsacc, sm1, brick, col, total;
+    size_t xcl, wt, gxcl, gwacc, goutp, auxacc, gcol, counts, entries, ovf, gsacc, sm1, brick, gemm, col, total;
 };
 // `saved_columns`: the caller brings the sampled columns of the forward call (no column region, no slices)
 BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns = false)
@@ -682,6 +685,8 @@ BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns =
     if (s.ss.on) w.total += d2c_align_up((size_t)s.N * 3 * s.P * sizeof(float));
     w.brick = w.total;
     if (use_brick(q, s)) w.total += d2c_brick_ws(s).total + d2c_brick_ws(s).res_bytes;
+    w.gemm = w.total;      // operands of the grad-column product
+    if (use_brick(q, s) && d2c_grad_col_supported(q)) w.total += d2c_grad_col_ws(q);
     w.col = w.total;       // sampled columns for the grad-weight product
     if (!saved_columns && use_col_weight(q, s) && !col_in_place(q, s))
         w.total += d2c_align_up(d2c_bwd_col_bytes(s, q.dtype, sl.cgs ? sl.cgs * (s.cpg / 64) : 0));
@@ -842,7 +847,9 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
                 L = d2c_lists_make(s, Elem<T>::DT, base + l.counts, base + l.entries, base + l.ovf);
                 if (int rc = (auxk && !gw_in_place) ? d2c_lists_clear(L, st) : d2c_lists_build(s, off, mask, L, st)) return rc;
             }
-            if (int rc = d2c_tiled_bwd_data_launch<T>(s, gout, xcl_p, off, mask, w, wt_p,
+            if (brick && !prep && d2c_grad_col_supported(q)) {
+                if (int rc = d2c_grad_col(q, gout, w, base + l.gcol, base + l.gemm, st)) return rc;
+            } else if (int rc = d2c_tiled_bwd_data_launch<T>(s, gout, xcl_p, off, mask, w, wt_p,
                                                      lists ? nullptr : gxcl, (lists || auxk) ? base + l.gcol : nullptr,
                                                      auxk ? nullptr : goff, auxk ? nullptr : gmask,
                                                      (float *)(base + l.auxacc), st, 3, 0, 0, wt_packed))

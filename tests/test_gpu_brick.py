@@ -1,7 +1,7 @@
 """The kernels over sampling points sorted by 1x3x3 blocks of voxels, bfloat16: forward and all gradients against the CPU
 oracle where a block, a product of 32 points, a set of channel chunks or the volume ends, with points on, across and beyond the
-border; and the matrix product of the forward pass over sampled columns at the edges of its tiles, at zero offsets against
-the plain convolution."""
+border; and the matrix products of the forward pass over sampled columns and of the grad-column rows at the edges of their tiles, at zero
+offsets against the plain convolution."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -63,3 +63,19 @@ def test_columns_forward_at_tile_edges(Cin, Cout, dims, dev):
     b = torch.randn(Cout, generator=g).bfloat16()
     out = d2c.deform_conv3d(x.to(dev), torch.zeros(1, 81, *dims, device=dev), None, w.to(dev), b.to(dev), 1, 1, 1, 1, 1)
     assert rel_l2(out, F.conv3d(x.float(), w.float(), b.float(), padding=1)) < 5e-3
+
+
+# (reductions of one to four steps, last column tiles that are not full, one to eight ranges of column tiles, positions of a
+# sample that are not a multiple of eight)
+@pytest.mark.parametrize("N,Cin,Cout,dims", [(1, 256, 40, (1, 95, 131)), (2, 64, 72, (6, 61, 67)), (1, 256, 130, (13, 31, 32)),
+                                             (1, 320, 256, (2, 63, 65)), (1, 1024, 64, (1, 61, 60)), (1, 1024, 200, (1, 62, 60))])
+def test_grad_columns_at_tile_edges(N, Cin, Cout, dims, dev):
+    g = torch.Generator().manual_seed(Cin + Cout)
+    x = torch.randn(N, Cin, *dims, generator=g).bfloat16()
+    w = (torch.randn(Cout, Cin, 3, 3, 3, generator=g) / (Cin * 27) ** 0.5).bfloat16()
+    gout = torch.randn(N, Cout, *dims, generator=g).bfloat16()
+    xr = x.float().requires_grad_(True)
+    F.conv3d(xr, w.float(), padding=1).backward(gout.float())
+    xd = x.to(dev).requires_grad_(True)
+    d2c.deform_conv3d(xd, torch.zeros(N, 81, *dims, device=dev), None, w.to(dev), None, 1, 1, 1, 1, 1).backward(gout.to(dev))
+    assert rel_l2(xd.grad, xr.grad) < 1e-2
