@@ -460,7 +460,7 @@ def _ptr_at(t, channel):
     """Device pointer of t[:, channel] of a contiguous [N, C, *spatial] tensor (first sample)."""
     per_channel = 1
     for d in t.shape[2:]:
-        per_channel *= d
+        per_channel *= int(d)      # (torch.jit.trace makes the extents tensors)
     return ctypes.c_void_p(t.data_ptr() + channel * per_channel * t.element_size())
 
 

@@ -14,6 +14,7 @@
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/pybind.h>
 #include <torch/types.h>
 
@@ -41,10 +42,11 @@ void check(int rc, const char *what)
     if (rc != D2C_OK) throw std::runtime_error(std::string(what) + ": " + d2c_last_error() + " (code " + std::to_string(rc) + ")");
 }
 // (a tensor whose memory the kernels can take as it is: no subclass with its own dispatch, no functorch wrapper, no
-// forward-mode tangent)
+// forward-mode tangent; and no call that torch.jit.trace records: of one it would see the allocation of the result
+// alone, where the Python functions are recorded as operations)
 bool plain(const Tensor &t)
 {
-    return t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.has_storage() && !t.unsafeGetTensorImpl()->is_python_dispatch() &&
+    return t.defined() && !torch::jit::tracer::isTracing() && t.is_cuda() && t.layout() == at::kStrided && t.has_storage() && !t.unsafeGetTensorImpl()->is_python_dispatch() &&
            t.is_contiguous() && !t._fw_grad(0).defined();
 }
 int dtype_code(const Tensor &t)
