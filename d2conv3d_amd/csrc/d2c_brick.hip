@@ -25,7 +25,8 @@ typedef short v4s __attribute__((ext_vector_type(4)));
 struct BrickPoint {
     bool in;              // a corner is inside the volume
     int seg;              // its block
-    float y, x, hz;       // place inside the block along y and x, fraction along z
+    unsigned cell;        // its base voxel in the block: y | x << 2
+    float hz, hy, hx;     // fractions, as make_tap3 gives them
 };
 D2C_DEV int brick_seg(const BrickDims &d, int bg, int zi, int by, int bx) { return ((bg * d.nz + zi) * d.nby + by) * d.nbx + bx; }
 // (`c`: what tap_offsets_issue() read)
@@ -41,11 +42,8 @@ D2C_DEV BrickPoint brick_point(const TiledShape &s, const BrickDims &d, float *c
     BrickPoint r;
     r.in = t.inrange != 0;
     const int yq = (t.y0 + 1) / 3, xq = (t.x0 + 1) / 3;       // (base voxels start at -1)
-    // (exact from position 4 on, where a fraction has at most 21 bits, and within 2^-23 of a voxel below)
-    // (and never rounded up to the next base voxel, where the derivative is another one)
-    const float yb = (float)(t.y0 + 1 - yq * 3), xb = (float)(t.x0 + 1 - xq * 3);
-    r.y = fminf(yb + t.hy, yb + (1.f - 0x1p-22f)); r.x = fminf(xb + t.hx, xb + (1.f - 0x1p-22f));
-    r.hz = t.hz;
+    r.cell = (unsigned)(t.y0 + 1 - yq * 3) | (unsigned)(t.x0 + 1 - xq * 3) << 2;
+    r.hz = t.hz; r.hy = t.hy; r.hx = t.hx;
     r.seg = brick_seg(d, b * s.G + g, t.z0 + 1, yq, xq);
     return r;
 }
@@ -176,8 +174,8 @@ brick_file_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, cons
         if (rank[i] < 0) continue;
         const int at = start[i] + rank[i];
         place[(long)i * s.P] = at;
-        L.pt[at] = make_uint4((unsigned)((k0 + i) * s.M + b * s.P + p) * 128u, __float_as_uint(q[i].y), __float_as_uint(q[i].x),
-                              __float_as_uint(q[i].hz));
+        L.pt[at] = make_uint4((unsigned)((k0 + i) * s.M + b * s.P + p) * 128u | q[i].cell, __float_as_uint(q[i].hy),
+                              __float_as_uint(q[i].hx), __float_as_uint(q[i].hz));
         L.alpha[at] = (mask && s.mact) ? mask_act<AT>(s.mact, al[i]) : al[i];
     }
     // points outside the volume: their rows among all groups' rows, listed downwards from the end of the entries (which the
@@ -203,6 +201,27 @@ brick_file_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, cons
     }
 }
 
+// ---- the weights as matrix operands -----------------------------------------------------------------------------------
+// A corner weight is a float and stays one: it travels as three bfloat16 terms that add up to it exactly (its top 8
+// significant bits, the next 8, the last 8), each multiplied with the bfloat16 rows and summed in float32 -- what fmaf
+// of the float weight gives.  (Truncated, not rounded: no term is larger than the weight.)
+// The pair of a row of two corners along x, in the row of four voxels of a brick: 16-bit elements x .. x + 1 of 8 bytes
+// (`xs`: 16 x), zeros beside them.  The zeros are not products: a weight that is no number stays at its corners.
+struct WeightRow {
+    unsigned long long t[3];
+};
+D2C_DEV WeightRow weight_row(float w0, float w1, unsigned xs)
+{
+    WeightRow r;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const unsigned b0 = __float_as_uint(w0), b1 = __float_as_uint(w1);
+        r.t[i] = (unsigned long long)__builtin_amdgcn_perm(b1, b0, 0x07060302u) << xs;
+        w0 -= __uint_as_float(b0 & 0xffff0000u); w1 -= __uint_as_float(b1 & 0xffff0000u);
+    }
+    return r;
+}
+
 // ---- the products -------------------------------------------------------------------------------------------------
 // A workgroup takes a column of bricks (one 3 x 3 block of base voxels along y and x, a range of z) and up to four chunks
 // of 64 channels, a wavefront each; all walk the same points, 32 at a time.  Going up in z, the upper plane of a brick is the
@@ -211,7 +230,7 @@ brick_file_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, cons
 //
 // Matrix operands (v_mfma_f32_32x32x16_bf16):
 //   T:  A = x rows (lane = voxel), B = grad-column rows (lane = point), both from LDS
-//   gx: A = the weights, two bfloat16 terms, B = the rows, both through LDS (lane = point there, transposing reads)
+//   gx: A = the weights, three bfloat16 terms, B = the rows, both through LDS (lane = point there, transposing reads)
 // Voxel m of the brick: plane slot m / 16, y (m / 4) % 4, x m % 4.  A lane of T holds point lane % 32 and, in
 // register r, voxel 8 * (r / 4) + 4 * (lane / 32) + r % 4: x = r % 4, slot = r / 8, y = 2 * ((r / 4) % 2) + lane / 32, so
 // that of a point's two corner rows along y each half of the wavefront holds one.
@@ -230,7 +249,7 @@ struct BrickArgs {
 };
 
 constexpr int kMaxWaves = 4;
-constexpr int kWaveLds = 32 * 128 + 2 * 32 * 64;
+constexpr int kWaveLds = 32 * 128 + 3 * 32 * 64;
 D2C_DEV void lds_only_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 D2C_DEV void wave_fence() { asm volatile("" ::: "memory"); __builtin_amdgcn_wave_barrier(); }
 
@@ -313,9 +332,9 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
     // another row cost the L1 four times the lookups), as the operand of T, weights as they are made, and transposing
     // reads of both (within 16 lanes, lane l element j comes from lane 4j + l/4, element l%4)
     const int pv = lane >> 3, pc = lane & 7;
-    unsigned char *const g_st = s_g + pv * 128 + ((pc ^ g_swz(pv)) << 4), *const g_st1 = s_g + pv * 128 + ((pc ^ g_swz(pv) ^ 1) << 4);
+    const unsigned g_st = lds_address(s_g) + pv * 128 + ((pc ^ g_swz(pv)) << 4);
     const unsigned g_ld = lds_address(s_g) + n * 128 + ((h ^ g_swz(n)) << 4);
-    unsigned char *const w_st = s_w + n * 64 + (((h * 2) ^ ((n >> 2) & 3)) << 4), *const w_st1 = s_w + n * 64 + (((h * 2 + 1) ^ ((n >> 2) & 3)) << 4);
+    const unsigned w_st = lds_address(s_w) + n * 64 + (((h * 2) ^ ((n >> 2) & 3)) << 4);     // (^ 8 y: the lane's row y of voxels)
     const int tr_row = h * 8 + ((lane & 15) >> 2), tr_pc = ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1), tr_in = (lane & 1) * 8;
     const unsigned g_tr = lds_address(s_g) + tr_row * 128 + ((tr_pc ^ g_swz(tr_row)) << 4) + tr_in;
     const unsigned w_tr = lds_address(s_w) + tr_row * 64 + ((tr_pc ^ (h * 2)) << 4) + tr_in;
@@ -337,7 +356,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
     auto rows = [&](const uint4 &q, u32x4_t (&row)[4]) INLINE {
         for_each_const([&](auto I) INLINE {
             constexpr int i = decltype(I)::value;
-            row[i] = __builtin_amdgcn_raw_buffer_load_b128(rsg, __builtin_amdgcn_ds_bpermute((i * 8 + pv) << 2, (int)q.x) + pc * 16, 0, 0);
+            row[i] = __builtin_amdgcn_raw_buffer_load_b128(rsg, __builtin_amdgcn_ds_bpermute((i * 8 + pv) << 2, (int)(q.x & ~127u)) + pc * 16, 0, 0);
         }, std::make_integer_sequence<int, 4>{});
     };
     // what base plane zi - 1 needs: its points (the range `range` asked for) and the plane above it
@@ -372,33 +391,31 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
             // wanted first.  Past the last point: its row again.)
             entry(i0 + 96, e3, a3);
             __builtin_amdgcn_sched_barrier(0);
-            *reinterpret_cast<u32x4_t *>(g_st) = row[0];
-            *reinterpret_cast<u32x4_t *>(g_st1 + 1024) = row[1];
-            *reinterpret_cast<u32x4_t *>(g_st + 2048) = row[2];
-            *reinterpret_cast<u32x4_t *>(g_st1 + 3072) = row[3];
+            typedef __attribute__((address_space(3))) u32x4_t *lds128;
+            *(lds128)(size_t)g_st = row[0];
+            *(lds128)(size_t)((g_st ^ 16) + 1024) = row[1];
+            *(lds128)(size_t)(g_st + 2048) = row[2];
+            *(lds128)(size_t)((g_st ^ 16) + 3072) = row[3];
             rows(e2, row);
             __builtin_amdgcn_sched_barrier(0);
             const bool ok = i0 + n < cnt;
-            const float py = __uint_as_float(e0.y), px = __uint_as_float(e0.z), hz = __uint_as_float(e0.w), lz = 1.f - hz;
-            // ---- weights (lane = point, the 16 voxels of slot h)
+            const unsigned yb = e0.x & 3u, xs = (e0.x & 12u) << 2;
+            const float hy = __uint_as_float(e0.y), hx = __uint_as_float(e0.z), hz = __uint_as_float(e0.w), lz = 1.f - hz;
+            // ---- weights (lane = point, the 16 voxels of slot h): rows yb, yb + 1 of four voxels, zeros in the other two
             {
                 const float wz = (ok ? a0 : 0.f) * ((h != 0) == low ? lz : hz);
-                float tx[4];
+                const float wy0 = wz * (1.f - hy), wy1 = wz * hy, lx = 1.f - hx;
+                const WeightRow r0 = weight_row(wy0 * lx, wy0 * hx, xs), r1 = weight_row(wy1 * lx, wy1 * hx, xs);
+                typedef __attribute__((address_space(3))) unsigned long long *lds64;
+                const unsigned sy = yb << 3;
+                const unsigned at0 = w_st ^ sy, at1 = w_st ^ (sy + 8), at2 = w_st ^ ((sy + 16) & 24), at3 = w_st ^ ((sy + 24) & 24);
 #pragma unroll
-                for (int i = 0; i < 4; i++) tx[i] = __builtin_amdgcn_fmed3f(1.f - fabsf((float)i - px), 0.f, 1.f);
-                for_each_const([&](auto Y) INLINE {
-                    constexpr int y = decltype(Y)::value * 2;
-                    uint32_t wh[4], wl[4];
-#pragma unroll
-                    for (int j = 0; j < 8; j += 2) {
-                        const float ty = __builtin_amdgcn_fmed3f(1.f - fabsf((float)(y + j / 4) - py), 0.f, 1.f) * wz;
-                        const float w0 = ty * tx[j & 3], w1 = ty * tx[(j & 3) + 1];
-                        wh[j / 2] = pack_bf16x2(w0, w1);
-                        wl[j / 2] = pack_bf16x2(w0 - __uint_as_float(wh[j / 2] << 16), w1 - __uint_as_float(wh[j / 2] & 0xffff0000u));
-                    }
-                    *reinterpret_cast<uint4 *>(y ? w_st1 : w_st) = make_uint4(wh[0], wh[1], wh[2], wh[3]);
-                    *reinterpret_cast<uint4 *>((y ? w_st1 : w_st) + 2048) = make_uint4(wl[0], wl[1], wl[2], wl[3]);
-                }, std::make_integer_sequence<int, 2>{});
+                for (int i = 0; i < 3; i++) {
+                    *(lds64)(size_t)(at0 + i * 2048) = r0.t[i];
+                    *(lds64)(size_t)(at1 + i * 2048) = r1.t[i];
+                    *(lds64)(size_t)(at2 + i * 2048) = 0;
+                    *(lds64)(size_t)(at3 + i * 2048) = 0;
+                }
             }
             wave_fence();
             // ---- the two products
@@ -408,21 +425,22 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
             for_each_const([&](auto KG) INLINE {
                 constexpr int kg = decltype(KG)::value;            // 16 points, and half of T's channels
                 const bf16x8_t wh = operand(tr_read(w_tr + kg * 1024), tr_read((w_tr ^ 16) + kg * 1024 + 256));
-                const bf16x8_t wl = operand(tr_read(w_tr + kg * 1024 + 2048), tr_read((w_tr ^ 16) + kg * 1024 + 2304));
+                const bf16x8_t wm = operand(tr_read(w_tr + kg * 1024 + 2048), tr_read((w_tr ^ 16) + kg * 1024 + 2304));
+                const bf16x8_t wl = operand(tr_read(w_tr + kg * 1024 + 4096), tr_read((w_tr ^ 16) + kg * 1024 + 4352));
                 for_each_const([&](auto Q) INLINE {
                     constexpr int q = decltype(Q)::value, ks = kg * 2 + q;
                     const u32x4_t gq = *reinterpret_cast<const __attribute__((address_space(3))) u32x4_t *>((size_t)(g_ld ^ (ks * 32)));
                     T = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, xa[ks]), __builtin_bit_cast(bf16x8_t, gq), T, 0, 0, 0);
                     const bf16x8_t gb = operand(tr_read((g_tr ^ (q * 64)) + kg * 2048), tr_read((g_tr ^ (q * 64) ^ 32) + kg * 2048 + 512));
                     gacc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wh, gb, gacc[q], 0, 0, 0);
+                    gacc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wm, gb, gacc[q], 0, 0, 0);
                     gacc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wl, gb, gacc[q], 0, 0, 0);
                 }, std::make_integer_sequence<int, 2>{});
             }, std::make_integer_sequence<int, 2>{});
             wave_fence();
             // ---- grad_offset / grad_mask from the point's corner dots
             {
-                const bool y1 = py >= 1.f, y2 = py >= 2.f, x1 = px >= 1.f, x2 = px >= 2.f;
-                const float hy = py - (y2 ? 2.f : (y1 ? 1.f : 0.f)), hx = px - (x2 ? 2.f : (x1 ? 1.f : 0.f));
+                const bool y1 = yb >= 1, y2 = yb >= 2, x1 = xs >= 16, x2 = xs >= 32;
                 const bool q = h ? y2 : y1;                       // the corner row along y this half holds ...
                 const bool hi = (y1 != y2) != (h != 0);           // ... and whether it is the upper one
                 // (single registers from here on: a choice between two elements of T is not to become a variable index)
@@ -489,7 +507,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
 
 // ---- sampled columns ------------------------------------------------------------------------------------------------
 // col[chunk][tap][rows][64] = modulation * interpolated input of every point (rows: N*P and a few): x^T[64 channels, 32 voxels] * W[32 voxels, 32
-// points], two bfloat16 terms of the weights.  W is made by the lanes that hold the points, in the operand's own order
+// points], three bfloat16 terms of the weights.  W is made by the lanes that hold the points, in the operand's own order
 // (lane = point, half h of the wavefront: the voxels of rows y = 2h, 2h + 1 of each plane); the brick's input is kept as
 // the other operand, one plane changed per step in z.  Rows leave whole, through LDS.  Bound by the rows it writes:
 // 5.6 M points x 256 channels (32x60x108, 27 taps), 2.9 GB: 700 us (the whole forward pass: 2.3 ms gathering, 1.7 ms sorted).
@@ -610,32 +628,24 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 4) brick_sample_kernel(BrickSa
             // (the next entries: of this block, or the first of the next plane's)
             if (i0 + 32 < cnt) entry(lo, cnt, i0 + 32, e1, a1);
             else entry(nlo, ncnt, 0, e1, a1);
-            const float py = __uint_as_float(e0.y), px = __uint_as_float(e0.z), hz = __uint_as_float(e0.w);
-            const float wlo = a0 * (1.f - hz), whi = a0 * hz;
-            float tx[4], ty[2];
-#pragma unroll
-            for (int i = 0; i < 4; i++) tx[i] = __builtin_amdgcn_fmed3f(1.f - fabsf((float)i - px), 0.f, 1.f);
-            const float yb = py - (float)(2 * h);
-#pragma unroll
-            for (int i = 0; i < 2; i++) ty[i] = __builtin_amdgcn_fmed3f(1.f - fabsf((float)i - yb), 0.f, 1.f);
+            const unsigned xs = (e0.x & 12u) << 2;
+            const int dy = 2 * h - (int)(e0.x & 3u);                     // the half's first row of voxels, from the base voxel
+            const float hy = __uint_as_float(e0.y), hx = __uint_as_float(e0.z), hz = __uint_as_float(e0.w), lx = 1.f - hx;
             f32x16 r0, r1;
 #pragma unroll
             for (int r = 0; r < 16; r++) r0[r] = r1[r] = 0.f;
             for_each_const([&](auto S) INLINE {
                 constexpr int slot = decltype(S)::value;
-                uint32_t wh[4], wl[4];
+                const float wz = a0 * (slot ? hz : 1.f - hz), wy0 = wz * (1.f - hy), wy1 = wz * hy;
+                const float u0 = dy == 0 ? wy0 : (dy == 1 ? wy1 : 0.f), u1 = dy == -1 ? wy0 : (dy == 0 ? wy1 : 0.f);
+                const WeightRow w0 = weight_row(u0 * lx, u0 * hx, xs), w1 = weight_row(u1 * lx, u1 * hx, xs);
 #pragma unroll
-                for (int j = 0; j < 8; j += 2) {
-                    const float t2 = ty[j / 4] * (slot ? whi : wlo), w0 = t2 * tx[j & 3], w1 = t2 * tx[(j & 3) + 1];
-                    wh[j / 2] = pack_bf16x2(w0, w1);
-                    wl[j / 2] = pack_bf16x2(w0 - __uint_as_float(wh[j / 2] << 16), w1 - __uint_as_float(wh[j / 2] & 0xffff0000u));
+                for (int i = 0; i < 3; i++) {
+                    const bf16x8_t wt = __builtin_bit_cast(bf16x8_t, make_uint4((unsigned)w0.t[i], (unsigned)(w0.t[i] >> 32),
+                                                                                (unsigned)w1.t[i], (unsigned)(w1.t[i] >> 32)));
+                    r0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(slot ? xh[0] : xl[0], wt, r0, 0, 0, 0);
+                    r1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(slot ? xh[1] : xl[1], wt, r1, 0, 0, 0);
                 }
-                const bf16x8_t bh = __builtin_bit_cast(bf16x8_t, make_uint4(wh[0], wh[1], wh[2], wh[3]));
-                const bf16x8_t bl = __builtin_bit_cast(bf16x8_t, make_uint4(wl[0], wl[1], wl[2], wl[3]));
-                r0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(slot ? xh[0] : xl[0], bh, r0, 0, 0, 0);
-                r1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(slot ? xh[1] : xl[1], bh, r1, 0, 0, 0);
-                r0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(slot ? xh[0] : xl[0], bl, r0, 0, 0, 0);
-                r1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(slot ? xh[1] : xl[1], bl, r1, 0, 0, 0);
             }, std::make_integer_sequence<int, 2>{});
             for_each_const([&](auto P) INLINE {
                 constexpr int q = decltype(P)::value, c = q >> 1, r = (q & 1) * 8;      // channels 32 c + 16 h + r ..
@@ -645,7 +655,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 4) brick_sample_kernel(BrickSa
                                pack_bf16x2(v[r + 6], v[r + 7]));
             }, std::make_integer_sequence<int, 4>{});
             wave_fence();
-            const unsigned to = e0.x + (unsigned)(fdiv((int)(e0.x >> 7), a.dM) * a.pad) * 128u;      // (the entry counts N*P rows per tap)
+            const unsigned to = (e0.x & ~127u) + (unsigned)(fdiv((int)(e0.x >> 7), a.dM) * a.pad) * 128u;      // (the entry counts N*P rows per tap)
             for_each_const([&](auto I) INLINE {
                 constexpr int i = decltype(I)::value;
                 const int row = i * 8 + pv;

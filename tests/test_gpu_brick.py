@@ -79,3 +79,50 @@ def test_grad_columns_at_tile_edges(N, Cin, Cout, dims, dev):
     xd = x.to(dev).requires_grad_(True)
     d2c.deform_conv3d(xd, torch.zeros(N, 81, *dims, device=dev), None, w.to(dev), None, 1, 1, 1, 1, 1).backward(gout.to(dev))
     assert rel_l2(xd.grad, xr.grad) < 1e-2
+
+
+def _one_tap(Cin, Cout, ks, dev):
+    """Weights that hand channel 0 of the middle tap to output channel 0."""
+    w = torch.zeros(Cout, Cin, *ks)
+    w[0, 0, ks[0] // 2, ks[1] // 2, ks[2] // 2] = 1
+    return w.bfloat16().to(dev)
+
+
+def test_a_sample_is_interpolated_with_float32_weights(dev):
+    """Neighbours r0 and -r1 sampled where they cancel but for 2^-17 (r0 + r1): float32 weights leave an error of about 2^-25,
+    0.3 % of the value, and its rounding to bfloat16 0.2 %; weights of 16 or 17 bits leave 5 % and more."""
+    N, C, O, dims, ks = 1, 256, 64, (9, 105, 14), (1, 3, 3)
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(N, C, *dims, generator=g).bfloat16()
+    r = (1 + torch.rand(dims, generator=g)).bfloat16()
+    pos = torch.arange(dims[2])
+    x[0, 0] = r * (1 - 2 * (pos % 2))
+    r0, r1 = r[..., :-1].double(), r[..., 1:].double()
+    frac = torch.zeros(dims)
+    frac[..., :-1] = (r0 / (r0 + r1) + 2.0 ** -17).float()
+    frac = (frac + pos) - pos                         # (what float32 keeps of it at this position)
+    off = torch.zeros(N, 27, *dims)
+    off[0, 3 * 4 + 2] = frac
+    out = d2c.deform_conv3d(x.to(dev), off.to(dev), None, _one_tap(C, O, ks, dev), None, 1, (0, 1, 1), 1, 1, 1)
+    f = frac[..., :-1].double()
+    want = ((1 - f) * r0 - f * r1) * (1 - 2 * (pos[:-1] % 2))
+    assert rel_l2(out[0, 0, ..., :-1], want) < 1e-2
+
+
+def test_grad_input_adds_float32_weights(dev):
+    """Two points of opposite grad_out in the same cell, their fractions f and f + 2^-19: the differences +-2^-19 remain, exact
+    in bfloat16."""
+    N, C, O, dims, ks = 1, 64, 64, (4, 30, 14), (1, 3, 3)
+    g = torch.Generator().manual_seed(4)
+    x = torch.randn(N, C, *dims, generator=g).bfloat16().to(dev).requires_grad_(True)
+    f = (torch.randint(2 ** 16, 2 ** 19, (*dims[:2], dims[2] // 2), generator=g) | 1).float() * 2.0 ** -20       # (a 20-bit fraction)
+    off = torch.zeros(N, 27, *dims)
+    off[0, 3 * 4 + 2, ..., 0::2] = f
+    off[0, 3 * 4 + 2, ..., 1::2] = f + 2.0 ** -19 - 1
+    gout = torch.zeros(N, O, *dims)
+    gout[:, 0, ..., 0::2], gout[:, 0, ..., 1::2] = 1, -1
+    out = d2c.deform_conv3d(x, off.to(dev), None, _one_tap(C, O, ks, dev), None, 1, (0, 1, 1), 1, 1, 1)
+    out.backward(gout.bfloat16().to(dev))
+    want = torch.full(dims, 2.0 ** -19)
+    want[..., 1::2] *= -1
+    assert torch.equal(x.grad[0, 0].float().cpu(), want)
