@@ -126,3 +126,51 @@ def test_grad_input_adds_float32_weights(dev):
     want = torch.full(dims, 2.0 ** -19)
     want[..., 1::2] *= -1
     assert torch.equal(x.grad[0, 0].float().cpu(), want)
+
+
+# infinities and NaN reach what touches them and nothing else: as in the oracle, whatever shares a brick, a product of 32 points
+# or a set of chunks with them.  (The same masks; values where they are finite.)
+@pytest.mark.parametrize("what", ["input", "mask", "grad_out"])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("Cin,Cout,dims,G", [(128, 40, (13, 31, 31), 2), (320, 33, (3, 9, 11), 1)])
+def test_infinities_and_nan_stay_where_they_are(Cin, Cout, dims, G, bad, what, dev):
+    g = torch.Generator().manual_seed(11)
+    x = torch.randn(1, Cin, *dims, generator=g).bfloat16()
+    w = (torch.randn(Cout, Cin, 3, 3, 3, generator=g) / (Cin * 27) ** 0.5).bfloat16()
+    off = torch.randn(1, G * 81, *dims, generator=g)
+    m = torch.sigmoid(torch.randn(1, G * 27, *dims, generator=g))
+    gout = torch.randn(1, Cout, *dims, generator=g).bfloat16()
+    mid = tuple(d // 2 for d in dims)
+    if what == "input":
+        x[0, 3][0, 0, 0] = x[0, 70][mid] = x[0, Cin - 1][tuple(d - 1 for d in dims)] = bad
+    elif what == "mask":
+        m[0, 13][mid] = m[0, 13][1, 1, 1] = bad
+    else:
+        gout[0, 5][mid] = gout[0, 0][1, 1, 1] = bad
+    for at in (mid, (1, 1, 1)):                       # (points outside the volume, where the oracle forms 0 * inf, are not meant)
+        off[(0, slice(None)) + at] *= 0.1
+    exp = cpu.conv3d_forward(x.float(), off, m, w.float(), None, 1, 1, 1, 1, G)
+    eg = cpu.conv3d_backward(gout.float(), x.float(), off, m, w.float(), False, 1, 1, 1, 1, G)
+    ts = [t.to(dev).requires_grad_(True) for t in (x, off, m, w)]
+    out = d2c.deform_conv3d(*ts[:3], ts[3], None, 1, 1, 1, 1, G)
+    out.backward(gout.to(dev))
+    for name, t, e in zip(("out", "grad_input", "grad_offset", "grad_mask", "grad_weight"), [out] + [t.grad for t in ts], (exp,) + eg[:4]):
+        t = t.detach().float().cpu()
+        assert torch.equal(t.isfinite(), e.isfinite()), (name, int((~t.isfinite()).sum()), int((~e.isfinite()).sum()))
+        ok = e.isfinite()
+        if ok.any():
+            assert rel_l2(t[ok], e[ok]) < 2e-2, name
+
+
+def test_a_bad_voxel_stays_where_it_is_in_inference(dev):
+    g = torch.Generator().manual_seed(12)
+    dims = (1, 95, 131)
+    x = torch.randn(1, 256, *dims, generator=g).bfloat16()
+    w = (torch.randn(16, 256, 3, 3, 3, generator=g) / (256 * 27) ** 0.5).bfloat16()
+    off = torch.randn(1, 81, *dims, generator=g)
+    x[0, 200, 0, 50, 60] = float("nan")
+    x[0, 0, 0, 94, 130] = float("inf")
+    exp = cpu.conv3d_forward(x.float(), off, None, w.float(), None, 1, 1, 1, 1, 1)
+    out = d2c.deform_conv3d(x.to(dev), off.to(dev), None, w.to(dev), None, 1, 1, 1, 1, 1).float().cpu()
+    assert torch.equal(out.isfinite(), exp.isfinite())
+    assert rel_l2(out[exp.isfinite()], exp[exp.isfinite()]) < 1e-2
