@@ -18,6 +18,7 @@ ALGO_NAMES = {ALGO_GENERIC: "generic", ALGO_MFMA: "mfma", ALGO_DEPTHWISE: "depth
 EXPORTS = (
     "d2c_output_size", "d2c_conv3d_check", "d2c_conv3d_algo", "d2c_conv3d_packed_supported",
     "d2c_conv3d_forward_workspace_bytes", "d2c_conv3d_backward_workspace_bytes",
+    "d2c_conv3d_forward_least_workspace_bytes",
     "d2c_conv3d_forward", "d2c_conv3d_backward", "d2c_conv3d_forward_static", "d2c_static_workspace_bytes",
     "d2c_conv3d_prepared_bytes", "d2c_conv3d_forward_prepared", "d2c_conv3d_backward_prepared",
     "d2c_conv3d_columns_bytes", "d2c_conv3d_keep_bytes", "d2c_conv3d_forward_columns", "d2c_conv3d_backward_columns_workspace_bytes",
@@ -137,8 +138,9 @@ def load():
     # (the second argument: a pointer to a size-map description, or None)
     lib.d2c_conv3d_columns_bytes.argtypes, lib.d2c_conv3d_columns_bytes.restype = [p3, vp], sz
     lib.d2c_conv3d_keep_bytes.argtypes, lib.d2c_conv3d_keep_bytes.restype = [p3, vp], sz
-    lib.d2c_conv3d_backward_columns_workspace_bytes.argtypes = [p3, vp]
-    lib.d2c_conv3d_backward_columns_workspace_bytes.restype = sz
+    for name in ("forward_least", "backward_columns"):
+        f = getattr(lib, f"d2c_conv3d_{name}_workspace_bytes")
+        f.argtypes, f.restype = [p3, vp], sz
     lib.d2c_conv3d_forward_columns.argtypes = [p3, vp] + [vp] * 6 + [vp, sz, vp, sz, vp]
     lib.d2c_conv3d_forward_columns.restype = ctypes.c_int
     lib.d2c_conv3d_backward_columns.argtypes = [p3, vp] + [vp] * 5 + [vp, sz] + [vp] * 5 + [vp, sz, vp]

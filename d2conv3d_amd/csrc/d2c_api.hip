@@ -398,8 +398,8 @@ int d2c_conv3d_forward(const d2c_conv3d_desc *q, const void *x, const void *offs
     if (a < 0) return D2C_ERR_UNSUPPORTED;
     hipStream_t st = (hipStream_t)stream;
     if (a == D2C_ALGO_GENERIC) return d2c_generic_conv3d_forward(*q, x, offset, mask, weight, bias, out, st);
-    if (int rc = check_ws(d2c_tiled_forward_ws(*q), ws, ws_bytes)) return rc;
-    return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, st);
+    if (int rc = check_ws(d2c_tiled_forward_ws(*q, D2C_FWD_WS_LEAST), ws, ws_bytes)) return rc;
+    return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, ws_bytes, st);
 }
 
 size_t d2c_conv3d_prepared_bytes(const d2c_conv3d_desc *q)
@@ -439,8 +439,8 @@ int d2c_conv3d_forward_prepared(const d2c_conv3d_desc *q, const void *x, const v
     if (a == D2C_ALGO_GENERIC) return d2c_generic_conv3d_forward(*q, x, offset, mask, weight, bias, out, st);
     D2cPrepared prep;
     if (int rc = check_prepared(*q, prepared, prepared_bytes, reuse, &prep)) return rc;
-    if (int rc = check_ws(d2c_tiled_forward_ws(*q), ws, ws_bytes)) return rc;
-    return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, st, nullptr, nullptr, prep.base ? &prep : nullptr);
+    if (int rc = check_ws(d2c_tiled_forward_ws(*q, D2C_FWD_WS_LEAST), ws, ws_bytes)) return rc;
+    return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, ws_bytes, st, nullptr, nullptr, prep.base ? &prep : nullptr);
 }
 
 int d2c_conv3d_backward_prepared(const d2c_conv3d_desc *q, const void *gout, const void *x, const void *offset,
@@ -516,7 +516,7 @@ int d2c_conv3d_forward_static(const d2c_conv3d_desc *q, const void *x, const voi
     if (a < 0) return D2C_ERR_UNSUPPORTED;
     hipStream_t st = (hipStream_t)stream;
     if (a == D2C_ALGO_GENERIC) return d2c_generic_conv3d_forward(*q, x, offset, mask, weight, bias, out, st);
-    const size_t need = d2c_tiled_forward_ws(*q);
+    const size_t need = d2c_tiled_forward_ws(*q, D2C_FWD_WS_LEAST);
     if (need > (size_t)D2C_STATIC_WORKSPACE_BYTES) {
         d2c_set_error("d2c_conv3d_forward_static: this description needs %zu bytes of workspace, the static one holds "
                       "%zu; use d2c_conv3d_forward with a caller-provided workspace",
@@ -525,7 +525,7 @@ int d2c_conv3d_forward_static(const d2c_conv3d_desc *q, const void *x, const voi
     }
     void *ws = nullptr;
     if (int rc = static_scratch(&ws)) return rc;
-    return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, st);
+    return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, (size_t)D2C_STATIC_WORKSPACE_BYTES, st);
 }
 
 int d2c_conv3d_backward(const d2c_conv3d_desc *q, const void *gout, const void *x, const void *offset,
@@ -592,6 +592,14 @@ size_t d2c_conv3d_sized_forward_workspace_bytes(const d2c_conv3d_desc *q, const 
     return expanded_offsets_bytes(*q) + d2c_conv3d_forward_workspace_bytes(q);
 }
 
+size_t d2c_conv3d_forward_least_workspace_bytes(const d2c_conv3d_desc *q, const d2c_size_map_desc *z)
+{
+    if ((z ? sized_check(q, z) : d2c_conv3d_check(q)) != D2C_OK) return 0;
+    const int a = choose_algo(*q, true);
+    const size_t least = a == D2C_ALGO_MFMA || a == D2C_ALGO_DEPTHWISE ? d2c_tiled_forward_ws(*q, D2C_FWD_WS_LEAST) : 0;
+    return z && !sized_fused(*q, false) ? expanded_offsets_bytes(*q) + least : least;
+}
+
 size_t d2c_conv3d_sized_backward_workspace_bytes(const d2c_conv3d_desc *q, const d2c_size_map_desc *z)
 {
     if (sized_check(q, z) != D2C_OK) return 0;
@@ -606,9 +614,9 @@ int d2c_conv3d_sized_forward(const d2c_conv3d_desc *q, const d2c_size_map_desc *
     if (int rc = sized_check(q, z)) return rc;
     if (!x || !size_raw || !weight || !out) { d2c_set_error("null tensor pointer"); return D2C_ERR_SHAPE; }
     if (choose_algo(*q, false) < 0) return D2C_ERR_UNSUPPORTED;
-    if (int rc = check_ws(d2c_conv3d_sized_forward_workspace_bytes(q, z), ws, ws_bytes)) return rc;
+    if (int rc = check_ws(d2c_conv3d_forward_least_workspace_bytes(q, z), ws, ws_bytes)) return rc;
     if (sized_fused(*q, false))
-        return d2c_tiled_forward(*q, x, size_raw, mask, weight, bias, out, ws, (hipStream_t)stream, z);
+        return d2c_tiled_forward(*q, x, size_raw, mask, weight, bias, out, ws, ws_bytes, (hipStream_t)stream, z);
     const size_t ob = expanded_offsets_bytes(*q);
     if (int rc = d2c_size_map_offsets_forward(z, size_raw, ws, stream)) return rc;
     return d2c_conv3d_forward(q, x, ws, mask, weight, bias, out, (char *)ws + ob, ws_bytes - ob, stream);
@@ -643,7 +651,7 @@ static bool stats_fused(const d2c_conv3d_desc &q, const d2c_size_map_desc *z)
 size_t d2c_conv3d_forward_stats_workspace_bytes(const d2c_conv3d_desc *q, const d2c_size_map_desc *z)
 {
     if ((z ? sized_check(q, z) : d2c_conv3d_check(q)) != D2C_OK) return 0;
-    if (stats_fused(*q, z)) return d2c_tiled_forward_ws(*q, true);
+    if (stats_fused(*q, z)) return d2c_tiled_forward_ws(*q, D2C_FWD_WS_STATS);
     return z ? d2c_conv3d_sized_forward_workspace_bytes(q, z) : d2c_conv3d_forward_workspace_bytes(q);
 }
 
@@ -658,8 +666,8 @@ int d2c_conv3d_forward_stats(const d2c_conv3d_desc *q, const d2c_size_map_desc *
     if (a < 0) return D2C_ERR_UNSUPPORTED;
     // the kernels that add the sums up on their way: matrix-core family, offsets from a tensor or formed in the sampler
     if (stats_fused(*q, z)) {
-        if (int rc = check_ws(d2c_tiled_forward_ws(*q, true), ws, ws_bytes)) return rc;
-        return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, (hipStream_t)stream, z, chan_stats);
+        if (int rc = check_ws(d2c_tiled_forward_ws(*q, D2C_FWD_WS_STATS), ws, ws_bytes)) return rc;
+        return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, ws_bytes, (hipStream_t)stream, z, chan_stats);
     }
     if (int rc = z ? d2c_conv3d_sized_forward(q, z, x, offset, mask, weight, bias, out, ws, ws_bytes, stream)
                    : d2c_conv3d_forward(q, x, offset, mask, weight, bias, out, ws, ws_bytes, stream))
@@ -709,7 +717,7 @@ int d2c_conv3d_forward_columns(const d2c_conv3d_desc *q, const d2c_size_map_desc
     if (!x || !offset || !weight || !out) { d2c_set_error("null tensor pointer"); return D2C_ERR_SHAPE; }
     if (int rc = check_columns(*q, z, columns, columns_bytes)) return rc;
     if (int rc = check_ws(d2c_tiled_forward_ws(*q), ws, ws_bytes)) return rc;
-    return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, (hipStream_t)stream, z, nullptr, nullptr, columns,
+    return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, ws_bytes, (hipStream_t)stream, z, nullptr, nullptr, columns,
                              columns_bytes);
 }
 

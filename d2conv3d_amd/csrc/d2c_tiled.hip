@@ -379,8 +379,10 @@ __global__ void __launch_bounds__(256) size_minus_one_kernel(TiledShape s, const
 }
 
 struct FwdWs {
-    size_t xcl, wp, outacc, total;
-    size_t lists, col, gemm;        // forward over sampled columns: sorted points, columns, operands of the product
+    size_t xcl, wp, outacc;
+    size_t least;                   // what the gathering kernels need
+    size_t gemm, lists, col, end;   // forward over sampled columns: operands of the product, sorted points, columns
+    size_t total;                   // what the call is fastest with
 };
 bool use_brick_forward(const d2c_conv3d_desc &q, const TiledShape &s, bool kept);
 // columns; and what a forward call can leave for its backward call: the sorted points behind them
@@ -397,21 +399,21 @@ FwdWs fwd_ws(const d2c_conv3d_desc &q, const TiledShape &s)
     FwdWs w{};
     w.xcl = 0;
     w.wp = d2c_align_up((size_t)s.N * s.vol * s.Cin * es + 256);   // input, then a 256-byte row of zeros
-    if (use_brick_forward(q, s, true)) {
-        w.gemm = w.wp;
-        w.lists = w.gemm + d2c_align_up(d2c_col_forward_ws(q));
-        w.col = w.lists + d2c_brick_ws(s).total;
-        w.total = w.col + (use_brick_forward(q, s, false) ? brick_col_bytes(s) : 0);
-        // (a call with a prepared region runs on the gather kernels, whose workspace this covers)
-    }
-    const size_t brick_total = w.total;
     w.outacc = w.wp + d2c_align_up((size_t)s.groups * s.nchunk * s.K * s.ogp * bkc_of(q.dtype) * es);
     // fp32 partial sums of the output, used only when the forward kernel splits its steps (as whole tiles of
     // 64 positions x padded output channels in the DMA-gather kernel)
-    w.total = w.outacc;
+    w.least = w.outacc;
     if (d2c_fwd_split(s) > 1)
-        w.total += d2c_align_up((size_t)((s.M + 63) / 64 * 64) * s.ogp * s.groups * sizeof(float));
-    if (w.total < brick_total) w.total = brick_total;
+        w.least += d2c_align_up((size_t)((s.M + 63) / 64 * 64) * s.ogp * s.groups * sizeof(float));
+    w.total = w.least;
+    if (use_brick_forward(q, s, true)) {
+        // (a call that keeps its columns holds them, and the sorted points, in the caller's buffer)
+        w.gemm = w.wp;
+        w.lists = w.gemm + d2c_align_up(d2c_col_forward_ws(q));
+        w.col = w.lists + d2c_brick_ws(s).total;
+        w.end = w.col + brick_col_bytes(s);
+        w.total = std::max(w.total, use_brick_forward(q, s, false) ? w.end : w.col);
+    }
     return w;
 }
 
@@ -510,7 +512,8 @@ DwWs dw_ws(const d2c_conv3d_desc &q, const TiledShape &s)
 template <typename T>
 int forward_t(const d2c_conv3d_desc &q, const void *x, const void *off, const void *mask, const void *w,
               const void *bias, void *out, void *ws, hipStream_t st, int nd = 3, const d2c_size_map_desc *sz = nullptr,
-              float *stats = nullptr, const D2cPrepared *prep = nullptr, void *columns = nullptr, size_t columns_bytes = 0)
+              float *stats = nullptr, const D2cPrepared *prep = nullptr, void *columns = nullptr, size_t columns_bytes = 0,
+              size_t ws_bytes = 0)
 {
     const TiledShape s = tiled_shape(q, nd, 0, sz);
     char *base = (char *)ws;
@@ -529,12 +532,17 @@ int forward_t(const d2c_conv3d_desc &q, const void *x, const void *off, const vo
         if (int rc = pack_input<T>(s, x, xcl_p, st, true)) return rc;   // with the row of zeros behind it
     if (nd == 3 && !prep && !stats && use_brick_forward(q, s, columns != nullptr)) {
         // sort the points, sample the columns (the caller's buffer, with the sorted points behind them for its backward
-        // call, or the workspace), multiply
+        // call, or the workspace), multiply.  A smaller workspace: the gathering kernels, below.
+        const bool keep = columns && columns_bytes >= brick_keep_bytes(s);
+        const bool fits = ws_bytes >= (keep ? l.lists : (columns ? l.col : l.end));
         char *col = columns ? (char *)columns : base + l.col;
-        char *lists = columns && columns_bytes >= brick_keep_bytes(s) ? col + brick_col_bytes(s) : base + l.lists;
-        if (int rc = d2c_brick_sort(s, off, mask, lists, st)) return rc;
-        if (int rc = d2c_brick_columns(s, xcl_p, col, (int)d2c_columns_rows(s), lists, st)) return rc;
-        return d2c_col_forward(q, col, (int)d2c_columns_rows(s), w, bias, out, base + l.gemm, st);
+        char *lists = keep ? col + brick_col_bytes(s) : base + l.lists;
+        if (fits || keep)
+            if (int rc = d2c_brick_sort(s, off, mask, lists, st)) return rc;
+        if (fits) {
+            if (int rc = d2c_brick_columns(s, xcl_p, col, (int)d2c_columns_rows(s), lists, st)) return rc;
+            return d2c_col_forward(q, col, (int)d2c_columns_rows(s), w, bias, out, base + l.gemm, st);
+        }
     }
     const long total = (long)s.groups * s.nchunk * s.K * (s.ogp / 32) * 4 * 64;
     long g = (total + 255) / 256;
@@ -553,7 +561,7 @@ int forward_t(const d2c_conv3d_desc &q, const void *x, const void *off, const vo
     if (int rc = d2c_check_launch("pack_weight_fwd_kernel")) return rc;
     // (the per-tile sums of the output statistics go behind everything else in the workspace)
     return d2c_tiled_fwd_launch<T>(s, xcl_p, off, mask, wp_p, bias, out, (float *)(base + l.outacc), st,
-                                   stats, stats ? (float *)(base + l.total) : nullptr, columns);
+                                   stats, stats ? (float *)(base + l.least) : nullptr, columns);
 }
 
 // grad_input by sample lists (see d2c_invlist.hip): from whole grad-column rows, i.e. the reduction over all output
@@ -641,7 +649,7 @@ BwdSlices bwd_slices(const d2c_conv3d_desc &q, const TiledShape &s)
 }
 
 struct BwdWs {
-    size_t xcl, wt, gxcl, gwacc, goutp, auxacc, gcol, counts, entries, ovf, gsacc, sm1, brick, gemm, col, total;
+    size_t xcl, wt, gxcl, gwacc, goutp, auxacc, gcol, counts, entries, ovf, gsacc, sm1, brick, res, gemm, col, total;
 };
 // `saved_columns`: the caller brings the sampled columns of the forward call (no column region, no slices)
 BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns = false)
@@ -683,8 +691,10 @@ BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns =
     if (s.ss.on) w.total += d2c_align_up((size_t)s.N * 3 * s.P * sizeof(float));
     w.sm1 = w.total;       // ... and (size - 1) per axis
     if (s.ss.on) w.total += d2c_align_up((size_t)s.N * 3 * s.P * sizeof(float));
-    w.brick = w.total;
-    if (use_brick(q, s)) w.total += d2c_brick_ws(s).total + d2c_brick_ws(s).res_bytes;
+    w.brick = w.total;     // sorted points
+    if (use_brick(q, s)) w.total += d2c_brick_ws(s).total;
+    w.res = w.total;       // ... and sums per point
+    if (use_brick(q, s)) w.total += d2c_brick_ws(s).res_bytes;
     w.gemm = w.total;      // operands of the grad-column product
     if (use_brick(q, s) && d2c_grad_col_supported(q)) w.total += d2c_grad_col_ws(q);
     w.col = w.total;       // sampled columns for the grad-weight product
@@ -733,6 +743,9 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
         }
         return D2C_OK;
     }
+    // (kept columns of a forward call over sorted points: those follow the columns)
+    const bool sorted = columns && use_brick_forward(q, s, true) && columns_bytes >= brick_keep_bytes(s);
+    const bool brick = use_brick(q, s) && !(gw && gw_mode(q) == 2);      // (not: columns in the rows' place)
     const BwdWs l = bwd_ws(q, s, columns != nullptr);
     const PreparedLayout pl = prepared_layout(q, s);
     char *xcl_p = prep ? (char *)prep->base + pl.xcl : base + l.xcl;
@@ -826,7 +839,6 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
             // size-map source: `goff` is the gradient of the raw size map; the offset / mask gradient kernel adds
             // into fp32 sums per axis, which a finishing kernel folds into it
             gw_from_col = gw && (columns ? d2c_bwd_weight_from_kept_col(s, q.dtype) : (auxk && use_col_weight(q, s)));
-            const bool brick = use_brick(q, s) && !(gw && gw_mode(q) == 2);      // (not: columns in the rows' place)
             void *goff_k = goff;
             if (s.ss.on && goff && !brick) {
                 goff_k = base + l.gsacc;
@@ -837,8 +849,6 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
             // offset / mask gradient kernel runs, so the samples are filed by a pass of their own)
             gw_in_place = gw_from_col && !columns && col_in_place(q, s);
             SampleLists L{nullptr, nullptr, nullptr, 0, 0, 0};
-            // (kept columns of a forward call over sorted points: those follow the columns)
-            const bool sorted = columns && use_brick_forward(q, s, true) && columns_bytes >= brick_keep_bytes(s);
             char *const lists_p = sorted ? (char *)const_cast<void *>(columns) + brick_col_bytes(s) : base + l.brick;
             if (brick) {
                 if (!sorted)
@@ -866,7 +876,7 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
                     if (int rc = d2c_brick_columns(s, xcl_p, base + l.col, (int)d2c_columns_rows(s), lists_p, st)) return rc;
                 }
                 if (int rc = d2c_brick_grad(s, xcl_p, base + l.gcol, mask, size_raw, gxcl, goff, gmask, lists_p,
-                                            base + l.brick + d2c_brick_ws(s).total, st)) return rc;
+                                            base + l.res, st)) return rc;
             } else if (auxk)
                 if (int rc = d2c_aux_grad_launch<T>(s, xcl_p, off, mask, base + l.gcol, goff_k, gmask,
                                                     (lists && !gw_in_place) ? &L : nullptr,
@@ -998,11 +1008,16 @@ bool d2c_tiled_axes_supported(const d2c_conv3d_desc &q)
     return d2c_tiled_bwd_data_supported(s, q.dtype) && d2c_tiled_bwd_weight_supported(s, q.dtype);
 }
 
-size_t d2c_tiled_forward_ws(const d2c_conv3d_desc &q, bool with_stats)
+size_t d2c_tiled_forward_ws(const d2c_conv3d_desc &q, D2cForwardWs which)
 {
     const TiledShape s = tiled_shape(q);
     if (is_depthwise(q)) return dw_ws(q, s).total_fwd;
-    return fwd_ws(q, s).total + (with_stats && d2c_fwd_fills_stats(s) ? d2c_fwd_stats_ws(s) : 0);
+    const FwdWs l = fwd_ws(q, s);
+    switch (which) {
+    case D2C_FWD_WS_LEAST: return l.least;
+    case D2C_FWD_WS_STATS: return l.least + (d2c_fwd_fills_stats(s) ? d2c_fwd_stats_ws(s) : 0);
+    default: return l.total;
+    }
 }
 
 size_t d2c_tiled_backward_ws(const d2c_conv3d_desc &q, const d2c_size_map_desc *sz, bool saved_columns)
@@ -1044,11 +1059,11 @@ bool d2c_tiled_sized_supported(const d2c_conv3d_desc &q, bool backward)
 }
 
 int d2c_tiled_forward(const d2c_conv3d_desc &q, const void *x, const void *off, const void *mask, const void *w,
-                      const void *bias, void *out, void *ws, hipStream_t st, const d2c_size_map_desc *sz, float *stats,
+                      const void *bias, void *out, void *ws, size_t ws_bytes, hipStream_t st, const d2c_size_map_desc *sz, float *stats,
                       const D2cPrepared *prep, void *columns, size_t columns_bytes)
 {
-    if (q.dtype == D2C_BF16) return forward_t<bf16_t>(q, x, off, mask, w, bias, out, ws, st, 3, sz, stats, prep, columns, columns_bytes);
-    return forward_t<float>(q, x, off, mask, w, bias, out, ws, st, 3, sz, stats, prep, columns, columns_bytes);
+    if (q.dtype == D2C_BF16) return forward_t<bf16_t>(q, x, off, mask, w, bias, out, ws, st, 3, sz, stats, prep, columns, columns_bytes, ws_bytes);
+    return forward_t<float>(q, x, off, mask, w, bias, out, ws, st, 3, sz, stats, prep, columns, columns_bytes, ws_bytes);
 }
 
 // Bytes of the caller-held prepared region of a description (0: the kernel family keeps nothing worth holding)

@@ -10,7 +10,10 @@ int d2c_tiled_algo(const d2c_conv3d_desc &q);  // D2C_ALGO_MFMA or D2C_ALGO_DEPT
 bool d2c_tiled_packed_supported(const d2c_conv3d_desc &q);
 // whether a description with some offset axes fixed (offset_axes != 7) stays on the tiled kernels in both directions
 bool d2c_tiled_axes_supported(const d2c_conv3d_desc &q);
-size_t d2c_tiled_forward_ws(const d2c_conv3d_desc &q, bool with_stats = false);
+// Workspace of a forward call: what it is fastest with; the least it runs with (gathering kernels); the least with output
+// statistics
+enum D2cForwardWs { D2C_FWD_WS_FAST, D2C_FWD_WS_LEAST, D2C_FWD_WS_STATS };
+size_t d2c_tiled_forward_ws(const d2c_conv3d_desc &q, D2cForwardWs which = D2C_FWD_WS_FAST);
 // `sz` != nullptr: the offsets are formed from a raw size map (`off` is that map [N, channels(mode), P], `goff` the
 // gradient with respect to it); only where d2c_tiled_sized_supported() says so.
 // `saved_columns`: for a backward call that is handed the sampled columns of its forward call (d2c_tiled_columns_bytes)
@@ -29,7 +32,7 @@ struct D2cPrepared {
 };
 size_t d2c_tiled_prepared_bytes(const d2c_conv3d_desc &q);
 int d2c_tiled_forward(const d2c_conv3d_desc &q, const void *x, const void *off, const void *mask, const void *w,
-                      const void *bias, void *out, void *ws, hipStream_t st, const d2c_size_map_desc *sz = nullptr,
+                      const void *bias, void *out, void *ws, size_t ws_bytes, hipStream_t st, const d2c_size_map_desc *sz = nullptr,
                       float *stats = nullptr, const D2cPrepared *prep = nullptr, void *columns = nullptr,
                       size_t columns_bytes = 0);
 int d2c_tiled_backward(const d2c_conv3d_desc &q, const void *gout, const void *x, const void *off,

@@ -188,3 +188,28 @@ def test_float32_backward_on_split_operands(name, dev):
         _ops.set_grad_weight_mode("columns")
         _ops.config.set_keep_columns(before["on"], before["max_bytes"])
     assert errs[True][-2 if b is not None else -1] > errs[False][-2 if b is not None else -1]   # (grad_weight: the flag did change the arithmetic)
+
+
+# bfloat16 problems whose forward pass samples columns first: at least 12288 positions, 256 channels to an offset group where
+# no backward pass keeps them
+def _large(dev, N=1, C=256, dims=(8, 30, 54), G=1):
+    g = torch.Generator(device=dev).manual_seed(31)
+    rn = lambda *s: torch.randn(*s, generator=g, device=dev)
+    x, w = rn(N, C, *dims).bfloat16(), (rn(C, C, 3, 3, 3) / (C * 27) ** 0.5).bfloat16()
+    desc = _lib.Conv3dDesc(N, C, C, *dims, 3, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, G, *dims, _lib.D2C_BF16, _lib.D2C_F32, 0, 1.0, 7, 0)
+    return (x, rn(N, G * 81, *dims), torch.sigmoid(rn(N, G * 27, *dims)), w, None), desc
+
+
+def test_the_static_workspace_serves_large_problems_without_columns(dev):
+    """The columns of this problem take 179 MB; the call runs on the kernels that need none, as it did before there were
+    columns in the workspace."""
+    ts, desc = _large(dev)
+    lib = _lib.load()
+    assert lib.d2c_conv3d_forward_least_workspace_bytes(ctypes.byref(desc), None) <= lib.d2c_static_workspace_bytes()
+    want = d2c.deform_conv3d(*ts, 1, 1, 1, 1, 1)
+    out = torch.empty_like(want)
+    p = lambda t: ctypes.c_void_p(t.data_ptr() if t is not None else 0)
+    rc = lib.d2c_conv3d_forward_static(ctypes.byref(desc), *(p(t) for t in ts), p(out),
+                                       ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    _lib.check(rc, "forward_static")
+    assert rel_l2(out, want) < 4e-3
