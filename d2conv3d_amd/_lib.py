@@ -22,7 +22,7 @@ EXPORTS = (
     "d2c_conv3d_forward", "d2c_conv3d_backward", "d2c_conv3d_forward_static", "d2c_static_workspace_bytes",
     "d2c_conv3d_prepared_bytes", "d2c_conv3d_forward_prepared", "d2c_conv3d_backward_prepared",
     "d2c_conv3d_columns_bytes", "d2c_conv3d_keep_bytes", "d2c_conv3d_forward_columns", "d2c_conv3d_backward_columns_workspace_bytes",
-    "d2c_conv3d_backward_columns",
+    "d2c_conv3d_backward_columns", "d2c_conv3d_forward_keep_workspace_bytes", "d2c_conv3d_backward_keep_workspace_bytes",
     "d2c_plain_conv3d_input_bytes", "d2c_plain_conv3d_forward_workspace_bytes",
     "d2c_plain_conv3d_backward_workspace_bytes", "d2c_plain_conv3d_forward", "d2c_plain_conv3d_backward",
     "d2c_conv1d_check", "d2c_conv1d_algo", "d2c_conv1d_forward_workspace_bytes", "d2c_conv1d_backward_workspace_bytes",
@@ -138,7 +138,7 @@ def load():
     # (the second argument: a pointer to a size-map description, or None)
     lib.d2c_conv3d_columns_bytes.argtypes, lib.d2c_conv3d_columns_bytes.restype = [p3, vp], sz
     lib.d2c_conv3d_keep_bytes.argtypes, lib.d2c_conv3d_keep_bytes.restype = [p3, vp], sz
-    for name in ("forward_least", "backward_columns"):
+    for name in ("forward_least", "backward_columns", "forward_keep", "backward_keep"):
         f = getattr(lib, f"d2c_conv3d_{name}_workspace_bytes")
         f.argtypes, f.restype = [p3, vp], sz
     lib.d2c_conv3d_forward_columns.argtypes = [p3, vp] + [vp] * 6 + [vp, sz, vp, sz, vp]

@@ -48,6 +48,18 @@ def _workspace(nbytes, dev):
     return ws
 
 
+def _forward_workspace(lib, nbytes, desc, sdesc, dev):
+    """Workspace of a forward call that keeps no columns, and its size.  What such a call takes beyond the least it runs with,
+    to hold the columns in, is not kept from call to call, and a call that does not get it runs with the least."""
+    least = lib.d2c_conv3d_forward_least_workspace_bytes(ctypes.byref(desc), ctypes.byref(sdesc) if sdesc is not None else None)
+    if nbytes > least:
+        try:
+            return torch.empty(nbytes, dtype=torch.uint8, device=dev), nbytes
+        except torch.cuda.OutOfMemoryError:
+            nbytes = least
+    return _workspace(nbytes, dev), nbytes
+
+
 def _release_workspaces():
     """Drops the cached workspace tensors (they return to torch's caching allocator)."""
     _WS_CACHE.clear()
@@ -216,13 +228,12 @@ class _DeformConv3dFunction(torch.autograd.Function):
         out = torch.empty((N, Cout, Do, Ho, Wo), dtype=input.dtype, device=dev)
         stats = torch.empty((N, Cout, 2), dtype=torch.float32, device=dev) if want_stats else None
         with torch.cuda.device(dev):
-            nb = (lib.d2c_conv3d_forward_stats_workspace_bytes(ctypes.byref(desc), None) if want_stats
-                  else lib.d2c_conv3d_forward_workspace_bytes(ctypes.byref(desc)))
-            ws = _workspace(nb, dev)
             npre = lib.d2c_conv3d_prepared_bytes(ctypes.byref(desc)) if (prepared is not None and not want_stats) else 0
             ctx.prepared = None
             columns = None
             if want_stats:
+                nb = lib.d2c_conv3d_forward_stats_workspace_bytes(ctypes.byref(desc), None)
+                ws, nb = _forward_workspace(lib, nb, desc, None, dev)
                 rc = lib.d2c_conv3d_forward_stats(ctypes.byref(desc), None, _ptr(input), _ptr(offset), _ptr(alpha),
                                                   _ptr(weight), _ptr(bias), _ptr(out), _ptr(stats), _ptr(ws), nb,
                                                   _stream(dev))
@@ -230,6 +241,8 @@ class _DeformConv3dFunction(torch.autograd.Function):
                 # the layer's prepared region: forward weights kept while the weight tensor is the same, the input's
                 # channels-last copy left there for the backward call of this forward call
                 buf = prepared.buffer(npre, dev)
+                nb = lib.d2c_conv3d_forward_least_workspace_bytes(ctypes.byref(desc), None)
+                ws = _workspace(nb, dev)
                 wkey = PreparedRegion.key(weight)
                 reuse = _lib.REUSE_FORWARD_WEIGHTS if prepared.fwd_weights == wkey else 0
                 rc = lib.d2c_conv3d_forward_prepared(ctypes.byref(desc), _ptr(input), _ptr(offset), _ptr(alpha),
@@ -241,10 +254,13 @@ class _DeformConv3dFunction(torch.autograd.Function):
             else:
                 columns = _columns_for(lib, desc, None, ctx.needs_input_grad[3], dev)
                 if columns is not None:
+                    nb = lib.d2c_conv3d_forward_keep_workspace_bytes(ctypes.byref(desc), None)
+                    ws = _workspace(nb, dev)
                     rc = lib.d2c_conv3d_forward_columns(ctypes.byref(desc), None, _ptr(input), _ptr(offset), _ptr(alpha),
                                                         _ptr(weight), _ptr(bias), _ptr(out), _ptr(columns),
                                                         columns.numel(), _ptr(ws), nb, _stream(dev))
                 else:
+                    ws, nb = _forward_workspace(lib, lib.d2c_conv3d_forward_workspace_bytes(ctypes.byref(desc)), desc, None, dev)
                     rc = lib.d2c_conv3d_forward(ctypes.byref(desc), _ptr(input), _ptr(offset), _ptr(alpha),
                                                 _ptr(weight), _ptr(bias), _ptr(out), _ptr(ws), nb, _stream(dev))
         _lib.check(rc, "deform_conv3d forward")
@@ -274,7 +290,7 @@ class _DeformConv3dFunction(torch.autograd.Function):
         gb = torch.empty_like(bias) if (bias is not None and need[4]) else None
         prepared = getattr(ctx, "prepared", None)
         with torch.cuda.device(dev):
-            nb = (lib.d2c_conv3d_backward_columns_workspace_bytes(ctypes.byref(desc), None) if columns is not None
+            nb = (lib.d2c_conv3d_backward_keep_workspace_bytes(ctypes.byref(desc), None) if columns is not None
                   else lib.d2c_conv3d_backward_workspace_bytes(ctypes.byref(desc)))
             ws = _workspace(nb, dev)
             if columns is not None:
@@ -354,21 +370,24 @@ class _DeformConv3dSizedFunction(torch.autograd.Function):
         out = torch.empty((N, Cout, Do, Ho, Wo), dtype=input.dtype, device=dev)
         stats = torch.empty((N, Cout, 2), dtype=torch.float32, device=dev) if want_stats else None
         with torch.cuda.device(dev):
-            nb = (lib.d2c_conv3d_forward_stats_workspace_bytes(ctypes.byref(desc), ctypes.byref(sdesc)) if want_stats
-                  else lib.d2c_conv3d_sized_forward_workspace_bytes(ctypes.byref(desc), ctypes.byref(sdesc)))
-            ws = _workspace(nb, dev)
             columns = None
             if want_stats:
+                nb = lib.d2c_conv3d_forward_stats_workspace_bytes(ctypes.byref(desc), ctypes.byref(sdesc))
+                ws, nb = _forward_workspace(lib, nb, desc, sdesc, dev)
                 rc = lib.d2c_conv3d_forward_stats(ctypes.byref(desc), ctypes.byref(sdesc), _ptr(input), _ptr(size_raw),
                                                   _ptr(alpha), _ptr(weight), _ptr(bias), _ptr(out), _ptr(stats),
                                                   _ptr(ws), nb, _stream(dev))
             else:
                 columns = _columns_for(lib, desc, sdesc, ctx.needs_input_grad[3], dev)
                 if columns is not None:
+                    nb = lib.d2c_conv3d_forward_keep_workspace_bytes(ctypes.byref(desc), ctypes.byref(sdesc))
+                    ws = _workspace(nb, dev)
                     rc = lib.d2c_conv3d_forward_columns(ctypes.byref(desc), ctypes.byref(sdesc), _ptr(input),
                                                         _ptr(size_raw), _ptr(alpha), _ptr(weight), _ptr(bias), _ptr(out),
                                                         _ptr(columns), columns.numel(), _ptr(ws), nb, _stream(dev))
                 else:
+                    nb = lib.d2c_conv3d_sized_forward_workspace_bytes(ctypes.byref(desc), ctypes.byref(sdesc))
+                    ws, nb = _forward_workspace(lib, nb, desc, sdesc, dev)
                     rc = lib.d2c_conv3d_sized_forward(ctypes.byref(desc), ctypes.byref(sdesc), _ptr(input),
                                                       _ptr(size_raw), _ptr(alpha), _ptr(weight), _ptr(bias), _ptr(out),
                                                       _ptr(ws), nb, _stream(dev))
@@ -399,7 +418,7 @@ class _DeformConv3dSizedFunction(torch.autograd.Function):
         gb = torch.empty_like(bias) if (bias is not None and need[4]) else None
         with torch.cuda.device(dev):
             if columns is not None:
-                nb = lib.d2c_conv3d_backward_columns_workspace_bytes(ctypes.byref(desc), ctypes.byref(sdesc))
+                nb = lib.d2c_conv3d_backward_keep_workspace_bytes(ctypes.byref(desc), ctypes.byref(sdesc))
                 ws = _workspace(nb, dev)
                 rc = lib.d2c_conv3d_backward_columns(ctypes.byref(desc), ctypes.byref(sdesc), _ptr(grad_out), _ptr(input),
                                                      _ptr(size_raw), _ptr(alpha), _ptr(weight), _ptr(columns),
@@ -501,25 +520,24 @@ class _DeformConv3dPackedFunction(torch.autograd.Function):
             if not want_stats:
                 columns = _columns_for(lib, desc, sdesc, ctx.needs_input_grad[2], dev)
             if columns is not None:
-                nb = (lib.d2c_conv3d_sized_forward_workspace_bytes(ctypes.byref(desc), sref) if sdesc is not None
-                      else lib.d2c_conv3d_forward_workspace_bytes(ctypes.byref(desc)))
+                nb = lib.d2c_conv3d_forward_keep_workspace_bytes(ctypes.byref(desc), sref)
                 ws = _workspace(nb, dev)
                 rc = lib.d2c_conv3d_forward_columns(ctypes.byref(desc), sref, _ptr(input), p_off, p_mask, _ptr(weight),
                                                     _ptr(bias), _ptr(out), _ptr(columns), columns.numel(), _ptr(ws), nb,
                                                     _stream(dev))
             elif want_stats:
                 nb = lib.d2c_conv3d_forward_stats_workspace_bytes(ctypes.byref(desc), sref)
-                ws = _workspace(nb, dev)
+                ws, nb = _forward_workspace(lib, nb, desc, sdesc, dev)
                 rc = lib.d2c_conv3d_forward_stats(ctypes.byref(desc), sref, _ptr(input), p_off, p_mask, _ptr(weight),
                                                   _ptr(bias), _ptr(out), _ptr(stats), _ptr(ws), nb, _stream(dev))
             elif sdesc is not None:
                 nb = lib.d2c_conv3d_sized_forward_workspace_bytes(ctypes.byref(desc), sref)
-                ws = _workspace(nb, dev)
+                ws, nb = _forward_workspace(lib, nb, desc, sdesc, dev)
                 rc = lib.d2c_conv3d_sized_forward(ctypes.byref(desc), sref, _ptr(input), p_off, p_mask, _ptr(weight),
                                                   _ptr(bias), _ptr(out), _ptr(ws), nb, _stream(dev))
             else:
                 nb = lib.d2c_conv3d_forward_workspace_bytes(ctypes.byref(desc))
-                ws = _workspace(nb, dev)
+                ws, nb = _forward_workspace(lib, nb, desc, sdesc, dev)
                 rc = lib.d2c_conv3d_forward(ctypes.byref(desc), _ptr(input), p_off, p_mask, _ptr(weight), _ptr(bias),
                                             _ptr(out), _ptr(ws), nb, _stream(dev))
         _lib.check(rc, "deform_conv3d_packed forward")
@@ -552,7 +570,7 @@ class _DeformConv3dPackedFunction(torch.autograd.Function):
         with torch.cuda.device(dev):
             if columns is not None:
                 sref = ctypes.byref(sdesc) if sdesc is not None else None
-                nb = lib.d2c_conv3d_backward_columns_workspace_bytes(ctypes.byref(desc), sref)
+                nb = lib.d2c_conv3d_backward_keep_workspace_bytes(ctypes.byref(desc), sref)
                 ws = _workspace(nb, dev)
                 rc = lib.d2c_conv3d_backward_columns(ctypes.byref(desc), sref, _ptr(grad_out), _ptr(input), p_off, p_mask,
                                                      _ptr(weight), _ptr(columns), columns.numel(), _ptr(gx), g_off, g_mask,

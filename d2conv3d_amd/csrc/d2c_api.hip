@@ -716,9 +716,22 @@ int d2c_conv3d_forward_columns(const d2c_conv3d_desc *q, const d2c_size_map_desc
     if (int rc = z ? sized_check(q, z) : d2c_conv3d_check(q)) return rc;
     if (!x || !offset || !weight || !out) { d2c_set_error("null tensor pointer"); return D2C_ERR_SHAPE; }
     if (int rc = check_columns(*q, z, columns, columns_bytes)) return rc;
-    if (int rc = check_ws(d2c_tiled_forward_ws(*q), ws, ws_bytes)) return rc;
+    const bool keep = columns_bytes >= d2c_tiled_keep_bytes(*q, z);
+    if (int rc = check_ws(d2c_tiled_forward_ws(*q, keep ? D2C_FWD_WS_KEEP_LEAST : D2C_FWD_WS_LEAST), ws, ws_bytes)) return rc;
     return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, ws_bytes, (hipStream_t)stream, z, nullptr, nullptr, columns,
                              columns_bytes);
+}
+
+size_t d2c_conv3d_forward_keep_workspace_bytes(const d2c_conv3d_desc *q, const d2c_size_map_desc *z)
+{
+    if ((z ? sized_check(q, z) : d2c_conv3d_check(q)) != D2C_OK || !columns_served(*q, z)) return 0;
+    return d2c_tiled_forward_ws(*q, D2C_FWD_WS_KEEP);
+}
+
+size_t d2c_conv3d_backward_keep_workspace_bytes(const d2c_conv3d_desc *q, const d2c_size_map_desc *z)
+{
+    if ((z ? sized_check(q, z) : d2c_conv3d_check(q)) != D2C_OK || !columns_served(*q, z)) return 0;
+    return d2c_tiled_backward_ws(*q, z, true, true);
 }
 
 size_t d2c_conv3d_backward_columns_workspace_bytes(const d2c_conv3d_desc *q, const d2c_size_map_desc *z)
@@ -735,7 +748,8 @@ int d2c_conv3d_backward_columns(const d2c_conv3d_desc *q, const d2c_size_map_des
     if (int rc = z ? sized_check(q, z) : d2c_conv3d_check(q)) return rc;
     if (!gout || !x || !offset || !weight) { d2c_set_error("null tensor pointer"); return D2C_ERR_SHAPE; }
     if (int rc = check_columns(*q, z, columns, columns_bytes)) return rc;
-    if (int rc = check_ws(d2c_tiled_backward_ws(*q, z, true), ws, ws_bytes)) return rc;
+    const bool keep = columns_bytes >= d2c_tiled_keep_bytes(*q, z);
+    if (int rc = check_ws(d2c_tiled_backward_ws(*q, z, true, keep), ws, ws_bytes)) return rc;
     return d2c_tiled_backward(*q, gout, x, offset, mask, weight, gx, goff, gmask, gw, gb, ws, (hipStream_t)stream, z,
                               nullptr, columns, columns_bytes);
 }

@@ -412,7 +412,9 @@ FwdWs fwd_ws(const d2c_conv3d_desc &q, const TiledShape &s)
         w.lists = w.gemm + d2c_align_up(d2c_col_forward_ws(q));
         w.col = w.lists + d2c_brick_ws(s).total;
         w.end = w.col + brick_col_bytes(s);
-        w.total = std::max(w.total, use_brick_forward(q, s, false) ? w.end : w.col);
+        if (use_brick_forward(q, s, false)) w.total = std::max(w.total, w.end);
+        // (where the gathering kernel writes no columns, every forward workspace has to do for a call that keeps them)
+        if (!d2c_fwd_writes_columns(s, q.dtype)) w.total = std::max(w.total, w.lists);
     }
     return w;
 }
@@ -651,8 +653,9 @@ BwdSlices bwd_slices(const d2c_conv3d_desc &q, const TiledShape &s)
 struct BwdWs {
     size_t xcl, wt, gxcl, gwacc, goutp, auxacc, gcol, counts, entries, ovf, gsacc, sm1, brick, res, gemm, col, total;
 };
-// `saved_columns`: the caller brings the sampled columns of the forward call (no column region, no slices)
-BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns = false)
+// `saved_columns`: the caller brings the sampled columns of the forward call (no column region, no slices); `sorted`: and
+// the sorted points behind them
+BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns = false, bool sorted = false)
 {
     const size_t es = d2c_elem_size(q.dtype);
     BwdWs w;
@@ -692,7 +695,7 @@ BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns =
     w.sm1 = w.total;       // ... and (size - 1) per axis
     if (s.ss.on) w.total += d2c_align_up((size_t)s.N * 3 * s.P * sizeof(float));
     w.brick = w.total;     // sorted points
-    if (use_brick(q, s)) w.total += d2c_brick_ws(s).total;
+    if (use_brick(q, s) && !sorted) w.total += d2c_brick_ws(s).total;
     w.res = w.total;       // ... and sums per point
     if (use_brick(q, s)) w.total += d2c_brick_ws(s).res_bytes;
     w.gemm = w.total;      // operands of the grad-column product
@@ -746,7 +749,7 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
     // (kept columns of a forward call over sorted points: those follow the columns)
     const bool sorted = columns && use_brick_forward(q, s, true) && columns_bytes >= brick_keep_bytes(s);
     const bool brick = use_brick(q, s) && !(gw && gw_mode(q) == 2);      // (not: columns in the rows' place)
-    const BwdWs l = bwd_ws(q, s, columns != nullptr);
+    const BwdWs l = bwd_ws(q, s, columns != nullptr, sorted);
     const PreparedLayout pl = prepared_layout(q, s);
     char *xcl_p = prep ? (char *)prep->base + pl.xcl : base + l.xcl;
     // (the transposed weights of the region serve single-pass reductions; wider weight groups re-pack per pass)
@@ -1016,14 +1019,17 @@ size_t d2c_tiled_forward_ws(const d2c_conv3d_desc &q, D2cForwardWs which)
     switch (which) {
     case D2C_FWD_WS_LEAST: return l.least;
     case D2C_FWD_WS_STATS: return l.least + (d2c_fwd_fills_stats(s) ? d2c_fwd_stats_ws(s) : 0);
+    case D2C_FWD_WS_KEEP: return use_brick_forward(q, s, true) ? l.lists : l.least;
+    case D2C_FWD_WS_KEEP_LEAST:
+        return !use_brick_forward(q, s, true) ? l.least : (d2c_fwd_writes_columns(s, q.dtype) ? std::min(l.least, l.lists) : l.lists);
     default: return l.total;
     }
 }
 
-size_t d2c_tiled_backward_ws(const d2c_conv3d_desc &q, const d2c_size_map_desc *sz, bool saved_columns)
+size_t d2c_tiled_backward_ws(const d2c_conv3d_desc &q, const d2c_size_map_desc *sz, bool saved_columns, bool keep)
 {
     const TiledShape s = tiled_shape(q, 3, 0, sz);
-    return is_depthwise(q) ? dw_ws(q, s).total_bwd : bwd_ws(q, s, saved_columns).total;
+    return is_depthwise(q) ? dw_ws(q, s).total_bwd : bwd_ws(q, s, saved_columns, keep && use_brick_forward(q, s, true)).total;
 }
 
 // Bytes of the sampled columns that a forward call can keep for the backward call of the same step:
@@ -1034,7 +1040,10 @@ size_t d2c_tiled_columns_bytes(const d2c_conv3d_desc &q, const d2c_size_map_desc
     if (is_depthwise(q) || !mfma_channels_ok(q)) return 0;
     if (sz && !d2c_tiled_sized_supported(q, true)) return 0;
     const TiledShape s = tiled_shape(q, 3, 0, sz);
-    if (use_brick_forward(q, s, true)) return d2c_bwd_weight_from_kept_col(s, q.dtype) && use_aux_kernel(q, s) ? brick_col_bytes(s) : 0;
+    // (where only the sorted points give columns, they are kept with them)
+    if (use_brick_forward(q, s, true))
+        return !d2c_bwd_weight_from_kept_col(s, q.dtype) || !use_aux_kernel(q, s) ? 0
+               : d2c_fwd_writes_columns(s, q.dtype) ? brick_col_bytes(s) : brick_keep_bytes(s);
     if (!d2c_fwd_writes_columns(s, q.dtype) || !d2c_bwd_weight_from_kept_col(s, q.dtype) || !use_aux_kernel(q, s)) return 0;
     const long rows = d2c_columns_rows(s), chunks = s.Cin / bkc_of(q.dtype);
     if (chunks * s.K * rows >= (1L << 31)) return 0;      // (the kernel counts rows in 32 bits)

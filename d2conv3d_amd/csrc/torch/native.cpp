@@ -87,6 +87,21 @@ Tensor workspace(size_t bytes, const Tensor &like, hipStream_t st)
     return THPVariable_Unpack(made.ptr());
 }
 
+// ... of a forward call that keeps no columns.  What it takes beyond the least it runs with, to hold the columns in, is not
+// kept from call to call, and a call that does not get it runs with the least.
+Tensor forward_workspace(size_t &bytes, const d2c_conv3d_desc &q, const d2c_size_map_desc *sz, const Tensor &like, hipStream_t st)
+{
+    const size_t least = d2c_conv3d_forward_least_workspace_bytes(&q, sz);
+    if (bytes > least) {
+        try {
+            return at::empty({(int64_t)bytes}, like.options().dtype(at::kByte).requires_grad(false));
+        } catch (const c10::OutOfMemoryError &) {
+            bytes = least;
+        }
+    }
+    return workspace(bytes, like, st);
+}
+
 Tensor no_grad_empty_like(const Tensor &t) { return at::empty(t.sizes(), t.options().requires_grad(false)); }
 
 // Gradients that leave a node while a graph of the backward pass is being recorded: differentiating them is an error
@@ -131,7 +146,6 @@ Tensor forward_3d(const Call3d &c, const Tensor &x, const Tensor &off, const Ten
     c10::DeviceGuard guard(x.device());
     const hipStream_t st = stream_of(x);
     Tensor out = at::empty({q.N, q.Cout, q.Do, q.Ho, q.Wo}, x.options().requires_grad(false));
-    const size_t nb = c.sized ? d2c_conv3d_sized_forward_workspace_bytes(&q, &c.size) : d2c_conv3d_forward_workspace_bytes(&q);
     if (keep) {
         const size_t n = d2c_conv3d_keep_bytes(&q, c.sz());
         if (n > 0 && n <= keep_max) {
@@ -141,7 +155,9 @@ Tensor forward_3d(const Call3d &c, const Tensor &x, const Tensor &off, const Ten
             }
         }
     }
-    const Tensor ws = workspace(nb, x, st);
+    size_t nb = columns.defined() ? d2c_conv3d_forward_keep_workspace_bytes(&q, c.sz())
+                : c.sized ? d2c_conv3d_sized_forward_workspace_bytes(&q, &c.size) : d2c_conv3d_forward_workspace_bytes(&q);
+    const Tensor ws = columns.defined() ? workspace(nb, x, st) : forward_workspace(nb, q, c.sz(), x, st);
     const void *po = ptr(off), *pm = c.form == PACKED ? ptr_at(off, c.lead) : ptr(alpha);
     int rc;
     if (columns.defined())
@@ -181,7 +197,7 @@ struct DeformConv3dBackward : public Node {
             if (has_bias && should_compute_output(4)) r[4] = at::empty({q.Cout}, vw.options().requires_grad(false));
             const void *pm = c.form == PACKED ? ptr_at(vo, c.lead) : ptr(va);
             void *gm = c.form == PACKED ? ptr_at(r[1], c.lead) : ptr(r[2]);
-            const size_t nb = columns.defined() ? d2c_conv3d_backward_columns_workspace_bytes(&q, c.sz())
+            const size_t nb = columns.defined() ? d2c_conv3d_backward_keep_workspace_bytes(&q, c.sz())
                               : c.sized ? d2c_conv3d_sized_backward_workspace_bytes(&q, &c.size) : d2c_conv3d_backward_workspace_bytes(&q);
             const Tensor ws = workspace(nb, vx, st);
             int rc;

@@ -213,8 +213,12 @@ struct d2c_size_map_desc;
 size_t d2c_conv3d_columns_bytes(const d2c_conv3d_desc *desc, const struct d2c_size_map_desc *size_map);
 /* What is worth keeping: d2c_conv3d_columns_bytes(), or more where the forward pass also sorts the sampling points by
  * their place in the volume and its backward call can take them over.  A buffer of this size handed to both calls (with
- * this size as columns_bytes) spares the backward call its own sort. */
+ * this size as columns_bytes) spares the backward call its own sort, and both part of their workspace: the
+ * *_keep_workspace_bytes() are for calls with such a buffer.  (With a buffer of d2c_conv3d_columns_bytes():
+ * d2c_conv3d_forward_workspace_bytes() and d2c_conv3d_backward_columns_workspace_bytes().) */
 size_t d2c_conv3d_keep_bytes(const d2c_conv3d_desc *desc, const struct d2c_size_map_desc *size_map);
+size_t d2c_conv3d_forward_keep_workspace_bytes(const d2c_conv3d_desc *desc, const struct d2c_size_map_desc *size_map);
+size_t d2c_conv3d_backward_keep_workspace_bytes(const d2c_conv3d_desc *desc, const struct d2c_size_map_desc *size_map);
 int d2c_conv3d_forward_columns(const d2c_conv3d_desc *desc, const struct d2c_size_map_desc *size_map, const void *x,
                                const void *offset, const void *mask, const void *weight, const void *bias, void *out,
                                void *columns, size_t columns_bytes, void *workspace, size_t workspace_bytes,

@@ -213,3 +213,74 @@ def test_the_static_workspace_serves_large_problems_without_columns(dev):
                                        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
     _lib.check(rc, "forward_static")
     assert rel_l2(out, want) < 4e-3
+
+
+def test_a_forward_call_without_room_for_its_columns_runs_without(dev):
+    ts, desc = _large(dev)
+    lib = _lib.load()
+    fast = lib.d2c_conv3d_forward_workspace_bytes(ctypes.byref(desc))
+    least = lib.d2c_conv3d_forward_least_workspace_bytes(ctypes.byref(desc), None)
+    assert fast > least + (100 << 20)
+    _ops.config.release_workspaces()
+    with torch.no_grad():
+        want = d2c.deform_conv3d(*ts, 1, 1, 1, 1, 1)
+        # (the columns are not kept from call to call)
+        assert all(n <= least for n in _ops.config.cached_workspace_bytes().values())
+        _ops.config.release_workspaces()
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        total = torch.cuda.get_device_properties(dev).total_memory
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + least + (64 << 20)) / total)
+        try:
+            with pytest.raises(torch.cuda.OutOfMemoryError):
+                torch.empty(fast, dtype=torch.uint8, device=dev)
+            native = d2c.deform_conv3d(*ts, 1, 1, 1, 1, 1)
+            python = _ops._DeformConv3dFunction.apply(*ts, *[1] * 11)
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+            _ops.config.release_workspaces()
+        assert rel_l2(python, want) < 4e-3
+        assert rel_l2(native, want) < 4e-3
+
+
+def test_forward_workspace_holds_what_the_call_uses(dev):
+    """8 offset groups of 64 channels: a call that keeps no columns gathers (no sorted points in its workspace), one that keeps
+    them finds room for both in the buffer it brings."""
+    _, desc = _large(dev, N=2, C=512, G=8)
+    lib, d = _lib.load(), ctypes.byref(desc)
+    least = lib.d2c_conv3d_forward_least_workspace_bytes(d, None)
+    assert lib.d2c_conv3d_forward_workspace_bytes(d) == least < 100e6
+    ncol, nkeep = lib.d2c_conv3d_columns_bytes(d, None), lib.d2c_conv3d_keep_bytes(d, None)
+    assert 0 < ncol < nkeep
+    # (the input channels-last, the weights in the operands' order, partial sums of a last round of tiles)
+    assert 0 < lib.d2c_conv3d_forward_keep_workspace_bytes(d, None) < 160e6
+
+
+@pytest.mark.parametrize("which", ["forward", "least"])
+def test_kept_points_do_not_depend_on_the_workspace(which, dev):
+    """d2c_conv3d_forward_columns with a buffer for columns and sorted points, and any workspace it accepts: the backward call
+    finds both."""
+    ts, desc = _large(dev, C=128)
+    lib, d = _lib.load(), ctypes.byref(desc)
+    p = lambda t: ctypes.c_void_p(t.data_ptr() if t is not None else 0)
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    x, off, m, w, _ = ts
+    nb = lib.d2c_conv3d_forward_keep_workspace_bytes(d, None)
+    if which == "least":
+        nb = min(nb, lib.d2c_conv3d_forward_least_workspace_bytes(d, None))
+    else:
+        nb = lib.d2c_conv3d_forward_workspace_bytes(d)
+    buf = torch.empty(lib.d2c_conv3d_keep_bytes(d, None), dtype=torch.uint8, device=dev)
+    ws = torch.empty(nb, dtype=torch.uint8, device=dev)
+    out, gx, goff, gm, gw = (torch.empty_like(t) for t in (x, x, off, m, w))
+    _lib.check(lib.d2c_conv3d_forward_columns(d, None, p(x), p(off), p(m), p(w), None, p(out), p(buf), buf.numel(), p(ws), nb, st), "forward")
+    nb = lib.d2c_conv3d_backward_keep_workspace_bytes(d, None)
+    assert nb < lib.d2c_conv3d_backward_columns_workspace_bytes(d, None)
+    ws = torch.empty(nb, dtype=torch.uint8, device=dev)
+    _lib.check(lib.d2c_conv3d_backward_columns(d, None, p(out), p(x), p(off), p(m), p(w), p(buf), buf.numel(), p(gx), p(goff), p(gm), p(gw),
+                                               None, p(ws), nb, st), "backward")
+    leaves = [t.detach().requires_grad_(True) for t in (x, off, m, w)]
+    want = d2c.deform_conv3d(*leaves, None, 1, 1, 1, 1, 1)
+    want.backward(out)
+    for a, e in zip((out, gx, goff, gm, gw), [want] + [t.grad for t in leaves]):
+        assert rel_l2(a, e) < 4e-3
