@@ -650,13 +650,20 @@ BwdSlices bwd_slices(const d2c_conv3d_desc &q, const TiledShape &s)
     return r;
 }
 
+// Whether a backward call runs on the bricks: not one slice by slice, and not one that writes its columns over the rows.
+// `saved_columns`: the caller brings the sampled columns of the forward call (no column region, no slices)
+bool brick_backward(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns)
+{
+    return use_brick(q, s) && (saved_columns || (gw_mode(q) != 2 && bwd_slices(q, s).gs == 0));
+}
+
 struct BwdWs {
     size_t xcl, wt, gxcl, gwacc, goutp, auxacc, gcol, counts, entries, ovf, gsacc, sm1, brick, res, gemm, col, total;
 };
-// `saved_columns`: the caller brings the sampled columns of the forward call (no column region, no slices); `sorted`: and
-// the sorted points behind them
+// `sorted`: ... and the sorted points behind them
 BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns = false, bool sorted = false)
 {
+    const bool brick = brick_backward(q, s, saved_columns);
     const size_t es = d2c_elem_size(q.dtype);
     BwdWs w;
     w.xcl = 0;
@@ -681,7 +688,7 @@ BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns =
         const size_t chunks = sl.gs ? (size_t)sl.gs * (s.cpg / bkc_of(q.dtype)) : (size_t)(s.Cin / bkc_of(q.dtype));
         w.total = w.gcol + d2c_align_up((chunks * s.K * s.M + 64) * bkc_of(q.dtype) * es);
     }
-    if (use_lists(q, s)) {
+    if (use_lists(q, s) && !brick) {
         size_t c, en, ov;
         d2c_lists_ws(s, q.dtype, &c, &en, &ov);
         w.counts = w.total;
@@ -695,11 +702,11 @@ BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns =
     w.sm1 = w.total;       // ... and (size - 1) per axis
     if (s.ss.on) w.total += d2c_align_up((size_t)s.N * 3 * s.P * sizeof(float));
     w.brick = w.total;     // sorted points
-    if (use_brick(q, s) && !sorted) w.total += d2c_brick_ws(s).total;
+    if (brick && !sorted) w.total += d2c_brick_ws(s).total;
     w.res = w.total;       // ... and sums per point
-    if (use_brick(q, s)) w.total += d2c_brick_ws(s).res_bytes;
+    if (brick) w.total += d2c_brick_ws(s).res_bytes;
     w.gemm = w.total;      // operands of the grad-column product
-    if (use_brick(q, s) && d2c_grad_col_supported(q)) w.total += d2c_grad_col_ws(q);
+    if (brick && d2c_grad_col_supported(q)) w.total += d2c_grad_col_ws(q);
     w.col = w.total;       // sampled columns for the grad-weight product
     if (!saved_columns && use_col_weight(q, s) && !col_in_place(q, s))
         w.total += d2c_align_up(d2c_bwd_col_bytes(s, q.dtype, sl.cgs ? sl.cgs * (s.cpg / 64) : 0));
@@ -748,7 +755,7 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
     }
     // (kept columns of a forward call over sorted points: those follow the columns)
     const bool sorted = columns && use_brick_forward(q, s, true) && columns_bytes >= brick_keep_bytes(s);
-    const bool brick = use_brick(q, s) && !(gw && gw_mode(q) == 2);      // (not: columns in the rows' place)
+    const bool brick = nd == 3 && brick_backward(q, s, columns != nullptr);
     const BwdWs l = bwd_ws(q, s, columns != nullptr, sorted);
     const PreparedLayout pl = prepared_layout(q, s);
     char *xcl_p = prep ? (char *)prep->base + pl.xcl : base + l.xcl;

@@ -284,3 +284,21 @@ def test_kept_points_do_not_depend_on_the_workspace(which, dev):
     want.backward(out)
     for a, e in zip((out, gx, goff, gm, gw), [want] + [t.grad for t in leaves]):
         assert rel_l2(a, e) < 4e-3
+
+
+def test_memory_saving_backward_holds_no_bricks(dev):
+    """2x512x8x30x54 in 8 offset groups: the settings that exist to save memory need what they needed when they were the only way
+    (1297 MB with the columns in the rows' place, 939 MB in four slices), and no call holds both kinds of lists."""
+    lib = _lib.load()
+    _, desc = _large(dev, N=2, C=512, G=8)
+    need = {}
+    for name, flags in (("default", 0), ("in_place", _lib.BWD_GW_IN_PLACE), ("slices4", _lib.bwd_slices(4))):
+        desc.backward_flags = flags
+        need[name] = lib.d2c_conv3d_backward_workspace_bytes(ctypes.byref(desc))
+    assert need["in_place"] < 1300e6 and need["slices4"] < 942e6, need
+    desc.backward_flags = 0
+    kept = lib.d2c_conv3d_backward_keep_workspace_bytes(ctypes.byref(desc), None)
+    sorts = lib.d2c_conv3d_backward_columns_workspace_bytes(ctypes.byref(desc), None)
+    columns = lib.d2c_conv3d_columns_bytes(ctypes.byref(desc), None)
+    assert kept < sorts <= need["default"] - columns + 1024
+    assert need["default"] < 2100e6, need
