@@ -5,7 +5,9 @@ with the flat argument lists of dconv1d.h:161-172 / dconv3d.h:188-205, and the
 arithmetic in the C-ABI HIP library.
 """
 import ctypes
+import importlib
 import types
+import warnings
 
 import torch
 from torch.autograd.function import once_differentiable
@@ -77,17 +79,40 @@ def _workspace_bytes_cached():
 
 # The calls that need nothing special, in native code (csrc/torch/native.cpp): operator call and autograd node.  A native
 # function returns None for a call that it leaves to the Python code below.
-try:
-    from . import _native
-except ImportError:
-    _native = None
-else:
-    _native.init(_WS_CACHE, _WS_CACHE_ON, _workspace)
+_native = None
+_NATIVE_MISSING = [None]      # why there is none, where nothing has been said of it yet
+
+
+def _load_native():
+    """Not fatal here: the package is imported to build it."""
+    global _native
+    _native, _NATIVE_MISSING[0] = None, None
+    try:
+        _native = importlib.import_module("._native", __package__)
+        _native.init(_WS_CACHE, _WS_CACHE_ON, _workspace)
+    except ImportError as e:
+        _NATIVE_MISSING[0] = e
+
+
+_load_native()
+
+
+def _no_native():
+    """A binding that was built and does not load is an error; without one the Python functions below do every call, at
+    their cost in host time, which is said once."""
+    e, _NATIVE_MISSING[0] = _NATIVE_MISSING[0], None
+    if isinstance(e, ModuleNotFoundError):
+        warnings.warn("d2conv3d_amd: the torch binding _native.so is not built (python -m d2conv3d_amd.build); calls run through "
+                      "Python, 40 - 130 us each more on the host")
+    elif e is not None:
+        _NATIVE_MISSING[0] = e
+        raise RuntimeError("d2conv3d_amd: the torch binding _native.so does not load; build it again (python -m "
+                           "d2conv3d_amd.build --force)") from e
 
 
 def _try_native(name, *args):
     if _native is None:
-        return None
+        return _no_native()
     try:
         return getattr(_native, name)(*args)
     except TypeError:      # (an argument of another type: the Python code converts it or says what is wrong)

@@ -104,11 +104,11 @@ Tensor forward_workspace(size_t &bytes, const d2c_conv3d_desc &q, const d2c_size
 
 Tensor no_grad_empty_like(const Tensor &t) { return at::empty(t.sizes(), t.options().requires_grad(false)); }
 
-// Gradients that leave a node while a graph of the backward pass is being recorded: differentiating them is an error
-// (torch's once_differentiable).
-void once_differentiable(variable_list &grads)
+// Gradients that leave a node while a graph of the backward pass is being recorded through its grad_out: differentiating
+// them is an error (torch's once_differentiable).
+void once_differentiable(variable_list &grads, const Tensor &grad_out)
 {
-    if (!at::GradMode::is_enabled()) return;
+    if (!at::GradMode::is_enabled() || !grad_out.requires_grad()) return;
     auto err = std::make_shared<torch::autograd::DelayedError>(
         "trying to differentiate twice a function that was marked with @once_differentiable", 1);
     for (auto &g : grads)
@@ -176,12 +176,14 @@ struct DeformConv3dBackward : public Node {
     std::string name() const override { return "DeformConv3dBackward"; }
     void release_variables() override
     {
+        const std::lock_guard<std::mutex> lock(mutex_);
         x.reset_data(); off.reset_data(); alpha.reset_data(); w.reset_data(); kept.reset_data();
     }
     variable_list apply(variable_list &&grads) override
     {
         variable_list r(5);
-        if (!grads[0].defined()) return r;
+        const std::lock_guard<std::mutex> lock(mutex_);
+        if (!grads[0].defined()) grads[0] = input_metadata(0).zeros_like();
         {
             at::NoGradGuard no_grad;
             const Tensor vx = x.unpack(), vo = off.unpack(), va = has_alpha ? alpha.unpack() : Tensor(), vw = w.unpack();
@@ -212,7 +214,7 @@ struct DeformConv3dBackward : public Node {
                                          nb, st);
             check(rc, c.form == OFFSETS ? "deform_conv3d backward" : (c.form == SIZED ? "deform_conv3d_sized backward" : "deform_conv3d_packed backward"));
         }
-        once_differentiable(r);
+        once_differentiable(r, grads[0]);
         return r;
     }
 };
@@ -326,11 +328,16 @@ struct DeformConv1dBackward : public Node {
     SavedVariable x, off, alpha, w;
     bool has_alpha = false, has_bias = false;
     std::string name() const override { return "DeformConv1dBackward"; }
-    void release_variables() override { x.reset_data(); off.reset_data(); alpha.reset_data(); w.reset_data(); }
+    void release_variables() override
+    {
+        const std::lock_guard<std::mutex> lock(mutex_);
+        x.reset_data(); off.reset_data(); alpha.reset_data(); w.reset_data();
+    }
     variable_list apply(variable_list &&grads) override
     {
         variable_list r(5);
-        if (!grads[0].defined()) return r;
+        const std::lock_guard<std::mutex> lock(mutex_);
+        if (!grads[0].defined()) grads[0] = input_metadata(0).zeros_like();
         {
             at::NoGradGuard no_grad;
             const Tensor vx = x.unpack(), vo = off.unpack(), va = has_alpha ? alpha.unpack() : Tensor(), vw = w.unpack();
@@ -347,7 +354,7 @@ struct DeformConv1dBackward : public Node {
             check(d2c_conv1d_backward(&q, ptr(g), ptr(vx), ptr(vo), ptr(va), ptr(vw), ptr(r[0]), ptr(r[1]), ptr(r[2]), ptr(r[3]), ptr(r[4]),
                                       ptr(ws), nb, st), "deform_conv1d backward");
         }
-        once_differentiable(r);
+        once_differentiable(r, grads[0]);
         return r;
     }
 };
@@ -405,11 +412,16 @@ struct PlainConv3dBackward : public Node {
     SavedVariable kept, w;           // the input channels-last, as the forward call made it
     bool has_bias = false;
     std::string name() const override { return "PlainConv3dBackward"; }
-    void release_variables() override { w.reset_data(); kept.reset_data(); }
+    void release_variables() override
+    {
+        const std::lock_guard<std::mutex> lock(mutex_);
+        w.reset_data(); kept.reset_data();
+    }
     variable_list apply(variable_list &&grads) override
     {
         variable_list r(3);
-        if (!grads[0].defined()) return r;
+        const std::lock_guard<std::mutex> lock(mutex_);
+        if (!grads[0].defined()) grads[0] = input_metadata(0).zeros_like();
         {
             at::NoGradGuard no_grad;
             const Tensor vw = w.unpack(), copy = kept.unpack();
@@ -425,7 +437,7 @@ struct PlainConv3dBackward : public Node {
             check(d2c_plain_conv3d_backward(&q, ptr(g), ptr(copy), copy.numel(), ptr(vw), ptr(r[0]), ptr(r[1]), ptr(r[2]), ptr(ws), nb, st),
                   "plain_conv3d backward");
         }
-        once_differentiable(r);
+        once_differentiable(r, grads[0]);
         return r;
     }
 };
@@ -483,11 +495,16 @@ struct DepthwiseConv3dBackward : public Node {
     SavedVariable x, w;
     bool has_bias = false;
     std::string name() const override { return "DepthwiseConv3dBackward"; }
-    void release_variables() override { x.reset_data(); w.reset_data(); }
+    void release_variables() override
+    {
+        const std::lock_guard<std::mutex> lock(mutex_);
+        x.reset_data(); w.reset_data();
+    }
     variable_list apply(variable_list &&grads) override
     {
         variable_list r(3);
-        if (!grads[0].defined()) return r;
+        const std::lock_guard<std::mutex> lock(mutex_);
+        if (!grads[0].defined()) grads[0] = input_metadata(0).zeros_like();
         {
             at::NoGradGuard no_grad;
             const Tensor vx = x.unpack(), vw = w.unpack();
@@ -503,7 +520,6 @@ struct DepthwiseConv3dBackward : public Node {
             check(d2c_dwconv3d_backward(&q, ptr(g), ptr(vx), ptr(vw), ptr(r[0]), ptr(r[1]), ptr(r[2]), ptr(ws), nb, st),
                   "depthwise_separable_conv3d backward");
         }
-        once_differentiable(r);
         return r;
     }
 };

@@ -4,6 +4,7 @@ the reference's, and the Python surface has the reference's names."""
 import ctypes
 import os
 import re
+import warnings
 
 import pytest
 import torch
@@ -151,3 +152,26 @@ def test_plain_depthwise_boundary_without_gpu():
     from fast_depthwise_conv3d import DepthwiseConv3d  # noqa: F401
     import fast_depthwise_conv3d._ops as ops
     assert callable(ops.depthwise_separable_conv3d)
+
+
+def test_a_torch_binding_that_does_not_load_is_not_passed_over(monkeypatch):
+    """Built and broken: an error at the first call.  Not built: said once, and the Python functions do the calls."""
+    def load(error):
+        def fail(*a):
+            raise error
+        monkeypatch.setattr(_ops.importlib, "import_module", fail)
+        _ops._load_native()
+        monkeypatch.undo()
+    try:
+        load(ImportError("undefined symbol: d2c_conv3d_forward"))
+        for _ in range(2):
+            with pytest.raises(RuntimeError, match="does not load"):
+                _ops._try_native("conv3d")
+        load(ModuleNotFoundError("No module named 'd2conv3d_amd._native'"))
+        with pytest.warns(UserWarning, match="not built"):
+            assert _ops._try_native("conv3d") is None
+        with warnings.catch_warnings():
+            warnings.simplefilter("error")
+            assert _ops._try_native("conv3d") is None
+    finally:
+        _ops._load_native()

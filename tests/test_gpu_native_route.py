@@ -1,9 +1,11 @@
 """The operators' calls in native code (csrc/torch/native.cpp) against the Python functions that they stand in for."""
+import contextlib
+
 import pytest
 import torch
 
 import d2conv3d_amd as d2c
-from d2conv3d_amd import _ops
+from d2conv3d_amd import _ops, depthwise_conv
 from d2conv3d_amd.depthwise_conv import depthwise_separable_conv3d
 from _util import rel_l2
 
@@ -66,6 +68,142 @@ ENTRIES = {"conv3d": _conv3d(), "conv3d_bf16": _conv3d(torch.bfloat16), "sized":
 
 def _on(dev, ts, grad=False):
     return [t.to(dev).requires_grad_(grad) for t in ts]
+
+
+@pytest.fixture
+def python_route():
+    """A context in which every call goes through the Python functions."""
+    @contextlib.contextmanager
+    def route():
+        with pytest.MonkeyPatch.context() as mp:
+            mp.setattr(_ops, "_try_native", lambda *a: None)
+            mp.setattr(depthwise_conv, "_try_native", lambda *a: None)
+            yield
+    return route
+
+
+def _out_grad(out, seed=9):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(*out.shape, generator=g).to(out)
+
+
+def _plain_step(fn, ts, dev):
+    out = fn(*ts)
+    out.backward(_out_grad(out))
+    return [out] + [t.grad for t in ts]
+
+
+def _side_stream(fn, ts, dev):
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        out = fn(*ts)
+        out.backward(_out_grad(out))
+    torch.cuda.current_stream().wait_stream(side)
+    return [out] + [t.grad for t in ts]
+
+
+def _offloaded(fn, ts, dev):
+    """Everything a step keeps goes to host memory and comes back."""
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.detach().cpu(), lambda t: t.to(dev)):
+        out = fn(*ts)
+    out.backward(_out_grad(out))
+    return [out] + [t.grad for t in ts]
+
+
+def _retained(fn, ts, dev):
+    out = fn(*ts)
+    out.backward(_out_grad(out), retain_graph=True)
+    out.backward(_out_grad(out, seed=10))
+    with pytest.raises(RuntimeError, match="second time"):
+        out.backward(_out_grad(out))
+    return [out] + [t.grad for t in ts]
+
+
+def _strided(fn, ts, dev):
+    ts = [t.detach().transpose(0, -1).contiguous().transpose(0, -1).requires_grad_(True) for t in ts]
+    out = fn(*ts)
+    out.backward(_out_grad(out)[:1, :1].expand_as(out))
+    return [out] + [t.grad for t in ts]
+
+
+def _one_leaf(fn, ts, dev):
+    leaf = len(ts) - 2                                # (the weight)
+    ts = [t.detach().requires_grad_(i == leaf) for i, t in enumerate(ts)]
+    out = fn(*ts)
+    out.backward(_out_grad(out))
+    assert all(t.grad is None for i, t in enumerate(ts) if i != leaf)
+    return [out, ts[leaf].grad]
+
+
+class _NoGradient(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, g):
+        return None
+
+
+def _undefined(fn, ts, dev):
+    """A consumer whose backward pass hands nothing on: gradients of zero, as for any Python autograd function."""
+    out = fn(*ts)
+    _NoGradient.apply(out).sum().backward()
+    return [out] + [t.grad for t in ts]
+
+
+SCENARIOS = {f.__name__.strip("_"): f for f in (_plain_step, _side_stream, _offloaded, _retained, _strided, _one_leaf, _undefined)}
+
+
+@pytest.mark.parametrize("scenario", list(SCENARIOS))
+@pytest.mark.parametrize("name", list(ENTRIES))
+def test_native_and_python_routes_agree(name, scenario, dev, python_route):
+    fn, tensors = ENTRIES[name]
+    native = SCENARIOS[scenario](fn, _on(dev, tensors(4), True), dev)
+    with python_route():
+        python = SCENARIOS[scenario](fn, _on(dev, tensors(4), True), dev)
+    if scenario != "strided":                         # (the route that was meant: non-contiguous tensors are Python's)
+        assert native[0].grad_fn.name() != python[0].grad_fn.name() and "Function" not in native[0].grad_fn.name()
+    tol = 4e-3 if python[0].dtype == torch.bfloat16 else 1e-5         # (atomics: sums in another order, one rounding)
+    for i, (a, e) in enumerate(zip(native, python)):
+        assert a is not None and e is not None, i
+        assert a.dtype == e.dtype and a.shape == e.shape
+        if scenario == "undefined" and i > 0:
+            assert not a.any() and not e.any(), i
+        else:
+            assert rel_l2(a, e) < tol, (i, rel_l2(a, e))
+
+
+@pytest.mark.parametrize("name", [n for n in ENTRIES if n != "depthwise"])
+def test_differentiating_twice_is_an_error_on_both_routes(name, dev, python_route):
+    fn, tensors = ENTRIES[name]
+    def twice():
+        ts = _on(dev, tensors(5), True)
+        out = fn(*ts)
+        gx = torch.autograd.grad(out, ts, _out_grad(out), create_graph=True)
+        assert not any(g.requires_grad for g in gx)
+        out = fn(*ts)
+        for g in torch.autograd.grad(out, ts, _out_grad(out).requires_grad_(True), create_graph=True):
+            with pytest.raises(RuntimeError, match="differentiate twice"):
+                g.sum().backward(retain_graph=True)
+    twice()
+    with python_route():
+        twice()
+
+
+def test_what_native_code_leaves_to_python(dev, python_route):
+    """Types to unify, arguments of other types: the same results, not an error."""
+    fn, tensors = ENTRIES["conv3d_bf16"]
+    x, off, m, w, b = _on(dev, tensors(6))
+    want = fn(x, off, m, w, b)
+    for args in ((x, off, m.double(), w.float(), b), (x, off, m, w, b.float())):
+        assert rel_l2(fn(*args), want) < 4e-3
+    assert rel_l2(_ops.deform_conv3d(x, off, m, w, b, 1.0, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1), want) < 4e-3
+    with pytest.raises(RuntimeError, match="ndimension"):
+        fn(x, off, m, w, b[None])
+    with pytest.raises(RuntimeError, match="offset.size"):
+        fn(x, off[:, :3], m, w, b)
 
 
 @pytest.mark.parametrize("name", list(ENTRIES))
