@@ -25,11 +25,6 @@ int d2c_gx_mode();
 
 namespace {
 
-template <class F, int... I> D2C_DEV void for_each_const(F &&f, std::integer_sequence<int, I...>)
-{
-    (f(std::integral_constant<int, I>{}), ...);
-}
-
 D2C_DEV int xcd_swizzle(int bid, int n)
 {
     const int x = bid & 7, idx = bid >> 3;

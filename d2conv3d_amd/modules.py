@@ -53,16 +53,16 @@ def release_zero_offsets():
 
 def _branch_conv(layer, x):
     """The deformation branch of a layer: its stock convolution `deform_params` (network/layers.py:66-68).  Where that
-    is a plain nn.Conv3d whose shape the matrix-core kernels serve, it is evaluated by the deformable operator at
-    all-zero offsets without modulation -- the same convolution (sampling points on the voxels, zero padding outside
-    the volume), on this library's kernels instead of the vendor library's im2col + GEMM + col2im: 1.3 - 2.3 times
-    faster forward + backward at the reference networks' layer sizes (1024 -> 108 channels, 8x30x54, bfloat16: 2.5
-    against 3.6 ms; 256 -> 108, 8x60x107, float32: 4.7 against 10.8 ms).  `layer.branch_on_operator`: True (default) does
-    so for bfloat16, where the two convolutions differ by less than either differs from a float64 run of the layer;
-    "all" also for float32, where the forward kernel's two-term bfloat16 operands move the predicted offsets by a few
-    1e-6 of their size -- enough to put one sampling point in 10^4 .. 10^5 on the other side of a voxel boundary, where
-    grad_offset jumps (the layer's grad_input then agrees with a float64 run to 2e-3 instead of 4e-6 in relative
-    L2); False keeps the stock call.  Parameters, state dict and initialisation are those of the nn.Conv3d either way."""
+    is a plain nn.Conv3d of bfloat16 tensors with input channels a multiple of 64, it runs as plain_conv3d, an implicit-GEMM
+    convolution of this library in both directions, instead of the vendor library's im2col + GEMM + col2im.  Other shapes
+    that the matrix-core kernels serve run on the deformable operator at all-zero offsets without modulation: the same
+    convolution (sampling points on the voxels, zero padding outside the volume).
+    `layer.branch_on_operator`: True (default) does so for bfloat16, where the two convolutions differ by less than either
+    differs from a float64 run of the layer; "all" also for float32, on the operator, where the forward kernel's two-term
+    bfloat16 operands move the predicted offsets by a few 1e-6 of their size -- enough to put one sampling point in
+    10^4 .. 10^5 on the other side of a voxel boundary, where grad_offset jumps (the layer's grad_input then agrees with a
+    float64 run to 2e-3 instead of 4e-6 in relative L2); False keeps the stock call.  Parameters, state dict and
+    initialisation are those of the nn.Conv3d either way."""
     conv = layer.deform_params
     wanted = layer.branch_on_operator
     if (wanted and (x.dtype == torch.bfloat16 or wanted == "all") and type(conv) is nn.Conv3d and x.is_cuda and x.dim() == 5
