@@ -619,15 +619,17 @@ def main():
         ws = torch.empty(max(nf, nb, 256), dtype=torch.uint8, device=dev)
 
     # The sampled columns of the forward call, kept for the backward call of the step (what the Python layer does by
-    # default where the description is served): d2c_conv3d_forward_columns / _backward_columns.
+    # default where the description is served): d2c_conv3d_forward_columns / _backward_columns, with the sorted sampling points
+    # behind them where the forward call sorts.
     kept_cols = None
     if args.columns == "on" and nd == 3 and c["backward"] and args.prepared == "off" and args.grad_weight_mode == 1 \
             and not args.backward_slices:
         zdesc = ctypes.byref(sdesc) if sized else None
-        ncol = lib.d2c_conv3d_columns_bytes(ctypes.byref(desc), zdesc)
-        if ncol:
-            kept_cols = torch.empty(ncol, dtype=torch.uint8, device=dev)
-            nb = lib.d2c_conv3d_backward_columns_workspace_bytes(ctypes.byref(desc), zdesc)
+        nkeep = lib.d2c_conv3d_keep_bytes(ctypes.byref(desc), zdesc)
+        if nkeep:
+            kept_cols = torch.empty(nkeep, dtype=torch.uint8, device=dev)
+            nf = lib.d2c_conv3d_forward_keep_workspace_bytes(ctypes.byref(desc), zdesc)
+            nb = lib.d2c_conv3d_backward_keep_workspace_bytes(ctypes.byref(desc), zdesc)
 
     prep = None
     if args.prepared != "off" and nd == 3 and not sized:
@@ -737,22 +739,26 @@ def main():
         t_b += ev[1].elapsed_time(ev[2]) / nprof
     # With the columns kept, the forward kernel also writes them (work of the backward pass moved into it): its
     # duration in a plain forward call is measured as well, so that its GEMM rate can be read both ways.
-    plain_fwd_ms = None
+    plain_fwd_ms = plain_fwd = None
     if kept_cols is not None:
+        nplain = (lib.d2c_conv3d_sized_forward_workspace_bytes(ctypes.byref(desc), ctypes.byref(sdesc)) if sized
+                  else f_fwd_ws(ctypes.byref(desc)))
+        wsp = torch.empty(max(nplain, 256), dtype=torch.uint8, device=dev)
         lib.d2c_profile_reset()
         lib.d2c_profile_enable(1)
         for _ in range(nprof):
             if sized:
                 _lib.check(lib.d2c_conv3d_sized_forward(ctypes.byref(desc), ctypes.byref(sdesc), p(x), p(size), p(m), p(w),
-                                                        p(b), p(out), p(ws), nf, cur[0]), "forward")
+                                                        p(b), p(out), p(wsp), nplain, cur[0]), "forward")
             else:
-                _lib.check(f_fwd(ctypes.byref(desc), p(x), p(off), p(m), p(w), p(b), p(out), p(ws), nf, cur[0]), "forward")
+                _lib.check(f_fwd(ctypes.byref(desc), p(x), p(off), p(m), p(w), p(b), p(out), p(wsp), nplain, cur[0]), "forward")
         torch.cuda.synchronize()
+        del wsp
         lib.d2c_profile_enable(0)
         tot, cnt = ctypes.c_double(0), ctypes.c_int(0)
         lib.d2c_profile_read(_lib.PROF_FWD, ctypes.byref(tot), ctypes.byref(cnt))
         if cnt.value:
-            plain_fwd_ms = tot.value / nprof
+            plain_fwd_ms, plain_fwd = tot.value / nprof, lib.d2c_profile_kernel_name(_lib.PROF_FWD).decode()
     lib.d2c_profile_reset()
     lib.d2c_profile_enable(1)
     for _ in range(nprof):
@@ -762,7 +768,7 @@ def main():
     fam = {"mfma": "tiled", "depthwise": "dw", "generic": "generic"}[algo]
     # per-kernel time under the name a profiler trace shows (the library reports which kernel it launched)
     ids = {_lib.PROF_FWD: "fwd", _lib.PROF_BWD_DATA: "bwd_data", _lib.PROF_BWD_WEIGHT: "bwd_weight",
-           _lib.PROF_GX_OWNER: "gx_owner", _lib.PROF_BWD_AUX: "bwd_aux", _lib.PROF_PACK: "pack"}
+           _lib.PROF_GX_OWNER: "gx_owner", _lib.PROF_BWD_AUX: "bwd_aux", _lib.PROF_SAMPLE: "sample", _lib.PROF_PACK: "pack"}
     kern, role = {}, {}
     for kid, r in ids.items():
         tot, cnt = ctypes.c_double(0), ctypes.c_int(0)
@@ -805,7 +811,7 @@ def main():
                     "frac_of_bf16_peak": round(ex / PEAK_TFLOPS["bf16"], 4),
                     "note": "float operands as sums of bfloat16 terms on v_mfma_f32_32x32x16_bf16; `peak` above is "
                             "the float32 instruction's"}
-        if plain_fwd_ms and role[dom] == "fwd":
+        if plain_fwd_ms and role[dom] == "fwd" and dom == plain_fwd:
             ach0 = f_fwd_flops / (plain_fwd_ms * 1e-3) / 1e12
             roofline["note"] = ("this launch also writes the sampled columns that the backward call of the step "
                                 "multiplies over (config.columns_kept_for_backward_mbytes); `in_a_plain_forward_call` "
@@ -831,8 +837,16 @@ def main():
     if fam == "tiled":
         rows = N * P * K * C * es
         per = {}
+        # kernels over sorted points: entries of 20 bytes (points inside the volume), input rows, and rows of those points
+        # read, 16 bytes of sums per point and 256 channels written, float32 sums of the 16 voxels per plane of a brick
+        # added for each 9 of grad_input; or columns of all points written
+        inside = N * P * K * G * (1.0 - taps["dead"]) if taps else 0.0
         for kname, r in role.items():
-            if r == "bwd_aux":
+            if kname == "brick_grad_kernel":
+                per[kname] = inside * (20 + C // G * es + 16 * -(-C // (256 * G))) + N * P * C * (es + 4 * 16 / 9)
+            elif kname == "brick_sample_kernel":
+                per[kname] = inside * 20 + N * P * C * es + rows
+            elif r == "bwd_aux":
                 # (the sampled columns it writes -- unless the forward call kept them)
                 cols = rows if (dt == "bf16" and nd == 3 and args.grad_weight_mode >= 1 and (C // groups) % 128 == 0
                                 and kept_cols is None) else 0

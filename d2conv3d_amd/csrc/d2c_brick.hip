@@ -117,7 +117,7 @@ brick_count_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, int
 // Few points: one global addition each.  (62 000 points: 5 us, the table 17 us; 700 000: 27 and 20 us.)
 template <bool AUX16, bool SIZED>
 __global__ void __launch_bounds__(256)
-brick_count_few_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, int ngrp)
+brick_count_few_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off)
 {
     const int u = blockIdx.x, npb = (s.P + 255) / 256, bgk = u / npb, bg = bgk / s.K, k = bgk - bg * s.K, b = bg / s.G, g = bg - b * s.G;
     const int p = (u - bgk * npb) * 256 + threadIdx.x;
@@ -899,7 +899,7 @@ int d2c_brick_sort(const TiledShape &s, const void *off, const void *mask, void 
         constexpr bool A16 = decltype(A)::value, SZ = decltype(Z)::value;
         if (brick_points(s) <= kFewPoints)
             hipLaunchKernelGGL((brick_count_few_kernel<A16, SZ>), dim3((unsigned)((long)((s.P + 255) / 256) * s.K * s.N * s.G)), blk, 0, st, s, d, L,
-                               off, ngrp);
+                               off);
         else hipLaunchKernelGGL((brick_count_kernel<A16, SZ>), grid, blk, 0, st, s, d, L, off, ngrp);
         hipLaunchKernelGGL(brick_range_kernel, dim3((nseg + 255) / 256), blk, 0, st, L, nseg);
         hipLaunchKernelGGL((brick_file_kernel<A16, SZ>), grid, blk, 0, st, s, d, L, off, mask, ngrp, brick_points(s));
@@ -927,8 +927,7 @@ int d2c_brick_grad(const TiledShape &s, const void *xcl, const void *gcol, const
     a.G = s.G; a.cpc = s.cpg / 64; a.Cin = s.Cin; a.D = s.D; a.H = s.H; a.W = s.W; a.vol = s.vol;
     a.chunk_rows = (long)s.K * s.M;
     if (gxcl) {
-        // (what grad_input costs beside the kernel it shares with the offset / mask gradient)
-        D2cProfScope prof(D2C_PROF_GX_OWNER, st, "brick_grad_kernel");
+        D2cProfScope prof(D2C_PROF_PACK, st);
         d2c_fill_zero(gxcl, (size_t)s.N * s.vol * s.Cin * sizeof(float), st);
     }
     a.nset = brick_sets(s);
@@ -978,7 +977,7 @@ int d2c_brick_columns(const TiledShape &s, const void *xcl, void *col, int rows,
     a.nzr = (a.d.nz + a.zlen - 1) / a.zlen;
     a.npoint = brick_points(s);
     a.nzero = (int)std::min<long>(2048, (a.npoint + 511) / 512) / nw + 1;
-    D2cProfScope prof(D2C_PROF_BWD_AUX, st, "brick_sample_kernel");
+    D2cProfScope prof(D2C_PROF_SAMPLE, st, "brick_sample_kernel");
     hipLaunchKernelGGL(brick_sample_kernel, dim3((unsigned)(cols * a.nzr + a.nzero)), dim3(64 * nw), 0, st, a, a.L.start, a.L.count);
     return d2c_check_launch("brick_sample_kernel");
 }

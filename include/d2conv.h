@@ -353,8 +353,9 @@ enum {
     D2C_PROF_BWD_WEIGHT = 2,  /* grad_weight kernel */
     D2C_PROF_PACK = 3,        /* layout changes, clears, conversions, sample lists (sum) */
     D2C_PROF_GX_OWNER = 4,    /* grad_input accumulation from the sample lists */
-    D2C_PROF_BWD_AUX = 5,     /* grad_offset / grad_mask from the grad-column rows */
-    D2C_PROF_COUNT = 6
+    D2C_PROF_BWD_AUX = 5,     /* grad_offset / grad_mask from the grad-column rows (brick_grad_kernel: and grad_input) */
+    D2C_PROF_SAMPLE = 6,      /* sampled columns from sorted points, in either direction */
+    D2C_PROF_COUNT = 7
 };
 void d2c_profile_enable(int on);
 void d2c_profile_reset(void);
