@@ -114,7 +114,10 @@ brick_count_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, int
         if (p < s.P && k0 + i < s.K)
             L.place[((long)bg * s.K + k0 + i) * s.P + p] = pt[i] == ~0u ? -1 : s_cnt[pt[i] >> 16] + (int)(pt[i] & 0xffffu);
 }
-// Few points: one global addition each.  (62 000 points: 5 us, the table 17 us; 700 000: 27 and 20 us.)
+// Few points, or few to a block: one global addition each, which costs by the additions that meet at one count.  The two
+// kernels in us, this one first: 7 taps (63 points to a block) 12 and 17 at 90 000 points, 13 and 18 at 242 000, 20 and
+// 20 at 484 000; 27 taps (243 to a block) 12 and 15 at 22 000, 18 and 19 at 44 000, 24 and 22 at 87 000, 34 and 27 at
+// 350 000, 55 and 27 at 700 000 in two groups.
 template <bool AUX16, bool SIZED>
 __global__ void __launch_bounds__(256)
 brick_count_few_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off)
@@ -127,7 +130,6 @@ brick_count_few_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off)
     const BrickPoint q = brick_point<AUX16, SIZED>(s, d, c, b, g, k, p);
     L.place[((long)bg * s.K + k) * s.P + p] = q.in ? atomicAdd(&L.count[q.seg], 1) : -1;
 }
-constexpr long kFewPoints = 400000;
 // (the order of the ranges does not matter: a wavefront adds up its 64 counts and takes one range for all)
 __global__ void __launch_bounds__(256) brick_range_kernel(BrickLists L, int nseg)
 {
@@ -851,6 +853,7 @@ long brick_nseg(const TiledShape &s)
     return (long)s.N * s.G * d.nz * d.nby * d.nbx;
 }
 long brick_points(const TiledShape &s) { return (long)s.N * s.G * s.K * s.P; }
+double brick_mean(const TiledShape &s) { return 9.0 * s.K * s.P / s.vol; }      // points per block, were all inside
 int brick_sets(const TiledShape &s) { return (s.cpg / 64 + kMaxWaves - 1) / kMaxWaves; }
 BrickLists brick_lists(const TiledShape &s, char *base)
 {
@@ -866,8 +869,7 @@ BrickLists brick_lists(const TiledShape &s, char *base)
 bool d2c_brick_supported(const TiledShape &s, int dtype)
 {
     if (s.nd != 3 || dtype != D2C_BF16 || s.cpg % 64) return false;
-    const double mean = 9.0 * s.K * s.P / s.vol;
-    return mean >= 16.0 && s.K <= 65535 && (long)s.N * s.G <= 65535 && brick_nseg(s) < (1L << 31) - 1024 &&
+    return brick_mean(s) >= 16.0 && s.K <= 65535 && (long)s.N * s.G <= 65535 && brick_nseg(s) < (1L << 31) - 1024 &&
            brick_points(s) < (1L << 31) - 64 && (size_t)s.K * (s.M + 64) * 128 < 0xFFFFFF00u &&
            (size_t)s.H * s.W * s.Cin * 4 < 0xFFFFFFF0u;
 }
@@ -897,7 +899,7 @@ int d2c_brick_sort(const TiledShape &s, const void *off, const void *mask, void 
     const dim3 grid((unsigned)((long)((s.P + 255) / 256) * ngrp * s.N * s.G)), blk(256);
     auto go = [&](auto A, auto Z) {
         constexpr bool A16 = decltype(A)::value, SZ = decltype(Z)::value;
-        if (brick_points(s) <= kFewPoints)
+        if (brick_points(s) <= (brick_mean(s) < 128.0 ? 300000 : 64000))
             hipLaunchKernelGGL((brick_count_few_kernel<A16, SZ>), dim3((unsigned)((long)((s.P + 255) / 256) * s.K * s.N * s.G)), blk, 0, st, s, d, L,
                                off);
         else hipLaunchKernelGGL((brick_count_kernel<A16, SZ>), grid, blk, 0, st, s, d, L, off, ngrp);
