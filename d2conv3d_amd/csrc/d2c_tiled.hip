@@ -406,15 +406,16 @@ FwdWs fwd_ws(const d2c_conv3d_desc &q, const TiledShape &s)
     if (d2c_fwd_split(s) > 1)
         w.least += d2c_align_up((size_t)((s.M + 63) / 64 * 64) * s.ogp * s.groups * sizeof(float));
     w.total = w.least;
-    if (use_brick_forward(q, s, true)) {
+    const bool plain = use_brick_forward(q, s, false), keep = use_brick_forward(q, s, true);
+    if (plain || keep) {
         // (a call that keeps its columns holds them, and the sorted points, in the caller's buffer)
         w.gemm = w.wp;
         w.lists = w.gemm + d2c_align_up(d2c_col_forward_ws(q));
         w.col = w.lists + d2c_brick_ws(s).total;
         w.end = w.col + brick_col_bytes(s);
-        if (use_brick_forward(q, s, false)) w.total = std::max(w.total, w.end);
+        if (plain) w.total = std::max(w.total, w.end);
         // (where the gathering kernel writes no columns, every forward workspace has to do for a call that keeps them)
-        if (!d2c_fwd_writes_columns(s, q.dtype)) w.total = std::max(w.total, w.lists);
+        if (keep && !d2c_fwd_writes_columns(s, q.dtype)) w.total = std::max(w.total, w.lists);
     }
     return w;
 }
@@ -594,15 +595,23 @@ bool use_brick(const d2c_conv3d_desc &q, const TiledShape &s)
     return d2c_gx_mode() == 1 && use_lists(q, s) && use_aux_kernel(q, s) && d2c_brick_supported(s, q.dtype);
 }
 
-// The forward pass over sampled columns: sort, sample, multiply.  `kept`: the caller keeps the columns and the backward
-// call takes the sorted points over.  Picoseconds per point and chunk of 64 channels, C columns: sort 60 / chunks of a
+// The forward pass over sampled columns: sort, sample, multiply.  `kept`: the caller keeps the columns, where the backward call can
+// multiply over them, and that one takes the sorted points over.  Picoseconds per point and chunk of 64 channels, C columns: sort 60 / chunks of a
 // group, sampling 33, product 0.13 C; the gathering kernel 55 + 0.15 C (192 - 512 columns).  So with the sort paid for by
-// the backward pass the columns win throughout, without it from four chunks on (256 -> 192 channels on 5x72x100: 360 and
-// 356 us, 2048 -> 512 with its branch: 2.8 and 4.2 ms).  Below some 12 000 positions the fixed times of the six launches
-// take the difference.
+// the backward pass the columns win throughout, without it from four chunks on.
+// Small problems, where launches and half-filled rounds of tiles count, in us, gathering first (27 taps but for the last; the line lies
+// where the columns stop losing):
+//   training step:  128 -> 128: 405 positions 133, 140; 810 151, 145; 1296 176, 152; 5760 308, 190   128 -> 40: 810 132, 141; 1296 149, 138
+//                   256 -> 64: 405 143, 144; 810 168, 153    256 -> 256: 5760 338, 288    1024 -> 256: 810 308, 288; 5760 772, 674
+//   forward alone:  256 -> 256: 4320 91, 99; 7072 114, 119; 8512 151, 132; 11968 171, 158
+//                   512 -> 512: 4320 169, 156; 8512 300, 236    1024 -> 256: 3240 160, 175; 5760 270, 262
+//                   1024 -> 128: 4320 690, 164; 11968 471, 365   2048 -> 256, 7 taps: 3240 102, 116; 5808 168, 153
 bool use_brick_forward(const d2c_conv3d_desc &q, const TiledShape &s, bool kept)
 {
-    return use_brick(q, s) && s.groups == 1 && s.M >= 12288 && brick_col_bytes(s) < (4ull << 30) && (kept || s.cpg / 64 >= 4);
+    const long chunks = s.Cin / 64, of_group = s.cpg / 64;
+    const bool large = kept ? s.M >= 400 && s.M * chunks >= 2048 : of_group >= 4 && s.M >= 4096 && s.M * of_group >= 32768;
+    return large && use_brick(q, s) && s.groups == 1 && brick_col_bytes(s) < (4ull << 30) &&
+           (!kept || d2c_bwd_weight_from_kept_col(s, q.dtype));
 }
 
 // grad_weight as a matrix product over sampled columns that the offset / mask gradient kernel writes on its way
@@ -1048,9 +1057,7 @@ size_t d2c_tiled_columns_bytes(const d2c_conv3d_desc &q, const d2c_size_map_desc
     if (sz && !d2c_tiled_sized_supported(q, true)) return 0;
     const TiledShape s = tiled_shape(q, 3, 0, sz);
     // (where only the sorted points give columns, they are kept with them)
-    if (use_brick_forward(q, s, true))
-        return !d2c_bwd_weight_from_kept_col(s, q.dtype) || !use_aux_kernel(q, s) ? 0
-               : d2c_fwd_writes_columns(s, q.dtype) ? brick_col_bytes(s) : brick_keep_bytes(s);
+    if (use_brick_forward(q, s, true)) return d2c_fwd_writes_columns(s, q.dtype) ? brick_col_bytes(s) : brick_keep_bytes(s);
     if (!d2c_fwd_writes_columns(s, q.dtype) || !d2c_bwd_weight_from_kept_col(s, q.dtype) || !use_aux_kernel(q, s)) return 0;
     const long rows = d2c_columns_rows(s), chunks = s.Cin / bkc_of(q.dtype);
     if (chunks * s.K * rows >= (1L << 31)) return 0;      // (the kernel counts rows in 32 bits)

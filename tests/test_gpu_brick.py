@@ -21,6 +21,11 @@ CASES = {
     "nine_chunks_three_groups_dilated": (1, 576, 33, (2, 6, 8), (3, 3, 3), 1, 2, 3, True),
     "kept_columns_ragged": (1, 128, 72, (13, 31, 31), (3, 3, 3), 1, 1, 2, True),
     "columns_forward_ragged": (1, 256, 16, (1, 95, 131), (3, 3, 3), 1, 1, 1, True),
+    # the smallest problems that sample columns: kept for the backward pass, in a forward call alone
+    "kept_columns_two_chunks": (1, 128, 24, (2, 16, 33), (3, 3, 3), 1, 1, 1, True),
+    "kept_columns_few_positions": (1, 512, 72, (1, 19, 22), (3, 3, 3), 1, 1, 2, True),
+    "columns_forward_smallest": (1, 256, 130, (8, 32, 32), (3, 3, 3), 1, 1, 1, True),
+    "columns_forward_many_chunks": (1, 576, 40, (1, 63, 66), (1, 7, 1), 1, 1, 1, False),
 }
 
 
