@@ -621,6 +621,27 @@ __global__ void __launch_bounds__(kThreadsDw) dwc_march_bwd_kernel(d2c_dwconv3d_
         cur = nxt;
     }
     if (!part) return;
+    // Pairs with a position outside the volume, or an input of another range, were zero times something, which is no number
+    // where the something is infinite or none: then pair by pair.
+    float all = 0.f;
+#pragma unroll
+    for (int k = 0; k < 27; k++) all += gw[k];
+    if (__builtin_expect(!(fabsf(all) < __builtin_inff()), 0)) {
+#pragma unroll
+        for (int k = 0; k < 27; k++) gw[k] = 0.f;
+#pragma unroll 1
+        for (int e = 0; e < (p.z_hi - p.z_lo) * kMR * kVW; e++) {
+            const int z = p.z_lo + e / (kMR * kVW), y = p.y0 + e / kVW % kMR, xx = p.x0 + e % kVW;
+            if (y >= q.H || xx >= q.W) continue;
+            const float v = ldv<ST>(xc, z * HW + (long)y * q.W + xx);
+#pragma unroll
+            for (int k = 0; k < 27; k++) {
+                const int gz = z + 1 - k / 9, gy = y + 1 - k / 3 % 3, gxx = xx + 1 - k % 3;
+                if (gz >= 0 && gz < q.D && gy >= 0 && gy < q.H && gxx >= 0 && gxx < q.W)
+                    gw[k] = fmaf(v, ldv<ST>(gc, gz * HW + (long)gy * q.W + gxx), gw[k]);
+            }
+        }
+    }
     __shared__ float s_red[kThreadsDw / 64][kMTaps];
 #pragma unroll
     for (int k = 0; k < kMTaps; k++) {

@@ -32,3 +32,27 @@ def test_march_kernels_at_tile_edges(n, c, dims, dtype, dev):
         one = [t.to(dev).requires_grad_(j == i) for j, t in enumerate((x, w, b))]
         depthwise_separable_conv3d(*one, 1, 1, 1).backward(gout.to(dev))
         assert torch.equal(one[i].grad, ts[i].grad)
+
+
+@pytest.mark.parametrize("what", ["x", "grad_out"])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_a_bad_value_at_the_border_reaches_the_taps_that_meet_it(what, bad, dev):
+    """grad_weight: the taps that pair the corner voxel, or the position at the corner, with something inside the volume (eight
+    of 27), or a voxel in the first plane of another range of planes (all of them)."""
+    g = torch.Generator().manual_seed(8)
+    x, gout = (torch.randn(1, 3, 17, 33, 68, generator=g) for _ in range(2))
+    t = x if what == "x" else gout
+    t[0, 0, 0, 0, 0] = t[0, 2, 8, 5, 6] = bad
+    w = torch.randn(3, 1, 3, 3, 3, generator=g)
+    ts = [v.to(dev).requires_grad_(True) for v in (x, w)]
+    depthwise_separable_conv3d(*ts, None, 1, 1, 1).backward(gout.to(dev))
+    got = ts[1].grad.cpu()
+    # (w[k] meets x[p + k - 1] and grad_out[p]: pairs with the corner need k >= 1 on every axis for a position, k <= 1 for a voxel)
+    met = torch.zeros(3, 3, 3, dtype=torch.bool)
+    met[(slice(0, 2),) * 3 if what == "x" else (slice(1, 3),) * 3] = True
+    assert torch.equal(~got[0, 0].isfinite(), met)
+    assert got[1].isfinite().all() and not got[2].isfinite().any()
+    z = lambda v: torch.nan_to_num(v, 0.0, 0.0, 0.0)
+    wr = w.double().requires_grad_(True)
+    F.conv3d(z(x).double(), wr, padding=1, groups=3).backward(z(gout).double())
+    assert rel_l2(got[0, 0][~met].double(), wr.grad[0, 0][~met]) < 1e-5 and rel_l2(got[1].double(), wr.grad[1]) < 1e-5
