@@ -358,7 +358,7 @@ def bench_layer(args):
                    "deformation": "read by the operator inside the branch's output tensor, sigmoid in the sampler",
                    "split_and_sigmoid_in_front_ms_per_step": round(res[False], 4),
                    "relative_l2_fused_vs_split": err,
-                   "branch": "the layer's Conv3d 512 -> 864 evaluated by the operator at zero offsets",
+                   "branch": "the layer's Conv3d 512 -> 864 as an implicit-GEMM convolution of the library (d2c_plain_conv3d_*)",
                    "branch_on_the_vendor_library_ms_per_step": round(stock_branch_ms, 4),
                    "relative_l2_branch_on_operator_vs_vendor": err_branch,
                    "algorithmic_gflop": round(3 * (f_op + f_branch) / 1e9, 2)},
@@ -493,7 +493,7 @@ def bench_dwconv(args):
                    "forward_ms": round(ms_f, 4), "backward_ms": round(ms_b, 4),
                    "torch_grouped_conv_ms_per_step": round(ms_torch, 4), "max_error_vs_torch": err,
                    "algorithmic_mbytes": round(nbytes / 1e6, 1)},
-        "roofline": {"bound": "hbm", "kernel": "dwc_fwd_kernel + dwc_bwd_input_kernel + dwc_bwd_weight_kernel",
+        "roofline": {"bound": "hbm", "kernel": "dwc_march_fwd_kernel + dwc_march_bwd_kernel",
                      "achieved": round(gbs, 1), "peak": PEAK_GBS, "unit": "GB/s", "frac": round(gbs / PEAK_GBS, 4),
                      "traffic": None},
     }

@@ -11,7 +11,8 @@
 // Three quarters of the products are with zeros, on matrix cores that have them to spare; in exchange nothing is
 // gathered: a grad-column row is read once, for both results, and a brick's input rows stay in LDS.  (The kernels
 // that gather -- eight corner rows per point through the L1, grad-column rows 3.4 times -- took 1.73 + 1.47 ms for
-// 256 channels on 32x60x108, bound by the L1 path, the vector ALU and row latency.)
+// 256 channels on 32x60x108, bound by the L1 path, the vector ALU and row latency; this one takes 0.87, at 2.4 TB/s to and
+// from device memory, and 0.22 for 512 channels in 8 groups on 2x8x30x54, where they took 0.50 + 0.35.)
 
 #include "d2c_mma.hpp"
 #include "d2c_tiled.hpp"
@@ -52,7 +53,7 @@ D2C_DEV BrickPoint brick_point(const TiledShape &s, const BrickDims &d, float *c
 // A workgroup works on 256 positions and up to kTaps taps, and requests what it reads of all of them first.  Points of
 // neighbouring positions fall into few blocks: they are counted in a hash table in LDS, and each block's number goes to
 // the global count in one addition.  (One global atomic per point, taps in workgroups of their own: 0.24 ms for 5.6 M
-// points in 8 offset groups on 8x30x54.)
+// points in 8 offset groups on 8x30x54; this way 0.13, and 0.14 to file them.)
 // Workgroups of the passes over all points: an XCD takes a contiguous part of the positions, the tap groups of a block
 // of 256 one after the other, so that the lines which several workgroups write or read in parts meet in one L2.
 constexpr int kTaps = 9, kSlots = 4096;             // (more slots than a workgroup has points: a probe always ends)
@@ -574,7 +575,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
 // points], three bfloat16 terms of the weights.  W is made by the lanes that hold the points, in the operand's own order
 // (lane = point, half h of the wavefront: the voxels of rows y = 2h, 2h + 1 of each plane); the brick's input is kept as
 // the other operand, one plane changed per step in z.  Rows leave whole, through LDS.  Bound by the rows it writes:
-// 5.6 M points x 256 channels (32x60x108, 27 taps), 2.9 GB: 700 us (the whole forward pass: 2.3 ms gathering, 1.7 ms sorted).
+// 5.6 M points x 256 channels (32x60x108, 27 taps), 2.9 GB: 730 us (the whole forward pass: 2.3 ms gathering, 1.7 ms sorted).
 // (Workgroups as in brick_grad_kernel: a column of bricks, a wavefront per chunk.)
 struct BrickSampleArgs {
     BrickDims d;

@@ -197,15 +197,15 @@ int d2c_conv3d_backward(const d2c_conv3d_desc *desc, const void *grad_out, const
  * memory to spare hands d2c_conv3d_forward_columns a buffer of d2c_conv3d_columns_bytes() bytes (256-byte aligned;
  * taps x the size of the input, in the element type): the forward kernel writes there what it multiplies with the
  * weights anyway, and d2c_conv3d_backward_columns, given that buffer UNCHANGED together with the same tensors, runs
- * its grad-weight product over it instead of sampling again (N=2, C=512, 8x30x54, bfloat16: 2.46 -> 2.39 ms per step
- * for 717 MB held between the two calls, and 0.72 GB less backward workspace; N=2, C=256, 8x30x54, float32: 2.77 ->
- * 2.25 ms for 717 MB).  Results are those of the plain calls up to the order of floating-point sums; float32
+ * its grad-weight product over it instead of sampling again (N=2, C=512, 8x30x54, bfloat16: 2.33 -> 1.95 ms per step
+ * for 851 MB held between the two calls -- 717 of columns, the rest sorted sampling points, see d2c_conv3d_keep_bytes() -- and
+ * 0.85 GB less backward workspace; N=2, C=256, 8x30x54, float32: 2.29 -> 2.13 ms for 717 MB).  Results are those of the plain calls up to the order of floating-point sums; float32
  * columns are the interpolated floats themselves and their product keeps float32's accuracy (three bfloat16 terms
  * per float on the bfloat16 matrix instruction, or the float32 instruction), whatever D2C_BWD_F32_SPLIT says.  `size_map` as in d2c_conv3d_forward_stats: NULL, or the description of
  * the size map that `offset` then is.  d2c_conv3d_columns_bytes() is 0 where this is not served (anything but
- * bfloat16 and float32 problems on the matrix-core kernels with at least 48 tiles of 64 output positions (times
- * weight groups), offsets along all three axes and an even number of 64- / 32-channel chunks per weight group); the
- * two calls then
+ * bfloat16 and float32 problems on the matrix-core kernels with an even number of 64- / 32-channel chunks per weight
+ * group and at least 48 tiles of 64 output positions (times weight groups) and offsets along all three axes, or, bfloat16 with
+ * one weight group, at least 400 positions and 2048 positions times chunks); the two calls then
  * fail with D2C_ERR_UNSUPPORTED and the caller uses the plain ones.  The memory-saving bits of
  * d2c_conv3d_desc::backward_flags are ignored by d2c_conv3d_backward_columns.
  */
@@ -242,8 +242,9 @@ int d2c_conv3d_backward_columns(const d2c_conv3d_desc *desc, const struct d2c_si
  *   D2C_REUSE_FORWARD_WEIGHTS   ... the forward operand of THIS weight tensor: forward calls while the weights
  *                               do not change (inference);
  *   D2C_REUSE_BACKWARD_WEIGHTS  ... the backward operand of this weight tensor (made by a backward call).
- * Parts not named are made by the call (and may be named in the next one).  Results are those of the plain calls
- * (the same kernels on the same operands).  d2c_conv3d_prepared_bytes() is 0 for descriptions the other kernel families serve; the calls
+ * Parts not named are made by the call (and may be named in the next one).  Results are those of the plain calls.  The
+ * forward call runs on the gathering kernels, also where d2c_conv3d_forward samples columns first, which is faster and
+ * differs by the rounding of its sums.  d2c_conv3d_prepared_bytes() is 0 for descriptions the other kernel families serve; the calls
  * then ignore `prepared` and `reuse`.  The workspace is needed as before.
  */
 #define D2C_REUSE_INPUT            1
@@ -483,7 +484,7 @@ void d2c_set_grad_input_mode(int mode);
 /* Test hooks, not for production callers (those set d2c_conv3d_desc::backward_flags, which wins over the hooks
  * wherever it says something): the grad-weight path of the matrix-core backward pass for
  * descriptions whose backward_flags leave it at the default -- 1 (the library's default) lets the offset / mask
- * gradient kernel write the sampled columns, over which grad_weight then runs as a plain matrix product (the
+ * gradient kernel (bfloat16, sorted points: the sampling kernel) write the sampled columns, over which grad_weight then runs as a plain matrix product (the
  * reference's formulation, dconv3d_gpu.cu:1037-1088, with the column buffer filled by the kernel that has the
  * corner values in registers anyway); 2 is the same with the columns written over the grad-column rows (no buffer
  * of their own; grad_input is then taken from the rows first, from sample lists that a pass of their own files,
