@@ -336,8 +336,8 @@ def bench_layer(args):
         res[fused] = timed()
         outs[fused] = layer(x).detach().float()
     err = float((outs[True] - outs[False]).norm() / outs[False].norm())
-    # ... and with the branch's convolution on the vendor library (what the reference runs) instead of on the operator
-    # at zero offsets (modules._branch_conv, the default)
+    # ... and with the branch's convolution on the vendor library (what the reference runs) instead of on this library's
+    # (modules._branch_conv, the default)
     layer.branch_on_operator = False
     stock_branch_ms = timed()
     stock_out = layer(x).detach().float()

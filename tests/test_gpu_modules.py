@@ -161,8 +161,8 @@ def test_tap_statistics_match_the_oracle(dev):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("cls", ["MDConv3d", "DConv3d", "XYZSizeConditionedMDConv3d"])
 def test_branch_convolution_on_the_operator(cls, dtype, dev):
-    """The deformation branch's nn.Conv3d evaluated by the operator at zero offsets (modules._branch_conv: the default
-    for bfloat16, "all" for float32 too) against the stock call, both held to a float64 run of the same layer (direct
+    """The deformation branch's nn.Conv3d evaluated by this library (modules._branch_conv: plain_conv3d for bfloat16, the
+    default; "all" for float32 too, on the operator at zero offsets) against the stock call, both held to a float64 run of the same layer (direct
     kernels): in bfloat16 the operator's branch is no further from it than the stock one (both carry the 5 - 10 % that
     bfloat16 offsets leave in the gradients that pass through them); in float32 the output agrees to 1e-4 and the
     gradients through the offsets to 1e-2 (sampling points that change their voxel, see _branch_conv)."""
