@@ -724,7 +724,8 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 4) brick_sample_kernel(BrickSa
                                pack_bf16x2(v[r + 6], v[r + 7]));
             }, std::make_integer_sequence<int, 4>{});
             if (__builtin_expect(bad_l || bad_h, 0)) {
-                // point by point (lane = channel), over what the products have left in LDS
+                // point by point (lane = channel), over what the products have left in LDS (stores of another type: kept behind those)
+                wave_fence();
                 for (int j = 0; j < min(cnt - i0, 32); j++) {
                     const PointValues p = point_of_lane(e0, a0, j, y0, x0);
                     float v = 0.f;
