@@ -800,7 +800,7 @@ def main():
         # into two or three bfloat16 terms, so `frac` (against the float32 instruction's peak) can pass 1; the
         # instructions executed are the partial products
         if dt == "f32":
-            terms = {"tiled_fwd_dma_kernel": 4, "tiled_fwd_kernel": 4, "tiled_bwd_weight_col3_kernel": 6,
+            terms = {"tiled_fwd_dma_kernel": 4, "tiled_fwd_wave_kernel": 4, "tiled_bwd_weight_col3_kernel": 6,
                      "tiled_bwd_col_kernel": 4, "tiled_bwd_col32f_kernel": 3}
             if args.f32_split_backward:
                 terms.update({"tiled_bwd_weight_dma_kernel": 4, "tiled_bwd_data_kernel": 4})

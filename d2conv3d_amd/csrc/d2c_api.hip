@@ -596,7 +596,7 @@ size_t d2c_conv3d_forward_least_workspace_bytes(const d2c_conv3d_desc *q, const 
 {
     if ((z ? sized_check(q, z) : d2c_conv3d_check(q)) != D2C_OK) return 0;
     const int a = choose_algo(*q, true);
-    const size_t least = a == D2C_ALGO_MFMA || a == D2C_ALGO_DEPTHWISE ? d2c_tiled_forward_ws(*q, D2C_FWD_WS_LEAST) : 0;
+    const size_t least = a == D2C_ALGO_MFMA || a == D2C_ALGO_DEPTHWISE ? d2c_tiled_forward_ws(*q, D2C_FWD_WS_GATHER) : 0;
     return z && !sized_fused(*q, false) ? expanded_offsets_bytes(*q) + least : least;
 }
 
@@ -666,7 +666,7 @@ int d2c_conv3d_forward_stats(const d2c_conv3d_desc *q, const d2c_size_map_desc *
     if (a < 0) return D2C_ERR_UNSUPPORTED;
     // the kernels that add the sums up on their way: matrix-core family, offsets from a tensor or formed in the sampler
     if (stats_fused(*q, z)) {
-        if (int rc = check_ws(d2c_tiled_forward_ws(*q, D2C_FWD_WS_STATS), ws, ws_bytes)) return rc;
+        if (int rc = check_ws(d2c_tiled_forward_ws(*q, D2C_FWD_WS_STATS_LEAST), ws, ws_bytes)) return rc;
         return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, ws_bytes, (hipStream_t)stream, z, chan_stats);
     }
     if (int rc = z ? d2c_conv3d_sized_forward(q, z, x, offset, mask, weight, bias, out, ws, ws_bytes, stream)

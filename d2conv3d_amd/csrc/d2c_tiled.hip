@@ -19,7 +19,9 @@ bool d2c_fwd_writes_columns(const TiledShape &s, int dtype);
 long d2c_columns_rows(const TiledShape &s);
 bool d2c_fwd_fills_stats(const TiledShape &s);
 size_t d2c_fwd_stats_ws(const TiledShape &s);
-int d2c_fwd_split(const TiledShape &s);
+bool d2c_fwd_use_dma(const TiledShape &s);
+size_t d2c_fwd_split_count_bytes(const TiledShape &s);
+size_t d2c_fwd_split_bytes(const TiledShape &s);
 
 bool d2c_tiled_bwd_data_supported(const TiledShape &s, int dtype);
 bool d2c_tiled_bwd_weight_supported(const TiledShape &s, int dtype);
@@ -207,75 +209,16 @@ __global__ void __launch_bounds__(256) pack_input_bf16_kernel(const bf16_t *x, b
     pack_tile64_bf16(x + bo, xcl + bo, C, vol, blockIdx.x * 64, blockIdx.y * 64);
 }
 
-// Everything a depthwise call needs before its main kernels, as one launch: up to two tensors to channels-last (the
-// input, grad_out), the weights W[c][0][k] -> wt[k][c], a range of the workspace cleared, the bias gradient.  A
-// workgroup finds its job from its index; jobs a call does not need have no workgroups.
-struct DwPrepArgs {
-    struct Pack {
-        const void *src;
-        void *dst;
-        int C, vol, wide;     // wide: 64 x 64 bfloat16 tiles (see pack_tile64_bf16)
-        int nbx, nby, nblk;   // tiles along vol and C; workgroups of the job (tiles x batch)
-    } pack[2];
-    const void *w;
-    void *wt;
-    int wC, wK, nblk_w;
-    void *zrow;                // the row of zeros behind the channels-last input (wC elements)
-    uint32_t *zero;
-    size_t zero_words;
-    int nblk_z;
-    const void *gout;          // bias gradient: one workgroup per channel
-    void *gb;
-    int bN, bC, bP, nblk_b;
-};
-template <typename T> __global__ void __launch_bounds__(256) dw_prepare_kernel(DwPrepArgs a)
-{
-    int b = blockIdx.x;
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const DwPrepArgs::Pack &pk = a.pack[j];
-        if (b < pk.nblk) {
-            const int bx = b % pk.nbx, by = (b / pk.nbx) % pk.nby;
-            const long bo = (long)(b / (pk.nbx * pk.nby)) * pk.C * pk.vol;
-            if constexpr (sizeof(T) == 2) {
-                if (pk.wide) {
-                    pack_tile64_bf16((const bf16_t *)pk.src + bo, (bf16_t *)pk.dst + bo, pk.C, pk.vol, bx * 64, by * 64);
-                    return;
-                }
-            }
-            pack_tile32<T>((const T *)pk.src + bo, (T *)pk.dst + bo, pk.C, pk.vol, bx * 32, by * 32);
-            return;
-        }
-        b -= pk.nblk;
-    }
-    if (b < a.nblk_w) {
-        const T *w = (const T *)a.w;
-        T *wt = (T *)a.wt;
-        const int n = a.wC * a.wK;
-        for (int i = b * 256 + threadIdx.x; i < n; i += a.nblk_w * 256) wt[i] = w[(i % a.wC) * a.wK + i / a.wC];
-        if (b == 0)
-            for (int i = threadIdx.x; i < a.wC; i += 256) ((T *)a.zrow)[i] = (T)0;
-        return;
-    }
-    b -= a.nblk_w;
-    if (b < a.nblk_z) {
-        for (size_t i = (size_t)b * 256 + threadIdx.x; i < a.zero_words; i += (size_t)a.nblk_z * 256) a.zero[i] = 0u;
-        return;
-    }
-    b -= a.nblk_z;
-    if (b < a.nblk_b) bias_grad_body<T, 256>((const T *)a.gout, (T *)a.gb, a.bN, a.bC, a.bP, b);
-}
-
 // Forward weight operand in MFMA fragment order:
 //   wp[wg][step = chunk*K + k][o-block of 32][k-group][lane] = 16 bytes =
 //   W[wg*og + ob*32 + lane%32][chunk*BKC + (2*kg + lane/32)*VEC + 0..VEC-1][k]
 // (rows past og are zero), so a wavefront's fragment load is 1 KiB contiguous.
-template <typename T>
-__global__ void __launch_bounds__(256) pack_weight_fwd_kernel(const T *w, T *wp, TiledShape s, long total)
+template <typename T> D2C_DEV void pack_weight_fwd(const T *w, T *wp, const TiledShape &s, int b, int nb)
 {
     constexpr int VEC = Elem<T>::VEC, BKC = 8 * VEC;
     const int OBT = s.ogp / 32, S = s.nchunk * s.K;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (long)gridDim.x * blockDim.x) {
+    const long total = (long)s.groups * S * OBT * 4 * 64;
+    for (long i = (long)b * 256 + threadIdx.x; i < total; i += (long)nb * 256) {
         const int lane = (int)(i & 63);
         const int kg = (int)((i >> 6) & 3);
         long r = i >> 8;
@@ -297,13 +240,10 @@ __global__ void __launch_bounds__(256) pack_weight_fwd_kernel(const T *w, T *wp,
 // weights are runs of BKC * K consecutive elements in W, reads them with 16-byte loads and writes whole
 // 16-byte fragment vectors (kPackRows consecutive lanes each).  Needs a 16-byte aligned W and rows that fit LDS.
 constexpr int kPackRows = 8;
-template <typename T>
-__global__ void __launch_bounds__(256) pack_weight_fwd_lds_kernel(const T *w, T *wp, TiledShape s)
+template <typename T> D2C_DEV void pack_weight_fwd_lds(const T *w, T *wp, const TiledShape &s, int b, unsigned char *smem)
 {
     constexpr int VEC = Elem<T>::VEC, BKC = 8 * VEC, R = kPackRows;
-    extern __shared__ __align__(16) unsigned char smem[];
     const int OBT = s.ogp / 32, S = s.nchunk * s.K;
-    int b = blockIdx.x;
     const int part = b % (32 / R); b /= 32 / R;
     const int obg = b % OBT; b /= OBT;
     const int j = b % s.nchunk;
@@ -334,6 +274,74 @@ __global__ void __launch_bounds__(256) pack_weight_fwd_lds_kernel(const T *w, T 
         const long vi = ((((long)wg * S + j * s.K + k) * OBT + obg) * 4 + (khi >> 1)) * 64 + lane;
         *reinterpret_cast<uint4 *>(wp + vi * VEC) = operand_vec<T, kF32SplitFwd>(tmp);
     }
+}
+
+// What a call needs before its main kernels, as one launch: up to two tensors to channels-last (the input, grad_out) with
+// zeros behind the first, the weights in the order of the kernels behind, a range of the workspace cleared, the bias
+// gradient.  A workgroup finds its job from its index; jobs a call does not need have no workgroups.  (Each of these as
+// a kernel of its own costs 2 - 3 us of launch and drain: 64 -> 64 channels on 4x14x25, float32, 37 us in five launches.)
+enum { PREP_W_DEPTHWISE, PREP_W_FWD, PREP_W_FWD_LDS };
+struct PrepArgs {
+    struct Pack {
+        const void *src;
+        void *dst;
+        int C, vol, wide;     // wide: 64 x 64 bfloat16 tiles (see pack_tile64_bf16)
+        int nbx, nby, nblk;   // tiles along vol and C; workgroups of the job (tiles x batch)
+    } pack[2];
+    uint32_t *zrow;            // zeros behind the channels-last input
+    int zrow_words;
+    const void *w;
+    void *wt;
+    int wkind, wC, wK, nblk_w;
+    uint32_t *zero;
+    size_t zero_words;
+    int nblk_z;
+    const void *gout;          // bias gradient: one workgroup per channel
+    void *gb;
+    int bN, bC, bP, nblk_b;
+    size_t lds;
+    TiledShape s;
+};
+template <typename T> __global__ void __launch_bounds__(256) prepare_kernel(PrepArgs a)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    int b = blockIdx.x;
+    if (b == 0 && (int)threadIdx.x < a.zrow_words)
+        for (int i = threadIdx.x; i < a.zrow_words; i += 256) a.zrow[i] = 0u;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const PrepArgs::Pack &pk = a.pack[j];
+        if (b < pk.nblk) {
+            const int bx = b % pk.nbx, by = (b / pk.nbx) % pk.nby;
+            const long bo = (long)(b / (pk.nbx * pk.nby)) * pk.C * pk.vol;
+            if constexpr (sizeof(T) == 2) {
+                if (pk.wide) {
+                    pack_tile64_bf16((const bf16_t *)pk.src + bo, (bf16_t *)pk.dst + bo, pk.C, pk.vol, bx * 64, by * 64);
+                    return;
+                }
+            }
+            pack_tile32<T>((const T *)pk.src + bo, (T *)pk.dst + bo, pk.C, pk.vol, bx * 32, by * 32);
+            return;
+        }
+        b -= pk.nblk;
+    }
+    if (b < a.nblk_w) {
+        const T *w = (const T *)a.w;
+        T *wt = (T *)a.wt;
+        if (a.wkind == PREP_W_DEPTHWISE) {
+            const int n = a.wC * a.wK;
+            for (int i = b * 256 + threadIdx.x; i < n; i += a.nblk_w * 256) wt[i] = w[(i % a.wC) * a.wK + i / a.wC];
+        } else if (a.wkind == PREP_W_FWD) pack_weight_fwd<T>(w, wt, a.s, b, a.nblk_w);
+        else pack_weight_fwd_lds<T>(w, wt, a.s, b, smem);
+        return;
+    }
+    b -= a.nblk_w;
+    if (b < a.nblk_z) {
+        for (size_t i = (size_t)b * 256 + threadIdx.x; i < a.zero_words; i += (size_t)a.nblk_z * 256) a.zero[i] = 0u;
+        return;
+    }
+    b -= a.nblk_z;
+    if (b < a.nblk_b) bias_grad_body<T, 256>((const T *)a.gout, (T *)a.gb, a.bN, a.bC, a.bP, b);
 }
 
 // Size-map source, backward: fp32 sums per axis [N][3][P] -> gradient of the raw size prediction [N][channels][P]
@@ -400,12 +408,11 @@ FwdWs fwd_ws(const d2c_conv3d_desc &q, const TiledShape &s)
     w.xcl = 0;
     w.wp = d2c_align_up((size_t)s.N * s.vol * s.Cin * es + 256);   // input, then a 256-byte row of zeros
     w.outacc = w.wp + d2c_align_up((size_t)s.groups * s.nchunk * s.K * s.ogp * bkc_of(q.dtype) * es);
-    // fp32 partial sums of the output, used only when the forward kernel splits its steps (as whole tiles of
-    // 64 positions x padded output channels in the DMA-gather kernel)
+    // fp32 partial sums of the output for the work items whose steps the DMA-gather kernel shares out: whole tiles of
+    // 64 positions x padded output channels
     w.least = w.outacc;
-    if (d2c_fwd_split(s) > 1)
-        w.least += d2c_align_up((size_t)((s.M + 63) / 64 * 64) * s.ogp * s.groups * sizeof(float));
-    w.total = w.least;
+    if (d2c_fwd_use_dma(s)) w.least += d2c_align_up((size_t)((s.M + 63) / 64 * 64) * s.ogp * s.groups * sizeof(float));
+    w.total = w.least + d2c_fwd_split_bytes(s);      // (the kernel of the small problems: fastest with its steps split)
     const bool plain = use_brick_forward(q, s, false), keep = use_brick_forward(q, s, true);
     if (plain || keep) {
         // (a call that keeps its columns holds them, and the sorted points, in the caller's buffer)
@@ -450,34 +457,57 @@ int pack_input(const TiledShape &s, const void *x, void *xcl, hipStream_t st, bo
     return d2c_check_launch("pack_input_kernel");
 }
 
-// The jobs of dw_prepare_kernel for one call (gout == nullptr: no grad_out copy; zero_bytes == 0: nothing to clear;
-// gb == nullptr: no bias gradient).
+// The jobs of prepare_kernel.
+template <typename T> void prep_pack(PrepArgs::Pack &pk, const void *src, void *dst, int N, int C, int vol)
+{
+    pk.src = src; pk.dst = dst; pk.C = C; pk.vol = vol;
+    pk.wide = sizeof(T) == 2 && vol % 8 == 0 && C % 8 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(dst) % 16 == 0;
+    const int tl = pk.wide ? 64 : 32;
+    pk.nbx = (vol + tl - 1) / tl; pk.nby = (C + tl - 1) / tl;
+    pk.nblk = pk.nbx * pk.nby * N;
+}
+void prep_zero(PrepArgs &a, void *p, size_t bytes)
+{
+    a.zero = (uint32_t *)p; a.zero_words = bytes / 4;
+    a.nblk_z = (int)std::min<size_t>((a.zero_words + 1023) / 1024, 2048);
+}
+template <typename T> void prep_weight_fwd(PrepArgs &a, const TiledShape &s, const void *w, void *wp)
+{
+    a.s = s; a.w = w; a.wt = wp;
+    const size_t lds = (size_t)kPackRows * ((size_t)s.bkc * s.K * sizeof(T) + 4);
+    if (lds <= 48 * 1024 && reinterpret_cast<uintptr_t>(w) % 16 == 0) {
+        a.wkind = PREP_W_FWD_LDS; a.lds = lds;
+        a.nblk_w = s.groups * s.nchunk * (s.ogp / 32) * (32 / kPackRows);
+    } else {
+        a.wkind = PREP_W_FWD;
+        a.nblk_w = (int)std::min<long>(((long)s.groups * s.nchunk * s.K * (s.ogp / 32) * 4 * 64 + 255) / 256, 8192);
+    }
+}
+template <typename T> int prep_launch(const PrepArgs &a, hipStream_t st)
+{
+    const long nblk = (long)a.pack[0].nblk + a.pack[1].nblk + a.nblk_w + a.nblk_z + a.nblk_b;
+    if (nblk == 0) return D2C_OK;
+    D2cProfScope prof(D2C_PROF_PACK, st);
+    hipLaunchKernelGGL(prepare_kernel<T>, dim3((unsigned)nblk), dim3(256), a.lds, st, a);
+    return d2c_check_launch("prepare_kernel");
+}
+// ... for a depthwise call (gout == nullptr: no grad_out copy; zero_bytes == 0: nothing to clear; gb == nullptr: no
+// bias gradient)
 template <typename T>
 int dw_prepare(const TiledShape &s, const void *x, void *xcl, const void *gout, void *goutcl, const void *w, void *wt,
                void *zero, size_t zero_bytes, void *gb, hipStream_t st)
 {
-    DwPrepArgs a{};
-    auto job = [&](DwPrepArgs::Pack &pk, const void *src, void *dst, int C, int vol) {
-        pk.src = src; pk.dst = dst; pk.C = C; pk.vol = vol;
-        pk.wide = sizeof(T) == 2 && vol % 8 == 0 && C % 8 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0 &&
-                  reinterpret_cast<uintptr_t>(dst) % 16 == 0;
-        const int tl = pk.wide ? 64 : 32;
-        pk.nbx = (vol + tl - 1) / tl; pk.nby = (C + tl - 1) / tl;
-        pk.nblk = pk.nbx * pk.nby * s.N;
-    };
-    job(a.pack[0], x, xcl, s.Cin, s.vol);
-    if (gout) job(a.pack[1], gout, goutcl, s.Cout, s.P);
-    a.w = w; a.wt = wt; a.wC = s.Cin; a.wK = s.K;
-    a.zrow = (T *)xcl + (size_t)s.N * s.vol * s.Cin;
+    PrepArgs a{};
+    prep_pack<T>(a.pack[0], x, xcl, s.N, s.Cin, s.vol);
+    if (gout) prep_pack<T>(a.pack[1], gout, goutcl, s.N, s.Cout, s.P);
+    a.wkind = PREP_W_DEPTHWISE; a.w = w; a.wt = wt; a.wC = s.Cin; a.wK = s.K;
     a.nblk_w = std::min((s.Cin * s.K + 255) / 256, 1024);
-    a.zero = (uint32_t *)zero; a.zero_words = zero_bytes / 4;
-    a.nblk_z = (int)std::min<size_t>((a.zero_words + 1023) / 1024, 2048);
+    a.zrow = (uint32_t *)((T *)xcl + (size_t)s.N * s.vol * s.Cin); a.zrow_words = s.Cin * (int)sizeof(T) / 4;
+    prep_zero(a, zero, zero_bytes);
     a.gout = gout; a.gb = gb; a.bN = s.N; a.bC = s.Cout; a.bP = s.P;
     a.nblk_b = (gb && gout) ? s.Cout : 0;
-    const long nblk = (long)a.pack[0].nblk + a.pack[1].nblk + a.nblk_w + a.nblk_z + a.nblk_b;
-    D2cProfScope prof(D2C_PROF_PACK, st);
-    hipLaunchKernelGGL(dw_prepare_kernel<T>, dim3((unsigned)nblk), dim3(256), 0, st, a);
-    return d2c_check_launch("dw_prepare_kernel");
+    return prep_launch<T>(a, st);
 }
 
 bool is_depthwise(const d2c_conv3d_desc &q)
@@ -531,8 +561,7 @@ int forward_t(const d2c_conv3d_desc &q, const void *x, const void *off, const vo
     const PreparedLayout pl = prepared_layout(q, s);
     char *xcl_p = prep ? (char *)prep->base + pl.xcl : base + l.xcl;
     char *wp_p = prep ? (char *)prep->base + pl.wp : base + l.wp;
-    if (!(prep && (prep->reuse & D2C_REUSE_INPUT)))
-        if (int rc = pack_input<T>(s, x, xcl_p, st, true)) return rc;   // with the row of zeros behind it
+    const bool have_x = prep && (prep->reuse & D2C_REUSE_INPUT);
     if (nd == 3 && !prep && !stats && use_brick_forward(q, s, columns != nullptr)) {
         // sort the points, sample the columns (the caller's buffer, with the sorted points behind them for its backward
         // call, or the workspace), multiply.  A smaller workspace: the gathering kernels, below.
@@ -540,6 +569,8 @@ int forward_t(const d2c_conv3d_desc &q, const void *x, const void *off, const vo
         const bool fits = ws_bytes >= (keep ? l.lists : (columns ? l.col : l.end));
         char *col = columns ? (char *)columns : base + l.col;
         char *lists = keep ? col + brick_col_bytes(s) : base + l.lists;
+        if (fits)
+            if (int rc = pack_input<T>(s, x, xcl_p, st, true)) return rc;   // with the row of zeros behind it
         if (fits || keep)
             if (int rc = d2c_brick_sort(s, off, mask, lists, st)) return rc;
         if (fits) {
@@ -547,23 +578,19 @@ int forward_t(const d2c_conv3d_desc &q, const void *x, const void *off, const vo
             return d2c_col_forward(q, col, (int)d2c_columns_rows(s), w, bias, out, base + l.gemm, st);
         }
     }
-    const long total = (long)s.groups * s.nchunk * s.K * (s.ogp / 32) * 4 * 64;
-    long g = (total + 255) / 256;
-    if (g > 8192) g = 8192;
-    if (!(prep && (prep->reuse & D2C_REUSE_FORWARD_WEIGHTS))) {
-        D2cProfScope prof(D2C_PROF_PACK, st);
-        const size_t lds = (size_t)kPackRows * ((size_t)bkc_of(q.dtype) * s.K * sizeof(T) + 4);
-        if (lds <= 64 * 1024 && reinterpret_cast<uintptr_t>(w) % 16 == 0)
-            hipLaunchKernelGGL(pack_weight_fwd_lds_kernel<T>,
-                               dim3((unsigned)(s.groups * s.nchunk * (s.ogp / 32) * (32 / kPackRows))), dim3(256), lds, st,
-                               (const T *)w, (T *)wp_p, s);
-        else
-            hipLaunchKernelGGL(pack_weight_fwd_kernel<T>, dim3((unsigned)g), dim3(256), 0, st, (const T *)w,
-                               (T *)wp_p, s, total);
+    // input, weights, and the counters of the steps' split (which needs its scratch: a smaller workspace goes without)
+    PrepArgs pa{};
+    if (!have_x) {
+        prep_pack<T>(pa.pack[0], x, xcl_p, s.N, s.Cin, s.vol);
+        pa.zrow = (uint32_t *)((T *)xcl_p + (size_t)s.N * s.vol * s.Cin); pa.zrow_words = 64;
     }
-    if (int rc = d2c_check_launch("pack_weight_fwd_kernel")) return rc;
+    if (!(prep && (prep->reuse & D2C_REUSE_FORWARD_WEIGHTS))) prep_weight_fwd<T>(pa, s, w, wp_p);
+    const size_t split = d2c_fwd_split_bytes(s);
+    const bool shared = d2c_fwd_use_dma(s) || (split && (nd != 3 || ws_bytes >= l.outacc + split));
+    if (shared && split) prep_zero(pa, base + l.outacc, d2c_fwd_split_count_bytes(s));
+    if (int rc = prep_launch<T>(pa, st)) return rc;
     // (the per-tile sums of the output statistics go behind everything else in the workspace)
-    return d2c_tiled_fwd_launch<T>(s, xcl_p, off, mask, wp_p, bias, out, (float *)(base + l.outacc), st,
+    return d2c_tiled_fwd_launch<T>(s, xcl_p, off, mask, wp_p, bias, out, shared ? (float *)(base + l.outacc) : nullptr, st,
                                    stats, stats ? (float *)(base + l.least) : nullptr, columns);
 }
 
@@ -1033,8 +1060,11 @@ size_t d2c_tiled_forward_ws(const d2c_conv3d_desc &q, D2cForwardWs which)
     if (is_depthwise(q)) return dw_ws(q, s).total_fwd;
     const FwdWs l = fwd_ws(q, s);
     switch (which) {
+    case D2C_FWD_WS_GATHER: return l.least + d2c_fwd_split_bytes(s);
     case D2C_FWD_WS_LEAST: return l.least;
-    case D2C_FWD_WS_STATS: return l.least + (d2c_fwd_fills_stats(s) ? d2c_fwd_stats_ws(s) : 0);
+    case D2C_FWD_WS_STATS:
+    case D2C_FWD_WS_STATS_LEAST:
+        return l.least + (d2c_fwd_fills_stats(s) ? d2c_fwd_stats_ws(s) : 0) + (which == D2C_FWD_WS_STATS ? d2c_fwd_split_bytes(s) : 0);
     case D2C_FWD_WS_KEEP: return use_brick_forward(q, s, true) ? l.lists : l.least;
     case D2C_FWD_WS_KEEP_LEAST:
         return !use_brick_forward(q, s, true) ? l.least : (d2c_fwd_writes_columns(s, q.dtype) ? std::min(l.least, l.lists) : l.lists);

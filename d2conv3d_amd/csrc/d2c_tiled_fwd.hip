@@ -18,12 +18,18 @@
 #include "d2c_mma.hpp"
 #include "d2c_tiled.hpp"
 
+// the kernel of the small problems (d2c_tiled_wave.hip)
+size_t d2c_wave_count_bytes(const TiledShape &s, int nt);
+size_t d2c_wave_split_bytes(const TiledShape &s, int nt);
+template <typename T>
+int d2c_wave_launch(const TiledShape &s, int nt, const void *xcl, const void *off, const void *mask, const void *wp,
+                    const void *bias, void *out, float *split, float *stats, void *col, hipStream_t st);
+
 namespace {
 
 constexpr int kNV = 8;         // 16-byte vectors per sampled row (one chunk)
 constexpr int kRS = kNV * 16 + 16;  // LDS row stride in bytes (padded: conflict-free 16-byte reads)
 constexpr int kThreads = 512;
-constexpr int kMT = 128;       // positions per workgroup
 
 struct FwdArgs {
     TiledShape s;
@@ -32,10 +38,7 @@ struct FwdArgs {
     const void *wp;    // packed weights, see pack_weight_fwd
     const void *bias;
     void *out;
-    // Few tiles (small N*P): the steps are dealt to `nsplit` workgroups per tile, which add their partial
-    // sums into a zeroed fp32 array laid out like `out`; a finishing kernel adds the bias and converts.
-    float *outacc;
-    int nsplit;
+    float *outacc;     // fp32 tiles of the work items whose steps are shared out
     unsigned zrow;     // byte offset (from xcl) of a 128-byte row of zeros: what dead corners read
     // Schedule of the DMA-gather kernel, whose workgroups are persistent (one per compute unit).  A work item is
     // one (position tile, output tile, weight group) with all its steps.  Items [0, sk_full) are dealt whole,
@@ -65,258 +68,6 @@ D2C_DEV int xcd_swizzle(int bid, int n)
     const int q = n >> 3, r = n & 7;
     return x * q + (x < r ? x : r) + idx;
 }
-
-template <typename T, bool AUX16, int MT, int WAVES_O, int WAVES_P, bool SIZED>
-__global__ void __launch_bounds__(kThreads) tiled_fwd_kernel(FwdArgs a)
-{
-    constexpr int VEC = Elem<T>::VEC;
-    constexpr int BKC = kNV * VEC;
-    constexpr int WPOS = MT / WAVES_P;    // positions per MMA wave
-    constexpr int PB = WPOS / 32;         // 32-position blocks per MMA wave
-    constexpr int OB = 2;                 // 32-channel blocks per MMA wave
-    constexpr int NT = 64 * WAVES_O;      // output channels per workgroup
-    constexpr int NKG = kNV / 2;          // k-groups per step
-    constexpr int ITEMS = MT * kNV / kThreads;   // (position, vector) items per thread
-    static_assert(ITEMS >= 1 && ITEMS * kThreads == MT * kNV, "gather items divide evenly");
-    static_assert(WAVES_O * WAVES_P <= kThreads / 64 && PB >= 1, "MMA wave layout");
-
-    __shared__ __align__(16) unsigned char s_tile[2][MT * kRS];
-    __shared__ float s_w[2][8][MT];
-    __shared__ int s_idx[2][MT];
-    __shared__ int s_flag[2][MT];
-
-    const TiledShape &s = a.s;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int tile = xcd_swizzle(blockIdx.x, gridDim.x);
-    const int otile = blockIdx.y / a.nsplit, split = blockIdx.y - otile * a.nsplit, wg = blockIdx.z;
-    const int m0 = tile * MT;
-    const int S = s.nchunk * s.K;                           // steps of the whole reduction
-    const int st_lo = (int)((long)S * split / a.nsplit);    // this workgroup's share of them
-    const int st_hi = (int)((long)S * (split + 1) / a.nsplit);
-    const int dzc = s.H * s.W * s.Cin, dyc = s.W * s.Cin;   // element strides of a step in z / y
-
-    // --- per-position constants of the coordinate threads
-    int cb = 0, cp = 0, coz = 0, coy = 0, cox = 0;
-    bool cvalid = false;
-    if (tid < MT) {
-        const int m = m0 + tid;
-        cvalid = m < s.M;
-        if (cvalid) {
-            cb = m / s.P; cp = m - cb * s.P;
-            cox = cp % s.Wo; coy = (cp / s.Wo) % s.Ho; coz = cp / (s.Wo * s.Ho);
-        }
-    }
-
-    // offsets and modulation of step st: fetched early (coords_issue), turned into corner weights
-    // (modulation folded in, dead corners zero), base offset and live mask late (coords_finish)
-    float craw[4];
-    auto coords_issue = [&](int st) {
-        if (tid < MT && cvalid) {
-            const int j = st / s.K, k = st - j * s.K;
-            const int g = (wg * s.cg + j * BKC) / s.cpg;
-            tap_offsets_issue<AUX16, SIZED>(s, a.off, cb, g, k, cp, craw);
-            craw[3] = a.mask ? ld_auxT<AUX16>(a.mask, mask_index(s, cb, g, k, cp)) : 1.f;
-        }
-    };
-    auto coords_finish = [&](int st, int buf) {
-        if (tid < MT) {
-            float w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-            int idx = 0;
-            unsigned live = 0;
-            if (cvalid) {
-                const int k = st % s.K;
-                int bz, by, bx;
-                tap_base(s.geo, k, coz, coy, cox, bz, by, bx);
-                tap_offsets_finish<AUX16, SIZED>(s, k, craw);
-                const Tap3<float> t = tiled_tap3(s, bz, by, bx, craw[0], craw[1], craw[2]);
-                live = t.live;
-                idx = (cb * s.vol + (t.z0 * s.H + t.y0) * s.W + t.x0) * s.Cin;   // element offset of corner 000
-                typedef typename std::conditional<AUX16, bf16_t, float>::type AT;
-                const float al = (s.mact && a.mask) ? mask_act<AT>(s.mact, craw[3]) : craw[3];
-#pragma unroll
-                for (int c = 0; c < 8; c++) w[c] = ((live >> c) & 1u) ? tap3_weight(t, c) * al : 0.f;
-            }
-#pragma unroll
-            for (int c = 0; c < 8; c++) s_w[buf][c][tid] = w[c];
-            s_idx[buf][tid] = idx;
-            s_flag[buf][tid] = (int)live;
-        }
-    };
-
-    // --- gather: item i of this thread = (position, 16-byte channel vector)
-    uint4 gv[ITEMS][8];
-    auto gather_issue = [&](int st, int buf) {
-        const int j = st / s.K;
-        const int c0 = wg * s.cg + j * BKC;
-        // 32-bit byte offsets from a uniform base: the whole input is below 4 GiB (checked on the host)
-        const char *base = reinterpret_cast<const char *>(a.xcl);
-#pragma unroll
-        for (int i = 0; i < ITEMS; i++) {
-            const int item = tid + i * kThreads;
-            const int pos = item / kNV, vec = item % kNV;
-            const int idx = s_idx[buf][pos] + c0 + vec * VEC;
-            const unsigned live = (unsigned)s_flag[buf][pos];
-#pragma unroll
-            for (int c = 0; c < 8; c++) {
-                const unsigned o = (unsigned)(idx + ((c >> 2) & 1) * dzc + ((c >> 1) & 1) * dyc + (c & 1) * s.Cin)
-                                   * (unsigned)sizeof(T);
-                gv[i][c] = ((live >> c) & 1u) ? *reinterpret_cast<const uint4 *>(base + o) : make_uint4(0, 0, 0, 0);
-            }
-        }
-    };
-    auto interp_store = [&](int cbuf, int tbuf) {
-#pragma unroll
-        for (int i = 0; i < ITEMS; i++) {
-            const int item = tid + i * kThreads;
-            const int pos = item / kNV, vec = item % kNV;
-            VecAcc<T> acc;
-            acc.zero();
-#pragma unroll
-            for (int c = 0; c < 8; c++) acc.fma(s_w[cbuf][c][pos], gv[i][c]);
-            *reinterpret_cast<uint4 *>(&s_tile[tbuf][pos * kRS + vec * 16]) = acc.pack();
-        }
-    };
-
-    // --- MMA role
-    const bool mma_wave = wave < WAVES_O * WAVES_P;
-    const int wave_o = wave % WAVES_O, wave_p = wave / WAVES_O;
-    const int OBT = s.ogp / 32;  // 32-channel blocks per weight group in the packed weights
-    f32x16 acc[OB][PB];
-#pragma unroll
-    for (int ob = 0; ob < OB; ob++)
-#pragma unroll
-        for (int pb = 0; pb < PB; pb++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[ob][pb][r] = 0.f;
-
-    // weight fragments of one whole step live in registers; those of the next step are requested
-    // as soon as the matrix cores have taken the current ones
-    const uint4 *wp4 = reinterpret_cast<const uint4 *>(a.wp);
-    uint4 af[NKG][OB];
-    auto wfrag = [&](int st, int kg, int ob) {
-        const long wbase = (((long)wg * S + st) * OBT + (otile * (NT / 32) + wave_o * OB)) * NKG * 64 + lane;
-        return wp4[wbase + ((long)ob * NKG + kg) * 64];
-    };
-    auto mma_step = [&](int st, int tbuf) {
-        if (!mma_wave) return;
-        const unsigned char *tb = &s_tile[tbuf][(wave_p * WPOS + (lane & 31)) * kRS + (lane >> 5) * 16];
-#pragma unroll
-        for (int kg = 0; kg < NKG; kg++) {
-            uint4 bf[PB];
-#pragma unroll
-            for (int pb = 0; pb < PB; pb++)
-                bf[pb] = *reinterpret_cast<const uint4 *>(tb + pb * 32 * kRS + kg * 32);
-#pragma unroll
-            for (int ob = 0; ob < OB; ob++)
-#pragma unroll
-                for (int pb = 0; pb < PB; pb++) mma_kgroup<T, kF32SplitFwd>(acc[ob][pb], af[kg][ob], bf[pb]);
-            if (st + 1 < st_hi) {
-#pragma unroll
-                for (int ob = 0; ob < OB; ob++) af[kg][ob] = wfrag(st + 1, kg, ob);
-            }
-        }
-    };
-
-    // --- pipeline (buffers alternate with the parity of the step number)
-    coords_issue(st_lo);
-    if (mma_wave) {
-#pragma unroll
-        for (int kg = 0; kg < NKG; kg++)
-#pragma unroll
-            for (int ob = 0; ob < OB; ob++) af[kg][ob] = wfrag(st_lo, kg, ob);
-    }
-    coords_finish(st_lo, st_lo & 1);
-    if (st_lo + 1 < st_hi) coords_issue(st_lo + 1);
-    __syncthreads();
-    gather_issue(st_lo, st_lo & 1);
-    if (st_lo + 1 < st_hi) coords_finish(st_lo + 1, (st_lo + 1) & 1);
-    if (st_lo + 2 < st_hi) coords_issue(st_lo + 2);
-    interp_store(st_lo & 1, st_lo & 1);
-    __syncthreads();
-    for (int st = st_lo; st < st_hi; st++) {
-        if (st + 1 < st_hi) gather_issue(st + 1, (st + 1) & 1);
-        mma_step(st, st & 1);
-        if (st + 2 < st_hi) coords_finish(st + 2, st & 1);
-        if (st + 3 < st_hi) coords_issue(st + 3);
-        if (st + 1 < st_hi) interp_store((st + 1) & 1, (st + 1) & 1);
-        __syncthreads();
-    }
-
-    // --- epilogue: bias, convert, store (32 consecutive positions per row of a block)
-    if (mma_wave && a.stats && !a.outacc) {
-        // the same stores, and on the way the sum and the sum of squares of the stored values per (sample, output
-        // channel), added into the [N][Cout][2] result (zeroed by the launcher): the 32 lanes that hold the positions
-        // of a channel add up first when they lie in one sample (they nearly always do), so that one lane adds
-        T *out = reinterpret_cast<T *>(a.out);
-        const T *bias = reinterpret_cast<const T *>(a.bias);
-#pragma unroll
-        for (int pb = 0; pb < PB; pb++) {
-            const int m = m0 + wave_p * WPOS + pb * 32 + (lane & 31);
-            const bool ok = m < s.M;
-            const int b = ok ? m / s.P : -1, p = ok ? m - b * s.P : 0;
-            const int b0 = __shfl(b, lane & 32, 64);                    // sample of the half's first position
-            const unsigned long long odd = __ballot(ok && b != b0);
-            const bool uniform = ((odd >> (lane & 32)) & 0xffffffffull) == 0ull;
-#pragma unroll
-            for (int ob = 0; ob < OB; ob++) {
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const int ol = otile * NT + wave_o * 64 + ob * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                    const bool live = ok && ol < s.og;                  // (ol is uniform over the half)
-                    const int o = wg * s.og + ol;
-                    float fv = 0.f;
-                    if (live) {
-                        float v = acc[ob][pb][r];
-                        if (bias) v += elem_to_f32<T>(bias[o]);
-                        const T sv = f32_to_elem<T>(d2c_epilogue(v, s.act, s.act_scale));
-                        out[((long)b * s.Cout + o) * s.P + p] = sv;
-                        fv = elem_to_f32<T>(sv);
-                    }
-                    if (ol >= s.og) continue;
-                    if (uniform) {
-                        float q0 = fv, q1 = fv * fv;
-#pragma unroll
-                        for (int d = 1; d < 32; d <<= 1) { q0 += __shfl_xor(q0, d, 64); q1 += __shfl_xor(q1, d, 64); }
-                        if ((lane & 31) == 0 && b0 >= 0) {
-                            atomicAdd(a.stats + ((long)b0 * s.Cout + o) * 2, q0);
-                            atomicAdd(a.stats + ((long)b0 * s.Cout + o) * 2 + 1, q1);
-                        }
-                    } else if (live) {
-                        atomicAdd(a.stats + ((long)b * s.Cout + o) * 2, fv);
-                        atomicAdd(a.stats + ((long)b * s.Cout + o) * 2 + 1, fv * fv);
-                    }
-                }
-            }
-        }
-    } else if (mma_wave) {
-        T *out = reinterpret_cast<T *>(a.out);
-        const T *bias = reinterpret_cast<const T *>(a.bias);
-#pragma unroll
-        for (int pb = 0; pb < PB; pb++) {
-            const int m = m0 + wave_p * WPOS + pb * 32 + (lane & 31);
-            if (m >= s.M) continue;
-            const int b = m / s.P, p = m - b * s.P;
-#pragma unroll
-            for (int ob = 0; ob < OB; ob++) {
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const int ol = otile * NT + wave_o * 64 + ob * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                    if (ol < s.og) {
-                        const int o = wg * s.og + ol;
-                        float v = acc[ob][pb][r];
-                        if (a.outacc) {
-                            atomicAdd(a.outacc + ((long)b * s.Cout + o) * s.P + p, v);
-                        } else {
-                            if (bias) v += elem_to_f32<T>(bias[o]);
-                            out[((long)b * s.Cout + o) * s.P + p] = f32_to_elem<T>(d2c_epilogue(v, s.act, s.act_scale));
-                        }
-                    }
-                }
-            }
-        }
-    }
-}
-
 
 // ---------------------------------------------------------------------------
 // The same forward pass with the corner rows moved global -> LDS by DMA loads
@@ -1043,7 +794,6 @@ int launch_fwd_dma(FwdArgs a, float *outacc, hipStream_t st)
     }
     const int nshare = a.sk_items - a.sk_full;
     a.outacc = nshare ? outacc : nullptr;
-    a.nsplit = 1;
     if (nshare) {
         D2cProfScope prof(D2C_PROF_PACK, st);
         d2c_fill_zero(outacc, (size_t)nshare * NT * kDMT * sizeof(float), st);
@@ -1071,182 +821,106 @@ int launch_fwd_dma(FwdArgs a, float *outacc, hipStream_t st)
     return 0;
 }
 
-// out = epilogue(outacc + bias), in the element type of the output
-template <typename T>
-__global__ void __launch_bounds__(256) fwd_finish_kernel(const float *acc, const T *bias, T *out, int Cout, int P, long n,
-                                                         int act, float act_scale)
-{
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        float v = acc[i];
-        if (bias) v += elem_to_f32<T>(bias[(i / P) % Cout]);
-        out[i] = f32_to_elem<T>(d2c_epilogue(v, act, act_scale));
-    }
-}
-
-template <typename T, bool AUX16, int MT, int WO, int WP>
-int launch_fwd(const FwdArgs &a, hipStream_t st)
-{
-    const int ntile = (a.s.M + MT - 1) / MT;
-    const int NT = 64 * WO;
-    dim3 grid(ntile, a.s.ogp / NT * a.nsplit, a.s.groups);
-    D2cProfScope prof(D2C_PROF_FWD, st, "tiled_fwd_kernel");
-    if (a.s.ss.on) hipLaunchKernelGGL((tiled_fwd_kernel<T, AUX16, MT, WO, WP, true>), grid, dim3(kThreads), 0, st, a);
-    else hipLaunchKernelGGL((tiled_fwd_kernel<T, AUX16, MT, WO, WP, false>), grid, dim3(kThreads), 0, st, a);
-    return d2c_check_launch("tiled_fwd_kernel");
-}
-
-template <typename T, bool AUX16>
-int launch_fwd_cfg(const FwdArgs &a, int nt, hipStream_t st)
-{
-    switch (nt) {
-    case 512: return launch_fwd<T, AUX16, kMT, 8, 1>(a, st);
-    case 256: return launch_fwd<T, AUX16, kMT, 4, 2>(a, st);
-    case 128: return launch_fwd<T, AUX16, kMT, 2, 4>(a, st);
-    default: return launch_fwd<T, AUX16, kMT, 1, 4>(a, st);
-    }
-}
-
 }  // namespace
 
 // Which of the two forward kernels a shape runs on: the DMA-gather kernel (64-position tiles, 512 or 256 output channels
-// per workgroup, persistent, the steps of its last round of work items shared out) or the register-gather kernel
-// (128-position tiles).  Weight groups wider than 128 output channels take the DMA kernel when they fill the chip
-// with whole tiles (128 and more) or have at least 1024 steps in all: with few tiles it cuts their steps into as
-// many pieces as there are compute units (512 -> 512 channels on 8x15x27, 51 tiles: 0.74 -> 0.22 ms; 1024 -> 1024
-// on 4x8x14, 7 tiles of 432 steps: 0.46 -> 0.21 ms), which pays from about a thousand steps on (4 tiles of 48 steps,
-// 512 channels on 4 rows of 64 positions: 13 % slower; 2 tiles of 216 steps: 30 % slower).  Narrow weight groups leave
-// most of its output tile empty, but it is bound by its sampling, not by its matrix work: with enough tiles to fill
-// the chip without cutting their steps it is 1.3 - 2.2 x faster there too (1024 -> 108 channels on 8x30x54: 1.44 ->
-// 0.65 ms), and at the 128 tiles of 64 -> 64 channels on 8x32x32 it is 25 % slower.
-constexpr int kDmaTilesNarrow = 160, kDmaTilesWide = 128, kDmaStepsWide = 1024, kColsTiles = 48;
+// per workgroup, persistent, the steps of its last round of work items shared out) or the one whose wavefronts work alone
+// (32-position tiles, 128 or 64 output channels, d2c_tiled_wave.hip).  Measured on both, us per forward call, DMA first:
+//   up to 128 output channels the DMA kernel's output tile stays mostly empty.  64 -> 64, float32: 16000 positions 100,
+//   64; 51360 positions 281, 187.  128 -> 128: 171, 125; 509, 404.  256 -> 40: 319, 202; 1002, 705; bfloat16 128 -> 128:
+//   99, 75; 277, 229.  But wavefronts at different steps share no fragments, and weights that the L2 of an XCD does not
+//   hold come from further away: 512 -> 128, float32 (7 MB): 634, 539; 2106, 2130.  1024 -> 128 (14 MB): 1271, 1312;
+//   4876, 5703 (and 598, 598 at 8192 positions);
+//   above 128 the wavefronts sample once per 128 output channels.  256 -> 256, float32: 5120 positions 139, 200; 8192
+//   189, 232.  With few tiles both share out steps, and the DMA kernel's pieces are too many: 512 -> 512, bfloat16, 324
+//   positions 65, 53 (float32 70, 72), 1400 positions 82, 102; below about a thousand steps over all tiles (4 tiles of 48 steps,
+//   conv1d) its pipeline is not filled either.
+constexpr int kDmaTilesNarrow = 160, kDmaTilesWide = 128, kDmaTilesLeast = 10, kDmaStepsWide = 1024, kColsTiles = 48;
+constexpr size_t kDmaWeightBytes = 8u << 20;
 static long dma_tiles(const TiledShape &s) { return (long)((s.M + kDMT - 1) / kDMT) * s.groups; }
 bool d2c_fwd_use_dma(const TiledShape &s)
 {
     const long tiles = dma_tiles(s);
-    if (s.og <= 128) return tiles >= kDmaTilesNarrow;
-    return tiles >= kDmaTilesWide || tiles * s.nchunk * s.K >= kDmaStepsWide;
+    if (s.og <= 128)
+        return tiles >= kDmaTilesNarrow && s.og > 64 && (size_t)s.og * s.cg * s.K * (128 / s.bkc) >= kDmaWeightBytes;
+    return tiles >= kDmaTilesWide || (tiles >= kDmaTilesLeast && tiles * s.nchunk * s.K >= kDmaStepsWide);
 }
 
-int d2c_fwd_pos_tile(const TiledShape &s) { return d2c_fwd_use_dma(s) ? kDMT : kMT; }
-
-// Output channels per workgroup: as wide as the weight group needs (the sampled
-// tile is then produced once), but narrower when there are too few position
-// tiles to occupy the chip.
+// Output channels per workgroup.  The sampled tile of the DMA-gather kernel is produced once for all of them.
 int d2c_fwd_out_tile(const TiledShape &s)
 {
-    const int og = s.og;
-    if (d2c_fwd_use_dma(s)) return og > 256 ? 512 : 256;
-    int nt = og > 256 ? 512 : (og > 128 ? 256 : (og > 64 ? 128 : 64));
-    const int ntile = (s.M + kMT - 1) / kMT;
-    while (nt > 64 && ntile * ((og + nt - 1) / nt) < 128) nt >>= 1;
-    return nt;
+    if (d2c_fwd_use_dma(s)) return s.og > 256 ? 512 : 256;
+    return s.og > 64 ? 128 : 64;
 }
 
-// Workgroups per (position tile, output tile): 1 when the tiles alone fill the chip.
-int d2c_fwd_split(const TiledShape &s)
-{
-    // the DMA-gather kernel shares out the steps of its last round of work items, whatever their number
-    if (d2c_fwd_use_dma(s)) return 2;
-    const int mt = d2c_fwd_pos_tile(s), nt = d2c_fwd_out_tile(s);
-    const long wgs = (long)((s.M + mt - 1) / mt) * (s.ogp / nt) * s.groups;
-    if (wgs >= 128) return 1;
-    const int S = s.nchunk * s.K;
-    const long want = (256 + wgs - 1) / wgs;
-    return (int)(want < S ? want : S);
-}
+// Scratch of the other kernel where it shares the steps of a tile out between workgroups: the counters, all of it
+size_t d2c_fwd_split_count_bytes(const TiledShape &s) { return d2c_fwd_use_dma(s) ? 0 : d2c_wave_count_bytes(s, d2c_fwd_out_tile(s)); }
+size_t d2c_fwd_split_bytes(const TiledShape &s) { return d2c_fwd_use_dma(s) ? 0 : d2c_wave_split_bytes(s, d2c_fwd_out_tile(s)); }
 
-// Whether the forward kernels of this shape add up per-channel statistics themselves (FwdArgs::stats): the
-// DMA-gather kernel, on samples of at least one position tile (a tile then meets at most two samples).
-int d2c_fwd_split(const TiledShape &s);
 // The forward kernel of this shape adds the statistics of its output up while it stores: the DMA-gather kernel
-// (per position tile, see FwdArgs::stats) and the register-gather kernel when every workgroup holds whole sums (no
-// steps shared out between workgroups).
-bool d2c_fwd_fills_stats(const TiledShape &s)
-{
-    if (d2c_fwd_use_dma(s)) return s.P >= kDMT;
-    return d2c_fwd_split(s) == 1;
-}
+// (per position tile, see FwdArgs::stats; on samples of at least one position tile, which then meets at most two
+// samples), and the kernel of the small problems, which adds into the result itself.
+bool d2c_fwd_fills_stats(const TiledShape &s) { return !d2c_fwd_use_dma(s) || s.P >= kDMT; }
 size_t d2c_fwd_stats_ws(const TiledShape &s)
 {
-    if (!d2c_fwd_use_dma(s)) return 0;     // (the register-gather kernel adds into the result itself)
+    if (!d2c_fwd_use_dma(s)) return 0;
     return d2c_align_up((size_t)((s.M + kDMT - 1) / kDMT) * 2 * s.Cout * 2 * sizeof(float));
 }
 
-// Whether the forward kernel of this shape can write the sampled columns for the backward pass (FwdArgs::col): the
-// DMA-gather kernel on problems with offsets along all three axes and at least kColsTiles position tiles (below that
-// the backward kernels that read the columns lose to the ones that sample again: 256 -> 256 channels on 4x15x27, 26
-// tiles: 0.25 -> 0.30 ms).
+// Whether the forward kernel of this shape can write the sampled columns for the backward pass: on problems with
+// offsets along all three axes, wide weight groups from kColsTiles position tiles on (below that the backward kernels
+// that read the columns lose to the ones that sample again: 256 -> 256 channels on 4x15x27, 26 tiles: 0.25 -> 0.30 ms),
+// narrow ones from kDmaTilesNarrow tiles on.
 bool d2c_fwd_writes_columns(const TiledShape &s, int dtype)
 {
+    const long tiles = dma_tiles(s);
     return (dtype == D2C_BF16 || dtype == D2C_F32) && s.nd == 3 && (s.axes & 7) == 7 &&
-           d2c_fwd_use_dma(s) && dma_tiles(s) >= kColsTiles;
+           (s.og <= 128 ? tiles >= kDmaTilesNarrow : d2c_fwd_use_dma(s) && tiles >= kColsTiles);
 }
 long d2c_columns_rows(const TiledShape &s) { return (long)((s.M + kDMT - 1) / kDMT) * kDMT; }
 // `stats` / `stats_part`: the [N][Cout][2] result and the per-tile scratch of d2c_fwd_stats_ws() bytes, or NULL.
 // `col`: where the sampled columns go (d2c_fwd_writes_columns), or NULL.
+// `outacc`: partial sums of the DMA-gather kernel's shared work items, or the d2c_fwd_split_bytes() of the other kernel
+// (the counters first, cleared), NULL where that one is not to split its steps.
 template <typename T>
 int d2c_tiled_fwd_launch(const TiledShape &s, const void *xcl, const void *off, const void *mask, const void *wp,
                          const void *bias, void *out, float *outacc, hipStream_t st, float *stats, float *stats_part,
                          void *col)
 {
-    const bool dma = d2c_fwd_use_dma(s);
-    const int nsplit = (outacc && !dma) ? d2c_fwd_split(s) : 1;
-    const long n = (long)s.N * s.Cout * s.P;
+    const int nt = d2c_fwd_out_tile(s);
+    if (col && !d2c_fwd_writes_columns(s, (int)Elem<T>::DT)) col = nullptr;
+    if (!d2c_fwd_use_dma(s)) return d2c_wave_launch<T>(s, nt, xcl, off, mask, wp, bias, out, outacc, stats, col, st);
     // the channels-last input is followed by a row of zeros (see forward_t)
     const unsigned zrow = (unsigned)((size_t)s.N * s.vol * s.Cin * sizeof(T));
-    FwdArgs a{s, xcl, off, mask, wp, bias, out, nsplit > 1 ? outacc : nullptr, nsplit, zrow, 0, 0, 0, 0, 1,
-              stats ? (dma ? stats_part : (nsplit == 1 ? stats : nullptr)) : nullptr, nullptr, 0};
-    if (col && d2c_fwd_writes_columns(s, (int)Elem<T>::DT)) {
+    FwdArgs a{s, xcl, off, mask, wp, bias, out, nullptr, zrow, 0, 0, 0, 0, 1, stats ? stats_part : nullptr, nullptr, 0};
+    bool aux16 = false;
+    if constexpr (sizeof(T) == 2) aux16 = s.adt == D2C_BF16;
+    if (col) {
         a.col = col;
         a.col_rows = d2c_columns_rows(s);
     }
-    if (a.stats && !dma) {
-        D2cProfScope prof(D2C_PROF_PACK, st);
-        d2c_fill_zero(a.stats, (size_t)s.N * s.Cout * 2 * sizeof(float), st);
-    }
-    if (a.stats && dma && d2c_fwd_out_tile(s) != 512) {
+    if (a.stats && nt != 512) {
         // (the 256-channel tile has two wavefronts per channel, which add into their slots)
         D2cProfScope prof(D2C_PROF_PACK, st);
         d2c_fill_zero(a.stats, d2c_fwd_stats_ws(s), st);
     }
-    if (nsplit > 1) {
-        D2cProfScope prof(D2C_PROF_PACK, st);
-        d2c_fill_zero(outacc, (size_t)n * sizeof(float), st);
-    }
-    const int nt = d2c_fwd_out_tile(s);
     int rc = 0;
-    bool aux16 = false;
-    if constexpr (sizeof(T) == 2) aux16 = s.adt == D2C_BF16;
-    if (dma) {
-        if (nt == 512) {
-            if constexpr (sizeof(T) == 2) {
-                if (aux16) rc = launch_fwd_dma<T, true, 8, 1>(a, outacc, st);
-            }
-            if (!aux16) rc = launch_fwd_dma<T, false, 8, 1>(a, outacc, st);
-        } else {
-            if constexpr (sizeof(T) == 2) {
-                if (aux16) rc = launch_fwd_dma<T, true, 4, 2>(a, outacc, st);
-            }
-            if (!aux16) rc = launch_fwd_dma<T, false, 4, 2>(a, outacc, st);
+    if (nt == 512) {
+        if constexpr (sizeof(T) == 2) {
+            if (aux16) rc = launch_fwd_dma<T, true, 8, 1>(a, outacc, st);
         }
-        if (rc || !a.stats) return rc;
-        D2cProfScope prof(D2C_PROF_PACK, st);
-        hipLaunchKernelGGL(stats_reduce_kernel, dim3((unsigned)(s.N * ((s.Cout + kStatChan - 1) / kStatChan))), dim3(256), 0, st, a.stats,
-                           stats, s.N, s.Cout, s.P, s.M);
-        return d2c_check_launch("stats_reduce_kernel");
+        if (!aux16) rc = launch_fwd_dma<T, false, 8, 1>(a, outacc, st);
     } else {
         if constexpr (sizeof(T) == 2) {
-            if (aux16) rc = launch_fwd_cfg<T, true>(a, nt, st);
+            if (aux16) rc = launch_fwd_dma<T, true, 4, 2>(a, outacc, st);
         }
-        if (!aux16) rc = launch_fwd_cfg<T, false>(a, nt, st);
+        if (!aux16) rc = launch_fwd_dma<T, false, 4, 2>(a, outacc, st);
     }
-    if (rc || nsplit == 1) return rc;
-    long g = (n + 255) / 256;
-    if (g > 8192) g = 8192;
+    if (rc || !a.stats) return rc;
     D2cProfScope prof(D2C_PROF_PACK, st);
-    hipLaunchKernelGGL(fwd_finish_kernel<T>, dim3((unsigned)g), dim3(256), 0, st, outacc, (const T *)bias, (T *)out,
-                       s.Cout, s.P, n, s.act, s.act_scale);
-    return d2c_check_launch("fwd_finish_kernel");
+    hipLaunchKernelGGL(stats_reduce_kernel, dim3((unsigned)(s.N * ((s.Cout + kStatChan - 1) / kStatChan))), dim3(256), 0, st, a.stats,
+                       stats, s.N, s.Cout, s.P, s.M);
+    return d2c_check_launch("stats_reduce_kernel");
 }
 template int d2c_tiled_fwd_launch<bf16_t>(const TiledShape &, const void *, const void *, const void *, const void *,
                                           const void *, void *, float *, hipStream_t, float *, float *, void *);

@@ -160,7 +160,7 @@ size_t d2c_conv3d_forward_workspace_bytes(const d2c_conv3d_desc *desc);
 size_t d2c_conv3d_backward_workspace_bytes(const d2c_conv3d_desc *desc);
 /* d2c_conv3d_forward_workspace_bytes() is what a forward call is fastest with.  Large bfloat16 problems hold their sampled
  * columns there, taps x the size of the input; given less, but at least this much, the call runs on kernels that
- * need none (also d2c_conv3d_sized_forward with its `size_map`, else NULL, d2c_conv3d_forward_prepared, which always does, and
+ * need none, which on small problems includes room for partial sums that they can do without (also d2c_conv3d_sized_forward with its `size_map`, else NULL, d2c_conv3d_forward_prepared, which always does, and
  * d2c_conv3d_forward_stats on descriptions whose statistics are a pass of their own). */
 size_t d2c_conv3d_forward_least_workspace_bytes(const d2c_conv3d_desc *desc, const struct d2c_size_map_desc *size_map);
 
@@ -174,7 +174,7 @@ int d2c_conv3d_forward(const d2c_conv3d_desc *desc, const void *x, const void *o
  * capture, tight serving loops, harnesses that forbid hipMalloc.  The scratch memory is an array of
  * D2C_STATIC_WORKSPACE_BYTES inside the library's device image (each GPU the library runs on holds its own
  * copy until the process ends); the call makes no hipMalloc / hipFree and uses no allocating library routine.
- * A description whose d2c_conv3d_forward_least_workspace_bytes() exceeds that size is refused with
+ * A description that needs more than that size is refused with
  * D2C_ERR_WORKSPACE.  All calls on one GPU share that GPU's array: calls that overlap in time on one GPU
  * (different streams or threads) race; serialise them.  Otherwise identical to d2c_conv3d_forward
  * with a workspace of that size (same kernels, same results).  Instrumentation (d2c_profile_enable) must be off: it creates events.
