@@ -14,6 +14,7 @@
 // 256 channels on 32x60x108, bound by the L1 path, the vector ALU and row latency; this one takes 0.87, at 2.4 TB/s to and
 // from device memory, and 0.22 for 512 channels in 8 groups on 2x8x30x54, where they took 0.50 + 0.35.)
 
+#include <algorithm>
 #include "d2c_mma.hpp"
 #include "d2c_tiled.hpp"
 #include "d2c_brick.hpp"
@@ -25,38 +26,227 @@ typedef short v4s __attribute__((ext_vector_type(4)));
 // One sampling point as the sort sees it.
 struct BrickPoint {
     bool in;              // a corner is inside the volume
-    int seg;              // its block
+    int zi, yq, xq;       // its block
     unsigned cell;        // its base voxel in the block: y | x << 2
     float hz, hy, hx;     // fractions, as make_tap3 gives them
 };
 D2C_DEV int brick_seg(const BrickDims &d, int bg, int zi, int by, int bx) { return ((bg * d.nz + zi) * d.nby + by) * d.nbx + bx; }
-// (`c`: what tap_offsets_issue() read)
+// (`c`: what tap_offsets_issue() read for tap k of output position (oz, oy, ox))
 template <bool AUX16, bool SIZED>
-D2C_DEV BrickPoint brick_point(const TiledShape &s, const BrickDims &d, float *c, int b, int g, int k, int p)
+D2C_DEV BrickPoint brick_point(const TiledShape &s, const float *craw, int k, int oz, int oy, int ox)
 {
+    float c[3] = {craw[0], craw[1], craw[2]};
     tap_offsets_finish<AUX16, SIZED>(s, k, c);
-    const int oz = fdiv(p, s.dHW), rem = p - oz * (s.Wo * s.Ho);
-    const int oy = fdiv(rem, s.dW), ox = rem - oy * s.Wo;
     int bz, by, bx;
     tap_base(s.geo, k, oz, oy, ox, bz, by, bx);
     const Tap3<float> t = tiled_tap3(s, bz, by, bx, c[0], c[1], c[2]);
     BrickPoint r;
     r.in = t.inrange != 0;
-    const int yq = (t.y0 + 1) / 3, xq = (t.x0 + 1) / 3;       // (base voxels start at -1)
-    r.cell = (unsigned)(t.y0 + 1 - yq * 3) | (unsigned)(t.x0 + 1 - xq * 3) << 2;
+    r.zi = t.z0 + 1; r.yq = (t.y0 + 1) / 3; r.xq = (t.x0 + 1) / 3;       // (base voxels start at -1)
+    r.cell = (unsigned)(t.y0 + 1 - r.yq * 3) | (unsigned)(t.x0 + 1 - r.xq * 3) << 2;
     r.hz = t.hz; r.hy = t.hy; r.hx = t.hx;
-    r.seg = brick_seg(d, b * s.G + g, t.z0 + 1, yq, xq);
     return r;
 }
 
-// ---- the sort: count the points of every block (a point remembers its place), give every block a range, file ------
-// A workgroup works on 256 positions and up to kTaps taps, and requests what it reads of all of them first.  Points of
-// neighbouring positions fall into few blocks: they are counted in a hash table in LDS, and each block's number goes to
-// the global count in one addition.  (One global atomic per point, taps in workgroups of their own: 0.24 ms for 5.6 M
-// points in 8 offset groups on 8x30x54; this way 0.13, and 0.14 to file them.)
-// Workgroups of the passes over all points: an XCD takes a contiguous part of the positions, the tap groups of a block
-// of 256 one after the other, so that the lines which several workgroups write or read in parts meet in one L2.
-constexpr int kTaps = 9, kSlots = 4096;             // (more slots than a workgroup has points: a probe always ends)
+// ---- the sort: count the points of every block, give every block a range, file -------------------------------------
+// A workgroup works on 256 positions and up to 28 taps, 4 threads to a position, and requests what it reads of all of
+// them first.  Points of neighbouring positions fall into few blocks: they are counted in LDS, in a window of the blocks
+// around the workgroup's positions (all blocks of the sample and group where those fit), and a block's number goes to the
+// global count in one addition.  The filing pass counts in LDS again: a point's place among the workgroup's points of
+// its block is what the addition returned, and the workgroup takes its range of a block's entries in one addition.
+// So neither pass writes or reads anything per point that is not wanted in the end.  Points outside the window take
+// the global additions one by one; those outside the volume are counted per workgroup too (additions to one address
+// follow each other at about 10 ns: with one for every wavefront the list of them took half of the filing pass).
+// Bound: scattered stores of 20 bytes to a point, and the instructions of a point's place (about 150).  5.6 M points in 8
+// offset groups on 2x8x30x54, us for counting + ranges + filing: 134 + 8 + 146 with a hash table per workgroup, places
+// of the counting pass kept in memory and an addition per wavefront for the points outside; 46 + 5 + 89 this way.
+// 32x60x108 in one group 95 + 7 + 136 and 48 + 5 + 100; 2x8x30x54 in one group 24 + 4 + 35 and 12 + 5 + 21.
+// Workgroups: an XCD takes a contiguous part of the positions, the tap groups of a block of 256 one after the other, so
+// that the lines which several workgroups write or read in parts meet in one L2.
+constexpr int kTaps = 7, kTapGroups = 4, kSortThreads = 256 * kTapGroups;
+constexpr int kSortTaps = kTaps * kTapGroups;
+struct SortWindow {
+    int wz, wy, wx;       // blocks of the window along each axis
+    int ngrp, taps;       // groups of taps, taps to a group (up to kSortTaps)
+    int ly, lx;           // a workgroup's positions: 2^(8 - ly - lx) planes of 2^ly x 2^lx
+    int ny, nx, ntile;    // such tiles along y and x, and of a sample
+};
+struct SortUnit {
+    int b, g, bg, k0, k1; // taps k0, k0 + kTapGroups, ... below k1
+    int oz, oy, ox, p;    // the thread's position
+    bool ok;              // ... is one
+    int z0, y0, x0;       // first block of the window
+};
+D2C_DEV SortUnit sort_unit(const TiledShape &s, const BrickDims &d, const SortWindow &w)
+{
+    const int nt = (int)gridDim.x, q = nt >> 3, r = nt & 7, xcd = blockIdx.x & 7;
+    const int u = xcd * q + (xcd < r ? xcd : r) + (int)(blockIdx.x >> 3);
+    const int blk = u / w.ngrp;
+    SortUnit t;
+    t.bg = blk / w.ntile; t.b = t.bg / s.G; t.g = t.bg - t.b * s.G;
+    const int tile = blk - t.bg * w.ntile, tzy = tile / w.nx, tx = tile - tzy * w.nx, tz = tzy / w.ny, ty = tzy - tz * w.ny;
+    const int lz = 8 - w.ly - w.lx, i = threadIdx.x & 255;
+    t.oz = (tz << lz) + (i >> (w.ly + w.lx)); t.oy = (ty << w.ly) + ((i >> w.lx) & ((1 << w.ly) - 1)); t.ox = (tx << w.lx) + (i & ((1 << w.lx) - 1));
+    t.ok = t.oz < s.Do && t.oy < s.Ho && t.ox < s.Wo;
+    t.p = t.ok ? (t.oz * s.Ho + t.oy) * s.Wo + t.ox : 0;
+    t.k0 = (u - blk * w.ngrp) * w.taps;
+    t.k1 = min(t.k0 + w.taps, s.K);
+    t.k0 += __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    // the window lies around the middle of the workgroup's positions and taps
+    const int cz = ((tz << lz) + (1 << lz) / 2) * s.geo.sd - s.geo.pd + (s.geo.kd - 1) * s.geo.dd / 2 + 1;
+    const int cy = (((ty << w.ly) + (1 << w.ly) / 2) * s.geo.sh - s.geo.ph + (s.geo.kh - 1) * s.geo.dh / 2 + 1) / 3;
+    const int cx = (((tx << w.lx) + (1 << w.lx) / 2) * s.geo.sw - s.geo.pw + (s.geo.kw - 1) * s.geo.dw / 2 + 1) / 3;
+    t.z0 = max(0, min(cz - w.wz / 2, d.nz - w.wz));
+    t.y0 = max(0, min(cy - w.wy / 2, d.nby - w.wy));
+    t.x0 = max(0, min(cx - w.wx / 2, d.nbx - w.wx));
+    return t;
+}
+// slot of a point's block in the window, -1: outside
+D2C_DEV int sort_slot(const SortWindow &w, const SortUnit &t, const BrickPoint &q)
+{
+    const int z = q.zi - t.z0, y = q.yq - t.y0, x = q.xq - t.x0;
+    return (unsigned)z < (unsigned)w.wz && (unsigned)y < (unsigned)w.wy && (unsigned)x < (unsigned)w.wx ? (z * w.wy + y) * w.wx + x : -1;
+}
+D2C_DEV int sort_slot_seg(const BrickDims &d, const SortWindow &w, const SortUnit &t, int i)
+{
+    const int r = i / w.wx, x = i - r * w.wx, z = r / w.wy, y = r - z * w.wy;
+    return brick_seg(d, t.bg, t.z0 + z, t.y0 + y, t.x0 + x);
+}
+// the offsets of the thread's taps k0, k0 + kTapGroups, ...
+template <bool AUX16, bool SIZED>
+D2C_DEV void sort_offsets(const TiledShape &s, const void *off, const SortUnit &t, float (&c)[kTaps][3])
+{
+#pragma unroll
+    for (int i = 0; i < kTaps; i++)
+        if (t.k0 + i * kTapGroups < t.k1) tap_offsets_issue<AUX16, SIZED>(s, off, t.b, t.g, t.k0 + i * kTapGroups, t.p, c[i]);
+}
+template <bool AUX16, bool SIZED>
+__global__ void __launch_bounds__(kSortThreads, 8)     // (two workgroups to a compute unit)
+brick_count_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, SortWindow w)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    int *const s_cnt = reinterpret_cast<int *>(smem);
+    const int nslot = w.wz * w.wy * w.wx;
+    const SortUnit t = sort_unit(s, d, w);
+    float c[kTaps][3];
+    sort_offsets<AUX16, SIZED>(s, off, t, c);
+    for (int i = threadIdx.x; i < nslot; i += kSortThreads) s_cnt[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kTaps; i++) {
+        const int k = t.k0 + i * kTapGroups;
+        if (!t.ok || k >= t.k1) continue;
+        const BrickPoint q = brick_point<AUX16, SIZED>(s, c[i], k, t.oz, t.oy, t.ox);
+        if (!q.in) continue;
+        const int sl = sort_slot(w, t, q);
+        if (sl >= 0) atomicAdd(&s_cnt[sl], 1);
+        else atomicAdd(&L.count[brick_seg(d, t.bg, q.zi, q.yq, q.xq)], 1);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < nslot; i += kSortThreads) {
+        const int n = s_cnt[i];
+        if (n) atomicAdd(&L.count[sort_slot_seg(d, w, t, i)], n);
+    }
+}
+// (the order of the ranges does not matter: a workgroup adds up its 1024 counts and takes one range for all; additions to
+// one address follow each other at about 10 ns)
+__global__ void __launch_bounds__(1024) brick_range_kernel(BrickLists L, int nseg)
+{
+    __shared__ int s_sum[16];
+    const int i = blockIdx.x * 1024 + threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int n = i < nseg ? L.count[i] : 0;
+    int sum = n;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int v = __shfl_up(sum, d, 64);
+        if (lane >= d) sum += v;
+    }
+    if (lane == 63) s_sum[wave] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int all = 0;
+        for (int w = 0; w < 16; w++) { const int v = s_sum[w]; s_sum[w] = all; all += v; }
+        const int base = atomicAdd(L.cursor, all);
+        for (int w = 0; w < 16; w++) s_sum[w] += base;
+    }
+    __syncthreads();
+    if (i < nseg) L.end[i] = s_sum[wave] + sum - n;       // (the filing pass takes entries from here on and leaves the end)
+}
+template <bool AUX16, bool SIZED>
+__global__ void __launch_bounds__(kSortThreads, 8)     // (two workgroups to a compute unit)
+brick_file_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, const void *mask, SortWindow w, long n)
+{
+    typedef typename std::conditional<AUX16, bf16_t, float>::type AT;
+    extern __shared__ __align__(16) unsigned char smem[];
+    int *const s_cnt = reinterpret_cast<int *>(smem);
+    const int nslot = w.wz * w.wy * w.wx;
+    const SortUnit t = sort_unit(s, d, w);
+    float c[kTaps][3], al[kTaps];
+    sort_offsets<AUX16, SIZED>(s, off, t, c);
+#pragma unroll
+    for (int i = 0; i < kTaps; i++) {
+        const int k = t.k0 + i * kTapGroups;
+        al[i] = mask && k < t.k1 ? ld_auxT<AUX16>(mask, mask_index(s, t.b, t.g, k, t.p)) : 1.f;
+    }
+    for (int i = threadIdx.x; i <= nslot; i += kSortThreads) s_cnt[i] = 0;
+    __syncthreads();
+    // slot << 4 | base voxel (slot -1: outside the window, `rank` is the entry; all ones: no point)
+    int slot[kTaps], rank[kTaps];
+#pragma unroll
+    for (int i = 0; i < kTaps; i++) {
+        const int k = t.k0 + i * kTapGroups;
+        slot[i] = -1; rank[i] = 0;
+        if (!t.ok || k >= t.k1) continue;
+        const BrickPoint q = brick_point<AUX16, SIZED>(s, c[i], k, t.oz, t.oy, t.ox);
+        c[i][0] = q.hz; c[i][1] = q.hy; c[i][2] = q.hx;
+        if (!q.in) continue;
+        const int sl = sort_slot(w, t, q);
+        slot[i] = (int)((unsigned)sl << 4 | q.cell);
+        rank[i] = sl >= 0 ? atomicAdd(&s_cnt[sl], 1) : atomicAdd(&L.end[brick_seg(d, t.bg, q.zi, q.yq, q.xq)], 1);
+    }
+    // points outside the volume: behind the window's counts, a wavefront's together
+    unsigned long long m[kTaps];
+    int total = 0, out = 0;
+#pragma unroll
+    for (int i = 0; i < kTaps; i++) {
+        m[i] = __ballot(t.ok && t.k0 + i * kTapGroups < t.k1 && slot[i] == -1);
+        total += __popcll(m[i]);
+    }
+    const int lane = threadIdx.x & 63;
+    if (total && lane == 0) out = atomicAdd(&s_cnt[nslot], total);
+    __syncthreads();
+    if (threadIdx.x == 0 && s_cnt[nslot]) s_cnt[nslot] = atomicAdd(L.cursor + 1, s_cnt[nslot]);
+    for (int i = threadIdx.x; i < nslot; i += kSortThreads) {
+        const int m = s_cnt[i];
+        if (m) s_cnt[i] = atomicAdd(&L.end[sort_slot_seg(d, w, t, i)], m);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kTaps; i++) {
+        const int k = t.k0 + i * kTapGroups;
+        if (!t.ok || k >= t.k1) continue;
+        const int at = slot[i] >= 0 ? s_cnt[slot[i] >> 4] + rank[i] : (slot[i] == -1 ? -1 : rank[i]);
+        L.place[((long)t.bg * s.K + k) * s.P + t.p] = at;
+        if (at < 0) continue;
+        L.pt[at] = make_uint4((unsigned)(k * s.M + t.b * s.P + t.p) * 128u | (unsigned)(slot[i] & 15), __float_as_uint(c[i][1]),
+                              __float_as_uint(c[i][2]), __float_as_uint(c[i][0]));
+        L.alpha[at] = (mask && s.mact) ? mask_act<AT>(s.mact, al[i]) : al[i];
+    }
+    // points outside the volume: their rows among all groups' rows, listed downwards from the end of the entries (which the
+    // points inside leave free)
+    if (total == 0) return;
+    int at = __builtin_amdgcn_readfirstlane(out) + s_cnt[nslot];
+    unsigned *const end = reinterpret_cast<unsigned *>(L.pt + n) - 1;
+#pragma unroll
+    for (int i = 0; i < kTaps; i++) {
+        if ((m[i] >> lane) & 1)
+            end[-(long)(at + __popcll(m[i] & ((1ull << lane) - 1)))] =
+                (unsigned)((t.g * s.K + t.k0 + i * kTapGroups) * s.M + t.b * s.P + t.p);
+        at += __popcll(m[i]);
+    }
+}
+// Workgroups of a pass over all points that needs no window: 256 positions, kPassTaps taps
+constexpr int kPassTaps = 9;
 struct PointUnit {
     int b, g, bg, k0, p;
 };
@@ -67,141 +257,8 @@ D2C_DEV PointUnit point_unit(const TiledShape &s, int ngrp)
     const int npb = (s.P + 255) / 256, blk = u / ngrp;
     PointUnit t;
     t.bg = blk / npb; t.b = t.bg / s.G; t.g = t.bg - t.b * s.G;
-    t.k0 = (u - blk * ngrp) * kTaps; t.p = (blk - t.bg * npb) * 256 + threadIdx.x;
+    t.k0 = (u - blk * ngrp) * kPassTaps; t.p = (blk - t.bg * npb) * 256 + threadIdx.x;
     return t;
-}
-template <bool AUX16, bool SIZED>
-__global__ void __launch_bounds__(256)
-brick_count_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, int ngrp)
-{
-    __shared__ int s_key[kSlots], s_cnt[kSlots];
-    static_assert(kTaps * 256 < kSlots && kSlots <= 65536, "table size");
-    const PointUnit un = point_unit(s, ngrp);
-    const int k0 = un.k0, bg = un.bg, b = un.b, g = un.g, p = un.p, pl = min(p, s.P - 1);
-    float c[kTaps][3];
-#pragma unroll
-    for (int i = 0; i < kTaps; i++) tap_offsets_issue<AUX16, SIZED>(s, off, b, g, min(k0 + i, s.K - 1), pl, c[i]);
-    for (int i = threadIdx.x; i < kSlots; i += 256) { s_key[i] = -1; s_cnt[i] = 0; }
-    __syncthreads();
-    unsigned pt[kTaps];                              // slot << 16 | place among the workgroup's points there, or all ones
-#pragma unroll
-    for (int i = 0; i < kTaps; i++) {
-        pt[i] = ~0u;
-        if (p >= s.P || k0 + i >= s.K) continue;
-        const BrickPoint q = brick_point<AUX16, SIZED>(s, d, c[i], b, g, k0 + i, p);
-        if (!q.in) continue;
-        unsigned sl = ((unsigned)q.seg * 2654435761u) >> 20;
-        for (;;) {
-            const int old = atomicCAS(&s_key[sl], -1, q.seg);
-            if (old == -1 || old == q.seg) break;
-            sl = (sl + 1) & (kSlots - 1);
-        }
-        pt[i] = (sl << 16) | (unsigned)atomicAdd(&s_cnt[sl], 1);
-    }
-    __syncthreads();
-    // (through a buffer descriptor, an empty slot's addition past its end: no branch, so that all are on their way at once)
-    const auto rs = __builtin_amdgcn_make_buffer_rsrc(L.count, 0, L.cursor - L.count > 0 ? (int)((L.cursor - L.count) * 4) : 0, 0x00020000);
-    int base[kSlots / 256];
-#pragma unroll
-    for (int i = 0; i < kSlots / 256; i++) {
-        const int key = s_key[i * 256 + threadIdx.x];
-        base[i] = __builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(s_cnt[i * 256 + threadIdx.x], rs, key >= 0 ? key * 4 : -16, 0, 0);
-    }
-#pragma unroll
-    for (int i = 0; i < kSlots / 256; i++) s_cnt[i * 256 + threadIdx.x] = base[i];
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kTaps; i++)
-        if (p < s.P && k0 + i < s.K)
-            L.place[((long)bg * s.K + k0 + i) * s.P + p] = pt[i] == ~0u ? -1 : s_cnt[pt[i] >> 16] + (int)(pt[i] & 0xffffu);
-}
-// Few points, or few to a block: one global addition each, which costs by the additions that meet at one count.  The two
-// kernels in us, this one first: 7 taps (63 points to a block) 12 and 17 at 90 000 points, 13 and 18 at 242 000, 20 and
-// 20 at 484 000; 27 taps (243 to a block) 12 and 15 at 22 000, 18 and 19 at 44 000, 24 and 22 at 87 000, 34 and 27 at
-// 350 000, 55 and 27 at 700 000 in two groups.
-template <bool AUX16, bool SIZED>
-__global__ void __launch_bounds__(256)
-brick_count_few_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off)
-{
-    const int u = blockIdx.x, npb = (s.P + 255) / 256, bgk = u / npb, bg = bgk / s.K, k = bgk - bg * s.K, b = bg / s.G, g = bg - b * s.G;
-    const int p = (u - bgk * npb) * 256 + threadIdx.x;
-    if (p >= s.P) return;
-    float c[3];
-    tap_offsets_issue<AUX16, SIZED>(s, off, b, g, k, p, c);
-    const BrickPoint q = brick_point<AUX16, SIZED>(s, d, c, b, g, k, p);
-    L.place[((long)bg * s.K + k) * s.P + p] = q.in ? atomicAdd(&L.count[q.seg], 1) : -1;
-}
-// (the order of the ranges does not matter: a wavefront adds up its 64 counts and takes one range for all)
-__global__ void __launch_bounds__(256) brick_range_kernel(BrickLists L, int nseg)
-{
-    const int i = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63;
-    const int n = i < nseg ? L.count[i] : 0;
-    int sum = n;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int v = __shfl_up(sum, d, 64);
-        if (lane >= d) sum += v;
-    }
-    int base = 0;
-    if (lane == 63) base = atomicAdd(L.cursor, sum);
-    base = __shfl(base, 63, 64);
-    if (i < nseg) L.start[i] = base + sum - n;
-}
-// (all taps of a position in one workgroup: the places a workgroup's points were given in a block follow each other)
-template <bool AUX16, bool SIZED>
-__global__ void __launch_bounds__(256)
-brick_file_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, const void *mask, int ngrp, long n)
-{
-    typedef typename std::conditional<AUX16, bf16_t, float>::type AT;
-    const PointUnit un = point_unit(s, ngrp);
-    const int k0 = un.k0, bg = un.bg, b = un.b, g = un.g, p = un.p;
-    if (p >= s.P) return;
-    int *place = L.place + ((long)bg * s.K + k0) * s.P + p;
-    float c[kTaps][3], al[kTaps];
-    int rank[kTaps], start[kTaps];
-    BrickPoint q[kTaps];
-#pragma unroll
-    for (int i = 0; i < kTaps; i++) {
-        const int k = min(k0 + i, s.K - 1);
-        rank[i] = k0 + i < s.K ? place[(long)i * s.P] : -1;
-        tap_offsets_issue<AUX16, SIZED>(s, off, b, g, k, p, c[i]);
-        al[i] = mask ? ld_auxT<AUX16>(mask, mask_index(s, b, g, k, p)) : 1.f;
-    }
-#pragma unroll
-    for (int i = 0; i < kTaps; i++) {
-        q[i] = brick_point<AUX16, SIZED>(s, d, c[i], b, g, min(k0 + i, s.K - 1), p);
-        start[i] = rank[i] >= 0 ? L.start[q[i].seg] : 0;
-    }
-#pragma unroll
-    for (int i = 0; i < kTaps; i++) {
-        if (rank[i] < 0) continue;
-        const int at = start[i] + rank[i];
-        place[(long)i * s.P] = at;
-        L.pt[at] = make_uint4((unsigned)((k0 + i) * s.M + b * s.P + p) * 128u | q[i].cell, __float_as_uint(q[i].hy),
-                              __float_as_uint(q[i].hx), __float_as_uint(q[i].hz));
-        L.alpha[at] = (mask && s.mact) ? mask_act<AT>(s.mact, al[i]) : al[i];
-    }
-    // points outside the volume: their rows among all groups' rows, listed downwards from the end of the entries (which the
-    // points inside leave free), one addition to the counter per wavefront
-    unsigned long long m[kTaps];
-    int total = 0;
-#pragma unroll
-    for (int i = 0; i < kTaps; i++) {
-        m[i] = __ballot(rank[i] < 0 && k0 + i < s.K);
-        total += __popcll(m[i]);
-    }
-    if (total == 0) return;
-    const int lane = threadIdx.x & 63;
-    int at = 0;
-    if (lane == 0) at = atomicAdd(L.cursor + 1, total);
-    at = __builtin_amdgcn_readfirstlane(at);
-    unsigned *const end = reinterpret_cast<unsigned *>(L.pt + n) - 1;
-#pragma unroll
-    for (int i = 0; i < kTaps; i++) {
-        if (rank[i] < 0 && k0 + i < s.K)
-            end[-(long)(at + __popcll(m[i] & ((1ull << lane) - 1)))] = (unsigned)((g * s.K + k0 + i) * s.M + b * s.P + p);
-        at += __popcll(m[i]);
-    }
 }
 
 // ---- the weights as matrix operands -----------------------------------------------------------------------------------
@@ -290,7 +347,7 @@ constexpr int kWaveLds = 32 * 128 + 3 * 32 * 64;
 D2C_DEV void lds_only_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 D2C_DEV void wave_fence() { asm volatile("" ::: "memory"); __builtin_amdgcn_wave_barrier(); }
 
-__global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs a, const int *__restrict__ seg_start, const int *__restrict__ seg_count)
+__global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs a, const int *__restrict__ seg_end, const int *__restrict__ seg_count)
 {
     const int lane = threadIdx.x & 63, h = lane >> 5, n = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
@@ -407,10 +464,10 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
     int r_lo, r_n;
     auto range = [&](int zi) INLINE {
         const int sg = brick_seg(a.d, bg, min(zi, zi_hi - 1), by, bx);
-        r_lo = seg_start[sg]; r_n = seg_count[sg];
+        r_lo = seg_end[sg]; r_n = seg_count[sg];
     };
     auto begin = [&](int zi) INLINE {
-        e_lo = __builtin_amdgcn_readfirstlane(r_lo); cnt = __builtin_amdgcn_readfirstlane(r_n);
+        cnt = __builtin_amdgcn_readfirstlane(r_n); e_lo = __builtin_amdgcn_readfirstlane(r_lo) - cnt;
         if (cnt > 0) {
             entry(0, e0, a0);
             entry(32, e1, a1);
@@ -551,7 +608,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
     // The planes whose sums hold infinities or NaN, and those above them, point by point (see above; lane = channel).
     for (int zi = max(bad_from, zi_lo); zi < zi_hi; zi++) {
         const int sg = brick_seg(a.d, bg, zi, by, bx);
-        const int lo = __builtin_amdgcn_readfirstlane(seg_start[sg]), np = __builtin_amdgcn_readfirstlane(seg_count[sg]);
+        const int np = __builtin_amdgcn_readfirstlane(seg_count[sg]), lo = __builtin_amdgcn_readfirstlane(seg_end[sg]) - np;
         for (int i = 0; i < np; i += 64) {
             const int e = lo + min(i + lane, np - 1);
             const uint4 q = a.L.pt[e];
@@ -589,7 +646,7 @@ struct BrickSampleArgs {
     long npoint;
     FastDiv dM, dKM;
 };
-__global__ void __launch_bounds__(64 * kMaxWaves, 4) brick_sample_kernel(BrickSampleArgs a, const int *__restrict__ seg_start, const int *__restrict__ seg_count)
+__global__ void __launch_bounds__(64 * kMaxWaves, 4) brick_sample_kernel(BrickSampleArgs a, const int *__restrict__ seg_end, const int *__restrict__ seg_count)
 {
     const int lane = threadIdx.x & 63, h = lane >> 5, n = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
@@ -672,7 +729,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 4) brick_sample_kernel(BrickSa
 
     auto range = [&](int zi, int &lo, int &cnt) INLINE {
         const int sg = brick_seg(a.d, bg, min(zi, zi_hi - 1), by, bx);
-        lo = __builtin_amdgcn_readfirstlane(seg_start[sg]); cnt = __builtin_amdgcn_readfirstlane(seg_count[sg]);
+        cnt = __builtin_amdgcn_readfirstlane(seg_count[sg]); lo = __builtin_amdgcn_readfirstlane(seg_end[sg]) - cnt;
     };
     uint4 e0, e1;
     float a0, a1;
@@ -776,19 +833,19 @@ brick_finish_kernel(TiledShape s, BrickLists L, const float2 *res, long nres, in
     const PointUnit un = point_unit(s, ngrp);
     const int k0 = un.k0, bg = un.bg, b = un.b, g = un.g, p = un.p;
     if (p >= s.P) return;
-    int at[kTaps];
-    float al[kTaps];
-    float2 mx[kTaps], zy[kTaps];
+    int at[kPassTaps];
+    float al[kPassTaps];
+    float2 mx[kPassTaps], zy[kPassTaps];
 #pragma unroll
-    for (int i = 0; i < kTaps; i++) {
+    for (int i = 0; i < kPassTaps; i++) {
         const int k = min(k0 + i, s.K - 1);
         at[i] = L.place[((long)bg * s.K + k) * s.P + p];
         al[i] = mask ? ld_auxT<AUX16>(mask, mask_index(s, b, g, k, p)) : 1.f;
     }
 #pragma unroll
-    for (int i = 0; i < kTaps; i++) brick_point_sums(res, nres, nset, at[i], mx[i], zy[i]);
+    for (int i = 0; i < kPassTaps; i++) brick_point_sums(res, nres, nset, at[i], mx[i], zy[i]);
 #pragma unroll
-    for (int i = 0; i < kTaps; i++) {
+    for (int i = 0; i < kPassTaps; i++) {
         const int k = k0 + i;
         if (k >= s.K) break;
         const bool in = at[i] >= 0;
@@ -856,11 +913,40 @@ long brick_nseg(const TiledShape &s)
 }
 long brick_points(const TiledShape &s) { return (long)s.N * s.G * s.K * s.P; }
 double brick_mean(const TiledShape &s) { return 9.0 * s.K * s.P / s.vol; }      // points per block, were all inside
+// Blocks that a workgroup of the sort counts in LDS: all of a sample and group, or what fits of those around its
+// positions, planes first, then rows (a point displaced out of the window costs a global addition of its own).
+constexpr int kSortSlots = 8192;
+SortWindow sort_window(const TiledShape &s, const BrickDims &d)
+{
+    SortWindow w{d.nz, d.nby, d.nbx, 0, 0, 0, 0, 0, 0, 0};
+    // A tile of 4 x 8 x 8 positions reaches fewer blocks than 64 positions of a few rows (filing 32x60x108: 122 us, 136).  With
+    // few tiles the taps of one are dealt to several workgroups (counting + filing 1024 -> 256 channels on 8x30x54: 20 + 32 us
+    // on 56 workgroups, 10 + 15 on 224; on four times as many as compute units no faster).
+    const int lz = s.Do >= 3 ? 2 : (s.Do >= 2 ? 1 : 0);
+    w.lx = 3; w.ly = 5 - lz;
+    w.ny = (s.Ho + (1 << w.ly) - 1) >> w.ly; w.nx = (s.Wo + (1 << w.lx) - 1) >> w.lx;
+    w.ntile = ((s.Do + (1 << lz) - 1) >> lz) * w.ny * w.nx;
+    w.taps = std::min(s.K, kSortTaps);
+    while (w.taps > kTapGroups && (long)w.ntile * s.N * s.G * ((s.K + w.taps - 1) / w.taps) < 256) w.taps = (w.taps + 1) / 2;
+    w.ngrp = (s.K + w.taps - 1) / w.taps;
+    const int least[3] = {(s.geo.kd - 1) * s.geo.dd + 9, ((s.geo.kh - 1) * s.geo.dh + 2) / 3 + 7, ((s.geo.kw - 1) * s.geo.dw + 2) / 3 + 7};
+    auto shrink = [](int &v, int lo, long others, int slots) {
+        if ((long)v * others > slots) v = (int)std::max<long>(std::min(v, lo), slots / others);
+    };
+    shrink(w.wz, least[0], (long)w.wy * w.wx, kSortSlots);
+    shrink(w.wy, least[1], (long)w.wz * w.wx, kSortSlots);
+    shrink(w.wx, least[2], (long)w.wz * w.wy, kSortSlots);
+    // (a kernel of great extent: whatever still fits)
+    shrink(w.wz, 1, (long)w.wy * w.wx, kSortSlots);
+    shrink(w.wy, 1, (long)w.wz * w.wx, kSortSlots);
+    shrink(w.wx, 1, (long)w.wz * w.wy, kSortSlots);
+    return w;
+}
 int brick_sets(const TiledShape &s) { return (s.cpg / 64 + kMaxWaves - 1) / kMaxWaves; }
 BrickLists brick_lists(const TiledShape &s, char *base)
 {
     const BrickWs w = d2c_brick_ws(s);
-    return BrickLists{(int *)(base + w.count), (int *)(base + w.count) + brick_nseg(s), (int *)(base + w.start), (int *)(base + w.place),
+    return BrickLists{(int *)(base + w.count), (int *)(base + w.count) + brick_nseg(s), (int *)(base + w.end), (int *)(base + w.place),
                       (uint4 *)(base + w.pt), (float *)(base + w.alpha)};
 }
 
@@ -880,8 +966,8 @@ BrickWs d2c_brick_ws(const TiledShape &s)
     const size_t n = (size_t)brick_points(s), nseg = (size_t)brick_nseg(s);
     BrickWs w;
     w.count = 0;                                                   // [nseg] counts, then the cursor and the number of points outside: one clear
-    w.start = d2c_align_up((nseg + 2) * 4);
-    w.place = w.start + d2c_align_up(nseg * 4);
+    w.end = d2c_align_up((nseg + 2) * 4);
+    w.place = w.end + d2c_align_up(nseg * 4);
     w.pt = w.place + d2c_align_up(n * 4);
     w.alpha = w.pt + d2c_align_up(n * 16);
     w.total = w.alpha + d2c_align_up(n * 4);
@@ -897,16 +983,14 @@ int d2c_brick_sort(const TiledShape &s, const void *off, const void *mask, void 
     const BrickLists L = brick_lists(s, (char *)ws);
     const int nseg = (int)brick_nseg(s);
     d2c_fill_zero(L.count, ((size_t)nseg + 2) * 4, st);
-    const int ngrp = (s.K + kTaps - 1) / kTaps;
-    const dim3 grid((unsigned)((long)((s.P + 255) / 256) * ngrp * s.N * s.G)), blk(256);
+    const SortWindow w = sort_window(s, d);
+    const size_t lds = ((size_t)w.wz * w.wy * w.wx + 1) * 4;
+    const dim3 grid((unsigned)((long)w.ntile * w.ngrp * s.N * s.G)), blk(kSortThreads);
     auto go = [&](auto A, auto Z) {
         constexpr bool A16 = decltype(A)::value, SZ = decltype(Z)::value;
-        if (brick_points(s) <= (brick_mean(s) < 128.0 ? 300000 : 64000))
-            hipLaunchKernelGGL((brick_count_few_kernel<A16, SZ>), dim3((unsigned)((long)((s.P + 255) / 256) * s.K * s.N * s.G)), blk, 0, st, s, d, L,
-                               off);
-        else hipLaunchKernelGGL((brick_count_kernel<A16, SZ>), grid, blk, 0, st, s, d, L, off, ngrp);
-        hipLaunchKernelGGL(brick_range_kernel, dim3((nseg + 255) / 256), blk, 0, st, L, nseg);
-        hipLaunchKernelGGL((brick_file_kernel<A16, SZ>), grid, blk, 0, st, s, d, L, off, mask, ngrp, brick_points(s));
+        hipLaunchKernelGGL((brick_count_kernel<A16, SZ>), grid, blk, lds, st, s, d, L, off, w);
+        hipLaunchKernelGGL(brick_range_kernel, dim3((nseg + 1023) / 1024), dim3(1024), 0, st, L, nseg);
+        hipLaunchKernelGGL((brick_file_kernel<A16, SZ>), grid, blk, lds, st, s, d, L, off, mask, w, brick_points(s));
     };
     if (s.adt == D2C_BF16) {
         if (s.ss.on) go(std::true_type{}, std::true_type{});
@@ -945,7 +1029,7 @@ int d2c_brick_grad(const TiledShape &s, const void *xcl, const void *gcol, const
     const unsigned grid = (unsigned)(cols * a.nzr);
     {
         D2cProfScope prof(D2C_PROF_BWD_AUX, st, "brick_grad_kernel");
-        hipLaunchKernelGGL(brick_grad_kernel, dim3(grid), dim3(64 * nw), nw * kWaveLds + (nw > 1 ? nw * 1024 : 0), st, a, a.L.start, a.L.count);
+        hipLaunchKernelGGL(brick_grad_kernel, dim3(grid), dim3(64 * nw), nw * kWaveLds + (nw > 1 ? nw * 1024 : 0), st, a, a.L.end, a.L.count);
         if (int rc = d2c_check_launch("brick_grad_kernel")) return rc;
     }
     if (!a.res) return D2C_OK;
@@ -956,7 +1040,7 @@ int d2c_brick_grad(const TiledShape &s, const void *xcl, const void *gcol, const
         hipLaunchKernelGGL(fin, dim3((s.P + 63) / 64, s.N), dim3(256), 0, st, s, a.L, a.res, a.nres, a.nset, mask, raw, goff, gmask);
     } else {
         auto fin = a16 ? &brick_finish_kernel<true> : &brick_finish_kernel<false>;
-        const int ngrp = (s.K + kTaps - 1) / kTaps;
+        const int ngrp = (s.K + kPassTaps - 1) / kPassTaps;
         hipLaunchKernelGGL(fin, dim3((unsigned)((long)((s.P + 255) / 256) * ngrp * s.N * s.G)), dim3(256), 0, st, s, a.L, a.res, a.nres, a.nset, mask,
                            goff, gmask, ngrp);
     }
@@ -982,6 +1066,6 @@ int d2c_brick_columns(const TiledShape &s, const void *xcl, void *col, int rows,
     a.npoint = brick_points(s);
     a.nzero = (int)std::min<long>(2048, (a.npoint + 511) / 512) / nw + 1;
     D2cProfScope prof(D2C_PROF_SAMPLE, st, "brick_sample_kernel");
-    hipLaunchKernelGGL(brick_sample_kernel, dim3((unsigned)(cols * a.nzr + a.nzero)), dim3(64 * nw), 0, st, a, a.L.start, a.L.count);
+    hipLaunchKernelGGL(brick_sample_kernel, dim3((unsigned)(cols * a.nzr + a.nzero)), dim3(64 * nw), 0, st, a, a.L.end, a.L.count);
     return d2c_check_launch("brick_sample_kernel");
 }

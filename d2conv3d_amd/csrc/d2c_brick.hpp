@@ -9,13 +9,13 @@ struct BrickDims {
 struct BrickLists {
     int *count;              // points per block
     int *cursor;             // entries given out, then: points outside the volume
-    int *start;              // first entry of a block
+    int *end;                // end of a block's entries (they begin `count` before it)
     int *place;              // [n * G + g][tap][p]: a point's entry, -1: no corner inside the volume
     uint4 *pt;               // byte offset of the point's row of 64 channels | its base voxel in the block (y | x << 2); fractions along y, x, z
     float *alpha;            // modulation
 };
 struct BrickWs {
-    size_t count, start, place, pt, alpha, total;     // the sorted points
+    size_t count, end, place, pt, alpha, total;     // the sorted points
     size_t res_bytes;                                 // per-point sums of d2c_brick_grad
 };
 bool d2c_brick_supported(const TiledShape &s, int dtype);
