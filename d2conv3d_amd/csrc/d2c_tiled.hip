@@ -62,6 +62,11 @@ size_t d2c_bwd_goutp_bytes(const TiledShape &s, int dtype);
 template <typename T> int d2c_tiled_unpack_gx(const TiledShape &s, const float *gxcl, void *gx, hipStream_t st);
 template <typename T> int d2c_tiled_bias_grad(const TiledShape &s, const void *gout, void *gb, hipStream_t st);
 
+bool d2c_conv1d_bwd_use(const TiledShape &s, int dtype);
+size_t d2c_conv1d_bwd_ws(const TiledShape &s, int dtype);
+template <typename T>
+int d2c_conv1d_bwd(const TiledShape &s, const void *gout, const void *x, const void *off, const void *mask, const void *w, void *gx,
+                   void *goff, void *gmask, void *gw, void *gb, void *ws, hipStream_t st);
 bool d2c_depthwise_supported(const TiledShape &s);
 template <typename T>
 int d2c_depthwise_forward(const TiledShape &s, const void *xcl, const void *off, const void *mask, const void *wt,
@@ -1006,7 +1011,8 @@ size_t d2c_tiled1d_forward_ws(const d2c_conv1d_desc &q1)
 size_t d2c_tiled1d_backward_ws(const d2c_conv1d_desc &q1)
 {
     const d2c_conv3d_desc q = as_3d(q1);
-    return bwd_ws(q, tiled_shape(q, 1, 0)).total;
+    const TiledShape s = tiled_shape(q, 1, 0);
+    return d2c_conv1d_bwd_use(s, q.dtype) ? d2c_conv1d_bwd_ws(s, q.dtype) : bwd_ws(q, s).total;
 }
 int d2c_tiled1d_forward(const d2c_conv1d_desc &q1, const void *x, const void *off, const void *mask, const void *w,
                         const void *bias, void *out, void *ws, hipStream_t st)
@@ -1020,6 +1026,11 @@ int d2c_tiled1d_backward(const d2c_conv1d_desc &q1, const void *gout, const void
                          void *ws, hipStream_t st)
 {
     const d2c_conv3d_desc q = as_3d(q1);
+    const TiledShape s = tiled_shape(q, 1, q1.reference_quirks);
+    if (!mask) gmask = nullptr;
+    if (d2c_conv1d_bwd_use(s, q.dtype))
+        return q.dtype == D2C_BF16 ? d2c_conv1d_bwd<bf16_t>(s, gout, x, off, mask, w, gx, goff, gmask, gw, gb, ws, st)
+                                   : d2c_conv1d_bwd<float>(s, gout, x, off, mask, w, gx, goff, gmask, gw, gb, ws, st);
     if (q.dtype == D2C_BF16)
         return backward_t<bf16_t>(q, gout, x, off, mask, w, gx, goff, gmask, gw, gb, ws, st, 1, q1.reference_quirks);
     return backward_t<float>(q, gout, x, off, mask, w, gx, goff, gmask, gw, gb, ws, st, 1, q1.reference_quirks);
