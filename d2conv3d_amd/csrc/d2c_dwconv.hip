@@ -22,7 +22,7 @@
 //   grad_weight : gw[co,k]      = sum_{n,o} gout[n,co,o] * x[n, co/m, o*s - p + k*d]   (registers, wavefront and
 //                                  workgroup reduction, one atomic per workgroup and tap into a scratch array)
 //   grad_bias   : gb[co]        = sum_{n,o} gout[n,co,o]
-#include "d2c_common.hpp"
+#include "d2c_mma.hpp"
 
 namespace {
 
@@ -395,9 +395,10 @@ __global__ void __launch_bounds__(kThreadsDw) dwc_bias_grad_kernel(DwcShape s, c
 }
 
 // ---------------------------------------------------------------- marching kernels
-// A workgroup = one (sample, channel), kTY * kMR rows, kTX * kVW columns, a range of planes.  What bounds them is memory:
-// 2x256x8x56x56 float moves 103 MB forward, 154 MB backward (20 and 30 us at the rate of a large copy); with a row of
-// nine segments read per output row (the kernels above) forward took 48 us, backward 66 + 102 us and three small launches.
+// A workgroup = one (sample, channel), kTY * kMR rows, kTX * kVW columns, a range of planes.  What bounds them is the vector
+// ALU (27 and 54 products to an element at a quarter of the lanes per clock), then memory: 2x256x8x56x56 float moves 103 MB
+// forward, 154 MB backward (20 and 30 us at the rate of a large copy) and takes 24 and 46.  With all taps of every plane it took 30
+// and 59; rows of any width are read in vectors (2x128x8x60x107: 48 and 76 us element by element, 30 and 63).
 constexpr int kMR = 2;                          // rows per thread
 constexpr int kMTaps = 28;                      // 27 taps and the bias
 struct MarchTiles {
@@ -408,8 +409,9 @@ MarchTiles march_tiles(const d2c_dwconv3d_desc &q)
     MarchTiles t;
     t.ty = (q.H + kTY * kMR - 1) / (kTY * kMR); t.tx = (q.W + kTX * kVW - 1) / (kTX * kVW);
     t.zlen = q.D;
-    // (a range reads two planes more than it has: no shorter than 4 for the sake of more workgroups)
-    while (t.zlen > 4 && (long)q.N * q.C * t.ty * t.tx * ((q.D + t.zlen - 1) / t.zlen) < 2048) t.zlen = (t.zlen + 1) / 2;
+    // (a range reads two planes more than it has: shorter than 8 for the sake of 1024 workgroups only, never than 4.  Forward +
+    // backward, us, float32: 2x256x8x56x56 in one range 72, in two 80; 1x64x32x112x112 in two 150, in four 141)
+    while (t.zlen > 4 && (long)q.N * q.C * t.ty * t.tx * ((q.D + t.zlen - 1) / t.zlen) < (t.zlen > 8 ? 2048 : 1024)) t.zlen = (t.zlen + 1) / 2;
     t.nz = (q.D + t.zlen - 1) / t.zlen;
     return t;
 }
@@ -418,6 +420,8 @@ bool march_ok(const d2c_dwconv3d_desc &q)
     return q.dtype != D2C_F64 && q.Cout == q.C && q.kd == 3 && q.kh == 3 && q.kw == 3 && q.sd == 1 && q.sh == 1 && q.sw == 1 &&
            q.pd == 1 && q.ph == 1 && q.pw == 1 && q.dd == 1 && q.dh == 1 && q.dw == 1;
 }
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned short u16x4_any __attribute__((ext_vector_type(4), aligned(2)));
 // kVW elements of a row of `width` from x0 on, zeros outside it.  VEC: rows kVW-aligned in memory, whole groups.
 template <typename ST, bool VEC> D2C_DEV void march_load(const ST *row, int x0, int width, bool ok, float *m)
 {
@@ -434,8 +438,21 @@ template <typename ST, bool VEC> D2C_DEV void march_load(const ST *row, int x0, 
             }
         }
     } else {
+        m[0] = m[1] = m[2] = m[3] = 0.f;
+        if (ok && x0 + kVW <= width) {
+            // (one load all the same, of a type that says how it is aligned)
+            if constexpr (sizeof(ST) == 4) {
+                const f32x4_any t = *reinterpret_cast<const f32x4_any *>(row + x0);
+                m[0] = t[0]; m[1] = t[1]; m[2] = t[2]; m[3] = t[3];
+            } else {
+                const u16x4_any t = *reinterpret_cast<const u16x4_any *>(row + x0);
+                m[0] = bf16_to_f32(t[0]); m[1] = bf16_to_f32(t[1]); m[2] = bf16_to_f32(t[2]); m[3] = bf16_to_f32(t[3]);
+            }
+        } else if (ok && x0 < width) {
 #pragma unroll
-        for (int i = 0; i < kVW; i++) m[i] = (ok && x0 + i < width) ? ldv<ST>(row, x0 + i) : 0.f;
+            for (int i = 0; i < kVW - 1; i++)
+                if (x0 + i < width) m[i] = ldv<ST>(row, x0 + i);
+        }
     }
 }
 template <typename ST, bool VEC> D2C_DEV void march_store(ST *row, int x0, int width, const float *m)
@@ -443,11 +460,16 @@ template <typename ST, bool VEC> D2C_DEV void march_store(ST *row, int x0, int w
     if constexpr (VEC) {
         if (x0 >= width) return;
         if constexpr (sizeof(ST) == 4) *reinterpret_cast<float4 *>(row + x0) = make_float4(m[0], m[1], m[2], m[3]);
-        else *reinterpret_cast<uint2 *>(row + x0) = make_uint2(f32_to_bf16(m[0]) | ((uint32_t)f32_to_bf16(m[1]) << 16),
-                                                               f32_to_bf16(m[2]) | ((uint32_t)f32_to_bf16(m[3]) << 16));
+        else *reinterpret_cast<uint2 *>(row + x0) = make_uint2(pack_bf16x2(m[0], m[1]), pack_bf16x2(m[2], m[3]));
+    } else if (x0 + kVW <= width) {
+        if constexpr (sizeof(ST) == 4) *reinterpret_cast<f32x4_any *>(row + x0) = f32x4_any{m[0], m[1], m[2], m[3]};
+        else {
+            const uint32_t a = pack_bf16x2(m[0], m[1]), b = pack_bf16x2(m[2], m[3]);
+            *reinterpret_cast<u16x4_any *>(row + x0) = u16x4_any{(unsigned short)a, (unsigned short)(a >> 16), (unsigned short)b, (unsigned short)(b >> 16)};
+        }
     } else {
 #pragma unroll
-        for (int i = 0; i < kVW; i++)
+        for (int i = 0; i < kVW - 1; i++)
             if (x0 + i < width) stv<ST>(row, x0 + i, m[i]);
     }
 }
@@ -456,7 +478,8 @@ struct MarchRows {
     float m[kMR + 2][kVW];
     float l[kMR + 2], r[kMR + 2];               // the elements beside the tile (its first and last lane)
 };
-template <typename ST, bool VEC>
+// (EDGE: more than one tile along x)
+template <typename ST, bool VEC, bool EDGE>
 D2C_DEV void march_rows(const ST *plane, bool plane_ok, int y0, int x0, int H, int W, MarchRows &o)
 {
     const int tx = threadIdx.x % kTX;
@@ -466,19 +489,22 @@ D2C_DEV void march_rows(const ST *plane, bool plane_ok, int y0, int x0, int H, i
         const bool ok = plane_ok && y >= 0 && y < H;
         const ST *row = plane + (long)(ok ? y : 0) * W;
         march_load<ST, VEC>(row, x0, W, ok, o.m[j]);
-        o.l[j] = (ok && tx == 0 && x0 > 0) ? ldv<ST>(row, x0 - 1) : 0.f;
-        o.r[j] = (ok && tx == kTX - 1 && x0 + kVW < W) ? ldv<ST>(row, x0 + kVW) : 0.f;
+        if constexpr (EDGE) {
+            o.l[j] = (ok && tx == 0 && x0 > 0) ? ldv<ST>(row, x0 - 1) : 0.f;
+            o.r[j] = (ok && tx == kTX - 1 && x0 + kVW < W) ? ldv<ST>(row, x0 + kVW) : 0.f;
+        }
     }
 }
 // ... and row j with its neighbours along x: v[i] is element x0 - 1 + i.  (The 16 lanes of a row are one DPP row.)
-D2C_DEV void march_segment(const MarchRows &o, int j, float *v)
+template <bool EDGE> D2C_DEV void march_segment(const MarchRows &o, int j, float *v)
 {
     const int tx = threadIdx.x % kTX;
     const float left = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(o.m[j][3]), 0x111, 0xF, 0xF, true));    // row_shr 1
     const float right = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(o.m[j][0]), 0x101, 0xF, 0xF, true));   // row_shl 1
-    v[0] = tx == 0 ? o.l[j] : left;
+    // (a lane without a neighbour in its row of 16 gets zero)
+    v[0] = EDGE && tx == 0 ? o.l[j] : left;
     v[1] = o.m[j][0]; v[2] = o.m[j][1]; v[3] = o.m[j][2]; v[4] = o.m[j][3];
-    v[5] = tx == kTX - 1 ? o.r[j] : right;
+    v[5] = EDGE && tx == kTX - 1 ? o.r[j] : right;
 }
 struct MarchPos {
     int nc, c, y0, x0, z_lo, z_hi, tile;
@@ -498,12 +524,15 @@ D2C_DEV MarchPos march_pos(const d2c_dwconv3d_desc &q, const MarchTiles &t)
     return p;
 }
 
-template <typename ST, bool VEC>
+// A plane of input touches three planes of results; those of another range are not worked on (the planes in front of and
+// behind a range of four, with all 27 taps, were a third of the instructions), nor are rows by wavefronts below the volume.
+template <typename ST, bool VEC, bool EDGE>
 __global__ void __launch_bounds__(kThreadsDw) dwc_march_fwd_kernel(d2c_dwconv3d_desc q, MarchTiles t, const ST *__restrict__ x,
                                                                    const ST *__restrict__ w, const ST *__restrict__ bias,
                                                                    ST *__restrict__ out)
 {
     const MarchPos p = march_pos(q, t);
+    if (__builtin_amdgcn_readfirstlane(p.y0) >= q.H) return;
     const long HW = (long)q.H * q.W;
     const ST *xc = x + (long)p.nc * q.D * HW;
     ST *oc = out + (long)p.nc * q.D * HW;
@@ -515,25 +544,28 @@ __global__ void __launch_bounds__(kThreadsDw) dwc_march_fwd_kernel(d2c_dwconv3d_
 #pragma unroll
     for (int i = 0; i < 3 * kMR * kVW; i++) (&acc[0][0][0])[i] = bv;
     MarchRows cur, nxt;
-    march_rows<ST, VEC>(xc + max(p.z_lo - 1, 0) * HW, p.z_lo > 0, p.y0, p.x0, q.H, q.W, cur);
+    march_rows<ST, VEC, EDGE>(xc + max(p.z_lo - 1, 0) * HW, p.z_lo > 0, p.y0, p.x0, q.H, q.W, cur);
     for (int z = p.z_lo - 1; z <= p.z_hi; z++) {
-        if (z < p.z_hi) march_rows<ST, VEC>(xc + min(z + 1, q.D - 1) * HW, z + 1 < q.D, p.y0, p.x0, q.H, q.W, nxt);
+        if (z < p.z_hi) march_rows<ST, VEC, EDGE>(xc + min(z + 1, q.D - 1) * HW, z + 1 < q.D, p.y0, p.x0, q.H, q.W, nxt);
+        float v[kMR + 2][kVW + 2];
 #pragma unroll
-        for (int j = 0; j < kMR + 2; j++) {
-            float v[kVW + 2];
-            march_segment(cur, j, v);
+        for (int j = 0; j < kMR + 2; j++) march_segment<EDGE>(cur, j, v[j]);
 #pragma unroll
-            for (int r = 0; r < kMR; r++) {
-                const int ky = j - r;           // row y0 + r reads rows y0 + r - 1 + ky
-                if (ky < 0 || ky > 2) continue;
+        for (int kz = 0; kz < 3; kz++) {
+            const int zo = z + 1 - kz;          // the plane that tap kz of this one adds to
+            if (zo < p.z_lo || zo >= p.z_hi) continue;
 #pragma unroll
-                for (int kz = 0; kz < 3; kz++)
+            for (int j = 0; j < kMR + 2; j++)
+#pragma unroll
+                for (int r = 0; r < kMR; r++) {
+                    const int ky = j - r;       // row y0 + r reads rows y0 + r - 1 + ky
+                    if (ky < 0 || ky > 2) continue;
 #pragma unroll
                     for (int kx = 0; kx < 3; kx++)
 #pragma unroll
                         for (int i = 0; i < kVW; i++)
-                            acc[2 - kz][r][i] = fmaf(wv[(kz * 3 + ky) * 3 + kx], v[i + kx], acc[2 - kz][r][i]);
-            }
+                            acc[2 - kz][r][i] = fmaf(wv[(kz * 3 + ky) * 3 + kx], v[j][i + kx], acc[2 - kz][r][i]);
+                }
         }
         if (z - 1 >= p.z_lo) {
 #pragma unroll
@@ -549,8 +581,8 @@ __global__ void __launch_bounds__(kThreadsDw) dwc_march_fwd_kernel(d2c_dwconv3d_
 }
 
 // part[tile][channel][kMTaps]: the workgroup's sums of grad_weight and grad_bias (or NULL); gx or NULL
-template <typename ST, bool VEC>
-__global__ void __launch_bounds__(kThreadsDw) dwc_march_bwd_kernel(d2c_dwconv3d_desc q, MarchTiles t, const ST *__restrict__ gout,
+template <typename ST, bool VEC, bool EDGE>
+__global__ void __launch_bounds__(kThreadsDw, 3) dwc_march_bwd_kernel(d2c_dwconv3d_desc q, MarchTiles t, const ST *__restrict__ gout,
                                                                    const ST *__restrict__ x, const ST *__restrict__ w,
                                                                    ST *__restrict__ gx, float *__restrict__ part)
 {
@@ -566,7 +598,7 @@ __global__ void __launch_bounds__(kThreadsDw) dwc_march_bwd_kernel(d2c_dwconv3d_
     for (int i = 0; i < 3 * kMR * kVW; i++) (&acc[0][0][0])[i] = (&xv[0][0][0])[i] = 0.f;
 #pragma unroll
     for (int k = 0; k < kMTaps; k++) gw[k] = 0.f;
-    // (input outside the range is another workgroup's: zero here)
+    // (input outside the range is another workgroup's)
     auto load_x = [&](int z, float (*o)[kVW]) {
 #pragma unroll
         for (int r = 0; r < kMR; r++)
@@ -575,35 +607,44 @@ __global__ void __launch_bounds__(kThreadsDw) dwc_march_bwd_kernel(d2c_dwconv3d_
     };
     MarchRows cur, nxt;
     float xn[kMR][kVW];
-    march_rows<ST, VEC>(gc + max(p.z_lo - 1, 0) * HW, p.z_lo > 0, p.y0, p.x0, q.H, q.W, cur);
-    load_x(p.z_lo, xv[2]);
-    for (int z = p.z_lo - 1; z <= p.z_hi; z++) {
+    // (a wavefront below the volume only takes part in the sums)
+    const int z_end = __builtin_amdgcn_readfirstlane(p.y0) < q.H ? p.z_hi : p.z_lo - 2;
+    if (z_end >= p.z_lo) {
+        march_rows<ST, VEC, EDGE>(gc + max(p.z_lo - 1, 0) * HW, p.z_lo > 0, p.y0, p.x0, q.H, q.W, cur);
+        load_x(p.z_lo, xv[2]);
+    }
+    for (int z = p.z_lo - 1; z <= z_end; z++) {
         if (z < p.z_hi) {
-            march_rows<ST, VEC>(gc + min(z + 1, q.D - 1) * HW, z + 1 < q.D, p.y0, p.x0, q.H, q.W, nxt);
+            march_rows<ST, VEC, EDGE>(gc + min(z + 1, q.D - 1) * HW, z + 1 < q.D, p.y0, p.x0, q.H, q.W, nxt);
             load_x(z + 2, xn);
+        }
+        float v[kMR + 2][kVW + 2];
+#pragma unroll
+        for (int j = 0; j < kMR + 2; j++) {
+            march_segment<EDGE>(cur, j, v[j]);
+            if (j >= 1 && j <= kMR && z >= p.z_lo && z < p.z_hi) gw[27] += (v[j][1] + v[j][2]) + (v[j][3] + v[j][4]);
         }
         // grad_input plane z' takes tap kz of grad_out plane z = z' + 1 - kz: z' = z - 1 + kz; and grad_weight the same pair
 #pragma unroll
-        for (int j = 0; j < kMR + 2; j++) {
-            float v[kVW + 2];
-            march_segment(cur, j, v);
-            if (j >= 1 && j <= kMR && z >= p.z_lo && z < p.z_hi) gw[27] += (v[1] + v[2]) + (v[3] + v[4]);
+        for (int kz = 0; kz < 3; kz++) {
+            const int zo = z - 1 + kz;
+            if (zo < p.z_lo || zo >= p.z_hi) continue;
 #pragma unroll
-            for (int r = 0; r < kMR; r++) {
-                const int ky = r + 2 - j;       // row y0 + r takes tap ky from row y0 + r + 1 - ky
-                if (ky < 0 || ky > 2) continue;
+            for (int j = 0; j < kMR + 2; j++)
 #pragma unroll
-                for (int kz = 0; kz < 3; kz++)
+                for (int r = 0; r < kMR; r++) {
+                    const int ky = r + 2 - j;   // row y0 + r takes tap ky from row y0 + r + 1 - ky
+                    if (ky < 0 || ky > 2) continue;
 #pragma unroll
                     for (int kx = 0; kx < 3; kx++) {
                         const int k = (kz * 3 + ky) * 3 + kx;
 #pragma unroll
                         for (int i = 0; i < kVW; i++) {
-                            acc[kz][r][i] = fmaf(wv[k], v[i + 2 - kx], acc[kz][r][i]);
-                            gw[k] = fmaf(xv[kz][r][i], v[i + 2 - kx], gw[k]);
+                            acc[kz][r][i] = fmaf(wv[k], v[j][i + 2 - kx], acc[kz][r][i]);
+                            gw[k] = fmaf(xv[kz][r][i], v[j][i + 2 - kx], gw[k]);
                         }
                     }
-            }
+                }
         }
         if (gx && z - 1 >= p.z_lo) {
 #pragma unroll
@@ -711,12 +752,9 @@ int forward_t(const d2c_dwconv3d_desc &q, const void *x, const void *w, const vo
         if (march_ok(q)) {
             const MarchTiles t = march_tiles(q);
             const dim3 grid((unsigned)(q.N * q.C), (unsigned)(t.ty * t.tx * t.nz));
-            if (vec_ok<ST>(q, x, out))
-                hipLaunchKernelGGL((dwc_march_fwd_kernel<ST, true>), grid, dim3(kThreadsDw), 0, st, q, t, (const ST *)x, (const ST *)w,
-                                   (const ST *)bias, (ST *)out);
-            else
-                hipLaunchKernelGGL((dwc_march_fwd_kernel<ST, false>), grid, dim3(kThreadsDw), 0, st, q, t, (const ST *)x, (const ST *)w,
-                                   (const ST *)bias, (ST *)out);
+            auto kern = vec_ok<ST>(q, x, out) ? (t.tx > 1 ? &dwc_march_fwd_kernel<ST, true, true> : &dwc_march_fwd_kernel<ST, true, false>)
+                                              : (t.tx > 1 ? &dwc_march_fwd_kernel<ST, false, true> : &dwc_march_fwd_kernel<ST, false, false>);
+            hipLaunchKernelGGL(kern, grid, dim3(kThreadsDw), 0, st, q, t, (const ST *)x, (const ST *)w, (const ST *)bias, (ST *)out);
             return d2c_check_launch("dwc_march_fwd_kernel");
         }
     }
@@ -754,7 +792,8 @@ int backward_t(const d2c_dwconv3d_desc &q, const void *gout, const void *x, cons
             const dim3 grid((unsigned)(q.N * q.C), (unsigned)(t.ty * t.tx * t.nz));
             float *part = gw || gb ? (float *)ws : nullptr;
             auto kern = vec_ok<ST>(q, gout, x) && reinterpret_cast<uintptr_t>(gx) % (kVW * sizeof(ST)) == 0
-                            ? &dwc_march_bwd_kernel<ST, true> : &dwc_march_bwd_kernel<ST, false>;
+                            ? (t.tx > 1 ? &dwc_march_bwd_kernel<ST, true, true> : &dwc_march_bwd_kernel<ST, true, false>)
+                            : (t.tx > 1 ? &dwc_march_bwd_kernel<ST, false, true> : &dwc_march_bwd_kernel<ST, false, false>);
             hipLaunchKernelGGL(kern, grid, dim3(kThreadsDw), 0, st, q, t, (const ST *)gout, (const ST *)x, (const ST *)w, (ST *)gx, part);
             if (int rc = d2c_check_launch("dwc_march_bwd_kernel")) return rc;
             if (!part) return D2C_OK;
