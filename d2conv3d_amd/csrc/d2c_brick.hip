@@ -975,14 +975,20 @@ BrickWs d2c_brick_ws(const TiledShape &s)
     return w;
 }
 
-// Sorts the points.
-int d2c_brick_sort(const TiledShape &s, const void *off, const void *mask, void *ws, hipStream_t st)
+// What has to be zero in front of the sort.
+void *d2c_brick_zero(const TiledShape &s, void *ws, size_t *bytes)
+{
+    *bytes = ((size_t)brick_nseg(s) + 2) * 4;
+    return (char *)ws + d2c_brick_ws(s).count;
+}
+// Sorts the points (`cleared`: d2c_brick_zero() has been).
+int d2c_brick_sort(const TiledShape &s, const void *off, const void *mask, void *ws, hipStream_t st, bool cleared)
 {
     D2cProfScope prof(D2C_PROF_PACK, st);
     const BrickDims d = brick_dims(s);
     const BrickLists L = brick_lists(s, (char *)ws);
     const int nseg = (int)brick_nseg(s);
-    d2c_fill_zero(L.count, ((size_t)nseg + 2) * 4, st);
+    if (!cleared) d2c_fill_zero(L.count, ((size_t)nseg + 2) * 4, st);
     const SortWindow w = sort_window(s, d);
     const size_t lds = ((size_t)w.wz * w.wy * w.wx + 1) * 4;
     const dim3 grid((unsigned)((long)w.ntile * w.ngrp * s.N * s.G)), blk(kSortThreads);
@@ -1002,7 +1008,7 @@ int d2c_brick_sort(const TiledShape &s, const void *off, const void *mask, void 
     return d2c_check_launch("brick_file_kernel");
 }
 
-// `gxcl` (cleared here), `goff` (size-map source: the gradient of the raw map `raw`) and `gmask` may be NULL.
+// `gxcl` (cleared), `goff` (size-map source: the gradient of the raw map `raw`) and `gmask` may be NULL.
 int d2c_brick_grad(const TiledShape &s, const void *xcl, const void *gcol, const void *mask, const void *raw, float *gxcl,
                    void *goff, void *gmask, const void *lists, void *res, hipStream_t st)
 {
@@ -1014,10 +1020,6 @@ int d2c_brick_grad(const TiledShape &s, const void *xcl, const void *gcol, const
     a.nres = (long)(d2c_align_up((size_t)n * 16) / 16);
     a.G = s.G; a.cpc = s.cpg / 64; a.Cin = s.Cin; a.D = s.D; a.H = s.H; a.W = s.W; a.vol = s.vol;
     a.chunk_rows = (long)s.K * s.M;
-    if (gxcl) {
-        D2cProfScope prof(D2C_PROF_PACK, st);
-        d2c_fill_zero(gxcl, (size_t)s.N * s.vol * s.Cin * sizeof(float), st);
-    }
     a.nset = brick_sets(s);
     const int nw = (a.cpc + a.nset - 1) / a.nset;
     // enough workgroups to fill the chip several times over; a range of z costs one more plane than it has bases

@@ -20,7 +20,8 @@ struct BrickWs {
 };
 bool d2c_brick_supported(const TiledShape &s, int dtype);
 BrickWs d2c_brick_ws(const TiledShape &s);
-int d2c_brick_sort(const TiledShape &s, const void *off, const void *mask, void *ws, hipStream_t st);
+void *d2c_brick_zero(const TiledShape &s, void *ws, size_t *bytes);
+int d2c_brick_sort(const TiledShape &s, const void *off, const void *mask, void *ws, hipStream_t st, bool cleared = false);
 int d2c_brick_grad(const TiledShape &s, const void *xcl, const void *gcol, const void *mask, const void *raw, float *gxcl,
                    void *goff, void *gmask, const void *lists, void *res, hipStream_t st);
 int d2c_brick_columns(const TiledShape &s, const void *xcl, void *col, int rows, const void *lists, hipStream_t st);

@@ -701,10 +701,10 @@ __global__ void __launch_bounds__(kThreads, 1) grad_col_kernel(GradColArgs a)
     for (int pb = 0; pb < PB; pb++) asm volatile("" : "+v"(fa[0][pb]));
     wait_vm<0>();
 }
-// W[o][c][tap] -> the operand order above: a thread makes one vector of eight o of a (channel, tap)
-__global__ void __launch_bounds__(256) grad_col_weights_kernel(const bf16_t *w, uint4 *wt, int Cout, int Cin, int K, FastDiv dK, int S)
+// W[o][c][tap] -> the operand order above: a thread makes vector v of eight o of (channel, tap) e
+D2C_DEV void grad_col_weight(const bf16_t *w, uint4 *wt, int Cout, int Cin, int K, const FastDiv &dK, int S, int e, int v)
 {
-    const int e = blockIdx.x * 256 + threadIdx.x, v = blockIdx.y, CK = Cin * K;
+    const int CK = Cin * K;
     if (e >= CK) return;
     alignas(16) bf16_t t[8];
 #pragma unroll
@@ -869,24 +869,32 @@ __global__ void __launch_bounds__(256) conv_weight_finish_kernel(const float *pa
 
 // ============================================================ operand orders, one launch per direction
 struct ConvPrepArgs {
-    // input -> channels-last rows, then a row of zeros
+    // input -> channels-last rows, then zeros
     const bf16_t *x;
     bf16_t *xcl;
-    int C, vol, N, nbx, nby, nblk_x, wide;
+    int C, vol, N, nbx, nby, nblk_x, wide, zrow_words;
     // weights: column tiles [step][tile][NT][KC]; back: the transposed product (columns = input channels)
     const bf16_t *w;
     uint4 *wt;
     int Cout, Cin, K, NT, KC, nchunk, nct, back, nblk_w;
     long nvec;
-    // grad_out -> channels-last rows of Cp channels (+ a row of zeros) and fragments
+    // grad_out -> channels-last rows of Cp channels (+ a row of zeros) and fragments of tiles of 64 << gp_wide positions
     const bf16_t *gout;
     bf16_t *gcl;
     uint4 *gp;
-    int Cp, OBP, P, M, ngt, ngc, nblk_g, gwide;
+    int Cp, OBP, P, M, ngt, ngc, nblk_g, gwide, gp_wide;
     FastDiv dP;
     // bias gradient
     bf16_t *gb;
     int nblk_b;
+    // weights of grad_col_kernel
+    uint4 *gcw;
+    int gcS, ngcw, nblk_gcw;          // steps; workgroups per vector, in all
+    FastDiv dK;
+    // ranges of the workspace to clear
+    uint32_t *zero[2];
+    size_t zwords[2];
+    int nblk_z;
 };
 // eight positions at a time: whole in a sample, and aligned
 inline int wide_gout(const void *gout, int P) { return P % 8 == 0 && reinterpret_cast<uintptr_t>(gout) % 16 == 0; }
@@ -902,7 +910,7 @@ __global__ void __launch_bounds__(256) conv_prepare_kernel(ConvPrepArgs a)
         const int v0 = bx * 64, c0 = by * 64;
         const bf16_t *xb = a.x + (long)n * a.C * a.vol;
         bf16_t *ob = a.xcl + (long)n * a.C * a.vol;
-        if (b == 0 && threadIdx.x < 128) reinterpret_cast<unsigned *>(a.xcl + (long)a.N * a.C * a.vol)[threadIdx.x] = 0u;
+        if (b == 0 && (int)threadIdx.x < a.zrow_words) reinterpret_cast<unsigned *>(a.xcl + (long)a.N * a.C * a.vol)[threadIdx.x] = 0u;
         if (a.wide) {
             for (int i = threadIdx.x; i < 512; i += 256) {
                 const int c = c0 + i / 8, v = v0 + (i % 8) * 8;
@@ -987,7 +995,7 @@ __global__ void __launch_bounds__(256) conv_prepare_kernel(ConvPrepArgs a)
             for (int i = threadIdx.x; i < 512; i += 256) {
                 const int ln = i & 63, kg = (i >> 6) & 3, ob = i >> 8;
                 if (gc * 2 + ob < a.OBP)
-                    a.gp[(((long)gt * a.OBP + gc * 2 + ob) * 4 + kg) * 64 + ln] =
+                    a.gp[((((long)(gt >> a.gp_wide) * a.OBP + gc * 2 + ob) * (4 << a.gp_wide)) + (gt & ((1 << a.gp_wide) - 1)) * 4 + kg) * 64 + ln] =
                         *reinterpret_cast<const uint4 *>(s_t + (ob * 32 + (ln & 31)) * GS + kg * 16 + (ln >> 5) * 8);
             }
         }
@@ -1006,7 +1014,23 @@ __global__ void __launch_bounds__(256) conv_prepare_kernel(ConvPrepArgs a)
         return;
     }
     b -= a.nblk_g;
-    if (b < a.nblk_b) bias_grad_body<bf16_t, 256>(a.gout, a.gb, a.N, a.Cout, a.P, b);
+    if (b < a.nblk_b) {
+        bias_grad_body<bf16_t, 256>(a.gout, a.gb, a.N, a.Cout, a.P, b);
+        return;
+    }
+    b -= a.nblk_b;
+    if (b < a.nblk_gcw) {
+        grad_col_weight(a.w, a.gcw, a.Cout, a.Cin, a.K, a.dK, a.gcS, b % a.ngcw * 256 + threadIdx.x, b / a.ngcw);
+        return;
+    }
+    b -= a.nblk_gcw;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        uint4 *z = reinterpret_cast<uint4 *>(a.zero[j]);
+        const size_t n = a.zwords[j] / 4;
+        for (size_t i = (size_t)b * 256 + threadIdx.x; i < n; i += (size_t)a.nblk_z * 256) z[i] = make_uint4(0, 0, 0, 0);
+        if (b == 0 && threadIdx.x < a.zwords[j] % 4) a.zero[j][n * 4 + threadIdx.x] = 0u;
+    }
 }
 
 // ============================================================ host side
@@ -1126,6 +1150,33 @@ inline bool plain_shape_ok(const d2c_conv3d_desc &q)
            (size_t)q.N * P < (1u << 30) && (size_t)q.N * q.D * q.H * q.W < (1u << 30);
 }
 inline int weight_blocks(long nvec) { return (int)std::min<long>((nvec + 255) / 256, 4096); }
+void prep_input(ConvPrepArgs &a, const d2c_conv3d_desc &q, const void *x, void *xcl, int zrow_words)
+{
+    const int vol = q.D * q.H * q.W;
+    a.x = (const bf16_t *)x; a.xcl = (bf16_t *)xcl; a.C = q.Cin; a.vol = vol; a.N = q.N; a.zrow_words = zrow_words;
+    a.nbx = (vol + 63) / 64; a.nby = q.Cin / 64; a.nblk_x = a.nbx * a.nby * q.N;
+    a.wide = vol % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+}
+void prep_weights(ConvPrepArgs &a, const d2c_conv3d_desc &q, const RowsPlan &p, const void *w, void *wt, bool back)
+{
+    a.w = (const bf16_t *)w; a.wt = (uint4 *)wt; a.Cout = q.Cout; a.Cin = q.Cin; a.K = q.kd * q.kh * q.kw;
+    a.NT = p.NT; a.KC = p.KC; a.nchunk = p.nchunk; a.nct = p.nct; a.back = back;
+    a.nvec = (long)p.nct * p.NT * p.nchunk * (p.KC / 8) * a.K;
+    a.nblk_w = weight_blocks(a.nvec);
+}
+void prep_zero(ConvPrepArgs &a, int j, void *p, size_t bytes)
+{
+    a.zero[j] = (uint32_t *)p; a.zwords[j] = p ? bytes / 4 : 0;
+    a.nblk_z = (int)std::min<size_t>((std::max(a.zwords[0], a.zwords[1]) + 4095) / 4096, 2048);
+}
+int prep_launch(const ConvPrepArgs &a, hipStream_t st)
+{
+    const long n = (long)a.nblk_x + a.nblk_w + a.nblk_g + a.nblk_b + a.nblk_gcw + a.nblk_z;
+    if (n == 0) return D2C_OK;
+    D2cProfScope prof(D2C_PROF_PACK, st);
+    hipLaunchKernelGGL(conv_prepare_kernel, dim3((unsigned)n), dim3(256), 0, st, a);
+    return d2c_check_launch("conv_prepare_kernel");
+}
 
 }  // namespace
 
@@ -1138,21 +1189,24 @@ size_t d2c_col_forward_ws(const d2c_conv3d_desc &q)
     const RowsPlan p = rows_plan(q.Cout, q.Cin, q.kd * q.kh * q.kw, q.N * q.Do * q.Ho * q.Wo, ncu);
     return p.wt_bytes + p.part_bytes;
 }
-int d2c_col_forward(const d2c_conv3d_desc &q, const void *col, int rows, const void *w, const void *bias, void *out, void *ws, hipStream_t st)
+// What the sorted points, the sampling and the product need in front, as one launch: the input channels-last with a row of
+// zeros of 256 bytes (x == nullptr: it is there), the weights, the counts of the sort cleared.
+int d2c_col_forward_prepare(const d2c_conv3d_desc &q, const void *x, void *xcl, const void *w, void *ws, void *zero, size_t zero_bytes,
+                            hipStream_t st)
+{
+    const int ncu = d2c_num_cus();
+    if (ncu <= 0) return D2C_ERR_LAUNCH;
+    ConvPrepArgs a{};
+    if (x) prep_input(a, q, x, xcl, 64);
+    prep_weights(a, q, rows_plan(q.Cout, q.Cin, q.kd * q.kh * q.kw, q.N * q.Do * q.Ho * q.Wo, ncu), w, ws, false);
+    prep_zero(a, 0, zero, zero_bytes);
+    return prep_launch(a, st);
+}
+int d2c_col_forward(const d2c_conv3d_desc &q, const void *col, int rows, const void *bias, void *out, void *ws, hipStream_t st)
 {
     const int K = q.kd * q.kh * q.kw, ncu = d2c_num_cus();
     if (ncu <= 0) return D2C_ERR_LAUNCH;
     const RowsPlan p = rows_plan(q.Cout, q.Cin, K, q.N * q.Do * q.Ho * q.Wo, ncu);
-    {
-        ConvPrepArgs a{};
-        a.w = (const bf16_t *)w; a.wt = (uint4 *)ws; a.Cout = q.Cout; a.Cin = q.Cin; a.K = K;
-        a.NT = p.NT; a.KC = p.KC; a.nchunk = p.nchunk; a.nct = p.nct; a.back = 0;
-        a.nvec = (long)p.nct * p.NT * p.nchunk * (p.KC / 8) * K;
-        a.nblk_w = weight_blocks(a.nvec);
-        D2cProfScope prof(D2C_PROF_PACK, st);
-        hipLaunchKernelGGL(conv_prepare_kernel, dim3((unsigned)a.nblk_w), dim3(256), 0, st, a);
-        if (int rc = d2c_check_launch("conv_prepare_kernel")) return rc;
-    }
     return run_rows(p, row_map(q, false), col, 0, 0, ws, bias, out, (float *)((char *)ws + p.wt_bytes), q.Cout, st, K, rows, q.epilogue,
                     q.epilogue_scale);
 }
@@ -1189,24 +1243,36 @@ bool d2c_grad_col_supported(const d2c_conv3d_desc &q)
            (long)p.ntile * p.nct * p.S < (1L << 30) && (size_t)q.N * q.Do * q.Ho * q.Wo * 128 < 0xFFFF0000u;
 }
 size_t d2c_grad_col_ws(const d2c_conv3d_desc &q) { return grad_col_plan(q).total; }
-int d2c_grad_col(const d2c_conv3d_desc &q, const void *gout, const void *w, void *gcol, void *ws, hipStream_t st)
+// What the backward pass over sorted points needs of grad_out and the weights, and what it adds into, as one launch (one
+// weight group): the operands of d2c_grad_col in its workspace `col_ws`, grad_out in fragment order for the grad_weight
+// product (`goutp`, see pack_gout_kernel), the bias gradient, two ranges cleared; any of them NULL.  grad_out is read once
+// for both orders.
+int d2c_brick_bwd_prepare(const d2c_conv3d_desc &q, const void *gout, const void *w, void *col_ws, void *goutp, void *gb, void *zero0,
+                          size_t zero0_bytes, void *zero1, size_t zero1_bytes, hipStream_t st)
 {
     const GradColPlan p = grad_col_plan(q);
-    const int K = q.kd * q.kh * q.kw, P = q.Do * q.Ho * q.Wo, M = q.N * P, ncu = d2c_num_cus();
-    if (ncu <= 0) return D2C_ERR_LAUNCH;
-    char *const gcl = (char *)ws + p.wt_bytes;
-    {
-        D2cProfScope prof(D2C_PROF_PACK, st);
-        hipLaunchKernelGGL(grad_col_weights_kernel, dim3((unsigned)((q.Cin * K + 255) / 256), (unsigned)(p.S * 8)), dim3(256), 0, st,
-                           (const bf16_t *)w, (uint4 *)ws, q.Cout, q.Cin, K, make_fastdiv(K), p.S);
-        ConvPrepArgs a{};
-        a.gout = (const bf16_t *)gout; a.gcl = (bf16_t *)gcl; a.Cout = q.Cout; a.Cp = p.Cp; a.P = P; a.M = M; a.dP = make_fastdiv(P);
-        a.gwide = wide_gout(gout, P); a.ngt = (M + 63) / 64; a.ngc = p.Cp / 64; a.nblk_g = a.ngt * a.ngc;
-        hipLaunchKernelGGL(conv_prepare_kernel, dim3((unsigned)a.nblk_g), dim3(256), 0, st, a);
-        if (int rc = d2c_check_launch("conv_prepare_kernel")) return rc;
+    const int K = q.kd * q.kh * q.kw, P = q.Do * q.Ho * q.Wo, M = q.N * P;
+    ConvPrepArgs a{};
+    a.w = (const bf16_t *)w; a.Cout = q.Cout; a.Cin = q.Cin; a.K = K; a.N = q.N; a.dK = make_fastdiv(K);
+    if (col_ws) {
+        a.gcw = (uint4 *)col_ws; a.gcS = p.S; a.ngcw = (q.Cin * K + 255) / 256; a.nblk_gcw = a.ngcw * p.S * 8;
+        a.gcl = (bf16_t *)((char *)col_ws + p.wt_bytes);
     }
-    GradColArgs a{(const unsigned char *)gcl, (const unsigned char *)ws, (bf16_t *)gcol, (unsigned)p.Cp * 2u, M, q.Cin / 64 * K, p.S, p.ntile,
-                  p.nct, p.cgroups};
+    a.gout = (const bf16_t *)gout; a.gp = (uint4 *)goutp; a.gp_wide = 1;
+    a.Cp = p.Cp; a.OBP = p.Cp / 32; a.P = P; a.M = M; a.dP = make_fastdiv(P);
+    a.gwide = wide_gout(gout, P); a.ngt = (M + 127) / 128 * 2; a.ngc = p.Cp / 64; a.nblk_g = col_ws || goutp ? a.ngt * a.ngc : 0;
+    a.gb = (bf16_t *)gb; a.nblk_b = gb ? q.Cout : 0;
+    prep_zero(a, 0, zero0, zero0_bytes);
+    prep_zero(a, 1, zero1, zero1_bytes);
+    return prep_launch(a, st);
+}
+int d2c_grad_col(const d2c_conv3d_desc &q, void *gcol, void *ws, hipStream_t st)
+{
+    const GradColPlan p = grad_col_plan(q);
+    const int K = q.kd * q.kh * q.kw, M = q.N * q.Do * q.Ho * q.Wo, ncu = d2c_num_cus();
+    if (ncu <= 0) return D2C_ERR_LAUNCH;
+    GradColArgs a{(const unsigned char *)ws + p.wt_bytes, (const unsigned char *)ws, (bf16_t *)gcol, (unsigned)p.Cp * 2u, M, q.Cin / 64 * K,
+                  p.S, p.ntile, p.nct, p.cgroups};
     D2cProfScope prof(D2C_PROF_BWD_DATA, st, "grad_col_kernel");
     hipLaunchKernelGGL(grad_col_kernel, dim3((unsigned)std::max(8, ncu / 8 * 8)), dim3(kThreads), 0, st, a);
     return d2c_check_launch("grad_col_kernel");
@@ -1232,16 +1298,9 @@ int d2c_plain_forward(const d2c_conv3d_desc &q, const void *x, const void *w, co
     char *base = (char *)ws;
     {
         ConvPrepArgs a{};
-        a.x = (const bf16_t *)x; a.xcl = (bf16_t *)xcl; a.C = q.Cin; a.vol = vol; a.N = q.N;
-        a.nbx = (vol + 63) / 64; a.nby = q.Cin / 64; a.nblk_x = a.nbx * a.nby * q.N;
-        a.wide = vol % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
-        a.w = (const bf16_t *)w; a.wt = (uint4 *)base; a.Cout = q.Cout; a.Cin = q.Cin; a.K = K;
-        a.NT = p.NT; a.KC = p.KC; a.nchunk = p.nchunk; a.nct = p.nct; a.back = 0;
-        a.nvec = (long)p.nct * p.NT * p.nchunk * (p.KC / 8) * K;
-        a.nblk_w = weight_blocks(a.nvec);
-        D2cProfScope prof(D2C_PROF_PACK, st);
-        hipLaunchKernelGGL(conv_prepare_kernel, dim3((unsigned)(a.nblk_x + a.nblk_w)), dim3(256), 0, st, a);
-        if (int rc = d2c_check_launch("conv_prepare_kernel")) return rc;
+        prep_input(a, q, x, xcl, 128);
+        prep_weights(a, q, p, w, base, false);
+        if (int rc = prep_launch(a, st)) return rc;
     }
     return run_rows(p, row_map(q, false), xcl, (unsigned)q.Cin * 2u, (unsigned)((size_t)q.N * q.Cin * vol * 2), base, bias, out,
                     (float *)(base + p.wt_bytes), q.Cout, st);
@@ -1284,10 +1343,8 @@ int d2c_plain_backward(const d2c_conv3d_desc &q, const void *gout, const void *x
     char *base = (char *)ws;
     {
         ConvPrepArgs a{};
-        a.w = (const bf16_t *)w; a.wt = (uint4 *)(base + l.wt); a.Cout = q.Cout; a.Cin = q.Cin; a.K = K;
-        a.NT = r.NT; a.KC = r.KC; a.nchunk = r.nchunk; a.nct = r.nct; a.back = 1; a.N = q.N;
-        a.nvec = (long)r.nct * r.NT * r.nchunk * (r.KC / 8) * K;
-        a.nblk_w = gx ? weight_blocks(a.nvec) : 0;
+        a.N = q.N; a.Cout = q.Cout;
+        if (gx) prep_weights(a, q, r, w, base + l.wt, true);
         a.gout = (const bf16_t *)gout;
         a.gcl = gx ? (bf16_t *)(base + l.gcl) : nullptr;
         a.gp = gw ? (uint4 *)(base + l.gp) : nullptr;
@@ -1298,9 +1355,7 @@ int d2c_plain_backward(const d2c_conv3d_desc &q, const void *gout, const void *x
         a.nblk_g = (gx || gw) ? a.ngt * a.ngc : 0;
         a.gb = (bf16_t *)gb;
         a.nblk_b = gb ? q.Cout : 0;
-        D2cProfScope prof(D2C_PROF_PACK, st);
-        hipLaunchKernelGGL(conv_prepare_kernel, dim3((unsigned)(a.nblk_w + a.nblk_g + a.nblk_b)), dim3(256), 0, st, a);
-        if (int rc = d2c_check_launch("conv_prepare_kernel")) return rc;
+        if (int rc = prep_launch(a, st)) return rc;
     }
     if (gx) {
         if (int rc = run_rows(r, row_map(q, true), base + l.gcl, (unsigned)Cp * 2u, (unsigned)((size_t)M * Cp * 2), base + l.wt, nullptr,

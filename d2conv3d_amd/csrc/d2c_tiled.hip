@@ -6,10 +6,14 @@
 #include "d2c_mma.hpp"
 
 size_t d2c_col_forward_ws(const d2c_conv3d_desc &q);
-int d2c_col_forward(const d2c_conv3d_desc &q, const void *col, int rows, const void *w, const void *bias, void *out, void *ws, hipStream_t st);
+int d2c_col_forward_prepare(const d2c_conv3d_desc &q, const void *x, void *xcl, const void *w, void *ws, void *zero, size_t zero_bytes,
+                            hipStream_t st);
+int d2c_col_forward(const d2c_conv3d_desc &q, const void *col, int rows, const void *bias, void *out, void *ws, hipStream_t st);
 bool d2c_grad_col_supported(const d2c_conv3d_desc &q);
 size_t d2c_grad_col_ws(const d2c_conv3d_desc &q);
-int d2c_grad_col(const d2c_conv3d_desc &q, const void *gout, const void *w, void *gcol, void *ws, hipStream_t st);
+int d2c_brick_bwd_prepare(const d2c_conv3d_desc &q, const void *gout, const void *w, void *col_ws, void *goutp, void *gb, void *zero0,
+                          size_t zero0_bytes, void *zero1, size_t zero1_bytes, hipStream_t st);
+int d2c_grad_col(const d2c_conv3d_desc &q, void *gcol, void *ws, hipStream_t st);
 int d2c_fwd_out_tile(const TiledShape &s);
 template <typename T>
 int d2c_tiled_fwd_launch(const TiledShape &s, const void *xcl, const void *off, const void *mask, const void *wp,
@@ -398,9 +402,10 @@ struct FwdWs {
     size_t total;                   // what the call is fastest with
 };
 bool use_brick_forward(const d2c_conv3d_desc &q, const TiledShape &s, bool kept);
-// columns; and what a forward call can leave for its backward call: the sorted points behind them
+// columns; and what a forward call can leave for its backward call: behind them the sorted points, then the input channels-last
 size_t brick_col_bytes(const TiledShape &s) { return (size_t)(s.Cin / 64) * s.K * d2c_columns_rows(s) * 128; }
-size_t brick_keep_bytes(const TiledShape &s) { return brick_col_bytes(s) + d2c_brick_ws(s).total; }
+size_t brick_keep_input(const TiledShape &s) { return brick_col_bytes(s) + d2c_brick_ws(s).total; }
+size_t brick_keep_bytes(const TiledShape &s) { return brick_keep_input(s) + d2c_align_up((size_t)s.N * s.vol * s.Cin * 2 + 256); }
 // Caller-held prepared region (d2c_conv3d_prepared_bytes): channels-last input + zero row | forward weights in
 // fragment order | backward weights transposed per step (single-pass reductions only)
 struct PreparedLayout {
@@ -568,19 +573,23 @@ int forward_t(const d2c_conv3d_desc &q, const void *x, const void *off, const vo
     char *wp_p = prep ? (char *)prep->base + pl.wp : base + l.wp;
     const bool have_x = prep && (prep->reuse & D2C_REUSE_INPUT);
     if (nd == 3 && !prep && !stats && use_brick_forward(q, s, columns != nullptr)) {
-        // sort the points, sample the columns (the caller's buffer, with the sorted points behind them for its backward
-        // call, or the workspace), multiply.  A smaller workspace: the gathering kernels, below.
+        // sort the points, sample the columns (the caller's buffer, with the sorted points and the input behind them for its
+        // backward call, or the workspace), multiply.  A smaller workspace: the gathering kernels, below.
         const bool keep = columns && columns_bytes >= brick_keep_bytes(s);
         const bool fits = ws_bytes >= (keep ? l.lists : (columns ? l.col : l.end));
         char *col = columns ? (char *)columns : base + l.col;
         char *lists = keep ? col + brick_col_bytes(s) : base + l.lists;
-        if (fits)
-            if (int rc = pack_input<T>(s, x, xcl_p, st, true)) return rc;   // with the row of zeros behind it
+        if (keep) xcl_p = col + brick_keep_input(s);
+        if (fits) {
+            size_t zb;
+            void *const zp = d2c_brick_zero(s, lists, &zb);
+            if (int rc = d2c_col_forward_prepare(q, x, xcl_p, w, base + l.gemm, zp, zb, st)) return rc;
+        }
         if (fits || keep)
-            if (int rc = d2c_brick_sort(s, off, mask, lists, st)) return rc;
+            if (int rc = d2c_brick_sort(s, off, mask, lists, st, fits)) return rc;
         if (fits) {
             if (int rc = d2c_brick_columns(s, xcl_p, col, (int)d2c_columns_rows(s), lists, st)) return rc;
-            return d2c_col_forward(q, col, (int)d2c_columns_rows(s), w, bias, out, base + l.gemm, st);
+            return d2c_col_forward(q, col, (int)d2c_columns_rows(s), bias, out, base + l.gemm, st);
         }
     }
     // input, weights, and the counters of the steps' split (which needs its scratch: a smaller workspace goes without)
@@ -701,14 +710,14 @@ bool brick_backward(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_co
 struct BwdWs {
     size_t xcl, wt, gxcl, gwacc, goutp, auxacc, gcol, counts, entries, ovf, gsacc, sm1, brick, res, gemm, col, total;
 };
-// `sorted`: ... and the sorted points behind them
+// `sorted`: ... and the sorted points and the input behind them
 BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns = false, bool sorted = false)
 {
     const bool brick = brick_backward(q, s, saved_columns);
     const size_t es = d2c_elem_size(q.dtype);
     BwdWs w;
     w.xcl = 0;
-    w.wt = d2c_align_up((size_t)s.N * s.vol * s.Cin * es + 256);   // input, then a 256-byte row of zeros
+    w.wt = sorted ? 0 : d2c_align_up((size_t)s.N * s.vol * s.Cin * es + 256);   // input, then a 256-byte row of zeros
     const int omax = d2c_bwd_pass_channels(q.dtype);
     const int ogk = d2c_bwd_ogk(s.og < omax ? s.og : omax, q.dtype);
     w.gxcl = w.wt + d2c_align_up((size_t)s.groups * s.K * s.nchunk * bkc_of(q.dtype) * ogk * es);
@@ -799,14 +808,16 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
     const bool brick = nd == 3 && brick_backward(q, s, columns != nullptr);
     const BwdWs l = bwd_ws(q, s, columns != nullptr, sorted);
     const PreparedLayout pl = prepared_layout(q, s);
-    char *xcl_p = prep ? (char *)prep->base + pl.xcl : base + l.xcl;
+    // (a forward call over sorted points has left the input behind them)
+    const bool have_x = (prep && (prep->reuse & D2C_REUSE_INPUT)) || (sorted && !prep);
+    char *xcl_p = prep ? (char *)prep->base + pl.xcl : (sorted ? (char *)const_cast<void *>(columns) + brick_keep_input(s) : base + l.xcl);
     // (the transposed weights of the region serve single-pass reductions; wider weight groups re-pack per pass)
     const bool wt_prep = prep && pl.wt_bytes > 0;
     char *wt_p = wt_prep ? (char *)prep->base + pl.wt : base + l.wt;
     const bool wt_packed = wt_prep && (prep->reuse & D2C_REUSE_BACKWARD_WEIGHTS);
-    if (!(prep && (prep->reuse & D2C_REUSE_INPUT)))
+    if (!have_x)
         if (int rc = pack_input<T>(s, x, xcl_p, st, true)) return rc;   // with the row of zeros behind it
-    if (s.ss.on) {
+    if (s.ss.on && !(brick && sorted && (goff || gmask || gx))) {
         D2cProfScope prof(D2C_PROF_PACK, st);
         long gr = ((long)s.N * s.P + 255) / 256;
         if (gr > 8192) gr = 8192;
@@ -819,7 +830,7 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
         s.ss.on = 2;
         off = sm1;
     }
-    bool gw_from_col = false, gw_in_place = false, gw_done = false;
+    bool gw_from_col = false, gw_in_place = false, gw_done = false, gw_ready = false;
     // (`columns`: the sampled columns the forward call kept -- the offset / mask gradient kernel then writes none, the
     // grad-weight product takes these, and the settings that save workspace by other means do not apply)
     const BwdSlices sl = columns ? BwdSlices{0, 0} : bwd_slices(q, s);
@@ -908,8 +919,21 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
                 L = d2c_lists_make(s, Elem<T>::DT, base + l.counts, base + l.entries, base + l.ovf);
                 if (int rc = (auxk && !gw_in_place) ? d2c_lists_clear(L, st) : d2c_lists_build(s, off, mask, L, st)) return rc;
             }
-            if (brick && !prep && d2c_grad_col_supported(q)) {
-                if (int rc = d2c_grad_col(q, gout, w, base + l.gcol, base + l.gemm, st)) return rc;
+            const bool grad_col = brick && !prep && d2c_grad_col_supported(q);
+            if (brick && s.groups == 1) {
+                // grad_out and the weights in the orders of the products, the bias gradient, what is added into cleared
+                gw_ready = gw_from_col;
+                if (int rc = d2c_brick_bwd_prepare(q, gout, w, grad_col ? base + l.gemm : nullptr, gw_ready ? base + l.goutp : nullptr, gb,
+                                                   gxcl, gxcl ? (size_t)s.N * s.vol * s.Cin * sizeof(float) : 0,
+                                                   gw_ready ? base + l.gwacc : nullptr, (size_t)s.Cout * s.cg * s.K * sizeof(float), st))
+                    return rc;
+                gb = nullptr;
+            } else if (brick && gxcl) {
+                D2cProfScope prof(D2C_PROF_PACK, st);
+                d2c_fill_zero(gxcl, (size_t)s.N * s.vol * s.Cin * sizeof(float), st);
+            }
+            if (grad_col) {
+                if (int rc = d2c_grad_col(q, base + l.gcol, base + l.gemm, st)) return rc;
             } else if (int rc = d2c_tiled_bwd_data_launch<T>(s, gout, xcl_p, off, mask, w, wt_p,
                                                      lists ? nullptr : gxcl, (lists || auxk) ? base + l.gcol : nullptr,
                                                      auxk ? nullptr : goff, auxk ? nullptr : gmask,
@@ -963,7 +987,7 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
             if (int rc = d2c_tiled_bwd_weight_launch<T>(s, gout, xcl_p, off, mask, base + l.goutp,
                                                        (float *)(base + l.gwacc),
                                                        gw, gw_from_col ? (columns ? (char *)columns : (gw_in_place ? base + l.gcol : base + l.col)) : nullptr,
-                                                       gw_in_place ? (long)s.M : (long)((s.M + 63) / 64) * 64, st))
+                                                       gw_in_place ? (long)s.M : (long)((s.M + 63) / 64) * 64, st, gw_ready ? 6 : 7))
                 return rc;
         } else {
             if (int rc = d2c_generic_conv3d_backward(q, gout, x, off, mask, w, nullptr, nullptr, nullptr, gw, nullptr,

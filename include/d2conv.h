@@ -198,8 +198,8 @@ int d2c_conv3d_backward(const d2c_conv3d_desc *desc, const void *grad_out, const
  * taps x the size of the input, in the element type): the forward kernel writes there what it multiplies with the
  * weights anyway, and d2c_conv3d_backward_columns, given that buffer UNCHANGED together with the same tensors, runs
  * its grad-weight product over it instead of sampling again (N=2, C=512, 8x30x54, bfloat16: 2.33 -> 1.95 ms per step
- * for 851 MB held between the two calls -- 717 of columns, the rest sorted sampling points, see d2c_conv3d_keep_bytes() -- and
- * 0.85 GB less backward workspace; N=2, C=256, 8x30x54, float32: 2.29 -> 2.13 ms for 717 MB).  Results are those of the plain calls up to the order of floating-point sums; float32
+ * for 878 MB held between the two calls -- 717 of columns, sorted sampling points, the input channels-last, see d2c_conv3d_keep_bytes() -- and
+ * 0.88 GB less backward workspace; N=2, C=256, 8x30x54, float32: 2.29 -> 2.13 ms for 717 MB).  Results are those of the plain calls up to the order of floating-point sums; float32
  * columns are the interpolated floats themselves and their product keeps float32's accuracy (three bfloat16 terms
  * per float on the bfloat16 matrix instruction, or the float32 instruction), whatever D2C_BWD_F32_SPLIT says.  `size_map` as in d2c_conv3d_forward_stats: NULL, or the description of
  * the size map that `offset` then is.  d2c_conv3d_columns_bytes() is 0 where this is not served (anything but
@@ -212,8 +212,8 @@ int d2c_conv3d_backward(const d2c_conv3d_desc *desc, const void *grad_out, const
 struct d2c_size_map_desc;
 size_t d2c_conv3d_columns_bytes(const d2c_conv3d_desc *desc, const struct d2c_size_map_desc *size_map);
 /* What is worth keeping: d2c_conv3d_columns_bytes(), or more where the forward pass also sorts the sampling points by
- * their place in the volume and its backward call can take them over.  A buffer of this size handed to both calls (with
- * this size as columns_bytes) spares the backward call its own sort, and both part of their workspace: the
+ * their place in the volume and its backward call can take them, and the input in the order it reads, over.  A buffer of
+ * this size handed to both calls (with this size as columns_bytes) spares the backward call its own sort, and both part of their workspace: the
  * *_keep_workspace_bytes() are for calls with such a buffer.  (With a buffer of d2c_conv3d_columns_bytes():
  * d2c_conv3d_forward_workspace_bytes() and d2c_conv3d_backward_columns_workspace_bytes().) */
 size_t d2c_conv3d_keep_bytes(const d2c_conv3d_desc *desc, const struct d2c_size_map_desc *size_map);
