@@ -331,8 +331,8 @@ D2C_DEV PointValues point_of_lane(const uint4 &e, float alpha, int l, int y0, in
 struct BrickArgs {
     BrickDims d;
     BrickLists L;
-    const bf16_t *xcl;       // [N][vol][Cin]
-    const bf16_t *gcol;      // [chunk][tap][N*P][64]
+    const void *xcl;         // [N][vol][Cin]
+    const void *gcol;        // [chunk][tap][N*P][64 bfloat16 / 32 float]
     float *gxcl;             // [N][vol][Cin] sums (cleared), or NULL
     float2 *res;             // [set][point][2]: sum over its channels of (mask, x), (z, y) per unit of modulation; or NULL
     long nres;               // points per set
@@ -388,7 +388,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
         if ((fn >> 4) != (z & 1)) return;
         const int vox_y = y0 + ((fn >> 2) & 3), vox_x = x0 + (fn & 3);
         const bool in = vox_y >= 0 && vox_y < a.H && vox_x >= 0 && vox_x < a.W && z >= 0 && z < a.D;
-        const bf16_t *xp = a.xcl + ((long)b * a.vol + ((long)(in ? z : 0) * a.H + (in ? vox_y : 0)) * a.W + (in ? vox_x : 0)) * a.Cin
+        const bf16_t *xp = (const bf16_t *)a.xcl + ((long)b * a.vol + ((long)(in ? z : 0) * a.H + (in ? vox_y : 0)) * a.W + (in ? vox_x : 0)) * a.Cin
                            + cc0 * 64 + h * 8;
         for_each_const([&](auto I) INLINE {
             constexpr int ks = decltype(I)::value;
@@ -453,7 +453,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
         const int e = max(e_lo + min(i + n, cnt - 1), 0);
         q = a.L.pt[e]; al = a.L.alpha[e];
     };
-    const auto rsg = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(a.gcol) + (long)cc0 * a.chunk_rows * 64, 0, (int)(unsigned)(a.chunk_rows * 128), 0x00020000);
+    const auto rsg = __builtin_amdgcn_make_buffer_rsrc((bf16_t *)const_cast<void *>(a.gcol) + (long)cc0 * a.chunk_rows * 64, 0, (int)(unsigned)(a.chunk_rows * 128), 0x00020000);
     auto rows = [&](const uint4 &q, u32x4_t (&row)[4]) INLINE {
         for_each_const([&](auto I) INLINE {
             constexpr int i = decltype(I)::value;
@@ -615,12 +615,351 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
             const float al = a.L.alpha[e];
             for (int j = 0; j < min(np - i, 64); j++) {
                 const PointValues p = point_of_lane(q, al, j, y0, x0);
-                const float gv = bf16_to_f32(a.gcol[(long)cc0 * a.chunk_rows * 64 + (p.row >> 1) + lane]);
+                const float gv = bf16_to_f32(((const bf16_t *)a.gcol)[(long)cc0 * a.chunk_rows * 64 + (p.row >> 1) + lane]);
                 for (int c = 0; c < 8; c++) {
                     const int z = zi - 1 + (c >> 2), y = p.y + ((c >> 1) & 1), x = p.x + (c & 1);
                     const float wz = c & 4 ? p.hz : 1.f - p.hz, wy = c & 2 ? p.hy : 1.f - p.hy, wx = c & 1 ? p.hx : 1.f - p.hx;
                     if (wz > 0.f && wy > 0.f && wx > 0.f && z >= bad_from && z >= 0 && z < a.D && y >= 0 && y < a.H && x >= 0 && x < a.W)
                         atomicAdd(a.gxcl + ((long)b * a.vol + ((long)z * a.H + y) * a.W + x) * a.Cin + cc0 * 64 + lane, p.alpha * wz * wy * wx * gv);
+                }
+            }
+        }
+    }
+}
+
+// ---- the same for float32 -------------------------------------------------------------------------------------------
+// Rows are 32 channels (128 bytes).  Weights, rows and input each travel as three bfloat16 terms that add up to the float
+// (what the third leaves is below 2^-26 of it); of the nine products of two numbers the six largest are summed in float32:
+// what is left out is below 2^-25 of a product, less than a rounding in float32 leaves.  A wavefront takes its
+// rows apart as they come (16 floats to a lane) into three planes [point][32 channels] in LDS, laid out like the weights'.
+// A number that is none, or that the first term would round to an infinity, has no such terms: where a plane of the input or
+// the rows of a step hold one, the corner dots of the step are worked out point by point; the sums of grad_input as above.
+// To 32 points x 32 channels 24 matrix instructions, 364 of the vector ALU and 57 of LDS: the matrix pipes are busy 29 % of
+// the time, instruction issue as a whole about 60 %, and the rows alone (0.72 GB) would take 0.14 ms.  Sized operator, 256 -> 256 channels on 2x8x30x54, us:
+// 279 and 70 for the sort and the results; gathering (a dot product per corner and channel, then the lists of a voxel's points) 389 + 311.
+// Not it: two wavefronts per SIMD with the rows of two steps in flight, 333.
+// (numbers that the first term would round to an infinity count as none)
+D2C_DEV void split3(float a, float b, uint32_t (&o)[3])
+{
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        o[i] = pack_bf16x2(a, b);
+        a -= __uint_as_float(o[i] << 16); b -= __uint_as_float(o[i] & 0xffff0000u);
+    }
+}
+constexpr int kWaveLdsF = 2 * 3 * 32 * 64;
+__global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_f32_kernel(BrickArgs a, const int *__restrict__ seg_end, const int *__restrict__ seg_count)
+{
+    const int lane = threadIdx.x & 63, h = lane >> 5, n = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+    extern __shared__ __align__(16) unsigned char smem[];
+    unsigned char *const s_g = smem + wave * kWaveLdsF, *const s_w = s_g + 3 * 32 * 64;      // rows and weights: [term][point][32]
+    float2 *const s_part = reinterpret_cast<float2 *>(smem + nw * kWaveLdsF);                // [2][wave][lane]: sums over a chunk each
+
+    // task: as in brick_grad_kernel
+    const int nt = (int)gridDim.x, xq = nt >> 3, xr = nt & 7, xcd = blockIdx.x & 7;
+    int t = xcd * xq + (xcd < xr ? xcd : xr) + (int)(blockIdx.x >> 3);
+    const int set = t % a.nset; t /= a.nset;
+    const int bx = t % a.d.nbx; t /= a.d.nbx;
+    const int by = t % a.d.nby; t /= a.d.nby;
+    const int zr = t % a.nzr; const int bg = t / a.nzr;
+    const int b = bg / a.G, g = bg - b * a.G;
+    const bool here = set * nw + wave < a.cpc;
+    const int cc0 = g * a.cpc + (here ? set * nw + wave : 0);
+    const bool want_gx = a.gxcl != nullptr && here;
+    const int res_bytes = a.res ? 16 : 0;
+    const int y0 = by * 3 - 1, x0 = bx * 3 - 1;
+    const int zi_lo = zr * a.zlen, zi_hi = min(zi_lo + a.zlen, a.d.nz);
+    constexpr unsigned kNone = 0xFFFFFFF0u;
+    const float *const xin = reinterpret_cast<const float *>(a.xcl), *const rows_in = reinterpret_cast<const float *>(a.gcol);
+
+    f32x16 gacc;
+#pragma unroll
+    for (int r = 0; r < 16; r++) gacc[r] = 0.f;
+
+    // input rows as the operand of T: lane = voxel n of the brick, 8 channels of each of two k-steps, three terms.
+    // load_plane changes the lanes of slot z & 1.
+    u32x4_t xa[2][3];
+    bool bad_x = false;                                  // this lane's row holds infinities or NaN
+    auto load_plane = [&](int z) INLINE {
+        int fn = n;
+        opaque_v(fn);
+        if ((fn >> 4) != (z & 1)) return;
+        const int vox_y = y0 + ((fn >> 2) & 3), vox_x = x0 + (fn & 3);
+        const bool in = vox_y >= 0 && vox_y < a.H && vox_x >= 0 && vox_x < a.W && z >= 0 && z < a.D;
+        const float *xp = xin + ((long)b * a.vol + ((long)(in ? z : 0) * a.H + (in ? vox_y : 0)) * a.W + (in ? vox_x : 0)) * a.Cin + cc0 * 32 + h * 8;
+        float4 v[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (in && here) v[i] = *reinterpret_cast<const float4 *>(xp + (i >> 1) * 16 + (i & 1) * 4);
+        }
+        unsigned top[8];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            uint32_t lo[3], hi[3];
+            split3(v[i].x, v[i].y, lo);
+            split3(v[i].z, v[i].w, hi);
+            top[2 * i] = lo[0]; top[2 * i + 1] = hi[0];
+#pragma unroll
+            for (int q = 0; q < 3; q++) { xa[i >> 1][q][(i & 1) * 2] = lo[q]; xa[i >> 1][q][(i & 1) * 2 + 1] = hi[q]; }
+        }
+        bad_x = no_number_bf16(top, 8);
+    };
+    int bad_from = 0x7fffffff;
+    const unsigned plane_bytes = (unsigned)a.H * (unsigned)a.W * (unsigned)a.Cin * 4u;
+    auto flush_plane = [&](int z) INLINE {
+        const bool odd = z & 1;
+        float all = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; r++) all += gacc[r];
+        if (any_lane(no_number(all))) bad_from = min(bad_from, z);
+        const bool zin = z >= 0 && z < a.D && z < bad_from;
+        int fn = n, fh = h;
+        opaque_v(fn); opaque_v(fh);
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc(a.gxcl + ((long)b * a.vol + (long)(zin ? z : 0) * a.H * a.W) * a.Cin, 0,
+                                                          (int)plane_bytes, 0x00020000);
+        for_each_const([&](auto I) INLINE {
+            constexpr int r = decltype(I)::value;
+            constexpr int dy = 2 * (r >> 2), dx = r & 3;
+            const int y = y0 + fh + dy, x = x0 + dx;
+            const bool in = zin && y >= 0 && y < a.H && x >= 0 && x < a.W;
+            const unsigned o = in ? (unsigned)((y * a.W + x) * a.Cin + cc0 * 32 + fn) * 4u : kNone;
+            const float v = odd ? gacc[8 + r] : gacc[r];
+            gacc[r] = odd ? gacc[r] : 0.f;
+            gacc[8 + r] = odd ? 0.f : gacc[8 + r];
+            __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(v, rs, (int)o, 0, 0);
+        }, std::make_integer_sequence<int, 8>{});
+    };
+
+    // LDS places of this lane: rows and weights in the same layout, 64 bytes to a point, its 16-byte pieces permuted
+    const int pv = lane >> 3, pc = lane & 7;
+    const unsigned g_ld = lds_address(s_g) + n * 64, g_sw = (unsigned)((n >> 2) & 3);
+    const unsigned w_st = lds_address(s_w) + n * 64 + (((h * 2) ^ ((n >> 2) & 3)) << 4);
+    const int tr_row = h * 8 + ((lane & 15) >> 2), tr_pc = ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1), tr_in = (lane & 1) * 8;
+    const unsigned tr = tr_row * 64 + ((tr_pc ^ (h * 2)) << 4) + tr_in;
+    const unsigned g_tr = lds_address(s_g) + tr, w_tr = lds_address(s_w) + tr;
+    auto tr_read = [](unsigned addr) INLINE {
+        return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s *)(size_t)addr));
+    };
+    auto operand = [&](unsigned at, int kg, int term) INLINE {
+        const uint2 lo = tr_read(at + kg * 1024 + term * 2048), hi = tr_read((at ^ 16) + kg * 1024 + 256 + term * 2048);
+        return __builtin_bit_cast(bf16x8_t, make_uint4(lo.x, lo.y, hi.x, hi.y));
+    };
+
+    uint4 e0, e1, e2;
+    float a0, a1, a2;
+    u32x4_t row_a[4];
+    int e_lo = 0, cnt = 0;
+    auto entry = [&](int i, uint4 &q, float &al) INLINE {
+        const int e = max(e_lo + min(i + n, cnt - 1), 0);
+        q = a.L.pt[e]; al = a.L.alpha[e];
+    };
+    const auto rsg = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(rows_in) + (long)cc0 * a.chunk_rows * 32, 0, (int)(unsigned)(a.chunk_rows * 128), 0x00020000);
+    auto rows = [&](const uint4 &q, u32x4_t (&row)[4]) INLINE {
+        for_each_const([&](auto I) INLINE {
+            constexpr int i = decltype(I)::value;
+            row[i] = __builtin_amdgcn_raw_buffer_load_b128(rsg, __builtin_amdgcn_ds_bpermute((i * 8 + pv) << 2, (int)(q.x & ~127u)) + pc * 16, 0, 0);
+        }, std::make_integer_sequence<int, 4>{});
+    };
+    int r_lo, r_n;
+    auto range = [&](int zi) INLINE {
+        const int sg = brick_seg(a.d, bg, min(zi, zi_hi - 1), by, bx);
+        r_lo = seg_end[sg]; r_n = seg_count[sg];
+    };
+    auto begin = [&](int zi) INLINE {
+        cnt = __builtin_amdgcn_readfirstlane(r_n); e_lo = __builtin_amdgcn_readfirstlane(r_lo) - cnt;
+        if (cnt > 0) {
+            entry(0, e0, a0);
+            entry(32, e1, a1);
+        }
+        load_plane(zi);
+        if (cnt > 0) {
+            rows(e0, row_a);
+        }
+    };
+    int par = 0, turn = 0;
+    range(zi_lo);
+    load_plane(zi_lo - 1);
+    begin(zi_lo);
+    for (int zi = zi_lo; zi < zi_hi; zi++) {
+        const int z = zi - 1;
+        const bool low = z & 1;                      // slot of the base plane
+        range(zi + 1);
+        const bool bad_plane = any_lane(bad_x);
+        auto step = [&](int i0, u32x4_t (&row)[4]) INLINE {
+            entry(i0 + 64, e2, a2);
+            __builtin_amdgcn_sched_barrier(0);
+            // the rows to LDS, term by term; others requested in their place
+            unsigned top[8];
+            for_each_const([&](auto I) INLINE {
+                constexpr int i = decltype(I)::value;
+                const float v[4] = {__uint_as_float(row[i][0]), __uint_as_float(row[i][1]), __uint_as_float(row[i][2]), __uint_as_float(row[i][3])};
+                uint32_t lo[3], hi[3];
+                split3(v[0], v[1], lo);
+                split3(v[2], v[3], hi);
+                top[2 * i] = lo[0]; top[2 * i + 1] = hi[0];
+                const int pt = i * 8 + pv;
+                const unsigned at = lds_address(s_g) + pt * 64 + (((pc >> 1) ^ ((pt >> 2) & 3)) << 4) + (pc & 1) * 8;
+                typedef __attribute__((address_space(3))) unsigned long long *lds64;
+#pragma unroll
+                for (int q = 0; q < 3; q++) *(lds64)(size_t)(at + q * 2048) = (unsigned long long)hi[q] << 32 | lo[q];
+            }, std::make_integer_sequence<int, 4>{});
+            const bool bad = bad_plane || any_lane(no_number_bf16(top, 8));
+            rows(e1, row);
+            __builtin_amdgcn_sched_barrier(0);
+            const bool ok = i0 + n < cnt;
+            const unsigned yb = e0.x & 3u, xs = (e0.x & 12u) << 2;
+            const float hy = __uint_as_float(e0.y), hx = __uint_as_float(e0.z), hz = __uint_as_float(e0.w), lz = 1.f - hz;
+            {
+                const float wz = (ok ? a0 : 0.f) * ((h != 0) == low ? lz : hz);
+                const float wy0 = wz * (1.f - hy), wy1 = wz * hy, lx = 1.f - hx;
+                const WeightRow r0 = weight_row(wy0 * lx, wy0 * hx, xs), r1 = weight_row(wy1 * lx, wy1 * hx, xs);
+                typedef __attribute__((address_space(3))) unsigned long long *lds64;
+                const unsigned sy = yb << 3;
+                const unsigned at0 = w_st ^ sy, at1 = w_st ^ (sy + 8), at2 = w_st ^ ((sy + 16) & 24), at3 = w_st ^ ((sy + 24) & 24);
+#pragma unroll
+                for (int i = 0; i < 3; i++) {
+                    *(lds64)(size_t)(at0 + i * 2048) = r0.t[i];
+                    *(lds64)(size_t)(at1 + i * 2048) = r1.t[i];
+                    *(lds64)(size_t)(at2 + i * 2048) = 0;
+                    *(lds64)(size_t)(at3 + i * 2048) = 0;
+                }
+            }
+            wave_fence();
+            // ---- the two products, the smallest terms first
+            f32x16 T;
+#pragma unroll
+            for (int r = 0; r < 16; r++) T[r] = 0.f;
+            constexpr int order[6][2] = {{1, 1}, {0, 2}, {2, 0}, {0, 1}, {1, 0}, {0, 0}};
+            for_each_const([&](auto KG) INLINE {
+                constexpr int kg = decltype(KG)::value;            // 16 channels
+                bf16x8_t gq[3];
+#pragma unroll
+                for (int q = 0; q < 3; q++)
+                    gq[q] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const __attribute__((address_space(3))) u32x4_t *>(
+                                                   (size_t)(g_ld + (((kg * 2 + h) ^ g_sw) << 4) + q * 2048)));
+#pragma unroll
+                for (int i = 0; i < 6; i++)
+                    T = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, xa[kg][order[i][0]]), gq[order[i][1]], T, 0, 0, 0);
+            }, std::make_integer_sequence<int, 2>{});
+            __builtin_amdgcn_sched_barrier(0);
+            for_each_const([&](auto KG) INLINE {
+                constexpr int kg = decltype(KG)::value;            // 16 points
+                bf16x8_t w[3], gb[3];
+#pragma unroll
+                for (int q = 0; q < 3; q++) {
+                    w[q] = operand(w_tr, kg, q);
+                    gb[q] = operand(g_tr, kg, q);
+                }
+#pragma unroll
+                for (int i = 0; i < 6; i++) gacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[order[i][0]], gb[order[i][1]], gacc, 0, 0, 0);
+            }, std::make_integer_sequence<int, 2>{});
+            wave_fence();
+            // ---- grad_offset / grad_mask from the point's corner dots
+            {
+                const bool y1 = yb >= 1, y2 = yb >= 2, x1 = xs >= 16, x2 = xs >= 32;
+                const bool q = h ? y2 : y1;
+                const bool hi = (y1 != y2) != (h != 0);
+                float tv[16];
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    tv[r] = T[r];
+                    opaque_v(tv[r]);
+                }
+                float d[2][2];                                    // [plane slot][corner along x] of the row along y that this half holds
+#pragma unroll
+                for (int zz = 0; zz < 2; zz++) {
+                    float ty[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) ty[i] = q ? tv[zz * 8 + 4 + i] : tv[zz * 8 + i];
+                    d[zz][0] = x2 ? ty[2] : (x1 ? ty[1] : ty[0]);
+                    d[zz][1] = x2 ? ty[3] : (x1 ? ty[2] : ty[1]);
+                }
+                if (__builtin_expect(bad, 0)) {
+                    // point by point (lane = channel of either half, which takes one plane): corner dots as plain sums
+                    for (int j = 0; j < min(cnt - i0, 32); j++) {
+                        const PointValues p = point_of_lane(e0, a0, j, y0, x0);
+                        const float gv = rows_in[(long)cc0 * a.chunk_rows * 32 + (p.row >> 2) + n];
+                        float dot[4];                             // y, x of plane z + h
+#pragma unroll
+                        for (int c = 0; c < 4; c++) {
+                            const int zc = z + h, yc = p.y + (c >> 1), xc = p.x + (c & 1);
+                            const bool in = here && zc >= 0 && zc < a.D && yc >= 0 && yc < a.H && xc >= 0 && xc < a.W;
+                            float v = in ? gv * xin[((long)b * a.vol + ((long)zc * a.H + yc) * a.W + xc) * a.Cin + cc0 * 32 + n] : 0.f;
+#pragma unroll
+                            for (int m = 1; m < 32; m <<= 1) v += __shfl_xor(v, m, 64);
+                            dot[c] = v;
+                        }
+                        // (plane z + h lies in slot low ^ h: what lane j of half 0, 1 wants of either half)
+                        const int ry = hi ? 1 : 0;
+#pragma unroll
+                        for (int zz = 0; zz < 2; zz++)
+#pragma unroll
+                            for (int xx = 0; xx < 2; xx++) {
+                                const float v0 = lane_value(dot[xx], ((zz != 0) != low) ? 32 : 0), v1 = lane_value(dot[2 + xx], ((zz != 0) != low) ? 32 : 0);
+                                if (n == j) d[zz][xx] = ry ? v1 : v0;
+                            }
+                    }
+                }
+                float sx[2], ex[2];
+#pragma unroll
+                for (int zz = 0; zz < 2; zz++) {
+                    sx[zz] = fmaf(hx, d[zz][1] - d[zz][0], d[zz][0]);
+                    ex[zz] = d[zz][1] - d[zz][0];
+                }
+                const float w0 = low ? hz : lz, w1 = low ? lz : hz;
+                const float sz = fmaf(w1, sx[1], w0 * sx[0]), ez = fmaf(w1, ex[1], w0 * ex[0]);
+                const float dz = low ? sx[0] - sx[1] : sx[1] - sx[0];
+                const float wy = hi ? hy : 1.f - hy;
+                const float r_m = wy * sz, r_y = hi ? sz : -sz, r_x = wy * ez, r_z = wy * dz;
+                const auto u = __builtin_amdgcn_permlane32_swap(__float_as_uint(r_m), __float_as_uint(r_z), false, false);
+                const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(r_x), __float_as_uint(r_y), false, false);
+                float2 r = make_float2(__uint_as_float(u[0]) + __uint_as_float(u[1]), __uint_as_float(v[0]) + __uint_as_float(v[1]));
+                if (nw > 1) {
+                    s_part[(par * nw + wave) * 64 + lane] = r;
+                    lds_only_barrier();
+                    if (turn == wave) {
+                        r = make_float2(0.f, 0.f);
+                        for (int w = 0; w < nw; w++) {
+                            const float2 q2 = s_part[(par * nw + w) * 64 + lane];
+                            r.x += q2.x; r.y += q2.y;
+                        }
+                    }
+                }
+                typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+                const auto rs = __builtin_amdgcn_make_buffer_rsrc(a.res + (set * a.nres + e_lo + i0) * 2, 0,
+                                                                  turn == wave ? min(cnt - i0, 32) * res_bytes : 0, 0x00020000);
+                __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(r.x), __float_as_uint(r.y)}, rs, n * 16 + h * 8, 0, 0);
+                par ^= 1;
+                if (++turn == nw) turn = 0;
+            }
+            e0 = e1; a0 = a1;
+            e1 = e2; a1 = a2;
+        };
+        for (int i0 = 0; i0 < cnt; i0 += 32) step(i0, row_a);
+        if (zi + 1 < zi_hi) begin(zi + 1);
+        if (want_gx) flush_plane(z);
+    }
+    if (want_gx) flush_plane(zi_hi - 1);
+    if (bad_from >= zi_hi || !want_gx) return;
+    // (as in brick_grad_kernel; lane = channel)
+    for (int zi = max(bad_from, zi_lo); zi < zi_hi; zi++) {
+        const int sg = brick_seg(a.d, bg, zi, by, bx);
+        const int np = __builtin_amdgcn_readfirstlane(seg_count[sg]), lo = __builtin_amdgcn_readfirstlane(seg_end[sg]) - np;
+        for (int i = 0; i < np; i += 64) {
+            const int e = lo + min(i + lane, np - 1);
+            const uint4 q = a.L.pt[e];
+            const float al = a.L.alpha[e];
+            for (int j = 0; j < min(np - i, 64); j++) {
+                const PointValues p = point_of_lane(q, al, j, y0, x0);
+                if (h) continue;
+                const float gv = rows_in[(long)cc0 * a.chunk_rows * 32 + (p.row >> 2) + n];
+                for (int c = 0; c < 8; c++) {
+                    const int z = zi - 1 + (c >> 2), y = p.y + ((c >> 1) & 1), x = p.x + (c & 1);
+                    const float wz = c & 4 ? p.hz : 1.f - p.hz, wy = c & 2 ? p.hy : 1.f - p.hy, wx = c & 1 ? p.hx : 1.f - p.hx;
+                    if (wz > 0.f && wy > 0.f && wx > 0.f && z >= bad_from && z >= 0 && z < a.D && y >= 0 && y < a.H && x >= 0 && x < a.W)
+                        atomicAdd(a.gxcl + ((long)b * a.vol + ((long)z * a.H + y) * a.W + x) * a.Cin + cc0 * 32 + n, p.alpha * wz * wy * wx * gv);
                 }
             }
         }
@@ -942,7 +1281,7 @@ SortWindow sort_window(const TiledShape &s, const BrickDims &d)
     shrink(w.wx, 1, (long)w.wz * w.wy, kSortSlots);
     return w;
 }
-int brick_sets(const TiledShape &s) { return (s.cpg / 64 + kMaxWaves - 1) / kMaxWaves; }
+int brick_sets(const TiledShape &s) { return (s.cpg / s.bkc + kMaxWaves - 1) / kMaxWaves; }
 BrickLists brick_lists(const TiledShape &s, char *base)
 {
     const BrickWs w = d2c_brick_ws(s);
@@ -952,11 +1291,12 @@ BrickLists brick_lists(const TiledShape &s, char *base)
 
 }  // namespace
 
-// The bricks serve bfloat16 problems in three dimensions whose blocks hold enough points to fill most of a matrix
+// The bricks serve problems in three dimensions whose blocks hold enough points to fill most of a matrix
 // product of 32: below about half a product on average (few taps, strided outputs) the gathering kernels are as good.
+// (Float32: grad_input, grad_offset and grad_mask; sampled columns are bfloat16 only.)
 bool d2c_brick_supported(const TiledShape &s, int dtype)
 {
-    if (s.nd != 3 || dtype != D2C_BF16 || s.cpg % 64) return false;
+    if (s.nd != 3 || (dtype != D2C_BF16 && dtype != D2C_F32) || s.cpg % s.bkc) return false;
     return brick_mean(s) >= 16.0 && s.K <= 65535 && (long)s.N * s.G <= 65535 && brick_nseg(s) < (1L << 31) - 1024 &&
            brick_points(s) < (1L << 31) - 64 && (size_t)s.K * (s.M + 64) * 128 < 0xFFFFFF00u &&
            (size_t)s.H * s.W * s.Cin * 4 < 0xFFFFFFF0u;
@@ -1015,10 +1355,10 @@ int d2c_brick_grad(const TiledShape &s, const void *xcl, const void *gcol, const
     const long n = brick_points(s);
     BrickArgs a{};
     a.d = brick_dims(s); a.L = brick_lists(s, (char *)const_cast<void *>(lists));
-    a.xcl = (const bf16_t *)xcl; a.gcol = (const bf16_t *)gcol; a.gxcl = gxcl;
+    a.xcl = xcl; a.gcol = gcol; a.gxcl = gxcl;
     a.res = (goff || gmask) ? (float2 *)res : nullptr;
     a.nres = (long)(d2c_align_up((size_t)n * 16) / 16);
-    a.G = s.G; a.cpc = s.cpg / 64; a.Cin = s.Cin; a.D = s.D; a.H = s.H; a.W = s.W; a.vol = s.vol;
+    a.G = s.G; a.cpc = s.cpg / s.bkc; a.Cin = s.Cin; a.D = s.D; a.H = s.H; a.W = s.W; a.vol = s.vol;
     a.chunk_rows = (long)s.K * s.M;
     a.nset = brick_sets(s);
     const int nw = (a.cpc + a.nset - 1) / a.nset;
@@ -1030,8 +1370,10 @@ int d2c_brick_grad(const TiledShape &s, const void *xcl, const void *gcol, const
     a.nzr = (a.d.nz + a.zlen - 1) / a.zlen;
     const unsigned grid = (unsigned)(cols * a.nzr);
     {
-        D2cProfScope prof(D2C_PROF_BWD_AUX, st, "brick_grad_kernel");
-        hipLaunchKernelGGL(brick_grad_kernel, dim3(grid), dim3(64 * nw), nw * kWaveLds + (nw > 1 ? nw * 1024 : 0), st, a, a.L.end, a.L.count);
+        D2cProfScope prof(D2C_PROF_BWD_AUX, st, s.bkc == 64 ? "brick_grad_kernel" : "brick_grad_f32_kernel");
+        const int lds = nw * (s.bkc == 64 ? kWaveLds : kWaveLdsF) + (nw > 1 ? nw * 1024 : 0);
+        auto kern = s.bkc == 64 ? &brick_grad_kernel : &brick_grad_f32_kernel;
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * nw), lds, st, a, a.L.end, a.L.count);
         if (int rc = d2c_check_launch("brick_grad_kernel")) return rc;
     }
     if (!a.res) return D2C_OK;

@@ -633,7 +633,10 @@ bool use_aux_kernel(const d2c_conv3d_desc &q, const TiledShape &s)
 // at hand.  (A bucket capacity asked for by the test hook is a matter of the lists.)
 bool use_brick(const d2c_conv3d_desc &q, const TiledShape &s)
 {
-    return d2c_gx_mode() == 1 && use_lists(q, s) && use_aux_kernel(q, s) && d2c_brick_supported(s, q.dtype);
+    // (float32 weight groups that take several passes of the grad-column product keep the lists: what those groups run is pinned by a test,
+    // and the products are most of their time, 64 -> 512 channels on 8x40x50 715 us, 640)
+    return d2c_gx_mode() == 1 && use_lists(q, s) && use_aux_kernel(q, s) && d2c_brick_supported(s, q.dtype) &&
+           (q.dtype == D2C_BF16 || d2c_tiled_bwd_single_pass(s, q.dtype));
 }
 
 // The forward pass over sampled columns: sort, sample, multiply.  `kept`: the caller keeps the columns, where the backward call can
@@ -651,7 +654,7 @@ bool use_brick_forward(const d2c_conv3d_desc &q, const TiledShape &s, bool kept)
 {
     const long chunks = s.Cin / 64, of_group = s.cpg / 64;
     const bool large = kept ? s.M >= 400 && s.M * chunks >= 2048 : of_group >= 4 && s.M >= 4096 && s.M * of_group >= 32768;
-    return large && use_brick(q, s) && s.groups == 1 && brick_col_bytes(s) < (4ull << 30) &&
+    return large && q.dtype == D2C_BF16 && use_brick(q, s) && s.groups == 1 && brick_col_bytes(s) < (4ull << 30) &&
            (!kept || d2c_bwd_weight_from_kept_col(s, q.dtype));
 }
 
@@ -666,7 +669,10 @@ int gw_mode(const d2c_conv3d_desc &q)
 }
 bool use_col_weight(const d2c_conv3d_desc &q, const TiledShape &s)
 {
-    if (q.dtype != D2C_BF16 && gw_mode(q) != 1) return false;
+    // (float32 over sorted points samples again: those kernels write no columns, and the ones that do take longer than the second
+    // sampling saves.  Training steps, us, sorted points first: 64 -> 64 channels on 4x14x25 130, 136; 256 -> 256 on 4x9x9 181, 232;
+    // 1024 -> 128 on 8x20x32 1730, 1808)
+    if (q.dtype != D2C_BF16 && (gw_mode(q) != 1 || ((q.backward_flags & D2C_BWD_GW_MASK) == D2C_BWD_GW_DEFAULT && use_brick(q, s)))) return false;
     return gw_mode(q) && use_aux_kernel(q, s) && d2c_bwd_weight_from_col(s, q.dtype);
 }
 // ... written over the grad-column rows (mode 2): grad_input is taken from those rows first, from sample lists
@@ -704,7 +710,10 @@ BwdSlices bwd_slices(const d2c_conv3d_desc &q, const TiledShape &s)
 // `saved_columns`: the caller brings the sampled columns of the forward call (no column region, no slices)
 bool brick_backward(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns)
 {
-    return use_brick(q, s) && (saved_columns || (gw_mode(q) != 2 && bwd_slices(q, s).gs == 0));
+    if (!use_brick(q, s)) return false;
+    if (saved_columns) return true;
+    // (float32 columns come from the gathering kernel)
+    return gw_mode(q) != 2 && bwd_slices(q, s).gs == 0 && !(q.dtype == D2C_F32 && use_col_weight(q, s));
 }
 
 struct BwdWs {
@@ -815,7 +824,18 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
     const bool wt_prep = prep && pl.wt_bytes > 0;
     char *wt_p = wt_prep ? (char *)prep->base + pl.wt : base + l.wt;
     const bool wt_packed = wt_prep && (prep->reuse & D2C_REUSE_BACKWARD_WEIGHTS);
-    if (!have_x)
+    if (brick && sizeof(T) == 4) {
+        // one launch: the input with the row of zeros behind it, the clear of what is added into, the bias gradient
+        PrepArgs pa{};
+        if (!have_x) {
+            prep_pack<T>(pa.pack[0], x, xcl_p, s.N, s.Cin, s.vol);
+            pa.zrow = (uint32_t *)((T *)xcl_p + (size_t)s.N * s.vol * s.Cin); pa.zrow_words = 64;
+        }
+        if (gx) prep_zero(pa, base + l.gxcl, (size_t)s.N * s.vol * s.Cin * sizeof(float));
+        pa.gout = gout; pa.gb = gb; pa.bN = s.N; pa.bC = s.Cout; pa.bP = s.P; pa.nblk_b = gb ? s.Cout : 0;
+        if (int rc = prep_launch<T>(pa, st)) return rc;
+        gb = nullptr;
+    } else if (!have_x)
         if (int rc = pack_input<T>(s, x, xcl_p, st, true)) return rc;   // with the row of zeros behind it
     if (s.ss.on && !(brick && sorted && (goff || gmask || gx))) {
         D2cProfScope prof(D2C_PROF_PACK, st);
@@ -920,7 +940,7 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
                 if (int rc = (auxk && !gw_in_place) ? d2c_lists_clear(L, st) : d2c_lists_build(s, off, mask, L, st)) return rc;
             }
             const bool grad_col = brick && !prep && d2c_grad_col_supported(q);
-            if (brick && s.groups == 1) {
+            if (brick && sizeof(T) == 2 && s.groups == 1) {
                 // grad_out and the weights in the orders of the products, the bias gradient, what is added into cleared
                 gw_ready = gw_from_col;
                 if (int rc = d2c_brick_bwd_prepare(q, gout, w, grad_col ? base + l.gemm : nullptr, gw_ready ? base + l.goutp : nullptr, gb,
@@ -928,7 +948,7 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
                                                    gw_ready ? base + l.gwacc : nullptr, (size_t)s.Cout * s.cg * s.K * sizeof(float), st))
                     return rc;
                 gb = nullptr;
-            } else if (brick && gxcl) {
+            } else if (brick && sizeof(T) == 2 && gxcl) {
                 D2cProfScope prof(D2C_PROF_PACK, st);
                 d2c_fill_zero(gxcl, (size_t)s.N * s.vol * s.Cin * sizeof(float), st);
             }

@@ -1166,13 +1166,20 @@ __global__ void __launch_bounds__(kThreads + 64) tiled_bwd_weight_dma_kernel(Bwd
     const int o_base = otile * NT + wave * 64;
     const bool mma_wave = worker && o_base < s.og;
 
-    f32x16 acc[OB][CB];
+    // Float32: the sums of a tile of positions go into sums of their own, whose roundings do not add up over the whole
+    // piece (relative error of grad_weight against 64 bits, 256 -> 64 channels on 4x20x32: 1.18e-6 -> 9.1e-7).
+    constexpr bool TILE_SUMS = sizeof(T) == 4 && !SPLIT;
+    f32x16 acc[OB][CB], sum[TILE_SUMS ? OB : 1];
 #pragma unroll
     for (int ob = 0; ob < OB; ob++)
 #pragma unroll
         for (int cb = 0; cb < CB; cb++)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[ob][cb][r] = 0.f;
+    if constexpr (TILE_SUMS) {
+#pragma unroll
+        for (int ob = 0; ob < OB; ob++) sum[ob] = acc[ob][0];
+    }
 
     // --- coordinate wavefront: lane = position of tile i.  The tap is the workgroup's own: its constants are formed
     // once; an iteration takes the position apart (multiplications, no division) and builds the table row.
@@ -1379,6 +1386,13 @@ __global__ void __launch_bounds__(kThreads + 64) tiled_bwd_weight_dma_kernel(Bwd
                 for (int ob = 0; ob < OB; ob++) ld[kq * 2 + ob] = gfrag(i + 1, kg + 4 - NKG, ob);
             }
         }
+        if constexpr (TILE_SUMS) {
+            static_assert(!TILE_SUMS || CB == 1, "one block of channels");
+#pragma unroll
+            for (int ob = 0; ob < OB; ob++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) { sum[ob][r] += acc[ob][0][r]; acc[ob][0][r] = 0.f; }
+        }
     };
 
     if (nmy > 0) {
@@ -1435,7 +1449,7 @@ __global__ void __launch_bounds__(kThreads + 64) tiled_bwd_weight_dma_kernel(Bwd
                     const int ol = o_base + ob * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
                     if (ol < s.og)
                         atomicAdd(a.gwacc + (((long)wg * s.nchunk * s.K + st) * s.og + ol) * BKC + cb * 32 + (lane & 31),
-                                  acc[ob][cb][r]);
+                                  TILE_SUMS ? sum[TILE_SUMS ? ob : 0][r] : acc[ob][cb][r]);
                 }
     }
 }
