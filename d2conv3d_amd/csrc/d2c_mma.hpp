@@ -48,6 +48,33 @@ D2C_DEV uint32_t pack_bf16x2(float lo, float hi)
     return __builtin_bit_cast(uint32_t, r);
 }
 
+// in [rows][cols] -> out [cols][rows], float32: a 64 x 64 tile through LDS with 16-byte accesses on both sides, by 256 threads
+// (the 4-byte accesses of 32 x 32 tiles keep a quarter of the bytes in flight: 2 x 256 x 12960 elements of grad_input 16 us, 9);
+// rows and cols are multiples of 4, both tensors 16-byte aligned.  (Bank of an element: row stride 65 words, so that 16 vectors x 4 rows
+// meet 64 banks either way.)
+constexpr int kTransposeLds = 64 * 65 * 4;             // [column][row]
+D2C_DEV void transpose_tile64(float *tile, const float *in, float *out, int rows, int cols, int r0, int c0)
+{
+#pragma unroll
+    for (int k = 0; k < 4; k++) {                      // 64 rows x 16 vectors of 4 columns
+        const int i = k * 256 + threadIdx.x, r = r0 + i / 16, c = c0 + (i % 16) * 4;
+        if (r < rows && c < cols) {
+            const float4 q = *reinterpret_cast<const float4 *>(in + (long)r * cols + c);
+            float *t = tile + (i % 16) * 4 * 65 + i / 16;
+            t[0] = q.x; t[65] = q.y; t[130] = q.z; t[195] = q.w;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; k++) {                      // 64 columns x 16 vectors of 4 rows
+        const int i = k * 256 + threadIdx.x, c = c0 + i / 16, r = r0 + (i % 16) * 4;
+        if (r < rows && c < cols) {
+            const float *t = tile + (i / 16) * 65 + (i % 16) * 4;
+            *reinterpret_cast<float4 *>(out + (long)c * rows + r) = make_float4(t[0], t[1], t[2], t[3]);
+        }
+    }
+}
+
 // ---- float problems on the bfloat16 matrix instruction ---------------------------------------------------------
 // The float MFMA (v_mfma_f32_32x32x2_f32) runs at 1/16 of the bfloat16 rate.  In the FORWARD kernels a float MFMA
 // operand therefore travels as TWO bfloat16 values per element, v ~ hi + lo with hi = bf16(v) and lo = bf16(v - hi)

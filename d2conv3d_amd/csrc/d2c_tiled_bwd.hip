@@ -2025,6 +2025,12 @@ __global__ void __launch_bounds__(256) pack_weight_bwd_lds_kernel(const T *w, T 
     }
 }
 
+__global__ void __launch_bounds__(256) unpack_grad_input_f32_kernel(const float *gxcl, float *gx, int C, int vol)
+{
+    __shared__ float tile[kTransposeLds / 4];
+    const long bo = (long)blockIdx.z * C * vol;
+    transpose_tile64(tile, gxcl + bo, gx + bo, vol, C, blockIdx.x * 64, blockIdx.y * 64);
+}
 // fp32 channels-last accumulator [N][vol][C] -> grad_input [N][C][vol] of type T
 template <typename T>
 __global__ void __launch_bounds__(256) unpack_grad_input_kernel(const float *gxcl, T *gx, int C, int vol)
@@ -2599,6 +2605,10 @@ int d2c_tiled_unpack_gx(const TiledShape &s, const float *gxcl, void *gx, hipStr
                                st, gxcl, (bf16_t *)gx, s.Cin, s.vol);
             return d2c_check_launch("unpack_grad_input_bf16_kernel");
         }
+    } else if (s.vol % 4 == 0 && s.Cin % 4 == 0 && reinterpret_cast<uintptr_t>(gx) % 16 == 0) {
+        hipLaunchKernelGGL(unpack_grad_input_f32_kernel, dim3((s.vol + 63) / 64, (s.Cin + 63) / 64, s.N), dim3(256), 0, st, gxcl,
+                           (float *)gx, s.Cin, s.vol);
+        return d2c_check_launch("unpack_grad_input_f32_kernel");
     }
     hipLaunchKernelGGL(unpack_grad_input_kernel<T>, grid, dim3(256), 0, st, gxcl, (T *)gx, s.Cin, s.vol);
     return d2c_check_launch("unpack_grad_input_kernel");
