@@ -102,7 +102,7 @@ D2C_DEV float bf16_residual(float v, uint32_t hi_bits)
 {
     const float h = __uint_as_float(hi_bits);
     // (an infinite value keeps its infinity in `hi` alone)
-    return (__float_as_uint(h) & 0x7fffffffu) == 0x7f800000u ? 0.f : v - h;
+    return __builtin_amdgcn_classf(h, 0x204) ? 0.f : v - h;
 }
 D2C_DEV uint4 split_f32x4(float v0, float v1, float v2, float v3)
 {

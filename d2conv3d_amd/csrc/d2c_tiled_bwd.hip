@@ -1691,7 +1691,7 @@ __global__ void __launch_bounds__(kThreads) tiled_bwd_weight_col_kernel(BwdWeigh
 // The same product for float problems on the bfloat16 matrix instruction, with float32's accuracy: every float is
 // taken apart into THREE bfloat16 terms, v = h + m + l exactly (8 + 8 + 8 significant bits), and of the nine partial
 // products of a pair the six largest are summed,
-//     h h' + m h'   |   h m' + m m'   |   l h' + h l'
+//     h h' + h m'   |   m h' + m m'   |   l h' + h l'       (grad_out first)
 // three v_mfma_f32_32x32x16_bf16 per 8 positions (each 16-deep reduction holds two partial products of 8 pairs)
 // against four v_mfma_f32_32x32x2_f32 of twice their length: 3/8 of the matrix-pipe time.  What is dropped
 // (m l' + l m' + l l') is below 2^-25 of a product, under float32's own rounding.  The first instruction carries the
@@ -1702,17 +1702,22 @@ __global__ void __launch_bounds__(kThreads) tiled_bwd_weight_col_kernel(BwdWeigh
 // looping over its piece of the 64-position tiles like tiled_bwd_weight_col_kernel.  The float columns are taken
 // apart where they are stored to LDS -- three planes [position][32 channels] of bfloat16 per chunk, read with the
 // transposing LDS load -- and grad_out comes from a fragment-ordered copy that holds the three terms (pack_gout3_kernel).
+// The vector ALU has about half as much to do as the matrix pipes: columns come apart in pairs (the hardware's conversion of two, 26 + 8
+// instructions for four floats; rounding in software, three times as many, cost 668 us against 533 for 256 x 256 channels,
+// 27 taps, 25920 positions), and of the products' operands it is grad_out's that are doubled, once per four column tiles (533 -> 519).
 constexpr int kCol3Chunks = 4;
 constexpr int kCol3Rows = 256;     // output channels per workgroup
 constexpr size_t kCol3Lds = (size_t)2 * kCol3Chunks * 3 * kWDT * 64;
 
-// v -> (h, m, l), bfloat16 bits
-D2C_DEV void split3(float v, uint32_t &h, uint32_t &m, uint32_t &l)
+// four floats -> their terms, pairs to a word: h the nearest bfloat16, m and l those of what is left
+D2C_DEV void split3(float v0, float v1, float v2, float v3, uint2 &h, uint2 &m, uint2 &l)
 {
-    h = f32_to_bf16(v);
-    const float r1 = bf16_residual(v, h << 16);
-    m = f32_to_bf16(r1);
-    l = f32_to_bf16(r1 - __uint_as_float(m << 16));
+    auto rest = [](float v, uint32_t bits) { return v - __uint_as_float(bits); };
+    h = make_uint2(pack_bf16x2(v0, v1), pack_bf16x2(v2, v3));
+    v0 = bf16_residual(v0, h.x << 16); v1 = bf16_residual(v1, h.x & 0xffff0000u);
+    v2 = bf16_residual(v2, h.y << 16); v3 = bf16_residual(v3, h.y & 0xffff0000u);
+    m = make_uint2(pack_bf16x2(v0, v1), pack_bf16x2(v2, v3));
+    l = make_uint2(pack_bf16x2(rest(v0, m.x << 16), rest(v1, m.x & 0xffff0000u)), pack_bf16x2(rest(v2, m.y << 16), rest(v3, m.y & 0xffff0000u)));
 }
 
 // grad_out [N][Cout][P] -> fragments of the three terms, indexed like pack_gout_kernel's (float: 16 k-groups of 8
@@ -1732,19 +1737,19 @@ __global__ void __launch_bounds__(256) pack_gout3_kernel(const float *gout, uint
         const int wg = (int)(r / ntile);
         const int ol = ob * 32 + (lane & 31);
         const long m0 = (long)tile * kWMT + (2 * kg + (lane >> 5)) * VEC;
-        uint32_t h[VEC], m[VEC], l[VEC];
+        float v[VEC] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int q = 0; q < VEC; q++) {
             const long mm = m0 + q;
-            float v = 0.f;
             if (ol < s.og && mm < s.M) {
                 const int b = (int)(mm / s.P), pp = (int)(mm - (long)b * s.P);
-                v = gout[((long)b * s.Cout + wg * s.og + ol) * s.P + pp];
+                v[q] = gout[((long)b * s.Cout + wg * s.og + ol) * s.P + pp];
             }
-            split3(v, h[q], m[q], l[q]);
         }
-        lh[i] = make_uint4(l[0] | (l[1] << 16), l[2] | (l[3] << 16), h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-        md[i] = make_uint2(m[0] | (m[1] << 16), m[2] | (m[3] << 16));
+        uint2 h, m, l;
+        split3(v[0], v[1], v[2], v[3], h, m, l);
+        lh[i] = make_uint4(l.x, l.y, h.x, h.y);
+        md[i] = m;
     }
 }
 
@@ -1810,15 +1815,12 @@ __global__ void __launch_bounds__(kThreads) tiled_bwd_weight_col3_kernel(BwdWeig
     uint4 cr[NCH];       // the tile after the one on the matrix cores, requested a whole step before it is stored
     unsigned char *const st_p = s_tile + ipos * 64 + ivec * 8;
     auto put = [&](int buf, int c, const uint4 &v) {
-        uint32_t h[4], m[4], l[4];
-        split3(__uint_as_float(v.x), h[0], m[0], l[0]);
-        split3(__uint_as_float(v.y), h[1], m[1], l[1]);
-        split3(__uint_as_float(v.z), h[2], m[2], l[2]);
-        split3(__uint_as_float(v.w), h[3], m[3], l[3]);
+        uint2 h, m, l;
+        split3(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w), h, m, l);
         unsigned char *d = st_p + ((buf * NCH + c) * 3) * PLANE;
-        *reinterpret_cast<uint2 *>(d) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-        *reinterpret_cast<uint2 *>(d + PLANE) = make_uint2(m[0] | (m[1] << 16), m[2] | (m[3] << 16));
-        *reinterpret_cast<uint2 *>(d + 2 * PLANE) = make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
+        *reinterpret_cast<uint2 *>(d) = h;
+        *reinterpret_cast<uint2 *>(d + PLANE) = m;
+        *reinterpret_cast<uint2 *>(d + 2 * PLANE) = l;
     };
 
     // --- grad_out fragments of this wavefront's 32 rows
@@ -1869,17 +1871,16 @@ __global__ void __launch_bounds__(kThreads) tiled_bwd_weight_col3_kernel(BwdWeig
                 for (int kg = 0; kg < NKG; kg++) {
                     const int q = kg % LAK;
                     const uint4 a_lh = alh[q];
-                    const uint4 a_hm = make_uint4(alh[q].z, alh[q].w, amd[q].x, amd[q].y);
+                    const uint4 a_hh = make_uint4(a_lh.z, a_lh.w, a_lh.z, a_lh.w), a_mm = make_uint4(amd[q].x, amd[q].y, amd[q].x, amd[q].y);
 #pragma unroll
                     for (int cb = 0; cb < CB; cb++) {
                         const unsigned char *bp = rd_p + ((dbuf * NCH + cb) * 3) * PLANE + kg * 8 * 64;
                         const uint2 bh = tr(bp), bm = tr(bp + PLANE), bl = tr(bp + 2 * PLANE);
-                        const uint4 b_hh = make_uint4(bh.x, bh.y, bh.x, bh.y), b_mm = make_uint4(bm.x, bm.y, bm.x, bm.y);
-                        const uint4 b_hl = make_uint4(bh.x, bh.y, bl.x, bl.y);
-                        big[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a_hm),
-                                                                          __builtin_bit_cast(bf16x8_t, b_hh), big[cb], 0, 0, 0);
-                        small[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a_hm),
-                                                                            __builtin_bit_cast(bf16x8_t, b_mm), small[cb], 0, 0, 0);
+                        const uint4 b_hm = make_uint4(bh.x, bh.y, bm.x, bm.y), b_hl = make_uint4(bh.x, bh.y, bl.x, bl.y);
+                        big[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a_hh),
+                                                                          __builtin_bit_cast(bf16x8_t, b_hm), big[cb], 0, 0, 0);
+                        small[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a_mm),
+                                                                            __builtin_bit_cast(bf16x8_t, b_hm), small[cb], 0, 0, 0);
                         small[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a_lh),
                                                                             __builtin_bit_cast(bf16x8_t, b_hl), small[cb], 0, 0, 0);
                     }
