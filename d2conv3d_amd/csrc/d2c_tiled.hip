@@ -302,9 +302,11 @@ struct PrepArgs {
     const void *w;
     void *wt;
     int wkind, wC, wK, nblk_w;
-    uint32_t *zero;
-    size_t zero_words;
-    int nblk_z;
+    struct Zero {
+        uint32_t *p;
+        size_t words;
+        int nblk;
+    } zero[3];
     const void *gout;          // bias gradient: one workgroup per channel
     void *gb;
     int bN, bC, bP, nblk_b;
@@ -349,11 +351,15 @@ template <typename T, bool WIDE> __global__ void __launch_bounds__(256) prepare_
         return;
     }
     b -= a.nblk_w;
-    if (b < a.nblk_z) {
-        for (size_t i = (size_t)b * 256 + threadIdx.x; i < a.zero_words; i += (size_t)a.nblk_z * 256) a.zero[i] = 0u;
-        return;
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        const PrepArgs::Zero &z = a.zero[j];
+        if (b < z.nblk) {
+            for (size_t i = (size_t)b * 256 + threadIdx.x; i < z.words; i += (size_t)z.nblk * 256) z.p[i] = 0u;
+            return;
+        }
+        b -= z.nblk;
     }
-    b -= a.nblk_z;
     if (b < a.nblk_b) bias_grad_body<T, 256>((const T *)a.gout, (T *)a.gb, a.bN, a.bC, a.bP, b);
 }
 
@@ -485,10 +491,9 @@ template <typename T> void prep_pack(PrepArgs::Pack &pk, const void *src, void *
     pk.nbx = (vol + tl - 1) / tl; pk.nby = (C + tl - 1) / tl;
     pk.nblk = pk.nbx * pk.nby * N;
 }
-void prep_zero(PrepArgs &a, void *p, size_t bytes)
+void prep_zero(PrepArgs &a, int j, void *p, size_t bytes)
 {
-    a.zero = (uint32_t *)p; a.zero_words = bytes / 4;
-    a.nblk_z = (int)std::min<size_t>((a.zero_words + 1023) / 1024, 2048);
+    a.zero[j] = PrepArgs::Zero{(uint32_t *)p, bytes / 4, (int)std::min<size_t>((bytes / 4 + 1023) / 1024, 2048)};
 }
 template <typename T> void prep_weight_fwd(PrepArgs &a, const TiledShape &s, const void *w, void *wp)
 {
@@ -504,7 +509,7 @@ template <typename T> void prep_weight_fwd(PrepArgs &a, const TiledShape &s, con
 }
 template <typename T> int prep_launch(const PrepArgs &a, hipStream_t st)
 {
-    const long nblk = (long)a.pack[0].nblk + a.pack[1].nblk + a.nblk_w + a.nblk_z + a.nblk_b;
+    const long nblk = (long)a.pack[0].nblk + a.pack[1].nblk + a.nblk_w + a.zero[0].nblk + a.zero[1].nblk + a.zero[2].nblk + a.nblk_b;
     if (nblk == 0) return D2C_OK;
     D2cProfScope prof(D2C_PROF_PACK, st);
     const bool wide = sizeof(T) == 4 && (a.pack[0].wide || a.pack[1].wide);
@@ -524,7 +529,7 @@ int dw_prepare(const TiledShape &s, const void *x, void *xcl, const void *gout, 
     a.wkind = PREP_W_DEPTHWISE; a.w = w; a.wt = wt; a.wC = s.Cin; a.wK = s.K;
     a.nblk_w = std::min((s.Cin * s.K + 255) / 256, 1024);
     a.zrow = (uint32_t *)((T *)xcl + (size_t)s.N * s.vol * s.Cin); a.zrow_words = s.Cin * (int)sizeof(T) / 4;
-    prep_zero(a, zero, zero_bytes);
+    prep_zero(a, 0, zero, zero_bytes);
     a.gout = gout; a.gb = gb; a.bN = s.N; a.bC = s.Cout; a.bP = s.P;
     a.nblk_b = (gb && gout) ? s.Cout : 0;
     return prep_launch<T>(a, st);
@@ -611,7 +616,7 @@ int forward_t(const d2c_conv3d_desc &q, const void *x, const void *off, const vo
     if (!(prep && (prep->reuse & D2C_REUSE_FORWARD_WEIGHTS))) prep_weight_fwd<T>(pa, s, w, wp_p);
     const size_t split = d2c_fwd_split_bytes(s);
     const bool shared = d2c_fwd_use_dma(s) || (split && (nd != 3 || ws_bytes >= l.outacc + split));
-    if (shared && split) prep_zero(pa, base + l.outacc, d2c_fwd_split_count_bytes(s));
+    if (shared && split) prep_zero(pa, 0, base + l.outacc, d2c_fwd_split_count_bytes(s));
     if (int rc = prep_launch<T>(pa, st)) return rc;
     // (the per-tile sums of the output statistics go behind everything else in the workspace)
     return d2c_tiled_fwd_launch<T>(s, xcl_p, off, mask, wp_p, bias, out, shared ? (float *)(base + l.outacc) : nullptr, st,
@@ -834,6 +839,7 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
     const bool wt_prep = prep && pl.wt_bytes > 0;
     char *wt_p = wt_prep ? (char *)prep->base + pl.wt : base + l.wt;
     const bool wt_packed = wt_prep && (prep->reuse & D2C_REUSE_BACKWARD_WEIGHTS);
+    bool gw_cleared = false;
     if (brick && sizeof(T) == 4) {
         // one launch: the input with the row of zeros behind it, the clear of what is added into, the bias gradient
         PrepArgs pa{};
@@ -841,7 +847,16 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
             prep_pack<T>(pa.pack[0], x, xcl_p, s.N, s.Cin, s.vol);
             pa.zrow = (uint32_t *)((T *)xcl_p + (size_t)s.N * s.vol * s.Cin); pa.zrow_words = 64;
         }
-        if (gx) prep_zero(pa, base + l.gxcl, (size_t)s.N * s.vol * s.Cin * sizeof(float));
+        if (gx) prep_zero(pa, 0, base + l.gxcl, (size_t)s.N * s.vol * s.Cin * sizeof(float));
+        if (gx || goff || gmask) {
+            size_t zb;
+            void *const zp = d2c_brick_zero(s, base + l.brick, &zb);
+            prep_zero(pa, 1, zp, zb);
+        }
+        if (gw) {
+            prep_zero(pa, 2, base + l.gwacc, (size_t)s.Cout * s.cg * s.K * sizeof(float));
+            gw_cleared = true;
+        }
         pa.gout = gout; pa.gb = gb; pa.bN = s.N; pa.bC = s.Cout; pa.bP = s.P; pa.nblk_b = gb ? s.Cout : 0;
         if (int rc = prep_launch<T>(pa, st)) return rc;
         gb = nullptr;
@@ -944,7 +959,7 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
             char *const lists_p = sorted ? (char *)const_cast<void *>(columns) + brick_col_bytes(s) : base + l.brick;
             if (brick) {
                 if (!sorted)
-                    if (int rc = d2c_brick_sort(s, off, mask, lists_p, st)) return rc;
+                    if (int rc = d2c_brick_sort(s, off, mask, lists_p, st, sizeof(T) == 4)) return rc;
             } else if (lists) {
                 L = d2c_lists_make(s, Elem<T>::DT, base + l.counts, base + l.entries, base + l.ovf);
                 if (int rc = (auxk && !gw_in_place) ? d2c_lists_clear(L, st) : d2c_lists_build(s, off, mask, L, st)) return rc;
@@ -1017,7 +1032,7 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
             if (int rc = d2c_tiled_bwd_weight_launch<T>(s, gout, xcl_p, off, mask, base + l.goutp,
                                                        (float *)(base + l.gwacc),
                                                        gw, gw_from_col ? (columns ? (char *)columns : (gw_in_place ? base + l.gcol : base + l.col)) : nullptr,
-                                                       gw_in_place ? (long)s.M : (long)((s.M + 63) / 64) * 64, st, gw_ready ? 6 : 7))
+                                                       gw_in_place ? (long)s.M : (long)((s.M + 63) / 64) * 64, st, (gw_ready ? 6 : 7) | (gw_cleared ? 8 : 0)))
                 return rc;
         } else {
             if (int rc = d2c_generic_conv3d_backward(q, gout, x, off, mask, w, nullptr, nullptr, nullptr, gw, nullptr,

@@ -1724,7 +1724,7 @@ D2C_DEV void split3(float v0, float v1, float v2, float v3, uint2 &h, uint2 &m, 
 // positions per tile of kWMT): lh[i] = (l0 l1)(l2 l3)(h0 h1)(h2 h3) of the lane's four positions, md[i] = (m0 m1)(m2 m3);
 // `md` follows the `total` 16-byte entries of `lh`
 __global__ void __launch_bounds__(256) pack_gout3_kernel(const float *gout, uint4 *lh, TiledShape s, int ntile, int OBT,
-                                                         long total)
+                                                         long total, bool vec)
 {
     constexpr int VEC = 4, NKGT = kWMT / (2 * VEC);
     uint2 *md = reinterpret_cast<uint2 *>(lh + total);
@@ -1738,10 +1738,15 @@ __global__ void __launch_bounds__(256) pack_gout3_kernel(const float *gout, uint
         const int ol = ob * 32 + (lane & 31);
         const long m0 = (long)tile * kWMT + (2 * kg + (lane >> 5)) * VEC;
         float v[VEC] = {0.f, 0.f, 0.f, 0.f};
+        if (vec && ol < s.og && m0 < s.M) {          // (four positions of one sample, as one load)
+            const int b = (int)(m0 / s.P), pp = (int)(m0 - (long)b * s.P);
+            const float4 t = *reinterpret_cast<const float4 *>(gout + ((long)b * s.Cout + wg * s.og + ol) * s.P + pp);
+            v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+        }
 #pragma unroll
         for (int q = 0; q < VEC; q++) {
             const long mm = m0 + q;
-            if (ol < s.og && mm < s.M) {
+            if (!vec && ol < s.og && mm < s.M) {
                 const int b = (int)(mm / s.P), pp = (int)(mm - (long)b * s.P);
                 v[q] = gout[((long)b * s.Cout + wg * s.og + ol) * s.P + pp];
             }
@@ -2479,13 +2484,13 @@ int d2c_tiled_bwd_weight_launch(const TiledShape &s, const void *gout, const voi
     const long total = (long)s.groups * ntp * OBT * (kWMT / (2 * Elem<T>::VEC)) * 64;
     if ((phase & 1) && col3) {
         D2cProfScope prof(D2C_PROF_PACK, st);
-        d2c_fill_zero(gwacc, (size_t)nw * sizeof(float), st);
+        if (!(phase & 8)) d2c_fill_zero(gwacc, (size_t)nw * sizeof(float), st);
         hipLaunchKernelGGL(pack_gout3_kernel, dim3(grid1d(total, 16384)), dim3(256), 0, st, (const float *)gout,
-                           (uint4 *)goutp, s, ntp, OBT, total);
+                           (uint4 *)goutp, s, ntp, OBT, total, s.P % 4 == 0 && reinterpret_cast<uintptr_t>(gout) % 16 == 0);
         if (int rc = d2c_check_launch("pack_gout3_kernel")) return rc;
     } else if (phase & 1) {
         D2cProfScope prof(D2C_PROF_PACK, st);
-        d2c_fill_zero(gwacc, (size_t)nw * sizeof(float), st);
+        if (!(phase & 8)) d2c_fill_zero(gwacc, (size_t)nw * sizeof(float), st);
         // (the channels-last input is followed by a 256-byte row of zeros, written by the kernel that packed it:
         // what dead corners read)
         const bool vec = s.P % Elem<T>::VEC == 0 && reinterpret_cast<uintptr_t>(gout) % 16 == 0;
