@@ -343,10 +343,16 @@ struct BrickArgs {
 };
 
 constexpr int kMaxWaves = 4;
-constexpr int kWaveLds = 32 * 128 + 3 * 32 * 64;
+constexpr int kWeightLds = 3 * 32 * 64;                       // weights of 32 points
+constexpr int kRowLds = 32 * 128, kRowLdsF = 3 * 32 * 64;     // a wavefront's rows of 32 points; float32: as three terms
 D2C_DEV void lds_only_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 D2C_DEV void wave_fence() { asm volatile("" ::: "memory"); __builtin_amdgcn_wave_barrier(); }
 
+// The wavefronts of a workgroup need the same weights.  SHARE: they take turns in making those of the next 32 points, a step
+// ahead (the barrier in front of the sums over chunks keeps them in step), in two buffers of the workgroup; the first ones of a plane are waited for.
+// Else, where there is one wavefront or a plane has few points, a buffer for each, filled when it is wanted.  (us, each its own first: 256 channels on
+// 32x60x108, 27 taps, 862, 830; float32 on 2x8x30x54 283, 259; 2048 channels on 8x30x54, 7 taps, two steps to a plane, 230, 236.)
+template <bool SHARE>
 __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs a, const int *__restrict__ seg_end, const int *__restrict__ seg_count)
 {
     const int lane = threadIdx.x & 63, h = lane >> 5, n = lane & 31;
@@ -355,8 +361,8 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
     // permuted so that neither the row-wise accesses (16 lanes on the same piece of 16 rows) nor the transposing reads
     // (4 rows x 64 bytes) meet a bank twice.
     extern __shared__ __align__(16) unsigned char smem[];
-    unsigned char *const s_g = smem + wave * kWaveLds, *const s_w = s_g + 32 * 128;
-    float2 *const s_part = reinterpret_cast<float2 *>(smem + nw * kWaveLds);       // [2][wave][lane]: sums over a chunk each
+    unsigned char *const s_g = smem + wave * kRowLds, *const s_w = smem + nw * kRowLds + (SHARE ? 0 : wave * kWeightLds);
+    float2 *const s_part = reinterpret_cast<float2 *>(smem + nw * kRowLds + (SHARE ? 2 : nw) * kWeightLds);       // [2][wave][lane]: sums over a chunk each
     auto g_swz = [](int row) INLINE { return (((row >> 1) & 1) << 2) | (((row >> 2) & 1) << 1) | ((row >> 3) & 1); };
 
     // task: set of chunks, then block column along x, y, then z range, group and sample; an XCD takes a contiguous part of them
@@ -438,7 +444,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
     const unsigned w_st = lds_address(s_w) + n * 64 + (((h * 2) ^ ((n >> 2) & 3)) << 4);     // (^ 8 y: the lane's row y of voxels)
     const int tr_row = h * 8 + ((lane & 15) >> 2), tr_pc = ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1), tr_in = (lane & 1) * 8;
     const unsigned g_tr = lds_address(s_g) + tr_row * 128 + ((tr_pc ^ g_swz(tr_row)) << 4) + tr_in;
-    const unsigned w_tr = lds_address(s_w) + tr_row * 64 + ((tr_pc ^ (h * 2)) << 4) + tr_in;
+    unsigned w_tr = lds_address(s_w) + tr_row * 64 + ((tr_pc ^ (h * 2)) << 4) + tr_in;
     auto tr_read = [](unsigned addr) INLINE {
         return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s *)(size_t)addr));
     };
@@ -466,6 +472,25 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
         const int sg = brick_seg(a.d, bg, min(zi, zi_hi - 1), by, bx);
         r_lo = seg_end[sg]; r_n = seg_count[sg];
     };
+    // weights of points i .. (lane = point, the 16 voxels of slot h): rows yb, yb + 1 of four voxels, zeros in the other two
+    int wofs = 0;                                    // the buffer of this step's weights
+    auto weights = [&](const uint4 &e, float al, int i, int to, bool low) INLINE {
+        const unsigned yb = e.x & 3u, xs = (e.x & 12u) << 2;
+        const float hy = __uint_as_float(e.y), hx = __uint_as_float(e.z), hz = __uint_as_float(e.w);
+        const float wz = (i + n < cnt ? al : 0.f) * ((h != 0) == low ? 1.f - hz : hz);
+        const float wy0 = wz * (1.f - hy), wy1 = wz * hy, lx = 1.f - hx;
+        const WeightRow r0 = weight_row(wy0 * lx, wy0 * hx, xs), r1 = weight_row(wy1 * lx, wy1 * hx, xs);
+        typedef __attribute__((address_space(3))) unsigned long long *lds64;
+        const unsigned sy = yb << 3, st = w_st + to;
+        const unsigned at0 = st ^ sy, at1 = st ^ (sy + 8), at2 = st ^ ((sy + 16) & 24), at3 = st ^ ((sy + 24) & 24);
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+            *(lds64)(size_t)(at0 + q * 2048) = r0.t[q];
+            *(lds64)(size_t)(at1 + q * 2048) = r1.t[q];
+            *(lds64)(size_t)(at2 + q * 2048) = 0;
+            *(lds64)(size_t)(at3 + q * 2048) = 0;
+        }
+    };
     auto begin = [&](int zi) INLINE {
         cnt = __builtin_amdgcn_readfirstlane(r_n); e_lo = __builtin_amdgcn_readfirstlane(r_lo) - cnt;
         if (cnt > 0) {
@@ -479,7 +504,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
             rows(e1, row_b);
         }
     };
-    int par = 0, turn = 0;
+    int par = 0, turn = 0, turn2 = nw / 2;           // whose turn it is to store sums, to make weights
     range(zi_lo);
     load_plane(zi_lo - 1);
     begin(zi_lo);
@@ -487,6 +512,10 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
         const int z = zi - 1;
         const bool low = z & 1;                      // slot of the base plane
         range(zi + 1);
+        if (SHARE && cnt > 0) {
+            if (turn2 == wave) weights(e0, a0, 0, wofs, low);
+            lds_only_barrier();
+        }
         auto step = [&](int i0, u32x4_t (&row)[4]) INLINE {
             // the rows to LDS, others requested in their place.  (The entry first: loads complete in order, and it is
             // wanted first.  Past the last point: its row again.)
@@ -499,25 +528,10 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
             *(lds128)(size_t)((g_st ^ 16) + 3072) = row[3];
             rows(e2, row);
             __builtin_amdgcn_sched_barrier(0);
-            const bool ok = i0 + n < cnt;
             const unsigned yb = e0.x & 3u, xs = (e0.x & 12u) << 2;
             const float hy = __uint_as_float(e0.y), hx = __uint_as_float(e0.z), hz = __uint_as_float(e0.w), lz = 1.f - hz;
-            // ---- weights (lane = point, the 16 voxels of slot h): rows yb, yb + 1 of four voxels, zeros in the other two
-            {
-                const float wz = (ok ? a0 : 0.f) * ((h != 0) == low ? lz : hz);
-                const float wy0 = wz * (1.f - hy), wy1 = wz * hy, lx = 1.f - hx;
-                const WeightRow r0 = weight_row(wy0 * lx, wy0 * hx, xs), r1 = weight_row(wy1 * lx, wy1 * hx, xs);
-                typedef __attribute__((address_space(3))) unsigned long long *lds64;
-                const unsigned sy = yb << 3;
-                const unsigned at0 = w_st ^ sy, at1 = w_st ^ (sy + 8), at2 = w_st ^ ((sy + 16) & 24), at3 = w_st ^ ((sy + 24) & 24);
-#pragma unroll
-                for (int i = 0; i < 3; i++) {
-                    *(lds64)(size_t)(at0 + i * 2048) = r0.t[i];
-                    *(lds64)(size_t)(at1 + i * 2048) = r1.t[i];
-                    *(lds64)(size_t)(at2 + i * 2048) = 0;
-                    *(lds64)(size_t)(at3 + i * 2048) = 0;
-                }
-            }
+            if constexpr (!SHARE) weights(e0, a0, i0, 0, low);
+            else if (turn2 == wave && i0 + 32 < cnt) weights(e1, a1, i0 + 32, wofs ^ kWeightLds, low);
             wave_fence();
             // ---- the two products
             f32x16 T;
@@ -571,7 +585,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
                 const auto u = __builtin_amdgcn_permlane32_swap(__float_as_uint(r_m), __float_as_uint(r_z), false, false);
                 const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(r_x), __float_as_uint(r_y), false, false);
                 float2 r = make_float2(__uint_as_float(u[0]) + __uint_as_float(u[1]), __uint_as_float(v[0]) + __uint_as_float(v[1]));
-                if (nw > 1) {
+                if (SHARE || nw > 1) {
                     // the chunks of the other wavefronts, which take turns in adding up and storing
                     s_part[(par * nw + wave) * 64 + lane] = r;
                     lds_only_barrier();
@@ -590,6 +604,8 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_kernel(BrickArgs
                 __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(r.x), __float_as_uint(r.y)}, rs, n * 16 + h * 8, 0, 0);
                 par ^= 1;
                 if (++turn == nw) turn = 0;
+                if (++turn2 == nw) turn2 = 0;
+                if (SHARE) { w_tr += wofs ? -kWeightLds : kWeightLds; wofs ^= kWeightLds; }
             }
             e0 = e1; a0 = a1;
             e1 = e2; a1 = a2;
@@ -647,14 +663,14 @@ D2C_DEV void split3(float a, float b, uint32_t (&o)[3])
         a -= __uint_as_float(o[i] << 16); b -= __uint_as_float(o[i] & 0xffff0000u);
     }
 }
-constexpr int kWaveLdsF = 2 * 3 * 32 * 64;
+template <bool SHARE>
 __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_f32_kernel(BrickArgs a, const int *__restrict__ seg_end, const int *__restrict__ seg_count)
 {
     const int lane = threadIdx.x & 63, h = lane >> 5, n = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
     extern __shared__ __align__(16) unsigned char smem[];
-    unsigned char *const s_g = smem + wave * kWaveLdsF, *const s_w = s_g + 3 * 32 * 64;      // rows and weights: [term][point][32]
-    float2 *const s_part = reinterpret_cast<float2 *>(smem + nw * kWaveLdsF);                // [2][wave][lane]: sums over a chunk each
+    unsigned char *const s_g = smem + wave * kRowLdsF, *const s_w = smem + nw * kRowLdsF + (SHARE ? 0 : wave * kWeightLds);   // rows and weights: [term][point][32]
+    float2 *const s_part = reinterpret_cast<float2 *>(smem + nw * kRowLdsF + (SHARE ? 2 : nw) * kWeightLds);     // [2][wave][lane]: sums over a chunk each
 
     // task: as in brick_grad_kernel
     const int nt = (int)gridDim.x, xq = nt >> 3, xr = nt & 7, xcd = blockIdx.x & 7;
@@ -738,7 +754,8 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_f32_kernel(Brick
     const unsigned w_st = lds_address(s_w) + n * 64 + (((h * 2) ^ ((n >> 2) & 3)) << 4);
     const int tr_row = h * 8 + ((lane & 15) >> 2), tr_pc = ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1), tr_in = (lane & 1) * 8;
     const unsigned tr = tr_row * 64 + ((tr_pc ^ (h * 2)) << 4) + tr_in;
-    const unsigned g_tr = lds_address(s_g) + tr, w_tr = lds_address(s_w) + tr;
+    const unsigned g_tr = lds_address(s_g) + tr;
+    unsigned w_tr = lds_address(s_w) + tr;              // (of this step's buffer)
     auto tr_read = [](unsigned addr) INLINE {
         return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s *)(size_t)addr));
     };
@@ -767,6 +784,25 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_f32_kernel(Brick
         const int sg = brick_seg(a.d, bg, min(zi, zi_hi - 1), by, bx);
         r_lo = seg_end[sg]; r_n = seg_count[sg];
     };
+    // weights of points i .. (lane = point, the 16 voxels of slot h): rows yb, yb + 1 of four voxels, zeros in the other two
+    int wofs = 0;                                    // the buffer of this step's weights
+    auto weights = [&](const uint4 &e, float al, int i, int to, bool low) INLINE {
+        const unsigned yb = e.x & 3u, xs = (e.x & 12u) << 2;
+        const float hy = __uint_as_float(e.y), hx = __uint_as_float(e.z), hz = __uint_as_float(e.w);
+        const float wz = (i + n < cnt ? al : 0.f) * ((h != 0) == low ? 1.f - hz : hz);
+        const float wy0 = wz * (1.f - hy), wy1 = wz * hy, lx = 1.f - hx;
+        const WeightRow r0 = weight_row(wy0 * lx, wy0 * hx, xs), r1 = weight_row(wy1 * lx, wy1 * hx, xs);
+        typedef __attribute__((address_space(3))) unsigned long long *lds64;
+        const unsigned sy = yb << 3, st = w_st + to;
+        const unsigned at0 = st ^ sy, at1 = st ^ (sy + 8), at2 = st ^ ((sy + 16) & 24), at3 = st ^ ((sy + 24) & 24);
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+            *(lds64)(size_t)(at0 + q * 2048) = r0.t[q];
+            *(lds64)(size_t)(at1 + q * 2048) = r1.t[q];
+            *(lds64)(size_t)(at2 + q * 2048) = 0;
+            *(lds64)(size_t)(at3 + q * 2048) = 0;
+        }
+    };
     auto begin = [&](int zi) INLINE {
         cnt = __builtin_amdgcn_readfirstlane(r_n); e_lo = __builtin_amdgcn_readfirstlane(r_lo) - cnt;
         if (cnt > 0) {
@@ -778,7 +814,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_f32_kernel(Brick
             rows(e0, row_a);
         }
     };
-    int par = 0, turn = 0;
+    int par = 0, turn = 0, turn2 = nw / 2;           // whose turn it is to store sums, to make weights
     range(zi_lo);
     load_plane(zi_lo - 1);
     begin(zi_lo);
@@ -787,6 +823,10 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_f32_kernel(Brick
         const bool low = z & 1;                      // slot of the base plane
         range(zi + 1);
         const bool bad_plane = any_lane(bad_x);
+        if (SHARE && cnt > 0) {
+            if (turn2 == wave) weights(e0, a0, 0, wofs, low);
+            lds_only_barrier();
+        }
         auto step = [&](int i0, u32x4_t (&row)[4]) INLINE {
             entry(i0 + 64, e2, a2);
             __builtin_amdgcn_sched_barrier(0);
@@ -808,24 +848,10 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_f32_kernel(Brick
             const bool bad = bad_plane || any_lane(no_number_bf16(top, 8));
             rows(e1, row);
             __builtin_amdgcn_sched_barrier(0);
-            const bool ok = i0 + n < cnt;
             const unsigned yb = e0.x & 3u, xs = (e0.x & 12u) << 2;
             const float hy = __uint_as_float(e0.y), hx = __uint_as_float(e0.z), hz = __uint_as_float(e0.w), lz = 1.f - hz;
-            {
-                const float wz = (ok ? a0 : 0.f) * ((h != 0) == low ? lz : hz);
-                const float wy0 = wz * (1.f - hy), wy1 = wz * hy, lx = 1.f - hx;
-                const WeightRow r0 = weight_row(wy0 * lx, wy0 * hx, xs), r1 = weight_row(wy1 * lx, wy1 * hx, xs);
-                typedef __attribute__((address_space(3))) unsigned long long *lds64;
-                const unsigned sy = yb << 3;
-                const unsigned at0 = w_st ^ sy, at1 = w_st ^ (sy + 8), at2 = w_st ^ ((sy + 16) & 24), at3 = w_st ^ ((sy + 24) & 24);
-#pragma unroll
-                for (int i = 0; i < 3; i++) {
-                    *(lds64)(size_t)(at0 + i * 2048) = r0.t[i];
-                    *(lds64)(size_t)(at1 + i * 2048) = r1.t[i];
-                    *(lds64)(size_t)(at2 + i * 2048) = 0;
-                    *(lds64)(size_t)(at3 + i * 2048) = 0;
-                }
-            }
+            if constexpr (!SHARE) weights(e0, a0, i0, 0, low);
+            else if (turn2 == wave && i0 + 32 < cnt) weights(e1, a1, i0 + 32, wofs ^ kWeightLds, low);
             wave_fence();
             // ---- the two products, the smallest terms first
             f32x16 T;
@@ -916,7 +942,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_f32_kernel(Brick
                 const auto u = __builtin_amdgcn_permlane32_swap(__float_as_uint(r_m), __float_as_uint(r_z), false, false);
                 const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(r_x), __float_as_uint(r_y), false, false);
                 float2 r = make_float2(__uint_as_float(u[0]) + __uint_as_float(u[1]), __uint_as_float(v[0]) + __uint_as_float(v[1]));
-                if (nw > 1) {
+                if (SHARE || nw > 1) {
                     s_part[(par * nw + wave) * 64 + lane] = r;
                     lds_only_barrier();
                     if (turn == wave) {
@@ -933,6 +959,8 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 3) brick_grad_f32_kernel(Brick
                 __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(r.x), __float_as_uint(r.y)}, rs, n * 16 + h * 8, 0, 0);
                 par ^= 1;
                 if (++turn == nw) turn = 0;
+                if (++turn2 == nw) turn2 = 0;
+                if (SHARE) { w_tr += wofs ? -kWeightLds : kWeightLds; wofs ^= kWeightLds; }
             }
             e0 = e1; a0 = a1;
             e1 = e2; a1 = a2;
@@ -1371,8 +1399,10 @@ int d2c_brick_grad(const TiledShape &s, const void *xcl, const void *gcol, const
     const unsigned grid = (unsigned)(cols * a.nzr);
     {
         D2cProfScope prof(D2C_PROF_BWD_AUX, st, s.bkc == 64 ? "brick_grad_kernel" : "brick_grad_f32_kernel");
-        const int lds = nw * (s.bkc == 64 ? kWaveLds : kWaveLdsF) + (nw > 1 ? nw * 1024 : 0);
-        auto kern = s.bkc == 64 ? &brick_grad_kernel : &brick_grad_f32_kernel;
+        const bool share = nw > 1 && brick_mean(s) >= 128.0;      // (four steps to a plane)
+        const int lds = nw * (s.bkc == 64 ? kRowLds : kRowLdsF) + (share ? 2 : nw) * kWeightLds + (nw > 1 ? nw * 1024 : 0);
+        auto kern = s.bkc == 64 ? (share ? &brick_grad_kernel<true> : &brick_grad_kernel<false>)
+                                : (share ? &brick_grad_f32_kernel<true> : &brick_grad_f32_kernel<false>);
         hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * nw), lds, st, a, a.L.end, a.L.count);
         if (int rc = d2c_check_launch("brick_grad_kernel")) return rc;
     }
