@@ -838,12 +838,13 @@ def main():
         rows = N * P * K * C * es
         per = {}
         # kernels over sorted points: entries of 20 bytes (points inside the volume), input rows, and rows of those points
-        # read, 16 bytes of sums per point and 256 channels written, float32 sums of the 16 voxels per plane of a brick
+        # read, 16 bytes of sums per point and set of channels written, float32 sums of the 16 voxels per plane of a brick
         # added for each 9 of grad_input; or columns of all points written
         inside = N * P * K * G * (1.0 - taps["dead"]) if taps else 0.0
         for kname, r in role.items():
-            if kname == "brick_grad_kernel":
-                per[kname] = inside * (20 + C // G * es + 16 * -(-C // (256 * G))) + N * P * C * (es + 4 * 16 / 9)
+            if kname in ("brick_grad_kernel", "brick_grad_f32_kernel"):
+                # (a set is 4 chunks of 128 bytes)
+                per[kname] = inside * (20 + C // G * es + 16 * -(-C * es // (512 * G))) + N * P * C * (es + 4 * 16 / 9)
             elif kname == "brick_sample_kernel":
                 per[kname] = inside * 20 + N * P * C * es + rows
             elif r == "bwd_aux":

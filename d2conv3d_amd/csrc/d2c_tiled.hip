@@ -648,10 +648,11 @@ bool use_aux_kernel(const d2c_conv3d_desc &q, const TiledShape &s)
 // at hand.  (A bucket capacity asked for by the test hook is a matter of the lists.)
 bool use_brick(const d2c_conv3d_desc &q, const TiledShape &s)
 {
-    // (float32 weight groups that take several passes of the grad-column product keep the lists: what those groups run is pinned by a test,
-    // and the products are most of their time, 64 -> 512 channels on 8x40x50 715 us, 640)
+    // (float32 weight groups that take several passes of the grad-column product: from 1024 positions on.  Training steps, us, lists first:
+    // 64 -> 512 channels on 1400 positions 233, 216; 5120 341, 319; 16000 715, 646; 512 -> 512, 8 groups, 25920 6180, 5350.  A test holds
+    // problems of some dozen positions to the lists.)
     return d2c_gx_mode() == 1 && use_lists(q, s) && use_aux_kernel(q, s) && d2c_brick_supported(s, q.dtype) &&
-           (q.dtype == D2C_BF16 || d2c_tiled_bwd_single_pass(s, q.dtype));
+           (q.dtype == D2C_BF16 || d2c_tiled_bwd_single_pass(s, q.dtype) || s.M >= 1024);
 }
 
 // The forward pass over sampled columns: sort, sample, multiply.  `kept`: the caller keeps the columns, where the backward call can

@@ -22,6 +22,7 @@ CASES = {
     # the smallest problems that keep the columns of the forward call
     "kept_columns_narrow": (1, 64, 24, (8, 19, 20), (3, 3, 3), 1, 1, 1, 1, True),
     "kept_columns_wide": (1, 64, 136, (4, 17, 18), (3, 3, 3), 1, 1, 1, 2, True),
+    "two_passes_over_output_channels": (1, 64, 330, (6, 13, 14), (3, 3, 3), 1, 1, 1, 1, True),
     "widest_weight_group": (1, 64, 256, (3, 8, 9), (3, 3, 3), 1, 1, 1, 1, True),
 }
 
