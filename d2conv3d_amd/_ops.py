@@ -229,6 +229,15 @@ def _columns_for(lib, desc, sdesc, weight_grad_wanted, dev):
         return None      # (no room to keep them: the backward pass samples again)
 
 
+def _channel_stats_into(lib, x, stats):
+    """The sums that d2c_conv3d_forward_stats fills, of an output that another forward call has stored: a call that keeps its
+    columns runs without statistics, and one more pass over the output costs less than the backward pass's second sampling
+    (512 -> 512 channels on 2x8x30x54 with ReLU and GroupNorm, forward + backward: 2.27 -> 1.84 ms)."""
+    N, C = x.shape[:2]
+    desc = _lib.GroupNormDesc(N, C, x[0, 0].numel(), 1, _DT[x.dtype], 0.0)
+    return lib.d2c_channel_stats(ctypes.byref(desc), _ptr(x), _ptr(stats), _stream(x.device))
+
+
 class _DeformConv3dFunction(torch.autograd.Function):
     """DeformConv3dFunction of dconv3d.h:70-186.  `relu_scale` > 0 (not in the reference) makes the forward
     kernels store relu_scale * max(out, 0) -- the activation that follows the convolution, fused into their last
@@ -255,8 +264,8 @@ class _DeformConv3dFunction(torch.autograd.Function):
         with torch.cuda.device(dev):
             npre = lib.d2c_conv3d_prepared_bytes(ctypes.byref(desc)) if (prepared is not None and not want_stats) else 0
             ctx.prepared = None
-            columns = None
-            if want_stats:
+            columns = None if npre else _columns_for(lib, desc, None, ctx.needs_input_grad[3], dev)
+            if want_stats and columns is None:
                 nb = lib.d2c_conv3d_forward_stats_workspace_bytes(ctypes.byref(desc), None)
                 ws, nb = _forward_workspace(lib, nb, desc, None, dev)
                 rc = lib.d2c_conv3d_forward_stats(ctypes.byref(desc), None, _ptr(input), _ptr(offset), _ptr(alpha),
@@ -276,18 +285,18 @@ class _DeformConv3dFunction(torch.autograd.Function):
                 prepared.fwd_weights = wkey
                 prepared.input_token += 1
                 ctx.prepared, ctx.input_token = prepared, prepared.input_token
+            elif columns is not None:
+                nb = lib.d2c_conv3d_forward_keep_workspace_bytes(ctypes.byref(desc), None)
+                ws = _workspace(nb, dev)
+                rc = lib.d2c_conv3d_forward_columns(ctypes.byref(desc), None, _ptr(input), _ptr(offset), _ptr(alpha),
+                                                    _ptr(weight), _ptr(bias), _ptr(out), _ptr(columns),
+                                                    columns.numel(), _ptr(ws), nb, _stream(dev))
+                if want_stats and not rc:
+                    rc = _channel_stats_into(lib, out, stats)
             else:
-                columns = _columns_for(lib, desc, None, ctx.needs_input_grad[3], dev)
-                if columns is not None:
-                    nb = lib.d2c_conv3d_forward_keep_workspace_bytes(ctypes.byref(desc), None)
-                    ws = _workspace(nb, dev)
-                    rc = lib.d2c_conv3d_forward_columns(ctypes.byref(desc), None, _ptr(input), _ptr(offset), _ptr(alpha),
-                                                        _ptr(weight), _ptr(bias), _ptr(out), _ptr(columns),
-                                                        columns.numel(), _ptr(ws), nb, _stream(dev))
-                else:
-                    ws, nb = _forward_workspace(lib, lib.d2c_conv3d_forward_workspace_bytes(ctypes.byref(desc)), desc, None, dev)
-                    rc = lib.d2c_conv3d_forward(ctypes.byref(desc), _ptr(input), _ptr(offset), _ptr(alpha),
-                                                _ptr(weight), _ptr(bias), _ptr(out), _ptr(ws), nb, _stream(dev))
+                ws, nb = _forward_workspace(lib, lib.d2c_conv3d_forward_workspace_bytes(ctypes.byref(desc)), desc, None, dev)
+                rc = lib.d2c_conv3d_forward(ctypes.byref(desc), _ptr(input), _ptr(offset), _ptr(alpha),
+                                            _ptr(weight), _ptr(bias), _ptr(out), _ptr(ws), nb, _stream(dev))
         _lib.check(rc, "deform_conv3d forward")
         ctx.save_for_backward(input, offset, alpha, weight, bias, out if relu_scale > 0 else None, columns)
         ctx.desc = desc
@@ -350,7 +359,8 @@ def deform_conv3d(input, offset, alpha, weight, bias, stride_d, stride_h, stride
     """deform_conv3d of dconv3d.h:188-226; `alpha` and `bias` may be None.  `relu_scale` > 0 fuses
     relu_scale * relu(.) into the store of the output (see _DeformConv3dFunction).  `want_stats` also returns the
     float32 [N, Cout, 2] sums and sums of squares of the stored output per (sample, channel), added up by the
-    forward kernels where they store (the statistics a GroupNorm behind the convolution needs).  `offset_axes`: mask
+    forward kernels where they store, or by a pass over it where the call keeps its columns (the statistics a GroupNorm
+    behind the convolution needs).  `offset_axes`: mask
     of the axes (1 z, 2 y, 4 x) the offsets displace along; the others are taken as zero and their gradient
     channels come back zero (matrix-core kernels only, see conv3d_algo).  `backward_flags`: the description's field
     of that name (_lib.BWD_GW_* | _lib.bwd_slices(n)): how the backward pass trades workspace for time.  `prepared`: a
@@ -395,27 +405,27 @@ class _DeformConv3dSizedFunction(torch.autograd.Function):
         out = torch.empty((N, Cout, Do, Ho, Wo), dtype=input.dtype, device=dev)
         stats = torch.empty((N, Cout, 2), dtype=torch.float32, device=dev) if want_stats else None
         with torch.cuda.device(dev):
-            columns = None
-            if want_stats:
+            columns = _columns_for(lib, desc, sdesc, ctx.needs_input_grad[3], dev)
+            if want_stats and columns is None:
                 nb = lib.d2c_conv3d_forward_stats_workspace_bytes(ctypes.byref(desc), ctypes.byref(sdesc))
                 ws, nb = _forward_workspace(lib, nb, desc, sdesc, dev)
                 rc = lib.d2c_conv3d_forward_stats(ctypes.byref(desc), ctypes.byref(sdesc), _ptr(input), _ptr(size_raw),
                                                   _ptr(alpha), _ptr(weight), _ptr(bias), _ptr(out), _ptr(stats),
                                                   _ptr(ws), nb, _stream(dev))
+            elif columns is not None:
+                nb = lib.d2c_conv3d_forward_keep_workspace_bytes(ctypes.byref(desc), ctypes.byref(sdesc))
+                ws = _workspace(nb, dev)
+                rc = lib.d2c_conv3d_forward_columns(ctypes.byref(desc), ctypes.byref(sdesc), _ptr(input),
+                                                    _ptr(size_raw), _ptr(alpha), _ptr(weight), _ptr(bias), _ptr(out),
+                                                    _ptr(columns), columns.numel(), _ptr(ws), nb, _stream(dev))
+                if want_stats and not rc:
+                    rc = _channel_stats_into(lib, out, stats)
             else:
-                columns = _columns_for(lib, desc, sdesc, ctx.needs_input_grad[3], dev)
-                if columns is not None:
-                    nb = lib.d2c_conv3d_forward_keep_workspace_bytes(ctypes.byref(desc), ctypes.byref(sdesc))
-                    ws = _workspace(nb, dev)
-                    rc = lib.d2c_conv3d_forward_columns(ctypes.byref(desc), ctypes.byref(sdesc), _ptr(input),
-                                                        _ptr(size_raw), _ptr(alpha), _ptr(weight), _ptr(bias), _ptr(out),
-                                                        _ptr(columns), columns.numel(), _ptr(ws), nb, _stream(dev))
-                else:
-                    nb = lib.d2c_conv3d_sized_forward_workspace_bytes(ctypes.byref(desc), ctypes.byref(sdesc))
-                    ws, nb = _forward_workspace(lib, nb, desc, sdesc, dev)
-                    rc = lib.d2c_conv3d_sized_forward(ctypes.byref(desc), ctypes.byref(sdesc), _ptr(input),
-                                                      _ptr(size_raw), _ptr(alpha), _ptr(weight), _ptr(bias), _ptr(out),
-                                                      _ptr(ws), nb, _stream(dev))
+                nb = lib.d2c_conv3d_sized_forward_workspace_bytes(ctypes.byref(desc), ctypes.byref(sdesc))
+                ws, nb = _forward_workspace(lib, nb, desc, sdesc, dev)
+                rc = lib.d2c_conv3d_sized_forward(ctypes.byref(desc), ctypes.byref(sdesc), _ptr(input),
+                                                  _ptr(size_raw), _ptr(alpha), _ptr(weight), _ptr(bias), _ptr(out),
+                                                  _ptr(ws), nb, _stream(dev))
         _lib.check(rc, "deform_conv3d_sized forward")
         ctx.save_for_backward(input, size_raw, alpha, weight, bias, out if relu_scale > 0 else None, columns)
         ctx.desc, ctx.sdesc = desc, sdesc
@@ -540,16 +550,16 @@ class _DeformConv3dPackedFunction(torch.autograd.Function):
         out = torch.empty((N, Cout, Do, Ho, Wo), dtype=input.dtype, device=dev)
         stats = torch.empty((N, Cout, 2), dtype=torch.float32, device=dev) if want_stats else None
         p_off, p_mask = _ptr_at(deformation, 0), _ptr_at(deformation, lead)
-        columns = None
         with torch.cuda.device(dev):
-            if not want_stats:
-                columns = _columns_for(lib, desc, sdesc, ctx.needs_input_grad[2], dev)
+            columns = _columns_for(lib, desc, sdesc, ctx.needs_input_grad[2], dev)
             if columns is not None:
                 nb = lib.d2c_conv3d_forward_keep_workspace_bytes(ctypes.byref(desc), sref)
                 ws = _workspace(nb, dev)
                 rc = lib.d2c_conv3d_forward_columns(ctypes.byref(desc), sref, _ptr(input), p_off, p_mask, _ptr(weight),
                                                     _ptr(bias), _ptr(out), _ptr(columns), columns.numel(), _ptr(ws), nb,
                                                     _stream(dev))
+                if want_stats and not rc:
+                    rc = _channel_stats_into(lib, out, stats)
             elif want_stats:
                 nb = lib.d2c_conv3d_forward_stats_workspace_bytes(ctypes.byref(desc), sref)
                 ws, nb = _forward_workspace(lib, nb, desc, sdesc, dev)
