@@ -513,7 +513,7 @@ bool d2c_depthwise_supported(const TiledShape &s)
     return s.cg == 1 && s.og == 1 && s.cpg % kCV == 0;
 }
 
-// `wt`: the weights as [K][C] (see dw_prepare_kernel)
+// `wt`: the weights as [K][C] (see prepare_kernel)
 template <typename T>
 int d2c_depthwise_forward(const TiledShape &s, const void *xcl, const void *off, const void *mask, const void *wt,
                           const void *bias, void *out, hipStream_t st)

@@ -10,11 +10,9 @@
 // weights, and drops the result into an LDS tile in MFMA operand order.  The
 // im2col column buffer of the reference (dconv3d_gpu.cu:297) never exists.
 //
-// One workgroup = 512 threads = MT positions x NT output channels.  Steps are
-// software-pipelined over three stages: while the matrix cores work on step s,
-// the corner rows of step s+1 and the weight fragments of step s+1 are in
-// flight and the offsets of step s+2 are being fetched; nothing waits on
-// memory inside a step except at its one barrier.
+// Here: the DMA-gather kernel, whose corner rows go to LDS without passing through registers, for weight groups wide enough or
+// problems large enough to fill its output tile; and the choice between it and the kernel of the other problems
+// (d2c_tiled_wave.hip).
 #include "d2c_mma.hpp"
 #include "d2c_tiled.hpp"
 

@@ -74,8 +74,9 @@ enum {
 /* d2c_conv3d_desc::backward_flags: how the matrix-core backward pass trades workspace for time.
  * Both d2c_conv3d_backward_workspace_bytes() and d2c_conv3d_backward() read the field from the description they
  * are given, so the size asked for and the call agree per description.  0 = the defaults. */
-#define D2C_BWD_GW_DEFAULT   0   /* grad_weight as a matrix product over sampled columns in a buffer of their own */
-#define D2C_BWD_GW_COLUMNS   1   /* the same, said explicitly */
+#define D2C_BWD_GW_DEFAULT   0   /* grad_weight as a matrix product over sampled columns in a buffer of their own; float32 problems
+                                  * whose gradients run over sorted sampling points sample again instead (faster, half the memory) */
+#define D2C_BWD_GW_COLUMNS   1   /* such columns whatever the type */
 #define D2C_BWD_GW_IN_PLACE  2   /* the columns written over the grad-column rows: no buffer of their own
                                   * (bfloat16; float32 problems then sample again) */
 #define D2C_BWD_GW_RESAMPLE  3   /* no columns at all: the grad-weight kernel samples the input again */
@@ -197,14 +198,15 @@ int d2c_conv3d_backward(const d2c_conv3d_desc *desc, const void *grad_out, const
  * memory to spare hands d2c_conv3d_forward_columns a buffer of d2c_conv3d_columns_bytes() bytes (256-byte aligned;
  * taps x the size of the input, in the element type): the forward kernel writes there what it multiplies with the
  * weights anyway, and d2c_conv3d_backward_columns, given that buffer UNCHANGED together with the same tensors, runs
- * its grad-weight product over it instead of sampling again (N=2, C=512, 8x30x54, bfloat16: 2.33 -> 1.95 ms per step
+ * its grad-weight product over it instead of sampling again (N=2, C=512, 8x30x54, bfloat16: 2.14 -> 1.78 ms per step
  * for 878 MB held between the two calls -- 717 of columns, sorted sampling points, the input channels-last, see d2c_conv3d_keep_bytes() -- and
- * 0.88 GB less backward workspace; N=2, C=256, 8x30x54, float32: 2.29 -> 2.13 ms for 717 MB).  Results are those of the plain calls up to the order of floating-point sums; float32
+ * 0.88 GB less backward workspace; N=2, C=256, 8x30x54, float32: 1.68 ms for 717 MB).  Results are those of the plain calls up to the order of floating-point sums; float32
  * columns are the interpolated floats themselves and their product keeps float32's accuracy (three bfloat16 terms
  * per float on the bfloat16 matrix instruction, or the float32 instruction), whatever D2C_BWD_F32_SPLIT says.  `size_map` as in d2c_conv3d_forward_stats: NULL, or the description of
  * the size map that `offset` then is.  d2c_conv3d_columns_bytes() is 0 where this is not served (anything but
  * bfloat16 and float32 problems on the matrix-core kernels with an even number of 64- / 32-channel chunks per weight
- * group and at least 48 tiles of 64 output positions (times weight groups) and offsets along all three axes, or, bfloat16 with
+ * group, offsets along all three axes, and enough output positions: tiles of 64 times weight groups at least 48 -- bfloat16 with up to 128
+ * output channels per weight group 160, float32 with more 20 --, or, bfloat16 with
  * one weight group, at least 400 positions and 2048 positions times chunks); the two calls then
  * fail with D2C_ERR_UNSUPPORTED and the caller uses the plain ones.  The memory-saving bits of
  * d2c_conv3d_desc::backward_flags are ignored by d2c_conv3d_backward_columns.
