@@ -245,8 +245,10 @@ brick_file_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, cons
         at += __popcll(m[i]);
     }
 }
-// Workgroups of a pass over all points that needs no window: 256 positions, kPassTaps taps
-constexpr int kPassTaps = 9;
+// Workgroups of a pass over all points that needs no window: 256 positions, kPassTaps taps.  (A wavefront waits for the places,
+// then for the sums they name: few taps in each of many.  Results of 27 and 7 taps, C3 and 2048 channels on 8x30x54, us: 9 taps
+// 61, 36; 3 52, 16; 2 54, 12; 1 56, 10.)
+constexpr int kPassTaps = 2;
 struct PointUnit {
     int b, g, bg, k0, p;
 };
@@ -1227,21 +1229,23 @@ brick_finish_kernel(TiledShape s, BrickLists L, const float2 *res, long nres, in
     }
 }
 // Size-map source: d(offset_a) / d(size_a) = base_a[k_a], so the taps of a position add up; the axes that a channel of
-// the raw map feeds add up, times the derivative of the size activation.  A workgroup is 64 positions x 4 shares of the
-// taps.
+// the raw map feeds add up, times the derivative of the size activation.  A workgroup is 64 positions x kTapShares shares of the
+// taps.  (Four shares leave a third of the chip's wavefronts out: 1024 -> 256 channels on 8x30x54, 27 taps, 4, 9 and 14 shares 28, 18
+// and 17 us; 256 channels on 2x8x30x54, float32, 24, 18 and 20.)
+constexpr int kTapShares = 9;
 template <bool AUX16>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(64 * kTapShares)
 brick_finish_size_kernel(TiledShape s, BrickLists L, const float2 *res, long nres, int nset, const void *mask, const void *raw,
                          void *graw, void *gmask)
 {
     typedef typename std::conditional<AUX16, bf16_t, float>::type AT;
-    __shared__ float s_sum[4][3][64];
+    __shared__ float s_sum[kTapShares][3][64];
     const int b = blockIdx.y, lane = threadIdx.x & 63, part = threadIdx.x >> 6;
     const int p = blockIdx.x * 64 + lane;
     float sum[3] = {0.f, 0.f, 0.f};
     if (p < s.P)
 #pragma unroll 4
-        for (int k = part; k < s.K; k += 4) {
+        for (int k = part; k < s.K; k += kTapShares) {
             const int at = L.place[((long)b * s.K + k) * s.P + p];
             float2 mx, zy;
             brick_point_sums(res, nres, nset, at, mx, zy);
@@ -1266,7 +1270,9 @@ brick_finish_size_kernel(TiledShape s, BrickLists L, const float2 *res, long nre
     float v = 0.f;
 #pragma unroll
     for (int ax = 0; ax < 3; ax++)
-        if (axis_channel(s.ss.mode, ax) == c) v += (s_sum[0][ax][lane] + s_sum[1][ax][lane]) + (s_sum[2][ax][lane] + s_sum[3][ax][lane]);
+        if (axis_channel(s.ss.mode, ax) == c)
+#pragma unroll
+            for (int i = 0; i < kTapShares; i++) v += s_sum[i][ax][lane];
     const long ri = (long)b * s.obs + (long)c * s.P + p;
     v *= size_act_grad(s.ss.act, ld_auxT<AUX16>(raw, ri));
     reinterpret_cast<AT *>(graw)[ri] = f32_to_elem<AT>(v);
@@ -1411,7 +1417,7 @@ int d2c_brick_grad(const TiledShape &s, const void *xcl, const void *gcol, const
     const bool a16 = s.adt == D2C_BF16;
     if (s.ss.on) {
         auto fin = a16 ? &brick_finish_size_kernel<true> : &brick_finish_size_kernel<false>;
-        hipLaunchKernelGGL(fin, dim3((s.P + 63) / 64, s.N), dim3(256), 0, st, s, a.L, a.res, a.nres, a.nset, mask, raw, goff, gmask);
+        hipLaunchKernelGGL(fin, dim3((s.P + 63) / 64, s.N), dim3(64 * kTapShares), 0, st, s, a.L, a.res, a.nres, a.nset, mask, raw, goff, gmask);
     } else {
         auto fin = a16 ? &brick_finish_kernel<true> : &brick_finish_kernel<false>;
         const int ngrp = (s.K + kPassTaps - 1) / kPassTaps;
