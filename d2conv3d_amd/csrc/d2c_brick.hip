@@ -18,6 +18,7 @@
 #include "d2c_mma.hpp"
 #include "d2c_tiled.hpp"
 #include "d2c_brick.hpp"
+#include <cmath>
 
 namespace {
 
@@ -1315,6 +1316,23 @@ SortWindow sort_window(const TiledShape &s, const BrickDims &d)
     shrink(w.wx, 1, (long)w.wz * w.wy, kSortSlots);
     return w;
 }
+// Base planes per workgroup of the gradient kernel: a range costs one plane more than it has bases, to be loaded and added, and
+// the last round of workgroups (twelve wavefronts to a compute unit) leaves the chip part empty; half of that is taken for lost.  us, planes
+// per range: 256 channels on 2x8x30x54 1 115, 2 116, 3 104; float32 2 262, 3 232, 5 253; 1024 channels on 8x30x54 1 227, 2 240, 3 230,
+// 5 234; 2048, 7 taps, 2 260, 3 227, 5 224, 9 209; 512, 8 groups, 2x8x30x54 1 229, 2 223, 3 225, 5 232; 256 on 32x60x108 3 824, 5 822, 9 890.
+// Below three quarters of a round the shortest ranges even out best (steps: 256 -> 64 channels, float32, 8x20x32, 0.6 rounds of 3 planes
+// 294, of 1 289; bfloat16 8x40x50 0.9 rounds of 3 planes 332, of 1 340; 8x60x107 one round of 9 931, of 1 956).
+int brick_range_planes(int nz, long cols, int nw)
+{
+    const double slots = 12.0 / nw * std::max(d2c_num_cus(), 1);
+    int best = nz;
+    double least = 1e300;
+    for (int z = nz;; z = (z + 1) / 2) {
+        const double r = cols * ((nz + z - 1) / z) / slots, t = 0.5 * (r + 0.5 + std::ceil(r)) * (z + 1.25);
+        if (z == 1 ? t < least : (r >= 0.75 && t < least)) { least = t; best = z; }
+        if (z == 1) return best;
+    }
+}
 int brick_sets(const TiledShape &s) { return (s.cpg / s.bkc + kMaxWaves - 1) / kMaxWaves; }
 BrickLists brick_lists(const TiledShape &s, char *base)
 {
@@ -1396,11 +1414,8 @@ int d2c_brick_grad(const TiledShape &s, const void *xcl, const void *gcol, const
     a.chunk_rows = (long)s.K * s.M;
     a.nset = brick_sets(s);
     const int nw = (a.cpc + a.nset - 1) / a.nset;
-    // enough workgroups to fill the chip several times over; a range of z costs one more plane than it has bases
-    const int ncu = d2c_num_cus();
     const long cols = (long)a.d.nbx * a.d.nby * s.N * s.G * a.nset;
-    a.zlen = a.d.nz;
-    while (a.zlen > 1 && cols * ((a.d.nz + a.zlen - 1) / a.zlen)  * nw < 64L * ncu) a.zlen = (a.zlen + 1) / 2;
+    a.zlen = brick_range_planes(a.d.nz, cols, nw);
     a.nzr = (a.d.nz + a.zlen - 1) / a.zlen;
     const unsigned grid = (unsigned)(cols * a.nzr);
     {
@@ -1441,7 +1456,9 @@ int d2c_brick_columns(const TiledShape &s, const void *xcl, void *col, int rows,
     const int ncu = d2c_num_cus();
     const long cols = (long)a.d.nbx * a.d.nby * s.N * s.G * a.nset;
     a.zlen = a.d.nz;
-    while (a.zlen > 1 && cols * ((a.d.nz + a.zlen - 1) / a.zlen) * nw < 64L * ncu) a.zlen = (a.zlen + 1) / 2;
+    // (enough workgroups to fill the chip several times over, fewer where a plane has few points: 2048 channels, 7 taps, 100 us, 88)
+    const long want = (brick_mean(s) >= 128.0 ? 64L : 16L) * ncu;
+    while (a.zlen > 1 && cols * ((a.d.nz + a.zlen - 1) / a.zlen) * nw < want) a.zlen = (a.zlen + 1) / 2;
     a.nzr = (a.d.nz + a.zlen - 1) / a.zlen;
     a.npoint = brick_points(s);
     a.nzero = (int)std::min<long>(2048, (a.npoint + 511) / 512) / nw + 1;
