@@ -11,14 +11,14 @@
 // Three quarters of the products are with zeros, on matrix cores that have them to spare; in exchange nothing is
 // gathered: a grad-column row is read once, for both results, and a brick's input rows stay in LDS.  (The kernels
 // that gather -- eight corner rows per point through the L1, grad-column rows 3.4 times -- took 1.73 + 1.47 ms for
-// 256 channels on 32x60x108, bound by the L1 path, the vector ALU and row latency; this one takes 0.87, at 2.4 TB/s to and
+// 256 channels on 32x60x108, bound by the L1 path, the vector ALU and row latency; this one takes 0.82, at 2.6 TB/s to and
 // from device memory, and 0.22 for 512 channels in 8 groups on 2x8x30x54, where they took 0.50 + 0.35.)
 
 #include <algorithm>
+#include <cmath>
 #include "d2c_mma.hpp"
 #include "d2c_tiled.hpp"
 #include "d2c_brick.hpp"
-#include <cmath>
 
 namespace {
 

@@ -11,7 +11,7 @@ struct BrickLists {
     int *cursor;             // entries given out, then: points outside the volume
     int *end;                // end of a block's entries (they begin `count` before it)
     int *place;              // [n * G + g][tap][p]: a point's entry, -1: no corner inside the volume
-    uint4 *pt;               // byte offset of the point's row of 64 channels | its base voxel in the block (y | x << 2); fractions along y, x, z
+    uint4 *pt;               // byte offset of the point's row of 128 bytes (64 channels, float32 32) | its base voxel in the block (y | x << 2); fractions along y, x, z
     float *alpha;            // modulation
 };
 struct BrickWs {
