@@ -20,7 +20,7 @@
 size_t d2c_wave_count_bytes(const TiledShape &s, int nt);
 size_t d2c_wave_split_bytes(const TiledShape &s, int nt);
 template <typename T>
-int d2c_wave_launch(const TiledShape &s, int nt, const void *xcl, const void *off, const void *mask, const void *wp,
+int d2c_wave_launch(const TiledShape &s, int nt, bool skip_zero, const void *xcl, const void *off, const void *mask, const void *wp,
                     const void *bias, void *out, float *split, float *stats, void *col, hipStream_t st);
 
 namespace {
@@ -845,6 +845,15 @@ bool d2c_fwd_use_dma(const TiledShape &s)
     return tiles >= kDmaTilesWide || (tiles >= kDmaTilesLeast && tiles * s.nchunk * s.K >= kDmaStepsWide);
 }
 
+// Whether an infinity in a corner of weight zero stays out of the result: in the DMA-gather kernel and over sorted points always.
+// The other kernel keeps to that for problems of the size that those serve otherwise; in smaller ones such a
+// corner is multiplied like any other (0 * inf is NaN), as the direct kernels do.
+static bool d2c_fwd_skips_zero_weights(const TiledShape &s)
+{
+    const long tiles = dma_tiles(s);
+    return s.og <= 128 ? tiles >= kDmaTilesNarrow : tiles >= kDmaTilesWide || tiles * s.nchunk * s.K >= kDmaStepsWide;
+}
+
 // Output channels per workgroup.  The sampled tile of the DMA-gather kernel is produced once for all of them.
 int d2c_fwd_out_tile(const TiledShape &s)
 {
@@ -891,7 +900,7 @@ int d2c_tiled_fwd_launch(const TiledShape &s, const void *xcl, const void *off, 
 {
     const int nt = d2c_fwd_out_tile(s);
     if (col && !d2c_fwd_writes_columns(s, (int)Elem<T>::DT)) col = nullptr;
-    if (!d2c_fwd_use_dma(s)) return d2c_wave_launch<T>(s, nt, xcl, off, mask, wp, bias, out, outacc, stats, col, st);
+    if (!d2c_fwd_use_dma(s)) return d2c_wave_launch<T>(s, nt, d2c_fwd_skips_zero_weights(s), xcl, off, mask, wp, bias, out, outacc, stats, col, st);
     // the channels-last input is followed by a row of zeros (see forward_t)
     const unsigned zrow = (unsigned)((size_t)s.N * s.vol * s.Cin * sizeof(T));
     FwdArgs a{s, xcl, off, mask, wp, bias, out, nullptr, zrow, 0, 0, 0, 0, 1, stats ? stats_part : nullptr, nullptr, 0};

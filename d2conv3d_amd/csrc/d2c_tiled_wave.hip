@@ -28,6 +28,9 @@ struct WaveArgs {
     // zeros past the last position (col_rows is a whole number of tiles, and the grid has that many)
     void *col;
     long col_rows;
+    // Corners of weight zero (a point on a voxel plane, a modulation of exactly zero): not read, so that an infinity there
+    // reaches nothing, or read and multiplied like any other, which makes NaN of it (see d2c_fwd_skips_zero_weights)
+    int skip_zero;
     float *stats;      // [N][Cout][2] sums and sums of squares of the stored values (zero in front of the launch), or NULL
 };
 
@@ -155,9 +158,12 @@ __global__ void __launch_bounds__(kThreads) tiled_fwd_wave_kernel(WaveArgs a)
                                                  cox * s.geo.sw - s.geo.pw + w.kx * s.geo.dw, craw[0], craw[1], craw[2]);
                 const float al = (s.mact && a.mask) ? mask_act<AT>(s.mact, craw[3]) : craw[3];
                 const unsigned o0 = (unsigned)(cb * s.vol + (t.z0 * s.H + t.y0) * s.W + t.x0) * dx;
+                unsigned read = t.live;
+                if (a.skip_zero)
+                    read &= (t.hz > 0.f ? 0xFFu : 0x0Fu) & (t.hy > 0.f ? 0xFFu : 0x33u) & (t.hx > 0.f ? 0xFFu : 0x55u) & (al != 0.f ? 0xFFu : 0u);
 #pragma unroll
                 for (int c = 0; c < 8; c++) {
-                    const bool live = (t.live >> c) & 1u;
+                    const bool live = (read >> c) & 1u;
                     cw[c] = live ? tap3_weight(t, c) * al : 0.f;
                     if (live) co[c] = o0 + (c >> 2) * dz + ((c >> 1) & 1) * dy + (c & 1) * dx;
                 }
@@ -409,11 +415,11 @@ size_t d2c_wave_split_bytes(const TiledShape &s, int nt)
 
 // `split`: d2c_wave_split_bytes() of scratch, or NULL: the steps of a tile stay with one workgroup
 template <typename T>
-int d2c_wave_launch(const TiledShape &s, int nt, const void *xcl, const void *off, const void *mask, const void *wp,
+int d2c_wave_launch(const TiledShape &s, int nt, bool skip_zero, const void *xcl, const void *off, const void *mask, const void *wp,
                     const void *bias, void *out, float *split, float *stats, void *col, hipStream_t st)
 {
     WaveArgs a{s, xcl, off, mask, wp, bias, out, nullptr, nullptr, 1, (unsigned)((size_t)s.N * s.vol * s.Cin * sizeof(T)),
-               col, d2c_columns_rows(s), stats};
+               col, d2c_columns_rows(s), skip_zero, stats};
     if (split && d2c_wave_split_bytes(s, nt)) {
         a.nsplit = wave_split(s, nt);
         a.arrived = reinterpret_cast<unsigned *>(split);
@@ -428,7 +434,7 @@ int d2c_wave_launch(const TiledShape &s, int nt, const void *xcl, const void *of
     }
     return nt == 128 ? launch_wave<T, false, 4, 2>(a, st) : launch_wave<T, false, 2, 4>(a, st);
 }
-template int d2c_wave_launch<bf16_t>(const TiledShape &, int, const void *, const void *, const void *, const void *, const void *,
+template int d2c_wave_launch<bf16_t>(const TiledShape &, int, bool, const void *, const void *, const void *, const void *, const void *,
                                      void *, float *, float *, void *, hipStream_t);
-template int d2c_wave_launch<float>(const TiledShape &, int, const void *, const void *, const void *, const void *, const void *,
+template int d2c_wave_launch<float>(const TiledShape &, int, bool, const void *, const void *, const void *, const void *, const void *,
                                     void *, float *, float *, void *, hipStream_t);
