@@ -133,9 +133,12 @@ __global__ void __launch_bounds__(kThreads) conv1d_data_kernel(Conv1dArgs a)
             vq[i] = x0q == t.x0 && l0 ? v0[i] : (r0 ? ld_elem<T>(a.x, xi + x0q) : 0.f);
         }
         if (a.col && there) {
+            // (a corner of weight zero, of a point on a voxel or a modulation of exactly zero, is left out: an infinity there
+            // reaches nothing, as in the kernels of the larger problems)
+            const bool has0 = l0 && al != 0.f, has1 = l1 && t.hx > 0.f && al != 0.f;
 #pragma unroll
             for (int i = 0; i < 2; i++) {
-                const float v = (l0 ? t.lx * al * v0[i] : 0.f) + (l1 ? t.hx * al * v1[i] : 0.f);
+                const float v = (has0 ? t.lx * al * v0[i] : 0.f) + (has1 ? t.hx * al * v1[i] : 0.f);
                 reinterpret_cast<T *>(a.col)[((long)(c0 + cl + i * 16) * s.K + k) * ((long)s.N * a.Pp) + mp] = f32_to_elem<T>(ok ? v : 0.f);
             }
         }
