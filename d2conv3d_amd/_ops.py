@@ -359,8 +359,7 @@ def deform_conv3d(input, offset, alpha, weight, bias, stride_d, stride_h, stride
     """deform_conv3d of dconv3d.h:188-226; `alpha` and `bias` may be None.  `relu_scale` > 0 fuses
     relu_scale * relu(.) into the store of the output (see _DeformConv3dFunction).  `want_stats` also returns the
     float32 [N, Cout, 2] sums and sums of squares of the stored output per (sample, channel), added up by the
-    forward kernels where they store, or by a pass over it where the call keeps its columns (the statistics a GroupNorm
-    behind the convolution needs).  `offset_axes`: mask
+    forward kernel where it stores, or by a pass over it (the statistics a GroupNorm behind the convolution needs).  `offset_axes`: mask
     of the axes (1 z, 2 y, 4 x) the offsets displace along; the others are taken as zero and their gradient
     channels come back zero (matrix-core kernels only, see conv3d_algo).  `backward_flags`: the description's field
     of that name (_lib.BWD_GW_* | _lib.bwd_slices(n)): how the backward pass trades workspace for time.  `prepared`: a

@@ -666,7 +666,7 @@ int d2c_conv3d_forward_stats(const d2c_conv3d_desc *q, const d2c_size_map_desc *
     if (a < 0) return D2C_ERR_UNSUPPORTED;
     // the kernels that add the sums up on their way: matrix-core family, offsets from a tensor or formed in the sampler
     if (stats_fused(*q, z)) {
-        if (int rc = check_ws(d2c_tiled_forward_ws(*q, D2C_FWD_WS_STATS_LEAST), ws, ws_bytes)) return rc;
+        if (int rc = check_ws(d2c_tiled_forward_ws(*q, D2C_FWD_WS_STATS), ws, ws_bytes)) return rc;
         return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, ws_bytes, (hipStream_t)stream, z, chan_stats);
     }
     if (int rc = z ? d2c_conv3d_sized_forward(q, z, x, offset, mask, weight, bias, out, ws, ws_bytes, stream)

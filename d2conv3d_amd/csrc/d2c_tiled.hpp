@@ -11,10 +11,9 @@ bool d2c_tiled_packed_supported(const d2c_conv3d_desc &q);
 // whether a description with some offset axes fixed (offset_axes != 7) stays on the tiled kernels in both directions
 bool d2c_tiled_axes_supported(const d2c_conv3d_desc &q);
 // Workspace of a forward call: what it is fastest with; what the gathering kernels are fastest with (with room for the
-// partial sums of a small problem); the least it runs with; the two for a call with output statistics; what a call that
-// keeps its columns is fastest with, given a buffer of d2c_tiled_keep_bytes(); the least that one runs with
-enum D2cForwardWs { D2C_FWD_WS_FAST, D2C_FWD_WS_GATHER, D2C_FWD_WS_LEAST, D2C_FWD_WS_STATS, D2C_FWD_WS_STATS_LEAST, D2C_FWD_WS_KEEP,
-                    D2C_FWD_WS_KEEP_LEAST };
+// partial sums of a small problem); the least it runs with; what one that adds up output statistics on its way needs; what a
+// call that keeps its columns is fastest with, given a buffer of d2c_tiled_keep_bytes(); the least that one runs with
+enum D2cForwardWs { D2C_FWD_WS_FAST, D2C_FWD_WS_GATHER, D2C_FWD_WS_LEAST, D2C_FWD_WS_STATS, D2C_FWD_WS_KEEP, D2C_FWD_WS_KEEP_LEAST };
 size_t d2c_tiled_forward_ws(const d2c_conv3d_desc &q, D2cForwardWs which = D2C_FWD_WS_FAST);
 // `sz` != nullptr: the offsets are formed from a raw size map (`off` is that map [N, channels(mode), P], `goff` the
 // gradient with respect to it); only where d2c_tiled_sized_supported() says so.

@@ -31,7 +31,6 @@ struct WaveArgs {
     // Corners of weight zero (a point on a voxel plane, a modulation of exactly zero): not read, so that an infinity there
     // reaches nothing, or read and multiplied like any other, which makes NaN of it (see d2c_fwd_skips_zero_weights)
     int skip_zero;
-    float *stats;      // [N][Cout][2] sums and sums of squares of the stored values (zero in front of the launch), or NULL
 };
 
 // Tiles that are neighbours in space go to the same XCD (workgroups are dealt
@@ -343,31 +342,10 @@ __global__ void __launch_bounds__(kThreads) tiled_fwd_wave_kernel(WaveArgs a)
         const int ol = otile * NT + (i * kThreads + tid) / kWP;
         if (ol >= s.og) continue;                           // (uniform over the half)
         const int o = wg * s.og + ol;
-        float fv = 0.f;
         if (ok) {
             float t = v[i];
             if (bias) t += elem_to_f32<T>(bias[o]);
-            const T sv = f32_to_elem<T>(d2c_epilogue(t, s.act, s.act_scale));
-            out[((long)b * s.Cout + o) * s.P + p] = sv;
-            fv = elem_to_f32<T>(sv);
-        }
-        if (a.stats) {
-            // sum and sum of squares of the stored values per (sample, channel), into the [N][Cout][2] result that the
-            // launcher cleared: one lane adds for the half when its positions lie in one sample, as they nearly always do
-            const int b0 = __shfl(b, lane & 32, 64);
-            const unsigned long long odd = __ballot(ok && b != b0);
-            if (((odd >> (lane & 32)) & 0xffffffffull) == 0ull) {
-                float q0 = fv, q1 = fv * fv;
-#pragma unroll
-                for (int d = 1; d < 32; d <<= 1) { q0 += __shfl_xor(q0, d, 64); q1 += __shfl_xor(q1, d, 64); }
-                if ((lane & 31) == 0 && b0 >= 0) {
-                    atomicAdd(a.stats + ((long)b0 * s.Cout + o) * 2, q0);
-                    atomicAdd(a.stats + ((long)b0 * s.Cout + o) * 2 + 1, q1);
-                }
-            } else if (ok) {
-                atomicAdd(a.stats + ((long)b * s.Cout + o) * 2, fv);
-                atomicAdd(a.stats + ((long)b * s.Cout + o) * 2 + 1, fv * fv);
-            }
+            out[((long)b * s.Cout + o) * s.P + p] = f32_to_elem<T>(d2c_epilogue(t, s.act, s.act_scale));
         }
     }
 }
@@ -416,18 +394,14 @@ size_t d2c_wave_split_bytes(const TiledShape &s, int nt)
 // `split`: d2c_wave_split_bytes() of scratch, or NULL: the steps of a tile stay with one workgroup
 template <typename T>
 int d2c_wave_launch(const TiledShape &s, int nt, bool skip_zero, const void *xcl, const void *off, const void *mask, const void *wp,
-                    const void *bias, void *out, float *split, float *stats, void *col, hipStream_t st)
+                    const void *bias, void *out, float *split, void *col, hipStream_t st)
 {
     WaveArgs a{s, xcl, off, mask, wp, bias, out, nullptr, nullptr, 1, (unsigned)((size_t)s.N * s.vol * s.Cin * sizeof(T)),
-               col, d2c_columns_rows(s), skip_zero, stats};
+               col, d2c_columns_rows(s), skip_zero};
     if (split && d2c_wave_split_bytes(s, nt)) {
         a.nsplit = wave_split(s, nt);
         a.arrived = reinterpret_cast<unsigned *>(split);
         a.part = reinterpret_cast<float *>(reinterpret_cast<char *>(split) + d2c_align_up(d2c_wave_count_bytes(s, nt)));
-    }
-    if (stats) {
-        D2cProfScope prof(D2C_PROF_PACK, st);
-        d2c_fill_zero(stats, (size_t)s.N * s.Cout * 2 * sizeof(float), st);
     }
     if constexpr (sizeof(T) == 2) {
         if (s.adt == D2C_BF16) return nt == 128 ? launch_wave<T, true, 4, 2>(a, st) : launch_wave<T, true, 2, 4>(a, st);
@@ -435,6 +409,6 @@ int d2c_wave_launch(const TiledShape &s, int nt, bool skip_zero, const void *xcl
     return nt == 128 ? launch_wave<T, false, 4, 2>(a, st) : launch_wave<T, false, 2, 4>(a, st);
 }
 template int d2c_wave_launch<bf16_t>(const TiledShape &, int, bool, const void *, const void *, const void *, const void *, const void *,
-                                     void *, float *, float *, void *, hipStream_t);
+                                     void *, float *, void *, hipStream_t);
 template int d2c_wave_launch<float>(const TiledShape &, int, bool, const void *, const void *, const void *, const void *, const void *,
-                                    void *, float *, float *, void *, hipStream_t);
+                                    void *, float *, void *, hipStream_t);
