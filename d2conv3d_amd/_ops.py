@@ -217,6 +217,12 @@ def _set_keep_columns(on=True, max_bytes=None):
         _KEEP_COLUMNS["max_bytes"] = int(max_bytes)
 
 
+def _records(weight):
+    """Whether a backward call may follow that wants the weight's gradient.  Asked in front of Function.apply: inside, the grad mode
+    is off, and needs_input_grad is true of every Parameter whatever the mode."""
+    return torch.is_grad_enabled() and weight.requires_grad
+
+
 def _columns_for(lib, desc, sdesc, weight_grad_wanted, dev):
     if not (_KEEP_COLUMNS["on"] and weight_grad_wanted):
         return None
@@ -245,7 +251,7 @@ class _DeformConv3dFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, input, offset, alpha, weight, bias, sd, sh, sw, pd, ph, pw, dd, dh, dw, groups, offset_groups,
-                relu_scale=0.0, want_stats=False, offset_axes=7, backward_flags=0, prepared=None):
+                relu_scale=0.0, want_stats=False, offset_axes=7, backward_flags=0, prepared=None, records=False):
         lib = _lib.load()
         input, offset, weight = input.contiguous(), offset.contiguous(), weight.contiguous()
         alpha = alpha.contiguous() if alpha is not None else None
@@ -264,7 +270,7 @@ class _DeformConv3dFunction(torch.autograd.Function):
         with torch.cuda.device(dev):
             npre = lib.d2c_conv3d_prepared_bytes(ctypes.byref(desc)) if (prepared is not None and not want_stats) else 0
             ctx.prepared = None
-            columns = None if npre else _columns_for(lib, desc, None, ctx.needs_input_grad[3], dev)
+            columns = None if npre else _columns_for(lib, desc, None, records, dev)
             if want_stats and columns is None:
                 nb = lib.d2c_conv3d_forward_stats_workspace_bytes(ctypes.byref(desc), None)
                 ws, nb = _forward_workspace(lib, nb, desc, None, dev)
@@ -350,7 +356,7 @@ class _DeformConv3dFunction(torch.autograd.Function):
                                              _ptr(weight), _ptr(gx), _ptr(goff), _ptr(galpha), _ptr(gw), _ptr(gb),
                                              _ptr(ws), nb, _stream(dev))
         _lib.check(rc, "deform_conv3d backward")
-        return (gx, goff, galpha, gw, gb) + (None,) * 16
+        return (gx, goff, galpha, gw, gb) + (None,) * 17
 
 
 def deform_conv3d(input, offset, alpha, weight, bias, stride_d, stride_h, stride_w, pad_d, pad_h, pad_w,
@@ -375,7 +381,7 @@ def deform_conv3d(input, offset, alpha, weight, bias, stride_d, stride_h, stride
         input, offset, alpha, weight, bias, int(stride_d), int(stride_h), int(stride_w),
         int(pad_d), int(pad_h), int(pad_w), int(dilation_d), int(dilation_h), int(dilation_w),
         int(groups), int(offset_groups), float(relu_scale), bool(want_stats), int(offset_axes), int(backward_flags),
-        prepared)
+        prepared, _records(weight))
 
 
 class _DeformConv3dSizedFunction(torch.autograd.Function):
@@ -386,7 +392,7 @@ class _DeformConv3dSizedFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, input, size_raw, alpha, weight, bias, mode, activation, stride, padding, dilation, groups,
-                relu_scale=0.0, want_stats=False):
+                relu_scale=0.0, want_stats=False, records=False):
         from .grid import size_map_desc
         lib = _lib.load()
         input, size_raw, weight = input.contiguous(), size_raw.contiguous(), weight.contiguous()
@@ -404,7 +410,7 @@ class _DeformConv3dSizedFunction(torch.autograd.Function):
         out = torch.empty((N, Cout, Do, Ho, Wo), dtype=input.dtype, device=dev)
         stats = torch.empty((N, Cout, 2), dtype=torch.float32, device=dev) if want_stats else None
         with torch.cuda.device(dev):
-            columns = _columns_for(lib, desc, sdesc, ctx.needs_input_grad[3], dev)
+            columns = _columns_for(lib, desc, sdesc, records, dev)
             if want_stats and columns is None:
                 nb = lib.d2c_conv3d_forward_stats_workspace_bytes(ctypes.byref(desc), ctypes.byref(sdesc))
                 ws, nb = _forward_workspace(lib, nb, desc, sdesc, dev)
@@ -465,7 +471,7 @@ class _DeformConv3dSizedFunction(torch.autograd.Function):
                                                    _ptr(size_raw), _ptr(alpha), _ptr(weight), _ptr(gx), _ptr(gsize),
                                                    _ptr(galpha), _ptr(gw), _ptr(gb), _ptr(ws), nb, _stream(dev))
         _lib.check(rc, "deform_conv3d_sized backward")
-        return (gx, gsize, galpha, gw, gb) + (None,) * 8
+        return (gx, gsize, galpha, gw, gb) + (None,) * 9
 
 
 _SIZE_CHANNELS = {"xyz": 3, "xxz": 2, "xy": 2, "x": 1}
@@ -506,7 +512,7 @@ def deform_conv3d_sized(input, size_raw, alpha, weight, bias, mode, activation, 
     _check_common(3, input, stand_in, alpha, weight, bias, groups, 1)
     input, size_raw, alpha, weight, bias = _unify(input, size_raw, alpha, weight, bias)
     return _DeformConv3dSizedFunction.apply(input, size_raw, alpha, weight, bias, mode, activation, stride, padding,
-                                            dilation, int(groups), float(relu_scale), bool(want_stats))
+                                            dilation, int(groups), float(relu_scale), bool(want_stats), _records(weight))
 
 
 def _ptr_at(t, channel):
@@ -527,7 +533,7 @@ class _DeformConv3dPackedFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, input, deformation, weight, bias, lead, mask_act, mode, size_activation, stride, padding,
-                dilation, groups, offset_groups, relu_scale, want_stats, offset_axes, backward_flags):
+                dilation, groups, offset_groups, relu_scale, want_stats, offset_axes, backward_flags, records=False):
         lib = _lib.load()
         input, deformation, weight = input.contiguous(), deformation.contiguous(), weight.contiguous()
         bias = bias.contiguous() if bias is not None else None
@@ -550,7 +556,7 @@ class _DeformConv3dPackedFunction(torch.autograd.Function):
         stats = torch.empty((N, Cout, 2), dtype=torch.float32, device=dev) if want_stats else None
         p_off, p_mask = _ptr_at(deformation, 0), _ptr_at(deformation, lead)
         with torch.cuda.device(dev):
-            columns = _columns_for(lib, desc, sdesc, ctx.needs_input_grad[2], dev)
+            columns = _columns_for(lib, desc, sdesc, records, dev)
             if columns is not None:
                 nb = lib.d2c_conv3d_forward_keep_workspace_bytes(ctypes.byref(desc), sref)
                 ws = _workspace(nb, dev)
@@ -622,7 +628,7 @@ class _DeformConv3dPackedFunction(torch.autograd.Function):
                                              _ptr(weight), _ptr(gx), g_off, g_mask, _ptr(gw), _ptr(gb), _ptr(ws), nb,
                                              _stream(dev))
         _lib.check(rc, "deform_conv3d_packed backward")
-        return (gx, gdef, gw, gb) + (None,) * 13
+        return (gx, gdef, gw, gb) + (None,) * 14
 
 
 def deform_conv3d_packed_supported(input, deformation, weight, lead, mask_activation, mode, size_activation, stride,
@@ -690,7 +696,7 @@ def deform_conv3d_packed(input, deformation, weight, bias, lead, mask_activation
     return _DeformConv3dPackedFunction.apply(
         input, deformation, weight, bias, int(lead), _lib.MASK_ACTIVATIONS[mask_activation], mode, size_activation,
         tuple(int(v) for v in stride), tuple(int(v) for v in padding), tuple(int(v) for v in dilation), int(groups),
-        int(offset_groups), float(relu_scale), bool(want_stats), int(offset_axes), int(backward_flags))
+        int(offset_groups), float(relu_scale), bool(want_stats), int(offset_axes), int(backward_flags), _records(weight))
 
 
 def _plain_desc(input, weight, stride, padding, dilation):
