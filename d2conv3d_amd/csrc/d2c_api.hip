@@ -592,12 +592,18 @@ size_t d2c_conv3d_sized_forward_workspace_bytes(const d2c_conv3d_desc *q, const 
     return expanded_offsets_bytes(*q) + d2c_conv3d_forward_workspace_bytes(q);
 }
 
+// `which`: D2C_FWD_WS_GATHER or D2C_FWD_WS_LEAST
+static size_t forward_least(const d2c_conv3d_desc &q, const d2c_size_map_desc *z, D2cForwardWs which)
+{
+    const int a = choose_algo(q, true);
+    const size_t least = a == D2C_ALGO_MFMA || a == D2C_ALGO_DEPTHWISE ? d2c_tiled_forward_ws(q, which) : 0;
+    return z && !sized_fused(q, false) ? expanded_offsets_bytes(q) + least : least;
+}
+
 size_t d2c_conv3d_forward_least_workspace_bytes(const d2c_conv3d_desc *q, const d2c_size_map_desc *z)
 {
     if ((z ? sized_check(q, z) : d2c_conv3d_check(q)) != D2C_OK) return 0;
-    const int a = choose_algo(*q, true);
-    const size_t least = a == D2C_ALGO_MFMA || a == D2C_ALGO_DEPTHWISE ? d2c_tiled_forward_ws(*q, D2C_FWD_WS_GATHER) : 0;
-    return z && !sized_fused(*q, false) ? expanded_offsets_bytes(*q) + least : least;
+    return forward_least(*q, z, D2C_FWD_WS_GATHER);
 }
 
 size_t d2c_conv3d_sized_backward_workspace_bytes(const d2c_conv3d_desc *q, const d2c_size_map_desc *z)
@@ -614,7 +620,7 @@ int d2c_conv3d_sized_forward(const d2c_conv3d_desc *q, const d2c_size_map_desc *
     if (int rc = sized_check(q, z)) return rc;
     if (!x || !size_raw || !weight || !out) { d2c_set_error("null tensor pointer"); return D2C_ERR_SHAPE; }
     if (choose_algo(*q, false) < 0) return D2C_ERR_UNSUPPORTED;
-    if (int rc = check_ws(d2c_conv3d_forward_least_workspace_bytes(q, z), ws, ws_bytes)) return rc;
+    if (int rc = check_ws(forward_least(*q, z, D2C_FWD_WS_LEAST), ws, ws_bytes)) return rc;
     if (sized_fused(*q, false))
         return d2c_tiled_forward(*q, x, size_raw, mask, weight, bias, out, ws, ws_bytes, (hipStream_t)stream, z);
     const size_t ob = expanded_offsets_bytes(*q);
