@@ -1144,7 +1144,7 @@ size_t d2c_tiled_forward_ws(const d2c_conv3d_desc &q, D2cForwardWs which)
     case D2C_FWD_WS_GATHER: return l.least + d2c_fwd_split_bytes(s);
     case D2C_FWD_WS_LEAST: return l.least;
     case D2C_FWD_WS_STATS: return l.least + (d2c_fwd_fills_stats(s) ? d2c_fwd_stats_ws(s) : 0);
-    case D2C_FWD_WS_KEEP: return use_brick_forward(q, s, true) ? l.lists : l.least;
+    case D2C_FWD_WS_KEEP: return use_brick_forward(q, s, true) ? l.lists : l.least + d2c_fwd_split_bytes(s);
     case D2C_FWD_WS_KEEP_LEAST:
         return !use_brick_forward(q, s, true) ? l.least : (d2c_fwd_writes_columns(s, q.dtype) ? std::min(l.least, l.lists) : l.lists);
     default: return l.total;
