@@ -834,7 +834,7 @@ int launch_fwd_dma(FwdArgs a, float *outacc, hipStream_t st)
 //   positions 65, 53 (float32 70, 72), 1400 positions 82, 102; below about a thousand steps over all tiles (4 tiles of 48 steps,
 //   conv1d) its pipeline is not filled either.
 constexpr int kDmaTilesNarrow = 160, kDmaTilesWide = 128, kDmaTilesLeast = 10, kDmaStepsWide = 1024, kColsTiles = 48,
-              kColsTilesNarrowF32 = 48, kColsTilesWideF32 = 20;
+              kColsStepsNarrowF32 = 2048, kColsTilesWideF32 = 20;
 constexpr size_t kDmaWeightBytes = 8u << 20;
 static long dma_tiles(const TiledShape &s) { return (long)((s.M + kDMT - 1) / kDMT) * s.groups; }
 bool d2c_fwd_use_dma(const TiledShape &s)
@@ -881,14 +881,16 @@ size_t d2c_fwd_stats_ws(const TiledShape &s)
 // offsets along all three axes, wide weight groups from kColsTiles position tiles on (below that the backward kernels
 // that read the columns lose to the ones that sample again: 256 -> 256 channels on 4x15x27, 26 tiles: 0.25 -> 0.30 ms),
 // narrow ones from kDmaTilesNarrow tiles on.  Float32, whose backward pass over sorted points samples again where no columns are
-// kept, from fewer (training steps, us, sampling again first: 128 -> 128 channels, 40 tiles 191, 197; 48 tiles 213, 203; 80 tiles
-// 296, 240; 512 -> 128: 480, 472; 567, 513; 938, 686; 64 -> 200: 16 tiles 142, 156; 22 tiles 164, 159; 256 -> 256: 239, 232; 267, 246).
+// kept, from fewer: wide groups from kColsTilesWideF32 tiles, narrow ones from kColsTiles on or by the steps of all tiles.  Training steps, us, columns kept,
+// sampling again; narrow, 27 taps: 64 -> 64 24 tiles 119, 117; 32 120, 124; 48 135, 147.  128 -> 128 8 130, 127; 12 128, 133; 20 134, 151.
+// 256 -> 128 4 141, 142; 8 146, 156; 12 154, 172.  512 -> 128 4 174, 191.  9 taps, 256 -> 64: 24 127, 124; 32 125, 135.  7 taps, 128 -> 128: 60 129,
+// 129; 80 127, 144.  Wide: 64 -> 200 20 154, 157; 32 166, 171.  256 -> 256 12 209, 218; 20 235, 259.  512 -> 512 12 534, 542; 20 522, 632.
 bool d2c_fwd_writes_columns(const TiledShape &s, int dtype)
 {
     const long tiles = dma_tiles(s);
-    return (dtype == D2C_BF16 || dtype == D2C_F32) && s.nd == 3 && (s.axes & 7) == 7 &&
-           (s.og <= 128 ? tiles >= (dtype == D2C_F32 ? kColsTilesNarrowF32 : kDmaTilesNarrow)
-                        : d2c_fwd_use_dma(s) && tiles >= (dtype == D2C_F32 ? kColsTilesWideF32 : kColsTiles));
+    if ((dtype != D2C_BF16 && dtype != D2C_F32) || s.nd != 3 || (s.axes & 7) != 7) return false;
+    if (s.og <= 128) return dtype == D2C_F32 ? tiles >= kColsTiles || tiles * s.nchunk * s.K >= kColsStepsNarrowF32 : tiles >= kDmaTilesNarrow;
+    return d2c_fwd_use_dma(s) && tiles >= (dtype == D2C_F32 ? kColsTilesWideF32 : kColsTiles);
 }
 long d2c_columns_rows(const TiledShape &s) { return (long)((s.M + kDMT - 1) / kDMT) * kDMT; }
 // `stats` / `stats_part`: the [N][Cout][2] result and the per-tile scratch of d2c_fwd_stats_ws() bytes, or NULL.

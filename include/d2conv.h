@@ -207,7 +207,8 @@ int d2c_conv3d_backward(const d2c_conv3d_desc *desc, const void *grad_out, const
  * the size map that `offset` then is.  d2c_conv3d_columns_bytes() is 0 where this is not served (anything but
  * bfloat16 and float32 problems on the matrix-core kernels with an even number of 64- / 32-channel chunks per weight
  * group, offsets along all three axes, and enough output positions: tiles of 64 times weight groups at least 48 -- bfloat16 with up to 128
- * output channels per weight group 160, float32 with more 20 --, or, bfloat16 with
+ * output channels per weight group 160, float32 with more 20, float32 with up to 128 also where tiles times taps times chunks are at
+ * least 2048 --, or, bfloat16 with
  * one weight group, at least 400 positions and 2048 positions times chunks); the two calls then
  * fail with D2C_ERR_UNSUPPORTED and the caller uses the plain ones.  The memory-saving bits of
  * d2c_conv3d_desc::backward_flags are ignored by d2c_conv3d_backward_columns.

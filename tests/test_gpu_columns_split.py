@@ -13,7 +13,7 @@ from _util import assert_close
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("cin,cout,dims", [(64, 64, (6, 17, 31)), (128, 100, (5, 25, 27))])     # 50 and 53 tiles of 64 positions
+@pytest.mark.parametrize("cin,cout,dims", [(64, 64, (6, 17, 31)), (128, 100, (5, 25, 27)), (256, 72, (3, 15, 15))])     # 50, 53 and 11 tiles of 64 positions
 def test_kept_columns_beside_partial_sums(cin, cout, dims, dev):
     g = torch.Generator().manual_seed(cout)
     rn = lambda *s: torch.randn(*s, generator=g)
