@@ -683,12 +683,27 @@ int gw_mode(const d2c_conv3d_desc &q)
     const int f = q.backward_flags & D2C_BWD_GW_MASK;
     return f == D2C_BWD_GW_DEFAULT ? d2c_col_weight_mode() : (f == D2C_BWD_GW_RESAMPLE ? 0 : f);
 }
+// Float32 problems that the bricks serve and that bring no columns have two ways: the bricks, which write none, and a second
+// sampling for grad_weight; or the gathering kernels, which write columns, and the product over them.  The second sampling multiplies on
+// the float32 instruction, in passes and tiles of 256 output channels, the product over whole sets of four chunks on the bfloat16 one; the
+// bricks gain most where the points are few.  Training steps, bricks and second sampling / gathering and columns, us:
+//   up to 128 output channels: 128 -> 64 on 2560 positions 1.05, 8192 1.23; 256 -> 128 1400 0.94, 3240 1.08, 12960 1.05; 1024 -> 128 1400 0.95, 3240 1.07
+//   up to 256 (the tile is full): 256 -> 256 on 1400 254, 283; 5120 557, 571; 12960 1259, 1257; 64 -> 256 1400 153, 173; 25600 768, 798
+//   more: 256 -> 512 on 504 270, 310; 1400 382, 392; 2560 516, 500; 12960 1940, 1793;  256 -> 1024 504 465, 474; 1008 576, 544; 12960 3994, 2985
+//   offset groups, whose points are sorted each on its own: 512 -> 512, 8 groups, 256 369, 370; 504 427, 410; 12960 4078, 3340;
+//   512 -> 128, 8 groups, 256 0.96, 784 1.11;  256 -> 128, 2 groups, 1008 0.96, 2000 1.09
+//   fewer taps: 256 -> 256, 9, 5120 269, 299; 12960 504, 489;  7 5120 235, 278; 25600 766, 741
+//   chunks that make no whole sets, on the float32 instruction both ways: 64 -> 64 on 5120 182, 192; 25600 602, 630;  320 -> 256 12960 0.94
+bool columns_pay(const d2c_conv3d_desc &q, const TiledShape &s)
+{
+    const int pass = d2c_bwd_pass_channels(q.dtype);
+    if (s.nchunk % 4 || (s.og > 128 && s.og <= pass)) return false;
+    return (double)s.M * s.K * ((s.og + pass - 1) / pass) * (s.G / s.groups + 1) >= 150000.0;
+}
 bool use_col_weight(const d2c_conv3d_desc &q, const TiledShape &s)
 {
-    // (float32 over sorted points samples again: those kernels write no columns, and the ones that do take longer than the second
-    // sampling saves.  Training steps, us, sorted points first: 64 -> 64 channels on 4x14x25 130, 136; 256 -> 256 on 4x9x9 181, 232;
-    // 1024 -> 128 on 8x20x32 1730, 1808)
-    if (q.dtype != D2C_BF16 && (gw_mode(q) != 1 || ((q.backward_flags & D2C_BWD_GW_MASK) == D2C_BWD_GW_DEFAULT && use_brick(q, s)))) return false;
+    if (q.dtype != D2C_BF16 && (gw_mode(q) != 1 || ((q.backward_flags & D2C_BWD_GW_MASK) == D2C_BWD_GW_DEFAULT && use_brick(q, s) && !columns_pay(q, s))))
+        return false;
     return gw_mode(q) && use_aux_kernel(q, s) && d2c_bwd_weight_from_col(s, q.dtype);
 }
 // ... written over the grad-column rows (mode 2): grad_input is taken from those rows first, from sample lists

@@ -75,8 +75,9 @@ enum {
  * Both d2c_conv3d_backward_workspace_bytes() and d2c_conv3d_backward() read the field from the description they
  * are given, so the size asked for and the call agree per description.  0 = the defaults. */
 #define D2C_BWD_GW_DEFAULT   0   /* grad_weight as a matrix product over sampled columns in a buffer of their own; float32 problems
-                                  * whose gradients run over sorted sampling points sample again instead (faster, half the memory) */
-#define D2C_BWD_GW_COLUMNS   1   /* such columns whatever the type */
+                                  * whose gradients run over sorted sampling points sample again where that is faster: few positions,
+                                  * 129 to 256 output channels, channels that are no multiple of 128 (half the memory, too) */
+#define D2C_BWD_GW_COLUMNS   1   /* such columns whatever the type and size */
 #define D2C_BWD_GW_IN_PLACE  2   /* the columns written over the grad-column rows: no buffer of their own
                                   * (bfloat16; float32 problems then sample again) */
 #define D2C_BWD_GW_RESAMPLE  3   /* no columns at all: the grad-weight kernel samples the input again */
