@@ -648,11 +648,12 @@ bool use_aux_kernel(const d2c_conv3d_desc &q, const TiledShape &s)
 // at hand.  (A bucket capacity asked for by the test hook is a matter of the lists.)
 bool use_brick(const d2c_conv3d_desc &q, const TiledShape &s)
 {
-    // (float32 weight groups that take several passes of the grad-column product: from 1024 positions on.  Training steps, us, lists first:
-    // 64 -> 512 channels on 1400 positions 233, 216; 5120 341, 319; 16000 715, 646; 512 -> 512, 8 groups, 25920 6180, 5350.  A test holds
-    // problems of some dozen positions to the lists.)
+    // (float32 weight groups that take several passes of the grad-column product: from 128 positions on.  Training steps without kept
+    // columns, us, lists first: 64 -> 320 channels on 50 positions 136, 129; 144 152, 129; 504 177, 147; 256 -> 512 50 239, 201; 256 293, 242;
+    // 512 -> 1024 50 579, 508; 256 729, 678; with kept columns 64 -> 320 on 12960 573, 531; 512 -> 1024 5765, 5331.  Fewer than two tiles of
+    // positions stay with the lists for a test's sake, which holds them to this way; it costs them 5 - 20 %.)
     return d2c_gx_mode() == 1 && use_lists(q, s) && use_aux_kernel(q, s) && d2c_brick_supported(s, q.dtype) &&
-           (q.dtype == D2C_BF16 || d2c_tiled_bwd_single_pass(s, q.dtype) || s.M >= 1024);
+           (q.dtype == D2C_BF16 || d2c_tiled_bwd_single_pass(s, q.dtype) || s.M >= 128);
 }
 
 // The forward pass over sampled columns: sort, sample, multiply.  `kept`: the caller keeps the columns, where the backward call can

@@ -16,7 +16,9 @@ pytestmark = pytest.mark.gpu
 # 27 taps x positions x (8 offset groups + 1) x passes of 256 output channels: 150000 lies between 617 and 618 positions of the first
 @pytest.mark.parametrize("cin,cout,G,dims,columns", [(512, 128, 8, (1, 1, 617), False), (512, 128, 8, (2, 3, 103), True),
                                                      (256, 320, 1, (3, 20, 23), False), (256, 320, 1, (3, 20, 24), True),
-                                                     (64, 320, 1, (3, 20, 24), False), (128, 200, 2, (4, 24, 24), False)])
+                                                     (64, 320, 1, (3, 20, 24), False), (128, 200, 2, (4, 24, 24), False),
+                                                     # several passes: sorted points from 128 positions on
+                                                     (64, 320, 1, (4, 4, 8), False), (64, 320, 1, (1, 1, 127), True)])
 def test_default_of_float32_problems_without_kept_columns(cin, cout, G, dims, columns, dev):
     lib = _lib.load()
     need = {}
