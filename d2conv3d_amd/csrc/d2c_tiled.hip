@@ -664,13 +664,18 @@ bool use_brick(const d2c_conv3d_desc &q, const TiledShape &s)
 // where the columns stop losing):
 //   training step:  128 -> 128: 405 positions 133, 140; 810 151, 145; 1296 176, 152; 5760 308, 190   128 -> 40: 810 132, 141; 1296 149, 138
 //                   256 -> 64: 405 143, 144; 810 168, 153    256 -> 256: 5760 338, 288    1024 -> 256: 810 308, 288; 5760 772, 674
-//   forward alone:  256 -> 256: 4320 91, 99; 7072 114, 119; 8512 151, 132; 11968 171, 158
-//                   512 -> 512: 4320 169, 156; 8512 300, 236    1024 -> 256: 3240 160, 175; 5760 270, 262
-//                   1024 -> 128: 4320 690, 164; 11968 471, 365   2048 -> 256, 7 taps: 3240 102, 116; 5808 168, 153
+//   forward alone:  256 -> 256: 4000 75, 80; 5120 88, 85; 6912 120, 96    192 -> 192: 5120 71, 71; 6912 94, 81; 28800 247, 195
+//                   512 -> 512: 1600 84, 85; 2560 106, 102; 4000 139, 129; in 2 groups 2560 105, 101; 6400 209, 180
+//                   1024 -> 256: 1600 92, 106; 2560 129, 121; 4000 178, 154   128 -> 128: 28800 135, 139
+//                   up to 128 output channels (the gathering kernel there is the one of the small problems): 256 -> 128: 6912 65, 83; 8880 105, 103;
+//                   512 -> 64: 4000 61, 87; 5120 97, 95; 1024 -> 128: 2560 78, 102; 4000 130, 132
+//                   7 taps: 256 -> 256: 5120 49, 52; 8880 64, 63    2048 -> 256: 3240 97, 101; 4000 111, 109
 bool use_brick_forward(const d2c_conv3d_desc &q, const TiledShape &s, bool kept)
 {
     const long chunks = s.Cin / 64, of_group = s.cpg / 64;
-    const bool large = kept ? s.M >= 400 && s.M * chunks >= 2048 : of_group >= 4 && s.M >= 4096 && s.M * of_group >= 32768;
+    const bool large = kept ? s.M >= 400 && s.M * chunks >= 2048
+                            : (of_group >= 4 && s.M >= 4096 && s.M * of_group >= 32768) ||
+                              (of_group >= 3 && s.K >= 27 && s.og > 128 && s.M >= 2560 && s.M * chunks >= 20480);
     return large && q.dtype == D2C_BF16 && use_brick(q, s) && s.groups == 1 && brick_col_bytes(s) < (4ull << 30) &&
            (!kept || d2c_bwd_weight_from_kept_col(s, q.dtype));
 }
