@@ -236,9 +236,7 @@ def _columns_for(lib, desc, sdesc, weight_grad_wanted, dev):
 
 
 def _channel_stats_into(lib, x, stats):
-    """The sums that d2c_conv3d_forward_stats fills, of an output that another forward call has stored: a call that keeps its
-    columns runs without statistics, and one more pass over the output costs less than the backward pass's second sampling
-    (512 -> 512 channels on 2x8x30x54 with ReLU and GroupNorm, forward + backward: 2.27 -> 1.84 ms)."""
+    """The sums that d2c_conv3d_forward_stats fills, of an output that the call which keeps its columns has stored."""
     N, C = x.shape[:2]
     desc = _lib.GroupNormDesc(N, C, x[0, 0].numel(), 1, _DT[x.dtype], 0.0)
     return lib.d2c_channel_stats(ctypes.byref(desc), _ptr(x), _ptr(stats), _stream(x.device))
@@ -364,8 +362,8 @@ def deform_conv3d(input, offset, alpha, weight, bias, stride_d, stride_h, stride
                   offset_axes=7, backward_flags=0, prepared=None):
     """deform_conv3d of dconv3d.h:188-226; `alpha` and `bias` may be None.  `relu_scale` > 0 fuses
     relu_scale * relu(.) into the store of the output (see _DeformConv3dFunction).  `want_stats` also returns the
-    float32 [N, Cout, 2] sums and sums of squares of the stored output per (sample, channel), added up by the
-    forward kernel where it stores, or by a pass over it (the statistics a GroupNorm behind the convolution needs).  `offset_axes`: mask
+    float32 [N, Cout, 2] sums and sums of squares of the stored output per (sample, channel), by a pass over it (the
+    statistics a GroupNorm behind the convolution needs).  `offset_axes`: mask
     of the axes (1 z, 2 y, 4 x) the offsets displace along; the others are taken as zero and their gradient
     channels come back zero (matrix-core kernels only, see conv3d_algo).  `backward_flags`: the description's field
     of that name (_lib.BWD_GW_* | _lib.bwd_slices(n)): how the backward pass trades workspace for time.  `prepared`: a
@@ -767,7 +765,7 @@ def plain_conv3d(input, weight, bias, stride, padding, dilation):
 
 
 class _GroupNormFromStats(torch.autograd.Function):
-    """torch.nn.functional.group_norm on the output of a convolution whose forward kernels already added up the
+    """torch.nn.functional.group_norm on the output of a convolution whose call returned the
     per-(sample, channel) sums (d2c_conv3d_forward_stats): d2c_group_norm_forward / _backward."""
 
     @staticmethod

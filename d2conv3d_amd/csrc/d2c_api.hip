@@ -440,7 +440,7 @@ int d2c_conv3d_forward_prepared(const d2c_conv3d_desc *q, const void *x, const v
     D2cPrepared prep;
     if (int rc = check_prepared(*q, prepared, prepared_bytes, reuse, &prep)) return rc;
     if (int rc = check_ws(d2c_tiled_forward_ws(*q, D2C_FWD_WS_LEAST), ws, ws_bytes)) return rc;
-    return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, ws_bytes, st, nullptr, nullptr, prep.base ? &prep : nullptr);
+    return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, ws_bytes, st, nullptr, prep.base ? &prep : nullptr);
 }
 
 int d2c_conv3d_backward_prepared(const d2c_conv3d_desc *q, const void *gout, const void *x, const void *offset,
@@ -649,15 +649,9 @@ int d2c_conv3d_sized_backward(const d2c_conv3d_desc *q, const d2c_size_map_desc 
     return D2C_OK;
 }
 
-static bool stats_fused(const d2c_conv3d_desc &q, const d2c_size_map_desc *z)
-{
-    return choose_algo(q, true) == D2C_ALGO_MFMA && d2c_tiled_forward_fills_stats(q) && (!z || sized_fused(q, false));
-}
-
 size_t d2c_conv3d_forward_stats_workspace_bytes(const d2c_conv3d_desc *q, const d2c_size_map_desc *z)
 {
     if ((z ? sized_check(q, z) : d2c_conv3d_check(q)) != D2C_OK) return 0;
-    if (stats_fused(*q, z)) return d2c_tiled_forward_ws(*q, D2C_FWD_WS_STATS);
     return z ? d2c_conv3d_sized_forward_workspace_bytes(q, z) : d2c_conv3d_forward_workspace_bytes(q);
 }
 
@@ -668,13 +662,9 @@ int d2c_conv3d_forward_stats(const d2c_conv3d_desc *q, const d2c_size_map_desc *
     if (int rc = z ? sized_check(q, z) : d2c_conv3d_check(q)) return rc;
     if (!x || !offset || !weight || !out || !chan_stats) { d2c_set_error("null tensor pointer"); return D2C_ERR_SHAPE; }
     if (q->dtype == D2C_F64) { d2c_set_error("output statistics: float32 or bfloat16 only"); return D2C_ERR_DTYPE; }
-    const int a = choose_algo(*q, false);
-    if (a < 0) return D2C_ERR_UNSUPPORTED;
-    // the kernels that add the sums up on their way: matrix-core family, offsets from a tensor or formed in the sampler
-    if (stats_fused(*q, z)) {
-        if (int rc = check_ws(d2c_tiled_forward_ws(*q, D2C_FWD_WS_STATS), ws, ws_bytes)) return rc;
-        return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, ws_bytes, (hipStream_t)stream, z, chan_stats);
-    }
+    // (a pass over the output: added up by the forward kernels' epilogues they cost more.  us beside the call alone, by the DMA-gather
+    // kernel, by the pass: 64 -> 256 channels, float32, 12960 positions 32, 6; 51360 75, 16; 256 -> 256 1400 8, 5; 51360 64, 13;
+    // bfloat16 128 -> 512 51360 59, 12; 256 -> 256 1400 13, 7)
     if (int rc = z ? d2c_conv3d_sized_forward(q, z, x, offset, mask, weight, bias, out, ws, ws_bytes, stream)
                    : d2c_conv3d_forward(q, x, offset, mask, weight, bias, out, ws, ws_bytes, stream))
         return rc;
@@ -724,7 +714,7 @@ int d2c_conv3d_forward_columns(const d2c_conv3d_desc *q, const d2c_size_map_desc
     if (int rc = check_columns(*q, z, columns, columns_bytes)) return rc;
     const bool keep = columns_bytes >= d2c_tiled_keep_bytes(*q, z);
     if (int rc = check_ws(d2c_tiled_forward_ws(*q, keep ? D2C_FWD_WS_KEEP_LEAST : D2C_FWD_WS_LEAST), ws, ws_bytes)) return rc;
-    return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, ws_bytes, (hipStream_t)stream, z, nullptr, nullptr, columns,
+    return d2c_tiled_forward(*q, x, offset, mask, weight, bias, out, ws, ws_bytes, (hipStream_t)stream, z, nullptr, columns,
                              columns_bytes);
 }
 

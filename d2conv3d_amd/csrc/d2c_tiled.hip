@@ -17,12 +17,9 @@ int d2c_grad_col(const d2c_conv3d_desc &q, void *gcol, void *ws, hipStream_t st)
 int d2c_fwd_out_tile(const TiledShape &s);
 template <typename T>
 int d2c_tiled_fwd_launch(const TiledShape &s, const void *xcl, const void *off, const void *mask, const void *wp,
-                         const void *bias, void *out, float *outacc, hipStream_t st, float *stats, float *stats_part,
-                         void *col = nullptr);
+                         const void *bias, void *out, float *outacc, hipStream_t st, void *col = nullptr);
 bool d2c_fwd_writes_columns(const TiledShape &s, int dtype);
 long d2c_columns_rows(const TiledShape &s);
-bool d2c_fwd_fills_stats(const TiledShape &s);
-size_t d2c_fwd_stats_ws(const TiledShape &s);
 bool d2c_fwd_use_dma(const TiledShape &s);
 size_t d2c_fwd_split_count_bytes(const TiledShape &s);
 size_t d2c_fwd_split_bytes(const TiledShape &s);
@@ -570,7 +567,7 @@ DwWs dw_ws(const d2c_conv3d_desc &q, const TiledShape &s)
 template <typename T>
 int forward_t(const d2c_conv3d_desc &q, const void *x, const void *off, const void *mask, const void *w,
               const void *bias, void *out, void *ws, hipStream_t st, int nd = 3, const d2c_size_map_desc *sz = nullptr,
-              float *stats = nullptr, const D2cPrepared *prep = nullptr, void *columns = nullptr, size_t columns_bytes = 0,
+              const D2cPrepared *prep = nullptr, void *columns = nullptr, size_t columns_bytes = 0,
               size_t ws_bytes = 0)
 {
     const TiledShape s = tiled_shape(q, nd, 0, sz);
@@ -587,7 +584,7 @@ int forward_t(const d2c_conv3d_desc &q, const void *x, const void *off, const vo
     char *xcl_p = prep ? (char *)prep->base + pl.xcl : base + l.xcl;
     char *wp_p = prep ? (char *)prep->base + pl.wp : base + l.wp;
     const bool have_x = prep && (prep->reuse & D2C_REUSE_INPUT);
-    if (nd == 3 && !prep && !stats && use_brick_forward(q, s, columns != nullptr)) {
+    if (nd == 3 && !prep && use_brick_forward(q, s, columns != nullptr)) {
         // sort the points, sample the columns (the caller's buffer, with the sorted points and the input behind them for its
         // backward call, or the workspace), multiply.  A smaller workspace: the gathering kernels, below.
         const bool keep = columns && columns_bytes >= brick_keep_bytes(s);
@@ -618,9 +615,7 @@ int forward_t(const d2c_conv3d_desc &q, const void *x, const void *off, const vo
     const bool shared = d2c_fwd_use_dma(s) || (split && (nd != 3 || ws_bytes >= l.outacc + split));
     if (shared && split) prep_zero(pa, 0, base + l.outacc, d2c_fwd_split_count_bytes(s));
     if (int rc = prep_launch<T>(pa, st)) return rc;
-    // (the per-tile sums of the output statistics go behind everything else in the workspace)
-    return d2c_tiled_fwd_launch<T>(s, xcl_p, off, mask, wp_p, bias, out, shared ? (float *)(base + l.outacc) : nullptr, st,
-                                   stats, stats ? (float *)(base + l.least) : nullptr, columns);
+    return d2c_tiled_fwd_launch<T>(s, xcl_p, off, mask, wp_p, bias, out, shared ? (float *)(base + l.outacc) : nullptr, st, columns);
 }
 
 // grad_input by sample lists (see d2c_invlist.hip): from whole grad-column rows, i.e. the reduction over all output
@@ -1164,7 +1159,6 @@ size_t d2c_tiled_forward_ws(const d2c_conv3d_desc &q, D2cForwardWs which)
     switch (which) {
     case D2C_FWD_WS_GATHER: return l.least + d2c_fwd_split_bytes(s);
     case D2C_FWD_WS_LEAST: return l.least;
-    case D2C_FWD_WS_STATS: return l.least + (d2c_fwd_fills_stats(s) ? d2c_fwd_stats_ws(s) : 0);
     case D2C_FWD_WS_KEEP: return use_brick_forward(q, s, true) ? l.lists : l.least + d2c_fwd_split_bytes(s);
     case D2C_FWD_WS_KEEP_LEAST:
         return !use_brick_forward(q, s, true) ? l.least : (d2c_fwd_writes_columns(s, q.dtype) ? std::min(l.least, l.lists) : l.lists);
@@ -1212,11 +1206,11 @@ bool d2c_tiled_sized_supported(const d2c_conv3d_desc &q, bool backward)
 }
 
 int d2c_tiled_forward(const d2c_conv3d_desc &q, const void *x, const void *off, const void *mask, const void *w,
-                      const void *bias, void *out, void *ws, size_t ws_bytes, hipStream_t st, const d2c_size_map_desc *sz, float *stats,
+                      const void *bias, void *out, void *ws, size_t ws_bytes, hipStream_t st, const d2c_size_map_desc *sz,
                       const D2cPrepared *prep, void *columns, size_t columns_bytes)
 {
-    if (q.dtype == D2C_BF16) return forward_t<bf16_t>(q, x, off, mask, w, bias, out, ws, st, 3, sz, stats, prep, columns, columns_bytes, ws_bytes);
-    return forward_t<float>(q, x, off, mask, w, bias, out, ws, st, 3, sz, stats, prep, columns, columns_bytes, ws_bytes);
+    if (q.dtype == D2C_BF16) return forward_t<bf16_t>(q, x, off, mask, w, bias, out, ws, st, 3, sz, prep, columns, columns_bytes, ws_bytes);
+    return forward_t<float>(q, x, off, mask, w, bias, out, ws, st, 3, sz, prep, columns, columns_bytes, ws_bytes);
 }
 
 // Bytes of the caller-held prepared region of a description (0: the kernel family keeps nothing worth holding)
@@ -1224,12 +1218,6 @@ size_t d2c_tiled_prepared_bytes(const d2c_conv3d_desc &q)
 {
     if (is_depthwise(q) || !mfma_channels_ok(q)) return 0;
     return prepared_layout(q, tiled_shape(q)).total;
-}
-
-// The forward kernels of this description add up per-channel statistics of the output on their way.
-bool d2c_tiled_forward_fills_stats(const d2c_conv3d_desc &q)
-{
-    return !is_depthwise(q) && mfma_channels_ok(q) && d2c_fwd_fills_stats(tiled_shape(q)) && !use_brick_forward(q, tiled_shape(q), false);
 }
 
 int d2c_tiled_backward(const d2c_conv3d_desc &q, const void *gout, const void *x, const void *off,

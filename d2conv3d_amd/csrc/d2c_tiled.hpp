@@ -11,9 +11,9 @@ bool d2c_tiled_packed_supported(const d2c_conv3d_desc &q);
 // whether a description with some offset axes fixed (offset_axes != 7) stays on the tiled kernels in both directions
 bool d2c_tiled_axes_supported(const d2c_conv3d_desc &q);
 // Workspace of a forward call: what it is fastest with; what the gathering kernels are fastest with (with room for the
-// partial sums of a small problem); the least it runs with; what one that adds up output statistics on its way needs; what a
-// call that keeps its columns is fastest with, given a buffer of d2c_tiled_keep_bytes(); the least that one runs with
-enum D2cForwardWs { D2C_FWD_WS_FAST, D2C_FWD_WS_GATHER, D2C_FWD_WS_LEAST, D2C_FWD_WS_STATS, D2C_FWD_WS_KEEP, D2C_FWD_WS_KEEP_LEAST };
+// partial sums of a small problem); the least it runs with; what a call that keeps its columns is fastest with, given a
+// buffer of d2c_tiled_keep_bytes(); the least that one runs with
+enum D2cForwardWs { D2C_FWD_WS_FAST, D2C_FWD_WS_GATHER, D2C_FWD_WS_LEAST, D2C_FWD_WS_KEEP, D2C_FWD_WS_KEEP_LEAST };
 size_t d2c_tiled_forward_ws(const d2c_conv3d_desc &q, D2cForwardWs which = D2C_FWD_WS_FAST);
 // `sz` != nullptr: the offsets are formed from a raw size map (`off` is that map [N, channels(mode), P], `goff` the
 // gradient with respect to it); only where d2c_tiled_sized_supported() says so.
@@ -24,9 +24,6 @@ size_t d2c_tiled_backward_ws(const d2c_conv3d_desc &q, const d2c_size_map_desc *
 size_t d2c_tiled_columns_bytes(const d2c_conv3d_desc &q, const d2c_size_map_desc *sz = nullptr);
 size_t d2c_tiled_keep_bytes(const d2c_conv3d_desc &q, const d2c_size_map_desc *sz = nullptr);
 bool d2c_tiled_sized_supported(const d2c_conv3d_desc &q, bool backward);
-// `stats` != nullptr (only where d2c_tiled_forward_fills_stats() says so): fp32 [N][Cout][2], the sum and the sum of
-// squares of the stored output per (sample, channel).
-bool d2c_tiled_forward_fills_stats(const d2c_conv3d_desc &q);
 // `prep` != nullptr: a caller-held region of d2c_tiled_prepared_bytes() bytes that takes the place of the
 // workspace's channels-last input and packed weights; the parts named in `reuse` (D2C_REUSE_*) are taken as they are.
 struct D2cPrepared {
@@ -36,8 +33,7 @@ struct D2cPrepared {
 size_t d2c_tiled_prepared_bytes(const d2c_conv3d_desc &q);
 int d2c_tiled_forward(const d2c_conv3d_desc &q, const void *x, const void *off, const void *mask, const void *w,
                       const void *bias, void *out, void *ws, size_t ws_bytes, hipStream_t st, const d2c_size_map_desc *sz = nullptr,
-                      float *stats = nullptr, const D2cPrepared *prep = nullptr, void *columns = nullptr,
-                      size_t columns_bytes = 0);
+                      const D2cPrepared *prep = nullptr, void *columns = nullptr, size_t columns_bytes = 0);
 int d2c_tiled_backward(const d2c_conv3d_desc &q, const void *gout, const void *x, const void *off,
                        const void *mask, const void *w, void *gx, void *goff, void *gmask, void *gw, void *gb,
                        void *ws, hipStream_t st, const d2c_size_map_desc *sz = nullptr, const D2cPrepared *prep = nullptr,

@@ -45,12 +45,6 @@ struct FwdArgs {
     // one time are at about the same steps and share their weight fragments in L2.  The pieces add into
     // `outacc`, here laid out [item - sk_full][output channel of the tile][position of the tile].
     int sk_items, sk_full, sk_ntile, sk_otiles, sk_cut;
-    // Statistics for a normalisation behind the convolution (GroupNorm), or NULL: the sum and the sum of squares of
-    // the values as stored, per position tile and output channel, fp32 [position tile][2][Cout][2] -- a tile of 64
-    // positions lies in one sample or straddles two (slot 0: the sample of its first position, slot 1: the next
-    // one); every entry has exactly one writer (no atomics: they would all land on the same few cache lines), and
-    // stats_reduce_kernel adds the tiles of a sample up.  Filled by the DMA-gather kernel and its finishing kernel.
-    float *stats;
     // The sampled, modulated columns kept for the backward pass (or NULL): what the matrix step multiplies with the
     // weights, [chunk][tap][col_rows][BKC] in the element type, col_rows = position tiles x 64 (zeros past the last
     // position) -- the layout tiled_bwd_weight_col_kernel reads.  Written by the DMA-gather kernel.
@@ -526,56 +520,6 @@ D2C_DEV void fwd_dma_body(const FwdArgs &a, unsigned char *__restrict__ s_raw, u
                         if (oo < nvalid) atomicAdd(tp + oo * MT + pb * 32, acc[ob][pb][r]);
                         acc[ob][pb][r] = 0.f;
                     }
-        } else if (a.stats) {
-            // the same stores, and on the way the sum and the sum of squares of the stored values per output channel
-            // and sample slot: over the positions a lane holds, then over the 32 lanes of its half
-            const T *bias = reinterpret_cast<const T *>(a.bias);
-            const int b_lo = (w.tile * MT) / s.P;
-            bool okq[PB], hiq[PB];
-            T *opq[PB];
-#pragma unroll
-            for (int pb = 0; pb < PB; pb++) {
-                const int m = w.tile * MT + wave_p * WPOS + pb * 32 + (elane & 31);
-                okq[pb] = m < s.M;
-                const int b = m / s.P;
-                hiq[pb] = b != b_lo;
-                opq[pb] = reinterpret_cast<T *>(a.out) + ((long)b * s.Cout + o0) * s.P + (m - b * s.P);
-            }
-            float *sp = a.stats + ((long)w.tile * 2 * s.Cout + o0) * 2;
-#pragma unroll
-            for (int ob = 0; ob < OB; ob++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const int oo = ob * 32 + 8 * (r >> 2) + (r & 3);
-                    float q4[4] = {0.f, 0.f, 0.f, 0.f};     // slot 0: sum, sum of squares; slot 1 likewise
-#pragma unroll
-                    for (int pb = 0; pb < PB; pb++) {
-                        if (okq[pb] && oo < nvalid) {
-                            float v = acc[ob][pb][r];
-                            if (bias) v += elem_to_f32<T>(bias[o0 + oo]);
-                            const T sv = f32_to_elem<T>(d2c_epilogue(v, s.act, s.act_scale));
-                            opq[pb][(long)oo * s.P] = sv;
-                            const float fv = elem_to_f32<T>(sv);
-                            q4[0] += hiq[pb] ? 0.f : fv; q4[1] += hiq[pb] ? 0.f : fv * fv;
-                            q4[2] += hiq[pb] ? fv : 0.f; q4[3] += hiq[pb] ? fv * fv : 0.f;
-                        }
-                        acc[ob][pb][r] = 0.f;
-                    }
-#pragma unroll
-                    for (int d = 1; d < 32; d <<= 1)
-#pragma unroll
-                        for (int i = 0; i < 4; i++) q4[i] += __shfl_xor(q4[i], d, 64);
-                    if ((elane & 31) == 0 && oo < nvalid) {
-                        if (WAVES_P == 1) {
-                            sp[oo * 2] = q4[0]; sp[oo * 2 + 1] = q4[1];
-                            sp[(s.Cout + oo) * 2] = q4[2]; sp[(s.Cout + oo) * 2 + 1] = q4[3];
-                        } else {
-                            // (several wavefronts share a channel's positions: the slots were zeroed)
-                            atomicAdd(sp + oo * 2, q4[0]); atomicAdd(sp + oo * 2 + 1, q4[1]);
-                            atomicAdd(sp + (s.Cout + oo) * 2, q4[2]); atomicAdd(sp + (s.Cout + oo) * 2 + 1, q4[3]);
-                        }
-                    }
-                }
         } else {
             const T *bias = reinterpret_cast<const T *>(a.bias);
 #pragma unroll
@@ -696,68 +640,14 @@ __global__ void __launch_bounds__(256) fwd_dma_finish_kernel(FwdArgs a, int NT)
     const float *acc = a.outacc + (long)blockIdx.x * NT * MT;
     const T *bias = reinterpret_cast<const T *>(a.bias);
     T *out = reinterpret_cast<T *>(a.out);
-    const int b_lo = (tile * MT) / s.P;
-    static_assert(MT == 64, "one wavefront = the positions of one channel");
     for (int e = threadIdx.x; e < 32 * MT; e += 256) {
         const int ot = blockIdx.y * 32 + e / MT, pl = e % MT;
         const int ol = otile * NT + ot, m = tile * MT + pl;
-        float fv = 0.f;
-        const bool ok = ol < s.og && m < s.M;
-        const int o = wg * s.og + ol, b = ok ? m / s.P : b_lo, p = m - b * s.P;
-        if (ok) {
-            float v = acc[(long)ot * MT + pl];
-            if (bias) v += elem_to_f32<T>(bias[o]);
-            const T sv = f32_to_elem<T>(d2c_epilogue(v, s.act, s.act_scale));
-            out[((long)b * s.Cout + o) * s.P + p] = sv;
-            fv = elem_to_f32<T>(sv);
-        }
-        if (a.stats) {
-            // (e / MT is uniform over a wavefront: its 64 lanes are the positions of one channel)
-            const bool hi = b != b_lo;
-            float q4[4] = {hi ? 0.f : fv, hi ? 0.f : fv * fv, hi ? fv : 0.f, hi ? fv * fv : 0.f};
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1)
-#pragma unroll
-                for (int i = 0; i < 4; i++) q4[i] += __shfl_xor(q4[i], d, 64);
-            if (pl == 0 && ol < s.og) {
-                float *sp = a.stats + ((long)tile * 2 * s.Cout + o) * 2;
-                sp[0] = q4[0]; sp[1] = q4[1];
-                sp[s.Cout * 2] = q4[2]; sp[s.Cout * 2 + 1] = q4[3];
-            }
-        }
-    }
-}
-
-// chan_stats[n][c] = sums over the position tiles of sample n (see FwdArgs::stats).  A workgroup takes 8 channels of a
-// sample: 32 threads per channel walk the tiles (a row of 8 channels is 64 consecutive bytes) and add up through LDS
-// in a fixed order.  One thread per channel, walking all tiles alone, is one long chain of loads: 239 us at 803 tiles
-// and 256 channels (8x60x107), 8 us this way.
-constexpr int kStatChan = 8;
-__global__ void __launch_bounds__(256) stats_reduce_kernel(const float *part, float *chan_stats, int N, int Cout, int P, int M)
-{
-    __shared__ float2 red[32][kStatChan];
-    const int nblk = (Cout + kStatChan - 1) / kStatChan, n = blockIdx.x / nblk;
-    const int cl = threadIdx.x % kStatChan, lane = threadIdx.x / kStatChan, c = (blockIdx.x - n * nblk) * kStatChan + cl;
-    const int t_lo = (int)(((long)n * P) / kDMT), t_hi = (int)((min((long)(n + 1) * P, (long)M) - 1) / kDMT);
-    float2 v = make_float2(0.f, 0.f);
-    if (c < Cout) {
-#pragma unroll 4
-        for (int t = t_lo + lane; t <= t_hi; t += 32) {
-            // slot 0, or 1 in the tile that began in the sample before (the first one only)
-            const int slot = (long)t * kDMT < (long)n * P ? 1 : 0;
-            const float2 q = *reinterpret_cast<const float2 *>(part + (((long)t * 2 + slot) * Cout + c) * 2);
-            v.x += q.x; v.y += q.y;
-        }
-    }
-    red[lane][cl] = v;
-    __syncthreads();
-    for (int h = 16; h > 0; h >>= 1) {
-        if (lane < h) { red[lane][cl].x += red[lane + h][cl].x; red[lane][cl].y += red[lane + h][cl].y; }
-        __syncthreads();
-    }
-    if (lane == 0 && c < Cout) {
-        chan_stats[((long)n * Cout + c) * 2] = red[0][cl].x;
-        chan_stats[((long)n * Cout + c) * 2 + 1] = red[0][cl].y;
+        if (ol >= s.og || m >= s.M) continue;
+        const int o = wg * s.og + ol, b = m / s.P, p = m - b * s.P;
+        float v = acc[(long)ot * MT + pl];
+        if (bias) v += elem_to_f32<T>(bias[o]);
+        out[((long)b * s.Cout + o) * s.P + p] = f32_to_elem<T>(d2c_epilogue(v, s.act, s.act_scale));
     }
 }
 
@@ -865,18 +755,6 @@ int d2c_fwd_out_tile(const TiledShape &s)
 size_t d2c_fwd_split_count_bytes(const TiledShape &s) { return d2c_fwd_use_dma(s) ? 0 : d2c_wave_count_bytes(s, d2c_fwd_out_tile(s)); }
 size_t d2c_fwd_split_bytes(const TiledShape &s) { return d2c_fwd_use_dma(s) ? 0 : d2c_wave_split_bytes(s, d2c_fwd_out_tile(s)); }
 
-// The forward kernel of this shape adds the statistics of its output up while it stores: the DMA-gather kernel, per
-// position tile, see FwdArgs::stats, on samples of at least one position tile (which then meets at most two samples).
-// Behind the other kernel they are a pass over the output (d2c_channel_stats): added by its workgroups as they store, they all meet
-// at a few cache lines, in another order every time.  us per call without statistics, with such additions, with the pass: 64 -> 64
-// channels, float32, 12960 positions 62, 145, 68; 51360 183, 407, 204; bfloat16 142, 390, 157; up to 1400 positions no difference.
-bool d2c_fwd_fills_stats(const TiledShape &s) { return d2c_fwd_use_dma(s) && s.P >= kDMT; }
-size_t d2c_fwd_stats_ws(const TiledShape &s)
-{
-    if (!d2c_fwd_use_dma(s)) return 0;
-    return d2c_align_up((size_t)((s.M + kDMT - 1) / kDMT) * 2 * s.Cout * 2 * sizeof(float));
-}
-
 // Whether the forward kernel of this shape can write the sampled columns for the backward pass: on problems with
 // offsets along all three axes, wide weight groups from kColsTiles position tiles on (below that the backward kernels
 // that read the columns lose to the ones that sample again: 256 -> 256 channels on 4x15x27, 26 tiles: 0.25 -> 0.30 ms),
@@ -893,51 +771,37 @@ bool d2c_fwd_writes_columns(const TiledShape &s, int dtype)
     return d2c_fwd_use_dma(s) && tiles >= (dtype == D2C_F32 ? kColsTilesWideF32 : kColsTiles);
 }
 long d2c_columns_rows(const TiledShape &s) { return (long)((s.M + kDMT - 1) / kDMT) * kDMT; }
-// `stats` / `stats_part`: the [N][Cout][2] result and the per-tile scratch of d2c_fwd_stats_ws() bytes, or NULL.
 // `col`: where the sampled columns go (d2c_fwd_writes_columns), or NULL.
 // `outacc`: partial sums of the DMA-gather kernel's shared work items, or the d2c_fwd_split_bytes() of the other kernel
 // (the counters first, cleared), NULL where that one is not to split its steps.
 template <typename T>
 int d2c_tiled_fwd_launch(const TiledShape &s, const void *xcl, const void *off, const void *mask, const void *wp,
-                         const void *bias, void *out, float *outacc, hipStream_t st, float *stats, float *stats_part,
-                         void *col)
+                         const void *bias, void *out, float *outacc, hipStream_t st, void *col)
 {
     const int nt = d2c_fwd_out_tile(s);
     if (col && !d2c_fwd_writes_columns(s, (int)Elem<T>::DT)) col = nullptr;
     if (!d2c_fwd_use_dma(s)) return d2c_wave_launch<T>(s, nt, d2c_fwd_skips_zero_weights(s), xcl, off, mask, wp, bias, out, outacc, col, st);
     // the channels-last input is followed by a row of zeros (see forward_t)
     const unsigned zrow = (unsigned)((size_t)s.N * s.vol * s.Cin * sizeof(T));
-    FwdArgs a{s, xcl, off, mask, wp, bias, out, nullptr, zrow, 0, 0, 0, 0, 1, stats ? stats_part : nullptr, nullptr, 0};
+    FwdArgs a{s, xcl, off, mask, wp, bias, out, nullptr, zrow, 0, 0, 0, 0, 1, nullptr, 0};
     bool aux16 = false;
     if constexpr (sizeof(T) == 2) aux16 = s.adt == D2C_BF16;
     if (col) {
         a.col = col;
         a.col_rows = d2c_columns_rows(s);
     }
-    if (a.stats && nt != 512) {
-        // (the 256-channel tile has two wavefronts per channel, which add into their slots)
-        D2cProfScope prof(D2C_PROF_PACK, st);
-        d2c_fill_zero(a.stats, d2c_fwd_stats_ws(s), st);
-    }
-    int rc = 0;
     if (nt == 512) {
         if constexpr (sizeof(T) == 2) {
-            if (aux16) rc = launch_fwd_dma<T, true, 8, 1>(a, outacc, st);
+            if (aux16) return launch_fwd_dma<T, true, 8, 1>(a, outacc, st);
         }
-        if (!aux16) rc = launch_fwd_dma<T, false, 8, 1>(a, outacc, st);
-    } else {
-        if constexpr (sizeof(T) == 2) {
-            if (aux16) rc = launch_fwd_dma<T, true, 4, 2>(a, outacc, st);
-        }
-        if (!aux16) rc = launch_fwd_dma<T, false, 4, 2>(a, outacc, st);
+        return launch_fwd_dma<T, false, 8, 1>(a, outacc, st);
     }
-    if (rc || !a.stats) return rc;
-    D2cProfScope prof(D2C_PROF_PACK, st);
-    hipLaunchKernelGGL(stats_reduce_kernel, dim3((unsigned)(s.N * ((s.Cout + kStatChan - 1) / kStatChan))), dim3(256), 0, st, a.stats,
-                       stats, s.N, s.Cout, s.P, s.M);
-    return d2c_check_launch("stats_reduce_kernel");
+    if constexpr (sizeof(T) == 2) {
+        if (aux16) return launch_fwd_dma<T, true, 4, 2>(a, outacc, st);
+    }
+    return launch_fwd_dma<T, false, 4, 2>(a, outacc, st);
 }
 template int d2c_tiled_fwd_launch<bf16_t>(const TiledShape &, const void *, const void *, const void *, const void *,
-                                          const void *, void *, float *, hipStream_t, float *, float *, void *);
+                                          const void *, void *, float *, hipStream_t, void *);
 template int d2c_tiled_fwd_launch<float>(const TiledShape &, const void *, const void *, const void *, const void *,
-                                         const void *, void *, float *, hipStream_t, float *, float *, void *);
+                                         const void *, void *, float *, hipStream_t, void *);

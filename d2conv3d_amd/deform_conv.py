@@ -84,8 +84,7 @@ def deform_conv3d(input, offset, alpha, weight, bias=None, stride=(1, 1, 1), pad
     """deform_conv.py:42-85.  `output_relu` (not in the reference): None, or the scale s of an activation
     s * relu(.) that is applied to the output inside the forward kernels (1.0 for nn.ReLU, 1.71285855 for the
     ScaledReLU of network/layers.py:409-419).  `output_stats` (not in the reference): also return the float32
-    [N, Cout, 2] sums and sums of squares of the output per (sample, channel), which the forward kernels add up
-    while they store it -- what the GroupNorm behind the convolution needs (network/modules/refinement.py:38-43).
+    [N, Cout, 2] sums and sums of squares of the output per (sample, channel), by a pass over it -- what the GroupNorm behind the convolution needs (network/modules/refinement.py:38-43).
     `offset_axes` (not in the reference): mask of the axes (1 z, 2 y, 4 x) along which the offsets displace; the
     other offset channels are read as zero and get zero gradient, which is what the Spatial / Temporal layers do to a
     copy of the tensor (dconv_native/modules.py:87-120).  Matrix-core kernels only.

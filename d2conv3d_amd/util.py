@@ -103,9 +103,9 @@ def fuse_output_activation(module):
 
 class ConvActGroupNorm(nn.Sequential):
     """Sequential(deformable convolution, ReLU | ScaledReLU | Identity, GroupNorm) -- the `_conv` block of the
-    reference's refinement modules (network/modules/refinement.py:38-43) -- run as two kernels' worth of passes:
-    the convolution applies the activation where it stores its output and adds up the per-channel sums on the
-    way, and the normalisation is one pass over the output from those sums (no statistics pass).  Children keep
+    reference's refinement modules (network/modules/refinement.py:38-43) -- without the activation's pass: the
+    convolution applies the activation where it stores its output; one pass over the output adds up the per-channel
+    sums, and one normalises from them.  Children keep
     their places and names, so state-dict keys do not change.  CPU / float64 inputs take the plain sequence."""
 
     def forward(self, input):

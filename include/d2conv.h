@@ -164,7 +164,7 @@ size_t d2c_conv3d_backward_workspace_bytes(const d2c_conv3d_desc *desc);
  * columns there, taps x the size of the input; given less, but at least this much, the call runs on kernels that
  * need none.  On small problems this includes room for partial sums (4 MB at most), without which the call runs too, on
  * fewer workgroups (also d2c_conv3d_sized_forward with its `size_map`, else NULL, d2c_conv3d_forward_prepared, which always does, and
- * d2c_conv3d_forward_stats on descriptions whose statistics are a pass of their own). */
+ * d2c_conv3d_forward_stats). */
 size_t d2c_conv3d_forward_least_workspace_bytes(const d2c_conv3d_desc *desc, const struct d2c_size_map_desc *size_map);
 
 int d2c_conv3d_forward(const d2c_conv3d_desc *desc, const void *x, const void *offset,
@@ -425,10 +425,8 @@ int d2c_conv3d_sized_backward(const d2c_conv3d_desc *desc, const d2c_size_map_de
  * d2c_conv3d_forward_stats is d2c_conv3d_forward (sdesc == NULL, `offset` = the offsets tensor) or
  * d2c_conv3d_sized_forward (sdesc != NULL, `offset` = the raw size map) that also returns
  *     chan_stats[n][c] = (sum_p out[n,c,p], sum_p out[n,c,p]^2)        float32 [N][Cout][2],
- * of the values as stored (bias and epilogue applied, rounded to `dtype`).  The matrix-core kernels for wide
- * weight groups add these sums up where they store the output (per position tile, without atomics; a small kernel
- * adds the tiles of a sample up); other descriptions run d2c_channel_stats behind the convolution.  Workspace:
- * d2c_conv3d_forward_stats_workspace_bytes().
+ * of the values as stored (bias and epilogue applied, rounded to `dtype`): d2c_channel_stats behind the convolution, in the
+ * same call.  Workspace: d2c_conv3d_forward_stats_workspace_bytes().
  * d2c_group_norm_forward / _backward are torch.nn.functional.group_norm and its gradients (biased variance,
  * var = sumsq / m - mean^2 in float32) from such statistics: one pass over x each way plus a reduction pass for the
  * backward sums; gamma, beta (may be NULL: 1, 0) and their gradients in `dtype`. */
