@@ -406,6 +406,7 @@ struct FwdWs {
     size_t xcl, wp, outacc;
     size_t least;                   // what the gathering kernels need
     size_t gemm, lists, col, end;   // forward over sampled columns: operands of the product, sorted points, columns
+    size_t keep;                    // ... in a call that holds input, points and columns in the caller's buffer: those operands, in front
     size_t total;                   // what the call is fastest with
 };
 bool use_brick_forward(const d2c_conv3d_desc &q, const TiledShape &s, bool kept);
@@ -432,14 +433,14 @@ FwdWs fwd_ws(const d2c_conv3d_desc &q, const TiledShape &s)
     w.total = w.least + d2c_fwd_split_bytes(s);      // (the kernel of the small problems: fastest with its steps split)
     const bool plain = use_brick_forward(q, s, false), keep = use_brick_forward(q, s, true);
     if (plain || keep) {
-        // (a call that keeps its columns holds them, and the sorted points, in the caller's buffer)
         w.gemm = w.wp;
         w.lists = w.gemm + d2c_align_up(d2c_col_forward_ws(q));
         w.col = w.lists + d2c_brick_ws(s).total;
         w.end = w.col + brick_col_bytes(s);
         if (plain) w.total = std::max(w.total, w.end);
         // (where the gathering kernel writes no columns, every forward workspace has to do for a call that keeps them)
-        if (keep && !d2c_fwd_writes_columns(s, q.dtype)) w.total = std::max(w.total, w.lists);
+        w.keep = w.lists - w.gemm;
+        if (keep && !d2c_fwd_writes_columns(s, q.dtype)) w.total = std::max(w.total, w.keep);
     }
     return w;
 }
@@ -588,20 +589,21 @@ int forward_t(const d2c_conv3d_desc &q, const void *x, const void *off, const vo
         // sort the points, sample the columns (the caller's buffer, with the sorted points and the input behind them for its
         // backward call, or the workspace), multiply.  A smaller workspace: the gathering kernels, below.
         const bool keep = columns && columns_bytes >= brick_keep_bytes(s);
-        const bool fits = ws_bytes >= (keep ? l.lists : (columns ? l.col : l.end));
+        const bool fits = ws_bytes >= (keep ? l.keep : (columns ? l.col : l.end));
+        char *const gemm = base + (keep ? 0 : l.gemm);
         char *col = columns ? (char *)columns : base + l.col;
         char *lists = keep ? col + brick_col_bytes(s) : base + l.lists;
         if (keep) xcl_p = col + brick_keep_input(s);
         if (fits) {
             size_t zb;
             void *const zp = d2c_brick_zero(s, lists, &zb);
-            if (int rc = d2c_col_forward_prepare(q, x, xcl_p, w, base + l.gemm, zp, zb, st)) return rc;
+            if (int rc = d2c_col_forward_prepare(q, x, xcl_p, w, gemm, zp, zb, st)) return rc;
         }
         if (fits || keep)
             if (int rc = d2c_brick_sort(s, off, mask, lists, st, fits)) return rc;
         if (fits) {
             if (int rc = d2c_brick_columns(s, xcl_p, col, (int)d2c_columns_rows(s), lists, st)) return rc;
-            return d2c_col_forward(q, col, (int)d2c_columns_rows(s), bias, out, base + l.gemm, st);
+            return d2c_col_forward(q, col, (int)d2c_columns_rows(s), bias, out, gemm, st);
         }
     }
     // input, weights, and the counters of the steps' split (which needs its scratch: a smaller workspace goes without)
@@ -1159,9 +1161,9 @@ size_t d2c_tiled_forward_ws(const d2c_conv3d_desc &q, D2cForwardWs which)
     switch (which) {
     case D2C_FWD_WS_GATHER: return l.least + d2c_fwd_split_bytes(s);
     case D2C_FWD_WS_LEAST: return l.least;
-    case D2C_FWD_WS_KEEP: return use_brick_forward(q, s, true) ? l.lists : l.least + d2c_fwd_split_bytes(s);
+    case D2C_FWD_WS_KEEP: return use_brick_forward(q, s, true) ? l.keep : l.least + d2c_fwd_split_bytes(s);
     case D2C_FWD_WS_KEEP_LEAST:
-        return !use_brick_forward(q, s, true) ? l.least : (d2c_fwd_writes_columns(s, q.dtype) ? std::min(l.least, l.lists) : l.lists);
+        return !use_brick_forward(q, s, true) ? l.least : (d2c_fwd_writes_columns(s, q.dtype) ? std::min(l.least, l.keep) : l.keep);
     default: return l.total;
     }
 }
