@@ -1047,8 +1047,8 @@ def set_algo_override(name):
 
 
 def set_grad_weight_mode(mode):
-    """Test hook for the matrix-core kernels: "columns" (default; grad_weight as a matrix product over the sampled
-    columns that the offset / mask gradient kernel writes), "in_place" (bfloat16: the same, the columns written over
+    """Test hook for the matrix-core kernels, for calls whose backward_flags say nothing: "columns" (default; grad_weight as a
+    matrix product over sampled columns; float32 problems where that is the faster way, BWD_GW_COLUMNS for all), "in_place" (bfloat16: the same, the columns written over
     the grad-column rows: no buffer of their own, grad_input taken from the rows first; float32 problems sample
     again) or "resample" (the grad-weight kernel samples the input again)."""
     _lib.load().d2c_set_grad_weight_mode(mode if isinstance(mode, int)

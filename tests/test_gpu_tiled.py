@@ -6,6 +6,8 @@ the gradients, which are long sums).  bfloat16: the oracle consumes the
 bfloat16-rounded tensors up-cast to float32; results must agree within 2e-2
 relative (L2 over the tensor, and element-wise against the tensor's scale).
 """
+import ctypes
+
 import pytest
 import torch
 
@@ -36,7 +38,7 @@ SHAPES = {
     # work item cut into step ranges
     "c256_o320_few_tiles": (1, 256, 320, (4, 12, 16), 3, 1, 1, 1, 1, 1, True, True, 1.5),   # N*P = 768: 12 tiles
     "c512_groups2_o512_few_tiles": (2, 512, 512, (3, 8, 9), 3, 1, 1, 1, 2, 2, True, True, 1.0),   # 7 tiles x 2 groups
-    # narrow weight groups with more than 160 position tiles: the same kernel, most of its output tile empty
+    # narrow weight groups with more than 160 position tiles: the kernel whose wavefronts work alone
     "c64_o96_many_tiles": (1, 64, 96, (9, 34, 35), 3, 1, 1, 1, 1, 1, True, True, 1.5),  # N*P = 10710: ragged
     "c128_groups2_o48_many_tiles": (1, 128, 48, (8, 32, 21), 3, 1, 1, 1, 2, 2, True, False, 1.0),   # 84 tiles x 2 groups
     # the same kernel's schedule: three output tiles per position tile (399 work items on 256 compute units: one
@@ -162,20 +164,25 @@ def test_float32_grad_weight_from_columns_matches_resampling(name, dev):
     (x, off, m, w, b), gout, (s, p, d, groups, G) = make(name, torch.float32, seed=6)
     dd = lambda t: t.double() if t is not None else None
     eg = cpu.conv3d_backward(dd(gout), dd(x), dd(off), dd(m), dd(w), b is not None, s, p, d, groups, G)
+    N, Cin, D, H, W = x.shape
+    Cout, _, kd, kh, kw = w.shape
+    need = {}
+    for mode, flags in (("columns", _lib.BWD_GW_COLUMNS), ("resample", _lib.BWD_GW_RESAMPLE)):
+        desc = _lib.Conv3dDesc(N, Cin, Cout, D, H, W, kd, kh, kw, *s, *p, *d, groups, G, *off.shape[2:], _lib.D2C_F32, _lib.D2C_F32, 0, 1.0, 7, flags)
+        need[mode] = _lib.load().d2c_conv3d_backward_workspace_bytes(ctypes.byref(desc))
+    assert need["columns"] >= need["resample"] + x[0].numel() * 4 * 27      # (two ways, not one)
     before = _ops.config.keep_columns()
     _ops.config.set_keep_columns(False)
     got = {}
     try:
         for mode in ("columns", "resample"):
-            _ops.set_grad_weight_mode(mode)
             ts = [t.to(dev).requires_grad_(True) if t is not None else None for t in (x, off, m, w, b)]
-            d2c.deform_conv3d(*ts, s, p, d, groups, G).backward(gout.to(dev))
+            d2c.deform_conv3d(*ts, s, p, d, groups, G, backward_memory=mode).backward(gout.to(dev))
             got[mode] = ts[3].grad
             err = ((got[mode].double().cpu() - eg[3]).abs().max() / eg[3].abs().max()).item()
             assert err < 3e-6, (name, mode, err)
             assert rel_l2(ts[0].grad, eg[0]) < 1e-5, (name, mode, rel_l2(ts[0].grad, eg[0]))
     finally:
-        _ops.set_grad_weight_mode("columns")
         _ops.config.set_keep_columns(before["on"], before["max_bytes"])
     assert rel_l2(got["columns"], got["resample"].cpu()) < 2e-6
 
@@ -187,7 +194,6 @@ def test_wide_weight_groups_stay_on_the_list_based_backward(name, dtype, dev):
     # passes' rows are added up and the backward pass stays on the product-only kernel, and on the offset / mask gradient
     # kernel and the owner kernel (float32) or the one over bricks of sorted points that does the work of both (bfloat16;
     # the fused kernel with its atomic scatter per pass is an order of magnitude slower at layer sizes).  Which kernels ran is read from the library's own instrumentation; the values against the oracle.
-    import ctypes
     lib = _lib.load()
     (x, off, m, w, b), gout, (s, p, d, groups, G) = make(name, dtype, seed=21)
     eg = cpu.conv3d_backward(f32(gout), f32(x), off, m, f32(w), b is not None, s, p, d, groups, G)
