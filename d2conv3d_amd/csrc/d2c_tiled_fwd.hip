@@ -716,22 +716,29 @@ int launch_fwd_dma(FwdArgs a, float *outacc, hipStream_t st)
 // (32-position tiles, 128 or 64 output channels, d2c_tiled_wave.hip).  Measured on both, us per forward call, DMA first:
 //   up to 128 output channels the DMA kernel's output tile stays mostly empty.  64 -> 64, float32: 16000 positions 100,
 //   64; 51360 positions 281, 187.  128 -> 128: 171, 125; 509, 404.  256 -> 40: 319, 202; 1002, 705; bfloat16 128 -> 128:
-//   99, 75; 277, 229.  But wavefronts at different steps share no fragments, and weights that the L2 of an XCD does not
-//   hold come from further away: 512 -> 128, float32 (7 MB): 634, 539; 2106, 2130.  1024 -> 128 (14 MB): 1271, 1312;
-//   4876, 5703 (and 598, 598 at 8192 positions);
+//   99, 75; 277, 229; 1024 -> 128 325, 299; 1396, 1340.  But wavefronts at different steps share no fragments, and weights that the L2
+//   of an XCD does not hold come from further away, as do rows of many channels.  Float32, 10496, 20000 and 51200 positions: 512 -> 128 (7 MB)
+//   426, 460; 807, 751; 2080, 2059.  576 -> 128 477, 529; 916, 870; 2341, 2458.  768 -> 96 (10 MB in tiles of 128) 631, 745; 1211, 1259; 3267, 3659.
+//   768 -> 64 626, 664; 1203, 1131; 3245, 3213.  1024 -> 64 800, 928; 1598, 1646; 4616, 4847.
+//   With offsets fixed along an axis the rows that are not read count less here than there: 576 -> 128, two free 463, 394; 2060, 1421; one 366, 395;
+//   1702, 1430.  1024 -> 64 777, 536; 3620, 2063; 609, 536; 2992, 1945;
 //   above 128 the wavefronts sample once per 128 output channels.  256 -> 256, float32: 5120 positions 139, 200; 8192
 //   189, 232.  With few tiles both share out steps, and the DMA kernel's pieces are too many: 512 -> 512, bfloat16, 324
 //   positions 65, 53 (float32 70, 72), 1400 positions 82, 102; below about a thousand steps over all tiles (4 tiles of 48 steps,
 //   conv1d) its pipeline is not filled either.
 constexpr int kDmaTilesNarrow = 160, kDmaTilesWide = 128, kDmaTilesLeast = 10, kDmaStepsWide = 1024, kColsTiles = 48,
               kColsStepsNarrowF32 = 2048, kColsTilesWideF32 = 20;
-constexpr size_t kDmaWeightBytes = 8u << 20;
+constexpr size_t kDmaWeightBytes = 8u << 20, kDmaRowsF32 = 27 * 1024;
 static long dma_tiles(const TiledShape &s) { return (long)((s.M + kDMT - 1) / kDMT) * s.groups; }
 bool d2c_fwd_use_dma(const TiledShape &s)
 {
     const long tiles = dma_tiles(s);
-    if (s.og <= 128)
-        return tiles >= kDmaTilesNarrow && s.og > 64 && (size_t)s.og * s.cg * s.K * (128 / s.bkc) >= kDmaWeightBytes;
+    if (s.og <= 128) {
+        const size_t rows = (size_t)s.cg * s.K;
+        if (tiles < kDmaTilesNarrow) return false;
+        if (s.bkc == 32 && s.nd == 3 && (s.axes & 7) == 7) return rows * (s.og > 64 ? 128 : 64) * 4 >= kDmaWeightBytes || rows >= kDmaRowsF32;
+        return s.og > 64 && (size_t)s.og * rows * (128 / s.bkc) >= kDmaWeightBytes;
+    }
     return tiles >= kDmaTilesWide || (tiles >= kDmaTilesLeast && tiles * s.nchunk * s.K >= kDmaStepsWide);
 }
 

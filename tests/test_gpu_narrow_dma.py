@@ -1,7 +1,6 @@
-"""The DMA-gather forward kernel on narrow weight groups: 65 to 128 output channels whose weights take 8 MB and more, on 160 tiles and more,
-most of its output tile empty.  Expected values: the same call in two halves of its output channels, which the kernel of the small
+"""The DMA-gather forward kernel on narrow weight groups: 65 to 128 output channels whose weights take 8 MB and more, or up to 128
+with 1024 input channels and 27 taps, on 160 tiles and more, most of its output tile empty.  Expected values: the same call in two halves of its output channels, which the kernel of the small
 problems serves (its own tests compare it with the oracle): sums of the same products, up to the order of their float32 additions."""
-
 import pytest
 import torch
 
@@ -11,7 +10,7 @@ from _util import rel_l2
 
 pytestmark = pytest.mark.gpu
 
-CIN, COUT, DIMS = 1024, 96, (8, 36, 37)            # 10.6 MB of weights; 166 tiles of 64 positions and 32 over
+CIN, COUT, DIMS = 960, 96, (8, 36, 37)             # 10 MB of weights; 166 tiles of 64 positions and 32 over
 
 
 def tensors(dev, K=27):
@@ -70,8 +69,15 @@ def test_inference(axes, dev):
     assert rel_l2(out, torch.cat(want, 1)) < 2e-6
 
 
-def test_weights_below_8_mb_run_on_the_other_kernel(dev):
-    ts = tensors(dev)[:5]
+@pytest.mark.parametrize("cin,cout,kernel", [(576, 128, "tiled_fwd_wave_kernel"), (608, 128, "tiled_fwd_dma_kernel"),
+                                             (992, 64, "tiled_fwd_wave_kernel"), (1024, 64, "tiled_fwd_dma_kernel")])
+def test_line_between_the_kernels(cin, cout, kernel, dev):
+    """Weights of 8 MB; 27 taps of 1024 channels."""
+    x, off, m, w, b = tensors(dev)[:5]
+    w = w.repeat(2, 2, 1, 1, 1)[:cout, :cin].contiguous()
+    x = torch.cat([x, x], 1)[:, :cin].contiguous()
     with torch.no_grad():
-        _, name = forward_kernel(lambda: d2c.deform_conv3d(*ts[:3], ts[3][:72].contiguous(), None, 1, 1, 1, 1, 1))
-    assert name == "tiled_fwd_wave_kernel"
+        out, name = forward_kernel(lambda: d2c.deform_conv3d(x, off, m, w, None, 1, 1, 1, 1, 1))
+        assert name == kernel
+        want = [d2c.deform_conv3d(x, off, m, w[h].contiguous(), None, 1, 1, 1, 1, 1) for h in (slice(0, 32), slice(32, cout))]
+    assert rel_l2(out, torch.cat(want, 1)) < 2e-6
