@@ -158,7 +158,7 @@ __global__ void __launch_bounds__(kThreads) tiled_fwd_wave_kernel(WaveArgs a)
                 const float al = (s.mact && a.mask) ? mask_act<AT>(s.mact, craw[3]) : craw[3];
                 const unsigned o0 = (unsigned)(cb * s.vol + (t.z0 * s.H + t.y0) * s.W + t.x0) * dx;
                 unsigned read = t.live;
-                if (a.skip_zero)
+                if (__builtin_expect(a.skip_zero, 0))
                     read &= (t.hz > 0.f ? 0xFFu : 0x0Fu) & (t.hy > 0.f ? 0xFFu : 0x33u) & (t.hx > 0.f ? 0xFFu : 0x55u) & (al != 0.f ? 0xFFu : 0u);
 #pragma unroll
                 for (int c = 0; c < 8; c++) {
