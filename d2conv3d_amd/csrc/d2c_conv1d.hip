@@ -1,4 +1,5 @@
-// Backward pass of small problems of the 1-D operator: three launches, everything read in the layout it has.
+// Backward pass of small problems of the 1-D operator: three launches (bfloat16: a fourth converts the sums), everything read in the
+// layout it has.
 //
 //   grad-column product, its uses, columns      conv1d_data_kernel
 //     gcol[c, pos] = sum_o W[o, c, k] * gout[o, pos]                               (dconv1d_gpu.cu:392-397)

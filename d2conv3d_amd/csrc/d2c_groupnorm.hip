@@ -1,7 +1,6 @@
 // Normalisation behind the convolution: the GroupNorm that follows every deformable convolution + activation of the
-// reference's refinement modules (network/modules/refinement.py:38-43), from per-channel statistics that the
-// forward kernels of the convolution add up while they store the output (FwdArgs::stats, d2c_tiled_fwd.hip), so
-// that the statistics pass over the output is not needed.
+// reference's refinement modules (network/modules/refinement.py:38-43), from per-channel statistics of the
+// convolution's output, made by a pass over it.
 //
 //   chan_stats[n][c] = (sum_p x[n,c,p], sum_p x[n,c,p]^2)                       fp32, per (sample, channel)
 //   group g of sample n:  mean = sum / m,  var = sumsq / m - mean^2,  m = (C / groups) * P    (biased, as torch)

@@ -1,6 +1,6 @@
 """The activation fused into the forward kernels' store (descriptor fields `epilogue`, `epilogue_scale`): every
-kernel family that writes the output -- direct, register-gather matrix-core (with and without shared-out steps),
-DMA-gather matrix-core incl. its shared-out last round, channel-separated -- against the unfused operator followed
+kernel family that writes the output -- direct, the matrix-core kernel of small problems (whose workgroups share out a tile's
+steps), DMA-gather matrix-core incl. its shared-out last round, channel-separated -- against the unfused operator followed
 by torch's relu, forward and all gradients; and the module-level folding of (D2Conv, ReLU | ScaledReLU) pairs, the
 `_conv` blocks of network/modules/refinement.py:38-43."""
 import ctypes
@@ -18,7 +18,7 @@ pytestmark = pytest.mark.gpu
 
 CASES = [
     # shape, forced family (None: the default choice), expected family
-    ("c64_g1", None, "mfma"),                    # few tiles: steps shared out, fp32 tiles finished by a second kernel
+    ("c64_g1", None, "mfma"),                    # few tiles: steps shared out, the last workgroup of a tile adds up
     ("c64_tail", None, "mfma"),
     ("c128_groups2", None, "mfma"),
     ("c64_o320_big", None, "mfma"),              # DMA-gather kernel, 512-wide tiles, ragged last tile

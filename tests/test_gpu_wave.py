@@ -1,6 +1,6 @@
 """The forward kernel of small problems (csrc/d2c_tiled_wave.hip), whose wavefronts and workgroups share out the steps of a
 tile of 32 positions, at the sizes where that can go wrong: tiles of one position and one past a tile's edge, fewer steps
-than wavefronts, output channels around its tiles of 64 and 128, several weight groups, statistics, columns.
+than wavefronts, output channels around its tiles of 64 and 128, several weight groups, statistics of its output, columns.
 
 Expected values: the CPU oracle, to the tolerances of test_gpu_tiled.py.  The partial sums are added in a fixed order, so
 repeated calls give the same bits; a sum of all products over `terms` in another order differs by about
