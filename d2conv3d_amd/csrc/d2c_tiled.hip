@@ -741,22 +741,23 @@ BwdSlices bwd_slices(const d2c_conv3d_desc &q, const TiledShape &s)
 }
 
 // Whether a backward call runs on the bricks: not one slice by slice, and not one that writes its columns over the rows.
-// `saved_columns`: the caller brings the sampled columns of the forward call (no column region, no slices)
-bool brick_backward(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns)
+// `saved_columns`: the caller brings the sampled columns of the forward call (no column region, no slices).  `col_weight`: the call
+// would multiply over columns of its own if there were any (it wants grad_weight, and grad_offset or grad_mask)
+bool brick_backward(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns, bool col_weight = true)
 {
     if (!use_brick(q, s)) return false;
     if (saved_columns) return true;
     // (float32 columns come from the gathering kernel)
-    return gw_mode(q) != 2 && bwd_slices(q, s).gs == 0 && !(q.dtype == D2C_F32 && use_col_weight(q, s));
+    return gw_mode(q) != 2 && bwd_slices(q, s).gs == 0 && !(q.dtype == D2C_F32 && col_weight && use_col_weight(q, s));
 }
 
 struct BwdWs {
     size_t xcl, wt, gxcl, gwacc, goutp, auxacc, gcol, counts, entries, ovf, gsacc, sm1, brick, res, gemm, col, total;
 };
 // `sorted`: ... and the sorted points and the input behind them
-BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns = false, bool sorted = false)
+BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns = false, bool sorted = false, bool col_weight = true)
 {
-    const bool brick = brick_backward(q, s, saved_columns);
+    const bool brick = brick_backward(q, s, saved_columns, col_weight);
     const size_t es = d2c_elem_size(q.dtype);
     BwdWs w;
     w.xcl = 0;
@@ -801,7 +802,7 @@ BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns =
     w.gemm = w.total;      // operands of the grad-column product
     if (brick && d2c_grad_col_supported(q)) w.total += d2c_grad_col_ws(q);
     w.col = w.total;       // sampled columns for the grad-weight product
-    if (!saved_columns && use_col_weight(q, s) && !col_in_place(q, s))
+    if (!saved_columns && col_weight && use_col_weight(q, s) && !col_in_place(q, s))
         w.total += d2c_align_up(d2c_bwd_col_bytes(s, q.dtype, sl.cgs ? sl.cgs * (s.cpg / 64) : 0));
     return w;
 }
@@ -848,8 +849,9 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
     }
     // (kept columns of a forward call over sorted points: those follow the columns)
     const bool sorted = columns && use_brick_forward(q, s, true) && columns_bytes >= brick_keep_bytes(s);
-    const bool brick = nd == 3 && brick_backward(q, s, columns != nullptr);
-    const BwdWs l = bwd_ws(q, s, columns != nullptr, sorted);
+    const bool col_weight = gw && (goff || gmask);
+    const bool brick = nd == 3 && brick_backward(q, s, columns != nullptr, col_weight);
+    const BwdWs l = bwd_ws(q, s, columns != nullptr, sorted, col_weight);
     const PreparedLayout pl = prepared_layout(q, s);
     // (a forward call over sorted points has left the input behind them)
     const bool have_x = (prep && (prep->reuse & D2C_REUSE_INPUT)) || (sorted && !prep);
@@ -1171,7 +1173,10 @@ size_t d2c_tiled_forward_ws(const d2c_conv3d_desc &q, D2cForwardWs which)
 size_t d2c_tiled_backward_ws(const d2c_conv3d_desc &q, const d2c_size_map_desc *sz, bool saved_columns, bool keep)
 {
     const TiledShape s = tiled_shape(q, 3, 0, sz);
-    return is_depthwise(q) ? dw_ws(q, s).total_bwd : bwd_ws(q, s, saved_columns, keep && use_brick_forward(q, s, true)).total;
+    if (is_depthwise(q)) return dw_ws(q, s).total_bwd;
+    // (which gradients a call wants is not known here)
+    const bool sorted = keep && use_brick_forward(q, s, true);
+    return std::max(bwd_ws(q, s, saved_columns, sorted, true).total, bwd_ws(q, s, saved_columns, sorted, false).total);
 }
 
 // Bytes of the sampled columns that a forward call can keep for the backward call of the same step:

@@ -42,3 +42,34 @@ def test_default_of_float32_problems_without_kept_columns(cin, cout, G, dims, co
                 assert rel_l2(t.grad, e) < 1e-5, kw
     finally:
         _ops.config.set_keep_columns(before["on"], before["max_bytes"])
+
+
+@pytest.mark.parametrize("wanted", ["all", "x+offset", "x+w", "w+offset"])
+def test_calls_that_want_no_such_product_run_over_sorted_points(wanted, dev):
+    """On the columns' side of the line: without grad_weight, or without grad_offset and grad_mask, nobody multiplies over columns."""
+    cin, cout, G, dims = 512, 128, 8, (2, 3, 103)
+    g = torch.Generator().manual_seed(8)
+    rn = lambda *s: torch.randn(*s, generator=g)
+    x, w, off = rn(1, cin, *dims), rn(cout, cin, 3, 3, 3) / (cin * 27) ** 0.5, rn(1, G * 81, *dims) * 1.5
+    m, gout = torch.sigmoid(rn(1, G * 27, *dims)), rn(1, cout, *dims)
+    eg = cpu.conv3d_backward(gout, x, off, m, w, False, 1, 1, 1, 1, G)
+    need = {"all": (1, 1, 1, 1), "x+offset": (1, 1, 0, 0), "x+w": (1, 0, 0, 1), "w+offset": (0, 1, 0, 1)}[wanted]
+    lib = _lib.load()
+    before = _ops.config.keep_columns()
+    _ops.config.set_keep_columns(False)
+    try:
+        ts = [t.to(dev).requires_grad_(bool(n)) for t, n in zip((x, off, m, w), need)]
+        out = d2c.deform_conv3d(*ts, None, 1, 1, 1, 1, G)
+        lib.d2c_profile_reset()
+        lib.d2c_profile_enable(1)
+        out.backward(gout.to(dev))
+        torch.cuda.synchronize()
+    finally:
+        lib.d2c_profile_enable(0)
+        _ops.config.set_keep_columns(before["on"], before["max_bytes"])
+    name = lib.d2c_profile_kernel_name(_lib.PROF_BWD_AUX).decode()
+    lib.d2c_profile_reset()
+    assert name == ("aux_grad_kernel" if wanted in ("all", "w+offset") else "brick_grad_f32_kernel")
+    for t, n, e in zip(ts, need, eg):
+        if n:
+            assert rel_l2(t.grad, e) < 1e-5
