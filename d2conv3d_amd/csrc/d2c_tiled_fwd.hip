@@ -722,12 +722,17 @@ int launch_fwd_dma(FwdArgs a, float *outacc, hipStream_t st)
 //   768 -> 64 626, 664; 1203, 1131; 3245, 3213.  1024 -> 64 800, 928; 1598, 1646; 4616, 4847.
 //   With offsets fixed along an axis the rows that are not read count less here than there: 576 -> 128, two free 463, 394; 2060, 1421; one 366, 395;
 //   1702, 1430.  1024 -> 64 777, 536; 3620, 2063; 609, 536; 2992, 1945;
+//   bfloat16 with one axis free has few rows to fetch, and coordinates and weights, which the DMA kernel takes once for all output channels,
+//   decide.  12960, 20736, 25600 and 51360 positions (203, 324, 400, 803 tiles): 64 -> 128 46, 47; 69, 68; 83, 88; 127, 147.  128 -> 128 70, 68; 98, 97;
+//   119, 124; 194, 212.  192 -> 96 93, 89; 126, 127; 154, 166; 261, 281.  3 taps, 128 -> 128 25, 25; 43, 37; 40, 45; 66, 73.  Up to 64 output channels they decide too,
+//   but a layer's call (modulation by a sigmoid in the sampler) is faster there: 64 -> 64 on 51360 positions, with its branch, 199, 190.  Two axes free: 128 -> 128
+//   on 51360 248, 212;
 //   above 128 the wavefronts sample once per 128 output channels.  256 -> 256, float32: 5120 positions 139, 200; 8192
 //   189, 232.  With few tiles both share out steps, and the DMA kernel's pieces are too many: 512 -> 512, bfloat16, 324
 //   positions 65, 53 (float32 70, 72), 1400 positions 82, 102; below about a thousand steps over all tiles (4 tiles of 48 steps,
 //   conv1d) its pipeline is not filled either.
-constexpr int kDmaTilesNarrow = 160, kDmaTilesWide = 128, kDmaTilesLeast = 10, kDmaStepsWide = 1024, kColsTiles = 48,
-              kColsStepsNarrowF32 = 2048, kColsTilesWideF32 = 20;
+constexpr int kDmaTilesNarrow = 160, kDmaTilesWide = 128, kDmaTilesLeast = 10, kDmaStepsWide = 1024, kDmaTilesOneAxis = 384,
+              kColsTiles = 48, kColsStepsNarrowF32 = 2048, kColsTilesWideF32 = 20;
 constexpr size_t kDmaWeightBytes = 8u << 20, kDmaRowsF32 = 27 * 1024;
 static long dma_tiles(const TiledShape &s) { return (long)((s.M + kDMT - 1) / kDMT) * s.groups; }
 bool d2c_fwd_use_dma(const TiledShape &s)
@@ -737,6 +742,7 @@ bool d2c_fwd_use_dma(const TiledShape &s)
         const size_t rows = (size_t)s.cg * s.K;
         if (tiles < kDmaTilesNarrow) return false;
         if (s.bkc == 32 && s.nd == 3 && (s.axes & 7) == 7) return rows * (s.og > 64 ? 128 : 64) * 4 >= kDmaWeightBytes || rows >= kDmaRowsF32;
+        if (s.bkc == 64 && s.nd == 3 && __builtin_popcount(s.axes & 7) == 1 && s.og > 64 && tiles >= kDmaTilesOneAxis) return true;
         return s.og > 64 && (size_t)s.og * rows * (128 / s.bkc) >= kDmaWeightBytes;
     }
     return tiles >= kDmaTilesWide || (tiles >= kDmaTilesLeast && tiles * s.nchunk * s.K >= kDmaStepsWide);
