@@ -730,9 +730,12 @@ int launch_fwd_dma(FwdArgs a, float *outacc, hipStream_t st)
 //   above 128 the wavefronts sample once per 128 output channels.  256 -> 256, float32: 5120 positions 139, 200; 8192
 //   189, 232.  With few tiles both share out steps, and the DMA kernel's pieces are too many: 512 -> 512, bfloat16, 324
 //   positions 65, 53 (float32 70, 72), 1400 positions 82, 102; below about a thousand steps over all tiles (4 tiles of 48 steps,
-//   conv1d) its pipeline is not filled either.
+//   conv1d) its pipeline is not filled either.  Where a tile's steps times the other kernel's samplings are many, it wins from four tiles on: 4, 6 and
+//   9 tiles, float32, 2560 and more: 1024 -> 512 88, 96; 97, 106; 117, 143.  2048 -> 512 130, 178; 151, 206; 185, 270.  512 -> 1024 88, 94; 100, 113; 119, 191.
+//   1536 -> 256 74, 80; 86, 87; 102, 108.  768 -> 512 79, 76; 82, 84; 99, 110; bfloat16 2048 -> 512 86, 96; 92, 106; 107, 140; fewer: 1024 -> 256 61, 57; 70, 62;
+//   81, 74.  512 -> 512 68, 55; 72, 60; 82, 80.  2048 -> 512, 9 taps, 78, 71; 84, 80; 94, 102; and on three tiles 512 -> 1024 81, 79.
 constexpr int kDmaTilesNarrow = 160, kDmaTilesWide = 128, kDmaTilesLeast = 10, kDmaStepsWide = 1024, kDmaTilesOneAxis = 384,
-              kColsTiles = 48, kColsStepsNarrowF32 = 2048, kColsTilesWideF32 = 20;
+              kDmaTilesFew = 4, kDmaStepsFew = 2560, kColsTiles = 48, kColsStepsNarrowF32 = 2048, kColsTilesWideF32 = 20;
 constexpr size_t kDmaWeightBytes = 8u << 20, kDmaRowsF32 = 27 * 1024;
 static long dma_tiles(const TiledShape &s) { return (long)((s.M + kDMT - 1) / kDMT) * s.groups; }
 bool d2c_fwd_use_dma(const TiledShape &s)
@@ -745,7 +748,9 @@ bool d2c_fwd_use_dma(const TiledShape &s)
         if (s.bkc == 64 && s.nd == 3 && __builtin_popcount(s.axes & 7) == 1 && s.og > 64 && tiles >= kDmaTilesOneAxis) return true;
         return s.og > 64 && (size_t)s.og * rows * (128 / s.bkc) >= kDmaWeightBytes;
     }
-    return tiles >= kDmaTilesWide || (tiles >= kDmaTilesLeast && tiles * s.nchunk * s.K >= kDmaStepsWide);
+    const long steps = (long)s.nchunk * s.K;
+    return tiles >= kDmaTilesWide || (tiles >= kDmaTilesLeast && tiles * steps >= kDmaStepsWide) ||
+           (tiles >= (long)kDmaTilesFew * s.groups && steps * ((s.og + 127) / 128) >= kDmaStepsFew);
 }
 
 // Whether an infinity in a corner of weight zero stays out of the result: in the DMA-gather kernel and over sorted points always.
