@@ -648,7 +648,8 @@ bool use_brick(const d2c_conv3d_desc &q, const TiledShape &s)
     // (float32 weight groups that take several passes of the grad-column product: from 128 positions on.  Training steps without kept
     // columns, us, lists first: 64 -> 320 channels on 50 positions 136, 129; 144 152, 129; 504 177, 147; 256 -> 512 50 239, 201; 256 293, 242;
     // 512 -> 1024 50 579, 508; 256 729, 678; with kept columns 64 -> 320 on 12960 573, 531; 512 -> 1024 5765, 5331.  Fewer than two tiles of
-    // positions stay with the lists for a test's sake, which holds them to this way; it costs them 5 - 20 %.)
+    // positions stay with the lists, which cost them 5 - 20 %: test_wide_weight_groups_stay_on_the_list_based_backward holds 50 and 75 positions
+    // to that way.)
     return d2c_gx_mode() == 1 && use_lists(q, s) && use_aux_kernel(q, s) && d2c_brick_supported(s, q.dtype) &&
            (q.dtype == D2C_BF16 || d2c_tiled_bwd_single_pass(s, q.dtype) || s.M >= 128);
 }
