@@ -720,6 +720,10 @@ int launch_fwd_dma(FwdArgs a, float *outacc, hipStream_t st)
 //   of an XCD does not hold come from further away, as do rows of many channels.  Float32, 10496, 20000 and 51200 positions: 512 -> 128 (7 MB)
 //   426, 460; 807, 751; 2080, 2059.  576 -> 128 477, 529; 916, 870; 2341, 2458.  768 -> 96 (10 MB in tiles of 128) 631, 745; 1211, 1259; 3267, 3659.
 //   768 -> 64 626, 664; 1203, 1131; 3245, 3213.  1024 -> 64 800, 928; 1598, 1646; 4616, 4847.
+//   In thin maps many taps lie outside, whose rows the other kernel leaves out and the DMA kernel fetches as zeros.  3x3x3, 1, 2, 3 and 4 planes:
+//   768 -> 96 1112, 775; 1130, 791; 2200, 1490; 1159, 970.  1024 -> 128 1491, 1030; 1524, 1068; 3032, 2148; 1564, 1347.  2048 -> 64 2918, 1628; 3011, 1826; 1606, 1289;
+//   3126, 2936.  2048 -> 128 2938, 2086; 3112, 2258; 1656, 1479; 3213, 3397.  8, 16 and 32 planes: 768 -> 96 661, 733; 649, 701; 618, 612.  1024 -> 64 855, 928; 837, 848;
+//   795, 715.  2048 -> 64 1666, 2131; 1612, 1934; 1554, 1703.
 //   With offsets fixed along an axis the rows that are not read count less here than there: 576 -> 128, two free 463, 394; 2060, 1421; one 366, 395;
 //   1702, 1430.  1024 -> 64 777, 536; 3620, 2063; 609, 536; 2992, 1945;
 //   bfloat16 with one axis free has few rows to fetch, and coordinates and weights, which the DMA kernel takes once for all output channels,
@@ -737,14 +741,32 @@ int launch_fwd_dma(FwdArgs a, float *outacc, hipStream_t st)
 constexpr int kDmaTilesNarrow = 160, kDmaTilesWide = 128, kDmaTilesLeast = 10, kDmaStepsWide = 1024, kDmaTilesOneAxis = 384,
               kDmaTilesFew = 4, kDmaStepsFew = 2560, kColsTiles = 48, kColsStepsNarrowF32 = 2048, kColsTilesWideF32 = 20;
 constexpr size_t kDmaWeightBytes = 8u << 20, kDmaRowsF32 = 27 * 1024;
+// Share of the (position, tap) pairs along an axis whose undisplaced sampling point lies in the volume
+static double taps_inside(int n, int out, int k, int stride, int pad, int dil)
+{
+    long inside = 0;
+    for (int t = 0; t < k; t++) {
+        const int at = t * dil - pad;                     // of output position 0
+        const int lo = at < 0 ? (-at + stride - 1) / stride : 0, hi = at < n ? std::min(out, (n - 1 - at) / stride + 1) : 0;
+        inside += std::max(0, hi - lo);
+    }
+    return (double)inside / ((double)out * k);
+}
 static long dma_tiles(const TiledShape &s) { return (long)((s.M + kDMT - 1) / kDMT) * s.groups; }
 bool d2c_fwd_use_dma(const TiledShape &s)
 {
     const long tiles = dma_tiles(s);
     if (s.og <= 128) {
-        const size_t rows = (size_t)s.cg * s.K;
+        size_t rows = (size_t)s.cg * s.K;
         if (tiles < kDmaTilesNarrow) return false;
-        if (s.bkc == 32 && s.nd == 3 && (s.axes & 7) == 7) return rows * (s.og > 64 ? 128 : 64) * 4 >= kDmaWeightBytes || rows >= kDmaRowsF32;
+        if (s.bkc == 32 && s.nd == 3 && (s.axes & 7) == 7) {
+            const double in = taps_inside(s.D, s.Do, s.geo.kd, s.geo.sd, s.geo.pd, s.geo.dd) *
+                              taps_inside(s.H, s.Ho, s.geo.kh, s.geo.sh, s.geo.ph, s.geo.dh) *
+                              taps_inside(s.W, s.Wo, s.geo.kw, s.geo.sw, s.geo.pw, s.geo.dw);
+            if (in < 0.8) return false;
+            if (in < 0.85) rows = rows * 9 / 20;          // (four planes: above, the line lies between 1024 -> 128 and 2048 -> 128, short of 2048 -> 64)
+            return rows * (s.og > 64 ? 128 : 64) * 4 >= kDmaWeightBytes || rows >= kDmaRowsF32;
+        }
         if (s.bkc == 64 && s.nd == 3 && __builtin_popcount(s.axes & 7) == 1 && s.og > 64 && tiles >= kDmaTilesOneAxis) return true;
         return s.og > 64 && (size_t)s.og * rows * (128 / s.bkc) >= kDmaWeightBytes;
     }

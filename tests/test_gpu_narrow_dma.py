@@ -81,3 +81,21 @@ def test_line_between_the_kernels(cin, cout, kernel, dev):
         assert name == kernel
         want = [d2c.deform_conv3d(x, off, m, w[h].contiguous(), None, 1, 1, 1, 1, 1) for h in (slice(0, 32), slice(32, cout))]
     assert rel_l2(out, torch.cat(want, 1)) < 2e-6
+
+
+@pytest.mark.parametrize("cin,dims,kernel", [(1376, (4, 51, 52), "tiled_fwd_dma_kernel"), (1344, (4, 51, 52), "tiled_fwd_wave_kernel"),
+                                             (1376, (3, 60, 60), "tiled_fwd_wave_kernel"), (1376, (1, 102, 103), "tiled_fwd_wave_kernel")])
+def test_thin_maps(cin, dims, kernel, dev):
+    """A third of the taps of one plane, three quarters of three planes', four fifths of four planes' lie inside."""
+    g = torch.Generator(device=dev).manual_seed(4)
+    rn = lambda *s: torch.randn(*s, generator=g, device=dev)
+    x, off, m, w = rn(1, cin, *dims), rn(1, 81, *dims) * 1.5, torch.sigmoid(rn(1, 27, *dims)), rn(128, cin, 3, 3, 3) / (cin * 27) ** 0.5
+    with torch.no_grad():
+        out, name = forward_kernel(lambda: d2c.deform_conv3d(x, off, m, w, None, 1, 1, 1, 1, 1))
+        assert name == kernel
+        want = []
+        for h in (slice(0, 64), slice(64, 128)):
+            o, name = forward_kernel(lambda: d2c.deform_conv3d(x, off, m, w[h].contiguous(), None, 1, 1, 1, 1, 1))
+            assert name == "tiled_fwd_wave_kernel"
+            want.append(o)
+    assert rel_l2(out, torch.cat(want, 1)) < 2e-6
