@@ -731,6 +731,9 @@ int launch_fwd_dma(FwdArgs a, float *outacc, hipStream_t st)
 //   119, 124; 194, 212.  192 -> 96 93, 89; 126, 127; 154, 166; 261, 281.  3 taps, 128 -> 128 25, 25; 43, 37; 40, 45; 66, 73.  Up to 64 output channels they decide too,
 //   but a layer's call (modulation by a sigmoid in the sampler) is faster there: 64 -> 64 on 51360 positions, with its branch, 199, 190.  Two axes free: 128 -> 128
 //   on 51360 248, 212;
+//   A few steps leave some of the eight wavefronts of the other kernel without work.  25600, 51360 and 102720 positions: one step 64 -> 128, bfloat16, 31, 38; 51, 65;
+//   76, 113; two, float32, 35, 42; 54, 66; 78, 112; 64 -> 64 34, 33; 51, 52; 73, 84.  Three, bfloat16, 64 -> 128 37, 39; 60, 66; 93, 114; 64 -> 64 87, 90 on 102720.  Four, float32,
+//   128 -> 128 41, 46; 64, 71; 106, 130.  Six 45, 45; 73, 72; 112, 124.  Twelve 62, 62; 100, 103; 175, 189.  18 121, 101; 199, 174; 379, 318;
 //   above 128 the wavefronts sample once per 128 output channels.  256 -> 256, float32: 5120 positions 139, 200; 8192
 //   189, 232.  With few tiles both share out steps, and the DMA kernel's pieces are too many: 512 -> 512, bfloat16, 324
 //   positions 65, 53 (float32 70, 72), 1400 positions 82, 102; below about a thousand steps over all tiles (4 tiles of 48 steps,
@@ -739,6 +742,7 @@ int launch_fwd_dma(FwdArgs a, float *outacc, hipStream_t st)
 //   1536 -> 256 74, 80; 86, 87; 102, 108.  768 -> 512 79, 76; 82, 84; 99, 110; bfloat16 2048 -> 512 86, 96; 92, 106; 107, 140; fewer: 1024 -> 256 61, 57; 70, 62;
 //   81, 74.  512 -> 512 68, 55; 72, 60; 82, 80.  2048 -> 512, 9 taps, 78, 71; 84, 80; 94, 102; and on three tiles 512 -> 1024 81, 79.
 constexpr int kDmaTilesNarrow = 160, kDmaTilesWide = 128, kDmaTilesLeast = 10, kDmaStepsWide = 1024, kDmaTilesOneAxis = 384,
+              kDmaTilesShort = 384, kDmaStepsShort = 4, kDmaTilesShortLong = 1600, kDmaStepsShortLong = 12,
               kDmaTilesFew = 4, kDmaStepsFew = 2560, kColsTiles = 48, kColsStepsNarrowF32 = 2048, kColsTilesWideF32 = 20;
 constexpr size_t kDmaWeightBytes = 8u << 20, kDmaRowsF32 = 27 * 1024;
 // Share of the (position, tap) pairs along an axis whose undisplaced sampling point lies in the volume
@@ -759,6 +763,12 @@ bool d2c_fwd_use_dma(const TiledShape &s)
     if (s.og <= 128) {
         size_t rows = (size_t)s.cg * s.K;
         if (tiles < kDmaTilesNarrow) return false;
+        if (s.nd == 3 && (s.axes & 7) == 7) {
+            const long steps = (long)s.nchunk * s.K;
+            if (s.og > 64 ? (tiles >= kDmaTilesShort && steps <= kDmaStepsShort) || (tiles >= kDmaTilesShortLong && steps <= kDmaStepsShortLong)
+                          : tiles >= kDmaTilesShortLong && 2 * steps <= kDmaStepsShort)
+                return true;
+        }
         if (s.bkc == 32 && s.nd == 3 && (s.axes & 7) == 7) {
             const double in = taps_inside(s.D, s.Do, s.geo.kd, s.geo.sd, s.geo.pd, s.geo.dd) *
                               taps_inside(s.H, s.Ho, s.geo.kh, s.geo.sh, s.geo.ph, s.geo.dh) *
