@@ -662,7 +662,9 @@ int launch_fwd_dma(FwdArgs a, float *outacc, hipStream_t st)
     a.sk_otiles = a.s.ogp / NT;
     a.sk_items = a.sk_ntile * a.sk_otiles * a.s.groups;
     // The last, partial round: cut its items into the number of step ranges that is estimated to finish first
-    // (a piece costs its steps plus about two steps' time for adding its result).
+    // (a piece costs its steps plus about two steps' time for adding its result; the launches that clear the sums and store them
+    // take as long as four.  Without those counted, us: 64 -> 512 channels, float32, three taps, on 5184 positions 54 -> 35, on 19440 69 -> 63; 128 -> 512 71 -> 58,
+    // one tap; seven taps, 64 -> 256, on 6600 46 -> 38).
     // A workgroup lists at most kMaxSeg segments: very large problems get more workgroups than compute units
     // (and no cut of their last round, which is a small part of them).
     const int S = a.s.nchunk * a.s.K;
@@ -678,7 +680,7 @@ int launch_fwd_dma(FwdArgs a, float *outacc, hipStream_t st)
             const long cost = rounds * ((S + k - 1) / k + 2);
             if (cost < best) { best = cost; a.sk_cut = k; }
         }
-        if (a.sk_cut > 1 && best * 10 < (long)S * 9) a.sk_full = a.sk_items - tail; else a.sk_cut = 1;
+        if (a.sk_cut > 1 && (best + 4) * 10 < (long)S * 9) a.sk_full = a.sk_items - tail; else a.sk_cut = 1;
     }
     const int nshare = a.sk_items - a.sk_full;
     a.outacc = nshare ? outacc : nullptr;
@@ -741,9 +743,11 @@ int launch_fwd_dma(FwdArgs a, float *outacc, hipStream_t st)
 //   9 tiles, float32, 2560 and more: 1024 -> 512 88, 96; 97, 106; 117, 143.  2048 -> 512 130, 178; 151, 206; 185, 270.  512 -> 1024 88, 94; 100, 113; 119, 191.
 //   1536 -> 256 74, 80; 86, 87; 102, 108.  768 -> 512 79, 76; 82, 84; 99, 110; bfloat16 2048 -> 512 86, 96; 92, 106; 107, 140; fewer: 1024 -> 256 61, 57; 70, 62;
 //   81, 74.  512 -> 512 68, 55; 72, 60; 82, 80.  2048 -> 512, 9 taps, 78, 71; 84, 80; 94, 102; and on three tiles 512 -> 1024 81, 79.
+//   Few steps on a hundred tiles and more, that kernel samples four times and more: 64 -> 512 on 5184, 6600 and 7920 positions, float32, one tap 28, 30; 29, 38; 30, 38;
+//   three 35, 32; 36, 41; 37, 42; bfloat16 31, 29; 32, 37; 32, 37, nine 40, 42; 41, 54; 41, 62.  64 -> 320 three taps 34, 24; 35, 32; 35, 33.
 constexpr int kDmaTilesNarrow = 160, kDmaTilesWide = 128, kDmaTilesLeast = 10, kDmaStepsWide = 1024, kDmaTilesOneAxis = 384,
               kDmaTilesShort = 384, kDmaStepsShort = 4, kDmaTilesShortLong = 1600, kDmaStepsShortLong = 12,
-              kDmaTilesFew = 4, kDmaStepsFew = 2560, kColsTiles = 48, kColsStepsNarrowF32 = 2048, kColsTilesWideF32 = 20;
+              kDmaTilesFew = 4, kDmaStepsFew = 2560, kDmaTilesWidest = 100, kColsTiles = 48, kColsStepsNarrowF32 = 2048, kColsTilesWideF32 = 20;
 constexpr size_t kDmaWeightBytes = 8u << 20, kDmaRowsF32 = 27 * 1024;
 // Share of the (position, tap) pairs along an axis whose undisplaced sampling point lies in the volume
 static double taps_inside(int n, int out, int k, int stride, int pad, int dil)
@@ -781,7 +785,7 @@ bool d2c_fwd_use_dma(const TiledShape &s)
         return s.og > 64 && (size_t)s.og * rows * (128 / s.bkc) >= kDmaWeightBytes;
     }
     const long steps = (long)s.nchunk * s.K;
-    return tiles >= kDmaTilesWide || (tiles >= kDmaTilesLeast && tiles * steps >= kDmaStepsWide) ||
+    return tiles >= (s.og > 384 ? kDmaTilesWidest : kDmaTilesWide) || (tiles >= kDmaTilesLeast && tiles * steps >= kDmaStepsWide) ||
            (tiles >= (long)kDmaTilesFew * s.groups && steps * ((s.og + 127) / 128) >= kDmaStepsFew);
 }
 

@@ -43,3 +43,33 @@ def test_few_tiles(cin, cout, dims, groups, kernel, dtype, dev):
     else:
         # (interpolated values and the output are rounded to bfloat16, 2^-9 each)
         assert rel_l2(out, want) < 4e-3
+
+
+# a hundred tiles of 64 positions, few steps: above 384 output channels the one, up to 384 the other; a hundred and some where the last round of work
+# items is too short to be cut
+@pytest.mark.parametrize("cin,cout,dims,k,kernel", [(64, 512, (4, 40, 40), 3, DMA), (64, 385, (1, 81, 79), 1, DMA), (64, 385, (1, 80, 79), 1, WAVE),
+                                                    (64, 384, (4, 40, 40), 3, WAVE), (128, 520, (3, 65, 67), 3, DMA), (64, 130, (2, 68, 98), 1, DMA)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_few_steps_of_many_channels(cin, cout, dims, k, kernel, dtype, dev):
+    g = torch.Generator().manual_seed(cin + cout)
+    rn = lambda *s: torch.randn(*s, generator=g)
+    x, w, b = rn(1, cin, *dims).to(dtype), (rn(cout, cin, k, 1, 1) / (cin * k) ** 0.5).to(dtype), rn(cout).to(dtype)
+    off, m = rn(1, 3 * k, *dims) * 1.5, torch.sigmoid(rn(1, k, *dims))
+    lib = _lib.load()
+    with torch.no_grad():
+        lib.d2c_profile_reset()
+        lib.d2c_profile_enable(1)
+        try:
+            out = d2c.deform_conv3d(*(t.to(dev) for t in (x, off, m, w, b)), 1, (k // 2, 0, 0), 1, 1, 1)
+            torch.cuda.synchronize()
+        finally:
+            lib.d2c_profile_enable(0)
+        name = lib.d2c_profile_kernel_name(_lib.PROF_FWD).decode()
+        lib.d2c_profile_reset()
+    assert name == kernel
+    want = cpu.conv3d_forward(x.float(), off, m, w.float(), b.float(), (1, 1, 1), (k // 2, 0, 0), (1, 1, 1), 1, 1)
+    if dtype == torch.float32:
+        assert_close(out, want, 1e-4, 1e-5, name)
+    else:
+        # (interpolated values and the output are rounded to bfloat16, 2^-9 each)
+        assert rel_l2(out, want) < 4e-3
