@@ -736,6 +736,10 @@ int launch_fwd_dma(FwdArgs a, float *outacc, hipStream_t st)
 //   A few steps leave some of the eight wavefronts of the other kernel without work.  25600, 51360 and 102720 positions: one step 64 -> 128, bfloat16, 31, 38; 51, 65;
 //   76, 113; two, float32, 35, 42; 54, 66; 78, 112; 64 -> 64 34, 33; 51, 52; 73, 84.  Three, bfloat16, 64 -> 128 37, 39; 60, 66; 93, 114; 64 -> 64 87, 90 on 102720.  Four, float32,
 //   128 -> 128 41, 46; 64, 71; 106, 130.  Six 45, 45; 73, 72; 112, 124.  Twelve 62, 62; 100, 103; 175, 189.  18 121, 101; 199, 174; 379, 318;
+//   Offsets formed from a size map make coordinates dearer, which the chunks of a tap share.  12960, 25600 and 51360 positions, bfloat16, 64 -> 128, 9 taps 30, 36; 50, 65;
+//   84, 109; 7 28, 28; 45, 48; 78, 80; 27 55, 60; 98, 111; 158, 188.  128 -> 128 9 43, 46; 75, 84; 122, 142; 27 94, 88; 157, 162; 267, 280.  192 -> 128 27 130, 117; 211, 222; 379, 384.
+//   64 -> 64 9 29, 30; 48, 54; 80, 90; 27 54, 51; 96, 95; 154, 161; 7, a step to a wavefront, 27, 22; 43, 39; 74, 65.  128 -> 64 9 73, 73 on 25600; 27 152, 142.  Float32,
+//   64 -> 128 9 42, 44; 74, 78; 119, 132; 27 93, 83; 156, 152; 266, 260.  128 -> 128 9 68, 60; 119, 111; 195, 187.  64 -> 64 9 41, 36; 73, 66; 117, 113;
 //   above 128 the wavefronts sample once per 128 output channels.  256 -> 256, float32: 5120 positions 139, 200; 8192
 //   189, 232.  With few tiles both share out steps, and the DMA kernel's pieces are too many: 512 -> 512, bfloat16, 324
 //   positions 65, 53 (float32 70, 72), 1400 positions 82, 102; below about a thousand steps over all tiles (4 tiles of 48 steps,
@@ -771,6 +775,11 @@ bool d2c_fwd_use_dma(const TiledShape &s)
             const long steps = (long)s.nchunk * s.K;
             if (s.og > 64 ? (tiles >= kDmaTilesShort && steps <= kDmaStepsShort) || (tiles >= kDmaTilesShortLong && steps <= kDmaStepsShortLong)
                           : tiles >= kDmaTilesShortLong && 2 * steps <= kDmaStepsShort)
+                return true;
+            // (384 tiles as above)
+            if (s.ss.on && (s.bkc == 32 ? s.og > 64 && steps <= 18 && tiles >= kDmaTilesShort
+                                        : s.og > 64 ? s.nchunk == 1 || (s.nchunk == 2 && tiles >= kDmaTilesShort)
+                                                    : s.nchunk == 1 && steps > 8 && tiles >= kDmaTilesShort))
                 return true;
         }
         if (s.bkc == 32 && s.nd == 3 && (s.axes & 7) == 7) {
