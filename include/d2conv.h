@@ -162,8 +162,8 @@ size_t d2c_conv3d_forward_workspace_bytes(const d2c_conv3d_desc *desc);
 size_t d2c_conv3d_backward_workspace_bytes(const d2c_conv3d_desc *desc);
 /* d2c_conv3d_forward_workspace_bytes() is what a forward call is fastest with.  Large bfloat16 problems hold their sampled
  * columns there, taps x the size of the input; given less, but at least this much, the call runs on kernels that
- * need none.  On small problems this includes room for partial sums (4 MB at most), without which the call runs too, on
- * fewer workgroups (also d2c_conv3d_sized_forward with its `size_map`, else NULL, d2c_conv3d_forward_prepared, which always does, and
+ * need none.  On small problems with up to 128 output channels to a weight group, and the smallest with more, this includes room for partial
+ * sums (4 MB at most), without which the call runs too, on fewer workgroups (also d2c_conv3d_sized_forward with its `size_map`, else NULL, d2c_conv3d_forward_prepared, which always does, and
  * d2c_conv3d_forward_stats). */
 size_t d2c_conv3d_forward_least_workspace_bytes(const d2c_conv3d_desc *desc, const struct d2c_size_map_desc *size_map);
 
