@@ -317,22 +317,14 @@ Conv1dWs conv1d_ws(const TiledShape &s, int dtype)
 }  // namespace
 
 // Small problems: few (32 positions, 32 channels, tap) items of the first kernel, whose operands nobody shares; the others
-// run on the kernels of d2c_tiled_bwd.hip, whose time starts high, with every tap of every input channel, and once more for every 256
-// output channels in float32.  us per forward + backward call of 3 taps, those first here (Cin -> Cout, items):
-//   bfloat16, and float32 below 256 output channels: 512 -> 64 1968 119, 179; 4992 274, 216    256 -> 192 1992 136, 156; 3480 230, 198
-//     bfloat16 256 -> 512 1992 157, 168; 3480 277, 180    1024 -> 512 1920 151, 216; 3456 248, 238
-//   float32, one pass: 512 -> 256 1968 142, 201; 3456 256, 243    1024 -> 256 4992 335, 358; 6912 443, 391    2048 -> 256 8832 487, 599; 11904 640, 644
-//   two: 256 -> 512 4992 423, 454; 6984 599, 600; 9000 692, 654    512 -> 384 3456 297, 308; 4992 401, 401; 6960 542, 499
-//     768 -> 512 4968 418, 445; 6984 567, 562; 9000 693, 522    1024 -> 512 8928 644, 693; 12000 842, 629
-//   four: 512 -> 1024 8976 981, 1307; 12000 1206, 1091    2048 -> 1024 8832 950, 1310    256 -> 1024 9000 1060, 1202; 12000 1390, 1349
+// run on the kernels of d2c_tiled_bwd.hip.  us per forward + backward call, those first (N x Cin -> Cout, positions, taps):
+//   384 items, 4 x 512 -> 512, 64, 3: float32 151, 95; bfloat16 144, 98       2016, 4 x 512 -> 512, 333, 3: 358, 220; 215, 183
+//   2350, 320 -> 192, 1500, 5: 190, 169; 152, 163                             2880, 3 x 192 -> 64, 1024, 5: 151, 180; 133, 168
+//   9600, 4 x 2048 -> 256, 400, 3: 614, 540; 345, 487                         18000, 4 x 1024 -> 512, 1500, 3: 1217, 1287; 397, 1327
 bool d2c_conv1d_bwd_use(const TiledShape &s, int dtype)
 {
-    if (s.nd != 1 || s.cg % 32 || s.cpg % 32) return false;
-    const long items = ((long)s.N * s.P + 31) / 32 * (s.Cin / 32) * s.K, passes = (s.og + 255) / 256;
-    long most = 2048;
-    if (dtype == D2C_F32 && s.og >= 256)
-        most = passes == 1 ? std::min(10240l, std::max(2048l, 5l * s.cg)) : std::min(9216l, passes * std::max(2750l, 9l * s.cg / 2));
-    return items <= most;
+    const long items = ((long)s.N * s.P + 31) / 32 * (s.Cin / 32) * s.K;
+    return s.nd == 1 && s.cg % 32 == 0 && s.cpg % 32 == 0 && items <= (dtype == D2C_F32 && s.og >= 256 ? 10240 : 2048);
 }
 size_t d2c_conv1d_bwd_ws(const TiledShape &s, int dtype) { return conv1d_ws(s, dtype).total; }
 
