@@ -321,8 +321,8 @@ Conv1dWs conv1d_ws(const TiledShape &s, int dtype)
 //   384 items, 4 x 512 -> 512, 64, 3: float32 151, 95; bfloat16 144, 98       2016, 4 x 512 -> 512, 333, 3: 358, 220; 215, 183
 //   2350, 320 -> 192, 1500, 5: 190, 169; 152, 163                             2880, 3 x 192 -> 64, 1024, 5: 151, 180; 133, 168
 //   9600, 4 x 2048 -> 256, 400, 3: 614, 540; 345, 487                         18000, 4 x 1024 -> 512, 1500, 3: 1217, 1287; 397, 1327
-// (Float32 problems of few input channels to an output channel are faster there from fewer items on -- 512 -> 256 on 4640 positions 434, 291, 512 -> 384 on 6000
-// 675, 616 -- but the grad-column product there adds up in longer chains, and on two-term operands with up to 256 output channels: grad_input
+// (Float32 problems of few input channels to an output channel are faster there from fewer items on -- 512 -> 256 on 4640 positions 291, 434 here, 512 -> 384 on 6000
+// 616, 675 -- but the grad-column product there adds up in longer chains, and on two-term operands with up to 256 output channels: grad_input
 // 4.4e-6 off float64 against 1.3e-7 here, 2.7e-7 against 1.5e-7 with more.)
 bool d2c_conv1d_bwd_use(const TiledShape &s, int dtype)
 {
