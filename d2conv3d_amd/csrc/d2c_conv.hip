@@ -130,7 +130,7 @@ struct ConvRowsArgs {
     const unsigned char *wt;          // [step][column tile][NT][KC] bfloat16, slots swizzled
     const bf16_t *bias;               // or NULL
     bf16_t *out;                      // [N][C][P], or NULL: partial sums
-    float *part;                      // [split][C][N * P]
+    float *part;                      // [split][C][N * P]; conv_wide_kernel: [piece][column / 4][row of the tile][4]
     unsigned rowb, zrow;
     int C;                            // columns that exist
     int nchunk, S;                    // KC-channel chunks per row, steps
@@ -140,6 +140,7 @@ struct ConvRowsArgs {
     int K, tap_rows;                  // taps, rows of a tap
     int act;                          // epilogue (d2c_epilogue)
     float act_scale;
+    int wide_out;                     // rows of `out` come in fours: P a multiple of four, `out` on eight bytes
 };
 
 template <int NT, int KC, bool COLS>
@@ -423,6 +424,15 @@ __global__ void __launch_bounds__(kThreads, 1) conv_wide_kernel(ConvRowsArgs a)
         v = i < OB ? lds_read16(pb + sl + i * 32 * ROWB) : lds_read16(pa + sl + (i - OB) * 32 * ROWB);
     };
 
+    // the bias of this wavefront's columns, one to a lane.  (Read here: a load between the stores at the end would wait for
+    // those in front of it.)
+    float bias_l[OB / 2];
+#pragma unroll
+    for (int i = 0; i < OB / 2; i++) {
+        const int n = ct * NT + wo * OB * 32 + i * 64 + lane;
+        bias_l[i] = a.bias && n < a.C ? bf16_to_f32(a.bias[n]) : 0.f;
+    }
+
     tap_rows();
     for (int i = 0; i < AD; i++) row_request(i, 0);
     for (int i = 0; i < BD; i++) weight_request(i, 0);
@@ -465,54 +475,102 @@ __global__ void __launch_bounds__(kThreads, 1) conv_wide_kernel(ConvRowsArgs a)
     for (int pb = 0; pb < PB; pb++) asm volatile("" : "+v"(fa[0][pb]));
     wait_vm<0>();
 
-    // results, by stores that drop what lies outside (offset kNone); how they end is one choice for all of them
+    // Results, by stores that drop what lies outside (offset kNone).  A lane holds four consecutive columns of its row in four
+    // registers: partial sums leave as they lie (16 bytes a lane); results, where rows come in fours (wide_out), after
+    // the lanes of four rows have exchanged theirs (8 bytes a lane, a column of four rows), else one by one.
+    // (256 -> 256 channels on 32x60x108, the kernel: 655 us one by one with the bias read in between, where each read waits for the
+    // stores in front of it; 638 with the bias read ahead; 618 this way.  Without sampling, 8x60x107: 127, 126, 120.)
     constexpr unsigned kNone = 0xFFFFFFF0u;
-    const int h4 = (lane >> 5) * 4, nl = ct * NT + wo * OB * 32;
-    auto finish = [&](auto MODE) INLINE {
-        constexpr int mode = decltype(MODE)::value;        // 0: partial sums, 1: results, 2: results through the epilogue
-        const auto rs = mode == 0 ? __builtin_amdgcn_make_buffer_rsrc(a.part + (long)piece * NT * kWMT, 0, NT * kWMT * 4, 0x00020000)
-                                  : __builtin_amdgcn_make_buffer_rsrc(a.out, 0, (int)((unsigned)a.C * (unsigned)M * 2u), 0x00020000);
-        unsigned at[PB];
-        const unsigned step = mode == 0 ? kWMT * 4u : (unsigned)a.map.P * 2u;
-        const int n_lo = mode == 0 ? wo * OB * 32 : nl;
-#pragma unroll
-        for (int pb = 0; pb < PB; pb++) {
-            const int mt = (wp * PB + pb) * 32 + (lane & 31), m = m0 + mt, b = fdiv(m, a.map.dP), p = m - b * a.map.P;
-            at[pb] = mode == 0 ? (unsigned)mt * 4u + (unsigned)h4 * step
-                               : (m >= M ? kNone : ((unsigned)b * a.C * a.map.P + p) * 2u + (unsigned)h4 * step);
-        }
+    const int h4 = (lane >> 5) * 4, q = lane & 3;
+    const unsigned step = (unsigned)a.map.P * 2u;
+    if (!whole) {
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc(a.part + (long)piece * NT * kWMT, 0, NT * kWMT * 4, 0x00020000);
         for_each_const([&](auto I) INLINE {
-            constexpr int ob = decltype(I)::value / 16, r = decltype(I)::value % 16;
-            const int n0 = n_lo + ob * 32 + 8 * (r >> 2) + (r & 3);
-            const bool ok = mode == 0 || n0 + h4 < a.C;
-            float bias = 0.f;
-            if (mode != 0 && a.bias) bias = bf16_to_f32(a.bias[ok ? n0 + h4 : 0]);
+            constexpr int ob = decltype(I)::value / 4, r4 = decltype(I)::value % 4;
             for_each_const([&](auto J) INLINE {
                 constexpr int pb = decltype(J)::value;
-                const unsigned o = ok && at[pb] != kNone ? at[pb] + (unsigned)n0 * step : kNone;
-                const float v = acc[ob][pb][r] + bias;
-                if constexpr (mode == 0) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rs, (int)o, 0, 0);
-                else __builtin_amdgcn_raw_buffer_store_b16((short)f32_to_bf16(mode == 2 ? d2c_epilogue(v, a.act, a.act_scale) : v), rs, (int)o, 0, 0);
+                const f32x16 &v = acc[ob][pb];
+                const u32x4_t t = {__float_as_uint(v[r4 * 4]), __float_as_uint(v[r4 * 4 + 1]), __float_as_uint(v[r4 * 4 + 2]), __float_as_uint(v[r4 * 4 + 3])};
+                const int c4 = (wo * OB + ob) * 8 + r4 * 2 + (lane >> 5), mt = (wp * PB + pb) * 32 + (lane & 31);
+                __builtin_amdgcn_raw_buffer_store_b128(t, rs, (c4 * kWMT + mt) * 16, 0, 0);
             }, std::make_integer_sequence<int, PB>{});
             __builtin_amdgcn_sched_barrier(0);
-        }, std::make_integer_sequence<int, OB * 16>{});
+        }, std::make_integer_sequence<int, OB * 4>{});
+        return;
+    }
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc(a.out, 0, (int)((unsigned)a.C * (unsigned)M * 2u), 0x00020000);
+    auto finish = [&](auto WIDE, auto ACT) INLINE {
+        constexpr bool wide = decltype(WIDE)::value, act = decltype(ACT)::value;
+        unsigned at[PB];
+#pragma unroll
+        for (int pb = 0; pb < PB; pb++) {
+            const int m = m0 + (wp * PB + pb) * 32 + (wide ? lane & 28 : lane & 31), b = fdiv(m, a.map.dP), p = m - b * a.map.P;
+            at[pb] = m >= M ? kNone : ((unsigned)b * a.C * a.map.P + p) * 2u + (unsigned)(h4 + (wide ? q : 0)) * step;
+        }
+        const unsigned sel = q & 1 ? 0x07060302u : 0x01000504u;        // the odd rows' lanes take the upper column of a pair
+        for_each_const([&](auto I) INLINE {
+            constexpr int ob = decltype(I)::value / 4, r4 = decltype(I)::value % 4, bl = (ob & 1) * 32 + 8 * r4;
+            const int n0 = ct * NT + (wo * OB + ob) * 32 + 8 * r4;
+            float bias[4], bv = bias_l[ob >> 1];
+            opaque_v(bv);
+#pragma unroll
+            for (int e = 0; e < 4; e++) bias[e] = h4 ? lane_value(bv, bl + 4 + e) : lane_value(bv, bl + e);
+            for_each_const([&](auto J) INLINE {
+                constexpr int pb = decltype(J)::value;
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    v[e] = acc[ob][pb][r4 * 4 + e];
+                    opaque_v(v[e]);                        // (from here on its own: what the four ways share is not to be made in front of them, at once)
+                    v[e] += bias[e];
+                    if constexpr (act) v[e] = d2c_epilogue(v[e], a.act, a.act_scale);
+                }
+                if constexpr (wide) {
+                    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+                    // columns (0, 1), (2, 3) of a row -> column q & 1, 2 + (q & 1) of two rows -> column q of four rows
+                    const unsigned u0 = pack_bf16x2(v[0], v[1]), u1 = pack_bf16x2(v[2], v[3]);
+                    const unsigned w0 = __builtin_amdgcn_perm(u0, (unsigned)__builtin_amdgcn_mov_dpp((int)u0, 0xB1, 0xF, 0xF, true), sel);
+                    const unsigned w1 = __builtin_amdgcn_perm(u1, (unsigned)__builtin_amdgcn_mov_dpp((int)u1, 0xB1, 0xF, 0xF, true), sel);
+                    const unsigned t = (unsigned)__builtin_amdgcn_mov_dpp((int)(q & 2 ? w0 : w1), 0x4E, 0xF, 0xF, true);
+                    const unsigned o = n0 + h4 + q < a.C && at[pb] != kNone ? at[pb] + (unsigned)n0 * step : kNone;
+                    __builtin_amdgcn_raw_buffer_store_b64(q & 2 ? u32x2{t, w1} : u32x2{w0, t}, rs, (int)o, 0, 0);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const unsigned o = n0 + h4 + e < a.C && at[pb] != kNone ? at[pb] + (unsigned)(n0 + e) * step : kNone;
+                        __builtin_amdgcn_raw_buffer_store_b16((short)f32_to_bf16(v[e]), rs, (int)o, 0, 0);
+                    }
+                }
+            }, std::make_integer_sequence<int, PB>{});
+            __builtin_amdgcn_sched_barrier(0);
+        }, std::make_integer_sequence<int, OB * 4>{});
     };
-    if (!whole) finish(std::integral_constant<int, 0>{});
-    else if (a.act == D2C_EPILOGUE_NONE) finish(std::integral_constant<int, 1>{});
-    else finish(std::integral_constant<int, 2>{});
+    const bool act = a.act != D2C_EPILOGUE_NONE;
+    if (a.wide_out) { if (act) finish(std::true_type{}, std::true_type{}); else finish(std::true_type{}, std::false_type{}); }
+    else if (act) finish(std::false_type{}, std::true_type{});
+    else finish(std::false_type{}, std::false_type{});
 }
 
-// out = bias + the partial sums of conv_wide_kernel's tiles from `nfull` on: a workgroup = a column of a tile
+// out = bias + the partial sums of conv_wide_kernel's tiles from `nfull` on ([piece][column / 4][row][4]): a workgroup = four
+// columns of a tile, a thread = a row.  (2048 -> 256 channels, 7 taps, on 8x30x54, five pieces: 21 us with a column to a
+// workgroup, 13 this way)
 __global__ void __launch_bounds__(kWMT) conv_wide_finish_kernel(ConvRowsArgs a, int NT)
 {
-    const int rest = blockIdx.x / NT, nt = blockIdx.x - rest * NT, item = a.nfull + rest, ct = item % a.nctile, tile = item / a.nctile;
-    const int n = ct * NT + nt, m = tile * kWMT + threadIdx.x;
+    const int nq = NT / 4, rest = blockIdx.x / nq, c4 = blockIdx.x - rest * nq, item = a.nfull + rest, ct = item % a.nctile, tile = item / a.nctile;
+    const int n = ct * NT + c4 * 4, m = tile * kWMT + threadIdx.x;
     if (n >= a.C || m >= a.map.N * a.map.P) return;
-    float v = a.bias ? bf16_to_f32(a.bias[n]) : 0.f;
-    const float *q = a.part + ((long)rest * a.nsplit * NT + nt) * kWMT + threadIdx.x;
-    for (int s = 0; s < a.nsplit; s++) v += q[(long)s * NT * kWMT];
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = a.bias && n + e < a.C ? bf16_to_f32(a.bias[n + e]) : 0.f;
+    const float4 *q = reinterpret_cast<const float4 *>(a.part) + ((long)rest * a.nsplit * nq + c4) * kWMT + threadIdx.x;
+    for (int s = 0; s < a.nsplit; s++) {
+        const float4 t = q[(long)s * nq * kWMT];
+        v[0] += t.x; v[1] += t.y; v[2] += t.z; v[3] += t.w;
+    }
     const int b = fdiv(m, a.map.dP), p = m - b * a.map.P;
-    a.out[((long)b * a.C + n) * a.map.P + p] = f32_to_bf16(d2c_epilogue(v, a.act, a.act_scale));
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        if (n + e < a.C) a.out[((long)b * a.C + n + e) * a.map.P + p] = f32_to_bf16(d2c_epilogue(v[e], a.act, a.act_scale));
 }
 
 // out[b][n][p] = bias[n] + the partial sums of (n, b * P + p)
@@ -1089,7 +1147,7 @@ template <int NT, bool COLS> int launch_wide(const ConvRowsArgs &a, hipStream_t 
     D2cProfScope prof(D2C_PROF_FWD, st, "conv_wide_kernel");
     const int rest = a.ntile * a.nctile - a.nfull;
     hipLaunchKernelGGL((conv_wide_kernel<NT, COLS>), dim3((unsigned)(a.nfull + rest * a.nsplit)), dim3(kThreads), 0, st, a);
-    if (rest > 0) hipLaunchKernelGGL(conv_wide_finish_kernel, dim3((unsigned)(rest * NT)), dim3(kWMT), 0, st, a, NT);
+    if (rest > 0) hipLaunchKernelGGL(conv_wide_finish_kernel, dim3((unsigned)(rest * (NT / 4))), dim3(kWMT), 0, st, a, NT);
     return d2c_check_launch("conv_wide_kernel");
 }
 
@@ -1099,7 +1157,7 @@ int run_rows(const RowsPlan &p, const RowMap &map, const void *src, unsigned row
     const bool wide = p.MT == kWMT, sums = p.nsplit > 1 && !wide;
     ConvRowsArgs a{map, (const unsigned char *)src, (const unsigned char *)wt, sums ? nullptr : (const bf16_t *)bias,
                    sums ? nullptr : (bf16_t *)out, part, rowb, zrow, C, p.nchunk, p.S, p.ntile, p.nct, p.nsplit, p.nfull,
-                   cols_K, cols_rows, act, act_scale};
+                   cols_K, cols_rows, act, act_scale, map.P % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0};
     int rc;
     if (wide)
         rc = p.NT == 256 ? (cols_K > 0 ? launch_wide<256, true>(a, st) : launch_wide<256, false>(a, st))
