@@ -287,31 +287,43 @@ __global__ void __launch_bounds__(kThreads, 2) conv_rows_kernel(ConvRowsArgs a)
     }
 }
 
+typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
+// Operands that take one LDS read, and those that take two (a transposing read brings half of the vector).
+struct TrVec { u32x2_t lo, hi; };
+template <int N> D2C_DEV void wait_lds(TrVec &a) { asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(a.lo), "+v"(a.hi) : "n"(N)); }
+D2C_DEV void landed(u32x4_t &a) { asm volatile("" : "+v"(a)); }
+D2C_DEV void landed(TrVec &a) { asm volatile("" : "+v"(a.lo), "+v"(a.hi)); }
+D2C_DEV uint4 operand_of(const u32x4_t &a) { return __builtin_bit_cast(uint4, a); }
+D2C_DEV uint4 operand_of(const TrVec &a) { return make_uint4(a.lo.x, a.lo.y, a.hi.x, a.hi.y); }
+
 // One k-group of the wide kernels below: OB x PB matrix instructions on operand set KG & 1, and between them the reads of the
 // next k-group's operands into the other set and whatever `request` has for a slot.  The reads are spread over the group (the
 // four wavefronts share the LDS)
 // and waited for one by one, in the order in which the instructions need them: weights 0, rows 0 .. PB-1, weights 1 ...
 // The last k-group of a step meets `sync` in slot kSync and reads from the next step's buffers after it.
-template <int OB, int PB, int KG, class Read, class Request, class Sync>
-D2C_DEV void wide_group(f32x16 (&acc)[OB][PB], u32x4_t (&fa)[2][PB], u32x4_t (&fb)[2][OB], Read read, Request request, Sync sync)
+template <int OB, int PB, int KG, class FB, class Read, class Request, class Sync>
+D2C_DEV void wide_group(f32x16 (&acc)[OB][PB], u32x4_t (&fa)[2][PB], FB (&fb)[2][OB], Read read, Request request, Sync sync)
 {
     constexpr int NM = OB * PB, NR = OB + PB, s = KG & 1, lo = KG == 3 ? NM * 3 / 8 : 0;
     for_each_const([&](auto I) INLINE {
         constexpr int i = decltype(I)::value, ob = i / PB, pb = i % PB;
-        constexpr int issued = i <= lo ? 0 : ((i - lo) * NR + NM - lo - 1) / (NM - lo);        // reads of this group before slot i
+        // (LDS reads that the first r operands take)
+        constexpr auto reads = [](int r) { return r + (std::is_same<FB, TrVec>::value ? (r > 0) + (r > PB + 1 ? r - PB - 1 : 0) : 0); };
+        constexpr int issued = i <= lo ? 0 : ((i - lo) * NR + NM - lo - 1) / (NM - lo);        // operands of this group before slot i
         if constexpr (KG == 3 && i == lo) sync();
         if constexpr (pb == 0 || ob == 0) {
             // the operand(s) that this instruction is the first to need
-            constexpr int need = ob == 0 ? 1 + pb : PB + ob, later = NR - 1 - need + issued;
+            constexpr int need = ob == 0 ? 1 + pb : PB + ob, later = reads(NR) - reads(need + 1) + reads(issued);
+            static_assert(later <= 15, "the counter of LDS reads");
             if constexpr (KG == 3 && i >= lo) {
-                if constexpr (pb == 0) asm volatile("" : "+v"(fb[s][ob]));
-                if constexpr (ob == 0) asm volatile("" : "+v"(fa[s][pb]));
+                if constexpr (pb == 0) landed(fb[s][ob]);
+                if constexpr (ob == 0) landed(fa[s][pb]);
             } else {
                 if constexpr (pb == 0) wait_lds<later>(fb[s][ob]);
                 if constexpr (ob == 0) wait_lds<later>(fa[s][pb]);
             }
         }
-        mma_kgroup<bf16_t, false>(acc[ob][pb], __builtin_bit_cast(uint4, fb[s][ob]), __builtin_bit_cast(uint4, fa[s][pb]));
+        mma_kgroup<bf16_t, false>(acc[ob][pb], operand_of(fb[s][ob]), operand_of(fa[s][pb]));
         constexpr int next = i < lo ? 0 : ((i + 1 - lo) * NR + NM - lo - 1) / (NM - lo);
         for_each_const([&](auto R) INLINE {
             constexpr int r = issued + decltype(R)::value;
@@ -526,14 +538,13 @@ __global__ void __launch_bounds__(kThreads, 1) conv_wide_kernel(ConvRowsArgs a)
                     if constexpr (act) v[e] = d2c_epilogue(v[e], a.act, a.act_scale);
                 }
                 if constexpr (wide) {
-                    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
                     // columns (0, 1), (2, 3) of a row -> column q & 1, 2 + (q & 1) of two rows -> column q of four rows
                     const unsigned u0 = pack_bf16x2(v[0], v[1]), u1 = pack_bf16x2(v[2], v[3]);
                     const unsigned w0 = __builtin_amdgcn_perm(u0, (unsigned)__builtin_amdgcn_mov_dpp((int)u0, 0xB1, 0xF, 0xF, true), sel);
                     const unsigned w1 = __builtin_amdgcn_perm(u1, (unsigned)__builtin_amdgcn_mov_dpp((int)u1, 0xB1, 0xF, 0xF, true), sel);
                     const unsigned t = (unsigned)__builtin_amdgcn_mov_dpp((int)(q & 2 ? w0 : w1), 0x4E, 0xF, 0xF, true);
                     const unsigned o = n0 + h4 + q < a.C && at[pb] != kNone ? at[pb] + (unsigned)n0 * step : kNone;
-                    __builtin_amdgcn_raw_buffer_store_b64(q & 2 ? u32x2{t, w1} : u32x2{w0, t}, rs, (int)o, 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b64(q & 2 ? u32x2_t{t, w1} : u32x2_t{w0, t}, rs, (int)o, 0, 0);
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
@@ -759,6 +770,206 @@ __global__ void __launch_bounds__(kThreads, 1) grad_col_kernel(GradColArgs a)
     for (int pb = 0; pb < PB; pb++) asm volatile("" : "+v"(fa[0][pb]));
     wait_vm<0>();
 }
+// ============================================================ grad_weight over sampled columns
+//   gW[o][(pair, c)] = sum_m gout[o][m] * col[pair][m][c]          (pair = chunk of 64 input channels and tap)
+// The pipeline of conv_wide_kernel once more, the reduction over positions: a workgroup = four pairs (256 columns) x OT output
+// channels over a share of the 64-position tiles, four wavefronts of 128 columns x OT / 2, one workgroup per compute unit.  A
+// step's columns (three buffers, two steps ahead: they come from device memory) are read with the transposing LDS load,
+// grad_out comes in fragment order (pack_gout_kernel; two buffers).  Bound as conv_wide_kernel: OT * 8 matrix clocks a step
+// against 64 KB of operands.  Shares of all items run side by side on an XCD, so that grad_out is read there once.
+// Every workgroup stores its sums; col_weight_finish_kernel adds them up on their way into grad_weight.  (Float atomics into one
+// accumulator, all workgroups at the end of the launch, take 40 us for the 62 MB of 256 -> 256 channels, these stores 10.)
+// The kernel it took the place of (tiled_bwd_weight_col_kernel: 512 output channels x 128 columns, with 256 channels half of its
+// wavefronts multiply nothing; kept for the calls that have no room for the sums), us, the sums brought into grad_weight included:
+// 512 -> 512 in 8 groups on 2x8x30x54 413, 332; 256 -> 256 there 146, 114; on 32x60x108 869, 619 (reading 2.9 GB of columns once takes
+// 520); 1024 -> 256 on 8x30x54 230, 192; 2048 -> 256 with 7 taps 130, 116.  Whole training steps of small problems gain too:
+// 128 -> 64 on 420 positions 104, 101; 128 -> 128 on 1400 122, 112; 512 -> 512 267, 238.
+struct ColWeightArgs {
+    const unsigned char *gp;          // [weight group][tile of 128 positions][row block of 32][k-group of 16][lane] 16 bytes
+    const unsigned char *col;         // [pair][position][64] bfloat16
+    float *part;                      // [piece][item][pair of 4][16 x 4 channels][OT][4]
+    long pair_bytes;
+    int npair, nci, otiles, nitem;    // pairs of a weight group, sets of four, tiles of OT output channels; items in all
+    int OBT, ntp;                     // row blocks and tiles of the fragments
+    int ntile, nsplit;
+};
+template <int OT>
+__global__ void __launch_bounds__(kThreads, 1) col_weight_kernel(ColWeightArgs a)
+{
+    constexpr int OB = 4, PB = OT / 64;                    // 32-blocks of a wavefront: columns, output channels
+    constexpr int ABYTES = 4 * 64 * 128, BBYTES = OT * 128;
+    constexpr int AD = 8, BD = BBYTES / 4096, NM = OB * PB;
+    __shared__ __align__(1024) unsigned char s_t[3 * ABYTES + 2 * BBYTES];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int id = xcd_swizzle(blockIdx.x, gridDim.x), piece = id / a.nitem, item = id - piece * a.nitem;
+    const int ot = item % a.otiles, set = item / a.otiles, wg = set / a.nci, ci = set - wg * a.nci;
+    const int t_lo = (int)((long)a.ntile * piece / a.nsplit), t_hi = (int)((long)a.ntile * (piece + 1) / a.nsplit);
+
+    // --- requests: a wavefront fetches the columns of a pair (past the last pair: that one again, stored in no gradient), eight
+    // rows at a time; 16-byte pieces of a row are permuted so that the transposing reads, 64 bytes of four consecutive rows,
+    // meet no bank twice
+    const int pair = min(ci * 4 + wave, a.npair - 1);
+    const unsigned char *asrc = a.col + ((long)wg * a.npair + pair) * a.pair_bytes + (long)t_lo * 8192 + (lane >> 3) * 128 +
+                                ((lane & 7) ^ ((lane >> 4) & 1) << 2) * 16;
+    int at = t_lo, bt = t_lo;                              // the tiles that the next requests belong to
+    // (after the last tile: that one again, which nothing reads)
+    auto advance_cols = [&]() { if (at + 1 < t_hi) { at++; asrc += 8192; } };
+    // ... and k-group `wave` of every row block (past the last block: that one again)
+    const unsigned char *bsrc = a.gp + (((long)wg * a.ntp + (t_lo >> 1)) * a.OBT * 8 + (t_lo & 1) * 4 + wave) * 1024 + lane * 16;
+    unsigned bo[BD];
+#pragma unroll
+    for (int i = 0; i < BD; i++) bo[i] = (unsigned)min(ot * (OT / 32) + i, a.OBT - 1) * 8192u;
+    auto advance_gout = [&]() {
+        if (bt + 1 >= t_hi) return;
+        bsrc += bt & 1 ? (long)a.OBT * 8192 - 4096 : 4096;
+        bt++;
+    };
+    unsigned char *const sa = s_t + wave * 8192, *const sb = s_t + 3 * ABYTES + wave * 1024;
+    auto col_request = [&](int i, int buf) { dma16(asrc + i * 1024, sa + buf * ABYTES + i * 1024); };
+    auto gout_request = [&](int i, int buf) { dma16(bsrc + bo[i], sb + buf * BBYTES + i * 4096); };
+
+    f32x16 acc[OB][PB];
+#pragma unroll
+    for (int ob = 0; ob < OB; ob++)
+#pragma unroll
+        for (int pb = 0; pb < PB; pb++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[ob][pb][r] = 0.f;
+    const int wo = wave & 1, wp = wave >> 1;               // halves of the columns, of the output channels
+    // transposing reads: position (lane / 32) * 8 + (lane % 16) / 4 (and four more), channel (lane / 16 % 2) * 16 + lane % 4 * 4
+    const unsigned tr = (unsigned)((lane >> 5) * 8 + ((lane & 15) >> 2)) * 128u + (unsigned)(((lane >> 4) & 1) * 32 + (lane & 3) * 8);
+    const unsigned fl = (unsigned)((lane >> 3) & 1) * 64u; // (rows 2, 3 of four: the 64-byte halves changed over)
+    const unsigned ra0 = lds_address(s_t) + wo * 16384 + tr + fl, ra1 = lds_address(s_t) + wo * 16384 + tr + (64u - fl);
+    const unsigned rb = lds_address(s_t) + 3 * ABYTES + wp * PB * 4096 + lane * 16;
+    TrVec fb[2][OB];
+    u32x4_t fa[2][PB];
+    // operand vector i of k-group KG: columns, then output channels
+    auto cols = [](auto I, auto KG, TrVec &v, unsigned p0, unsigned p1) INLINE {
+        constexpr int i = decltype(I)::value, o = (i >> 1) * 8192 + decltype(KG)::value * 2048;
+        asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v.lo) : "v"(i & 1 ? p1 : p0), "n"(o));
+        asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v.hi) : "v"(i & 1 ? p1 : p0), "n"(o + 512));
+    };
+    auto gout = [](auto I, auto KG, u32x4_t &v, unsigned p) INLINE {
+        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(p), "n"((decltype(I)::value - OB) * 4096 + decltype(KG)::value * 1024));
+    };
+
+    for (int i = 0; i < AD; i++) col_request(i, 0);
+#pragma unroll
+    for (int i = 0; i < BD; i++) gout_request(i, 0);
+    advance_cols();
+    for (int i = 0; i < AD; i++) col_request(i, 1);
+    advance_cols();
+    advance_gout();
+#pragma unroll
+    for (int i = 0; i < BD; i++) gout_request(i, 1);
+    wait_vm<AD + BD>();
+    group_barrier();
+    // (in the order of wide_group)
+    constexpr std::integral_constant<int, 0> k0{};
+    cols(k0, k0, fb[0][0], ra0, ra1);
+    for_each_const([&](auto I) INLINE { gout(std::integral_constant<int, OB + decltype(I)::value>{}, k0, fa[0][decltype(I)::value], rb); },
+                   std::make_integer_sequence<int, PB>{});
+    for_each_const([&](auto I) INLINE { cols(std::integral_constant<int, 1 + decltype(I)::value>{}, k0, fb[0][1 + decltype(I)::value], ra0, ra1); },
+                   std::make_integer_sequence<int, OB - 1>{});
+    int abuf = 0, bbuf = 0;
+    for (int t = t_lo; t < t_hi; t++) {
+        advance_gout();
+        const int a1 = abuf == 2 ? 0 : abuf + 1, a2 = a1 == 2 ? 0 : a1 + 1, b1 = bbuf ^ 1;
+        for_each_const([&](auto KG) INLINE {
+            constexpr int kg = decltype(KG)::value;
+            constexpr std::integral_constant<int, (kg + 1) & 3> nk{};
+            const unsigned ab = (kg == 3 ? a1 : abuf) * ABYTES, p0 = ra0 + ab, p1 = ra1 + ab, pb_ = rb + (kg == 3 ? b1 : bbuf) * BBYTES;
+            wide_group<OB, PB, kg>(acc, fa, fb,
+                [&](auto I, auto &v) INLINE {
+                    if constexpr (decltype(I)::value < OB) cols(I, nk, v, p0, p1);
+                    else gout(I, nk, v, pb_);
+                },
+                [&](auto I) INLINE {
+                    constexpr int i = decltype(I)::value, n = NM / (AD / 2), lo = NM * 3 / 8, g = (BD + NM - lo - 1) / (NM - lo);
+                    if constexpr ((kg == 1 || kg == 2) && i % n == 0) col_request((kg - 1) * (AD / 2) + i / n, a2);
+                    if constexpr (kg == 3 && i >= lo)
+                        for_each_const([&](auto Q) INLINE {
+                            constexpr int q = (i - lo) * g + decltype(Q)::value;
+                            if constexpr (q < BD) gout_request(q, bbuf);
+                        }, std::make_integer_sequence<int, g>{});
+                },
+                // (the columns of the step after the next one may be under way)
+                [&]() INLINE { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(AD) : "memory"); });
+        }, std::make_integer_sequence<int, 4>{});
+        advance_cols();
+        abuf = a1; bbuf = b1;
+    }
+    // (the reads and requests behind the last step)
+#pragma unroll
+    for (int ob = 0; ob < OB; ob++) wait_lds<0>(fb[0][ob]);
+#pragma unroll
+    for (int pb = 0; pb < PB; pb++) landed(fa[0][pb]);
+    wait_vm<0>();
+
+    // a lane holds four consecutive channels of its output channel
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc(a.part + (long)id * (256 * OT), 0, 256 * OT * 4, 0x00020000);
+    for_each_const([&](auto I) INLINE {
+        constexpr int ob = decltype(I)::value / 4, r4 = decltype(I)::value % 4;
+        for_each_const([&](auto J) INLINE {
+            constexpr int pb = decltype(J)::value;
+            const f32x16 &v = acc[ob][pb];
+            const u32x4_t t = {__float_as_uint(v[r4 * 4]), __float_as_uint(v[r4 * 4 + 1]), __float_as_uint(v[r4 * 4 + 2]), __float_as_uint(v[r4 * 4 + 3])};
+            const int c4 = (wo * 4 + ob) * 8 + r4 * 2 + (lane >> 5), o = (wp * PB + pb) * 32 + (lane & 31);
+            __builtin_amdgcn_raw_buffer_store_b128(t, rs, (c4 * OT + o) * 16, 0, 0);
+        }, std::make_integer_sequence<int, PB>{});
+        __builtin_amdgcn_sched_barrier(0);
+    }, std::make_integer_sequence<int, OB * 4>{});
+}
+
+// grad_weight[o][c][tap] = the sums above: a workgroup = kFinOut output channels x 16 input channels, all taps, through LDS
+constexpr int kFinOut = 8;
+struct ColWeightFinishArgs {
+    const float *part;
+    bf16_t *gw;
+    int nsplit, nitem, nci, otiles, OT, K, og, cg, nob;    // nob: sets of kFinOut output channels of a weight group
+    int wide;                                              // `gw` on 16 bytes
+};
+__global__ void __launch_bounds__(256) col_weight_finish_kernel(ColWeightFinishArgs a)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    int b = blockIdx.x;
+    const int ob = b % a.nob; b /= a.nob;
+    const int c16 = b % (a.cg / 16), wg = b / (a.cg / 16);
+    const int j = c16 >> 2, run = 16 * a.K, rs = run * 2 + 16;         // chunk; elements of a row, bytes of it in LDS
+    const int o0 = ob * kFinOut, ot = o0 / a.OT, nr = min(kFinOut, a.og - o0);
+    const float4 *const part = reinterpret_cast<const float4 *>(a.part) + (o0 - ot * a.OT);
+    const long piece = (long)a.nitem * 64 * a.OT;
+    for (int i = threadIdx.x; i < a.K * 32; i += 256) {
+        const int o = i & 7, c4 = (i >> 3) & 3, k = i >> 5, pair = j * a.K + k;
+        const float4 *q = part + ((((long)wg * a.nci + (pair >> 2)) * a.otiles + ot) * 64 + (pair & 3) * 16 + (c16 & 3) * 4 + c4) * a.OT + o;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+        for (int s = 0; s < a.nsplit; s++) {
+            const float4 t = q[s * piece];
+            v.x += t.x; v.y += t.y; v.z += t.z; v.w += t.w;
+        }
+        bf16_t *d = reinterpret_cast<bf16_t *>(smem + o * rs) + c4 * 4 * a.K + k;
+        d[0] = f32_to_bf16(v.x); d[a.K] = f32_to_bf16(v.y); d[2 * a.K] = f32_to_bf16(v.z); d[3 * a.K] = f32_to_bf16(v.w);
+    }
+    __syncthreads();
+    bf16_t *const dst = a.gw + (((long)wg * a.og + o0) * a.cg + c16 * 16) * a.K;
+    const long row = (long)a.cg * a.K;
+    if (a.wide) {
+        const int nv = run / 8;
+        for (int i = threadIdx.x; i < nr * nv; i += 256) {
+            const int r = i / nv, v = i - r * nv;
+            *reinterpret_cast<uint4 *>(dst + r * row + v * 8) = *reinterpret_cast<const uint4 *>(smem + r * rs + v * 16);
+        }
+    } else {
+        for (int i = threadIdx.x; i < nr * run; i += 256) {
+            const int r = i / run, v = i - r * run;
+            dst[r * row + v] = *reinterpret_cast<const bf16_t *>(smem + r * rs + v * 2);
+        }
+    }
+}
+
 // W[o][c][tap] -> the operand order above: a thread makes vector v of eight o of (channel, tap) e
 D2C_DEV void grad_col_weight(const bf16_t *w, uint4 *wt, int Cout, int Cin, int K, const FastDiv &dK, int S, int e, int v)
 {
@@ -1334,6 +1545,60 @@ int d2c_grad_col(const d2c_conv3d_desc &q, void *gcol, void *ws, hipStream_t st)
     D2cProfScope prof(D2C_PROF_BWD_DATA, st, "grad_col_kernel");
     hipLaunchKernelGGL(grad_col_kernel, dim3((unsigned)std::max(8, ncu / 8 * 8)), dim3(kThreads), 0, st, a);
     return d2c_check_launch("grad_col_kernel");
+}
+
+// ---- grad_weight over sampled columns, sums in `scratch`
+namespace {
+struct ColWeightPlan {
+    int OT, otiles, nci, nitem, ntile, nsplit;
+    size_t bytes;                     // of the sums; 0: not on this kernel
+};
+ColWeightPlan col_weight_plan(const TiledShape &s, size_t scratch, int ncu)
+{
+    ColWeightPlan p{};
+    p.OT = s.og > 128 ? 256 : 128;
+    p.otiles = (s.og + p.OT - 1) / p.OT;
+    p.nci = (s.nchunk * s.K + 3) / 4;
+    p.nitem = p.nci * p.otiles * s.groups;
+    p.ntile = (s.M + 63) / 64;
+    if (kFinOut * ((size_t)s.K * 32 + 16) > 64 * 1024) return p;
+    // pieces by what they cost in steps of a compute unit: rounds, each its steps and about eight more for its start and end, and
+    // the sums, written and read once more
+    double best = -1;
+    for (int n = 1; n <= 32 && n <= p.ntile; n++) {
+        const size_t bytes = (size_t)p.nitem * n * p.OT * 1024;
+        if (bytes > scratch) break;
+        const double cost = (double)(((long)p.nitem * n + ncu - 1) / ncu) * ((p.ntile + n - 1) / n + 8) + (double)p.nitem * n * p.OT / 2560;
+        if (best < 0 || cost < best) { best = cost; p.nsplit = n; p.bytes = bytes; }
+    }
+    return p;
+}
+}  // namespace
+bool d2c_col_weight_use(const TiledShape &s, size_t scratch)
+{
+    const int ncu = d2c_num_cus();
+    return ncu > 0 && col_weight_plan(s, scratch, ncu).bytes > 0;
+}
+int d2c_col_weight(const TiledShape &s, const void *goutp, const void *col, long col_rows, void *gw, void *scratch, size_t scratch_bytes,
+                   hipStream_t st)
+{
+    const int ncu = d2c_num_cus();
+    if (ncu <= 0) return D2C_ERR_LAUNCH;
+    const ColWeightPlan p = col_weight_plan(s, scratch_bytes, ncu);
+    {
+        ColWeightArgs a{(const unsigned char *)goutp, (const unsigned char *)col, (float *)scratch, col_rows * 128, s.nchunk * s.K, p.nci, p.otiles,
+                        p.nitem, (s.og + 63) / 64 * 2, (s.M + 127) / 128, p.ntile, p.nsplit};
+        D2cProfScope prof(D2C_PROF_BWD_WEIGHT, st, "col_weight_kernel");
+        const dim3 grid((unsigned)(p.nitem * p.nsplit));
+        if (p.OT == 256) hipLaunchKernelGGL(col_weight_kernel<256>, grid, dim3(kThreads), 0, st, a);
+        else hipLaunchKernelGGL(col_weight_kernel<128>, grid, dim3(kThreads), 0, st, a);
+        if (int rc = d2c_check_launch("col_weight_kernel")) return rc;
+    }
+    D2cProfScope prof(D2C_PROF_PACK, st);
+    ColWeightFinishArgs f{(const float *)scratch, (bf16_t *)gw, p.nsplit, p.nitem, p.nci, p.otiles, p.OT, s.K, s.og, s.cg,
+                          (s.og + kFinOut - 1) / kFinOut, reinterpret_cast<uintptr_t>(gw) % 16 == 0};
+    hipLaunchKernelGGL(col_weight_finish_kernel, dim3((unsigned)(s.groups * (s.cg / 16) * f.nob)), dim3(256), kFinOut * ((size_t)s.K * 32 + 16), st, f);
+    return d2c_check_launch("col_weight_finish_kernel");
 }
 
 bool d2c_plain_supported(const d2c_conv3d_desc &q) { return plain_shape_ok(q); }

@@ -14,6 +14,9 @@ size_t d2c_grad_col_ws(const d2c_conv3d_desc &q);
 int d2c_brick_bwd_prepare(const d2c_conv3d_desc &q, const void *gout, const void *w, void *col_ws, void *goutp, void *gb, void *zero0,
                           size_t zero0_bytes, void *zero1, size_t zero1_bytes, hipStream_t st);
 int d2c_grad_col(const d2c_conv3d_desc &q, void *gcol, void *ws, hipStream_t st);
+bool d2c_col_weight_use(const TiledShape &s, size_t scratch);
+int d2c_col_weight(const TiledShape &s, const void *goutp, const void *col, long col_rows, void *gw, void *scratch, size_t scratch_bytes,
+                   hipStream_t st);
 int d2c_fwd_out_tile(const TiledShape &s);
 template <typename T>
 int d2c_tiled_fwd_launch(const TiledShape &s, const void *xcl, const void *off, const void *mask, const void *wp,
@@ -897,7 +900,8 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
         s.ss.on = 2;
         off = sm1;
     }
-    bool gw_from_col = false, gw_in_place = false, gw_done = false, gw_ready = false;
+    bool gw_from_col = false, gw_in_place = false, gw_done = false, gw_ready = false, gw_wide = false;
+    const size_t rows_bytes = l.gcol ? (size_t)s.Cin * s.K * s.M * sizeof(T) : 0;
     // (`columns`: the sampled columns the forward call kept -- the offset / mask gradient kernel then writes none, the
     // grad-weight product takes these, and the settings that save workspace by other means do not apply)
     const BwdSlices sl = columns ? BwdSlices{0, 0} : bwd_slices(q, s);
@@ -990,9 +994,10 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
             if (brick && sizeof(T) == 2 && s.groups == 1) {
                 // grad_out and the weights in the orders of the products, the bias gradient, what is added into cleared
                 gw_ready = gw_from_col;
+                gw_wide = gw_ready && !gw_in_place && d2c_col_weight_use(s, rows_bytes);
                 if (int rc = d2c_brick_bwd_prepare(q, gout, w, grad_col ? base + l.gemm : nullptr, gw_ready ? base + l.goutp : nullptr, gb,
                                                    gxcl, gxcl ? (size_t)s.N * s.vol * s.Cin * sizeof(float) : 0,
-                                                   gw_ready ? base + l.gwacc : nullptr, (size_t)s.Cout * s.cg * s.K * sizeof(float), st))
+                                                   gw_ready && !gw_wide ? base + l.gwacc : nullptr, (size_t)s.Cout * s.cg * s.K * sizeof(float), st))
                     return rc;
                 gb = nullptr;
             } else if (brick && sizeof(T) == 2 && gxcl) {
@@ -1050,7 +1055,12 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
     }
     if (gw && !gw_done) {
         if (columns && d2c_bwd_weight_from_kept_col(s, q.dtype)) gw_from_col = true;   // (also when nothing else was wanted)
-        if (d2c_tiled_bwd_weight_supported(s, q.dtype)) {
+        if (gw_wide) {
+            // (its sums take the place of the grad-column rows, which are done with)
+            if (int rc = d2c_col_weight(s, base + l.goutp, columns ? columns : base + l.col, (long)((s.M + 63) / 64) * 64, gw, base + l.gcol,
+                                        rows_bytes, st))
+                return rc;
+        } else if (d2c_tiled_bwd_weight_supported(s, q.dtype)) {
             if (int rc = d2c_tiled_bwd_weight_launch<T>(s, gout, xcl_p, off, mask, base + l.goutp,
                                                        (float *)(base + l.gwacc),
                                                        gw, gw_from_col ? (columns ? (char *)columns : (gw_in_place ? base + l.gcol : base + l.col)) : nullptr,
