@@ -108,6 +108,13 @@ D2C_DEV u32x4_t lds_read16(unsigned a)
     return v;
 }
 
+template <int OFF> D2C_DEV u32x4_t lds_read16_at(unsigned a)
+{
+    u32x4_t v;
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(a), "n"(OFF));
+    return v;
+}
+
 // 16-byte slot of channel vector v of row r in an LDS tile of KC-channel rows: consecutive rows spread over all 16
 // slots of the 64 banks, so that the reads of 16 lanes, one row each, do not meet.  The copies in device memory that
 // are read as whole tiles (the weights) have it built in.
@@ -599,177 +606,195 @@ __global__ void __launch_bounds__(256) conv_rows_finish_kernel(const float *part
 
 // ============================================================ grad-column rows of the deformable operator
 //   gcol[pair][m][c] = sum_o gout[m][o] * W[o][64 j + c][tap]     (pair = chunk j of 64 input channels and tap)
-// The pipeline of conv_wide_kernel over 256 rows x 256 columns (four pairs), with a reduction of a few steps only: so a
-// workgroup goes through a run of tiles, one per compute unit in all, and the requests for the next tile's first steps are
-// under way while a tile ends.  Runs go along the columns of a row tile.  An XCD's workgroups share a range of column tiles
-// whose weights fit its L2 (cgroups ranges) and, where there are fewer than eight, a range of row tiles.  The rows of the
-// weight operand are permuted so that a lane's 16 results of a 32 x 32 block are 16 consecutive channels.  Results leave by
-// whole rows, through LDS (16 bytes a lane, 64 rows apart: twice the time for the whole kernel).  Both operands come from the
-// caches, so one step of requests ahead is enough.
-// 256 -> 256 channels on 32x60x108: 0.97 ms and 0.06 for the operands, before 1.23; writing 2.9 GB of rows takes 0.6.
+// The reduction is short (S steps of 64 output channels), the results are many.  A wavefront holds its 64 rows of grad_out in
+// registers, all output channels of them (S * 32 registers), and goes along the pairs; a workgroup = 4 wavefronts, 256 rows,
+// one per compute unit.  Only the weights go through LDS: 64 columns x 64 output channels a step, kGradBuf steps deep.
+// Each is read by four wavefronts for 64 rows each: LDS is busy half of the matrix instructions' time, and a step brings
+// 8 KB for 512 matrix clocks.  Two sets of accumulators: the results of a tile leave between the matrix instructions
+// of the next one.  Column n of the two blocks of 32 holds the channels 2n and 2n + 1, so that a lane has both in its own
+// registers and 32 lanes write a whole row, without LDS and without an exchange between lanes.
+// An XCD's workgroups share a range of pairs whose weights fit its L2 (cgroups ranges) and, where there are fewer than
+// eight, a range of row tiles; runs go along the pairs of a row tile.
+// MEASURED
 struct GradColArgs {
     const unsigned char *src;         // channels-last grad_out, rows of `rowb` bytes
-    const unsigned char *wt;          // [column tile][step][256][64] bfloat16, slots swizzled
+    const unsigned char *wt;          // [pair][step][64 columns][64] bfloat16, slots swizzled
     bf16_t *gcol;
     unsigned rowb;
-    int M, npair, S, ntile, nct, cgroups;
+    int M, npair, ntile, cgroups;
 };
+constexpr int kGradBuf = 8;
+template <int S>
 __global__ void __launch_bounds__(kThreads, 1) grad_col_kernel(GradColArgs a)
 {
-    constexpr int OB = 4, PB = 4, NT = 256;
-    constexpr int ROWB = 128, ABYTES = kWMT * ROWB, BBYTES = NT * ROWB;
-    constexpr int AD = 8, BD = BBYTES / 4096, NM = OB * PB;
-    __shared__ __align__(1024) unsigned char s_t[2 * ABYTES + 2 * BBYTES + 4 * 4096];
+    constexpr int RB = 2, CB = 2, NB = kGradBuf, WB = 8192, RQ = 2, NM = RB * CB;          // RQ: requests of a wavefront and step
+    constexpr int TS = S * 4 * NM, NST = RB * 16;                                          // matrix instructions and stores of a tile
+    // requests and stores of a wavefront between the requests for a step and the wait for it, at least: while the pipeline
+    // fills, and later
+    constexpr int kYoung = RQ * (NB - 2), kOld = kYoung + NST * (NB - 2) / S - 2, kLater = kOld < kYoung ? kYoung : (kOld > 63 ? 63 : kOld);
+    __shared__ __align__(1024) unsigned char s_t[NB * WB];
 
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, n = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int xcd = blockIdx.x & 7, j = (int)blockIdx.x >> 3, per = (int)gridDim.x >> 3, rgroups = 8 / a.cgroups;
     const int cg = xcd % a.cgroups, rg = xcd / a.cgroups;
-    const int c_lo = a.nct * cg / a.cgroups, c_hi = a.nct * (cg + 1) / a.cgroups, nc = c_hi - c_lo;
+    const int c_lo = a.npair * cg / a.cgroups, c_hi = a.npair * (cg + 1) / a.cgroups, nc = c_hi - c_lo;
     const int r_lo = a.ntile * rg / rgroups, r_hi = a.ntile * (rg + 1) / rgroups;
     const long units = (long)(r_hi - r_lo) * nc;
     const int u_lo = (int)(units * j / per), u_hi = (int)(units * (j + 1) / per);
     if (u_lo >= u_hi) return;
 
-    // --- what is requested next: a step of the rows, a step of the weights
-    const int lrow = lane >> 3;
-    int arow = r_lo + u_lo / nc, acol = c_lo + u_lo % nc, aj = 0, aleft = (u_hi - u_lo) * a.S - 1;
-    int bj = 0, bcol = acol, bleft = aleft;
-    unsigned aoff[AD];
-    const unsigned char *asrc = a.src;
-    auto row_tile = [&]() {
-#pragma unroll
-        for (int i = 0; i < AD; i++) {
-            const int rl = wave * 64 + i * 8 + lrow;       // (rows past the last one: the last one, stored nowhere)
-            aoff[i] = (unsigned)min(arow * kWMT + rl, a.M - 1) * a.rowb + (unsigned)tile_slot<64>(rl & 31, lane & 7) * 16u;
-        }
-    };
-    // (after the last step: that step again, which nothing reads)
-    auto advance_rows = [&]() {
-        if (aleft == 0) return;
-        aleft--;
-        asrc += ROWB;
-        if (++aj < a.S) return;
-        aj = 0; asrc = a.src;
-        if (++acol < c_hi) return;
-        acol = c_lo; arow++;
-        row_tile();
-    };
-    const unsigned char *bsrc = a.wt + (long)bcol * a.S * BBYTES + wave * 1024 + lane * 16;
-    auto advance_weights = [&]() {
+    // --- requests: the steps of the weights in the order in which they are wanted (after the last one: that one again, which
+    // nothing reads)
+    int row = r_lo + u_lo / nc, col = c_lo + u_lo % nc;
+    int bj = 0, bcol = col, bleft = (u_hi - u_lo) * S - 1;
+    const unsigned char *bsrc = a.wt + (long)bcol * S * WB + wave * 1024 + lane * 16;
+    auto advance = [&]() {
         if (bleft == 0) return;
         bleft--;
-        bsrc += BBYTES;
-        if (++bj < a.S) return;
+        bsrc += WB;
+        if (++bj < S) return;
         bj = 0;
         if (++bcol < c_hi) return;
         bcol = c_lo;
-        bsrc -= (long)nc * a.S * BBYTES;
+        bsrc -= (long)nc * S * WB;
     };
-    unsigned char *const sa = s_t + wave * (64 * ROWB), *const sb = s_t + 2 * ABYTES + wave * 1024;
-    auto row_request = [&](int i, int buf) { dma16(asrc + aoff[i], sa + buf * ABYTES + i * 1024); };
-    auto weight_request = [&](int i, int buf) { dma16(bsrc + i * 4096, sb + buf * BBYTES + i * 4096); };
+    auto request = [&](int i, int buf) { dma16(bsrc + i * 4096, s_t + buf * WB + wave * 1024 + i * 4096); };
 
-    f32x16 acc[OB][PB];
-    const int wo = wave & 1, wp = wave >> 1, h = lane >> 5;
+    // --- this wavefront's rows (those past the last one: the last one, stored nowhere)
+    u32x4_t x[RB][S * 4];
+    auto load_rows = [&]() {
+#pragma unroll
+        for (int rb = 0; rb < RB; rb++) {
+            const unsigned char *p = a.src + (unsigned)min(row * kWMT + wave * 64 + rb * 32 + n, a.M - 1) * (size_t)a.rowb + h * 16;
+#pragma unroll
+            for (int k = 0; k < S * 4; k++) x[rb][k] = *reinterpret_cast<const u32x4_t *>(p + k * 32);
+        }
+        // (waited for here: a wait behind the branch would be one of every tile)
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+    };
+
+    f32x16 acc[2][RB][CB];
+    u32x4_t fb[2][CB];
     unsigned slot[4];
 #pragma unroll
-    for (int kg = 0; kg < 4; kg++)
-        slot[kg] = (unsigned)((lane & 31) * ROWB + tile_slot<64>(lane & 31, kg * 2 + h) * 16);
-    const unsigned ra = lds_address(s_t) + wp * PB * 32 * ROWB, rb = lds_address(s_t) + 2 * ABYTES + wo * OB * 32 * ROWB;
-    u32x4_t fa[2][PB], fb[2][OB];
-    // operand vector i of a k-group: weights, then rows
-    auto operand = [&](auto I, u32x4_t &v, unsigned pa, unsigned pb, unsigned sl) INLINE {
-        constexpr int i = decltype(I)::value;
-        v = i < OB ? lds_read16(pb + sl + i * 32 * ROWB) : lds_read16(pa + sl + (i - OB) * 32 * ROWB);
+    for (int kg = 0; kg < 4; kg++) slot[kg] = lds_address(s_t) + (unsigned)(n * 128 + tile_slot<64>(n, kg * 2 + h) * 16);
+    // --- the tile whose results are on their way out: the first of its rows, a descriptor of it that ends with the pair's last
+    unsigned long long out_p = reinterpret_cast<unsigned long long>(a.gcol);
+    unsigned out_bytes = 0;
+    const unsigned lane_at = (unsigned)(wave * 64 + h * 4) * 128u + n * 4u;
+    auto store = [&](auto SET, auto Q, auto &rs, const unsigned (&base)[2]) INLINE {
+        constexpr int set = decltype(SET)::value, rb = decltype(Q)::value / 16, r = decltype(Q)::value % 16, at = (8 * (r >> 2) + (r & 3)) * 128;
+        __builtin_amdgcn_raw_buffer_store_b32(pack_bf16x2(acc[set][rb][0][r], acc[set][rb][1][r]), rs, (int)(base[rb] + at), 0, 2);
+    };
+    auto out_rsrc = [&]() INLINE {
+        const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)out_p), hi = __builtin_amdgcn_readfirstlane((unsigned)(out_p >> 32));
+        return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>((unsigned long long)hi << 32 | lo), 0,
+                                                 (int)__builtin_amdgcn_readfirstlane(out_bytes), 0x00020000);
     };
 
-    row_tile();
-    for (int i = 0; i < AD; i++) row_request(i, 0);
-    for (int i = 0; i < BD; i++) weight_request(i, 0);
-    advance_rows();
-    advance_weights();
-    for (int i = 0; i < AD; i++) row_request(i, 1);
-    for (int i = 0; i < BD; i++) weight_request(i, 1);
-    wait_vm<AD + BD>();
-    group_barrier();
-    // (in the order of wide_group)
-    operand(std::integral_constant<int, 0>{}, fb[0][0], ra, rb, slot[0]);
-    for_each_const([&](auto I) INLINE { operand(std::integral_constant<int, OB + decltype(I)::value>{}, fa[0][decltype(I)::value], ra, rb, slot[0]); },
-                   std::make_integer_sequence<int, PB>{});
-    for_each_const([&](auto I) INLINE { operand(std::integral_constant<int, 1 + decltype(I)::value>{}, fb[0][1 + decltype(I)::value], ra, rb, slot[0]); },
-                   std::make_integer_sequence<int, OB - 1>{});
-    // a wavefront's results on their way out: 32 rows of a pair, written by (row, half), read 8 lanes to a row
-    const unsigned stage = lds_address(s_t) + 2 * ABYTES + 2 * BBYTES + wave * 4096;
-    const unsigned ov = (lane >> 3) * 128u + (lane & 7) * 16u;
-    int buf = 0;
-    int row = r_lo + u_lo / nc, col = c_lo + u_lo % nc;
-    for (int u = u_lo; u < u_hi; u++) {
+    for (int b = 0; b < NB; b++) {
 #pragma unroll
-        for (int ob = 0; ob < OB; ob++)
-#pragma unroll
-            for (int pb = 0; pb < PB; pb++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) acc[ob][pb][r] = 0.f;
-        for (int st = 0; st < a.S; st++) {
-            advance_rows();
-            advance_weights();
-            const int nbuf = buf ^ 1;
-            auto group = [&](auto KG) INLINE {
-                constexpr int kg = decltype(KG)::value;
-                const int b = kg == 3 ? nbuf : buf;
-                const unsigned pa = ra + b * ABYTES, pb_ = rb + b * BBYTES;
-                wide_group<OB, PB, kg>(acc, fa, fb, [&](auto I, u32x4_t &v) INLINE { operand(I, v, pa, pb_, slot[(kg + 1) & 3]); },
-                    [&](auto I) INLINE {
-                        constexpr int d = decltype(I)::value - NM * 3 / 8;
-                        if constexpr (kg == 3 && d >= 0 && d < AD) { row_request(d, buf); weight_request(d, buf); }
-                    },
-                    [&]() INLINE {
-                        // (the stores of the tile before, younger than these requests, may be under way)
-                        if (st == 0 && u > u_lo) wait_vm<32>(); else wait_vm<0>();
-                        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                    });
-            };
-            for_each_const(group, std::make_integer_sequence<int, 4>{});
-            buf = nbuf;
-        }
-        // results, 32 rows of a pair at a time, by whole rows; those past the last one fall outside the pair's descriptor
-        u32x4_t v[2][4];
-        for_each_const([&](auto R) INLINE {
-            constexpr int r = decltype(R)::value;
-            if constexpr (r < 8) {
-                constexpr int pb = r & 3;
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const f32x16 &x = acc[(r >> 2) * 2 + (q >> 1)][pb];
-                    const int e = (q & 1) * 8;
-                    u32x4_t t = {pack_bf16x2(x[e], x[e + 1]), pack_bf16x2(x[e + 2], x[e + 3]), pack_bf16x2(x[e + 4], x[e + 5]), pack_bf16x2(x[e + 6], x[e + 7])};
-                    asm volatile("ds_write_b128 %0, %1" ::"v"(stage + (lane & 31) * 128u + tile_slot<64>(lane & 31, (q >> 1) * 4 + h * 2 + (q & 1)) * 16u), "v"(t));
-                }
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    v[r & 1][i] = lds_read16(stage + i * 1024 + (lane >> 3) * 128u + tile_slot<64>(i * 8 + (lane >> 3), lane & 7) * 16u);
-            }
-            if constexpr (r > 0) {
-                constexpr int o = r - 1, pb = o & 3;
-                const int pair = col * 4 + wo * 2 + (o >> 2);
-                const auto rs = __builtin_amdgcn_make_buffer_rsrc(a.gcol + (long)pair * a.M * 64, 0, pair < a.npair ? (int)((unsigned)a.M * 128u) : 0, 0x00020000);
-#pragma unroll
-                for (int i = 0; i < 4; i++) wait_lds<r < 8 ? 8 : 0>(v[o & 1][i]);
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    __builtin_amdgcn_raw_buffer_store_b128(v[o & 1][i], rs, (int)((unsigned)(row * kWMT + (wp * PB + pb) * 32 + i * 8) * 128u + ov), 0, 2);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }, std::make_integer_sequence<int, 9>{});
-        if (++col == c_hi) { col = c_lo; row++; }
+        for (int i = 0; i < RQ; i++) request(i, b);
+        advance();
     }
+    load_rows();
+    group_barrier();
 #pragma unroll
-    for (int ob = 0; ob < OB; ob++) wait_lds<0>(fb[0][ob]);
+    for (int cb = 0; cb < CB; cb++) fb[0][cb] = lds_read16(slot[0] + cb * 4096);
+    int buf = 0, done = 0;                                 // steps done, as far as it matters
+    auto tile = [&](auto SET) INLINE {
+        constexpr int set = decltype(SET)::value;
+        const auto rs = out_rsrc();
+        // (anew for every tile: what is added to these stays in the stores)
+        unsigned base[2] = {lane_at, lane_at + 4096u};
+        opaque_v(base[0]); opaque_v(base[1]);
+        for_each_const([&](auto ST) INLINE {
+            constexpr int st = decltype(ST)::value;
+            const int nbuf = buf + 1 == NB ? 0 : buf + 1;
+            for_each_const([&](auto KG) INLINE {
+                constexpr int kg = decltype(KG)::value, s = kg & 1, lo = kg == 3 ? NM * 3 / 8 : 0;
+                const unsigned p = slot[(kg + 1) & 3] + (kg == 3 ? nbuf : buf) * WB;
+                for_each_const([&](auto I) INLINE {
+                    constexpr int i = decltype(I)::value, cb = i / RB, rb = i % RB, e = (st * 4 + kg) * NM + i;
+                    constexpr int issued = i <= lo ? 0 : ((i - lo) * CB + NM - lo - 1) / (NM - lo), next = i < lo ? 0 : ((i + 1 - lo) * CB + NM - lo - 1) / (NM - lo);
+                    if constexpr (kg == 3 && i == lo) {
+                        // every wavefront holds the last operands of the step, its buffer is free; the next step's are there
+                        if (done >= NB) wait_vm<kLater>(); else wait_vm<kYoung>();
+                        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                    }
+                    if constexpr (rb == 0) {
+                        if constexpr (kg == 3 && i >= lo) landed(fb[s][cb]);
+                        else wait_lds<CB - 1 - cb + issued>(fb[s][cb]);
+                    }
+                    const bf16x8_t xv = __builtin_bit_cast(bf16x8_t, x[rb][st * 4 + kg]), wv = __builtin_bit_cast(bf16x8_t, fb[s][cb]);
+                    if constexpr (st == 0 && kg == 0) {
+                        f32x16 z;
 #pragma unroll
-    for (int pb = 0; pb < PB; pb++) asm volatile("" : "+v"(fa[0][pb]));
+                        for (int r = 0; r < 16; r++) z[r] = 0.f;
+                        acc[set][rb][cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xv, wv, z, 0, 0, 0);
+                    } else acc[set][rb][cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xv, wv, acc[set][rb][cb], 0, 0, 0);
+                    for_each_const([&](auto R) INLINE {
+                        constexpr int r = issued + decltype(R)::value;
+                        fb[s ^ 1][r] = lds_read16_at<r * 4096>(p);
+                    }, std::make_integer_sequence<int, next - issued>{});
+                    if constexpr (kg == 3 && i >= lo && i - lo < RQ) request(i - lo, buf);
+                    constexpr int q = (e * NST + TS - 1) / TS, q1 = ((e + 1) * NST + TS - 1) / TS;
+                    for_each_const([&](auto Q) INLINE { store(std::integral_constant<int, set ^ 1>{}, std::integral_constant<int, q + decltype(Q)::value>{}, rs, base); },
+                                   std::make_integer_sequence<int, q1 - q>{});
+                    __builtin_amdgcn_sched_barrier(0);
+                }, std::make_integer_sequence<int, NM>{});
+            }, std::make_integer_sequence<int, 4>{});
+            advance();
+            buf = nbuf;
+            done = min(done + 1, NB);
+        }, std::make_integer_sequence<int, S>{});
+        out_p = reinterpret_cast<unsigned long long>(a.gcol) + ((unsigned long long)col * a.M + row * kWMT) * 128;
+        out_bytes = (unsigned)(a.M - row * kWMT) * 128u;
+    };
+    auto next_tile = [&]() {
+        if (++col < c_hi) return;
+        col = c_lo; row++;
+        load_rows();
+    };
+    auto drain = [&](auto SET) INLINE {
+        const auto rs = out_rsrc();
+        const unsigned base[2] = {lane_at, lane_at + 4096u};
+        for_each_const([&](auto Q) INLINE { store(SET, Q, rs, base); __builtin_amdgcn_sched_barrier(0); }, std::make_integer_sequence<int, NST>{});
+    };
+    constexpr std::integral_constant<int, 0> k0{};
+    constexpr std::integral_constant<int, 1> k1{};
+#pragma unroll
+    for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+        for (int cb = 0; cb < CB; cb++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[1][rb][cb][r] = 0.f;
+    for (int u = u_lo;;) {
+        tile(k0);
+        if (++u == u_hi) { drain(k0); break; }
+        next_tile();
+        tile(k1);
+        if (++u == u_hi) { drain(k1); break; }
+        next_tile();
+    }
+    // (the reads and requests behind the last step)
+#pragma unroll
+    for (int cb = 0; cb < CB; cb++) wait_lds<0>(fb[0][cb]);
     wait_vm<0>();
 }
+// W[o][c][tap] -> the operand order above: a thread makes vector v of eight o of (channel, tap) e
+D2C_DEV void grad_col_weight(const bf16_t *w, uint4 *wt, int Cout, int Cin, int K, const FastDiv &dK, int S, int e, int v)
+{
+    const int CK = Cin * K;
+    if (e >= CK) return;
+    alignas(16) bf16_t t[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) t[q] = v * 8 + q < Cout ? w[(long)(v * 8 + q) * CK + e] : (bf16_t)0;
+    const int c = fdiv(e, dK), k = e - c * K, pair = (c >> 6) * K + k, ch = c & 63;
+    wt[(((long)pair * S + (v >> 3)) * 64 + (ch & 1) * 32 + (ch >> 1)) * 8 + tile_slot<64>(ch >> 1, v & 7)] = *reinterpret_cast<const uint4 *>(t);
+}
+
 // ============================================================ grad_weight over sampled columns
 //   gW[o][(pair, c)] = sum_m gout[o][m] * col[pair][m][c]          (pair = chunk of 64 input channels and tap)
 // The pipeline of conv_wide_kernel once more, the reduction over positions: a workgroup = four pairs (256 columns) x OT output
@@ -968,19 +993,6 @@ __global__ void __launch_bounds__(256) col_weight_finish_kernel(ColWeightFinishA
             dst[r * row + v] = *reinterpret_cast<const bf16_t *>(smem + r * rs + v * 2);
         }
     }
-}
-
-// W[o][c][tap] -> the operand order above: a thread makes vector v of eight o of (channel, tap) e
-D2C_DEV void grad_col_weight(const bf16_t *w, uint4 *wt, int Cout, int Cin, int K, const FastDiv &dK, int S, int e, int v)
-{
-    const int CK = Cin * K;
-    if (e >= CK) return;
-    alignas(16) bf16_t t[8];
-#pragma unroll
-    for (int q = 0; q < 8; q++) t[q] = v * 8 + q < Cout ? w[(long)(v * 8 + q) * CK + e] : (bf16_t)0;
-    const int c = fdiv(e, dK), k = e - c * K, pair = (c >> 6) * K + k, ch = c & 31;
-    const int r = (pair & 3) * 64 + (c & 32) + 8 * ((ch & 15) >> 2) + 4 * (ch >> 4) + (ch & 3);
-    wt[(((long)(pair >> 2) * S + (v >> 3)) * 256 + r) * 8 + tile_slot<64>(r & 31, v & 7)] = *reinterpret_cast<const uint4 *>(t);
 }
 
 // ============================================================ grad_weight
@@ -1483,7 +1495,7 @@ int d2c_col_forward(const d2c_conv3d_desc &q, const void *col, int rows, const v
 // ---- grad-column rows [chunk][tap][N*P][64] of the deformable operator's backward pass, one weight group
 namespace {
 struct GradColPlan {
-    int Cp, S, ntile, nct, cgroups;
+    int Cp, S, ntile, npair, cgroups;
     size_t wt_bytes, total;
 };
 GradColPlan grad_col_plan(const d2c_conv3d_desc &q)
@@ -1493,23 +1505,24 @@ GradColPlan grad_col_plan(const d2c_conv3d_desc &q)
     p.Cp = (q.Cout + 63) / 64 * 64;
     p.S = p.Cp / 64;
     p.ntile = (M + kWMT - 1) / kWMT;
-    p.nct = (q.Cin / 64 * q.kd * q.kh * q.kw + 3) / 4;
-    p.wt_bytes = d2c_align_up((size_t)p.nct * p.S * 256 * 128);
+    p.npair = q.Cin / 64 * q.kd * q.kh * q.kw;
+    p.wt_bytes = d2c_align_up((size_t)p.npair * p.S * 8192);
     p.total = p.wt_bytes + d2c_align_up((size_t)M * p.Cp * 2 + 1024);
     p.cgroups = 1;
     while (p.cgroups < 8 && p.wt_bytes / p.cgroups > (2u << 20)) p.cgroups *= 2;
     return p;
 }
 }  // namespace
-// Where there are tiles enough for every compute unit to take several, and up to 256 output channels (with more, the kernel
-// that holds a grad_out tile in LDS and reads grad_out where it lies reaches the same rate: 512 -> 512 on 2x8x30x54 380 us
-// against 400, and 40 to put the operands in order); grad_out within 32-bit offsets.
+// One weight group, as many output channels as the registers hold; grad_out and the rows of a pair within 32-bit offsets.  Of any
+// size: training steps, us, with the kernel of the other shapes (tiled_bwd_col32_kernel) and with this one: 64 -> 64 on 49
+// positions 84, 79; 512 -> 512 on 63 188, 142; 256 -> 256 on 420 160, 139; 1400 141, 126; 128 -> 128 on 12960 215, 204.
 bool d2c_grad_col_supported(const d2c_conv3d_desc &q)
 {
     const GradColPlan p = grad_col_plan(q);
-    return q.dtype == D2C_BF16 && q.groups == 1 && q.Cin % 64 == 0 && q.Cout > 32 && q.Cout <= 256 &&
-           (size_t)q.N * q.Do * q.Ho * q.Wo * p.Cp * 2 + 1024 < 0xFFFF0000u && (long)p.ntile * p.nct >= 4L * d2c_num_cus() &&
-           (long)p.ntile * p.nct * p.S < (1L << 30) && (size_t)q.N * q.Do * q.Ho * q.Wo * 128 < 0xFFFF0000u;
+    const size_t M = (size_t)q.N * q.Do * q.Ho * q.Wo;
+    return q.dtype == D2C_BF16 && q.groups == 1 && q.Cin % 64 == 0 && q.Cout <= 512 && M * p.Cp * 2 + 1024 < 0xFFFF0000u &&
+           (long)p.ntile * p.npair * p.S < (1L << 30) &&
+           M * 128 < 0xFFFF0000u;
 }
 size_t d2c_grad_col_ws(const d2c_conv3d_desc &q) { return grad_col_plan(q).total; }
 // What the backward pass over sorted points needs of grad_out and the weights, and what it adds into, as one launch (one
@@ -1538,12 +1551,22 @@ int d2c_brick_bwd_prepare(const d2c_conv3d_desc &q, const void *gout, const void
 int d2c_grad_col(const d2c_conv3d_desc &q, void *gcol, void *ws, hipStream_t st)
 {
     const GradColPlan p = grad_col_plan(q);
-    const int K = q.kd * q.kh * q.kw, M = q.N * q.Do * q.Ho * q.Wo, ncu = d2c_num_cus();
+    const int M = q.N * q.Do * q.Ho * q.Wo, ncu = d2c_num_cus();
     if (ncu <= 0) return D2C_ERR_LAUNCH;
-    GradColArgs a{(const unsigned char *)ws + p.wt_bytes, (const unsigned char *)ws, (bf16_t *)gcol, (unsigned)p.Cp * 2u, M, q.Cin / 64 * K,
-                  p.S, p.ntile, p.nct, p.cgroups};
+    GradColArgs a{(const unsigned char *)ws + p.wt_bytes, (const unsigned char *)ws, (bf16_t *)gcol, (unsigned)p.Cp * 2u, M, p.npair, p.ntile, p.cgroups};
     D2cProfScope prof(D2C_PROF_BWD_DATA, st, "grad_col_kernel");
-    hipLaunchKernelGGL(grad_col_kernel, dim3((unsigned)std::max(8, ncu / 8 * 8)), dim3(kThreads), 0, st, a);
+    const dim3 grid((unsigned)std::max(8, ncu / 8 * 8));
+    auto launch = [&](auto S) { hipLaunchKernelGGL((grad_col_kernel<decltype(S)::value>), grid, dim3(kThreads), 0, st, a); };
+    switch (p.S) {
+    case 1: launch(std::integral_constant<int, 1>{}); break;
+    case 2: launch(std::integral_constant<int, 2>{}); break;
+    case 3: launch(std::integral_constant<int, 3>{}); break;
+    case 4: launch(std::integral_constant<int, 4>{}); break;
+    case 5: launch(std::integral_constant<int, 5>{}); break;
+    case 6: launch(std::integral_constant<int, 6>{}); break;
+    case 7: launch(std::integral_constant<int, 7>{}); break;
+    default: launch(std::integral_constant<int, 8>{}); break;
+    }
     return d2c_check_launch("grad_col_kernel");
 }
 
