@@ -32,23 +32,6 @@ struct BrickPoint {
     float hz, hy, hx;     // fractions, as make_tap3 gives them
 };
 D2C_DEV int brick_seg(const BrickDims &d, int bg, int zi, int by, int bx) { return ((bg * d.nz + zi) * d.nby + by) * d.nbx + bx; }
-// (`c`: what tap_offsets_issue() read for tap k of output position (oz, oy, ox))
-template <bool AUX16, bool SIZED>
-D2C_DEV BrickPoint brick_point(const TiledShape &s, const float *craw, int k, int oz, int oy, int ox)
-{
-    float c[3] = {craw[0], craw[1], craw[2]};
-    tap_offsets_finish<AUX16, SIZED>(s, k, c);
-    int bz, by, bx;
-    tap_base(s.geo, k, oz, oy, ox, bz, by, bx);
-    const Tap3<float> t = tiled_tap3(s, bz, by, bx, c[0], c[1], c[2]);
-    BrickPoint r;
-    r.in = t.inrange != 0;
-    r.zi = t.z0 + 1; r.yq = (t.y0 + 1) / 3; r.xq = (t.x0 + 1) / 3;       // (base voxels start at -1)
-    r.cell = (unsigned)(t.y0 + 1 - r.yq * 3) | (unsigned)(t.x0 + 1 - r.xq * 3) << 2;
-    r.hz = t.hz; r.hy = t.hy; r.hx = t.hx;
-    return r;
-}
-
 // ---- the sort: count the points of every block, give every block a range, file -------------------------------------
 // A workgroup works on 256 positions and up to 28 taps, 4 threads to a position, and requests what it reads of all of
 // them first.  Points of neighbouring positions fall into few blocks: they are counted in LDS, in a window of the blocks
@@ -58,7 +41,7 @@ D2C_DEV BrickPoint brick_point(const TiledShape &s, const float *craw, int k, in
 // So neither pass writes or reads anything per point that is not wanted in the end.  Points outside the window take
 // the global additions one by one; those outside the volume are counted per workgroup too (additions to one address
 // follow each other at about 10 ns: with one for every wavefront the list of them took half of the filing pass).
-// Bound: scattered stores of 20 bytes to a point, and the instructions of a point's place (about 150).  5.6 M points in 8
+// Bound: scattered stores of 20 bytes to a point, and the instructions of a point's place.  5.6 M points in 8
 // offset groups on 2x8x30x54, us for counting + ranges + filing: 134 + 8 + 146 with a hash table per workgroup, places
 // of the counting pass kept in memory and an addition per wavefront for the points outside; 46 + 5 + 89 this way.
 // 32x60x108 in one group 95 + 7 + 136 and 48 + 5 + 100; 2x8x30x54 in one group 24 + 4 + 35 and 12 + 5 + 21.
@@ -71,10 +54,12 @@ struct SortWindow {
     int ngrp, taps;       // groups of taps, taps to a group (up to kSortTaps)
     int ly, lx;           // a workgroup's positions: 2^(8 - ly - lx) planes of 2^ly x 2^lx
     int ny, nx, ntile;    // such tiles along y and x, and of a sample
+    FastDiv dkw, dkh;     // divisions by the filter's extents
 };
 struct SortUnit {
     int b, g, bg, k0, k1; // taps k0, k0 + kTapGroups, ... below k1
     int oz, oy, ox, p;    // the thread's position
+    int bz, by, bx;       // ... in the input, without a tap
     bool ok;              // ... is one
     int z0, y0, x0;       // first block of the window
 };
@@ -90,6 +75,7 @@ D2C_DEV SortUnit sort_unit(const TiledShape &s, const BrickDims &d, const SortWi
     t.oz = (tz << lz) + (i >> (w.ly + w.lx)); t.oy = (ty << w.ly) + ((i >> w.lx) & ((1 << w.ly) - 1)); t.ox = (tx << w.lx) + (i & ((1 << w.lx) - 1));
     t.ok = t.oz < s.Do && t.oy < s.Ho && t.ox < s.Wo;
     t.p = t.ok ? (t.oz * s.Ho + t.oy) * s.Wo + t.ox : 0;
+    t.bz = t.oz * s.geo.sd - s.geo.pd; t.by = t.oy * s.geo.sh - s.geo.ph; t.bx = t.ox * s.geo.sw - s.geo.pw;
     t.k0 = (u - blk * w.ngrp) * w.taps;
     t.k1 = min(t.k0 + w.taps, s.K);
     t.k0 += __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
@@ -102,6 +88,30 @@ D2C_DEV SortUnit sort_unit(const TiledShape &s, const BrickDims &d, const SortWi
     t.x0 = max(0, min(cx - w.wx / 2, d.nbx - w.wx));
     return t;
 }
+// Tap k of the thread's position from its offsets (sort_offsets): make_tap3 with what the sort needs of it.  A
+// position is clamped to where no corner is inside, which is also what the median makes of one that is no number; along an axis that
+// is fixed the far plane has no corners.  All of a point's instructions count here: the passes are bound by them.
+template <bool AUX16, bool SIZED>
+D2C_DEV BrickPoint brick_point(const TiledShape &s, const SortWindow &w, const SortUnit &t, const float *craw, int k)
+{
+    const int kr = fdiv(k, w.dkw), kx = k - kr * s.geo.kw, kz = fdiv(kr, w.dkh), ky = kr - kz * s.geo.kh;
+    float c[3] = {craw[0], craw[1], craw[2]};
+    if constexpr (SIZED) size_tap_offsets<AUX16>(s, kz, ky, kx, c, c);
+    else tap_offsets_finish<AUX16, false>(s, k, c);
+    const float z = (float)(t.bz + kz * s.geo.dd) + c[0], y = (float)(t.by + ky * s.geo.dh) + c[1], x = (float)(t.bx + kx * s.geo.dw) + c[2];
+    const float fz = floorf(__builtin_amdgcn_fmed3f(z, -4.f, (float)(s.D + 4))), fy = floorf(__builtin_amdgcn_fmed3f(y, -4.f, (float)(s.H + 4))),
+                fx = floorf(__builtin_amdgcn_fmed3f(x, -4.f, (float)(s.W + 4)));
+    const int z0 = (int)fz, y0 = (int)fy, x0 = (int)fx;
+    const int ez = (s.keep & 0xF0u) != 0, ey = (s.keep & 0xCCu) != 0, ex = (s.keep & 0xAAu) != 0;
+    BrickPoint r;
+    r.in = (unsigned)(z0 + ez) < (unsigned)(s.D + ez) && (unsigned)(y0 + ey) < (unsigned)(s.H + ey) && (unsigned)(x0 + ex) < (unsigned)(s.W + ex);
+    // (base voxels start at -1; the quotients are off by a sixth at least from where rounding would matter)
+    r.zi = z0 + 1;
+    r.yq = (int)floorf(fmaf(fy, 1.f / 3.f, 0.5f)); r.xq = (int)floorf(fmaf(fx, 1.f / 3.f, 0.5f));
+    r.cell = (unsigned)(y0 + 1 - r.yq * 3) | (unsigned)(x0 + 1 - r.xq * 3) << 2;
+    r.hz = z - fz; r.hy = y - fy; r.hx = x - fx;
+    return r;
+}
 // slot of a point's block in the window, -1: outside
 D2C_DEV int sort_slot(const SortWindow &w, const SortUnit &t, const BrickPoint &q)
 {
@@ -113,13 +123,18 @@ D2C_DEV int sort_slot_seg(const BrickDims &d, const SortWindow &w, const SortUni
     const int r = i / w.wx, x = i - r * w.wx, z = r / w.wy, y = r - z * w.wy;
     return brick_seg(d, t.bg, t.z0 + z, t.y0 + y, t.x0 + x);
 }
-// the offsets of the thread's taps k0, k0 + kTapGroups, ...
+// the offsets of the thread's taps k0, k0 + kTapGroups, ...; of a size map: size - 1 of the position, in the first place
 template <bool AUX16, bool SIZED>
 D2C_DEV void sort_offsets(const TiledShape &s, const void *off, const SortUnit &t, float (&c)[kTaps][3])
 {
+    if constexpr (SIZED) {
+        tap_offsets_issue<AUX16, true>(s, off, t.b, t.g, 0, t.p, c[0]);
+        if (s.ss.on == 1) size_minus_one<AUX16>(s, c[0]);
+    } else {
 #pragma unroll
-    for (int i = 0; i < kTaps; i++)
-        if (t.k0 + i * kTapGroups < t.k1) tap_offsets_issue<AUX16, SIZED>(s, off, t.b, t.g, t.k0 + i * kTapGroups, t.p, c[i]);
+        for (int i = 0; i < kTaps; i++)
+            if (t.k0 + i * kTapGroups < t.k1) tap_offsets_issue<AUX16, false>(s, off, t.b, t.g, t.k0 + i * kTapGroups, t.p, c[i]);
+    }
 }
 template <bool AUX16, bool SIZED>
 __global__ void __launch_bounds__(kSortThreads, 8)     // (two workgroups to a compute unit)
@@ -137,7 +152,7 @@ brick_count_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, Sor
     for (int i = 0; i < kTaps; i++) {
         const int k = t.k0 + i * kTapGroups;
         if (!t.ok || k >= t.k1) continue;
-        const BrickPoint q = brick_point<AUX16, SIZED>(s, c[i], k, t.oz, t.oy, t.ox);
+        const BrickPoint q = brick_point<AUX16, SIZED>(s, w, t, c[SIZED ? 0 : i], k);
         if (!q.in) continue;
         const int sl = sort_slot(w, t, q);
         if (sl >= 0) atomicAdd(&s_cnt[sl], 1);
@@ -191,6 +206,7 @@ brick_file_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, cons
     }
     for (int i = threadIdx.x; i <= nslot; i += kSortThreads) s_cnt[i] = 0;
     __syncthreads();
+    const float size[3] = {c[0][0], c[0][1], c[0][2]};
     // slot << 4 | base voxel (slot -1: outside the window, `rank` is the entry; all ones: no point)
     int slot[kTaps], rank[kTaps];
 #pragma unroll
@@ -198,7 +214,7 @@ brick_file_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, cons
         const int k = t.k0 + i * kTapGroups;
         slot[i] = -1; rank[i] = 0;
         if (!t.ok || k >= t.k1) continue;
-        const BrickPoint q = brick_point<AUX16, SIZED>(s, c[i], k, t.oz, t.oy, t.ox);
+        const BrickPoint q = brick_point<AUX16, SIZED>(s, w, t, SIZED ? size : c[i], k);
         c[i][0] = q.hz; c[i][1] = q.hy; c[i][2] = q.hx;
         if (!q.in) continue;
         const int sl = sort_slot(w, t, q);
@@ -222,6 +238,8 @@ brick_file_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, cons
         if (m) s_cnt[i] = atomicAdd(&L.end[sort_slot_seg(d, w, t, i)], m);
     }
     __syncthreads();
+    // (everything that has been asked for is here: the stores below wait for nothing, least of all for one another)
+    __builtin_amdgcn_s_waitcnt(0x0F70);
 #pragma unroll
     for (int i = 0; i < kTaps; i++) {
         const int k = t.k0 + i * kTapGroups;
@@ -1292,7 +1310,7 @@ double brick_mean(const TiledShape &s) { return 9.0 * s.K * s.P / s.vol; }      
 constexpr int kSortSlots = 8192;
 SortWindow sort_window(const TiledShape &s, const BrickDims &d)
 {
-    SortWindow w{d.nz, d.nby, d.nbx, 0, 0, 0, 0, 0, 0, 0};
+    SortWindow w{d.nz, d.nby, d.nbx, 0, 0, 0, 0, 0, 0, 0, make_fastdiv(s.geo.kw), make_fastdiv(s.geo.kh)};
     // A tile of 4 x 8 x 8 positions reaches fewer blocks than 64 positions of a few rows (filing 32x60x108: 122 us, 136).  With
     // few tiles the taps of one are dealt to several workgroups (counting + filing 1024 -> 256 channels on 8x30x54: 20 + 32 us
     // on 56 workgroups, 10 + 15 on 224; on four times as many as compute units no faster).

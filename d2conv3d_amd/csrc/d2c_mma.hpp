@@ -399,18 +399,16 @@ D2C_DEV void tap_offsets_issue(const TiledShape &s, const void *off, int b, int 
         }
         return;
     }
-    const long ab = offset_index(s, b, g, k, p);
+    // (as they are stored: what is done to a value here would wait for it)
+    auto raw = [&](long i) { return AUX16 ? __uint_as_float((unsigned)reinterpret_cast<const bf16_t *>(off)[i]) : reinterpret_cast<const float *>(off)[i]; };
+    const long ob = offset_index(s, b, g, k, p);
     if (s.nd == 3) {
-        const long ob = ab;
-        // (all three are requested, a fixed axis is dropped by a select: no branches between the loads)
-        const float v0 = ld_auxT<AUX16>(off, ob), v1 = ld_auxT<AUX16>(off, ob + s.P);
-        const float v2 = ld_auxT<AUX16>(off, ob + 2 * (long)s.P);
-        c[0] = (s.axes & 1) ? v0 : 0.f;
-        c[1] = (s.axes & 2) ? v1 : 0.f;
-        c[2] = (s.axes & 4) ? v2 : 0.f;
+        c[0] = raw(ob);
+        c[1] = raw(ob + s.P);
+        c[2] = raw(ob + 2 * (long)s.P);
     } else {
         c[0] = 0.f; c[1] = 0.f;
-        c[2] = ld_auxT<AUX16>(off, ab);
+        c[2] = raw(ob);
     }
 }
 // size map: raw sizes of a position -> (size - 1) per axis, the part of a tap's offsets that all taps share
@@ -422,21 +420,31 @@ template <bool AUX16> D2C_DEV void size_minus_one(const TiledShape &s, float *c)
         c[ax] = axis_channel(s.ss.mode, ax) < 0 ? 0.f : rnd<AT>(size_act<AT>(s.ss.act, c[ax]) - 1.f);
 }
 // ... and from there the offsets of tap k
-template <bool AUX16> D2C_DEV void size_tap_offsets(const TiledShape &s, int k, const float *sm1, float *o)
+template <bool AUX16> D2C_DEV void size_tap_offsets(const TiledShape &s, int kz, int ky, int kx, const float *sm1, float *o)
 {
     typedef typename std::conditional<AUX16, bf16_t, float>::type AT;
-    const int kz = k / (s.geo.kw * s.geo.kh), ky = (k / s.geo.kw) % s.geo.kh, kx = k % s.geo.kw;
     const float b0 = s.ss.base[0][kz], b1 = s.ss.base[1][ky], b2 = s.ss.base[2][kx];
     const float s0 = sm1[0], s1 = sm1[1], s2 = sm1[2];
     o[0] = rnd<AT>(rnd<AT>(b0) * s0);
     o[1] = rnd<AT>(rnd<AT>(b1) * s1);
     o[2] = rnd<AT>(rnd<AT>(b2) * s2);
 }
+template <bool AUX16> D2C_DEV void size_tap_offsets(const TiledShape &s, int k, const float *sm1, float *o)
+{
+    size_tap_offsets<AUX16>(s, k / (s.geo.kw * s.geo.kh), (k / s.geo.kw) % s.geo.kh, k % s.geo.kw, sm1, o);
+}
 template <bool AUX16, bool SIZED> D2C_DEV void tap_offsets_finish(const TiledShape &s, int k, float *c)
 {
     if constexpr (SIZED) {
         if (s.ss.on == 1) size_minus_one<AUX16>(s, c);
         size_tap_offsets<AUX16>(s, k, c, c);
+    } else {
+#pragma unroll
+        for (int ax = 0; ax < 3; ax++) {
+            if (AUX16) c[ax] = __uint_as_float(__float_as_uint(c[ax]) << 16);
+            // (all three have been read, a fixed axis is dropped by a select: no branches between the loads)
+            if (s.nd == 3) c[ax] = (s.axes >> ax) & 1 ? c[ax] : 0.f;
+        }
     }
 }
 
