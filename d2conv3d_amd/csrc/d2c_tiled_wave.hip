@@ -47,11 +47,15 @@ D2C_DEV int xcd_swizzle(int bid, int n)
 // of the reduction.  A wavefront samples the 32 positions of its step into a tile of its own in LDS and multiplies it:
 // there is no barrier between the first step and the sum of the partial results, so eight chains of dependent
 // latencies (offsets, corner rows, fragments) run side by side instead of one.  The corners of step i + 1 and the
-// fragments of step i + 1 are in flight while step i is multiplied.
+// fragments of step i + 1 are in flight while step i is multiplied.  The corners of an item are requested into the
+// registers of the one that has just been interpolated, and a tap's offsets before the corners of the step in front of it, as they
+// are stored: a wait for them is no wait for corners.  (us per forward call, with all corners of a step requested behind the
+// interpolation and the offsets behind those, and this way: 64 -> 64 on 8x32x32 37.8, 35.6; bfloat16 28.3, 26.1; sized 42.0, 36.1;
+// 128 -> 64 on 8x30x54, bfloat16 71.3, 65.0; 64 -> 64 on 16x60x100 343.8, 327.)
 // Partial sums of workgroups go to the workspace; the one that finishes last adds them up, in a fixed order, applies bias
 // and activation and stores: no clear in front, no kernel behind.
 // Bound: few steps, by latency (64 -> 64 channels on 4x14x25, float32: one or two steps to a wavefront); many, by the corner
-// rows through L1 and the vector ALU's 4 clocks per instruction, about equally (8x32x32: 453 MB through L1, 12 us of 30).
+// rows through L1 and the vector ALU's 4 clocks per instruction, about equally (8x32x32: 453 MB through L1, 12 us of 28).
 // Against workgroups that take a step of 128 positions together, barrier by barrier, with atomic partial sums, a clear
 // and a finishing kernel, us per forward call: 4x14x25 37.5 -> 18.1, 8x32x32 62.2 -> 34.9; 128 -> 128 on 8x32x32 310 ->
 // 69; 1024 -> 128 on 4x14x25 425 -> 97; conv1d 4 x 512 -> 512 on 64 positions 31.8 -> 21.9.
@@ -139,10 +143,12 @@ __global__ void __launch_bounds__(kThreads) tiled_fwd_wave_kernel(WaveArgs a)
         }
         const unsigned dx = (unsigned)s.Cin * (unsigned)sizeof(T), dy = (unsigned)s.W * dx, dz = (unsigned)s.H * dy;
         float craw[4] = {0.f, 0.f, 0.f, 1.f};
+        // (as it is stored: nothing here waits for what it reads; a lane without a position reads the first one's)
         auto coords_issue = [&](const WaveWalk &w) INLINE {
-            if (cvalid) {
-                tap_offsets_issue<AUX16, SIZED>(s, a.off, cb, w.g, w.k, cp, craw);
-                craw[3] = a.mask ? ld_auxT<AUX16>(a.mask, mask_index(s, cb, w.g, w.k, cp)) : 1.f;
+            tap_offsets_issue<AUX16, SIZED>(s, a.off, cb, w.g, w.k, cp, craw);
+            if (a.mask) {
+                const long at = mask_index(s, cb, w.g, w.k, cp);
+                craw[3] = AUX16 ? __uint_as_float((unsigned)reinterpret_cast<const bf16_t *>(a.mask)[at]) : reinterpret_cast<const float *>(a.mask)[at];
             }
         };
         auto coords_finish = [&](const WaveWalk &w, int buf) INLINE {
@@ -155,7 +161,8 @@ __global__ void __launch_bounds__(kThreads) tiled_fwd_wave_kernel(WaveArgs a)
                 const Tap3<float> t = tiled_tap3(s, coz * s.geo.sd - s.geo.pd + w.kz * s.geo.dd,
                                                  coy * s.geo.sh - s.geo.ph + w.ky * s.geo.dh,
                                                  cox * s.geo.sw - s.geo.pw + w.kx * s.geo.dw, craw[0], craw[1], craw[2]);
-                const float al = (s.mact && a.mask) ? mask_act<AT>(s.mact, craw[3]) : craw[3];
+                const float am = AUX16 && a.mask ? __uint_as_float(__float_as_uint(craw[3]) << 16) : craw[3];
+                const float al = (s.mact && a.mask) ? mask_act<AT>(s.mact, am) : am;
                 const unsigned o0 = (unsigned)(cb * s.vol + (t.z0 * s.H + t.y0) * s.W + t.x0) * dx;
                 unsigned read = t.live;
                 if (__builtin_expect(a.skip_zero, 0))
@@ -184,30 +191,29 @@ __global__ void __launch_bounds__(kThreads) tiled_fwd_wave_kernel(WaveArgs a)
         // an offset past its end, which loads zeros without a request.
         const int gpos = lane >> 3, gvec = lane & 7;
         uint4 gv[NG][8];
-        auto gather_issue = [&](const WaveWalk &w, int buf, int i0) INLINE {
+        auto gather_issue = [&](const WaveWalk &w, int buf, auto I) INLINE {
+            constexpr int item = decltype(I)::value, i = item % NG;
             const unsigned c0 = (unsigned)(wg * s.cg + w.j * s.bkc) * (unsigned)sizeof(T);
             const __amdgpu_buffer_rsrc_t res = __builtin_amdgcn_make_buffer_rsrc(
                 const_cast<char *>(reinterpret_cast<const char *>(a.xcl)) + c0, 0, (int)(a.xbytes - c0), 0x00020000);
+            unsigned co[8];
 #pragma unroll
-            for (int i = 0; i < NG; i++) {
-                unsigned co[8];
-#pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    const uint4 v = *reinterpret_cast<const uint4 *>(tab_o + buf * kWTab + ((i0 + i) * 8 + gpos) * 8 + h * 4);
-                    co[4 * h] = v.x; co[4 * h + 1] = v.y; co[4 * h + 2] = v.z; co[4 * h + 3] = v.w;
-                }
-#pragma unroll
-                for (int c = 0; c < 8; c++) {
-                    typedef unsigned u32x4_b __attribute__((ext_vector_type(4)));
-                    const u32x4_b v = __builtin_amdgcn_raw_buffer_load_b128(res, (int)(co[c] + (unsigned)gvec * 16u), 0, 0);
-                    gv[i][c] = make_uint4(v[0], v[1], v[2], v[3]);
-                }
+            for (int h = 0; h < 2; h++) {
+                const uint4 v = *reinterpret_cast<const uint4 *>(tab_o + buf * kWTab + (item * 8 + gpos) * 8 + h * 4);
+                co[4 * h] = v.x; co[4 * h + 1] = v.y; co[4 * h + 2] = v.z; co[4 * h + 3] = v.w;
             }
-        };
-        auto interp = [&](const WaveWalk &w, int buf, int i0) INLINE {
 #pragma unroll
-            for (int i = 0; i < NG; i++) {
-                const int pos = (i0 + i) * 8 + gpos;
+            for (int c = 0; c < 8; c++) {
+                typedef unsigned u32x4_b __attribute__((ext_vector_type(4)));
+                const u32x4_b v = __builtin_amdgcn_raw_buffer_load_b128(res, (int)(co[c] + (unsigned)gvec * 16u), 0, 0);
+                gv[i][c] = make_uint4(v[0], v[1], v[2], v[3]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto interp = [&](const WaveWalk &w, int buf, auto I) INLINE {
+            constexpr int item = decltype(I)::value, i = item % NG;
+            {
+                const int pos = item * 8 + gpos;
                 const float4 w0 = *reinterpret_cast<const float4 *>(tab_w + buf * kWTab + pos * 8);
                 const float4 w1 = *reinterpret_cast<const float4 *>(tab_w + buf * kWTab + pos * 8 + 4);
                 const float cw[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
@@ -228,7 +234,6 @@ __global__ void __launch_bounds__(kThreads) tiled_fwd_wave_kernel(WaveArgs a)
                             + (((long)(wg * s.nchunk + w.j) * s.K + w.k) * a.col_rows + m0 + pos) * (kNV * 16) + gvec * 16));
                 }
             }
-            __builtin_amdgcn_wave_barrier();
         };
 
         // weight fragments: those of the next step are requested as soon as the matrix cores have taken the current ones
@@ -239,8 +244,16 @@ __global__ void __launch_bounds__(kThreads) tiled_fwd_wave_kernel(WaveArgs a)
             return wp4 + (((long)wg * S + w.j * s.K + w.k) * OBT + otile * OB) * (NKG * 64) + lane;
         };
 
-        WaveWalk wm = wave_walk(s, wg, st_lo), wn = wm;       // the step being multiplied; the one being fetched
-        coords_issue(wn);
+        // The step being multiplied, whose first corners are under way, and the next one, whose tap's coordinates are (where it
+        // is another tap).  Requests are waited for in their order: the coordinates of a step go in front of the corners of the step
+        // before, so that working them out leaves those in flight.
+        WaveWalk wm = wave_walk(s, wg, st_lo), wn = wm;
+        coords_issue(wm);
+        int cur = 0;
+        coords_finish(wm, 0);
+        bool fresh = wave_advance(wn, s);
+        if (fresh && wn.st < st_hi) coords_issue(wn);
+        for_each_const([&](auto I) INLINE { gather_issue(wm, 0, I); }, std::make_integer_sequence<int, NG>{});
         {
             const uint4 *fr = frag_row(wm);
 #pragma unroll
@@ -248,42 +261,44 @@ __global__ void __launch_bounds__(kThreads) tiled_fwd_wave_kernel(WaveArgs a)
 #pragma unroll
                 for (int ob = 0; ob < OB; ob++) af[kg][ob] = fr[(ob * NKG + kg) * 64];
         }
-        int cur = 0;
-        coords_finish(wn, 0);
-        gather_issue(wn, 0, 0);
-        bool fresh = wave_advance(wn, s);
-        if (fresh && wn.st < st_hi) coords_issue(wn);
-        for (;;) {
-            const bool more = wn.st < st_hi;
-            const int nxt = (more && fresh) ? cur ^ 1 : cur;
-            if (more && fresh) coords_finish(wn, nxt);
-            interp(wm, cur, 0);
-#pragma unroll
-            for (int i0 = NG; i0 < ITEMS; i0 += NG) {
-                gather_issue(wm, cur, i0);
-                interp(wm, cur, i0);
-            }
-            wm = wn;
+        const unsigned char *const t0 = tb + (lane & 31) * kRS + (lane >> 5) * 16;
+        while (wn.st < st_hi) {
+            int nxt = cur;
+            if (fresh) { nxt ^= 1; coords_finish(wn, nxt); }
+            WaveWalk w2 = wn;
+            fresh = wave_advance(w2, s);
+            if (fresh && w2.st < st_hi) coords_issue(w2);
+            // (the corners of the item NG further on, of this step or the next, into the registers that have just been read)
+            for_each_const([&](auto I) INLINE {
+                constexpr int item = decltype(I)::value;
+                interp(wm, cur, I);
+                if constexpr (item + NG < ITEMS) gather_issue(wm, cur, std::integral_constant<int, item + NG>{});
+                else gather_issue(wn, nxt, std::integral_constant<int, (item + NG) % ITEMS>{});
+            }, std::make_integer_sequence<int, ITEMS>{});
+            __builtin_amdgcn_wave_barrier();
             const uint4 *fr = frag_row(wn);
-            if (more) {
-                gather_issue(wn, nxt, 0);
-                fresh = wave_advance(wn, s);
-                if (fresh && wn.st < st_hi) coords_issue(wn);
-            }
-            const unsigned char *t0 = tb + (lane & 31) * kRS + (lane >> 5) * 16;
 #pragma unroll
             for (int kg = 0; kg < NKG; kg++) {
                 const uint4 bf = *reinterpret_cast<const uint4 *>(t0 + kg * 32);
 #pragma unroll
                 for (int ob = 0; ob < OB; ob++) mma_kgroup<T, kF32SplitFwd>(acc[ob], af[kg][ob], bf);
-                if (more) {
 #pragma unroll
-                    for (int ob = 0; ob < OB; ob++) af[kg][ob] = fr[(ob * NKG + kg) * 64];
-                }
+                for (int ob = 0; ob < OB; ob++) af[kg][ob] = fr[(ob * NKG + kg) * 64];
             }
             __builtin_amdgcn_wave_barrier();
-            if (!more) break;
-            cur = nxt;
+            wm = wn; wn = w2; cur = nxt;
+        }
+        for_each_const([&](auto I) INLINE {
+            constexpr int item = decltype(I)::value;
+            interp(wm, cur, I);
+            if constexpr (item + NG < ITEMS) gather_issue(wm, cur, std::integral_constant<int, item + NG>{});
+        }, std::make_integer_sequence<int, ITEMS>{});
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int kg = 0; kg < NKG; kg++) {
+            const uint4 bf = *reinterpret_cast<const uint4 *>(t0 + kg * 32);
+#pragma unroll
+            for (int ob = 0; ob < OB; ob++) mma_kgroup<T, kF32SplitFwd>(acc[ob], af[kg][ob], bf);
         }
     }
 
