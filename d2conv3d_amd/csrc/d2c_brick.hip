@@ -1038,8 +1038,10 @@ __global__ void __launch_bounds__(64 * kMaxWaves, 4) brick_sample_kernel(BrickSa
 {
     const int lane = threadIdx.x & 63, h = lane >> 5, n = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
-    __shared__ __align__(16) unsigned char s_all[kMaxWaves][32 * 128];
-    unsigned char *const s_r = s_all[wave];                          // a plane's 16 input rows; 32 rows on their way out
+    // (of as many wavefronts as there are: with four times what one needs, workgroups of one were ten to a compute unit: 512 channels in 8
+    // groups on 2x8x30x54 206 us, with sixteen 194)
+    extern __shared__ __align__(16) unsigned char smem[];
+    unsigned char *const s_r = smem + wave * kRowLds;                // a plane's 16 input rows; 32 rows on their way out
     const int pv = lane >> 3, pc = lane & 7;
     if ((int)blockIdx.x < a.nzero) {
         // rows of the points outside the volume, and those behind the last position: zeros (8 lanes to a chunk's row)
@@ -1481,6 +1483,6 @@ int d2c_brick_columns(const TiledShape &s, const void *xcl, void *col, int rows,
     a.npoint = brick_points(s);
     a.nzero = (int)std::min<long>(2048, (a.npoint + 511) / 512) / nw + 1;
     D2cProfScope prof(D2C_PROF_SAMPLE, st, "brick_sample_kernel");
-    hipLaunchKernelGGL(brick_sample_kernel, dim3((unsigned)(cols * a.nzr + a.nzero)), dim3(64 * nw), 0, st, a, a.L.end, a.L.count);
+    hipLaunchKernelGGL(brick_sample_kernel, dim3((unsigned)(cols * a.nzr + a.nzero)), dim3(64 * nw), nw * kRowLds, st, a, a.L.end, a.L.count);
     return d2c_check_launch("brick_sample_kernel");
 }
