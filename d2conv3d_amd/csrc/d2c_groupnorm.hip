@@ -10,7 +10,9 @@
 //         A = sum_{c' in g} gamma[c'] * r1[c'],  B = sum_{c' in g} gamma[c'] * (r2[c'] - mean * r1[c']) * rstd
 //     grad_gamma[c] = sum_n (r2 - mean * r1) * rstd,   grad_beta[c] = sum_n r1
 //
-// One workgroup per (sample, channel) row of P values; 16-byte accesses where the rows allow them.
+// One workgroup per (sample, channel) row of P values, or per piece of one where the output depends on single values; 16-byte
+// accesses, of rows of any alignment.
+#include <algorithm>
 #include "d2c_common.hpp"
 #include "d2c_mma.hpp"
 
@@ -26,6 +28,7 @@ struct GnArgs {
     void *y;                     // forward: y; backward: grad_x
     float *part;                 // backward: [N][C][2] (r1, r2)
     void *ggamma, *gbeta;
+    int pieces;                  // workgroups to a row
 };
 
 D2C_DEV float block_sum(float v, float *red)
@@ -41,24 +44,64 @@ D2C_DEV float block_sum(float v, float *red)
     return t;
 }
 
-// row of P values as 16-byte vectors where aligned: f(index, value) for every element
-template <typename T, typename F> D2C_DEV void for_row(const T *row, int P, F f)
-{
-    constexpr int VEC = 16 / (int)sizeof(T);
-    if (P % VEC == 0 && reinterpret_cast<uintptr_t>(row) % 16 == 0) {
-        for (int i = threadIdx.x; i < P / VEC; i += kGnThreads) {
-            const uint4 v = reinterpret_cast<const uint4 *>(row)[i];
-            const T *e = reinterpret_cast<const T *>(&v);
-#pragma unroll
-            for (int j = 0; j < VEC; j++) f(i * VEC + j, elem_to_f32<T>(e[j]));
-        }
-    } else {
-        for (int i = threadIdx.x; i < P; i += kGnThreads) f(i, elem_to_f32<T>(row[i]));
-    }
-}
-
 typedef unsigned int u32x4_by2 __attribute__((ext_vector_type(4), aligned(2)));
 typedef unsigned int u32x4_by4 __attribute__((ext_vector_type(4), aligned(4)));
+// (vectors of a type that says how they are aligned: rows of any length, one load or store each)
+template <typename T> using AnyVec = typename std::conditional<sizeof(T) == 2, u32x4_by2, u32x4_by4>::type;
+template <typename T> D2C_DEV AnyVec<T> load_any(const T *p) { return *reinterpret_cast<const AnyVec<T> *>(p); }
+// out[i] = f(in[0][i], ...) for a piece of a row, f = make().  Bound: memory; a thread requests up to kGnVectors vectors of each row, then works
+// out f (sums over a group, double).  Few rows are several workgroups each: four to a compute unit in all, since each works out f.(One workgroup
+// to a row, a vector at a time, rows of odd lengths element by element; us, before and after, forward and gradient, bfloat16: 256 rows of 51360
+// 19.6, 11.4 and 21.1, 15.0; of 51361 62, 13 and 74, 17; 1024 rows of 12960 12.3, 11.4 and 15.7, 14.9; float32 21.3, 17.3 and 25.8, 24.8; 55.8, 17.4 and
+// 59.8, 24.7; 64 rows of 50 3.4, 3.6.)
+constexpr int kGnVectors = 4;
+inline int row_pieces(const d2c_group_norm_desc &q)
+{
+    const long rows = (long)q.N * q.C, run = (long)kGnThreads * kGnVectors * (q.dtype == D2C_BF16 ? 8 : 4), want = 4L * std::max(d2c_num_cus(), 1);
+    return (int)std::max(std::min((q.P + run - 1) / run, (want + rows - 1) / rows), 1L);
+}
+template <typename T, int NIN, typename Make> D2C_DEV void map_piece(const T *const (&in)[NIN], T *out, int P, int piece, int pieces, Make make)
+{
+    constexpr int VEC = 16 / (int)sizeof(T);
+    const int nv = P / VEC, len = (nv + pieces - 1) / pieces, v1 = min(nv, (piece + 1) * len);
+    AnyVec<T> q[kGnVectors][NIN];
+    auto request = [&](int v0) INLINE {
+#pragma unroll
+        for (int k = 0; k < kGnVectors; k++)
+#pragma unroll
+            for (int j = 0; j < NIN; j++)
+                if (v0 + k * kGnThreads < v1) q[k][j] = load_any(in[j] + (long)(v0 + k * kGnThreads) * VEC);
+    };
+    int v0 = piece * len + (int)threadIdx.x;
+    request(v0);
+    const auto f = make();
+    while (v0 < v1) {
+#pragma unroll
+        for (int k = 0; k < kGnVectors; k++) {
+            if (v0 + k * kGnThreads >= v1) continue;
+            alignas(16) T e[NIN][VEC], o[VEC];
+#pragma unroll
+            for (int j = 0; j < NIN; j++) *reinterpret_cast<AnyVec<T> *>(e[j]) = q[k][j];
+#pragma unroll
+            for (int i = 0; i < VEC; i++) {
+                float v[NIN];
+#pragma unroll
+                for (int j = 0; j < NIN; j++) v[j] = elem_to_f32<T>(e[j][i]);
+                o[i] = f32_to_elem<T>(f(v));
+            }
+            *reinterpret_cast<AnyVec<T> *>(out + (long)(v0 + k * kGnThreads) * VEC) = *reinterpret_cast<const AnyVec<T> *>(o);
+        }
+        v0 += kGnThreads * kGnVectors;
+        request(v0);
+    }
+    if (piece + 1 == pieces && (int)threadIdx.x < P - nv * VEC) {
+        const int i = nv * VEC + threadIdx.x;
+        float v[NIN];
+#pragma unroll
+        for (int j = 0; j < NIN; j++) v[j] = elem_to_f32<T>(in[j][i]);
+        out[i] = f32_to_elem<T>(f(v));
+    }
+}
 // A thread's values go in sixteens, added up pairwise, then to sums in double: one chain of float additions loses up to 5e-6 of
 // a sum of squares on 205440 positions (bfloat16 squares are short and round to one side), this way 6e-8.  Bound: memory, and
 // latency where the rows are few.  us, chains first: 256 channels, float32, 51360 positions 18.1, 10.1; 51361 (rows of any alignment, which
@@ -81,16 +124,14 @@ template <typename T> __global__ void __launch_bounds__(kGnThreads) channel_stat
             for (int i = 0; i < n; i++) { t[i] += t[i + n]; u[i] += u[i + n]; }
         s += (double)t[0]; sq += (double)u[0];
     };
-    // (vectors of a type that says how they are aligned: rows of any length, one load each)
-    typedef typename std::conditional<sizeof(T) == 2, u32x4_by2, u32x4_by4>::type u32x4_any;
     const int nv = P / VEC;
     for (int i0 = threadIdx.x; i0 < nv; i0 += kGnThreads * NV) {
         float v[RUN];
 #pragma unroll
         for (int k = 0; k < NV; k++) {
             const int i = i0 + k * kGnThreads;
-            u32x4_any q = {0u, 0u, 0u, 0u};
-            if (i < nv) q = *reinterpret_cast<const u32x4_any *>(row + (long)i * VEC);
+            AnyVec<T> q = {0u, 0u, 0u, 0u};
+            if (i < nv) q = load_any(row + (long)i * VEC);
             const uint4 w = make_uint4(q[0], q[1], q[2], q[3]);
             const T *e = reinterpret_cast<const T *>(&w);
 #pragma unroll
@@ -136,49 +177,37 @@ D2C_DEV void group_moments(const GnArgs &a, int n, int c, float &mean, float &rs
     moments_from_sums(s, sq, (double)cpg * (double)a.q.P, a.q.eps, mean, rstd);
 }
 
-// the same by all threads of a workgroup together
-D2C_DEV void group_moments_block(const GnArgs &a, int n, int c, float &mean, float &rstd, float *)
+// the same for a workgroup: its first wavefront works it out (a division and a square root in double, on every SIMD as often as it
+// has wavefronts that do)
+D2C_DEV void group_moments_block(const GnArgs &a, int n, int c, float &mean, float &rstd)
 {
-    __shared__ double redd[2][kGnThreads / 64];
-    const int cpg = a.q.C / a.q.groups, g = c / cpg;
-    const float *st = a.stats + ((long)n * a.q.C + g * cpg) * 2;
-    double s = 0.0, sq = 0.0;
-    for (int i = threadIdx.x; i < cpg; i += kGnThreads) { s += (double)st[2 * i]; sq += (double)st[2 * i + 1]; }
+    __shared__ float2 res;
+    if (threadIdx.x < 64) {
+        const int cpg = a.q.C / a.q.groups, g = c / cpg;
+        const float *st = a.stats + ((long)n * a.q.C + g * cpg) * 2;
+        double s = 0.0, sq = 0.0;
+        for (int i = threadIdx.x; i < cpg; i += 64) { s += (double)st[2 * i]; sq += (double)st[2 * i + 1]; }
 #pragma unroll
-    for (int d = 32; d > 0; d >>= 1) { s += __shfl_xor(s, d, 64); sq += __shfl_xor(sq, d, 64); }
+        for (int d = 32; d > 0; d >>= 1) { s += __shfl_xor(s, d, 64); sq += __shfl_xor(sq, d, 64); }
+        moments_from_sums(s, sq, (double)cpg * (double)a.q.P, a.q.eps, mean, rstd);
+        if (threadIdx.x == 0) res = make_float2(mean, rstd);
+    }
     __syncthreads();
-    if ((threadIdx.x & 63) == 0) { redd[0][threadIdx.x >> 6] = s; redd[1][threadIdx.x >> 6] = sq; }
-    __syncthreads();
-    s = sq = 0.0;
-#pragma unroll
-    for (int i = 0; i < kGnThreads / 64; i++) { s += redd[0][i]; sq += redd[1][i]; }
-    moments_from_sums(s, sq, (double)cpg * (double)a.q.P, a.q.eps, mean, rstd);
+    mean = res.x; rstd = res.y;
 }
 
 template <typename T> __global__ void __launch_bounds__(kGnThreads) gn_fwd_kernel(GnArgs a)
 {
-    __shared__ float red[kGnThreads / 64];
-    const int n = blockIdx.x / a.q.C, c = blockIdx.x % a.q.C;
-    float mean, rstd;
-    group_moments_block(a, n, c, mean, rstd, red);
-    const float ga = a.gamma ? elem_to_f32<T>(reinterpret_cast<const T *>(a.gamma)[c]) : 1.f;
-    const float be = a.beta ? elem_to_f32<T>(reinterpret_cast<const T *>(a.beta)[c]) : 0.f;
-    const float sc = rstd * ga, sh = be - mean * sc;
-    const T *row = reinterpret_cast<const T *>(a.x) + (long)blockIdx.x * a.q.P;
-    T *out = reinterpret_cast<T *>(a.y) + (long)blockIdx.x * a.q.P;
-    constexpr int VEC = 16 / (int)sizeof(T);
-    if (a.q.P % VEC == 0 && reinterpret_cast<uintptr_t>(row) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0) {
-        for (int i = threadIdx.x; i < a.q.P / VEC; i += kGnThreads) {
-            const uint4 v = reinterpret_cast<const uint4 *>(row)[i];
-            const T *e = reinterpret_cast<const T *>(&v);
-            alignas(16) T o[VEC];
-#pragma unroll
-            for (int j = 0; j < VEC; j++) o[j] = f32_to_elem<T>(fmaf(elem_to_f32<T>(e[j]), sc, sh));
-            reinterpret_cast<uint4 *>(out)[i] = *reinterpret_cast<const uint4 *>(o);
-        }
-    } else {
-        for (int i = threadIdx.x; i < a.q.P; i += kGnThreads) out[i] = f32_to_elem<T>(fmaf(elem_to_f32<T>(row[i]), sc, sh));
-    }
+    const int row = (int)(blockIdx.x / (unsigned)a.pieces), piece = (int)blockIdx.x - row * a.pieces, n = row / a.q.C, c = row % a.q.C;
+    const T *const in[1] = {reinterpret_cast<const T *>(a.x) + (long)row * a.q.P};
+    map_piece<T, 1>(in, reinterpret_cast<T *>(a.y) + (long)row * a.q.P, a.q.P, piece, a.pieces, [&] {
+        float mean, rstd;
+        group_moments_block(a, n, c, mean, rstd);
+        const float ga = a.gamma ? elem_to_f32<T>(reinterpret_cast<const T *>(a.gamma)[c]) : 1.f;
+        const float be = a.beta ? elem_to_f32<T>(reinterpret_cast<const T *>(a.beta)[c]) : 0.f;
+        const float sc = rstd * ga, sh = be - mean * sc;
+        return [=](const float (&v)[1]) { return fmaf(v[0], sc, sh); };
+    });
 }
 
 template <typename T> __global__ void __launch_bounds__(kGnThreads) gn_bwd_reduce_kernel(GnArgs a)
@@ -189,10 +218,21 @@ template <typename T> __global__ void __launch_bounds__(kGnThreads) gn_bwd_reduc
     const T *gr = reinterpret_cast<const T *>(a.gy) + rowi * a.q.P;
     float r1 = 0.f, r2 = 0.f;
     constexpr int VEC = 16 / (int)sizeof(T);
-    if (a.q.P % VEC == 0 && reinterpret_cast<uintptr_t>(xr) % 16 == 0 && reinterpret_cast<uintptr_t>(gr) % 16 == 0) {
-        for (int i = threadIdx.x; i < a.q.P / VEC; i += kGnThreads) {
-            const uint4 xv = reinterpret_cast<const uint4 *>(xr)[i], gv = reinterpret_cast<const uint4 *>(gr)[i];
-            const T *xe = reinterpret_cast<const T *>(&xv), *ge = reinterpret_cast<const T *>(&gv);
+    const int nv = a.q.P / VEC;
+    // (a thread's vectors in the order of their addresses, kGnVectors of them requested at a time)
+    for (int i0 = threadIdx.x; i0 < nv; i0 += kGnThreads * kGnVectors) {
+        AnyVec<T> q[kGnVectors][2];
+#pragma unroll
+        for (int k = 0; k < kGnVectors; k++) {
+            const int i = i0 + k * kGnThreads;
+            q[k][0] = q[k][1] = AnyVec<T>{0u, 0u, 0u, 0u};
+            if (i < nv) { q[k][0] = load_any(xr + (long)i * VEC); q[k][1] = load_any(gr + (long)i * VEC); }
+        }
+#pragma unroll
+        for (int k = 0; k < kGnVectors; k++) {
+            if (i0 + k * kGnThreads >= nv) continue;
+            alignas(16) T xe[VEC], ge[VEC];
+            *reinterpret_cast<AnyVec<T> *>(xe) = q[k][0]; *reinterpret_cast<AnyVec<T> *>(ge) = q[k][1];
 #pragma unroll
             for (int j = 0; j < VEC; j++) {
                 const float g = elem_to_f32<T>(ge[j]);
@@ -200,12 +240,11 @@ template <typename T> __global__ void __launch_bounds__(kGnThreads) gn_bwd_reduc
                 r2 = fmaf(g, elem_to_f32<T>(xe[j]), r2);
             }
         }
-    } else {
-        for (int i = threadIdx.x; i < a.q.P; i += kGnThreads) {
-            const float g = elem_to_f32<T>(gr[i]);
-            r1 += g;
-            r2 = fmaf(g, elem_to_f32<T>(xr[i]), r2);
-        }
+    }
+    if ((int)threadIdx.x < a.q.P - nv * VEC) {
+        const float g = elem_to_f32<T>(gr[nv * VEC + threadIdx.x]);
+        r1 += g;
+        r2 = fmaf(g, elem_to_f32<T>(xr[nv * VEC + threadIdx.x]), r2);
     }
     r1 = block_sum(r1, red);
     r2 = block_sum(r2, red);
@@ -218,43 +257,28 @@ template <typename T> __global__ void __launch_bounds__(kGnThreads) gn_bwd_reduc
 template <typename T> __global__ void __launch_bounds__(kGnThreads) gn_bwd_apply_kernel(GnArgs a)
 {
     __shared__ float red[kGnThreads / 64];
-    const int n = blockIdx.x / a.q.C, c = blockIdx.x % a.q.C;
+    const int row = (int)(blockIdx.x / (unsigned)a.pieces), piece = (int)blockIdx.x - row * a.pieces, n = row / a.q.C, c = row % a.q.C;
     const int cpg = a.q.C / a.q.groups, g = c / cpg;
-    float mean, rstd;
-    group_moments_block(a, n, c, mean, rstd, red);
-    float A = 0.f, B = 0.f;
-    for (int i = threadIdx.x; i < cpg; i += kGnThreads) {
-        const int cc = g * cpg + i;
-        const float gm = a.gamma ? elem_to_f32<T>(reinterpret_cast<const T *>(a.gamma)[cc]) : 1.f;
-        const float r1 = a.part[((long)n * a.q.C + cc) * 2], r2 = a.part[((long)n * a.q.C + cc) * 2 + 1];
-        A = fmaf(gm, r1, A);
-        B = fmaf(gm, (r2 - mean * r1) * rstd, B);
-    }
-    A = block_sum(A, red);
-    B = block_sum(B, red);
-    const float m = (float)cpg * (float)a.q.P;
-    const float ga = a.gamma ? elem_to_f32<T>(reinterpret_cast<const T *>(a.gamma)[c]) : 1.f;
-    // grad_x = rstd * (ga * gy - A / m - xh * B / m) = c1 * gy + c2 * x + c3
-    const float c1 = rstd * ga, c2 = -rstd * rstd * B / m, c3 = -rstd * A / m - c2 * mean;
-    const T *xr = reinterpret_cast<const T *>(a.x) + (long)blockIdx.x * a.q.P;
-    const T *gr = reinterpret_cast<const T *>(a.gy) + (long)blockIdx.x * a.q.P;
-    T *out = reinterpret_cast<T *>(a.y) + (long)blockIdx.x * a.q.P;
-    constexpr int VEC = 16 / (int)sizeof(T);
-    if (a.q.P % VEC == 0 && reinterpret_cast<uintptr_t>(xr) % 16 == 0 && reinterpret_cast<uintptr_t>(gr) % 16 == 0
-        && reinterpret_cast<uintptr_t>(out) % 16 == 0) {
-        for (int i = threadIdx.x; i < a.q.P / VEC; i += kGnThreads) {
-            const uint4 xv = reinterpret_cast<const uint4 *>(xr)[i], gv = reinterpret_cast<const uint4 *>(gr)[i];
-            const T *xe = reinterpret_cast<const T *>(&xv), *ge = reinterpret_cast<const T *>(&gv);
-            alignas(16) T o[VEC];
-#pragma unroll
-            for (int j = 0; j < VEC; j++)
-                o[j] = f32_to_elem<T>(fmaf(c1, elem_to_f32<T>(ge[j]), fmaf(c2, elem_to_f32<T>(xe[j]), c3)));
-            reinterpret_cast<uint4 *>(out)[i] = *reinterpret_cast<const uint4 *>(o);
+    const T *const in[2] = {reinterpret_cast<const T *>(a.x) + (long)row * a.q.P, reinterpret_cast<const T *>(a.gy) + (long)row * a.q.P};
+    map_piece<T, 2>(in, reinterpret_cast<T *>(a.y) + (long)row * a.q.P, a.q.P, piece, a.pieces, [&] {
+        float mean, rstd;
+        group_moments_block(a, n, c, mean, rstd);
+        float A = 0.f, B = 0.f;
+        for (int i = threadIdx.x; i < cpg; i += kGnThreads) {
+            const int cc = g * cpg + i;
+            const float gm = a.gamma ? elem_to_f32<T>(reinterpret_cast<const T *>(a.gamma)[cc]) : 1.f;
+            const float r1 = a.part[((long)n * a.q.C + cc) * 2], r2 = a.part[((long)n * a.q.C + cc) * 2 + 1];
+            A = fmaf(gm, r1, A);
+            B = fmaf(gm, (r2 - mean * r1) * rstd, B);
         }
-    } else {
-        for (int i = threadIdx.x; i < a.q.P; i += kGnThreads)
-            out[i] = f32_to_elem<T>(fmaf(c1, elem_to_f32<T>(gr[i]), fmaf(c2, elem_to_f32<T>(xr[i]), c3)));
-    }
+        A = block_sum(A, red);
+        B = block_sum(B, red);
+        const float m = (float)cpg * (float)a.q.P;
+        const float ga = a.gamma ? elem_to_f32<T>(reinterpret_cast<const T *>(a.gamma)[c]) : 1.f;
+        // grad_x = rstd * (ga * gy - A / m - xh * B / m) = c1 * gy + c2 * x + c3
+        const float c1 = rstd * ga, c2 = -rstd * rstd * B / m, c3 = -rstd * A / m - c2 * mean;
+        return [=](const float (&v)[2]) { return fmaf(c1, v[1], fmaf(c2, v[0], c3)); };
+    });
 }
 
 // grad_gamma / grad_beta: one thread per channel, loop over the samples
@@ -300,7 +324,7 @@ extern "C" int d2c_channel_stats(const d2c_group_norm_desc *q, const void *x, fl
     if (int rc = check(q)) return rc;
     if (!x || !chan_stats) { d2c_set_error("null tensor pointer"); return D2C_ERR_SHAPE; }
     hipStream_t st = (hipStream_t)stream;
-    GnArgs a{*q, x, nullptr, chan_stats, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+    GnArgs a{*q, x, nullptr, chan_stats, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 1};
     GN_LAUNCH(channel_stats_kernel, dim3((unsigned)(q->N * q->C)), dim3(kGnThreads));
     return d2c_check_launch("channel_stats_kernel");
 }
@@ -311,8 +335,8 @@ extern "C" int d2c_group_norm_forward(const d2c_group_norm_desc *q, const void *
     if (int rc = check(q)) return rc;
     if (!x || !chan_stats || !y) { d2c_set_error("null tensor pointer"); return D2C_ERR_SHAPE; }
     hipStream_t st = (hipStream_t)stream;
-    GnArgs a{*q, x, nullptr, chan_stats, gamma, beta, y, nullptr, nullptr, nullptr};
-    GN_LAUNCH(gn_fwd_kernel, dim3((unsigned)(q->N * q->C)), dim3(kGnThreads));
+    GnArgs a{*q, x, nullptr, chan_stats, gamma, beta, y, nullptr, nullptr, nullptr, row_pieces(*q)};
+    GN_LAUNCH(gn_fwd_kernel, dim3((unsigned)(q->N * q->C) * (unsigned)a.pieces), dim3(kGnThreads));
     return d2c_check_launch("gn_fwd_kernel");
 }
 
@@ -334,11 +358,11 @@ extern "C" int d2c_group_norm_backward(const d2c_group_norm_desc *q, const void 
         return D2C_ERR_WORKSPACE;
     }
     hipStream_t st = (hipStream_t)stream;
-    GnArgs a{*q, x, grad_y, chan_stats, gamma, nullptr, grad_x, (float *)ws, grad_gamma, grad_beta};
+    GnArgs a{*q, x, grad_y, chan_stats, gamma, nullptr, grad_x, (float *)ws, grad_gamma, grad_beta, row_pieces(*q)};
     GN_LAUNCH(gn_bwd_reduce_kernel, dim3((unsigned)(q->N * q->C)), dim3(kGnThreads));
     if (int rc = d2c_check_launch("gn_bwd_reduce_kernel")) return rc;
     if (grad_x) {
-        GN_LAUNCH(gn_bwd_apply_kernel, dim3((unsigned)(q->N * q->C)), dim3(kGnThreads));
+        GN_LAUNCH(gn_bwd_apply_kernel, dim3((unsigned)(q->N * q->C) * (unsigned)a.pieces), dim3(kGnThreads));
         if (int rc = d2c_check_launch("gn_bwd_apply_kernel")) return rc;
     }
     if (grad_gamma || grad_beta) {
