@@ -1153,7 +1153,7 @@ struct ConvPrepArgs {
     // input -> channels-last rows, then zeros
     const bf16_t *x;
     bf16_t *xcl;
-    int C, vol, N, nbx, nby, nblk_x, wide, zrow_words;
+    int C, vol, N, nbx, nby, nblk_x, zrow_words;
     // weights: column tiles [step][tile][NT][KC]; back: the transposed product (columns = input channels)
     const bf16_t *w;
     uint4 *wt;
@@ -1163,7 +1163,7 @@ struct ConvPrepArgs {
     const bf16_t *gout;
     bf16_t *gcl;
     uint4 *gp;
-    int Cp, OBP, P, M, ngt, ngc, nblk_g, gwide, gp_wide;
+    int Cp, OBP, P, M, ngt, ngc, nblk_g, gp_wide;
     FastDiv dP;
     // bias gradient
     bf16_t *gb;
@@ -1177,8 +1177,6 @@ struct ConvPrepArgs {
     size_t zwords[2];
     int nblk_z;
 };
-// eight positions at a time: whole in a sample, and aligned
-inline int wide_gout(const void *gout, int P) { return P % 8 == 0 && reinterpret_cast<uintptr_t>(gout) % 16 == 0; }
 
 __global__ void __launch_bounds__(256) conv_prepare_kernel(ConvPrepArgs a)
 {
@@ -1192,24 +1190,17 @@ __global__ void __launch_bounds__(256) conv_prepare_kernel(ConvPrepArgs a)
         const bf16_t *xb = a.x + (long)n * a.C * a.vol;
         bf16_t *ob = a.xcl + (long)n * a.C * a.vol;
         if (b == 0 && (int)threadIdx.x < a.zrow_words) reinterpret_cast<unsigned *>(a.xcl + (long)a.N * a.C * a.vol)[threadIdx.x] = 0u;
-        if (a.wide) {
-            for (int i = threadIdx.x; i < 512; i += 256) {
-                const int c = c0 + i / 8, v = v0 + (i % 8) * 8;
-                if (v < a.vol) {
-                    const uint4 q = *reinterpret_cast<const uint4 *>(xb + (long)c * a.vol + v);
-                    const unsigned u[4] = {q.x, q.y, q.z, q.w};
-                    bf16_t *t = s_t + ((i % 8) * 8) * RS + i / 8;
+        for (int i = threadIdx.x; i < 512; i += 256) {
+            const int c = c0 + i / 8, v = v0 + (i % 8) * 8;
+            if (v < a.vol) {
+                const uint4 q = load_run<bf16_t>(xb + (long)c * a.vol + v, a.vol - v);
+                const unsigned u[4] = {q.x, q.y, q.z, q.w};
+                bf16_t *t = s_t + ((i % 8) * 8) * RS + i / 8;
 #pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        t[(2 * e) * RS] = (bf16_t)(u[e] & 0xffffu);
-                        t[(2 * e + 1) * RS] = (bf16_t)(u[e] >> 16);
-                    }
+                for (int e = 0; e < 4; e++) {
+                    t[(2 * e) * RS] = (bf16_t)(u[e] & 0xffffu);
+                    t[(2 * e + 1) * RS] = (bf16_t)(u[e] >> 16);
                 }
-            }
-        } else {
-            for (int i = threadIdx.x; i < 4096; i += 256) {
-                const int c = i / 64, v = i % 64;
-                if (v0 + v < a.vol) s_t[v * RS + c] = xb[(long)(c0 + c) * a.vol + v0 + v];
             }
         }
         __syncthreads();
@@ -1252,24 +1243,29 @@ __global__ void __launch_bounds__(256) conv_prepare_kernel(ConvPrepArgs a)
         // 64 positions x 64 channels of grad_out, into both orders
         const int gt = b % a.ngt, gc = b / a.ngt;
         constexpr int GS = 72;                               // [channel][position], 16-byte aligned rows
-        if (a.gwide) {
-            for (int i = threadIdx.x; i < 512; i += 256) {
-                const int c = gc * 64 + i / 8, m = gt * 64 + (i % 8) * 8;
-                uint4 v = make_uint4(0, 0, 0, 0);
-                if (c < a.Cout && m < a.M) {
-                    const int n = fdiv(m, a.dP), p = m - n * a.P;
-                    v = *reinterpret_cast<const uint4 *>(a.gout + ((long)n * a.Cout + c) * a.P + p);
-                }
-                *reinterpret_cast<uint4 *>(s_t + (i / 8) * GS + (i % 8) * 8) = v;
-            }
-        } else for (int i = threadIdx.x; i < 4096; i += 256) {
-            const int c = gc * 64 + i / 64, m = gt * 64 + i % 64;
-            bf16_t v = 0;
+        for (int i = threadIdx.x; i < 512; i += 256) {
+            const int c = gc * 64 + i / 8, m = gt * 64 + (i % 8) * 8;
+            uint4 v = make_uint4(0, 0, 0, 0);
             if (c < a.Cout && m < a.M) {
                 const int n = fdiv(m, a.dP), p = m - n * a.P;
-                v = a.gout[((long)n * a.Cout + c) * a.P + p];
+                const bf16_t *const src = a.gout + ((long)n * a.Cout + c) * a.P + p;
+                if (p + 8 <= a.P) {
+                    v = __builtin_bit_cast(uint4, load_any<bf16_t>(src));
+                } else {
+                    // (the rows of a channel in the next samples are Cout * P apart)
+                    alignas(16) bf16_t e[8];
+                    long at = 0;
+                    int r = p;
+#pragma unroll
+                    for (int q = 0; q < 8; q++) {
+                        e[q] = m + q < a.M ? src[at] : (bf16_t)0;
+                        at++;
+                        if (++r == a.P) { r = 0; at += (long)(a.Cout - 1) * a.P; }
+                    }
+                    v = *reinterpret_cast<const uint4 *>(e);
+                }
             }
-            s_t[(i / 64) * GS + i % 64] = v;
+            *reinterpret_cast<uint4 *>(s_t + (i / 8) * GS + (i % 8) * 8) = v;
         }
         __syncthreads();
         if (a.gp) {
@@ -1436,7 +1432,6 @@ void prep_input(ConvPrepArgs &a, const d2c_conv3d_desc &q, const void *x, void *
     const int vol = q.D * q.H * q.W;
     a.x = (const bf16_t *)x; a.xcl = (bf16_t *)xcl; a.C = q.Cin; a.vol = vol; a.N = q.N; a.zrow_words = zrow_words;
     a.nbx = (vol + 63) / 64; a.nby = q.Cin / 64; a.nblk_x = a.nbx * a.nby * q.N;
-    a.wide = vol % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
 }
 void prep_weights(ConvPrepArgs &a, const d2c_conv3d_desc &q, const RowsPlan &p, const void *w, void *wt, bool back)
 {
@@ -1542,7 +1537,7 @@ int d2c_brick_bwd_prepare(const d2c_conv3d_desc &q, const void *gout, const void
     }
     a.gout = (const bf16_t *)gout; a.gp = (uint4 *)goutp; a.gp_wide = 1;
     a.Cp = p.Cp; a.OBP = p.Cp / 32; a.P = P; a.M = M; a.dP = make_fastdiv(P);
-    a.gwide = wide_gout(gout, P); a.ngt = (M + 127) / 128 * 2; a.ngc = p.Cp / 64; a.nblk_g = col_ws || goutp ? a.ngt * a.ngc : 0;
+    a.ngt = (M + 127) / 128 * 2; a.ngc = p.Cp / 64; a.nblk_g = col_ws || goutp ? a.ngt * a.ngc : 0;
     a.gb = (bf16_t *)gb; a.nblk_b = gb ? q.Cout : 0;
     prep_zero(a, 0, zero0, zero0_bytes);
     prep_zero(a, 1, zero1, zero1_bytes);
@@ -1695,7 +1690,6 @@ int d2c_plain_backward(const d2c_conv3d_desc &q, const void *gout, const void *x
         a.gcl = gx ? (bf16_t *)(base + l.gcl) : nullptr;
         a.gp = gw ? (uint4 *)(base + l.gp) : nullptr;
         a.Cp = Cp; a.OBP = p.OBP; a.P = P; a.M = M; a.dP = make_fastdiv(P);
-        a.gwide = wide_gout(gout, P);
         a.ngt = (M + 63) / 64;
         a.ngc = std::max((Cp + 63) / 64, (p.OBP + 1) / 2);
         a.nblk_g = (gx || gw) ? a.ngt * a.ngc : 0;

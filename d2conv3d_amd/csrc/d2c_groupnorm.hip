@@ -44,13 +44,8 @@ D2C_DEV float block_sum(float v, float *red)
     return t;
 }
 
-typedef unsigned int u32x4_by2 __attribute__((ext_vector_type(4), aligned(2)));
-typedef unsigned int u32x4_by4 __attribute__((ext_vector_type(4), aligned(4)));
-// (vectors of a type that says how they are aligned: rows of any length, one load or store each)
-template <typename T> using AnyVec = typename std::conditional<sizeof(T) == 2, u32x4_by2, u32x4_by4>::type;
-template <typename T> D2C_DEV AnyVec<T> load_any(const T *p) { return *reinterpret_cast<const AnyVec<T> *>(p); }
 // out[i] = f(in[0][i], ...) for a piece of a row, f = make().  Bound: memory; a thread requests up to kGnVectors vectors of each row, then works
-// out f (sums over a group, double).  Few rows are several workgroups each: four to a compute unit in all, since each works out f.(One workgroup
+// out f (sums over a group, double).  Few rows are several workgroups each: four to a compute unit in all, since each works out f.  (One workgroup
 // to a row, a vector at a time, rows of odd lengths element by element; us, before and after, forward and gradient, bfloat16: 256 rows of 51360
 // 19.6, 11.4 and 21.1, 15.0; of 51361 62, 13 and 74, 17; 1024 rows of 12960 12.3, 11.4 and 15.7, 14.9; float32 21.3, 17.3 and 25.8, 24.8; 55.8, 17.4 and
 // 59.8, 24.7; 64 rows of 50 3.4, 3.6.)

@@ -48,9 +48,43 @@ D2C_DEV uint32_t pack_bf16x2(float lo, float hi)
     return __builtin_bit_cast(uint32_t, r);
 }
 
+// 16 bytes of a type that says how they are aligned: one load or store each, wherever a row of elements starts.  The layout kernels move
+// rows of odd lengths this way too (element by element before; us, 256 -> 256 channels on 7x59x107, bfloat16: preparations of a training
+// step 69, 48, grad_input 25.8, 17.8; float32 94, 77 and 28, 19, grad_out's terms 38, 27; on 7x60x104, where rows are aligned, 45, 15, 71, 16.5, 22).
+typedef unsigned int u32x4_by2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef unsigned int u32x4_by4 __attribute__((ext_vector_type(4), aligned(4)));
+template <typename T> using AnyVec = typename std::conditional<sizeof(T) == 2, u32x4_by2, u32x4_by4>::type;
+template <typename T> D2C_DEV AnyVec<T> load_any(const T *p) { return *reinterpret_cast<const AnyVec<T> *>(p); }
+// ... of a row that ends after `left` (> 0) elements: zeros behind them, nothing stored there
+template <typename T> D2C_DEV uint4 load_run(const T *p, int left)
+{
+    constexpr int VEC = 16 / (int)sizeof(T);
+    alignas(16) T e[VEC];
+    if (left >= VEC) {
+        *reinterpret_cast<AnyVec<T> *>(e) = load_any(p);
+    } else {
+#pragma unroll
+        for (int i = 0; i < VEC; i++) e[i] = i < left ? p[i] : (T)0;
+    }
+    return *reinterpret_cast<const uint4 *>(e);
+}
+template <typename T> D2C_DEV void store_run(T *p, const uint4 &v, int left)
+{
+    constexpr int VEC = 16 / (int)sizeof(T);
+    alignas(16) T e[VEC];
+    *reinterpret_cast<uint4 *>(e) = v;
+    if (left >= VEC) {
+        *reinterpret_cast<AnyVec<T> *>(p) = *reinterpret_cast<const AnyVec<T> *>(e);
+    } else {
+#pragma unroll
+        for (int i = 0; i < VEC; i++)
+            if (i < left) p[i] = e[i];
+    }
+}
+
 // in [rows][cols] -> out [cols][rows], float32: a 64 x 64 tile through LDS with 16-byte accesses on both sides, by 256 threads
 // (the 4-byte accesses of 32 x 32 tiles keep a quarter of the bytes in flight: 2 x 256 x 12960 elements of grad_input 16 us, 9);
-// rows and cols are multiples of 4, both tensors 16-byte aligned.  (Bank of an element: row stride 65 words, so that 16 vectors x 4 rows
+// rows and tensors of any length and alignment.  (Bank of an element: row stride 65 words, so that 16 vectors x 4 rows
 // meet 64 banks either way.)
 constexpr int kTransposeLds = 64 * 65 * 4;             // [column][row]
 D2C_DEV void transpose_tile64(float *tile, const float *in, float *out, int rows, int cols, int r0, int c0)
@@ -59,7 +93,7 @@ D2C_DEV void transpose_tile64(float *tile, const float *in, float *out, int rows
     for (int k = 0; k < 4; k++) {                      // 64 rows x 16 vectors of 4 columns
         const int i = k * 256 + threadIdx.x, r = r0 + i / 16, c = c0 + (i % 16) * 4;
         if (r < rows && c < cols) {
-            const float4 q = *reinterpret_cast<const float4 *>(in + (long)r * cols + c);
+            const float4 q = __builtin_bit_cast(float4, load_run<float>(in + (long)r * cols + c, cols - c));
             float *t = tile + (i % 16) * 4 * 65 + i / 16;
             t[0] = q.x; t[65] = q.y; t[130] = q.z; t[195] = q.w;
         }
@@ -70,7 +104,7 @@ D2C_DEV void transpose_tile64(float *tile, const float *in, float *out, int rows
         const int i = k * 256 + threadIdx.x, c = c0 + i / 16, r = r0 + (i % 16) * 4;
         if (r < rows && c < cols) {
             const float *t = tile + (i / 16) * 65 + (i % 16) * 4;
-            *reinterpret_cast<float4 *>(out + (long)c * rows + r) = make_float4(t[0], t[1], t[2], t[3]);
+            store_run<float>(out + (long)c * rows + r, __builtin_bit_cast(uint4, make_float4(t[0], t[1], t[2], t[3])), rows - r);
         }
     }
 }

@@ -174,15 +174,15 @@ template <typename T> D2C_DEV void pack_tile32(const T *xb, T *ob, int C, int vo
 }
 
 // The same for bfloat16 with 16-byte accesses on both sides (2-byte accesses of 32 lanes move 64 bytes per
-// request): a 64 x 64 element tile; needs vol and C to be multiples of 8 and 16-byte aligned tensors.
+// request): a 64 x 64 element tile; needs C to be a multiple of 8 and a 16-byte aligned `ob`.
 D2C_DEV void pack_tile64_bf16(const bf16_t *xb, bf16_t *ob, int C, int vol, int v0, int c0)
 {
     constexpr int RS = 66;                             // LDS row stride in elements (33 words)
     __shared__ bf16_t tile[64 * RS];                   // [v][c]
     for (int i = threadIdx.x; i < 512; i += 256) {     // 64 channels x 8 vectors of 8 positions
         const int c = c0 + i / 8, v = v0 + (i % 8) * 8;
-        if (c < C && v < vol) {                        // (vol % 8 == 0: the vector is inside or outside as a whole)
-            const uint4 q = *reinterpret_cast<const uint4 *>(xb + (long)c * vol + v);
+        if (c < C && v < vol) {
+            const uint4 q = load_run<bf16_t>(xb + (long)c * vol + v, vol - v);
             const unsigned u[4] = {q.x, q.y, q.z, q.w};
             bf16_t *t = tile + ((i % 8) * 8) * RS + i / 8;
 #pragma unroll
@@ -467,8 +467,7 @@ int pack_input(const TiledShape &s, const void *x, void *xcl, hipStream_t st, bo
     dim3 grid((s.vol + 31) / 32, (s.Cin + 31) / 32, s.N);
     D2cProfScope prof(D2C_PROF_PACK, st);
     if constexpr (sizeof(T) == 2) {
-        if (s.vol % 8 == 0 && s.Cin % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
-            reinterpret_cast<uintptr_t>(xcl) % 16 == 0) {
+        if (s.Cin % 8 == 0 && reinterpret_cast<uintptr_t>(xcl) % 16 == 0) {
             hipLaunchKernelGGL(pack_input_bf16_kernel, dim3((s.vol + 63) / 64, (s.Cin + 63) / 64, s.N), dim3(256), 0, st,
                                (const bf16_t *)x, (bf16_t *)xcl, s.Cin, s.vol, (int)zero_row);
             return d2c_check_launch("pack_input_bf16_kernel");
@@ -483,8 +482,7 @@ template <typename T> void prep_pack(PrepArgs::Pack &pk, const void *src, void *
 {
     pk.src = src; pk.dst = dst; pk.C = C; pk.vol = vol;
     constexpr int V = 16 / (int)sizeof(T);
-    pk.wide = vol % V == 0 && C % V == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0 &&
-              reinterpret_cast<uintptr_t>(dst) % 16 == 0;
+    pk.wide = C % V == 0 && reinterpret_cast<uintptr_t>(dst) % 16 == 0;
     // (float32: where large tiles give every compute unit one; below, the small ones are no slower and their kernel holds less code:
     // 64 x 1400 elements 18.3 us, 18.1 of a forward call)
     if (sizeof(T) == 4 && (long)((vol + 63) / 64) * ((C + 63) / 64) * N < 256) pk.wide = 0;

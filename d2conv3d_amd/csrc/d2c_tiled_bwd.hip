@@ -1724,7 +1724,7 @@ D2C_DEV void split3(float v0, float v1, float v2, float v3, uint2 &h, uint2 &m, 
 // positions per tile of kWMT): lh[i] = (l0 l1)(l2 l3)(h0 h1)(h2 h3) of the lane's four positions, md[i] = (m0 m1)(m2 m3);
 // `md` follows the `total` 16-byte entries of `lh`
 __global__ void __launch_bounds__(256) pack_gout3_kernel(const float *gout, uint4 *lh, TiledShape s, int ntile, int OBT,
-                                                         long total, bool vec)
+                                                         long total)
 {
     constexpr int VEC = 4, NKGT = kWMT / (2 * VEC);
     uint2 *md = reinterpret_cast<uint2 *>(lh + total);
@@ -1738,17 +1738,22 @@ __global__ void __launch_bounds__(256) pack_gout3_kernel(const float *gout, uint
         const int ol = ob * 32 + (lane & 31);
         const long m0 = (long)tile * kWMT + (2 * kg + (lane >> 5)) * VEC;
         float v[VEC] = {0.f, 0.f, 0.f, 0.f};
-        if (vec && ol < s.og && m0 < s.M) {          // (four positions of one sample, as one load)
+        if (ol < s.og && m0 < s.M) {
             const int b = (int)(m0 / s.P), pp = (int)(m0 - (long)b * s.P);
-            const float4 t = *reinterpret_cast<const float4 *>(gout + ((long)b * s.Cout + wg * s.og + ol) * s.P + pp);
-            v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
-        }
+            const float *const src = gout + ((long)b * s.Cout + wg * s.og + ol) * s.P + pp;
+            if (pp + VEC <= s.P) {                   // (four positions of one sample, as one load)
+                const float4 t = __builtin_bit_cast(float4, load_any<float>(src));
+                v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+            } else {
+                // (... of several samples, whose rows of this channel are Cout * P apart)
+                long at = 0;
+                int p = pp;
 #pragma unroll
-        for (int q = 0; q < VEC; q++) {
-            const long mm = m0 + q;
-            if (!vec && ol < s.og && mm < s.M) {
-                const int b = (int)(mm / s.P), pp = (int)(mm - (long)b * s.P);
-                v[q] = gout[((long)b * s.Cout + wg * s.og + ol) * s.P + pp];
+                for (int q = 0; q < VEC; q++) {
+                    if (m0 + q < s.M) v[q] = src[at];
+                    at++;
+                    if (++p == s.P) { p = 0; at += (long)(s.Cout - 1) * s.P; }
+                }
             }
         }
         uint2 h, m, l;
@@ -2059,8 +2064,7 @@ __global__ void __launch_bounds__(256) unpack_grad_input_kernel(const float *gxc
     }
 }
 
-// The same for bfloat16 with 16-byte accesses on both sides: 64 x 64 element tiles; needs vol and C to be
-// multiples of 8 and a 16-byte aligned grad_input.
+// The same for bfloat16 with 16-byte accesses on both sides: 64 x 64 element tiles; needs C to be a multiple of 4.
 __global__ void __launch_bounds__(256) unpack_grad_input_bf16_kernel(const float *gxcl, bf16_t *gx, int C, int vol)
 {
     constexpr int RS = 66;                             // LDS row stride in elements (33 words)
@@ -2081,7 +2085,7 @@ __global__ void __launch_bounds__(256) unpack_grad_input_bf16_kernel(const float
         const int c = c0 + i / 8, v = v0 + (i % 8) * 8;
         if (c < C && v < vol) {
             const unsigned *t = reinterpret_cast<const unsigned *>(tile + (i / 8) * RS + (i % 8) * 8);
-            *reinterpret_cast<uint4 *>(ob + (long)c * vol + v) = make_uint4(t[0], t[1], t[2], t[3]);
+            store_run<bf16_t>(ob + (long)c * vol + v, make_uint4(t[0], t[1], t[2], t[3]), vol - v);
         }
     }
 }
@@ -2486,7 +2490,7 @@ int d2c_tiled_bwd_weight_launch(const TiledShape &s, const void *gout, const voi
         D2cProfScope prof(D2C_PROF_PACK, st);
         if (!(phase & 8)) d2c_fill_zero(gwacc, (size_t)nw * sizeof(float), st);
         hipLaunchKernelGGL(pack_gout3_kernel, dim3(grid1d(total, 16384)), dim3(256), 0, st, (const float *)gout,
-                           (uint4 *)goutp, s, ntp, OBT, total, s.P % 4 == 0 && reinterpret_cast<uintptr_t>(gout) % 16 == 0);
+                           (uint4 *)goutp, s, ntp, OBT, total);
         if (int rc = d2c_check_launch("pack_gout3_kernel")) return rc;
     } else if (phase & 1) {
         D2cProfScope prof(D2C_PROF_PACK, st);
@@ -2606,12 +2610,12 @@ int d2c_tiled_unpack_gx(const TiledShape &s, const float *gxcl, void *gx, hipStr
     dim3 grid((s.vol + 31) / 32, (s.Cin + 31) / 32, s.N);
     D2cProfScope prof(D2C_PROF_PACK, st);
     if constexpr (sizeof(T) == 2) {
-        if (s.vol % 8 == 0 && s.Cin % 8 == 0 && reinterpret_cast<uintptr_t>(gx) % 16 == 0) {
+        if (s.Cin % 4 == 0) {
             hipLaunchKernelGGL(unpack_grad_input_bf16_kernel, dim3((s.vol + 63) / 64, (s.Cin + 63) / 64, s.N), dim3(256), 0,
                                st, gxcl, (bf16_t *)gx, s.Cin, s.vol);
             return d2c_check_launch("unpack_grad_input_bf16_kernel");
         }
-    } else if (s.vol % 4 == 0 && s.Cin % 4 == 0 && reinterpret_cast<uintptr_t>(gx) % 16 == 0) {
+    } else if (s.Cin % 4 == 0) {
         hipLaunchKernelGGL(unpack_grad_input_f32_kernel, dim3((s.vol + 63) / 64, (s.Cin + 63) / 64, s.N), dim3(256), 0, st, gxcl,
                            (float *)gx, s.Cin, s.vol);
         return d2c_check_launch("unpack_grad_input_f32_kernel");
