@@ -395,10 +395,12 @@ __global__ void __launch_bounds__(kThreadsDw) dwc_bias_grad_kernel(DwcShape s, c
 }
 
 // ---------------------------------------------------------------- marching kernels
-// A workgroup = one (sample, channel), kTY * kMR rows, kTX * kVW columns, a range of planes.  What bounds them is the vector
-// ALU (27 and 54 products to an element at a quarter of the lanes per clock), then memory: 2x256x8x56x56 float moves 103 MB
-// forward, 154 MB backward (20 and 30 us at the rate of a large copy) and takes 24 and 46.  With all taps of every plane it took 30
-// and 59; rows of any width are read in vectors (2x128x8x60x107: 48 and 76 us element by element, 30 and 63).
+// A workgroup = one (sample, channel), kTY * kMR rows, kTX * kVW columns, a range of planes.  What bounds them is memory, and close behind
+// it the vector ALU (27 and 54 products to an element at a quarter of the lanes per clock): 2x256x8x56x56 float moves 103 MB
+// forward, 154 MB backward (20 and 30 us at the rate of a large copy) and takes 21 and 32.  With all taps of every plane it took 30
+// and 59, with those of its planes 24 and 45; the rest were registers moved from plane to plane, cleared and branched around in front of every load, and
+// sums of the workgroup through LDS, 350 of 878 instructions.  bfloat16 25 and 59, 21 and 30; rows that are not vectors, 1x256x7x59x107: float 28 and
+// 50, 27 and 39, bfloat16 41 and 91, 25 and 38.
 constexpr int kMR = 2;                          // rows per thread
 constexpr int kMTaps = 28;                      // 27 taps and the bias
 struct MarchTiles {
@@ -418,50 +420,15 @@ MarchTiles march_tiles(const d2c_dwconv3d_desc &q)
 bool march_ok(const d2c_dwconv3d_desc &q)
 {
     return q.dtype != D2C_F64 && q.Cout == q.C && q.kd == 3 && q.kh == 3 && q.kw == 3 && q.sd == 1 && q.sh == 1 && q.sw == 1 &&
-           q.pd == 1 && q.ph == 1 && q.pw == 1 && q.dd == 1 && q.dh == 1 && q.dw == 1;
+           q.pd == 1 && q.ph == 1 && q.pw == 1 && q.dd == 1 && q.dh == 1 && q.dw == 1 &&
+           (long)q.D * q.H * q.W * 4 < (1l << 31);        // (a channel through 32-bit offsets)
 }
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 typedef unsigned short u16x4_any __attribute__((ext_vector_type(4), aligned(2)));
-// kVW elements of a row of `width` from x0 on, zeros outside it.  VEC: rows kVW-aligned in memory, whole groups.
-template <typename ST, bool VEC> D2C_DEV void march_load(const ST *row, int x0, int width, bool ok, float *m)
-{
-    if constexpr (VEC) {
-        m[0] = m[1] = m[2] = m[3] = 0.f;
-        if (ok && x0 < width) {
-            if constexpr (sizeof(ST) == 4) {
-                const float4 t = *reinterpret_cast<const float4 *>(row + x0);
-                m[0] = t.x; m[1] = t.y; m[2] = t.z; m[3] = t.w;
-            } else {
-                const uint2 t = *reinterpret_cast<const uint2 *>(row + x0);
-                m[0] = __uint_as_float(t.x << 16); m[1] = __uint_as_float(t.x & 0xffff0000u);
-                m[2] = __uint_as_float(t.y << 16); m[3] = __uint_as_float(t.y & 0xffff0000u);
-            }
-        }
-    } else {
-        m[0] = m[1] = m[2] = m[3] = 0.f;
-        if (ok && x0 + kVW <= width) {
-            // (one load all the same, of a type that says how it is aligned)
-            if constexpr (sizeof(ST) == 4) {
-                const f32x4_any t = *reinterpret_cast<const f32x4_any *>(row + x0);
-                m[0] = t[0]; m[1] = t[1]; m[2] = t[2]; m[3] = t[3];
-            } else {
-                const u16x4_any t = *reinterpret_cast<const u16x4_any *>(row + x0);
-                m[0] = bf16_to_f32(t[0]); m[1] = bf16_to_f32(t[1]); m[2] = bf16_to_f32(t[2]); m[3] = bf16_to_f32(t[3]);
-            }
-        } else if (ok && x0 < width) {
-#pragma unroll
-            for (int i = 0; i < kVW - 1; i++)
-                if (x0 + i < width) m[i] = ldv<ST>(row, x0 + i);
-        }
-    }
-}
 template <typename ST, bool VEC> D2C_DEV void march_store(ST *row, int x0, int width, const float *m)
 {
-    if constexpr (VEC) {
-        if (x0 >= width) return;
-        if constexpr (sizeof(ST) == 4) *reinterpret_cast<float4 *>(row + x0) = make_float4(m[0], m[1], m[2], m[3]);
-        else *reinterpret_cast<uint2 *>(row + x0) = make_uint2(pack_bf16x2(m[0], m[1]), pack_bf16x2(m[2], m[3]));
-    } else if (x0 + kVW <= width) {
+    static_assert(!VEC, "see march_put");
+    if (x0 + kVW <= width) {
         if constexpr (sizeof(ST) == 4) *reinterpret_cast<f32x4_any *>(row + x0) = f32x4_any{m[0], m[1], m[2], m[3]};
         else {
             const uint32_t a = pack_bf16x2(m[0], m[1]), b = pack_bf16x2(m[2], m[3]);
@@ -473,26 +440,87 @@ template <typename ST, bool VEC> D2C_DEV void march_store(ST *row, int x0, int w
             if (x0 + i < width) stv<ST>(row, x0 + i, m[i]);
     }
 }
-// One plane's rows y0 - 1 .. y0 + kMR of a thread, as they come from memory ...
-struct MarchRows {
-    float m[kMR + 2][kVW];
-    float l[kMR + 2], r[kMR + 2];               // the elements beside the tile (its first and last lane)
+// Rows are read through a buffer descriptor of what is left of the channel from a plane on.  What lies outside the volume has an offset
+// past the descriptor's end and is zero, without a branch and without registers cleared in front of the load; what a vector brings from
+// behind its row is cleared afterwards (not VEC).  bfloat16 rows that are not vectors: the words around their elements, shifted; the descriptor begins and
+// ends with a whole word then, `skip` bytes in front of the plane.
+constexpr unsigned kMarchNone = 0x80000000u;
+template <typename ST, bool VEC> struct MarchPlane {
+    decltype(__builtin_amdgcn_make_buffer_rsrc((void *)nullptr, 0, 0, 0)) rs;
+    unsigned skip;
+    D2C_DEV MarchPlane(const ST *channel, int z, long HW, int D, bool ok)
+    {
+        const bool in = ok && z >= 0 && z < D;
+        const uintptr_t at = reinterpret_cast<uintptr_t>(channel + (in ? z : 0) * HW);
+        const long bytes = (D - z) * HW * (long)sizeof(ST);
+        skip = sizeof(ST) == 2 && !VEC ? (unsigned)(at & 2) : 0u;
+        rs = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(at - skip), 0,
+                                               in ? (int)(sizeof(ST) == 2 && !VEC ? (bytes + skip + 3) & ~3l : bytes) : 0, 0x00020000);
+    }
 };
-// (EDGE: more than one tile along x)
-template <typename ST, bool VEC, bool EDGE>
-D2C_DEV void march_rows(const ST *plane, bool plane_ok, int y0, int x0, int H, int W, MarchRows &o)
+// byte offsets in a plane of a thread's rows y0 - 1 .. y0 + kMR, and of the element beside the tile (of its first and last lane)
+struct MarchOffsets {
+    unsigned o[kMR + 2], e[kMR + 2];
+};
+template <typename ST, bool EDGE> D2C_DEV MarchOffsets march_offsets(int y0, int x0, int H, int W)
 {
     const int tx = threadIdx.x % kTX;
+    const int beside = tx == 0 ? x0 - 1 : (tx == kTX - 1 && x0 + kVW < W ? x0 + kVW : -1);
+    MarchOffsets r;
 #pragma unroll
     for (int j = 0; j < kMR + 2; j++) {
         const int y = y0 - 1 + j;
-        const bool ok = plane_ok && y >= 0 && y < H;
-        const ST *row = plane + (long)(ok ? y : 0) * W;
-        march_load<ST, VEC>(row, x0, W, ok, o.m[j]);
-        if constexpr (EDGE) {
-            o.l[j] = (ok && tx == 0 && x0 > 0) ? ldv<ST>(row, x0 - 1) : 0.f;
-            o.r[j] = (ok && tx == kTX - 1 && x0 + kVW < W) ? ldv<ST>(row, x0 + kVW) : 0.f;
+        const bool ok = y >= 0 && y < H;
+        r.o[j] = ok && x0 < W ? (unsigned)((y * W + x0) * (int)sizeof(ST)) : kMarchNone;
+        if constexpr (EDGE) r.e[j] = ok && beside >= 0 ? (unsigned)((y * W + beside) * (int)sizeof(ST)) : kMarchNone;
+    }
+    return r;
+}
+// kVW elements from byte `o` of a plane on, the first of them element x0 of its row
+template <typename ST, bool VEC> D2C_DEV void march_load(const MarchPlane<ST, VEC> &p, unsigned o, int x0, int width, float *m)
+{
+    if constexpr (sizeof(ST) == 4) {
+        const auto t = __builtin_amdgcn_raw_buffer_load_b128(p.rs, (int)o, 0, 0);
+#pragma unroll
+        for (int i = 0; i < kVW; i++) m[i] = __uint_as_float(t[i]);
+    } else {
+        unsigned lo, hi;
+        if constexpr (VEC) {
+            const auto t = __builtin_amdgcn_raw_buffer_load_b64(p.rs, (int)o, 0, 0);
+            lo = t[0]; hi = t[1];
+        } else {
+            const unsigned at = o + p.skip;
+            const auto t = __builtin_amdgcn_raw_buffer_load_b96(p.rs, (int)(at & ~3u), 0, 0);
+            lo = __builtin_amdgcn_alignbit(t[1], t[0], (at & 2u) * 8u); hi = __builtin_amdgcn_alignbit(t[2], t[1], (at & 2u) * 8u);
         }
+        m[0] = __uint_as_float(lo << 16); m[1] = __uint_as_float(lo & 0xffff0000u);
+        m[2] = __uint_as_float(hi << 16); m[3] = __uint_as_float(hi & 0xffff0000u);
+    }
+    if constexpr (!VEC) {
+#pragma unroll
+        for (int i = 1; i < kVW; i++) m[i] = x0 + i < width ? m[i] : 0.f;
+        // (shifted, the first element of a vector outside the volume is one of nothing: zero already)
+    }
+}
+template <typename ST, bool VEC> D2C_DEV float march_element(const MarchPlane<ST, VEC> &p, unsigned o)
+{
+    if constexpr (sizeof(ST) == 4) return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(p.rs, (int)o, 0, 0));
+    else return __uint_as_float((unsigned)(unsigned short)__builtin_amdgcn_raw_buffer_load_b16(p.rs, (int)(o + p.skip), 0, 0) << 16);
+}
+// One plane's rows y0 - 1 .. y0 + kMR of a thread, as they come from memory ...
+struct MarchRows {
+    float m[kMR + 2][kVW];
+    float e[kMR + 2];                           // the element beside the tile (its first and last lane)
+};
+// (EDGE: more than one tile along x)
+template <typename ST, bool VEC, bool EDGE>
+D2C_DEV void march_rows(const ST *channel, int z, bool plane_ok, const MarchOffsets &f, const d2c_dwconv3d_desc &q, int x0, MarchRows &o)
+{
+    const MarchPlane<ST, VEC> p(channel, z, (long)q.H * q.W, q.D, plane_ok);
+#pragma unroll
+    for (int j = 0; j < kMR + 2; j++) {
+        march_load<ST, VEC>(p, f.o[j], x0, q.W, o.m[j]);
+        if constexpr (EDGE) o.e[j] = march_element<ST, VEC>(p, f.e[j]);
     }
 }
 // ... and row j with its neighbours along x: v[i] is element x0 - 1 + i.  (The 16 lanes of a row are one DPP row.)
@@ -502,9 +530,32 @@ template <bool EDGE> D2C_DEV void march_segment(const MarchRows &o, int j, float
     const float left = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(o.m[j][3]), 0x111, 0xF, 0xF, true));    // row_shr 1
     const float right = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(o.m[j][0]), 0x101, 0xF, 0xF, true));   // row_shl 1
     // (a lane without a neighbour in its row of 16 gets zero)
-    v[0] = EDGE && tx == 0 ? o.l[j] : left;
+    v[0] = EDGE && tx == 0 ? o.e[j] : left;
     v[1] = o.m[j][0]; v[2] = o.m[j][1]; v[3] = o.m[j][2]; v[4] = o.m[j][3];
-    v[5] = EDGE && tx == kTX - 1 ? o.r[j] : right;
+    v[5] = EDGE && tx == kTX - 1 ? o.e[j] : right;
+}
+// rows y0 .. y0 + kMR - 1 of plane z, from v
+template <typename ST, bool VEC>
+D2C_DEV void march_put(ST *channel, int z, const MarchOffsets &f, const d2c_dwconv3d_desc &q, int y0, int x0, const float (&v)[kMR][kVW])
+{
+    const long HW = (long)q.H * q.W;
+    if constexpr (VEC) {
+        const MarchPlane<ST, VEC> p(channel, z, HW, q.D, true);
+#pragma unroll
+        for (int r = 0; r < kMR; r++) {
+            if constexpr (sizeof(ST) == 4)
+                __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{__float_as_uint(v[r][0]), __float_as_uint(v[r][1]), __float_as_uint(v[r][2]), __float_as_uint(v[r][3])},
+                                                       p.rs, (int)f.o[r + 1], 0, 0);
+            else {
+                typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+                __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack_bf16x2(v[r][0], v[r][1]), pack_bf16x2(v[r][2], v[r][3])}, p.rs, (int)f.o[r + 1], 0, 0);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < kMR; r++)
+            if (y0 + r < q.H) march_store<ST, VEC>(channel + z * HW + (long)(y0 + r) * q.W, x0, q.W, v[r]);
+    }
 }
 struct MarchPos {
     int nc, c, y0, x0, z_lo, z_hi, tile;
@@ -522,6 +573,42 @@ D2C_DEV MarchPos march_pos(const d2c_dwconv3d_desc &q, const MarchTiles &t)
     p.z_lo = bz * t.zlen; p.z_hi = min(p.z_lo + t.zlen, q.D);
     p.tile = (p.nc / q.C) * (int)gridDim.y + (int)blockIdx.y;
     return p;
+}
+
+// f(z, phase) for the planes z0 .. z1.  What belongs to planes z - 1, z, z + 1 is entry (0, 1, 2 + phase) % 3 of its array: nothing moves from
+// plane to plane (the moves were a sixth of the instructions).
+template <class F> D2C_DEV void march_planes(int z0, int z1, F f)
+{
+    for (int z = z0; z <= z1; z += 3) {
+        f(z, std::integral_constant<int, 0>{});
+        if (z + 1 > z1) break;
+        f(z + 1, std::integral_constant<int, 1>{});
+        if (z + 2 > z1) break;
+        f(z + 2, std::integral_constant<int, 2>{});
+    }
+}
+// The wavefront's sums of kMTaps values a lane: two values change places half by half, those pairs row by row of 16 lanes, and each row adds up: 70
+// instructions (kMTaps sums of their own, six steps through the LDS path each: 340).  Lanes of row r end with values 7 r .. 7 r + 6.
+D2C_DEV void march_sums(const float (&v)[kMTaps], float (&o)[kMTaps / 4])
+{
+    static_assert(kMTaps == 28, "four rows of seven");
+    float h[14];
+#pragma unroll
+    for (int k = 0; k < 14; k++) {
+        const auto u = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[k]), __float_as_uint(v[k + 14]), false, false);
+        h[k] = __uint_as_float(u[0]) + __uint_as_float(u[1]);
+    }
+#pragma unroll
+    for (int k = 0; k < 7; k++) {
+        const auto u = __builtin_amdgcn_permlane16_swap(__float_as_uint(h[k]), __float_as_uint(h[k + 7]), false, false);
+        float t = __uint_as_float(u[0]) + __uint_as_float(u[1]);
+        auto turned = [&](auto N) INLINE {
+            return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(t), 0x120 + decltype(N)::value, 0xF, 0xF, true));   // row_ror
+        };
+        t += turned(std::integral_constant<int, 8>{}); t += turned(std::integral_constant<int, 4>{});
+        t += turned(std::integral_constant<int, 2>{}); t += turned(std::integral_constant<int, 1>{});
+        o[k] = t;
+    }
 }
 
 // A plane of input touches three planes of results; those of another range are not worked on (the planes in front of and
@@ -544,9 +631,11 @@ __global__ void __launch_bounds__(kThreadsDw) dwc_march_fwd_kernel(d2c_dwconv3d_
 #pragma unroll
     for (int i = 0; i < 3 * kMR * kVW; i++) (&acc[0][0][0])[i] = bv;
     MarchRows cur, nxt;
-    march_rows<ST, VEC, EDGE>(xc + max(p.z_lo - 1, 0) * HW, p.z_lo > 0, p.y0, p.x0, q.H, q.W, cur);
-    for (int z = p.z_lo - 1; z <= p.z_hi; z++) {
-        if (z < p.z_hi) march_rows<ST, VEC, EDGE>(xc + min(z + 1, q.D - 1) * HW, z + 1 < q.D, p.y0, p.x0, q.H, q.W, nxt);
+    const MarchOffsets f = march_offsets<ST, EDGE>(p.y0, p.x0, q.H, q.W);
+    march_rows<ST, VEC, EDGE>(xc, p.z_lo - 1, true, f, q, p.x0, cur);
+    march_planes(p.z_lo - 1, p.z_hi, [&](int z, auto PHASE) INLINE {
+        auto a = [&](int i) INLINE -> float (&)[kMR][kVW] { return acc[(i + decltype(PHASE)::value) % 3]; };
+        march_rows<ST, VEC, EDGE>(xc, z + 1, z < p.z_hi, f, q, p.x0, nxt);
         float v[kMR + 2][kVW + 2];
 #pragma unroll
         for (int j = 0; j < kMR + 2; j++) march_segment<EDGE>(cur, j, v[j]);
@@ -564,20 +653,16 @@ __global__ void __launch_bounds__(kThreadsDw) dwc_march_fwd_kernel(d2c_dwconv3d_
                     for (int kx = 0; kx < 3; kx++)
 #pragma unroll
                         for (int i = 0; i < kVW; i++)
-                            acc[2 - kz][r][i] = fmaf(wv[(kz * 3 + ky) * 3 + kx], v[j][i + kx], acc[2 - kz][r][i]);
+                            a(2 - kz)[r][i] = fmaf(wv[(kz * 3 + ky) * 3 + kx], v[j][i + kx], a(2 - kz)[r][i]);
                 }
         }
-        if (z - 1 >= p.z_lo) {
-#pragma unroll
-            for (int r = 0; r < kMR; r++)
-                if (p.y0 + r < q.H) march_store<ST, VEC>(oc + (z - 1) * HW + (long)(p.y0 + r) * q.W, p.x0, q.W, acc[0][r]);
-        }
+        if (z - 1 >= p.z_lo) march_put<ST, VEC>(oc, z - 1, f, q, p.y0, p.x0, a(0));
 #pragma unroll
         for (int r = 0; r < kMR; r++)
 #pragma unroll
-            for (int i = 0; i < kVW; i++) { acc[0][r][i] = acc[1][r][i]; acc[1][r][i] = acc[2][r][i]; acc[2][r][i] = bv; }
+            for (int i = 0; i < kVW; i++) a(0)[r][i] = bv;
         cur = nxt;
-    }
+    });
 }
 
 // part[tile][channel][kMTaps]: the workgroup's sums of grad_weight and grad_bias (or NULL); gx or NULL
@@ -598,26 +683,25 @@ __global__ void __launch_bounds__(kThreadsDw, 3) dwc_march_bwd_kernel(d2c_dwconv
     for (int i = 0; i < 3 * kMR * kVW; i++) (&acc[0][0][0])[i] = (&xv[0][0][0])[i] = 0.f;
 #pragma unroll
     for (int k = 0; k < kMTaps; k++) gw[k] = 0.f;
+    const MarchOffsets f = march_offsets<ST, EDGE>(p.y0, p.x0, q.H, q.W);
     // (input outside the range is another workgroup's)
-    auto load_x = [&](int z, float (*o)[kVW]) {
+    auto load_x = [&](int z, float (*o)[kVW]) INLINE {
+        const MarchPlane<ST, VEC> xp(xc, z, HW, q.D, part && z < p.z_hi);
 #pragma unroll
-        for (int r = 0; r < kMR; r++)
-            march_load<ST, VEC>(xc + min(z, q.D - 1) * HW + (long)min(p.y0 + r, q.H - 1) * q.W, p.x0, q.W,
-                                part && z < p.z_hi && p.y0 + r < q.H, o[r]);
+        for (int r = 0; r < kMR; r++) march_load<ST, VEC>(xp, f.o[r + 1], p.x0, q.W, o[r]);
     };
     MarchRows cur, nxt;
     float xn[kMR][kVW];
     // (a wavefront below the volume only takes part in the sums)
     const int z_end = __builtin_amdgcn_readfirstlane(p.y0) < q.H ? p.z_hi : p.z_lo - 2;
     if (z_end >= p.z_lo) {
-        march_rows<ST, VEC, EDGE>(gc + max(p.z_lo - 1, 0) * HW, p.z_lo > 0, p.y0, p.x0, q.H, q.W, cur);
+        march_rows<ST, VEC, EDGE>(gc, p.z_lo - 1, true, f, q, p.x0, cur);
         load_x(p.z_lo, xv[2]);
     }
-    for (int z = p.z_lo - 1; z <= z_end; z++) {
-        if (z < p.z_hi) {
-            march_rows<ST, VEC, EDGE>(gc + min(z + 1, q.D - 1) * HW, z + 1 < q.D, p.y0, p.x0, q.H, q.W, nxt);
-            load_x(z + 2, xn);
-        }
+    march_planes(p.z_lo - 1, z_end, [&](int z, auto PHASE) INLINE {
+        constexpr int P = decltype(PHASE)::value;
+        march_rows<ST, VEC, EDGE>(gc, z + 1, z < p.z_hi, f, q, p.x0, nxt);
+        load_x(z + 2, xn);
         float v[kMR + 2][kVW + 2];
 #pragma unroll
         for (int j = 0; j < kMR + 2; j++) {
@@ -640,27 +724,22 @@ __global__ void __launch_bounds__(kThreadsDw, 3) dwc_march_bwd_kernel(d2c_dwconv
                         const int k = (kz * 3 + ky) * 3 + kx;
 #pragma unroll
                         for (int i = 0; i < kVW; i++) {
-                            acc[kz][r][i] = fmaf(wv[k], v[j][i + 2 - kx], acc[kz][r][i]);
-                            gw[k] = fmaf(xv[kz][r][i], v[j][i + 2 - kx], gw[k]);
+                            acc[(kz + P) % 3][r][i] = fmaf(wv[k], v[j][i + 2 - kx], acc[(kz + P) % 3][r][i]);
+                            gw[k] = fmaf(xv[(kz + P) % 3][r][i], v[j][i + 2 - kx], gw[k]);
                         }
                     }
                 }
         }
-        if (gx && z - 1 >= p.z_lo) {
-#pragma unroll
-            for (int r = 0; r < kMR; r++)
-                if (p.y0 + r < q.H)
-                    march_store<ST, VEC>(gx + (long)p.nc * q.D * HW + (z - 1) * HW + (long)(p.y0 + r) * q.W, p.x0, q.W, acc[0][r]);
-        }
+        if (gx && z - 1 >= p.z_lo) march_put<ST, VEC>(gx + (long)p.nc * q.D * HW, z - 1, f, q, p.y0, p.x0, acc[P]);
 #pragma unroll
         for (int r = 0; r < kMR; r++)
 #pragma unroll
             for (int i = 0; i < kVW; i++) {
-                acc[0][r][i] = acc[1][r][i]; acc[1][r][i] = acc[2][r][i]; acc[2][r][i] = 0.f;
-                xv[0][r][i] = xv[1][r][i]; xv[1][r][i] = xv[2][r][i]; xv[2][r][i] = xn[r][i];
+                acc[P][r][i] = 0.f;
+                xv[P][r][i] = xn[r][i];
             }
         cur = nxt;
-    }
+    });
     if (!part) return;
     // Pairs with a position outside the volume, or an input of another range, were zero times something, which is no number
     // where the something is infinite or none: then pair by pair.
@@ -684,10 +763,11 @@ __global__ void __launch_bounds__(kThreadsDw, 3) dwc_march_bwd_kernel(d2c_dwconv
         }
     }
     __shared__ float s_red[kThreadsDw / 64][kMTaps];
+    float sum[kMTaps / 4];
+    march_sums(gw, sum);
+    if ((threadIdx.x & 15) == 0) {
 #pragma unroll
-    for (int k = 0; k < kMTaps; k++) {
-        const float v = wave_sum<float>(gw[k]);
-        if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6][k] = v;
+        for (int k = 0; k < kMTaps / 4; k++) s_red[threadIdx.x >> 6][(threadIdx.x >> 4 & 3) * (kMTaps / 4) + k] = sum[k];
     }
     __syncthreads();
     if (threadIdx.x < kMTaps) {

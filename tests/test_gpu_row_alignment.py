@@ -59,3 +59,25 @@ def test_branch_convolution_rows_of_any_alignment(n, c, o, dims, dev):
     assert rel_l2(results[1][0].cpu(), want.float()) <= 2.0 ** -8
     for got, ref in zip(results[1], results[0]):
         assert rel_l2(got, ref.float()) <= 2.0 ** -8
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,c,dims", [
+    (2, 3, (1, 1, 1)), (1, 5, (2, 3, 5)), (2, 3, (3, 33, 63)), (1, 2, (4, 7, 64)), (1, 3, (5, 9, 65)), (1, 2, (9, 34, 131)), (2, 2, (6, 32, 128)),
+])
+def test_depthwise_rows_of_any_alignment(n, c, dims, dtype, dev):
+    """The plain channel-separated convolution: widths around its vectors and tiles.  Expected: torch's convolution in float64, of values that
+    are rounded once (2^-8 in bfloat16; float32 sums of at most 27 products, of all positions for grad_weight: 1e-5 of the largest)."""
+    from d2conv3d_amd.depthwise_conv import depthwise_separable_conv3d
+    g = torch.Generator().manual_seed(dims[2])
+    rnd = lambda *s: torch.randn(*s, generator=g).to(dtype).to(dev)
+    args, gout = (rnd(n, c, *dims), rnd(c, 1, 3, 3, 3), rnd(c)), rnd(n, c, *dims)
+    ref = [v.double().cpu().requires_grad_(True) for v in args]
+    eo = torch.nn.functional.conv3d(*ref, 1, 1, 1, c)
+    want = (eo.detach(),) + torch.autograd.grad(eo, ref, gout.double().cpu())
+    for place in (torch.clone, _shifted):
+        a = [place(v).requires_grad_(True) for v in args]
+        out = depthwise_separable_conv3d(*a, 1, 1, 1)
+        for got, w in zip((out.detach(),) + torch.autograd.grad(out, a, place(gout)), want):
+            err = (got.double().cpu() - w).abs()
+            assert (err <= 1e-5 * max(1.0, w.abs().max().item()) + (2.0 ** -8 * w.abs() if dtype == torch.bfloat16 else 0.0)).all()
