@@ -67,27 +67,20 @@ inline unsigned dw_grid(const TiledShape &s, int TP, int ny) { return xcd_unit_g
 
 // View over dynamic LDS, one entry per (tap of the batch, position of the tile): the base voxel and
 // live | inrange << 8, and
-//   forward:  the live corner weights * alpha, corner-major (w[corner][entry]);
-//   backward: 16 floats per entry, read as 16-byte vectors: the 8 corner weights * alpha | the per-axis fractions
-//             lz ly lx hz | hy hx, alpha, a pad.
+//   the live corner weights * alpha, read as two 16-byte vectors, and behind them
+//   backward: the per-axis fractions lz ly lx hz | hy hx, alpha, a pad.
 template <int TP, int KB> struct DwTaps {
-    static constexpr int kNE = KB * TP;
-    float (*w)[kNE];
     float4 *pk;
     int *idx, *flag;
 };
 constexpr int kDwEntryVecs = 4;
+constexpr unsigned kNoRow = 0x80000000u;
 template <int TP, int KB> D2C_DEV DwTaps<TP, KB> dw_taps(unsigned char *smem, bool bwd)
 {
     constexpr int kNE = KB * TP;
     DwTaps<TP, KB> t;
     float *f = reinterpret_cast<float *>(smem);
-    t.w = nullptr; t.pk = nullptr;
-    if (bwd) {
-        t.pk = reinterpret_cast<float4 *>(f); f += 4 * kDwEntryVecs * kNE;
-    } else {
-        t.w = reinterpret_cast<float (*)[kNE]>(f); f += 8 * kNE;
-    }
+    t.pk = reinterpret_cast<float4 *>(f); f += 4 * (bwd ? kDwEntryVecs : 2) * kNE;
     t.idx = reinterpret_cast<int *>(f); f += kNE;
     t.flag = reinterpret_cast<int *>(f); f += kNE;
     return t;
@@ -126,15 +119,12 @@ D2C_DEV void dw_coords(const DwArgs &a, const DwTaps<TP, KB> &t, int m0, int m_e
             fr[0] = tp.lz; fr[1] = tp.ly; fr[2] = tp.lx; fr[3] = tp.hz; fr[4] = tp.hy; fr[5] = tp.hx;
         }
         const int e = kk * TP + pl;
+        float4 *q = t.pk + (BWD ? kDwEntryVecs : 2) * e;
+        q[0] = make_float4(w[0], w[1], w[2], w[3]);
+        q[1] = make_float4(w[4], w[5], w[6], w[7]);
         if (BWD) {
-            float4 *q = t.pk + kDwEntryVecs * e;
-            q[0] = make_float4(w[0], w[1], w[2], w[3]);
-            q[1] = make_float4(w[4], w[5], w[6], w[7]);
             q[2] = make_float4(fr[0], fr[1], fr[2], fr[3]);
             q[3] = make_float4(fr[4], fr[5], al, 0.f);
-        } else {
-#pragma unroll
-            for (int c = 0; c < 8; c++) t.w[c][e] = w[c];
         }
         t.idx[e] = idx;
         t.flag[e] = flag;
@@ -166,7 +156,22 @@ template <typename T> D2C_DEV void st4(T *p, const float *v)
 static_assert(kCV == 4, "vector loads of 4 channels");
 
 // ------------------------------------------------------------------ forward
-template <typename T>
+// kCV channels as they come from memory
+template <typename T> struct RawRow { typedef u32x4_t type; };
+template <> struct RawRow<bf16_t> { typedef unsigned type __attribute__((ext_vector_type(2))); };
+template <typename T> D2C_DEV void rows_of(const typename RawRow<T>::type &q, float *v)
+{
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+        for (int i = 0; i < kCV; i++) v[i] = __uint_as_float(q[i]);
+    } else {
+        v[0] = __uint_as_float(q[0] << 16); v[1] = __uint_as_float(q[0] & 0xffff0000u);
+        v[2] = __uint_as_float(q[1] << 16); v[3] = __uint_as_float(q[1] & 0xffff0000u);
+    }
+}
+// RAW: the corner rows of a position are requested one position ahead of their use, through a descriptor that begins at its base voxel; a corner
+// that is not live has an offset past the descriptor's end.  Else row by row, behind branches.
+template <typename T, bool RAW>
 __global__ void __launch_bounds__(kDwThreads) dw_fwd_kernel(DwArgs a)
 {
     constexpr int TP = kFwdTP, KB = kFwdKB, PW = TP / 4;   // PW positions per wavefront
@@ -192,44 +197,91 @@ __global__ void __launch_bounds__(kDwThreads) dw_fwd_kernel(DwArgs a)
     for (int i = 0; i < PW; i++)
 #pragma unroll
         for (int j = 0; j < kCV; j++) acc[i][j] = 0.f;
+    struct Rows {
+        typename RawRow<T>::type x[8];
+    } rows[2];
+    const unsigned cb = cok ? (unsigned)c * (unsigned)sizeof(T) : kNoRow;
+    auto issue = [&](Rows &r, int vflag, int vidx, int p) INLINE {
+        const unsigned live = (unsigned)__builtin_amdgcn_readlane(vflag, p) & 0xffu;
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(xcl + (long)__builtin_amdgcn_readlane(vidx, p) * s.Cin), 0, (int)kNoRow, 0x00020000);
+#pragma unroll
+        for (int cc = 0; cc < 8; cc++) {
+            const int so = (((cc >> 2) & 1) * HW + ((cc >> 1) & 1) * s.W + (cc & 1)) * s.Cin * (int)sizeof(T);
+            const int vo = (int)((live >> cc) & 1u ? cb : kNoRow);
+            if constexpr (sizeof(T) == 4) r.x[cc] = __builtin_amdgcn_raw_buffer_load_b128(rs, vo, so, 0);
+            else r.x[cc] = __builtin_amdgcn_raw_buffer_load_b64(rs, vo, so, 0);
+        }
+    };
 
     for (int k0 = 0; k0 < s.K; k0 += KB) {
         const int kn = min(KB, s.K - k0);
         __syncthreads();
         dw_coords<false, TP, KB>(a, taps, m0, m_end, g, k0, kn);
         __syncthreads();
-        if (!cok) continue;
-        for (int kk = 0; kk < kn; kk++) {
-            float wv[kCV];
-            ld4<T>(wt + (long)(k0 + kk) * s.Cin + c, wv);
+        if constexpr (RAW) {
+            // (entries of a tap's positions: lane p holds those of position p, the next tap's are read a tap ahead)
+            const int e0 = wave * PW + (lane & (PW - 1));
+            int vflag = taps.flag[e0], vidx = taps.idx[e0];
+            issue(rows[0], vflag, vidx, 0);
+            for (int kk = 0; kk < kn; kk++) {
+                float wv[kCV];
+                ld4<T>(wt + (long)(k0 + kk) * s.Cin + c, wv);
+                const int en = min(kk + 1, kn - 1) * TP + e0, nflag = kk + 1 < kn ? taps.flag[en] : 0, nidx = taps.idx[en];
+                for_each_const([&](auto I) INLINE {
+                    constexpr int i = decltype(I)::value;
+                    if constexpr (i + 1 < PW) issue(rows[(i + 1) & 1], vflag, vidx, i + 1);
+                    else issue(rows[(i + 1) & 1], nflag, nidx, 0);
+                    const int e = kk * TP + wave * PW + i;
+                    if (!((unsigned)__builtin_amdgcn_readlane(vflag, i) & 0xffu)) return;
+                    const float4 q0 = taps.pk[2 * e], q1 = taps.pk[2 * e + 1];
+                    const float wc[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+                    float sv[kCV] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int i = 0; i < PW; i++) {
-                const int e = kk * TP + wave * PW + i;
-                // the table entry is the same for the whole wavefront: keep it in scalar registers
-                const unsigned live = (unsigned)__builtin_amdgcn_readfirstlane(taps.flag[e]) & 0xffu;
-                if (!live) continue;
-                const int idx = __builtin_amdgcn_readfirstlane(taps.idx[e]);
-                float xv[8][kCV];
-                // all live corner rows are requested back to back
+                    for (int cc = 0; cc < 8; cc++) {
+                        float xv[kCV];
+                        rows_of<T>(rows[i & 1].x[cc], xv);
 #pragma unroll
-                for (int cc = 0; cc < 8; cc++) {
-                    const int v = idx + ((cc >> 2) & 1) * HW + ((cc >> 1) & 1) * s.W + (cc & 1);
-                    if ((live >> cc) & 1u) {
-                        ld4<T>(xcl + (long)v * s.Cin + c, xv[cc]);
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < kCV; j++) xv[cc][j] = 0.f;
+                        for (int j = 0; j < kCV; j++) sv[j] = fmaf(wc[cc], xv[j], sv[j]);
                     }
+#pragma unroll
+                    for (int j = 0; j < kCV; j++) acc[i][j] = fmaf(wv[j], sv[j], acc[i][j]);
+                }, std::make_integer_sequence<int, PW>{});
+                vflag = nflag; vidx = nidx;
+            }
+        } else {
+            if (!cok) continue;
+            for (int kk = 0; kk < kn; kk++) {
+                float wv[kCV];
+                ld4<T>(wt + (long)(k0 + kk) * s.Cin + c, wv);
+#pragma unroll
+                for (int i = 0; i < PW; i++) {
+                    const int e = kk * TP + wave * PW + i;
+                    // the table entry is the same for the whole wavefront: keep it in scalar registers
+                    const unsigned live = (unsigned)__builtin_amdgcn_readfirstlane(taps.flag[e]) & 0xffu;
+                    if (!live) continue;
+                    const int idx = __builtin_amdgcn_readfirstlane(taps.idx[e]);
+                    float xv[8][kCV];
+                    // all live corner rows are requested back to back
+#pragma unroll
+                    for (int cc = 0; cc < 8; cc++) {
+                        const int v = idx + ((cc >> 2) & 1) * HW + ((cc >> 1) & 1) * s.W + (cc & 1);
+                        if ((live >> cc) & 1u) {
+                            ld4<T>(xcl + (long)v * s.Cin + c, xv[cc]);
+                        } else {
+#pragma unroll
+                            for (int j = 0; j < kCV; j++) xv[cc][j] = 0.f;
+                        }
+                    }
+                    float sv[kCV] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int cc = 0; cc < 8; cc++) {
+                        const float wc = reinterpret_cast<const float *>(taps.pk + 2 * e)[cc];
+#pragma unroll
+                        for (int j = 0; j < kCV; j++) sv[j] = fmaf(wc, xv[cc][j], sv[j]);
+                    }
+#pragma unroll
+                    for (int j = 0; j < kCV; j++) acc[i][j] = fmaf(wv[j], sv[j], acc[i][j]);
                 }
-                float sv[kCV] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int cc = 0; cc < 8; cc++) {
-                    const float wc = taps.w[cc][e];
-#pragma unroll
-                    for (int j = 0; j < kCV; j++) sv[j] = fmaf(wc, xv[cc][j], sv[j]);
-                }
-#pragma unroll
-                for (int j = 0; j < kCV; j++) acc[i][j] = fmaf(wv[j], sv[j], acc[i][j]);
             }
         }
     }
@@ -521,7 +573,11 @@ int d2c_depthwise_forward(const TiledShape &s, const void *xcl, const void *off,
     DwArgs a{s, xcl, off, mask, wt, bias, out, nullptr, nullptr, nullptr, nullptr, nullptr};
     const int nsl = (s.cpg + kSlice - 1) / kSlice;
     D2cProfScope prof(D2C_PROF_FWD, st, "dw_fwd_kernel");
-    hipLaunchKernelGGL(dw_fwd_kernel<T>, dim3(dw_grid(s, kFwdTP, s.G * nsl)), dim3(kDwThreads), kDwLdsFwd, st, a);
+    // (float32 stays with the branches: a corner outside the volume costs the return path its 16 bytes a lane when it is requested, 1024 channels on
+    // 2x8x15x27 200 us and 227, 64 on 8x40x60 153 and 163; bfloat16, half of that, the branches first: 279 and 219, 315 and 169, 256 channels on 7x29x53 386 and 124)
+    const bool raw = sizeof(T) == 2 && ((size_t)s.H * s.W + s.W + 2) * s.Cin * sizeof(T) < (1u << 31);
+    auto kern = raw ? &dw_fwd_kernel<T, sizeof(T) == 2> : &dw_fwd_kernel<T, false>;
+    hipLaunchKernelGGL(kern, dim3(dw_grid(s, kFwdTP, s.G * nsl)), dim3(kDwThreads), kDwLdsFwd, st, a);
     return d2c_check_launch("dw_fwd_kernel");
 }
 
