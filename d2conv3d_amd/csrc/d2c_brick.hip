@@ -105,10 +105,10 @@ D2C_DEV BrickPoint brick_point(const TiledShape &s, const SortWindow &w, const S
     const int ez = (s.keep & 0xF0u) != 0, ey = (s.keep & 0xCCu) != 0, ex = (s.keep & 0xAAu) != 0;
     BrickPoint r;
     r.in = (unsigned)(z0 + ez) < (unsigned)(s.D + ez) && (unsigned)(y0 + ey) < (unsigned)(s.H + ey) && (unsigned)(x0 + ex) < (unsigned)(s.W + ex);
-    // (base voxels start at -1; the quotients are off by a sixth at least from where rounding would matter)
+    // (base voxels start at -1)
     r.zi = z0 + 1;
-    r.yq = (int)floorf(fmaf(fy, 1.f / 3.f, 0.5f)); r.xq = (int)floorf(fmaf(fx, 1.f / 3.f, 0.5f));
-    r.cell = (unsigned)(y0 + 1 - r.yq * 3) | (unsigned)(x0 + 1 - r.xq * 3) << 2;
+    r.yq = brick_block(y0); r.xq = brick_block(x0);
+    r.cell = ((unsigned)(y0 + 1) - (unsigned)r.yq * 3u) | ((unsigned)(x0 + 1) - (unsigned)r.xq * 3u) << 2;
     r.hz = z - fz; r.hy = y - fy; r.hx = x - fx;
     return r;
 }

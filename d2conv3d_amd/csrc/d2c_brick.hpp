@@ -6,6 +6,9 @@
 struct BrickDims {
     int nz, nby, nbx;        // base planes -1 .. D-1; blocks of three base voxels along y and x
 };
+// The block along y or x that base voxel v (-1 on) lies in.  In whole numbers: float quotients go wrong from base voxel 6291457 on, and
+// axes reach 2^23.
+__host__ __device__ __forceinline__ int brick_block(int v) { return (int)((unsigned)(v + 1) / 3u); }
 struct BrickLists {
     int *count;              // points per block
     int *cursor;             // entries given out, then: points outside the volume
