@@ -371,12 +371,17 @@ size_t d2c_conv3d_forward_workspace_bytes(const d2c_conv3d_desc *q)
     return 0;
 }
 
+// (`least`: what a call runs with)
+static size_t backward_ws(const d2c_conv3d_desc &q, bool least)
+{
+    const int a = choose_algo(q, true);
+    if (a == D2C_ALGO_MFMA || a == D2C_ALGO_DEPTHWISE) return d2c_tiled_backward_ws(q, nullptr, false, false, least);
+    return d2c_generic_conv3d_backward_ws(q);
+}
+
 size_t d2c_conv3d_backward_workspace_bytes(const d2c_conv3d_desc *q)
 {
-    if (d2c_conv3d_check(q) != D2C_OK) return 0;
-    const int a = choose_algo(*q, true);
-    if (a == D2C_ALGO_MFMA || a == D2C_ALGO_DEPTHWISE) return d2c_tiled_backward_ws(*q);
-    return d2c_generic_conv3d_backward_ws(*q);
+    return d2c_conv3d_check(q) == D2C_OK ? backward_ws(*q, false) : 0;
 }
 
 static int check_ws(size_t need, void *ws, size_t have)
@@ -459,8 +464,8 @@ int d2c_conv3d_backward_prepared(const d2c_conv3d_desc *q, const void *gout, con
     }
     D2cPrepared prep;
     if (int rc = check_prepared(*q, prepared, prepared_bytes, reuse, &prep)) return rc;
-    if (int rc = check_ws(d2c_tiled_backward_ws(*q), ws, ws_bytes)) return rc;
-    return d2c_tiled_backward(*q, gout, x, offset, mask, weight, gx, goff, gmask, gw, gb, ws, st, nullptr,
+    if (int rc = check_ws(d2c_tiled_backward_ws(*q, nullptr, false, false, true), ws, ws_bytes)) return rc;
+    return d2c_tiled_backward(*q, gout, x, offset, mask, weight, gx, goff, gmask, gw, gb, ws, ws_bytes, st, nullptr,
                               prep.base ? &prep : nullptr);
 }
 
@@ -541,8 +546,8 @@ int d2c_conv3d_backward(const d2c_conv3d_desc *q, const void *gout, const void *
         if (int rc = check_ws(d2c_generic_conv3d_backward_ws(*q), ws, ws_bytes)) return rc;
         return d2c_generic_conv3d_backward(*q, gout, x, offset, mask, weight, gx, goff, gmask, gw, gb, ws, st);
     }
-    if (int rc = check_ws(d2c_tiled_backward_ws(*q), ws, ws_bytes)) return rc;
-    return d2c_tiled_backward(*q, gout, x, offset, mask, weight, gx, goff, gmask, gw, gb, ws, st);
+    if (int rc = check_ws(d2c_tiled_backward_ws(*q, nullptr, false, false, true), ws, ws_bytes)) return rc;
+    return d2c_tiled_backward(*q, gout, x, offset, mask, weight, gx, goff, gmask, gw, gb, ws, ws_bytes, st);
 }
 
 // ---- the operator fed by a size map (dynamic dilation) ----
@@ -606,11 +611,15 @@ size_t d2c_conv3d_forward_least_workspace_bytes(const d2c_conv3d_desc *q, const 
     return forward_least(*q, z, D2C_FWD_WS_GATHER);
 }
 
+// (`least`: what a call runs with)
+static size_t sized_backward_ws(const d2c_conv3d_desc &q, const d2c_size_map_desc *z, bool least)
+{
+    return sized_fused(q, true) ? d2c_tiled_backward_ws(q, z, false, false, least) : 2 * expanded_offsets_bytes(q) + backward_ws(q, least);
+}
+
 size_t d2c_conv3d_sized_backward_workspace_bytes(const d2c_conv3d_desc *q, const d2c_size_map_desc *z)
 {
-    if (sized_check(q, z) != D2C_OK) return 0;
-    if (sized_fused(*q, true)) return d2c_tiled_backward_ws(*q, z);
-    return 2 * expanded_offsets_bytes(*q) + d2c_conv3d_backward_workspace_bytes(q);
+    return sized_check(q, z) == D2C_OK ? sized_backward_ws(*q, z, false) : 0;
 }
 
 int d2c_conv3d_sized_forward(const d2c_conv3d_desc *q, const d2c_size_map_desc *z, const void *x, const void *size_raw,
@@ -635,9 +644,9 @@ int d2c_conv3d_sized_backward(const d2c_conv3d_desc *q, const d2c_size_map_desc 
     if (int rc = sized_check(q, z)) return rc;
     if (!gout || !x || !size_raw || !weight) { d2c_set_error("null tensor pointer"); return D2C_ERR_SHAPE; }
     if (choose_algo(*q, false) < 0) return D2C_ERR_UNSUPPORTED;
-    if (int rc = check_ws(d2c_conv3d_sized_backward_workspace_bytes(q, z), ws, ws_bytes)) return rc;
+    if (int rc = check_ws(sized_backward_ws(*q, z, true), ws, ws_bytes)) return rc;
     if (sized_fused(*q, true))
-        return d2c_tiled_backward(*q, gout, x, size_raw, mask, weight, gx, gsize, gmask, gw, gb, ws,
+        return d2c_tiled_backward(*q, gout, x, size_raw, mask, weight, gx, gsize, gmask, gw, gb, ws, ws_bytes,
                                   (hipStream_t)stream, z);
     const size_t ob = expanded_offsets_bytes(*q);
     char *off = (char *)ws, *goff = off + ob;
@@ -745,8 +754,8 @@ int d2c_conv3d_backward_columns(const d2c_conv3d_desc *q, const d2c_size_map_des
     if (!gout || !x || !offset || !weight) { d2c_set_error("null tensor pointer"); return D2C_ERR_SHAPE; }
     if (int rc = check_columns(*q, z, columns, columns_bytes)) return rc;
     const bool keep = columns_bytes >= d2c_tiled_keep_bytes(*q, z);
-    if (int rc = check_ws(d2c_tiled_backward_ws(*q, z, true, keep), ws, ws_bytes)) return rc;
-    return d2c_tiled_backward(*q, gout, x, offset, mask, weight, gx, goff, gmask, gw, gb, ws, (hipStream_t)stream, z,
+    if (int rc = check_ws(d2c_tiled_backward_ws(*q, z, true, keep, true), ws, ws_bytes)) return rc;
+    return d2c_tiled_backward(*q, gout, x, offset, mask, weight, gx, goff, gmask, gw, gb, ws, ws_bytes, (hipStream_t)stream, z,
                               nullptr, columns, columns_bytes);
 }
 

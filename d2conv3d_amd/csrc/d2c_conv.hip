@@ -1491,7 +1491,7 @@ int d2c_col_forward(const d2c_conv3d_desc &q, const void *col, int rows, const v
 namespace {
 struct GradColPlan {
     int Cp, S, ntile, npair, cgroups;
-    size_t wt_bytes, total;
+    size_t wt_bytes;
 };
 GradColPlan grad_col_plan(const d2c_conv3d_desc &q)
 {
@@ -1502,7 +1502,6 @@ GradColPlan grad_col_plan(const d2c_conv3d_desc &q)
     p.ntile = (M + kWMT - 1) / kWMT;
     p.npair = q.Cin / 64 * q.kd * q.kh * q.kw;
     p.wt_bytes = d2c_align_up((size_t)p.npair * p.S * 8192);
-    p.total = p.wt_bytes + d2c_align_up((size_t)M * p.Cp * 2 + 1024);
     p.cgroups = 1;
     while (p.cgroups < 8 && p.wt_bytes / p.cgroups > (2u << 20)) p.cgroups *= 2;
     return p;
@@ -1519,36 +1518,40 @@ bool d2c_grad_col_supported(const d2c_conv3d_desc &q)
            (long)p.ntile * p.npair * p.S < (1L << 30) &&
            M * 128 < 0xFFFF0000u;
 }
-size_t d2c_grad_col_ws(const d2c_conv3d_desc &q) { return grad_col_plan(q).total; }
+// its operand of grad_out, channels-last (the weights, in its order, take as much as those of tiled_bwd_col32_kernel or less)
+size_t d2c_grad_col_gout_bytes(const d2c_conv3d_desc &q)
+{
+    return d2c_align_up((size_t)q.N * q.Do * q.Ho * q.Wo * grad_col_plan(q).Cp * 2 + 1024);
+}
 // What the backward pass over sorted points needs of grad_out and the weights, and what it adds into, as one launch (one
-// weight group): the operands of d2c_grad_col in its workspace `col_ws`, grad_out in fragment order for the grad_weight
+// weight group): the operands of d2c_grad_col (both or none), grad_out in fragment order for the grad_weight
 // product (`goutp`, see pack_gout_kernel), the bias gradient, two ranges cleared; any of them NULL.  grad_out is read once
 // for both orders.
-int d2c_brick_bwd_prepare(const d2c_conv3d_desc &q, const void *gout, const void *w, void *col_ws, void *goutp, void *gb, void *zero0,
-                          size_t zero0_bytes, void *zero1, size_t zero1_bytes, hipStream_t st)
+int d2c_brick_bwd_prepare(const d2c_conv3d_desc &q, const void *gout, const void *w, void *col_wt, void *col_gout, void *goutp, void *gb,
+                          void *zero0, size_t zero0_bytes, void *zero1, size_t zero1_bytes, hipStream_t st)
 {
     const GradColPlan p = grad_col_plan(q);
     const int K = q.kd * q.kh * q.kw, P = q.Do * q.Ho * q.Wo, M = q.N * P;
     ConvPrepArgs a{};
     a.w = (const bf16_t *)w; a.Cout = q.Cout; a.Cin = q.Cin; a.K = K; a.N = q.N; a.dK = make_fastdiv(K);
-    if (col_ws) {
-        a.gcw = (uint4 *)col_ws; a.gcS = p.S; a.ngcw = (q.Cin * K + 255) / 256; a.nblk_gcw = a.ngcw * p.S * 8;
-        a.gcl = (bf16_t *)((char *)col_ws + p.wt_bytes);
+    if (col_wt) {
+        a.gcw = (uint4 *)col_wt; a.gcS = p.S; a.ngcw = (q.Cin * K + 255) / 256; a.nblk_gcw = a.ngcw * p.S * 8;
+        a.gcl = (bf16_t *)col_gout;
     }
     a.gout = (const bf16_t *)gout; a.gp = (uint4 *)goutp; a.gp_wide = 1;
     a.Cp = p.Cp; a.OBP = p.Cp / 32; a.P = P; a.M = M; a.dP = make_fastdiv(P);
-    a.ngt = (M + 127) / 128 * 2; a.ngc = p.Cp / 64; a.nblk_g = col_ws || goutp ? a.ngt * a.ngc : 0;
+    a.ngt = (M + 127) / 128 * 2; a.ngc = p.Cp / 64; a.nblk_g = col_wt || goutp ? a.ngt * a.ngc : 0;
     a.gb = (bf16_t *)gb; a.nblk_b = gb ? q.Cout : 0;
     prep_zero(a, 0, zero0, zero0_bytes);
     prep_zero(a, 1, zero1, zero1_bytes);
     return prep_launch(a, st);
 }
-int d2c_grad_col(const d2c_conv3d_desc &q, void *gcol, void *ws, hipStream_t st)
+int d2c_grad_col(const d2c_conv3d_desc &q, void *gcol, const void *wt, const void *gcl, hipStream_t st)
 {
     const GradColPlan p = grad_col_plan(q);
     const int M = q.N * q.Do * q.Ho * q.Wo, ncu = d2c_num_cus();
     if (ncu <= 0) return D2C_ERR_LAUNCH;
-    GradColArgs a{(const unsigned char *)ws + p.wt_bytes, (const unsigned char *)ws, (bf16_t *)gcol, (unsigned)p.Cp * 2u, M, p.npair, p.ntile, p.cgroups};
+    GradColArgs a{(const unsigned char *)gcl, (const unsigned char *)wt, (bf16_t *)gcol, (unsigned)p.Cp * 2u, M, p.npair, p.ntile, p.cgroups};
     D2cProfScope prof(D2C_PROF_BWD_DATA, st, "grad_col_kernel");
     const dim3 grid((unsigned)std::max(8, ncu / 8 * 8));
     auto launch = [&](auto S) { hipLaunchKernelGGL((grad_col_kernel<decltype(S)::value>), grid, dim3(kThreads), 0, st, a); };
@@ -1592,11 +1595,7 @@ ColWeightPlan col_weight_plan(const TiledShape &s, size_t scratch, int ncu)
     return p;
 }
 }  // namespace
-bool d2c_col_weight_use(const TiledShape &s, size_t scratch)
-{
-    const int ncu = d2c_num_cus();
-    return ncu > 0 && col_weight_plan(s, scratch, ncu).bytes > 0;
-}
+bool d2c_col_weight_use(const TiledShape &s, size_t scratch) { return col_weight_plan(s, scratch, 1).bytes > 0; }
 int d2c_col_weight(const TiledShape &s, const void *goutp, const void *col, long col_rows, void *gw, void *scratch, size_t scratch_bytes,
                    hipStream_t st)
 {

@@ -10,10 +10,10 @@ int d2c_col_forward_prepare(const d2c_conv3d_desc &q, const void *x, void *xcl, 
                             hipStream_t st);
 int d2c_col_forward(const d2c_conv3d_desc &q, const void *col, int rows, const void *bias, void *out, void *ws, hipStream_t st);
 bool d2c_grad_col_supported(const d2c_conv3d_desc &q);
-size_t d2c_grad_col_ws(const d2c_conv3d_desc &q);
-int d2c_brick_bwd_prepare(const d2c_conv3d_desc &q, const void *gout, const void *w, void *col_ws, void *goutp, void *gb, void *zero0,
-                          size_t zero0_bytes, void *zero1, size_t zero1_bytes, hipStream_t st);
-int d2c_grad_col(const d2c_conv3d_desc &q, void *gcol, void *ws, hipStream_t st);
+size_t d2c_grad_col_gout_bytes(const d2c_conv3d_desc &q);
+int d2c_brick_bwd_prepare(const d2c_conv3d_desc &q, const void *gout, const void *w, void *col_wt, void *col_gout, void *goutp, void *gb,
+                          void *zero0, size_t zero0_bytes, void *zero1, size_t zero1_bytes, hipStream_t st);
+int d2c_grad_col(const d2c_conv3d_desc &q, void *gcol, const void *wt, const void *gcl, hipStream_t st);
 bool d2c_col_weight_use(const TiledShape &s, size_t scratch);
 int d2c_col_weight(const TiledShape &s, const void *goutp, const void *col, long col_rows, void *gw, void *scratch, size_t scratch_bytes,
                    hipStream_t st);
@@ -753,14 +753,23 @@ bool brick_backward(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_co
     return gw_mode(q) != 2 && bwd_slices(q, s).gs == 0 && !(q.dtype == D2C_F32 && col_weight && use_col_weight(q, s));
 }
 
+// grad_weight by col_weight_kernel, its sums in the place of the grad-column rows: where there are columns.  (The rows' place has room for
+// at least as much as `gwacc`.)
+size_t grad_rows_bytes(const d2c_conv3d_desc &q, const TiledShape &s) { return (size_t)s.Cin * s.K * s.M * d2c_elem_size(q.dtype); }
+bool use_wide_weight(const d2c_conv3d_desc &q, const TiledShape &s, bool brick)
+{
+    return brick && q.dtype == D2C_BF16 && s.groups == 1 && d2c_col_weight_use(s, grad_rows_bytes(q, s));
+}
+
 struct BwdWs {
-    size_t xcl, wt, gxcl, gwacc, goutp, auxacc, gcol, counts, entries, ovf, gsacc, sm1, brick, res, gemm, col, total;
+    size_t xcl, wt, gxcl, gwacc, goutp, auxacc, gcol, counts, entries, ovf, gsacc, sm1, brick, res, gcl, col, least, total;
 };
 // `sorted`: ... and the sorted points and the input behind them
 BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns = false, bool sorted = false, bool col_weight = true)
 {
     const bool brick = brick_backward(q, s, saved_columns, col_weight);
     const size_t es = d2c_elem_size(q.dtype);
+    const bool wide = use_wide_weight(q, s, brick);
     BwdWs w;
     w.xcl = 0;
     w.wt = sorted ? 0 : d2c_align_up((size_t)s.N * s.vol * s.Cin * es + 256);   // input, then a 256-byte row of zeros
@@ -768,7 +777,7 @@ BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns =
     const int ogk = d2c_bwd_ogk(s.og < omax ? s.og : omax, q.dtype);
     w.gxcl = w.wt + d2c_align_up((size_t)s.groups * s.K * s.nchunk * bkc_of(q.dtype) * ogk * es);
     w.gwacc = w.gxcl + d2c_align_up((size_t)s.N * s.vol * s.Cin * sizeof(float));
-    w.goutp = w.gwacc + d2c_align_up((size_t)s.Cout * s.cg * s.K * sizeof(float));
+    w.goutp = w.gwacc + (wide ? 0 : d2c_align_up((size_t)s.Cout * s.cg * s.K * sizeof(float)));
     w.auxacc = w.goutp + d2c_align_up(d2c_bwd_goutp_bytes(s, q.dtype));
     // fp32 scratch of the offset / mask gradient, used when the data kernel splits its steps or reduces the output
     // channels in several passes (the partial sums then add up in fp32, whatever the storage type of the result)
@@ -783,6 +792,8 @@ BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns =
         // the rows' place)
         const size_t chunks = sl.gs ? (size_t)sl.gs * (s.cpg / bkc_of(q.dtype)) : (size_t)(s.Cin / bkc_of(q.dtype));
         w.total = w.gcol + d2c_align_up((chunks * s.K * s.M + 64) * bkc_of(q.dtype) * es);
+        // (calls that bring no columns, or want no other gradient, add grad_weight up once the rows are done with, or were not made)
+        if (wide) w.gwacc = w.gcol;
     }
     if (use_lists(q, s) && !brick) {
         size_t c, en, ov;
@@ -801,11 +812,14 @@ BwdWs bwd_ws(const d2c_conv3d_desc &q, const TiledShape &s, bool saved_columns =
     if (brick && !sorted) w.total += d2c_brick_ws(s).total;
     w.res = w.total;       // ... and sums per point
     if (brick) w.total += d2c_brick_ws(s).res_bytes;
-    w.gemm = w.total;      // operands of the grad-column product
-    if (brick && d2c_grad_col_supported(q)) w.total += d2c_grad_col_ws(q);
     w.col = w.total;       // sampled columns for the grad-weight product
     if (!saved_columns && col_weight && use_col_weight(q, s) && !col_in_place(q, s))
         w.total += d2c_align_up(d2c_bwd_col_bytes(s, q.dtype, sl.cgs ? sl.cgs * (s.cpg / 64) : 0));
+    // Operands of grad_col_kernel: the weights in the place of `wt`, grad_out in that of the sums per point and the columns, which are
+    // written later.  Where it takes more than those have, a call with less workspace runs without, on tiled_bwd_col32_kernel.
+    w.gcl = w.res;
+    w.least = w.total;
+    if (brick && d2c_grad_col_supported(q)) w.total = std::max(w.total, w.gcl + d2c_grad_col_gout_bytes(q));
     return w;
 }
 
@@ -813,7 +827,7 @@ template <typename T>
 int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const void *off, const void *mask,
                const void *w, void *gx, void *goff, void *gmask, void *gw, void *gb, void *ws, hipStream_t st,
                int nd = 3, int quirks = 0, const d2c_size_map_desc *sz = nullptr, const D2cPrepared *prep = nullptr,
-               const void *columns = nullptr, size_t columns_bytes = 0)
+               const void *columns = nullptr, size_t columns_bytes = 0, size_t ws_bytes = 0)
 {
     TiledShape s = tiled_shape(q, nd, quirks, sz);
     char *base = (char *)ws;
@@ -899,7 +913,6 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
         off = sm1;
     }
     bool gw_from_col = false, gw_in_place = false, gw_done = false, gw_ready = false, gw_wide = false;
-    const size_t rows_bytes = l.gcol ? (size_t)s.Cin * s.K * s.M * sizeof(T) : 0;
     // (`columns`: the sampled columns the forward call kept -- the offset / mask gradient kernel then writes none, the
     // grad-weight product takes these, and the settings that save workspace by other means do not apply)
     const BwdSlices sl = columns ? BwdSlices{0, 0} : bwd_slices(q, s);
@@ -988,13 +1001,13 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
                 L = d2c_lists_make(s, Elem<T>::DT, base + l.counts, base + l.entries, base + l.ovf);
                 if (int rc = (auxk && !gw_in_place) ? d2c_lists_clear(L, st) : d2c_lists_build(s, off, mask, L, st)) return rc;
             }
-            const bool grad_col = brick && !prep && d2c_grad_col_supported(q);
+            const bool grad_col = brick && !prep && ws_bytes >= l.total && d2c_grad_col_supported(q);
             if (brick && sizeof(T) == 2 && s.groups == 1) {
                 // grad_out and the weights in the orders of the products, the bias gradient, what is added into cleared
                 gw_ready = gw_from_col;
-                gw_wide = gw_ready && !gw_in_place && d2c_col_weight_use(s, rows_bytes);
-                if (int rc = d2c_brick_bwd_prepare(q, gout, w, grad_col ? base + l.gemm : nullptr, gw_ready ? base + l.goutp : nullptr, gb,
-                                                   gxcl, gxcl ? (size_t)s.N * s.vol * s.Cin * sizeof(float) : 0,
+                gw_wide = gw_ready && use_wide_weight(q, s, brick);
+                if (int rc = d2c_brick_bwd_prepare(q, gout, w, grad_col ? base + l.wt : nullptr, base + l.gcl, gw_ready ? base + l.goutp : nullptr,
+                                                   gb, gxcl, gxcl ? (size_t)s.N * s.vol * s.Cin * sizeof(float) : 0,
                                                    gw_ready && !gw_wide ? base + l.gwacc : nullptr, (size_t)s.Cout * s.cg * s.K * sizeof(float), st))
                     return rc;
                 gb = nullptr;
@@ -1003,7 +1016,7 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
                 d2c_fill_zero(gxcl, (size_t)s.N * s.vol * s.Cin * sizeof(float), st);
             }
             if (grad_col) {
-                if (int rc = d2c_grad_col(q, base + l.gcol, base + l.gemm, st)) return rc;
+                if (int rc = d2c_grad_col(q, base + l.gcol, base + l.wt, base + l.gcl, st)) return rc;
             } else if (int rc = d2c_tiled_bwd_data_launch<T>(s, gout, xcl_p, off, mask, w, wt_p,
                                                      lists ? nullptr : gxcl, (lists || auxk) ? base + l.gcol : nullptr,
                                                      auxk ? nullptr : goff, auxk ? nullptr : gmask,
@@ -1056,7 +1069,7 @@ int backward_t(const d2c_conv3d_desc &q, const void *gout, const void *x, const 
         if (gw_wide) {
             // (its sums take the place of the grad-column rows, which are done with)
             if (int rc = d2c_col_weight(s, base + l.goutp, columns ? columns : base + l.col, (long)((s.M + 63) / 64) * 64, gw, base + l.gcol,
-                                        rows_bytes, st))
+                                        grad_rows_bytes(q, s), st))
                 return rc;
         } else if (d2c_tiled_bwd_weight_supported(s, q.dtype)) {
             if (int rc = d2c_tiled_bwd_weight_launch<T>(s, gout, xcl_p, off, mask, base + l.goutp,
@@ -1179,13 +1192,14 @@ size_t d2c_tiled_forward_ws(const d2c_conv3d_desc &q, D2cForwardWs which)
     }
 }
 
-size_t d2c_tiled_backward_ws(const d2c_conv3d_desc &q, const d2c_size_map_desc *sz, bool saved_columns, bool keep)
+size_t d2c_tiled_backward_ws(const d2c_conv3d_desc &q, const d2c_size_map_desc *sz, bool saved_columns, bool keep, bool least)
 {
     const TiledShape s = tiled_shape(q, 3, 0, sz);
     if (is_depthwise(q)) return dw_ws(q, s).total_bwd;
     // (which gradients a call wants is not known here)
     const bool sorted = keep && use_brick_forward(q, s, true);
-    return std::max(bwd_ws(q, s, saved_columns, sorted, true).total, bwd_ws(q, s, saved_columns, sorted, false).total);
+    const BwdWs a = bwd_ws(q, s, saved_columns, sorted, true), b = bwd_ws(q, s, saved_columns, sorted, false);
+    return least ? std::max(a.least, b.least) : std::max(a.total, b.total);
 }
 
 // Bytes of the sampled columns that a forward call can keep for the backward call of the same step:
@@ -1238,10 +1252,10 @@ size_t d2c_tiled_prepared_bytes(const d2c_conv3d_desc &q)
 
 int d2c_tiled_backward(const d2c_conv3d_desc &q, const void *gout, const void *x, const void *off,
                        const void *mask, const void *w, void *gx, void *goff, void *gmask, void *gw, void *gb,
-                       void *ws, hipStream_t st, const d2c_size_map_desc *sz, const D2cPrepared *prep,
+                       void *ws, size_t ws_bytes, hipStream_t st, const d2c_size_map_desc *sz, const D2cPrepared *prep,
                        const void *columns, size_t columns_bytes)
 {
     if (q.dtype == D2C_BF16)
-        return backward_t<bf16_t>(q, gout, x, off, mask, w, gx, goff, gmask, gw, gb, ws, st, 3, 0, sz, prep, columns, columns_bytes);
-    return backward_t<float>(q, gout, x, off, mask, w, gx, goff, gmask, gw, gb, ws, st, 3, 0, sz, prep, columns, columns_bytes);
+        return backward_t<bf16_t>(q, gout, x, off, mask, w, gx, goff, gmask, gw, gb, ws, st, 3, 0, sz, prep, columns, columns_bytes, ws_bytes);
+    return backward_t<float>(q, gout, x, off, mask, w, gx, goff, gmask, gw, gb, ws, st, 3, 0, sz, prep, columns, columns_bytes, ws_bytes);
 }

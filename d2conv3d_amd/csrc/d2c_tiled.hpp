@@ -18,9 +18,9 @@ size_t d2c_tiled_forward_ws(const d2c_conv3d_desc &q, D2cForwardWs which = D2C_F
 // `sz` != nullptr: the offsets are formed from a raw size map (`off` is that map [N, channels(mode), P], `goff` the
 // gradient with respect to it); only where d2c_tiled_sized_supported() says so.
 // `saved_columns`: for a backward call that is handed the sampled columns of its forward call (d2c_tiled_columns_bytes);
-// `keep`: in a buffer of d2c_tiled_keep_bytes()
+// `keep`: in a buffer of d2c_tiled_keep_bytes(); `least`: what the call runs with
 size_t d2c_tiled_backward_ws(const d2c_conv3d_desc &q, const d2c_size_map_desc *sz = nullptr, bool saved_columns = false,
-                             bool keep = false);
+                             bool keep = false, bool least = false);
 size_t d2c_tiled_columns_bytes(const d2c_conv3d_desc &q, const d2c_size_map_desc *sz = nullptr);
 size_t d2c_tiled_keep_bytes(const d2c_conv3d_desc &q, const d2c_size_map_desc *sz = nullptr);
 bool d2c_tiled_sized_supported(const d2c_conv3d_desc &q, bool backward);
@@ -36,8 +36,8 @@ int d2c_tiled_forward(const d2c_conv3d_desc &q, const void *x, const void *off, 
                       const D2cPrepared *prep = nullptr, void *columns = nullptr, size_t columns_bytes = 0);
 int d2c_tiled_backward(const d2c_conv3d_desc &q, const void *gout, const void *x, const void *off,
                        const void *mask, const void *w, void *gx, void *goff, void *gmask, void *gw, void *gb,
-                       void *ws, hipStream_t st, const d2c_size_map_desc *sz = nullptr, const D2cPrepared *prep = nullptr,
-                       const void *columns = nullptr, size_t columns_bytes = 0);
+                       void *ws, size_t ws_bytes, hipStream_t st, const d2c_size_map_desc *sz = nullptr,
+                       const D2cPrepared *prep = nullptr, const void *columns = nullptr, size_t columns_bytes = 0);
 
 // 1-D operator served by the same matrix-core kernels (1 x 1 x L volume).
 bool d2c_tiled1d_supported(const d2c_conv1d_desc &q);

@@ -160,7 +160,10 @@ struct d2c_size_map_desc;
 int d2c_conv3d_packed_supported(const d2c_conv3d_desc *desc, const struct d2c_size_map_desc *size_map);
 size_t d2c_conv3d_forward_workspace_bytes(const d2c_conv3d_desc *desc);
 size_t d2c_conv3d_backward_workspace_bytes(const d2c_conv3d_desc *desc);
-/* d2c_conv3d_forward_workspace_bytes() is what a forward call is fastest with.  Large bfloat16 problems hold their sampled
+/* d2c_conv3d_backward_workspace_bytes() is what a backward call is fastest with (so are the sized, _keep_ and _columns_ queries).  Large
+ * bfloat16 problems of many output channels and few taps may ask for up to two bytes an element of grad_out which a call runs without, too,
+ * on another kernel.
+ * d2c_conv3d_forward_workspace_bytes() is what a forward call is fastest with.  Large bfloat16 problems hold their sampled
  * columns there, taps x the size of the input; given less, but at least this much, the call runs on kernels that
  * need none.  On small problems with up to 128 output channels to a weight group, and the smallest with more, this includes room for partial
  * sums (4 MB at most), without which the call runs too, on fewer workgroups (also d2c_conv3d_sized_forward with its `size_map`, else NULL, d2c_conv3d_forward_prepared, which always does, and
