@@ -570,8 +570,8 @@ __global__ void __launch_bounds__(kThreads, 1) conv_wide_kernel(ConvRowsArgs a)
 }
 
 // out = bias + the partial sums of conv_wide_kernel's tiles from `nfull` on ([piece][column / 4][row][4]): a workgroup = four
-// columns of a tile, a thread = a row.  (2048 -> 256 channels, 7 taps, on 8x30x54, five pieces: 21 us with a column to a
-// workgroup, 13 this way)
+// columns of a tile, a thread = a row; four pieces are requested at a time.  (2048 -> 256 channels, 7 taps, on 8x30x54, five pieces: 21 us
+// with a column to a workgroup, 13 this way; 64 -> 108 on 4x14x25 4.8 with a column to a workgroup, 5.15 with a piece at a time, 4.1)
 __global__ void __launch_bounds__(kWMT) conv_wide_finish_kernel(ConvRowsArgs a, int NT)
 {
     const int nq = NT / 4, rest = blockIdx.x / nq, c4 = blockIdx.x - rest * nq, item = a.nfull + rest, ct = item % a.nctile, tile = item / a.nctile;
@@ -581,9 +581,14 @@ __global__ void __launch_bounds__(kWMT) conv_wide_finish_kernel(ConvRowsArgs a, 
 #pragma unroll
     for (int e = 0; e < 4; e++) v[e] = a.bias && n + e < a.C ? bf16_to_f32(a.bias[n + e]) : 0.f;
     const float4 *q = reinterpret_cast<const float4 *>(a.part) + ((long)rest * a.nsplit * nq + c4) * kWMT + threadIdx.x;
-    for (int s = 0; s < a.nsplit; s++) {
-        const float4 t = q[(long)s * nq * kWMT];
-        v[0] += t.x; v[1] += t.y; v[2] += t.z; v[3] += t.w;
+    for (int s0 = 0; s0 < a.nsplit; s0 += 4) {
+        float4 t[4];
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+            if (s0 + s < a.nsplit) t[s] = q[(long)(s0 + s) * nq * kWMT];
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+            if (s0 + s < a.nsplit) { v[0] += t[s].x; v[1] += t[s].y; v[2] += t[s].z; v[3] += t[s].w; }
     }
     const int b = fdiv(m, a.map.dP), p = m - b * a.map.P;
 #pragma unroll

@@ -48,7 +48,7 @@ D2C_DEV float block_sum(float v, float *red)
 // out f (sums over a group, double).  Few rows are several workgroups each: four to a compute unit in all, since each works out f.  (One workgroup
 // to a row, a vector at a time, rows of odd lengths element by element; us, before and after, forward and gradient, bfloat16: 256 rows of 51360
 // 19.6, 11.4 and 21.1, 15.0; of 51361 62, 13 and 74, 17; 1024 rows of 12960 12.3, 11.4 and 15.7, 14.9; float32 21.3, 17.3 and 25.8, 24.8; 55.8, 17.4 and
-// 59.8, 24.7; 64 rows of 50 3.4, 3.6.)
+// 59.8, 24.7; 64 rows of 50 3.4, 3.9; of 1400 3.8, 3.7.)
 constexpr int kGnVectors = 4;
 inline int row_pieces(const d2c_group_norm_desc &q)
 {
