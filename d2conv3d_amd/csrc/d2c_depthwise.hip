@@ -156,21 +156,8 @@ template <typename T> D2C_DEV void st4(T *p, const float *v)
 static_assert(kCV == 4, "vector loads of 4 channels");
 
 // ------------------------------------------------------------------ forward
-// kCV channels as they come from memory
-template <typename T> struct RawRow { typedef u32x4_t type; };
-template <> struct RawRow<bf16_t> { typedef unsigned type __attribute__((ext_vector_type(2))); };
-template <typename T> D2C_DEV void rows_of(const typename RawRow<T>::type &q, float *v)
-{
-    if constexpr (sizeof(T) == 4) {
-#pragma unroll
-        for (int i = 0; i < kCV; i++) v[i] = __uint_as_float(q[i]);
-    } else {
-        v[0] = __uint_as_float(q[0] << 16); v[1] = __uint_as_float(q[0] & 0xffff0000u);
-        v[2] = __uint_as_float(q[1] << 16); v[3] = __uint_as_float(q[1] & 0xffff0000u);
-    }
-}
-// RAW: the corner rows of a position are requested one position ahead of their use, through a descriptor that begins at its base voxel; a corner
-// that is not live has an offset past the descriptor's end.  Else row by row, behind branches.
+// RAW (bfloat16): the corner rows of a position are requested one position ahead of their use, as they are stored, through a descriptor that begins
+// at its base voxel; a corner that is not live has an offset past the descriptor's end.  Else row by row, behind branches.
 template <typename T, bool RAW>
 __global__ void __launch_bounds__(kDwThreads) dw_fwd_kernel(DwArgs a)
 {
@@ -197,8 +184,9 @@ __global__ void __launch_bounds__(kDwThreads) dw_fwd_kernel(DwArgs a)
     for (int i = 0; i < PW; i++)
 #pragma unroll
         for (int j = 0; j < kCV; j++) acc[i][j] = 0.f;
+    static_assert(!RAW || sizeof(T) == 2, "rows of four bfloat16 channels");
     struct Rows {
-        typename RawRow<T>::type x[8];
+        unsigned __attribute__((ext_vector_type(2))) x[8];
     } rows[2];
     const unsigned cb = cok ? (unsigned)c * (unsigned)sizeof(T) : kNoRow;
     auto issue = [&](Rows &r, int vflag, int vidx, int p) INLINE {
@@ -207,9 +195,7 @@ __global__ void __launch_bounds__(kDwThreads) dw_fwd_kernel(DwArgs a)
 #pragma unroll
         for (int cc = 0; cc < 8; cc++) {
             const int so = (((cc >> 2) & 1) * HW + ((cc >> 1) & 1) * s.W + (cc & 1)) * s.Cin * (int)sizeof(T);
-            const int vo = (int)((live >> cc) & 1u ? cb : kNoRow);
-            if constexpr (sizeof(T) == 4) r.x[cc] = __builtin_amdgcn_raw_buffer_load_b128(rs, vo, so, 0);
-            else r.x[cc] = __builtin_amdgcn_raw_buffer_load_b64(rs, vo, so, 0);
+            r.x[cc] = __builtin_amdgcn_raw_buffer_load_b64(rs, (int)((live >> cc) & 1u ? cb : kNoRow), so, 0);
         }
     };
 
@@ -238,8 +224,8 @@ __global__ void __launch_bounds__(kDwThreads) dw_fwd_kernel(DwArgs a)
                     float sv[kCV] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                     for (int cc = 0; cc < 8; cc++) {
-                        float xv[kCV];
-                        rows_of<T>(rows[i & 1].x[cc], xv);
+                        const unsigned lo = rows[i & 1].x[cc][0], hi = rows[i & 1].x[cc][1];
+                        const float xv[kCV] = {__uint_as_float(lo << 16), __uint_as_float(lo & 0xffff0000u), __uint_as_float(hi << 16), __uint_as_float(hi & 0xffff0000u)};
 #pragma unroll
                         for (int j = 0; j < kCV; j++) sv[j] = fmaf(wc[cc], xv[j], sv[j]);
                     }
