@@ -420,14 +420,12 @@ MarchTiles march_tiles(const d2c_dwconv3d_desc &q)
 bool march_ok(const d2c_dwconv3d_desc &q)
 {
     return q.dtype != D2C_F64 && q.Cout == q.C && q.kd == 3 && q.kh == 3 && q.kw == 3 && q.sd == 1 && q.sh == 1 && q.sw == 1 &&
-           q.pd == 1 && q.ph == 1 && q.pw == 1 && q.dd == 1 && q.dh == 1 && q.dw == 1 &&
-           (long)q.D * q.H * q.W * 4 < (1l << 31);        // (a channel through 32-bit offsets)
+           q.pd == 1 && q.ph == 1 && q.pw == 1 && q.dd == 1 && q.dh == 1 && q.dw == 1;
 }
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 typedef unsigned short u16x4_any __attribute__((ext_vector_type(4), aligned(2)));
-template <typename ST, bool VEC> D2C_DEV void march_store(ST *row, int x0, int width, const float *m)
+template <typename ST> D2C_DEV void march_store(ST *row, int x0, int width, const float *m)
 {
-    static_assert(!VEC, "see march_put");
     if (x0 + kVW <= width) {
         if constexpr (sizeof(ST) == 4) *reinterpret_cast<f32x4_any *>(row + x0) = f32x4_any{m[0], m[1], m[2], m[3]};
         else {
@@ -440,7 +438,8 @@ template <typename ST, bool VEC> D2C_DEV void march_store(ST *row, int x0, int w
             if (x0 + i < width) stv<ST>(row, x0 + i, m[i]);
     }
 }
-// Rows are read through a buffer descriptor of what is left of the channel from a plane on.  What lies outside the volume has an offset
+// Rows are read through a buffer descriptor of what is left of the channel from a plane on (65535 tiles of 16 x 64 elements to a channel, the
+// limit of d2c_dwconv3d_check, are far below 2 GiB).  What lies outside the volume has an offset
 // past the descriptor's end and is zero, without a branch and without registers cleared in front of the load; what a vector brings from
 // behind its row is cleared afterwards (not VEC).  bfloat16 rows that are not vectors: the words around their elements, shifted; the descriptor begins and
 // ends with a whole word then, `skip` bytes in front of the plane.
@@ -496,10 +495,10 @@ template <typename ST, bool VEC> D2C_DEV void march_load(const MarchPlane<ST, VE
         m[0] = __uint_as_float(lo << 16); m[1] = __uint_as_float(lo & 0xffff0000u);
         m[2] = __uint_as_float(hi << 16); m[3] = __uint_as_float(hi & 0xffff0000u);
     }
+    // (the first element is zero already where it lies outside, shifted or not)
     if constexpr (!VEC) {
 #pragma unroll
         for (int i = 1; i < kVW; i++) m[i] = x0 + i < width ? m[i] : 0.f;
-        // (shifted, the first element of a vector outside the volume is one of nothing: zero already)
     }
 }
 template <typename ST, bool VEC> D2C_DEV float march_element(const MarchPlane<ST, VEC> &p, unsigned o)
@@ -562,7 +561,7 @@ D2C_DEV void march_put(ST *channel, int z, const MarchOffsets &f, const d2c_dwco
     } else {
 #pragma unroll
         for (int r = 0; r < kMR; r++)
-            if (y0 + r < q.H) march_store<ST, VEC>(channel + z * HW + (long)(y0 + r) * q.W, x0, q.W, v[r]);
+            if (y0 + r < q.H) march_store<ST>(channel + z * HW + (long)(y0 + r) * q.W, x0, q.W, v[r]);
     }
 }
 struct MarchPos {
