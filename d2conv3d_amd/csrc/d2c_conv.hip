@@ -620,7 +620,10 @@ __global__ void __launch_bounds__(256) conv_rows_finish_kernel(const float *part
 // registers and 32 lanes write a whole row, without LDS and without an exchange between lanes.
 // An XCD's workgroups share a range of pairs whose weights fit its L2 (cgroups ranges) and, where there are fewer than
 // eight, a range of row tiles; runs go along the pairs of a row tile.
-// MEASURED
+// Bound: the rows it writes (256 -> 256 channels on 32x60x108: 2.9 GB at 3.9 TB/s), with more output channels the matrix instructions beside them
+// (512 -> 512 in 8 groups on 2x8x30x54: matrix cores busy for 61 % of the cycles, at the 2.0 GHz that the chip holds meanwhile, 2.4 TB/s).
+// us, tiles of 256 x 256 with both operands and the results through LDS (above 256 output channels: tiled_bwd_col32_kernel), and this way:
+// 256 -> 256 on 2x8x30x54 142, 106; on 32x60x108 965, 731; 1024 -> 256 on 8x30x54 263, 191; 512 -> 512 in 8 groups 427, 360.
 struct GradColArgs {
     const unsigned char *src;         // channels-last grad_out, rows of `rowb` bytes
     const unsigned char *wt;          // [pair][step][64 columns][64] bfloat16, slots swizzled
@@ -810,17 +813,20 @@ D2C_DEV void grad_col_weight(const bf16_t *w, uint4 *wt, int Cout, int Cin, int 
 // Every workgroup stores its sums; col_weight_finish_kernel adds them up on their way into grad_weight.  (Float atomics into one
 // accumulator, all workgroups at the end of the launch, take 40 us for the 62 MB of 256 -> 256 channels, these stores 10.)
 // The kernel it took the place of (tiled_bwd_weight_col_kernel: 512 output channels x 128 columns, with 256 channels half of its
-// wavefronts multiply nothing; kept for the calls that have no room for the sums), us, the sums brought into grad_weight included:
+// wavefronts multiply nothing; it still serves several weight groups, columns in the rows' place, slices, calls that want grad_weight alone
+// over kept columns, and sums that have no room where the grad-column rows were), us, the sums brought into grad_weight included:
 // 512 -> 512 in 8 groups on 2x8x30x54 413, 332; 256 -> 256 there 146, 114; on 32x60x108 869, 619 (reading 2.9 GB of columns once takes
 // 520); 1024 -> 256 on 8x30x54 230, 192; 2048 -> 256 with 7 taps 130, 116.  Whole training steps of small problems gain too:
-// 128 -> 64 on 420 positions 104, 101; 128 -> 128 on 1400 122, 112; 512 -> 512 267, 238.
+// 128 -> 64 on 420 positions 104, 101; 128 -> 128 on 1400 122, 112; 512 -> 512 267, 238; tiles that are mostly padding lose nothing (both
+// products' kernels of before, and these: 256 -> 1 on 12960 308, 285; 256 -> 40 291, 290; 256 -> 130 332, 323; 512 -> 144 564, 543).
+// One weight group.
 struct ColWeightArgs {
-    const unsigned char *gp;          // [weight group][tile of 128 positions][row block of 32][k-group of 16][lane] 16 bytes
+    const unsigned char *gp;          // [tile of 128 positions][row block of 32][k-group of 16][lane] 16 bytes
     const unsigned char *col;         // [pair][position][64] bfloat16
     float *part;                      // [piece][item][pair of 4][16 x 4 channels][OT][4]
     long pair_bytes;
-    int npair, nci, otiles, nitem;    // pairs of a weight group, sets of four, tiles of OT output channels; items in all
-    int OBT, ntp;                     // row blocks and tiles of the fragments
+    int npair, otiles, nitem;         // pairs, tiles of OT output channels, items (tiles x sets of four pairs)
+    int OBT;                          // row blocks of the fragments
     int ntile, nsplit;
 };
 template <int OT>
@@ -834,20 +840,20 @@ __global__ void __launch_bounds__(kThreads, 1) col_weight_kernel(ColWeightArgs a
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int id = xcd_swizzle(blockIdx.x, gridDim.x), piece = id / a.nitem, item = id - piece * a.nitem;
-    const int ot = item % a.otiles, set = item / a.otiles, wg = set / a.nci, ci = set - wg * a.nci;
+    const int ot = item % a.otiles, ci = item / a.otiles;
     const int t_lo = (int)((long)a.ntile * piece / a.nsplit), t_hi = (int)((long)a.ntile * (piece + 1) / a.nsplit);
 
     // --- requests: a wavefront fetches the columns of a pair (past the last pair: that one again, stored in no gradient), eight
     // rows at a time; 16-byte pieces of a row are permuted so that the transposing reads, 64 bytes of four consecutive rows,
     // meet no bank twice
     const int pair = min(ci * 4 + wave, a.npair - 1);
-    const unsigned char *asrc = a.col + ((long)wg * a.npair + pair) * a.pair_bytes + (long)t_lo * 8192 + (lane >> 3) * 128 +
+    const unsigned char *asrc = a.col + pair * a.pair_bytes + (long)t_lo * 8192 + (lane >> 3) * 128 +
                                 ((lane & 7) ^ ((lane >> 4) & 1) << 2) * 16;
     int at = t_lo, bt = t_lo;                              // the tiles that the next requests belong to
     // (after the last tile: that one again, which nothing reads)
     auto advance_cols = [&]() { if (at + 1 < t_hi) { at++; asrc += 8192; } };
     // ... and k-group `wave` of every row block (past the last block: that one again)
-    const unsigned char *bsrc = a.gp + (((long)wg * a.ntp + (t_lo >> 1)) * a.OBT * 8 + (t_lo & 1) * 4 + wave) * 1024 + lane * 16;
+    const unsigned char *bsrc = a.gp + ((long)(t_lo >> 1) * a.OBT * 8 + (t_lo & 1) * 4 + wave) * 1024 + lane * 16;
     unsigned bo[BD];
 #pragma unroll
     for (int i = 0; i < BD; i++) bo[i] = (unsigned)min(ot * (OT / 32) + i, a.OBT - 1) * 8192u;
@@ -958,22 +964,20 @@ constexpr int kFinOut = 8;
 struct ColWeightFinishArgs {
     const float *part;
     bf16_t *gw;
-    int nsplit, nitem, nci, otiles, OT, K, og, cg, nob;    // nob: sets of kFinOut output channels of a weight group
+    int nsplit, nitem, otiles, OT, K, Cout, Cin, nob;      // nob: sets of kFinOut output channels
     int wide;                                              // `gw` on 16 bytes
 };
 __global__ void __launch_bounds__(256) col_weight_finish_kernel(ColWeightFinishArgs a)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    int b = blockIdx.x;
-    const int ob = b % a.nob; b /= a.nob;
-    const int c16 = b % (a.cg / 16), wg = b / (a.cg / 16);
+    const int ob = blockIdx.x % a.nob, c16 = blockIdx.x / a.nob;
     const int j = c16 >> 2, run = 16 * a.K, rs = run * 2 + 16;         // chunk; elements of a row, bytes of it in LDS
-    const int o0 = ob * kFinOut, ot = o0 / a.OT, nr = min(kFinOut, a.og - o0);
+    const int o0 = ob * kFinOut, ot = o0 / a.OT, nr = min(kFinOut, a.Cout - o0);
     const float4 *const part = reinterpret_cast<const float4 *>(a.part) + (o0 - ot * a.OT);
     const long piece = (long)a.nitem * 64 * a.OT;
     for (int i = threadIdx.x; i < a.K * 32; i += 256) {
         const int o = i & 7, c4 = (i >> 3) & 3, k = i >> 5, pair = j * a.K + k;
-        const float4 *q = part + ((((long)wg * a.nci + (pair >> 2)) * a.otiles + ot) * 64 + (pair & 3) * 16 + (c16 & 3) * 4 + c4) * a.OT + o;
+        const float4 *q = part + (((long)(pair >> 2) * a.otiles + ot) * 64 + (pair & 3) * 16 + (c16 & 3) * 4 + c4) * a.OT + o;
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll 4
         for (int s = 0; s < a.nsplit; s++) {
@@ -984,8 +988,8 @@ __global__ void __launch_bounds__(256) col_weight_finish_kernel(ColWeightFinishA
         d[0] = f32_to_bf16(v.x); d[a.K] = f32_to_bf16(v.y); d[2 * a.K] = f32_to_bf16(v.z); d[3 * a.K] = f32_to_bf16(v.w);
     }
     __syncthreads();
-    bf16_t *const dst = a.gw + (((long)wg * a.og + o0) * a.cg + c16 * 16) * a.K;
-    const long row = (long)a.cg * a.K;
+    bf16_t *const dst = a.gw + ((long)o0 * a.Cin + c16 * 16) * a.K;
+    const long row = (long)a.Cin * a.K;
     if (a.wide) {
         const int nv = run / 8;
         for (int i = threadIdx.x; i < nr * nv; i += 256) {
@@ -1576,16 +1580,15 @@ int d2c_grad_col(const d2c_conv3d_desc &q, void *gcol, const void *wt, const voi
 // ---- grad_weight over sampled columns, sums in `scratch`
 namespace {
 struct ColWeightPlan {
-    int OT, otiles, nci, nitem, ntile, nsplit;
+    int OT, otiles, nitem, ntile, nsplit;
     size_t bytes;                     // of the sums; 0: not on this kernel
 };
 ColWeightPlan col_weight_plan(const TiledShape &s, size_t scratch, int ncu)
 {
     ColWeightPlan p{};
-    p.OT = s.og > 128 ? 256 : 128;
-    p.otiles = (s.og + p.OT - 1) / p.OT;
-    p.nci = (s.nchunk * s.K + 3) / 4;
-    p.nitem = p.nci * p.otiles * s.groups;
+    p.OT = s.Cout > 128 ? 256 : 128;
+    p.otiles = (s.Cout + p.OT - 1) / p.OT;
+    p.nitem = (s.nchunk * s.K + 3) / 4 * p.otiles;
     p.ntile = (s.M + 63) / 64;
     if (kFinOut * ((size_t)s.K * 32 + 16) > 64 * 1024) return p;
     // pieces by what they cost in steps of a compute unit: rounds, each its steps and about eight more for its start and end, and
@@ -1608,8 +1611,8 @@ int d2c_col_weight(const TiledShape &s, const void *goutp, const void *col, long
     if (ncu <= 0) return D2C_ERR_LAUNCH;
     const ColWeightPlan p = col_weight_plan(s, scratch_bytes, ncu);
     {
-        ColWeightArgs a{(const unsigned char *)goutp, (const unsigned char *)col, (float *)scratch, col_rows * 128, s.nchunk * s.K, p.nci, p.otiles,
-                        p.nitem, (s.og + 63) / 64 * 2, (s.M + 127) / 128, p.ntile, p.nsplit};
+        ColWeightArgs a{(const unsigned char *)goutp, (const unsigned char *)col, (float *)scratch, col_rows * 128, s.nchunk * s.K, p.otiles,
+                        p.nitem, (s.Cout + 63) / 64 * 2, p.ntile, p.nsplit};
         D2cProfScope prof(D2C_PROF_BWD_WEIGHT, st, "col_weight_kernel");
         const dim3 grid((unsigned)(p.nitem * p.nsplit));
         if (p.OT == 256) hipLaunchKernelGGL(col_weight_kernel<256>, grid, dim3(kThreads), 0, st, a);
@@ -1617,9 +1620,9 @@ int d2c_col_weight(const TiledShape &s, const void *goutp, const void *col, long
         if (int rc = d2c_check_launch("col_weight_kernel")) return rc;
     }
     D2cProfScope prof(D2C_PROF_PACK, st);
-    ColWeightFinishArgs f{(const float *)scratch, (bf16_t *)gw, p.nsplit, p.nitem, p.nci, p.otiles, p.OT, s.K, s.og, s.cg,
-                          (s.og + kFinOut - 1) / kFinOut, reinterpret_cast<uintptr_t>(gw) % 16 == 0};
-    hipLaunchKernelGGL(col_weight_finish_kernel, dim3((unsigned)(s.groups * (s.cg / 16) * f.nob)), dim3(256), kFinOut * ((size_t)s.K * 32 + 16), st, f);
+    ColWeightFinishArgs f{(const float *)scratch, (bf16_t *)gw, p.nsplit, p.nitem, p.otiles, p.OT, s.K, s.Cout, s.Cin,
+                          (s.Cout + kFinOut - 1) / kFinOut, reinterpret_cast<uintptr_t>(gw) % 16 == 0};
+    hipLaunchKernelGGL(col_weight_finish_kernel, dim3((unsigned)(s.Cin / 16 * f.nob)), dim3(256), kFinOut * ((size_t)s.K * 32 + 16), st, f);
     return d2c_check_launch("col_weight_finish_kernel");
 }
 
