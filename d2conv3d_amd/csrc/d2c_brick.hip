@@ -189,7 +189,7 @@ __global__ void __launch_bounds__(1024) brick_range_kernel(BrickLists L, int nse
     if (i < nseg) L.end[i] = s_sum[wave] + sum - n;       // (the filing pass takes entries from here on and leaves the end)
 }
 template <bool AUX16, bool SIZED>
-__global__ void __launch_bounds__(kSortThreads, 8)     // (two workgroups to a compute unit)
+__global__ void __launch_bounds__(kSortThreads, 8)     // (two workgroups to a compute unit, for 16 - 20 bytes of spills a lane)
 brick_file_kernel(TiledShape s, BrickDims d, BrickLists L, const void *off, const void *mask, SortWindow w, long n)
 {
     typedef typename std::conditional<AUX16, bf16_t, float>::type AT;
