@@ -621,7 +621,7 @@ __global__ void __launch_bounds__(256) conv_rows_finish_kernel(const float *part
 // An XCD's workgroups share a range of pairs whose weights fit its L2 (cgroups ranges) and, where there are fewer than
 // eight, a range of row tiles; runs go along the pairs of a row tile.
 // Bound: the rows it writes (256 -> 256 channels on 32x60x108: 2.9 GB at 3.9 TB/s), with more output channels the matrix instructions beside them
-// (512 -> 512 in 8 groups on 2x8x30x54: matrix cores busy for 61 % of the cycles, at the 2.0 GHz that the chip holds meanwhile, 2.4 TB/s).
+// (512 -> 512 in 8 groups on 2x8x30x54: matrix cores busy for 61 % of the cycles, at the 1.9 GHz that the chip holds meanwhile, 2.4 TB/s).
 // us, tiles of 256 x 256 with both operands and the results through LDS (above 256 output channels: tiled_bwd_col32_kernel), and this way:
 // 256 -> 256 on 2x8x30x54 142, 106; on 32x60x108 965, 731; 1024 -> 256 on 8x30x54 263, 191; 512 -> 512 in 8 groups 427, 360.
 struct GradColArgs {

@@ -203,7 +203,7 @@ int d2c_conv3d_backward(const d2c_conv3d_desc *desc, const void *grad_out, const
  * memory to spare hands d2c_conv3d_forward_columns a buffer of d2c_conv3d_columns_bytes() bytes (256-byte aligned;
  * taps x the size of the input, in the element type): the forward kernel writes there what it multiplies with the
  * weights anyway, and d2c_conv3d_backward_columns, given that buffer UNCHANGED together with the same tensors, runs
- * its grad-weight product over it instead of sampling again (N=2, C=512, 8x30x54, bfloat16: 2.14 -> 1.78 ms per step
+ * its grad-weight product over it instead of sampling again (N=2, C=512, 8x30x54, bfloat16: 2.00 -> 1.58 ms per step
  * for 878 MB held between the two calls -- 717 of columns, sorted sampling points, the input channels-last, see d2c_conv3d_keep_bytes() -- and
  * 0.88 GB less backward workspace; N=2, C=256, 8x30x54, float32: 1.68 ms for 717 MB).  Results are those of the plain calls up to the order of floating-point sums; float32
  * columns are the interpolated floats themselves and their product keeps float32's accuracy (three bfloat16 terms
